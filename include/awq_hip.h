@@ -67,6 +67,12 @@ int awq_dequantize_transposed(const int32_t* qweight, const void* qscales, const
 int awq_quantize_pack(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros,
                       int64_t N, int64_t K, int64_t group_size, int dtype, void* stream);
 
+/* The same; sets *nan_flag (a device int32 that the caller has zeroed; may be null) to 1 if the weight holds a
+ * NaN, in which case the packed buffers mean nothing. */
+int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros,
+                              int64_t N, int64_t K, int64_t group_size, int dtype, int32_t* nan_flag,
+                              void* stream);
+
 /* Bytes of device workspace awq_gemv / awq_gemm / awq_linear need for this
  * problem (0 is possible).  The workspace must be zero-filled ONCE when it is
  * allocated; every call leaves it in that state (its counters are reset by

@@ -49,7 +49,6 @@ def quantize_pack(weight: torch.Tensor, group_size: int, output_dtype: torch.dty
     if weight.device.type != "cuda":
         raise _lib.AwqHipError(f"quantize_pack runs on a HIP device only (tensor is on {weight.device})")
     assert weight.dim() == 2 and weight.dtype == torch.float32, "an fp32 [out_features, in_features] weight"
-    assert not bool(torch.isnan(weight).any()), "weight should not contain nan"
     weight = weight.contiguous()
     N, K = weight.shape
     g = K if group_size <= 0 else group_size
@@ -58,8 +57,11 @@ def quantize_pack(weight: torch.Tensor, group_size: int, output_dtype: torch.dty
     qweight = torch.empty(K, N // 8, dtype=torch.int32, device=dev)
     qzeros = torch.empty(K // g, N // 8, dtype=torch.int32, device=dev)
     qscales = torch.empty(K // g, N, dtype=output_dtype, device=dev)
+    # the kernel looks for NaN on its way: a pass of its own would read the whole weight twice more
+    nan = torch.zeros(1, dtype=torch.int32, device=dev)
     with torch.cuda.device(dev):
-        _lib.check(_lib.lib().awq_quantize_pack(weight.data_ptr(), qweight.data_ptr(), qscales.data_ptr(),
-                                                qzeros.data_ptr(), N, K, g, _lib.dtype_id(output_dtype),
-                                                torch.cuda.current_stream().cuda_stream))
+        _lib.check(_lib.lib().awq_quantize_pack_flagged(weight.data_ptr(), qweight.data_ptr(), qscales.data_ptr(),
+                                                        qzeros.data_ptr(), N, K, g, _lib.dtype_id(output_dtype),
+                                                        nan.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    assert not nan.item(), "weight should not contain nan"
     return qweight, qscales, qzeros

@@ -28,6 +28,43 @@ def test_quantize_pack_bit_exact(dtype, N, K, g):
     assert np.array_equal(qs.cpu().view(torch.int16).numpy().view(np.uint16), ref["qscales"])
 
 
+# both tile widths at their edges: words past the last tile, columns past K, the switch between the widths (4096 x 4096),
+# and rows that are not 16-byte aligned, which take the general kernel
+@pytest.mark.parametrize("N,K,g,offset", [(264, 192, 64, 0), (72, 96, 32, 0), (520, 160, 32, 0), (248, 128, 128, 0),
+                                          (4088, 4096, 128, 0), (4096, 4128, 32, 0), (264, 256, 128, 1)])
+def test_quantize_tiles_bit_exact(N, K, g, offset):
+    """Quotients exactly halfway between two codes, ones next to them, huge and tiny groups, infinities."""
+    import nanoquantization_amd as nq
+    rng = np.random.default_rng(N + K + g)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(np.float32)
+    half = (np.arange(g) % 31 - 0.5).astype(np.float32)      # lo = -0.5, hi = 29.5: s = 2, v / s in quarters
+    w[0, :g] = half
+    w[3, -g:] = np.nextafter(half, np.float32(np.inf))
+    w[5, -g:] = np.nextafter(half, np.float32(-np.inf))
+    w[N - 1, -g:] = 1000.0 + half * 1e-4                     # quotients with few fraction bits
+    w[N - 2, :g] *= np.float32(1e-30)
+    w[N - 3, :g] *= np.float32(1e30)
+    w[N - 4, :g] = np.where(np.arange(g) % 2, np.float32(3e38), np.float32(-3e38))     # hi - lo overflows
+    w[N - 5, g - 1] = np.inf
+    with np.errstate(all="ignore"):
+        ref = o.make_packed(w, g, "bf16")
+    buf = torch.zeros(N * K + offset, device="cuda")
+    wd = buf[offset:].view(N, K)
+    wd.copy_(torch.from_numpy(w))
+    qw, qs, qz = nq.quantize_pack(wd, g, torch.bfloat16)
+    finite = np.ones(N, bool)
+    finite[[N - 4, N - 5]] = False        # what the oracle makes of a NaN quotient is the host's conversion of a NaN
+    words = finite.reshape(-1, 8).all(axis=1)
+    assert np.array_equal(qw.cpu().numpy()[:, words], ref["qweight"][:, words])
+    assert np.array_equal(qz.cpu().numpy()[:, words], ref["qzeros"][:, words])
+    assert np.array_equal(qs.cpu().view(torch.int16).numpy().view(np.uint16)[:, finite], ref["qscales"][:, finite])
+    for at in ((0, 0), (N - 1, K - 1), (N // 2, g - 1)):
+        bad = wd.clone()
+        bad[at] = float("nan")
+        with pytest.raises(AssertionError, match="nan"):
+            nq.quantize_pack(bad, g, torch.bfloat16)
+
+
 def test_quantize_pack_feeds_the_linear():
     import nanoquantization_amd as nq
     torch.manual_seed(0)
