@@ -260,9 +260,8 @@ void launch_quantize(const float* w, uint32_t* qw, uint32_t* qz, uint16_t* qs, i
 
 using namespace awq;
 
-extern "C" int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros, int64_t N,
-                                         int64_t K, int64_t group_size, int dtype, int32_t* nan_flag, void* stream) {
-    const char* fn = "awq_quantize_pack";
+static int quantize_pack(const char* fn, const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros, int64_t N,
+                         int64_t K, int64_t group_size, int dtype, int32_t* nan_flag, void* stream) {
     if (!weight || !qweight || !qscales || !qzeros) {
         set_error("%s: null pointer argument", fn);
         return AWQ_ERR_INVALID_ARG;
@@ -295,5 +294,11 @@ extern "C" int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, 
 
 extern "C" int awq_quantize_pack(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros, int64_t N,
                                  int64_t K, int64_t group_size, int dtype, void* stream) {
-    return awq_quantize_pack_flagged(weight, qweight, qscales, qzeros, N, K, group_size, dtype, nullptr, stream);
+    return quantize_pack("awq_quantize_pack", weight, qweight, qscales, qzeros, N, K, group_size, dtype, nullptr, stream);
+}
+
+extern "C" int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros, int64_t N,
+                                         int64_t K, int64_t group_size, int dtype, int32_t* nan_flag, void* stream) {
+    return quantize_pack("awq_quantize_pack_flagged", weight, qweight, qscales, qzeros, N, K, group_size, dtype, nan_flag,
+                         stream);
 }
