@@ -73,6 +73,19 @@ int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, void* qscal
                               int64_t N, int64_t K, int64_t group_size, int dtype, int32_t* nan_flag,
                               void* stream);
 
+/* y = x @ dequant(W) (+ bias) for many rows: the weight is dequantised into `scratch`, a slab of columns at a time
+ * (the reference's own structure for 256 tokens and more, nanoquantization/layers/gemm.py:558-561), and multiplied by a dense
+ * kernel of this library.  gated: W is gate and up interleaved word by word, y [M, N/2] = dtype(SiLU(gate)) * up,
+ * no bias.  awq_linear_dense_scratch_bytes: at most 256 MiB (a single tile of 256 columns where those are wider); 0 if the
+ * sizes are not this path's (K % 64, a group size of 8, 16, 32 or a multiple of 64).  The scratch needs no
+ * initialisation and is free again when the call's work on the stream is done.
+ * awq_linear_dense_wanted_bytes: the same where this is the faster way (rows in the hundreds and more), else 0. */
+size_t awq_linear_dense_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size);
+size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size);
+int awq_linear_dense(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
+                     const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
+                     int gated, void* scratch, size_t scratch_bytes, void* stream);
+
 /* Bytes of device workspace awq_gemv / awq_gemm / awq_linear need for this
  * problem (0 is possible).  The workspace must be zero-filled ONCE when it is
  * allocated; every call leaves it in that state (its counters are reset by

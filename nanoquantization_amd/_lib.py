@@ -34,6 +34,9 @@ SYMBOLS = {
     "awq_dequantize_transposed": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "awq_quantize_pack": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "awq_quantize_pack_flagged": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _vp]),
+    "awq_linear_dense_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "awq_linear_dense_wanted_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "awq_linear_dense": (_int, [_vp] * 6 + [_i64] * 4 + [_int, _int, _vp, _sz, _vp]),
     "awq_gemv_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "awq_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "awq_linear_workspace_bytes": (_sz, [_i64, _i64, _i64]),
@@ -251,6 +254,18 @@ def workspace_bytes(entry: str, M: int, N: int, K: int, extra: tuple = ()) -> in
         if len(_ws_bytes_cache) < 65536:
             _ws_bytes_cache[key] = n
     return n
+
+
+def dense_scratch(device: torch.device, M: int, N: int, K: int, group_size: int) -> torch.Tensor | None:
+    """Scratch for awq_linear_dense where that is the faster way, else None.  It comes from torch's caching allocator for this
+    one call (ordered on the current stream like any temporary); without room for it the fused kernels run."""
+    nbytes = lib().awq_linear_dense_wanted_bytes(M, N, K, group_size)
+    if not nbytes:
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 # One zero-initialised split-K workspace per (device, stream).  The kernels leave

@@ -437,7 +437,7 @@ extern "C" int awq_dequantize_transposed(const int32_t* qweight, const void* qsc
         return AWQ_ERR_UNSUPPORTED;
     }
     const hipError_t e = awq::launch_dequant_transpose(dtype, qweight, qscales, qzeros, out, (int)N, (int)K,
-                                                       (int)group_size, reinterpret_cast<hipStream_t>(stream));
+                                                       (int)group_size, reinterpret_cast<hipStream_t>(stream), 0, N);
     return e == hipSuccess ? AWQ_OK : awq::hip_fail(fn, e);
 }
 
@@ -506,6 +506,26 @@ extern "C" size_t awq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
         a = a > c ? a : c;
     }
     return a > b ? a : b;
+}
+
+// Whether dequantising the weight first (awq_linear_dense) is the faster way, from estimates of both: the fused 256 x 256
+// kernels take 1.9 us a K step and round of 256 workgroups, 10 us to fill and store a round's tiles, and 0.05 us per K slice
+// of a tile for its fp32 partials and their sum (within 15 % of every size measured between 256 and 8192 rows).  Measured,
+// bf16, fused / dequantised first: 4096 x 12288 at 512 rows 74 / 69 us, 2048 rows 224 / 186, 8192 rows 787 / 575; 12288 x
+// 4096 at 512 rows (32 tiles cut in eight) 71 / 136, 2048 rows 209 / 176, 8192 rows 744 / 568; 1024 x 2048 at 4096 rows
+// 43 / 28; 2560 x 9728 at 333 rows 45 / 44, 8192 rows 441 / 309.
+// Short K at up to 2048 rows stays fused: awq_gemm_plan's kernel and K split are what a caller gets there, bit for bit, and
+// the difference is a few microseconds (1024 x 4096 at 1024 rows 31 / 22 us).
+extern "C" size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size) {
+    if (M <= 128 || (M <= 2048 && K < 2048)) return 0;
+    const double dense = awq::dense_linear_us(M, N, K, group_size);
+    if (dense < 0) return 0;
+    int v, split;
+    awq::pick_gemm(M, N, K, &v, &split);
+    const awq::PipePlan p = awq::make_pipe_plan(M, N, K, split, awq::is_tail_variant(v));
+    const double full = (double)awq::cdiv(p.full_tiles, 256), cut = (double)awq::cdiv((int64_t)p.tail_tiles * p.splits, 256);
+    const double fused = full * (1.9 * (double)(K / 64) + 10) + cut * (1.9 * p.iters_per_split + 10) + 0.05 * p.tail_tiles * p.splits;
+    return dense < fused ? awq_linear_dense_scratch_bytes(M, N, K, group_size) : 0;
 }
 
 extern "C" size_t awq_linear_swiglu_workspace_bytes(int64_t M, int64_t N, int64_t K) {

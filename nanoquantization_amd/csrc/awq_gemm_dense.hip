@@ -1,0 +1,184 @@
+// Kernel (c) for many rows: the weight dequantised once into scratch memory, [columns][K] (the exact RN_dtype((q - z) s) that
+// every other path multiplies), then the dense product of pingpong.hpp.
+//
+// The fused kernels unpack a weight tile for every 256 rows of x, which costs the SIMD's issue port as much as a third of the
+// MFMAs do (awq_gemm_regb.hip); from about a thousand rows on, one pass that writes the weight out (2.5 bytes a weight, and
+// the product then finds it in the Infinity Cache) is the cheaper way.  Scratch is a slab of columns of at most 256 MiB (the
+// size of that cache), wider weights are taken slab by slab.
+#include <algorithm>
+
+#include "awq_gemm_parts.hpp"
+#include "pingpong.hpp"
+
+namespace awq {
+namespace {
+
+constexpr int64_t kSlabBytes = 256ll << 20;
+
+// GATED: the slab's columns are gate and up words in turn; a tile is 128 gate columns and their up columns, a wave's first
+// tiles gate, the others up.
+template <typename T, int XR, bool GATED>
+__global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wt,
+                                                       const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int M,
+                                                       int cols, int K, int ldy, int x_tiles, int w_tiles) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
+    using P = PingPong<T, XR>;
+    int xt, nt;
+    if (!xcd_tile(x_tiles, w_tiles, xt, nt)) return;
+    P p;
+    const int m0 = xt * XR, n0 = nt * (GATED ? 128 : 256), out_cols = GATED ? cols / 2 : cols;
+    const uint32_t row_bytes = (uint32_t)K * 2;
+    uint32_t vw[4], vx[P::kXLoads];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int r = p.w_row(q);
+        int col = n0 + r;
+        if (GATED) {
+            const int c = n0 + r / (2 * P::kHalf) * P::kHalf + r % P::kHalf;
+            col = 16 * (c >> 3) + (c & 7) + 8 * (r / P::kHalf & 1);
+        }
+        vw[q] = (uint32_t)col * row_bytes + p.piece_bytes(r);
+    }
+#pragma unroll
+    for (int q = 0; q < P::kXLoads; ++q) vx[q] = (uint32_t)p.x_row(q) * row_bytes + p.piece_bytes(p.x_row(q));
+    // rows past the end of either operand read zeros
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wt), 0, cols * row_bytes, 0x00020000);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (size_t)m0 * K, 0,
+                                                      min(XR, M - m0) * row_bytes, 0x00020000);
+    p.run(s_mem, rw, vw, rx, vx, K / P::kStage);
+    const auto store = [&](int r, int c, u32x4 v) {
+        if (m0 + r < M && n0 + c < out_cols) *reinterpret_cast<u32x4*>(y + (size_t)(m0 + r) * ldy + n0 + c) = v;
+    };
+    if constexpr (GATED) {
+        p.template write<128>(s_mem, [&](int i, int j) {
+            const f32x4 g4 = p.acc[i][j], u4 = p.acc[i + P::MI / 2][j];
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {       // dtype(SiLU(gate)) * up of the rounded products, as swiglu_pair_store
+                const float g = T::to_f32(T::from_f32(g4[e])), u = T::to_f32(T::from_f32(u4[e]));
+                o[e] = T::to_f32(T::from_f32(g / (1.f + __expf(-g)))) * u;
+            }
+            return u32x2{T::pack2(o[0], o[1]), T::pack2(o[2], o[3])};
+        }, store);
+    } else if (bias) {
+        p.template write<256>(s_mem, [&](int i, int j) {
+            const f32x4 v = p.acc[i][j];
+            const int c = min(n0 + p.wm * (256 / P::kWM) + 16 * i + 4 * p.hi, cols - 4);
+            const u32x2 b = *reinterpret_cast<const u32x2*>(bias + c);
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = add_bias<T>(v[e], T::to_f32((uint16_t)(b[e >> 1] >> (16 * (e & 1)))));
+            return u32x2{T::pack2(o[0], o[1]), T::pack2(o[2], o[3])};
+        }, store);
+    } else {
+        p.template write<256>(s_mem, [&](int i, int j) {
+            const f32x4 v = p.acc[i][j];
+            return u32x2{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
+        }, store);
+    }
+}
+
+// Columns of a slab: all, or equal parts of at most kSlabBytes, in whole tiles.
+int64_t slab_columns(int64_t N, int64_t K) {
+    const int64_t most = std::max<int64_t>(256, kSlabBytes / (2 * K) / 256 * 256);
+    return std::min(cdiv(cdiv(N, cdiv(N, most)), 256) * 256, cdiv(N, 256) * 256);
+}
+
+// Microseconds of the product over one slab: rounds of 256 workgroups, a stage of 1.42 us with 256-row tiles and 0.8 with
+// 128-row ones (measured with full rounds; 8192 x 4096 x 12288 six rounds of 64 stages 560 us, 512 x 4096 x 12288 one round
+// of the small tile 48 us), and filling and storing a tile.
+double product_us(int64_t M, int64_t slab, int64_t K, int xr) {
+    return (double)cdiv(cdiv(M, xr) * cdiv(slab, 256), 256) * ((double)(K / 64) * (xr == 256 ? 1.42 : 0.8) + (xr == 256 ? 5 : 4));
+}
+
+template <typename T, int XR, bool GATED>
+hipError_t launch(const void* x, const void* wt, const void* bias, void* y, int M, int cols, int K, int ldy, hipStream_t st) {
+    using P = PingPong<T, XR>;
+    auto kern = dense_kernel<T, XR, GATED>;
+    static bool raised = false;      // once per process and instantiation
+    if (!raised) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 P::kLds);
+        if (e != hipSuccess) return e;
+        raised = true;
+    }
+    const int x_tiles = (int)cdiv(M, XR), w_tiles = (int)cdiv(cols, 256);
+    (void)hipGetLastError();
+    kern<<<dim3((unsigned)(cdiv((int64_t)x_tiles * w_tiles, 8) * 8)), dim3(P::kThreads), P::kLds, st>>>(
+        (const uint16_t*)x, (const uint16_t*)wt, (const uint16_t*)bias, (uint16_t*)y, M, cols, K, ldy, x_tiles, w_tiles);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_dense(const void* x, const void* wt, const void* bias, void* y, int M, int cols, int K, int ldy, int xr,
+                        bool gated, hipStream_t st) {
+    if (xr == 256)
+        return gated ? launch<T, 256, true>(x, wt, bias, y, M, cols, K, ldy, st)
+                     : launch<T, 256, false>(x, wt, bias, y, M, cols, K, ldy, st);
+    return gated ? launch<T, 128, true>(x, wt, bias, y, M, cols, K, ldy, st)
+                 : launch<T, 128, false>(x, wt, bias, y, M, cols, K, ldy, st);
+}
+
+// Sizes and group sizes the path takes; 32-bit offsets inside a tile's rows of x and inside a slab.
+bool takes(int64_t M, int64_t N, int64_t K, int64_t g) {
+    return M >= 1 && N >= 8 && N % 8 == 0 && K >= 64 && K % 64 == 0 && g > 0 && K % g == 0 && (g % 64 == 0 || (64 % g == 0 && g % 8 == 0)) &&
+           K <= (1 << 20) && M < (1ll << 31) - 256 && N < (1ll << 31) - 256 && cdiv(M, 128) * cdiv(N, 256) < (1ll << 31) - 8;
+}
+
+}  // namespace
+
+double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g) {
+    if (!takes(M, N, K, g)) return -1;
+    const int64_t slab = slab_columns(N, K);
+    // the dequantise pass moves 2.5 bytes a weight at 6 TB/s (4096 x 12288 20.5 us, 5120 x 25600 62)
+    return 4 + 2.5 * (double)(K * N) / 6.0e6 +
+           (double)cdiv(N, slab) * std::min(product_us(M, slab, K, 128), product_us(M, slab, K, 256));
+}
+
+}  // namespace awq
+
+using namespace awq;
+
+extern "C" size_t awq_linear_dense_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size) {
+    return takes(M, N, K, group_size) ? (size_t)(std::min(slab_columns(N, K), N) * K * 2) : 0;
+}
+
+extern "C" int awq_linear_dense(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
+                                const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
+                                int gated, void* scratch, size_t scratch_bytes, void* stream) {
+    const char* fn = "awq_linear_dense";
+    PrefetchRegions dropped;            // hints of this thread were meant for this call; the product fills the chip
+    take_prefetch_hint(&dropped);
+    const int rc = check_linear_args(fn, x, qweight, qscales, qzeros, y, M, N, K, group_size, dtype);
+    if (rc != AWQ_OK) return rc;
+    if (!takes(M, N, K, group_size) || (gated && (bias || N % 16 != 0))) {
+        set_error("%s: needs K %% 64 == 0, a group size of 8, 16, 32 or a multiple of 64, and for a gated product N %% 16 == 0 "
+                  "and no bias (M=%lld N=%lld K=%lld g=%lld)", fn, (long long)M, (long long)N, (long long)K,
+                  (long long)group_size);
+        return AWQ_ERR_UNSUPPORTED;
+    }
+    if ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(scratch)) & 15u) {
+        set_error("%s: bias and scratch must be 16-byte aligned", fn);
+        return AWQ_ERR_INVALID_ARG;
+    }
+    if (!scratch || scratch_bytes < awq_linear_dense_scratch_bytes(M, N, K, group_size)) {
+        set_error("%s: scratch of %zu bytes needed, %zu given", fn, awq_linear_dense_scratch_bytes(M, N, K, group_size),
+                  scratch ? scratch_bytes : (size_t)0);
+        return AWQ_ERR_WORKSPACE;
+    }
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const int64_t slab = slab_columns(N, K);
+    const int xr = product_us(M, slab, K, 128) < product_us(M, slab, K, 256) ? 128 : 256;
+    for (int64_t n = 0; n < N; n += slab) {
+        const int64_t cols = std::min(slab, N - n);
+        hipError_t e = launch_dequant_transpose(dtype, qweight, qscales, qzeros, scratch, (int)N, (int)K, (int)group_size, st, n, cols);
+        const void* b = bias ? static_cast<const uint16_t*>(bias) + n : nullptr;
+        void* out = static_cast<uint16_t*>(y) + (gated ? n / 2 : n);
+        const int ldy = (int)(gated ? N / 2 : N);
+        if (e == hipSuccess)
+            e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated != 0, st)
+                                 : launch_dense<BF16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated != 0, st);
+        if (e != hipSuccess) return hip_fail(fn, e);
+    }
+    return AWQ_OK;
+}

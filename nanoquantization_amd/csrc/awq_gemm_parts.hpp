@@ -217,9 +217,12 @@ hipError_t launch_gemm_regb(int dtype, const void* x, const int32_t* qweight, co
                             const int32_t* qzeros, const void* bias, void* y, int M, int N, int K, int g,
                             void* workspace, int split_k, bool tail_only, hipStream_t stream, int act = 0);
 
-// awq_gemm_pipe.hip: wt [N][K] = the dequantised weight, transposed (K % 64 == 0, group size a multiple of 64 or
-// a divisor of 64 that is a multiple of 8).
+// awq_gemm_pipe.hip: wt [count][K] = columns first .. first + count - 1 of the dequantised weight, transposed (K % 64 == 0,
+// group size a multiple of 64 or a divisor of 64 that is a multiple of 8; first % 8 == 0).
 hipError_t launch_dequant_transpose(int dtype, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
-                                    void* wt, int N, int K, int g, hipStream_t stream);
+                                    void* wt, int N, int K, int g, hipStream_t stream, int64_t first, int64_t count);
+
+// awq_gemm_dense.hip: estimated microseconds of awq_linear_dense, -1 where it does not take the sizes.
+double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g);
 
 }  // namespace awq

@@ -355,12 +355,13 @@ template <typename T>
 __global__ __launch_bounds__(256) void dequant_transpose_kernel(const uint32_t* __restrict__ qweight,
                                                                 const uint16_t* __restrict__ scales,
                                                                 const uint32_t* __restrict__ qzeros,
-                                                                uint16_t* __restrict__ wt, int N, int K, int g) {
+                                                                uint16_t* __restrict__ wt, int N, int K, int g, int first,
+                                                                int count) {
     __shared__ u32x4 tile[256 * 8];   // [n][8 chunks of 8 k], chunk kc of row n at n*8 + (kc ^ ((n >> 3) & 7))
     const int tid = threadIdx.x, wc = tid & 31, rb = tid >> 5;
     const int words = N >> 3;
     const int k0 = blockIdx.y * 64, n0 = blockIdx.x * 256;
-    const int gwc = min((n0 >> 3) + wc, words - 1);
+    const int gwc = min(((first + n0) >> 3) + wc, words - 1);
     const int krow = k0 + rb * 8;
     uint32_t w[8];
 #pragma unroll
@@ -386,7 +387,7 @@ __global__ __launch_bounds__(256) void dequant_transpose_kernel(const uint32_t* 
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int n = j * 32 + (tid >> 3), kc = tid & 7;
-        if (n0 + n < N)
+        if (n0 + n < count)
             *reinterpret_cast<u32x4*>(wt + (size_t)(n0 + n) * K + k0 + kc * 8) = tile[n * 8 + (kc ^ ((n >> 3) & 7))];
     }
 }
@@ -497,17 +498,17 @@ hipError_t launch_gemm_pipe(int dtype, const void* x, const int32_t* qweight, co
 }
 
 hipError_t launch_dequant_transpose(int dtype, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
-                                    void* wt, int N, int K, int g, hipStream_t stream) {
+                                    void* wt, int N, int K, int g, hipStream_t stream, int64_t first, int64_t count) {
     (void)hipGetLastError();
-    const dim3 grid((N + 255) / 256, K / 64), block(256);
+    const dim3 grid((unsigned)cdiv(count, 256), K / 64), block(256);
     if (dtype == AWQ_F16)
         hipLaunchKernelGGL(dequant_transpose_kernel<F16>, grid, block, 0, stream,
                            reinterpret_cast<const uint32_t*>(qweight), reinterpret_cast<const uint16_t*>(qscales),
-                           reinterpret_cast<const uint32_t*>(qzeros), reinterpret_cast<uint16_t*>(wt), N, K, g);
+                           reinterpret_cast<const uint32_t*>(qzeros), reinterpret_cast<uint16_t*>(wt), N, K, g, (int)first, (int)count);
     else
         hipLaunchKernelGGL(dequant_transpose_kernel<BF16>, grid, block, 0, stream,
                            reinterpret_cast<const uint32_t*>(qweight), reinterpret_cast<const uint16_t*>(qscales),
-                           reinterpret_cast<const uint32_t*>(qzeros), reinterpret_cast<uint16_t*>(wt), N, K, g);
+                           reinterpret_cast<const uint32_t*>(qzeros), reinterpret_cast<uint16_t*>(wt), N, K, g, (int)first, (int)count);
     return hipGetLastError();
 }
 

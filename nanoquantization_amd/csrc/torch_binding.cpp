@@ -91,6 +91,18 @@ at::Tensor workspace(const at::Device& dev, void* stream, size_t nbytes) {
     return ws;
 }
 
+// Scratch for awq_linear_dense where that is the faster way, else undefined.  From the caching allocator for this one call
+// (ordered on the current stream like any temporary); without room for it the fused kernels run.
+at::Tensor dense_scratch(const at::Device& dev, int64_t M, const Packed& p) {
+    const size_t nbytes = M > 128 ? awq_linear_dense_wanted_bytes(M, p.N, p.K, p.g) : 0;
+    if (!nbytes) return {};
+    try {
+        return at::empty({(int64_t)nbytes}, at::TensorOptions().dtype(at::kByte).device(dev));
+    } catch (const c10::OutOfMemoryError&) {
+        return {};
+    }
+}
+
 at::Tensor awq_dequantize_op(const at::Tensor& qweight, const at::Tensor& qscales, const at::Tensor& qzeros) {
     const Packed p = check_packed(qweight, qscales, qzeros);
     check_device(qweight, {&qscales, &qzeros});
@@ -130,6 +142,13 @@ at::Tensor awq_linear_op(const at::Tensor& x, const at::Tensor& qweight, const a
     at::Tensor out = at::empty({M, p.N}, qs.options());
     if (M == 0) return out;
     hipStream_t stream = current_stream(x.device().index());
+    if (const at::Tensor scratch = dense_scratch(x.device(), M, p); scratch.defined()) {
+        check_status(awq_linear_dense(xc.data_ptr(), qw.data_ptr<int32_t>(), qs.data_ptr(), qz.data_ptr<int32_t>(),
+                                      b.defined() ? b.data_ptr() : nullptr, out.data_ptr(), M, p.N, p.K, p.g, p.dtype, 0,
+                                      scratch.data_ptr(), (size_t)scratch.numel(), stream),
+                     "awq_linear_dense");
+        return out;
+    }
     const size_t nbytes = awq_linear_workspace_bytes(M, p.N, p.K);
     at::Tensor ws;
     if (nbytes) ws = workspace(x.device(), stream, nbytes);
@@ -159,6 +178,13 @@ at::Tensor awq_linear_swiglu_op(const at::Tensor& x, const at::Tensor& qweight, 
     at::Tensor out = at::empty({M, p.N / 2}, qs.options());
     if (M == 0) return out;
     hipStream_t stream = current_stream(x.device().index());
+    if (const at::Tensor scratch = dense_scratch(x.device(), M, p); scratch.defined()) {
+        check_status(awq_linear_dense(xc.data_ptr(), qw.data_ptr<int32_t>(), qs.data_ptr(), qz.data_ptr<int32_t>(), nullptr,
+                                      out.data_ptr(), M, p.N, p.K, p.g, p.dtype, 1, scratch.data_ptr(),
+                                      (size_t)scratch.numel(), stream),
+                     "awq_linear_dense");
+        return out;
+    }
     const size_t nbytes = awq_linear_swiglu_workspace_bytes(M, p.N, p.K);
     at::Tensor ws;
     if (nbytes) ws = workspace(x.device(), stream, nbytes);

@@ -342,6 +342,12 @@ def awq_linear_swiglu(x: torch.Tensor, qweight: torch.Tensor, qscales: torch.Ten
     L = _lib.lib()
     with _lib.on_device(dev):
         stream = _stream(dev)
+        scratch = _lib.dense_scratch(dev, M, N, K, g) if M > 128 else None
+        if scratch is not None:
+            _lib.check(L.awq_linear_dense(x.data_ptr(), qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(), None,
+                                          out.data_ptr(), M, N, K, g, _lib.dtype_id(x.dtype), 1, scratch.data_ptr(),
+                                          scratch.numel(), stream))
+            return out
         nbytes = L.awq_linear_swiglu_workspace_bytes(M, N, K)
         ws = _lib.workspace(dev, stream, nbytes)
         _lib.check(L.awq_linear_swiglu(x.data_ptr(), qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(),

@@ -66,8 +66,8 @@ def awq_dequantize(
 
 def awq_dequantize_transposed(qweight: torch.Tensor, qscales: torch.Tensor, qzeros: torch.Tensor) -> torch.Tensor:
     """Packed int4 -> [N, K] weight (k-contiguous rows) in qscales.dtype: awq_dequantize(...).t(), bit for bit.
-    A free-standing utility (the layout dense GEMM libraries like best); the linear itself never materialises the
-    weight: every M runs the fused dequant + MFMA kernel."""
+    A free-standing utility (the layout dense products like best); the linear of many rows runs the same kernel into
+    scratch memory."""
     K, N, g = _check_packed(qweight, qscales, qzeros)
     dev = _require_device(qweight, qscales, qzeros)
     qweight, qscales, qzeros = qweight.contiguous(), qscales.contiguous(), qzeros.contiguous()
@@ -97,6 +97,12 @@ def _linear(entry: str, x, qweight, qscales, qzeros, bias, extra=()):
     L = _lib.lib()
     with _lib.on_device(dev):
         stream = _lib.current_stream_ptr(dev)
+        scratch = _lib.dense_scratch(dev, M, N, K, g) if entry == "awq_linear" and M > 128 else None
+        if scratch is not None:
+            _lib.check(L.awq_linear_dense(x.data_ptr(), qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(), _ptr(bias),
+                                          out.data_ptr(), M, N, K, g, _lib.dtype_id(dt), 0, scratch.data_ptr(),
+                                          scratch.numel(), stream))
+            return out
         nbytes = _lib.workspace_bytes(entry, M, N, K, tuple(extra))
         ws = _lib.workspace(dev, stream, nbytes) if nbytes else None
         status = getattr(L, entry)(x.data_ptr(), qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(), _ptr(bias),
@@ -254,8 +260,8 @@ class WQLinear_GEMM(nn.Module):
         return awq_linear
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        # One regime switch inside the library: split-K GEMV for <= 16 tokens, fused dequant + MFMA GEMM above; the
-        # bias is added in the kernel epilogue.  The output is a fresh tensor outside autograd, as under the
+        # The regimes are the library's: split-K GEMV for few tokens, fused dequant + MFMA GEMM above, the weight
+        # dequantised first where there are many; the bias is added in the kernel epilogue.  The output is a fresh tensor outside autograd, as under the
         # reference's @torch.no_grad (layers/gemm.py:552); buffers are fetched from the module's dictionary directly
         # (nn.Module.__getattr__ costs more than the rest of this function).
         buf = self._buffers

@@ -277,6 +277,75 @@ def test_gemm_largest_shapes_properties(M, K, N):
     assert ((sub - ref).abs().max() / ref.abs().max()).item() <= TIGHT["bf16"]
 
 
+# one and several tiles of 256 and of 128 rows, rows and columns past the last tile, one, two and three stages of K (the
+# buffers in flight at the start), every group size form, a weight of two slabs (131072 x 1032: 270 MB)
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,K,N,g", [(1, 64, 8, 64), (129, 128, 264, 32), (300, 192, 520, 64), (256, 256, 256, 128),
+                                      (4352, 320, 4104, 64), (700, 1024, 1032, 1024), (40, 131072, 1032, 128)])
+def test_linear_dense(dtype, M, K, N, g):
+    """The weight dequantised first, with bias and with the gated epilogue, against the fp64 product of the dequantised
+    weight and against the separate activation kernel; rows of zeros stay zero, two runs give the same bits."""
+    from nanoquantization_amd.engine import ops
+    print(f"linear dense {dtype} M={M} K={K} N={N} g={g}", flush=True)
+    tdt = torch.float16 if dtype == "f16" else torch.bfloat16
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    qw = torch.randint(-2 ** 31, 2 ** 31 - 1, (K, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    qz = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // g, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    qs = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 + 0.001).to(tdt)
+    x = torch.randn(M, K, device="cuda", generator=gen).to(tdt)
+    bias = torch.randn(N, device="cuda", generator=gen).to(tdt)
+    if M > 1:
+        x[M // 2] = 0
+    L = _lib.lib()
+    scratch = torch.full((L.awq_linear_dense_scratch_bytes(M, N, K, g),), 0xFF, dtype=torch.uint8, device="cuda")   # NaN
+
+    def dense(b, gated):
+        y = torch.empty(M, N // 2 if gated else N, dtype=tdt, device="cuda")
+        _lib.check(L.awq_linear_dense(x.data_ptr(), qw.data_ptr(), qs.data_ptr(), qz.data_ptr(),
+                                      None if b is None else b.data_ptr(), y.data_ptr(), M, N, K, g, _lib.dtype_id(tdt),
+                                      int(gated), scratch.data_ptr(), scratch.numel(), _lib.current_stream_ptr(y.device)))
+        return y
+    y, yb = dense(None, False), dense(bias, False)
+    ref = x.double() @ nq.awq_dequantize(qw, qs, qz).double()
+    top = ref.abs().max().item()
+    assert (y.double() - ref).abs().max().item() <= TIGHT[dtype] * top
+    assert (yb.double() - ref - bias.double()).abs().max().item() <= (TIGHT[dtype] + BIAS_STEP[dtype]) * (top + 4)
+    assert torch.equal(y, dense(None, False))
+    assert M == 1 or torch.count_nonzero(y[M // 2]) == 0
+    if N % 16 == 0:
+        assert torch.equal(dense(None, True), ops.silu_mul(y, interleaved=True))
+
+
+def test_linear_dense_routes():
+    """The default linear takes the dense path where its estimate is the lower one, with the bits of the forced call, also
+    under graph capture; the fused kernels keep short prompts, short K at up to 2048 rows and what the path refuses."""
+    L = _lib.lib()
+    wanted = L.awq_linear_dense_wanted_bytes
+    assert wanted(8192, 12288, 4096, 128) == 2 * 12288 * 4096 and wanted(2048, 4096, 12288, 128) > 0
+    assert wanted(128, 12288, 4096, 128) == 0 and wanted(512, 4096, 12288, 128) == 0
+    assert wanted(2048, 4096, 1024, 128) == 0 and wanted(8192, 4096, 4096 + 32, 32) == 0
+    assert wanted(8192, 51200, 5120, 128) <= 256 << 20
+    M, K, N = 2100, 2048, 2056
+    p = random_packed(K, N, 128, "bf16", seed=7)
+    dev = [to_dev(p["qweight"]), to_dev(p["qscales"], "bf16"), to_dev(p["qzeros"])]
+    assert wanted(M, N, K, 128) > 0
+    x = to_dev(make_x(M, K, "bf16", seed=8), "bf16")
+    want = nq.awq_gemm(x, *dev, 8)
+    s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        assert torch.equal(nq.awq_gemm(x, *dev, 8), want)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            y = nq.awq_gemm(x, *dev, 8)
+    torch.cuda.synchronize()
+    for rep in range(3):
+        y.zero_()
+        graph.replay()
+        other = nq.awq_gemm(x * 2, *dev, 8)         # eager work with scratch of its own between the replays
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(other, nq.awq_gemm(x * 2, *dev, 8)), rep
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("M,K,N,g", [(48, 288, 512, 32), (200, 224, 384, 32), (65, 544, 1280, 32), (32, 32, 256, 32)])
 def test_linear_k_not_a_multiple_of_64(dtype, M, K, N, g):
