@@ -3,9 +3,11 @@
 // The grouped products exist in three forms, chosen by pairs per expert and operand alignment (moe_form):
 //   few pairs    tiles of 16, 32 or 64 pairs on the skinny core: the weights stream once, straight into MFMA operands
 //   many pairs   tiles of 64 or 128 pairs x 128 weight rows staged through LDS by load-to-LDS, double-buffered, MFMA 16x16x32
+//   most pairs   tiles of 128 or 256 pairs x 256 weight rows on the product core of pingpong.hpp (rows in whole stages of 64)
 //   any sizes    32 x 32 tiles in fp32 on the vector ALU (fp32 operands, rows that are not multiples of 8)
 #include <algorithm>
 
+#include "../pingpong.hpp"
 #include "moe_route.hpp"
 #include "skinny.hpp"
 
@@ -334,20 +336,107 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const uint16_t* __restric
     }
 }
 
-enum class MoeForm { simple, skinny16, skinny32, skinny64, gemm64, gemm128 };
+// ---- most pairs per expert: XR = 128 or 256 pairs x 256 weight rows per workgroup -------------------------------
+// A gathered row is one 32-bit offset per lane and load, so the gather costs nothing in the loop.  GATED: 128 gate rows and
+// their 128 up rows; a wave's first tiles are gate, the others the up rows of the same columns.  The same sums in the same
+// order as moe_gemm_kernel.  16,384 pairs of 8 experts, 4096 -> 2 x 6144 and back: 2805 us
+// with moe_gemm_kernel, 2007 like this.
+template <bool GATED, int XR>
+__global__ __launch_bounds__(512, 2) void moe_pingpong_kernel(const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
+                                                              const float* __restrict__ weight,
+                                                              const int32_t* __restrict__ order,
+                                                              const int32_t* __restrict__ tiles, uint16_t* __restrict__ out,
+                                                              int max_tiles, int top, int n_out, int n_in, int n_groups,
+                                                              uint32_t in_bytes) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char s_stage[];
+    using P = awq::PingPong<Bf, XR>;
+    constexpr int kCols = GATED ? 128 : 256;
+    int tile, group;
+    if (!awq::xcd_tile(tiles[3 * max_tiles], n_groups, tile, group)) return;
+    const int e = tiles[tile], first = tiles[max_tiles + tile], count = tiles[2 * max_tiles + tile];
+    const int n0 = group * kCols;
+    const uint32_t row_bytes = (uint32_t)n_in * 2, w_bytes = (GATED ? 2 : 1) * (uint32_t)n_out * row_bytes;
+    P p;
+    uint32_t vw[4], vx[P::kXLoads];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int r = p.w_row(q);
+        int row = n0 + r;
+        if (GATED) row = min(n0 + r / (2 * P::kHalf) * P::kHalf + r % P::kHalf, n_out - 1) + (r / P::kHalf & 1) * n_out;
+        vw[q] = (uint32_t)row * row_bytes + p.piece_bytes(r);
+    }
+#pragma unroll
+    for (int q = 0; q < P::kXLoads; ++q) {
+        const int r = p.x_row(q), place = first + min(r, count - 1);
+        vx[q] = (uint32_t)(GATED ? order[place] / top : place) * row_bytes + p.piece_bytes(r);
+    }
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w) + (int64_t)e * (GATED ? 2 : 1) * n_out * n_in, 0,
+                                                      w_bytes, 0x00020000);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(in), 0, in_bytes, 0x00020000);
+    p.run(s_stage, rw, vw, rx, vx, n_in / P::kStage);
+    if constexpr (GATED) {
+        float score[P::NJ];
+#pragma unroll
+        for (int j = 0; j < P::NJ; ++j) score[j] = weight[order[first + min(p.wn * (XR / P::kWN) + 16 * j + p.lo, count - 1)]];
+        p.template write<kCols>(s_stage, [&](int i, int j) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = silu_f32(score[j] * p.acc[i][j][r]) * (score[j] * p.acc[i + P::MI / 2][j][r]);
+            return u32x2{Bf::pack2(v[0], v[1]), Bf::pack2(v[2], v[3])};
+        }, [&](int r, int c, u32x4 v) {
+            if (r < count && n0 + c < n_out) *reinterpret_cast<u32x4*>(out + (int64_t)(first + r) * n_out + n0 + c) = v;
+        });
+    } else {
+        p.template write<kCols>(s_stage, [&](int i, int j) {
+            const f32x4 v = p.acc[i][j];
+            return u32x2{Bf::pack2(v[0], v[1]), Bf::pack2(v[2], v[3])};
+        }, [&](int r, int c, u32x4 v) {
+            if (r < count && n0 + c < n_out) *reinterpret_cast<u32x4*>(out + (int64_t)order[first + r] * n_out + n0 + c) = v;
+        });
+    }
+}
+
+template <bool GATED, int XR>
+void launch_pingpong(const uint16_t* in, const uint16_t* w, const float* weight, const int32_t* order, const int32_t* tiles,
+                     uint16_t* out, int64_t in_rows, int max_tiles, int top, int n_out, int n_in, hipStream_t st) {
+    using P = awq::PingPong<Bf, XR>;
+    auto kern = moe_pingpong_kernel<GATED, XR>;
+    static bool raised = false;          // once per process and instantiation
+    if (!raised) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, P::kLds) != hipSuccess)
+            return;                      // launched() reports it
+        raised = true;
+    }
+    const int64_t groups = cdiv(n_out, GATED ? 128 : 256);
+    kern<<<dim3((unsigned)(cdiv(max_tiles * groups, 8) * 8)), dim3(P::kThreads), P::kLds, st>>>(
+        in, w, weight, order, tiles, out, max_tiles, top, n_out, n_in, (int)groups, (uint32_t)(in_rows * n_in * 2));
+}
+
+enum class MoeForm { simple, skinny16, skinny32, skinny64, gemm64, gemm128, pingpong128, pingpong256 };
 MoeForm moe_form(int64_t pairs, int64_t experts, int64_t width, int64_t ff, int dtype) {
     if (dtype != NQH_BF16 || width % 8 != 0 || ff % 8 != 0) return MoeForm::simple;
     // by pairs per expert, so that one tile usually holds all pairs of an expert while there are few
     if (pairs <= 6 * experts || pairs <= 16) return MoeForm::skinny16;
     if (pairs <= 16 * experts || pairs <= 32) return MoeForm::skinny32;
     if (pairs <= 40 * experts || pairs <= 64) return MoeForm::skinny64;
+    // The ping-pong core wants whole stages and 32-bit offsets into the rows and into an expert's weights, pairs per expert that
+    // fill its tiles, and 128 workgroups in the smaller of the two products.  Both products, gemm / 128 / 256 pairs a tile:
+    // 4096 -> 2 x 6144, 8 experts, 192 pairs each 535 / 472 / 501 us, 512 each 898 / 793 / 743, 2048 each 2805 / - / 2007;
+    // 2048 -> 2 x 1024, 64 experts, 144 each 311 / 319 / 385, 192 each 363 / 335 / 416, 384 each 530 / 488 / 447;
+    // 1024 -> 2 x 1536, 8 experts, 256 each 50 / 61 / 65 (80 workgroups), 512 each 72 / 65 / 93, 1024 each 122 / - / 101.
+    const bool stages = width % 64 == 0 && ff % 64 == 0 && pairs * std::max(width, ff) * 2 < (1ll << 32) &&
+                        width * ff * 4 < (1ll << 32);
+    const int64_t groups = std::min(cdiv(width, 256), cdiv(ff, 128));
+    if (stages && pairs > 320 * experts && pairs * groups >= 128 * 256) return MoeForm::pingpong256;
+    if (stages && pairs > 160 * experts && pairs * groups >= 128 * 128) return MoeForm::pingpong128;
     return pairs <= 256 * experts ? MoeForm::gemm64 : MoeForm::gemm128;
 }
 int moe_form_rows(MoeForm f) {
     switch (f) {
         case MoeForm::skinny16: return 16;
         case MoeForm::skinny64: case MoeForm::gemm64: return 64;
-        case MoeForm::gemm128: return 128;
+        case MoeForm::gemm128: case MoeForm::pingpong128: return 128;
+        case MoeForm::pingpong256: return 256;
         default: return 32;
     }
 }
@@ -436,6 +525,16 @@ static bool launch_fast(const void* in, const void* w, const float* weight, cons
         const dim3 grid((unsigned)(cdiv(max_tiles, 8) * 8 * groups));
         if (form == MoeForm::gemm64) moe_gemm_kernel<GATED, 64><<<grid, dim3(256), 0, st>>>(NQH_ARGS, (int)groups);
         else moe_gemm_kernel<GATED, 128><<<grid, dim3(256), 0, st>>>(NQH_ARGS, (int)groups);
+        return true;
+    }
+    if (form == MoeForm::pingpong128 || form == MoeForm::pingpong256) {
+        const int64_t in_rows = GATED ? pairs / top : pairs;
+        if (form == MoeForm::pingpong128)
+            launch_pingpong<GATED, 128>((const uint16_t*)in, (const uint16_t*)w, weight, order, tiles, (uint16_t*)out, in_rows,
+                                        (int)max_tiles, (int)top, (int)n_out, (int)n_in, st);
+        else
+            launch_pingpong<GATED, 256>((const uint16_t*)in, (const uint16_t*)w, weight, order, tiles, (uint16_t*)out, in_rows,
+                                        (int)max_tiles, (int)top, (int)n_out, (int)n_in, st);
         return true;
     }
     const int64_t groups = cdiv(n_out, 16);

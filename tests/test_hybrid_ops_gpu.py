@@ -353,6 +353,35 @@ def test_router_and_experts(dtype, rows, width, experts, top, ff):
     close(y, want, dtype, "experts")
 
 
+# the two tile sizes of the product core, output widths past the last tile, one stage of contraction and an odd number of them
+@pytest.mark.parametrize("rows,width,experts,top,ff,tile", [(1200, 1600, 8, 2, 832, 128), (2500, 1600, 6, 2, 832, 256),
+                                                            (17000, 64, 8, 2, 192, 256), (17000, 192, 60, 1, 64, 128)])
+def test_experts_with_many_pairs(rows, width, experts, top, ff, tile):
+    """An expert without pairs, one with a single pair, one with exactly a tile, the others unequal."""
+    print(f"moe rows={rows} width={width} experts={experts} top={top} ff={ff}", flush=True)
+    bf = torch.bfloat16
+    h = rand(rows, width, seed=1, dtype=bf).cuda()
+    gu = rand(experts, 2 * ff, width, seed=3, dtype=bf, scale=width ** -0.5).cuda()
+    dn = rand(experts, width, ff, seed=4, dtype=bf, scale=ff ** -0.5).cuda()
+    r = ops.Routing(rows, experts, top, width, ff, 1, h.device)
+    assert r.tile_rows == tile
+    pairs = rows * top
+    e = 3 + (torch.rand(pairs, generator=torch.Generator().manual_seed(5)) ** 2 * (experts - 3)).int()
+    e[7], e[tile:2 * tile] = 1, 2
+    r.expert.copy_(e.view(rows, top))
+    r.weight.copy_(torch.rand(rows, top, generator=torch.Generator().manual_seed(6)))
+    r.order, r.tiles = ops.moe_plan(r.expert, experts, r.tile_rows)
+    y = ops.moe_experts(h, gu, dn, r)
+    u = h.double().unsqueeze(1) * r.weight.double().unsqueeze(-1)
+    want = torch.empty(rows, top, width, dtype=torch.float64, device="cuda")
+    for x in range(experts):
+        at = (r.expert == x).nonzero(as_tuple=True)
+        a, b = u[at] @ gu[x, :ff].double().T, u[at] @ gu[x, ff:].double().T
+        want[at] = (a * torch.sigmoid(a) * b) @ dn[x].double().T
+    close(y, want.cpu(), bf, "experts")
+    assert torch.equal(y, ops.moe_experts(h, gu, dn, r))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,width,experts,top,ff", [(1, 72, 5, 2, 48), (16, 2048, 8, 2, 64), (64, 256, 64, 6, 128),
                                                       (200, 1028, 128, 8, 32), (33, 4096, 3, 3, 24), (300, 64, 8, 2, 32)])
