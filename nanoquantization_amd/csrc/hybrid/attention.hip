@@ -7,6 +7,7 @@
 //   latent_decode_kernel decode of latent attention in bf16: one cache row is key and value of all heads
 //   attn_rows_kernel     any sizes, both element types: one wave per (query token, head), arithmetic on the vector ALU
 #include <algorithm>
+#include <type_traits>
 
 #include "hybrid_common.hpp"
 
@@ -188,11 +189,34 @@ struct DenseKV {
 
 __device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Prompt attention.  Four waves of 32 queries; tiles of KT keys, double-buffered; every wave skips the tiles none of its
-// queries sees.  Cache rows are addressed key by key, so a tile may start anywhere and straddle cache blocks.  R, RV: key and
-// value elements of a row in LDS.
+constexpr float kSlack = 8.f;
+
+// Maximum over the four lanes that share a column: lanes l, l ^ 16, l ^ 32, l ^ 48.
+__device__ __forceinline__ float across_hi(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+    x = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+    return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
+}
+
+// Prompt attention.  Four waves of 32 queries; tiles of KT keys; every wave skips the tiles none of its queries sees.  Cache
+// rows are addressed key by key, so a tile may start anywhere and straddle cache blocks.  R, RV: key and value elements of a
+// row in LDS.
+//
+// A wave multiplies the keys of tile t + 1 while it takes the exponentials of tile t, whose scores it has from the iteration
+// before: the two have nothing to do with each other, so matrix cores and vector ALU work side by side within a wave and not
+// only across the two waves of a SIMD.  Keys are therefore staged a tile ahead of the values.  The running maximum is only
+// moved (and sums and outputs rescaled) when a score exceeds it by a factor of 2^kSlack: probabilities are then at most 2^kSlack
+// instead of 1, with the same relative precision.
+// What bounds it: per wave and tile of 64 x 128 64 MFMAs (1024 cycles) and some 250 vector instructions, 32 of them 2^x at a
+// quarter of the rate; two waves a SIMD, which is why rows of up to 128 keep within 256 registers (the form before, one wave
+// a SIMD, had 294).  Operands are read a step before they are multiplied; steps are fenced, or the scheduler asks for all of
+// them first and spills.  Bases of the lane's source rows are kept once, not per load, for the same reason.  Head sizes of
+// 128, causal, forms before / now: 32 heads 4 x 2048 tokens 376 / 187 us, 1 x 8192 1218 / 635 (866 TFLOP/s); 16 heads
+// 16 x 512 70 / 45, 1 x 512 24 / 18.  Rows of 32: 89 / 68, 64: 116 / 87, 96: 230 / 104, 192: 400 / 323, 256: 533 / 417 (4 x
+// 2048, 16 heads); expanded latents of 192 / 128: 450 / 268 with tiles of 32 keys, two waves a SIMD (64 keys, one: 424).
 template <int R, int RV, int KT, bool DENSE>
-__global__ __launch_bounds__(256) void attn_tile_kernel(
+__global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
     const uint16_t* __restrict__ sink, DenseKV dense, uint16_t* __restrict__ out, int heads, int kv_heads, int vdim,
@@ -203,8 +227,8 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(
     constexpr int vBytes = KT * RV * 2, vLoads = KT * LV::kPieces / 256, kBuffer = kBytes + vBytes;
     static_assert(KT % 32 == 0 && KT * L::kPieces % 256 == 0 && KT * LV::kPieces % 256 == 0, "whole load-to-LDS instructions");
     // one array: with several the compiler waits for every load-to-LDS in flight before any LDS read
-    __shared__ __attribute__((aligned(1024))) unsigned char s_mem[2 * kBuffer + (DENSE ? 0 : 2 * KT * 4)];   // [buffer][K | V], rows
-    int* s_row = reinterpret_cast<int*>(s_mem + 2 * kBuffer);                                   // [buffer][KT]
+    __shared__ __attribute__((aligned(1024))) unsigned char s_mem[2 * kBuffer + (DENSE ? 0 : 4 * KT * 4)];   // [buffer][K | V], rows
+    int* s_row = reinterpret_cast<int*>(s_mem + 2 * kBuffer);                                   // [tile % 4][KT]
     // contiguous runs of (kv head, query tile, head of the group) per XCD: a kv head's cache is read through one L2
     const int per = gridDim.x >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (id >= q_tiles * heads) return;
@@ -226,6 +250,9 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(
     const bool wave_live = wq0 <= q_last;
     const int w_first = start + min(wq0, q_last), w_last = start + min(wq0 + 31, q_last);
     const int see_lo = visible_from(w_first), full_lo = visible_from(w_last);
+    // scores stay unscaled up to the exponential, so a negative scale changes the queries' signs instead
+    const uint32_t flip = scale < 0.f ? 0x80008000u : 0u;
+    const float sc = fmaxf(fabsf(scale), 1e-30f) * kLog2e;
     int pos[2], low[2];                                              // per column: query position, first visible key
     u32x4 bq[2][R / 32];
 #pragma unroll
@@ -235,151 +262,272 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(
         low[c] = visible_from(pos[c]);
         const uint16_t* p = q + ((int64_t)row * heads + h) * R + 8 * hi;
 #pragma unroll
-        for (int s = 0; s < R / 32; ++s) bq[c][s] = *reinterpret_cast<const u32x4*>(p + 32 * s);
+        for (int s = 0; s < R / 32; ++s) bq[c][s] = *reinterpret_cast<const u32x4*>(p + 32 * s) ^ flip;
     }
-    // cache rows of a tile's keys (past the end those of the last visible key): the block number is fetched ahead of the
-    // tile's other loads and turned into a row once they are under way
-    const int key = (int)threadIdx.x % KT;
-    int next_block = 0;
-    auto fetch_block = [&](int t0) {
-        if constexpr (!DENSE) next_block = block_table[min(t0 + key, k_end - 1) / block_size];
-    };
-    auto put_row = [&](int t0, int buf) {
+    const int n_tiles = (k_end - k_begin + KT - 1) / KT;
+    // cache rows of a tile's keys (past the end those of the last visible key), by one wave of the four in turn: the block
+    // number is fetched a tile before it is turned into a row, which is a tile before the row is needed.  A division per key
+    // would cost a wave more than its exponentials do; block sizes are powers of two but for odd configurations.
+    const int block_shift = (block_size & (block_size - 1)) == 0 ? 31 - __builtin_clz(block_size) : -1;
+    int next_block = 0, next_in_block = 0;
+    auto fetch_block = [&](int t) {
         if constexpr (DENSE) return;
+        if (wave != (t & 3)) return;
+        const int j = min(k_begin + t * KT + lane % KT, k_end - 1);
+        const int b = block_shift >= 0 ? j >> block_shift : j / block_size;
+        next_in_block = block_shift >= 0 ? j & (block_size - 1) : j - b * block_size;
+        next_block = block_table[b];
+    };
+    auto put_row = [&](int t) {
+        if constexpr (DENSE) return;
+        if (wave != (t & 3)) return;
         const int blk = next_block < 0 ? 0 : (next_block >= num_blocks ? num_blocks - 1 : next_block);
-        if (threadIdx.x < KT) s_row[buf * KT + key] = (blk * kv_heads + g) * block_size + min(t0 + key, k_end - 1) % block_size;
+        s_row[(t & 3) * KT + lane % KT] = (blk * kv_heads + g) * block_size + next_in_block;
     };
     const int64_t dense_first = DENSE ? dense.first[seg] : 0;
     const uint16_t* dense_k = dense.kv + (int64_t)h * dense.dim;
     const uint16_t* dense_v = dense.kv + dense.v_at + (int64_t)h * vdim;
-    auto stage_dense = [&](int t0, int buf) {
+    static_assert(DENSE || R == RV, "cache rows of keys and values are equally wide");
+    // the lane's row and element in load 0; those of load i are kRowsPerLoad rows further and, where the rotation of the rows
+    // comes round by then, the same element of them
+    constexpr int kRowsPerLoad = 256 / L::kPieces, vRowsPerLoad = 256 / LV::kPieces;
+    constexpr bool kSame = 256 % L::kPieces == 0 && kRowsPerLoad % (L::kTurn * L::kPieces) == 0;
+    constexpr bool vSame = 256 % LV::kPieces == 0 && vRowsPerLoad % (LV::kTurn * LV::kWindows) == 0;
+    const int n0 = wave * 64 + lane;
+    const int k_row0 = n0 / L::kPieces, k_e0 = L::k_source(k_row0, n0 % L::kPieces);
+    const int v_row0 = n0 / LV::kPieces, v_e0 = LV::v_source(v_row0, n0 % LV::kPieces);
+    // keys (values) of tile t into buffer buf = t % 2, which is a constant everywhere: LDS places of operands are then too
+    auto stage_keys = [&](int t, int buf) {
         unsigned char* base = s_mem + buf * kBuffer;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            const int n = (i * 4 + wave) * 64 + lane, row = n / L::kPieces, e = L::k_source(row, n % L::kPieces);
-            const int64_t at = dense_first + min(t0 + row, k_end - 1);
-            const uint16_t* src = e < dense.dim ? dense_k + at * dense.kv_stride + e
-                                  : e < dense.dim + dense.rot_dim ? dense.rot + at * dense.rot_stride + (e - dense.dim)
-                                                                  : (const uint16_t*)&g_zero_piece;
+            const int n = i * 256 + n0, row = kSame ? k_row0 + i * kRowsPerLoad : n / L::kPieces;
+            const int e = kSame ? k_e0 : L::k_source(row, n % L::kPieces);
+            const uint16_t* src;
+            if constexpr (DENSE) {
+                const int64_t at = dense_first + min(k_begin + t * KT + row, k_end - 1);
+                src = e < dense.dim ? dense_k + at * dense.kv_stride + e
+                      : e < dense.dim + dense.rot_dim ? dense.rot + at * dense.rot_stride + (e - dense.dim)
+                                                      : (const uint16_t*)&g_zero_piece;
+            } else {
+                src = k_cache + (int64_t)s_row[(t & 3) * KT + row] * R + e;
+            }
             __builtin_amdgcn_global_load_lds(NQH_GPTR(src), NQH_LPTR(base + (i * 4 + wave) * 1024), 16, 0, 0);
         }
+    };
+    auto stage_values = [&](int t, int buf) {
+        unsigned char* base = s_mem + buf * kBuffer + kBytes;
 #pragma unroll
         for (int i = 0; i < vLoads; ++i) {
-            const int n = (i * 4 + wave) * 64 + lane, row = n / LV::kPieces, e = LV::v_source(row, n % LV::kPieces);
-            const int64_t at = dense_first + min(t0 + row, k_end - 1);
-            const uint16_t* src = e < vdim ? dense_v + at * dense.kv_stride + e : (const uint16_t*)&g_zero_piece;
-            __builtin_amdgcn_global_load_lds(NQH_GPTR(src), NQH_LPTR(base + kBytes + (i * 4 + wave) * 1024), 16, 0, 0);
+            const int n = i * 256 + n0, row = vSame ? v_row0 + i * vRowsPerLoad : n / LV::kPieces;
+            const int e = vSame ? v_e0 : LV::v_source(row, n % LV::kPieces);
+            const uint16_t* src;
+            if constexpr (DENSE) {
+                const int64_t at = dense_first + min(k_begin + t * KT + row, k_end - 1);
+                src = e < vdim ? dense_v + at * dense.kv_stride + e : (const uint16_t*)&g_zero_piece;
+            } else {
+                src = v_cache + (int64_t)s_row[(t & 3) * KT + row] * R + e;
+            }
+            __builtin_amdgcn_global_load_lds(NQH_GPTR(src), NQH_LPTR(base + (i * 4 + wave) * 1024), 16, 0, 0);
         }
     };
-    auto stage = [&](int t0, int buf) {
-        if constexpr (DENSE) {
-            stage_dense(t0, buf);
-            return;
-        }
-        static_assert(DENSE || R == RV, "cache rows of keys and values are equally wide");
-        unsigned char* base = s_mem + buf * kBuffer;
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int n = (i * 4 + wave) * 64 + lane, row = n / L::kPieces, p = n % L::kPieces;
-            const int64_t at = (int64_t)s_row[buf * KT + row] * R;
-            __builtin_amdgcn_global_load_lds(NQH_GPTR(k_cache + at + L::k_source(row, p)),
-                                             NQH_LPTR(base + (i * 4 + wave) * 1024), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(NQH_GPTR(v_cache + at + L::v_source(row, p)),
-                                             NQH_LPTR(base + kBytes + (i * 4 + wave) * 1024), 16, 0, 0);
-        }
-    };
-    const float sc = scale * kLog2e;
     // a sink is where the running softmax starts; a column's sum is spread over four lanes, one of which counts it
-    const float m0 = sink ? Bf::to_f32(sink[h]) * kLog2e : kNegBig, l0 = sink && hi == 0 ? 1.f : 0.f;
+    const float m0 = sink ? fmaxf(Bf::to_f32(sink[h]) * kLog2e, kNegBig) : kNegBig, l0 = sink && hi == 0 ? 1.f : 0.f;
     float m[2] = {m0, m0}, l[2] = {l0, l0};
     f32x4 acc[2][RV / 16];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int w = 0; w < RV / 16; ++w) acc[c][w] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    fetch_block(k_begin);
-    put_row(k_begin, 0);
-    fetch_block(k_begin + KT);
-    __syncthreads();
-    stage(k_begin, 0);
-    put_row(k_begin + KT, 1);
-    int buf = 0;
-    for (int t0 = k_begin; t0 < k_end; t0 += KT) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's part of the tile has landed
-        __syncthreads();
-        const bool more = t0 + KT < k_end;
-        if (more) {
-            fetch_block(t0 + 2 * KT);
-            stage(t0 + KT, buf ^ 1);
+    using Scores = f32x4[2][KT / 16];
+    using Probs = u32x4[2][KT / 32];
+    auto active = [&](int t) {
+        const int t0 = k_begin + t * KT;
+        return wave_live && t < n_tiles && t0 <= w_last && t0 + KT > see_lo;
+    };
+    // operands of the 16 keys from 16 a on of a tile, and their scores
+    using KeyOps = u32x4[R / 32];
+    auto load_keys = [&](int buf, int a, KeyOps& ka) {
+        const unsigned char* k_tile = s_mem + buf * kBuffer;
+#pragma unroll
+        for (int s = 0; s < R / 32; ++s) ka[s] = *reinterpret_cast<const u32x4*>(k_tile + L::k_at(16 * a + lo, 4 * s + hi));
+    };
+    auto score = [&](int a, const KeyOps& ka, Scores& st) {
+        st[0][a] = st[1][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < R / 32; ++s) {
+            st[0][a] = Bf::mfma16(ka[s], bq[0][s], st[0][a]);
+            st[1][a] = Bf::mfma16(ka[s], bq[1][s], st[1][a]);
         }
-        const unsigned char *k_tile = s_mem + buf * kBuffer, *v_tile = k_tile + kBytes;
-        if (wave_live && t0 <= w_last && t0 + KT > see_lo) {
-            const bool masked = t0 + KT - 1 > w_first || t0 < full_lo;
-            f32x4 st[2][KT / 16];
+    };
+    // the mask, and the maximum where it has to move
+    auto settle = [&](int t, Scores& st) {
+        const int t0 = k_begin + t * KT;
+        if (t0 + KT - 1 > w_first || t0 < full_lo) {
 #pragma unroll
-            for (int a = 0; a < KT / 16; ++a) {
-                st[0][a] = st[1][a] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int s = 0; s < R / 32; ++s) {
-                    const u32x4 ka = *reinterpret_cast<const u32x4*>(k_tile + L::k_at(16 * a + lo, 4 * s + hi));
-                    st[0][a] = Bf::mfma16(ka, bq[0][s], st[0][a]);
-                    st[1][a] = Bf::mfma16(ka, bq[1][s], st[1][a]);
-                }
-            }
-            u32x4 pb[2][KT / 32];
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                float mx = kNegBig;
+            for (int c = 0; c < 2; ++c)
 #pragma unroll
                 for (int a = 0; a < KT / 16; ++a)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        float s = st[c][a][r] * sc;
-                        if (masked) {
-                            const int j = t0 + 16 * a + 4 * hi + r;
-                            s = (j <= pos[c] && j >= low[c]) ? s : -__builtin_inff();
-                        }
-                        st[c][a][r] = s;
-                        mx = fmaxf(mx, s);
+                        const int j = t0 + 16 * a + 4 * hi + r;
+                        st[c][a][r] = (j <= pos[c] && j >= low[c]) ? st[c][a][r] : -__builtin_inff();
                     }
-                mx = fmaxf(mx, __shfl_xor(mx, 16));
-                mx = fmaxf(mx, __shfl_xor(mx, 32));
-                const float mn = fmaxf(m[c], mx);
-                if (__any(mn > m[c])) {
-                    const float f = exp2_raw(m[c] - mn);
-                    m[c] = mn;
-                    l[c] *= f;
+        }
+        float mx[2];
 #pragma unroll
-                    for (int w = 0; w < RV / 16; ++w)
+        for (int c = 0; c < 2; ++c) {
+            float x = st[c][0][0];
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[c][w][r] *= f;
+            for (int a = 0; a < KT / 16; ++a)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (a + r) x = fmaxf(x, st[c][a][r]);
+            mx[c] = across_hi(x) * sc;
+        }
+        if (__any(mx[0] > m[0] + kSlack || mx[1] > m[1] + kSlack)) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float mn = fmaxf(m[c], mx[c]), f = exp2_raw(m[c] - mn);
+                m[c] = mn;
+                l[c] *= f;
+#pragma unroll
+                for (int w = 0; w < RV / 16; ++w)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[c][w][r] *= f;
+            }
+        }
+    };
+    // probabilities of the 32 keys from 32 u on and their share of the sum, for the columns c
+    auto exponentials = [&](const Scores& st, int u, int c, Probs& pb) {
+        float p[2][4];
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                p[a][r] = exp2_raw(__builtin_fmaf(st[c][2 * u + a][r], sc, -m[c]));   // exp2(-inf) = 0: m is finite always
+                l[c] += p[a][r];
+            }
+        pb[c][u] = u32x4{Bf::pack2(p[0][0], p[0][1]), Bf::pack2(p[0][2], p[0][3]), Bf::pack2(p[1][0], p[1][1]),
+                         Bf::pack2(p[1][2], p[1][3])};
+    };
+    // operands of group i of the value windows of a tile, and their part of the outputs
+    constexpr int kGroup = RV / 16 % 4 == 0 ? 4 : 2, kPerU = RV / 16 / kGroup, kGroups = KT / 32 * kPerU;
+    using ValueOps = u32x4[kGroup];
+    auto load_values = [&](int buf, int i, ValueOps& va) {
+        const unsigned char* v_tile = s_mem + buf * kBuffer + kBytes;
+#pragma unroll
+        for (int w = 0; w < kGroup; ++w) va[w] = value_operand<RV>(v_tile, 32 * (i / kPerU), i % kPerU * kGroup + w, lane);
+    };
+    auto gather = [&](int i, const ValueOps& va, const Probs& pb) {
+#pragma unroll
+        for (int w = 0; w < kGroup; ++w) {
+            const int at = i % kPerU * kGroup + w;
+            acc[0][at] = Bf::mfma16(va[w], pb[0][i / kPerU], acc[0][at]);
+            acc[1][at] = Bf::mfma16(va[w], pb[1][i / kPerU], acc[1][at]);
+        }
+    };
+
+    fetch_block(0);
+    put_row(0);
+    fetch_block(1);
+    put_row(1);
+    fetch_block(2);
+    put_row(2);
+    fetch_block(3);
+    __syncthreads();
+    stage_keys(0, 0);
+    stage_keys(1, 1);              // past the last tile: its last key again, like every row past the end
+    stage_values(0, 0);
+    __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if constexpr (R + RV < 512) {
+        Scores st_a, st_b;
+        if (active(0)) {
+#pragma unroll
+            for (int a = 0; a < KT / 16; ++a) {
+                KeyOps ka;
+                load_keys(0, a, ka);
+                score(a, ka, st_a);
+            }
+        }
+        const auto iteration = [&](int t, auto parity, Scores& st, Scores& st_next) {
+            constexpr int buf = decltype(parity)::value;
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's part of the keys of t + 1 and the values of t has landed
+            __syncthreads();                      // and everyone else's; the keys of t and the values of t - 1 are read
+            if (t + 2 < n_tiles) stage_keys(t + 2, buf);
+            if (t + 1 < n_tiles) stage_values(t + 1, buf ^ 1);
+            put_row(t + 3);
+            fetch_block(t + 4);
+            const bool now = active(t), then = active(t + 1);      // a wave's tiles follow one another
+            if (now) {
+                // operands are read one step before they are multiplied; nothing moves across the steps
+                KeyOps ka[2];
+                ValueOps va[2];
+                Probs pb;
+                load_keys(buf ^ 1, 0, ka[0]);
+                settle(t, st);
+#pragma unroll
+                for (int a = 0; a < KT / 16; ++a) {
+                    if (a + 1 < KT / 16) load_keys(buf ^ 1, a + 1, ka[(a + 1) & 1]);
+                    else load_values(buf, 0, va[0]);
+                    score(a, ka[a & 1], st_next);       // past the last tile: scores that nobody asks for
+                    exponentials(st, a >> 1, a & 1, pb);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
-                for (int u = 0; u < KT / 32; ++u) {
-                    float p[2][4];
+                for (int i = 0; i < kGroups; ++i) {
+                    if (i + 1 < kGroups) load_values(buf, i + 1, va[(i + 1) & 1]);
+                    gather(i, va[i & 1], pb);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else if (then) {
 #pragma unroll
-                    for (int a = 0; a < 2; ++a)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            p[a][r] = exp2_raw(st[c][2 * u + a][r] - mn);   // exp2(-inf) = 0: mn is finite always
-                            l[c] += p[a][r];
-                        }
-                    pb[c][u] = u32x4{Bf::pack2(p[0][0], p[0][1]), Bf::pack2(p[0][2], p[0][3]), Bf::pack2(p[1][0], p[1][1]),
-                                     Bf::pack2(p[1][2], p[1][3])};
+                for (int a = 0; a < KT / 16; ++a) {
+                    KeyOps ka;
+                    load_keys(buf ^ 1, a, ka);
+                    score(a, ka, st_next);
                 }
             }
-#pragma unroll
-            for (int u = 0; u < KT / 32; ++u)
-#pragma unroll
-                for (int w = 0; w < RV / 16; ++w) {
-                    const u32x4 va = value_operand<RV>(v_tile, 32 * u, w, lane);
-                    acc[0][w] = Bf::mfma16(va, pb[0][u], acc[0][w]);
-                    acc[1][w] = Bf::mfma16(va, pb[1][u], acc[1][w]);
-                }
+        };
+        for (int t = 0; t < n_tiles; t += 2) {
+            iteration(t, std::integral_constant<int, 0>{}, st_a, st_b);
+            if (t + 1 < n_tiles) iteration(t + 1, std::integral_constant<int, 1>{}, st_b, st_a);
         }
-        if (more) put_row(t0 + 2 * KT, buf);   // the slots were last read by the stage before this one
-        buf ^= 1;
+    } else {
+        // rows of 256 keys and values: the outputs and queries of a wave leave no room for the scores of two tiles
+        for (int t = 0; t < n_tiles; ++t) {
+            const int buf = t & 1;
+            __builtin_amdgcn_s_waitcnt(0x0F70);
+            __syncthreads();
+            if (t + 1 < n_tiles) {
+                if (t > 0) stage_keys(t + 1, buf ^ 1);
+                stage_values(t + 1, buf ^ 1);
+            }
+            put_row(t + 3);
+            fetch_block(t + 4);
+            if (!active(t)) continue;
+            Scores st;
+            Probs pb;
+#pragma unroll
+            for (int a = 0; a < KT / 16; ++a) {
+                KeyOps ka;
+                load_keys(buf, a, ka);
+                score(a, ka, st);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            settle(t, st);
+#pragma unroll
+            for (int a = 0; a < KT / 16; ++a) exponentials(st, a >> 1, a & 1, pb);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < kGroups; ++i) {
+                ValueOps va;
+                load_values(buf, i, va);
+                gather(i, va, pb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     }
     if (!wave_live) return;
 #pragma unroll
@@ -1007,7 +1155,7 @@ extern "C" int nqh_latent_attention_prefill(const void* q, const void* kv, int64
     else if (row == 128 && vdim <= 64) NQH_GO(128, 64, 64);
     else if (row == 128) NQH_GO(128, 128, 64);
     else if (row == 192 && vdim <= 64) NQH_GO(192, 64, 32);
-    else if (row == 192) NQH_GO(192, 128, 64);
+    else if (row == 192) NQH_GO(192, 128, 32);
     else if (vdim <= 128) NQH_GO(256, 128, 32);
     else NQH_GO(256, 256, 32);
 #undef NQH_GO

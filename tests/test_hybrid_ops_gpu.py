@@ -322,6 +322,42 @@ def test_ragged_pass_equals_each_sequence_alone(dtype):
         at += n
 
 
+@pytest.mark.parametrize("dim,block", [(32, 16), (64, 24), (96, 64), (128, 7), (128, 64), (192, 32), (256, 64)])
+def test_attention_prefill_tile_edges(dim, block):
+    """Contexts around the key tiles (32 and 64) and the query tiles (128), one to five tiles, blocks of any size; scores
+    that grow by less and by more than the slack from tile to tile, a row whose first tiles are masked, scales of any sign."""
+    H, G, bf = 4, 2, torch.bfloat16
+    row = ops.cache_rows(dim, dim, bf)[0]
+    lens = [1, 31, 33, 63, 64, 65, 127, 128, 129, 190, 257, 320]
+    per = [(n + block - 1) // block for n in lens]
+    first = [sum(per[:i]) for i in range(len(per))]
+    blocks = torch.randperm(sum(per), generator=torch.Generator().manual_seed(1)).tolist()
+    segs = [(0, n, blocks[f:f + p], 0) for n, f, p in zip(lens, first, per)]
+    k = torch.zeros(sum(per), G, block, row, dtype=bf)
+    v = torch.zeros_like(k)
+    ks, vs, qs = [], [], []
+    for i, (n, f, p) in enumerate(zip(lens, first, per)):
+        kk, vv, qq = rand(p * block, G, dim, seed=3 * i, dtype=bf), rand(p * block, G, dim, seed=3 * i + 1, dtype=bf), rand(n, H, dim, seed=3 * i + 2, dtype=bf)
+        kk *= (1 + torch.arange(p * block) / 40.0).view(-1, 1, 1).to(bf)       # later keys score higher and higher
+        for j, b in enumerate(blocks[f:f + p]):
+            k[b, :, :, :dim], v[b, :, :, :dim] = (x[j * block:(j + 1) * block].transpose(0, 1) for x in (kk, vv))
+        ks.append(kk[:n].double()), vs.append(vv[:n].double()), qs.append(qq)
+    q = torch.zeros(sum(lens), H, row, dtype=bf)
+    q[:, :, :dim] = torch.cat(qs)
+    lay = ops.PromptPass(segs, block, torch.device("cuda"))
+    for scale, window in ((dim ** -0.5, 0), (-dim ** -0.5, 0), (0.0, 0), (dim ** -0.5, 70)):
+        print(f"attention tiles dim={dim} block={block} scale={scale:.3f} window={window}", flush=True)
+        got = ops.attention_prefill(q.cuda(), k.cuda(), v.cuda(), lay, dim, dim, scale, window=window).cpu()
+        at = 0
+        for n, kk, vv, qq in zip(lens, ks, vs, qs):
+            s = torch.einsum("thd,shd->hts", qq.double(), kk.repeat_interleave(H // G, dim=1)) * scale
+            i, j = torch.arange(n).view(-1, 1), torch.arange(n).view(1, -1)
+            s = s.masked_fill((j > i) | (i - j >= (window or n + 1)), float("-inf"))
+            want = torch.einsum("hts,shd->thd", s.softmax(dim=2), vv.repeat_interleave(H // G, dim=1)).reshape(n, H * dim)
+            close(got[at:at + n], want, bf, (n, scale))
+            at += n
+
+
 # ---- mixture of experts --------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,width,experts,top,ff", [(1, 72, 5, 2, 48), (37, 64, 9, 1, 40), (20, 128, 7, 7, 64),
