@@ -5,7 +5,17 @@ from __future__ import annotations
 from dataclasses import dataclass, field
 from typing import List, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
+
+
+def upload(array: np.ndarray, device: torch.device, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The array on the device (in `out` if given), without waiting for work that is already on the stream: through pinned
+    memory of torch's host allocator, which keeps it until the copy is done."""
+    host = torch.from_numpy(array)
+    if torch.device(device).type == "cuda":
+        host = host.pin_memory()
+    return host.to(device, non_blocking=True) if out is None else out.copy_(host, non_blocking=True)
 
 
 @dataclass

@@ -18,10 +18,19 @@ from __future__ import annotations
 
 from typing import List, Optional
 
+import numpy as np
 import torch
 
 from . import ops
-from .cache import Lease, PagedKVCache, RecurrentStateCache
+from .cache import Lease, PagedKVCache, RecurrentStateCache, upload
+
+
+def _offsets(fields):
+    """Where fields (name, numpy type, shape) lie one after the other, each on a multiple of 256 bytes."""
+    at = 0
+    for _, kind, shape in fields:
+        yield at
+        at += -(-int(np.prod(shape)) * np.dtype(kind).itemsize // 256) * 256
 
 
 class EngineCore:
@@ -41,13 +50,20 @@ class EngineCore:
         self.use_graph = use_graph
         self._graph = None
         B, dev = max_batch, self.device
-        # static decode state, advanced on the device by the step itself
-        self.s_ids = torch.zeros(B, dtype=torch.long, device=dev)       # token fed at this step
-        self.s_pos = torch.zeros(B, dtype=torch.long, device=dev)       # its position
-        self.s_active = torch.zeros(B, dtype=torch.bool, device=dev)    # rows that own cache blocks
-        self.s_table = torch.zeros(B, self.max_blocks, dtype=torch.int32, device=dev)
-        self.s_slot = torch.zeros(B, dtype=torch.int32, device=dev)     # recurrent-state slot of the row
-        self.s_step = torch.zeros(1, dtype=torch.long, device=dev)      # row of s_out the step writes
+        # static decode state, advanced on the device by the step itself; one buffer, so that `decode` sets it in one copy
+        fields = [("s_ids", np.int64, (B,)),                    # token fed at this step
+                  ("s_pos", np.int64, (B,)),                    # its position
+                  ("s_step", np.int64, (1,)),                   # row of s_out the step writes
+                  ("s_table", np.int32, (B, self.max_blocks)),
+                  ("s_slot", np.int32, (B,)),                   # recurrent-state slot of the row
+                  ("s_active", np.bool_, (B,))]                 # rows that own cache blocks
+        self._state_fields = np.dtype({"names": [f[0] for f in fields], "formats": [f[1:] for f in fields],
+                                       "offsets": list(_offsets(fields))})
+        self._decode_state = torch.zeros(self._state_fields.itemsize, dtype=torch.uint8, device=dev)
+        for name, kind, shape in fields:
+            at = self._state_fields.fields[name][1]
+            part = self._decode_state[at:at + int(np.prod(shape)) * np.dtype(kind).itemsize]
+            setattr(self, name, part.view(getattr(torch, np.dtype(kind).name)).view(shape))
         self.s_out = torch.zeros(self.max_ctx + 1, B, dtype=torch.long, device=dev)
         self.s_logits: Optional[torch.Tensor] = None                    # logits of the last decode step [B, vocab]
 
@@ -99,15 +115,16 @@ class EngineCore:
         n = len(rows)
         if not 1 <= n <= self.max_batch:
             raise ValueError(f"{n} rows, the engine takes 1 to {self.max_batch}")
-        idle = self.max_batch - n
-        self.s_active.copy_(torch.tensor([True] * n + [False] * idle))
-        self.s_ids.copy_(torch.tensor([t for _, _, t in rows] + [0] * idle))
-        self.s_pos.copy_(torch.tensor([p for _, p, _ in rows] + [0] * idle))
-        self.s_step.zero_()
-        for i, (lease, pos, _) in enumerate(rows):
+        # the whole state in one copy from pinned memory that does not wait for the step before (a copy per row and field did,
+        # and took longer than a step)
+        state = np.zeros((), dtype=self._state_fields)
+        for i, (lease, pos, token) in enumerate(rows):
             if pos >= len(lease.blocks) * self.block_size:
                 raise ValueError(f"position {pos} has no cache block")
-            self._set_row(i, lease)
+            state["s_ids"][i], state["s_pos"][i], state["s_slot"][i] = int(token), int(pos), lease.slot
+            state["s_table"][i, :len(lease.blocks)] = lease.blocks
+        state["s_active"][:n] = True
+        upload(state.reshape(1).view(np.uint8), self.device, out=self._decode_state)
         self._run_decode()
         return self.s_logits[:n]
 

@@ -21,13 +21,14 @@ from __future__ import annotations
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence
 
+import numpy as np
 import torch
 import torch.nn.functional as F
 
 from ..models.hybrid import (AttentionSpec, DenseSpec, GatedLinearSpec, HybridDecoder, LatentAttentionSpec, RotarySpec,
                              SelectiveScanSpec, rotary_table)
 from . import hybrid_ops as ops
-from .cache import Lease, PagedKVCache, RecurrentStateCache
+from .cache import Lease, PagedKVCache, RecurrentStateCache, upload
 from .core import EngineCore
 
 
@@ -274,20 +275,21 @@ class HybridEngine(EngineCore):
             if n < 1 or p.start < 0 or p.start + n > min(len(p.lease.blocks) * bs, self.max_ctx):
                 raise ValueError(f"{n} tokens from position {p.start} do not fit the sequence's "
                                  f"{len(p.lease.blocks)} blocks of {bs} tokens")
-            if min(p.tokens) < 0 or max(p.tokens) >= self.spec.vocab:
+            plain = isinstance(p.tokens, (range, np.ndarray)) or all(type(t) is int for t in p.tokens)
+            tokens = np.array(p.tokens if plain else [int(t) for t in p.tokens], dtype=np.int64)
+            if tokens.min() < 0 or tokens.max() >= self.spec.vocab:
                 raise ValueError("token id outside the vocabulary")
-            ids += p.tokens
-            t = range(p.start, p.start + n)
-            pos += t
-            slots += [p.lease.blocks[i // bs] * bs + i % bs for i in t]
+            t = np.arange(p.start, p.start + n, dtype=np.int64)
+            ids.append(tokens)
+            pos.append(t)
+            slots.append(np.array(p.lease.blocks, dtype=np.int64)[t // bs] * bs + t % bs)
             want += [first + w for w in p.want]
             first += n
         layout = ops.PromptPass([(p.start, len(p.tokens), p.lease.blocks, p.lease.slot) for p in portions], bs, dev)
-        packed = torch.tensor([ids, pos, slots], dtype=torch.long).to(dev)
-        ids_d, pos_d, slots_d = packed[0], packed[1], packed[2]
+        packed = upload(np.concatenate(ids + pos + slots + [np.array(want, dtype=np.int64)]), dev)
+        ids_d, pos_d, slots_d, rows = packed.split([first, first, first, len(want)])
 
         step = Step(ids_d, pos_d, slots_d, layout=layout)
-        rows = torch.tensor(want, dtype=torch.long).to(dev)
         if not want:        # the pass still fills cache and state
             self._layers(step, trace=trace)
             return torch.empty(0, self.spec.vocab, dtype=torch.float32, device=dev)

@@ -6,9 +6,11 @@ from __future__ import annotations
 
 from typing import Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 from .. import _lib
+from .cache import upload
 
 _DTYPES = {torch.bfloat16: 1, torch.float32: 2}
 SKINNY_ROWS = 64
@@ -204,19 +206,20 @@ class PromptPass:
         self.rows = sum(s[1] for s in self.segments)
         tile = _lib.hybrid_lib().nqh_attention_tile_rows()
         width = max(1, max(len(s[2]) for s in self.segments))
-        table, seg, tiles, first = [], [], [], 0
+        table = np.zeros((len(self.segments), width), dtype=np.int32)
+        seg, tiles, first = [], [], 0
         for i, (start, rows, blocks, _) in enumerate(self.segments):
             if rows < 1 or start < 0 or start + rows > len(blocks) * block_size:
                 raise _lib.AwqHipError(f"segment {i}: positions {start} to {start + rows - 1} do not fit {len(blocks)} blocks")
-            table += list(blocks) + [0] * (width - len(blocks))
+            table[i, :len(blocks)] = blocks
             seg += [first, rows, start]
             tiles += [(min(start + q0 + tile, start + rows), i, q0) for q0 in range(0, rows, tile)]
             first += rows
         tiles.sort(reverse=True)                             # the tiles with the most keys first
         flat = [x for _, i, q0 in tiles for x in (i, q0)]
         self.num_tiles, self.max_blocks = len(tiles), width
-        packed = torch.tensor(table + seg + flat, dtype=torch.int32).to(device)
-        self.tables, self.seg, self.tiles = packed.split([len(table), len(seg), len(flat)])
+        packed = upload(np.concatenate([table.reshape(-1), np.array(seg + flat, dtype=np.int32)]), device)
+        self.tables, self.seg, self.tiles = packed.split([table.size, len(seg), len(flat)])
         self._pieces, self._contexts, self._row_tables = {}, None, None
 
     def contexts(self) -> Tuple[torch.Tensor, int, int]:
@@ -224,7 +227,7 @@ class PromptPass:
         if self._contexts is None:
             lens = [start + rows for start, rows, _, _ in self.segments]
             first = [sum(lens[:i]) for i in range(len(lens))]
-            self._contexts = torch.tensor(first, dtype=torch.int32).to(self.device), sum(lens), max(lens)
+            self._contexts = upload(np.array(first, dtype=np.int32), self.device), sum(lens), max(lens)
         return self._contexts
 
     def row_tables(self) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -233,7 +236,7 @@ class PromptPass:
         if self._row_tables is None:
             seg = [i for i, s in enumerate(self.segments) for _ in range(s[1])]
             ctx = [s[0] + t + 1 for s in self.segments for t in range(s[1])]
-            seg, ctx = torch.tensor([seg, ctx], dtype=torch.int32).to(self.device)
+            seg, ctx = upload(np.array([seg, ctx], dtype=np.int32), self.device)
             self._row_tables = self.tables.view(len(self.segments), self.max_blocks)[seg.long()].contiguous(), ctx.contiguous()
         return self._row_tables
 
@@ -248,7 +251,7 @@ class PromptPass:
                 for p in range(n):
                     out += [first + p * size, min(size, rows - p * size), slot, int(start == 0), p, n]
                 first += rows
-            self._pieces[size] = torch.tensor(out, dtype=torch.int32).to(self.device), len(out) // 6, chained
+            self._pieces[size] = upload(np.array(out, dtype=np.int32), self.device), len(out) // 6, chained
         return self._pieces[size]
 
 
