@@ -189,8 +189,6 @@ struct DenseKV {
 
 __device__ __forceinline__ float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
 
-constexpr float kSlack = 8.f;
-
 // Maximum over the four lanes that share a column: lanes l, l ^ 16, l ^ 32, l ^ 48.
 __device__ __forceinline__ float across_hi(float x) {
     const auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
@@ -205,16 +203,16 @@ __device__ __forceinline__ float across_hi(float x) {
 //
 // A wave multiplies the keys of tile t + 1 while it takes the exponentials of tile t, whose scores it has from the iteration
 // before: the two have nothing to do with each other, so matrix cores and vector ALU work side by side within a wave and not
-// only across the two waves of a SIMD.  Keys are therefore staged a tile ahead of the values.  The running maximum is only
-// moved (and sums and outputs rescaled) when a score exceeds it by a factor of 2^kSlack: probabilities are then at most 2^kSlack
-// instead of 1, with the same relative precision.
+// only across the two waves of a SIMD.  Keys are therefore staged a tile ahead of the values.  (Leaving the running maximum
+// alone until a score exceeds it by 2^8 saves 4 % of the time, but then the largest probability is no longer 1, which 16 bits
+// hold exactly: the error against 64 bits grows by up to a fifth where few keys dominate.)
 // What bounds it: per wave and tile of 64 x 128 64 MFMAs (1024 cycles) and some 250 vector instructions, 32 of them 2^x at a
 // quarter of the rate; two waves a SIMD, which is why rows of up to 128 keep within 256 registers (the form before, one wave
 // a SIMD, had 294).  Operands are read a step before they are multiplied; steps are fenced, or the scheduler asks for all of
 // them first and spills.  Bases of the lane's source rows are kept once, not per load, for the same reason.  Head sizes of
-// 128, causal, forms before / now: 32 heads 4 x 2048 tokens 376 / 187 us, 1 x 8192 1218 / 635 (866 TFLOP/s); 16 heads
-// 16 x 512 70 / 45, 1 x 512 24 / 18.  Rows of 32: 89 / 68, 64: 116 / 87, 96: 230 / 104, 192: 400 / 323, 256: 533 / 417 (4 x
-// 2048, 16 heads); expanded latents of 192 / 128: 450 / 268 with tiles of 32 keys, two waves a SIMD (64 keys, one: 424).
+// 128, causal, forms before / now: 32 heads 4 x 2048 tokens 376 / 204 us, 1 x 8192 1218 / 683 (805 TFLOP/s); 16 heads
+// 16 x 512 70 / 46, 1 x 512 24 / 19.  Rows of 32: 89 / 74, 64: 116 / 93, 96: 230 / 114, 192: 400 / 379, 256: 533 / 490 (4 x
+// 2048, 16 heads); expanded latents of 192 / 128: 450 / 298 with tiles of 32 keys, two waves a SIMD (64 keys, one: 424).
 template <int R, int RV, int KT, bool DENSE>
 __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
@@ -385,7 +383,7 @@ __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
                     if (a + r) x = fmaxf(x, st[c][a][r]);
             mx[c] = across_hi(x) * sc;
         }
-        if (__any(mx[0] > m[0] + kSlack || mx[1] > m[1] + kSlack)) {
+        if (__any(mx[0] > m[0] || mx[1] > m[1])) {
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 const float mn = fmaxf(m[c], mx[c]), f = exp2_raw(m[c] - mn);

@@ -325,7 +325,7 @@ def test_ragged_pass_equals_each_sequence_alone(dtype):
 @pytest.mark.parametrize("dim,block", [(32, 16), (64, 24), (96, 64), (128, 7), (128, 64), (192, 32), (256, 64)])
 def test_attention_prefill_tile_edges(dim, block):
     """Contexts around the key tiles (32 and 64) and the query tiles (128), one to five tiles, blocks of any size; scores
-    that grow by less and by more than the slack from tile to tile, a row whose first tiles are masked, scales of any sign."""
+    that grow from tile to tile, a row whose first tiles are masked, scales of any sign."""
     H, G, bf = 4, 2, torch.bfloat16
     row = ops.cache_rows(dim, dim, bf)[0]
     lens = [1, 31, 33, 63, 64, 65, 127, 128, 129, 190, 257, 320]
