@@ -85,6 +85,20 @@ int nq_silu_mul(const void* gate_up, void* out, int64_t rows, int64_t inter, int
  * awq_gemv_swiglu (include/awq_hip.h). */
 int nq_silu_mul_interleaved(const void* gate_up, void* out, int64_t rows, int64_t inter, int dtype, void* stream);
 
+/* The same for gate and up [rows, inter] as two tensors, the outputs of the projections one by one. */
+int nq_silu_mul_pair(const void* gate, const void* up, void* out, int64_t rows, int64_t inter, int dtype,
+                     void* stream);
+
+/* q [batch * tokens, num_heads * head_dim], k and v [.., num_kv_heads * head_dim]: outputs of the separate projections.
+ * q and k heads are normalised and rotated as by nq_qk_norm_rope_store, at positions[sequence][token] (per_sequence) or
+ * positions[token]; a negative position counts from the end of the table,
+ * and one outside the table gives NaN.  q_out keeps q's layout, k_out and v_out are
+ * [batch, num_kv_heads, tokens, head_dim].  head_dim 64, 128 or 256. */
+int nq_qkv_norm_rope(const void* q, const void* k, const void* v, const void* q_weight, const void* k_weight,
+                     const float* cos_sin, const int64_t* positions, int per_sequence, void* q_out, void* k_out,
+                     void* v_out, int64_t batch, int64_t tokens, int64_t num_heads, int64_t num_kv_heads,
+                     int64_t head_dim, int64_t max_positions, float q_eps, float k_eps, int dtype, void* stream);
+
 /* out[r] = argmax_i logits[r, i] as int64, the lowest index among equal maxima (NaNs are never selected);
  * logits [rows, vocab] dense.  Greedy sampling for the engine's decode loop; the reference has no generation
  * loop, the logits are those of Qwen3QuantizedForCausalLM.forward

@@ -86,6 +86,11 @@ int nqh_attention_prefill(const void* q, const void* k_cache, const void* v_cach
                           int64_t v_row, int64_t block_size, int64_t max_blocks, int64_t num_blocks, int64_t chunk,
                           int64_t window, float scale, int dtype, void* stream);
 
+/* Causal attention of `batch` sequences of `tokens` tokens over themselves, without a cache: q, out [batch, tokens, heads,
+ * dim], k, v [batch, kv_heads, tokens, dim].  bf16; dim 32, 64, 96, 128, 192 or 256. */
+int nqh_causal_attention(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t tokens, int64_t heads,
+                         int64_t kv_heads, int64_t dim, float scale, int dtype, void* stream);
+
 /* The same for one new token of each of `batch` sequences: context_lens[b] tokens are cached, the query is the last of
  * them.  block_table int32 [batch, max_blocks].  Workspace: nqh_attention_decode_workspace_bytes, uninitialised. */
 size_t nqh_attention_decode_workspace_bytes(int64_t batch, int64_t heads, int64_t kv_heads, int64_t v_row,

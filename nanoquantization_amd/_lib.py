@@ -73,6 +73,8 @@ SYMBOLS = {
     "nq_qk_norm_rope_store": (_int, [_vp] * 10 + [_i64] * 7 + [ctypes.c_float, _int, _vp]),
     "nq_paged_attention_workspace_bytes": (_sz, [_i64] * 5),
     "nq_paged_attention_decode": (_int, [_vp] * 6 + [_i64] * 7 + [ctypes.c_float, _int, _vp, _sz, _vp]),
+    "nq_silu_mul_pair": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _vp]),
+    "nq_qkv_norm_rope": (_int, [_vp] * 7 + [_int] + [_vp] * 3 + [_i64] * 6 + [ctypes.c_float] * 2 + [_int, _vp]),
     "nq_silu_mul": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nq_silu_mul_interleaved": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nq_argmax_rows": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
@@ -90,6 +92,7 @@ HYBRID_SYMBOLS = {
     "nqh_residual_norm_route": (_int, [_vp, _int, _vp, _i64, _vp, _vp, _vp, _i64] + [_vp] * 8 + [_i64] * 6 + [_f32, _int, _vp]),
     "nqh_qk_norm_rope_store": (_int, [_vp] * 9 + [_i64] * 11 + [_f32, _int, _vp]),
     "nqh_attention_tile_rows": (_i64, []),
+    "nqh_causal_attention": (_int, [_vp] * 4 + [_i64] * 5 + [_f32, _int, _vp]),
     "nqh_attention_prefill": (_int, [_vp] * 8 + [_i64] * 13 + [_f32, _int, _vp]),
     "nqh_attention_decode_workspace_bytes": (_sz, [_i64] * 7 + [_int]),
     "nqh_attention_decode": (_int, [_vp] * 7 + [_i64] * 12 + [_f32, _int, _vp, _sz, _vp]),

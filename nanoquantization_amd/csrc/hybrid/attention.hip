@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
     const uint16_t* __restrict__ sink, DenseKV dense, uint16_t* __restrict__ out, int heads, int kv_heads, int vdim,
-    int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles) {
+    int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles, int uniform) {
     using L = RowLayout<R>;
     using LV = RowLayout<RV>;
     constexpr int kBytes = KT * R * 2, kLoads = KT * L::kPieces / 256;
@@ -233,11 +233,20 @@ __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
     const int group = heads / kv_heads;
     const int g = id / (q_tiles * group), rest = id - g * q_tiles * group;
     const int qt = rest / group, h = g * group + rest % group;
-    const int seg = tiles[2 * qt], q0 = tiles[2 * qt + 1];
-    const int rows = segments[3 * seg + 1], start = segments[3 * seg + 2];
-    const int32_t* block_table = DENSE ? nullptr : block_tables + (int64_t)seg * max_blocks;
-    q += (int64_t)segments[3 * seg] * heads * R;
-    out += (int64_t)segments[3 * seg] * heads * vdim;
+    // `uniform`: no lists; sequences of that many tokens from position 0, one cache block each, the tiles with the most keys first
+    int seg, q0, rows, start;
+    int64_t first;
+    if (uniform) {
+        const int per = (uniform + kTileRows - 1) / kTileRows, batch = q_tiles / per;
+        seg = qt % batch, q0 = (per - 1 - qt / batch) * kTileRows, rows = uniform, start = 0;
+        first = (int64_t)seg * uniform;
+    } else {
+        seg = tiles[2 * qt], q0 = tiles[2 * qt + 1], rows = segments[3 * seg + 1], start = segments[3 * seg + 2];
+        first = segments[3 * seg];
+    }
+    const int32_t* block_table = DENSE || uniform ? nullptr : block_tables + (int64_t)seg * max_blocks;
+    q += first * heads * R;
+    out += first * heads * vdim;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lo = lane & 15, hi = lane >> 4;
     auto visible_from = [&](int p) { return first_visible(p, chunk, window); };
@@ -272,6 +281,10 @@ __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
         if constexpr (DENSE) return;
         if (wave != (t & 3)) return;
         const int j = min(k_begin + t * KT + lane % KT, k_end - 1);
+        if (uniform) {
+            next_block = seg, next_in_block = j;
+            return;
+        }
         const int b = block_shift >= 0 ? j >> block_shift : j / block_size;
         next_in_block = block_shift >= 0 ? j & (block_size - 1) : j - b * block_size;
         next_block = block_table[b];
@@ -987,7 +1000,7 @@ extern "C" int nqh_attention_prefill(const void* q, const void* k_cache, const v
             attn_tile_kernel<R, R, KT, false><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
                 (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables, segments, tiles,
                 (const uint16_t*)sink, DenseKV{}, (uint16_t*)out, (int)heads, (int)kv_heads, (int)vdim, (int)block_size,
-                (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale, (int)num_tiles);
+                (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale, (int)num_tiles, 0);
         });
         return launched(fn);
     }
@@ -997,6 +1010,28 @@ extern "C" int nqh_attention_prefill(const void* q, const void* k_cache, const v
             (const E*)q, (const E*)k_cache, (const E*)v_cache, block_tables, nullptr, segments, tiles, (const E*)sink,
             (E*)out, 0, (int)tile_groups, (int)heads, (int)kv_heads, (int)dim, (int)vdim, (int)k_row, (int)v_row,
             (int)block_size, (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale);
+    });
+    return launched(fn);
+}
+
+extern "C" int nqh_causal_attention(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t tokens,
+                                    int64_t heads, int64_t kv_heads, int64_t dim, float scale, int dtype, void* stream) {
+    const char* fn = "nqh_causal_attention";
+    if (!q || !k || !v || !out) return fail(NQH_ERR_ARG, fn, "null pointer");
+    if (batch <= 0 || tokens <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || dim <= 0)
+        return fail(NQH_ERR_ARG, fn, "sizes must be positive, heads a multiple of kv_heads");
+    if (!matrix_form(dim, dim, dtype))
+        return fail(NQH_ERR_UNSUPPORTED, fn, "bf16 and head dims of 32, 64, 96, 128, 192 or 256 only");
+    const int64_t num_tiles = batch * cdiv(tokens, kTileRows), groups = cdiv(num_tiles * heads, 8) * 8;
+    if (batch * kv_heads * tokens > kMaxI32 || groups > kMaxI32) return fail(NQH_ERR_ARG, fn, "problem too large");
+    if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 8)) return fail(NQH_ERR_ARG, fn, "misaligned pointer");
+    (void)hipGetLastError();
+    NQH_WITH_ROW(dim, {
+        constexpr int KT = R >= 192 ? 32 : 64;
+        attn_tile_kernel<R, R, KT, false><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
+            (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, nullptr, nullptr, nullptr, DenseKV{},
+            (uint16_t*)out, (int)heads, (int)kv_heads, (int)dim, (int)tokens, 1, (int)batch, 0, 0, scale, (int)num_tiles,
+            (int)tokens);
     });
     return launched(fn);
 }
@@ -1148,7 +1183,7 @@ extern "C" int nqh_latent_attention_prefill(const void* q, const void* kv, int64
 #define NQH_GO(R, RV, KT)                                                                                                   \
     attn_tile_kernel<R, RV, KT, true><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(                        \
         (const uint16_t*)q, nullptr, nullptr, nullptr, segments, tiles, nullptr, dense, (uint16_t*)out, (int)heads,          \
-        (int)heads, (int)vdim, 1, 0, 0, 0, 0, scale, (int)num_tiles)
+        (int)heads, (int)vdim, 1, 0, 0, 0, 0, scale, (int)num_tiles, 0)
     if (row == 64) NQH_GO(64, 64, 64);
     else if (row == 128 && vdim <= 64) NQH_GO(128, 64, 64);
     else if (row == 128) NQH_GO(128, 128, 64);

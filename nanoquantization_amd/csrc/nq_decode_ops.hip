@@ -227,6 +227,39 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
     }
 }
 
+// RMSNorm of a head and half-split rotary: HD / 8 neighbouring lanes hold a head, lane dc of them the dims a[0..7] = 8 dc ..;
+// cs: cos | sin of the head's position.  The summation order and rounding points of the q|k|v GEMV's fused epilogue (head_dim
+// 128: tile_ssq), so that all routes give the same bits.
+template <typename T, int HD>
+__device__ __forceinline__ u32x4 norm_rope(const float (&a)[8], const uint16_t* __restrict__ w, const float* __restrict__ cs,
+                                           int dc, float eps) {
+    constexpr int LPH = HD / 8, HALF = HD / 2;
+    float wf[8];
+    unpack8<T>(*reinterpret_cast<const u32x4*>(w + dc * 8), wf);
+    const int i0 = (dc % (LPH / 2)) * 8;   // index of this lane's first dim inside its half
+    const f32x4 c0 = *reinterpret_cast<const f32x4*>(cs + i0), c1 = *reinterpret_cast<const f32x4*>(cs + i0 + 4);
+    const f32x4 s0 = *reinterpret_cast<const f32x4*>(cs + HALF + i0), s1 = *reinterpret_cast<const f32x4*>(cs + HALF + i0 + 4);
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(a[e], a[e], ss);
+#pragma unroll
+    for (int o = LPH / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
+    const float r = rsqrtf(ss / (float)HD + eps);
+    float xn[8], y[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) xn[e] = round_to<T>(mul_round<T>(a[e], r) * wf[e]);
+    const bool first = dc < LPH / 2;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float other = __shfl_xor(xn[e], LPH / 2);
+        const float cc = e < 4 ? c0[e] : c1[e - 4], sn = e < 4 ? s0[e] : s1[e - 4];
+        const float x1 = first ? xn[e] : other, x2 = first ? other : xn[e];
+        y[e] = as_f32_result(first ? __fsub_rn(__fmul_rn(x1, cc), __fmul_rn(x2, sn))
+                                   : __fadd_rn(__fmul_rn(x1, sn), __fmul_rn(x2, cc)));
+    }
+    return pack8<T>(y);
+}
+
 // The same with 16-byte accesses, for head dims of 64, 128 or 256 and 16-byte aligned tensors (the scalar kernel
 // above moves 2 bytes per lane and instruction: 260 us per layer for a 16,384-token prefill of Qwen3-0.6B).
 // A lane owns 8 consecutive dims of a head, HD/8 lanes a head, a wave 64/(HD/8) heads; the rotary partner
@@ -259,37 +292,10 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_vec_kernel(
         // no return: heads of one wave differ in kind, and the shuffles below need every lane
     }
     const bool is_q = h < nh, is_k = !is_q && h < nh + nkv;
-    const uint16_t* w = is_q ? q_weight : k_weight;
-    float wf[8];
-    unpack8<T>(*reinterpret_cast<const u32x4*>(w + dc * 8), wf);
     int64_t pos = positions[row];
     pos = pos < 0 ? 0 : (pos >= max_positions ? max_positions - 1 : pos);
-    const int i0 = (dc % (LPH / 2)) * 8;   // index of this lane's first dim inside its half
-    const float* cs = cos_sin + pos * HD;
-    const f32x4 c0 = *reinterpret_cast<const f32x4*>(cs + i0), c1 = *reinterpret_cast<const f32x4*>(cs + i0 + 4);
-    const f32x4 s0 = *reinterpret_cast<const f32x4*>(cs + HALF + i0), s1 = *reinterpret_cast<const f32x4*>(cs + HALF + i0 + 4);
-    // the summation order and rounding points of the q|k|v GEMV's fused epilogue (head_dim 128: tile_ssq), so that
-    // both routes give the same bits
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(a[e], a[e], ss);
-#pragma unroll
-    for (int o = LPH / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
-    const float r = rsqrtf(ss / (float)HD + eps);
-    float xn[8], y[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) xn[e] = round_to<T>(mul_round<T>(a[e], r) * wf[e]);
-    const bool first = dc < LPH / 2;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float other = __shfl_xor(xn[e], LPH / 2);
-        const float cc = e < 4 ? c0[e] : c1[e - 4], sn = e < 4 ? s0[e] : s1[e - 4];
-        const float x1 = first ? xn[e] : other, x2 = first ? other : xn[e];
-        y[e] = as_f32_result(first ? __fsub_rn(__fmul_rn(x1, cc), __fmul_rn(x2, sn))
-                                   : __fadd_rn(__fmul_rn(x1, sn), __fmul_rn(x2, cc)));
-    }
+    const u32x4 packed = norm_rope<T, HD>(a, is_q ? q_weight : k_weight, cos_sin + pos * HD, dc, eps);
     if (!live || !(is_q || is_k)) return;
-    const u32x4 packed = pack8<T>(y);
     if (is_q) {
         *reinterpret_cast<u32x4*>(q_out + ((int64_t)row * nh + h) * HD + dc * 8) = packed;
         return;
@@ -298,6 +304,43 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_vec_kernel(
     if (slot_ok)
         *reinterpret_cast<u32x4*>(k_cache + (((slot / block_size) * nkv + (h - nh)) * block_size + slot % block_size) * HD +
                                   dc * 8) = packed;
+}
+
+// The same for the outputs of separate q, k and v projections of `batch` sequences of `tokens` tokens: q stays [token][head],
+// k and v become [sequence][kv head][token], where the attention over the sequences reads a head's tokens in a row.
+// Bound by memory: 8192 tokens of 16 + 8 + 8 heads of 128 (134 MB) 37 us, 3.6 TB/s; as torch
+// operations, which pass over fp32 copies a dozen times, 560.
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void qkv_norm_rope_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                                            const uint16_t* __restrict__ v, const uint16_t* __restrict__ q_weight,
+                                                            const uint16_t* __restrict__ k_weight,
+                                                            const float* __restrict__ cos_sin,
+                                                            const int64_t* __restrict__ positions, bool per_sequence,
+                                                            uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out,
+                                                            uint16_t* __restrict__ v_out, int64_t items, int tokens, int nh,
+                                                            int nkv, int64_t max_positions, float q_eps, float k_eps) {
+    constexpr int LPH = HD / 8, HPW = 64 / LPH;
+    const int heads = nh + 2 * nkv;
+    const int lane = threadIdx.x & 63, dc = lane % LPH;
+    int64_t item = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * HPW + lane / LPH;
+    const bool live = item < items;     // lanes past the end follow the last item (the shuffles need them) and store nothing
+    item = live ? item : items - 1;
+    const int64_t row = item / heads, seq = row / tokens;
+    const int h = (int)(item % heads), t = (int)(row % tokens);
+    const bool is_q = h < nh, is_k = !is_q && h < nh + nkv;
+    const int kv = is_k ? h - nh : h - nh - nkv;
+    const uint16_t* src = is_q ? q + (row * nh + h) * HD : (is_k ? k : v) + (row * nkv + kv) * HD;
+    const u32x4 raw = *reinterpret_cast<const u32x4*>(src + dc * 8);
+    float a[8];
+    unpack8<T>(raw, a);
+    int64_t pos = positions[per_sequence ? row : t];
+    pos += pos < 0 ? max_positions : 0;     // an index from the end, as the table's own indexing takes it
+    const bool known = pos >= 0 && pos < max_positions;     // no angles for any other: not a number, rather than a wrong turn
+    const u32x4 turned = norm_rope<T, HD>(a, is_q ? q_weight : k_weight, cos_sin + (known ? pos : 0) * HD, dc,
+                                          known ? (is_q ? q_eps : k_eps) : __builtin_nanf(""));
+    if (!live) return;
+    uint16_t* dst = is_q ? q_out + (row * nh + h) * HD : (is_k ? k_out : v_out) + ((seq * nkv + kv) * tokens + t) * HD;
+    *reinterpret_cast<u32x4*>(dst + dc * 8) = is_q || is_k ? turned : raw;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -887,23 +930,20 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const uint16_t* __res
     }
 }
 
-// IL: gate and up interleaved in words of 8 columns (word 2t = gate outputs 8t.., word 2t+1 = the up columns of the
-// same outputs) instead of side by side.
-template <typename T, bool IL>
-__global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gate_up,
-                                                       uint16_t* __restrict__ out, int64_t rows, int inter) {
+// Words of eight columns: word i of row r of gate and of up lies row_stride r + word_stride i elements from their starts.
+template <typename T>
+__global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gate, const uint16_t* __restrict__ up,
+                                                       uint16_t* __restrict__ out, int64_t rows, int words, int64_t row_stride,
+                                                       int word_stride) {
     const int64_t vec = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int per_row = inter / 8;
-    if (vec >= rows * per_row) return;
-    const int64_t r = vec / per_row;
-    const int i = (int)(vec % per_row) * 8;
+    if (vec >= rows * words) return;
+    const int64_t at = vec / words * row_stride + vec % words * word_stride;
     float g[8], u[8], o[8];
-    const uint16_t* row = gate_up + r * 2 * inter;
-    unpack8<T>(*reinterpret_cast<const u32x4*>(row + (IL ? 2 * i : i)), g);
-    unpack8<T>(*reinterpret_cast<const u32x4*>(row + (IL ? 2 * i + 8 : inter + i)), u);
+    unpack8<T>(*reinterpret_cast<const u32x4*>(gate + at), g);
+    unpack8<T>(*reinterpret_cast<const u32x4*>(up + at), u);
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = round_to<T>(g[e] / (1.f + __expf(-g[e]))) * u[e];
-    *reinterpret_cast<u32x4*>(out + r * inter + i) = pack8<T>(o);
+    *reinterpret_cast<u32x4*>(out + vec * 8) = pack8<T>(o);
 }
 
 int bad(const char* fn, const char* what) {
@@ -1233,10 +1273,10 @@ extern "C" int nq_decode_advance(const int64_t* next_tokens, const uint8_t* acti
     return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
 }
 
-static int silu_mul_entry(const char* fn, bool interleaved, const void* gate_up, void* out, int64_t rows, int64_t inter,
-                          int dtype, void* stream) {
-    if (!gate_up || !out) return bad(fn, "null pointer argument");
-    if (!aligned16(gate_up) || !aligned16(out)) return bad(fn, "tensors must be 16-byte aligned");
+static int silu_mul_entry(const char* fn, const void* gate, const void* up, void* out, int64_t rows, int64_t inter,
+                          int64_t row_stride, int word_stride, int dtype, void* stream) {
+    if (!gate || !up || !out) return bad(fn, "null pointer argument");
+    if (!aligned16(gate) || !aligned16(up) || !aligned16(out)) return bad(fn, "tensors must be 16-byte aligned");
     if (dtype != AWQ_F16 && dtype != AWQ_BF16) return bad(fn, "dtype must be AWQ_F16 or AWQ_BF16");
     if (rows <= 0 || inter <= 0 || inter % 8 != 0) return bad(fn, "rows > 0 and inter a positive multiple of 8");
     const int64_t vecs = rows * (inter / 8);
@@ -1244,22 +1284,68 @@ static int silu_mul_entry(const char* fn, bool interleaved, const void* gate_up,
     hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();
     const dim3 grid((unsigned)cdiv(vecs, 256)), block(256);
-    if (dtype == AWQ_F16) {
-        if (interleaved) silu_mul_kernel<F16, true><<<grid, block, 0, st>>>((const uint16_t*)gate_up, (uint16_t*)out, rows, (int)inter);
-        else silu_mul_kernel<F16, false><<<grid, block, 0, st>>>((const uint16_t*)gate_up, (uint16_t*)out, rows, (int)inter);
-    } else {
-        if (interleaved) silu_mul_kernel<BF16, true><<<grid, block, 0, st>>>((const uint16_t*)gate_up, (uint16_t*)out, rows, (int)inter);
-        else silu_mul_kernel<BF16, false><<<grid, block, 0, st>>>((const uint16_t*)gate_up, (uint16_t*)out, rows, (int)inter);
-    }
+    if (dtype == AWQ_F16)
+        silu_mul_kernel<F16><<<grid, block, 0, st>>>((const uint16_t*)gate, (const uint16_t*)up, (uint16_t*)out, rows,
+                                                     (int)(inter / 8), row_stride, word_stride);
+    else
+        silu_mul_kernel<BF16><<<grid, block, 0, st>>>((const uint16_t*)gate, (const uint16_t*)up, (uint16_t*)out, rows,
+                                                      (int)(inter / 8), row_stride, word_stride);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
 }
 
 extern "C" int nq_silu_mul(const void* gate_up, void* out, int64_t rows, int64_t inter, int dtype, void* stream) {
-    return silu_mul_entry("nq_silu_mul", false, gate_up, out, rows, inter, dtype, stream);
+    return silu_mul_entry("nq_silu_mul", gate_up, (const uint16_t*)gate_up + (inter > 0 ? inter : 0), out, rows, inter, 2 * inter, 8,
+                          dtype, stream);
 }
 
 extern "C" int nq_silu_mul_interleaved(const void* gate_up, void* out, int64_t rows, int64_t inter, int dtype,
                                        void* stream) {
-    return silu_mul_entry("nq_silu_mul_interleaved", true, gate_up, out, rows, inter, dtype, stream);
+    return silu_mul_entry("nq_silu_mul_interleaved", gate_up, (const uint16_t*)gate_up + 8, out, rows, inter, 2 * inter, 16, dtype,
+                          stream);
+}
+
+extern "C" int nq_silu_mul_pair(const void* gate, const void* up, void* out, int64_t rows, int64_t inter, int dtype,
+                                void* stream) {
+    return silu_mul_entry("nq_silu_mul_pair", gate, up, out, rows, inter, inter, 8, dtype, stream);
+}
+
+extern "C" int nq_qkv_norm_rope(const void* q, const void* k, const void* v, const void* q_weight, const void* k_weight,
+                                const float* cos_sin, const int64_t* positions, int per_sequence, void* q_out, void* k_out,
+                                void* v_out, int64_t batch, int64_t tokens, int64_t num_heads, int64_t num_kv_heads,
+                                int64_t head_dim, int64_t max_positions, float q_eps, float k_eps, int dtype, void* stream) {
+    const char* fn = "nq_qkv_norm_rope";
+    if (!q || !k || !v || !q_weight || !k_weight || !cos_sin || !positions || !q_out || !k_out || !v_out)
+        return bad(fn, "null pointer argument");
+    for (const void* p : {q, k, v, q_weight, k_weight, (const void*)cos_sin, (const void*)q_out, (const void*)k_out, (const void*)v_out})
+        if (!aligned16(p)) return bad(fn, "every tensor must be 16-byte aligned");
+    if (dtype != AWQ_F16 && dtype != AWQ_BF16) return bad(fn, "dtype must be AWQ_F16 or AWQ_BF16");
+    if (batch <= 0 || tokens <= 0 || num_heads <= 0 || num_kv_heads <= 0 || max_positions <= 0 || tokens > 0x7fffffff ||
+        num_heads + 2 * num_kv_heads > 0x7fffffff)
+        return bad(fn, "sizes must be positive 31-bit counts");
+    if (head_dim != 64 && head_dim != 128 && head_dim != 256) {
+        set_error("%s: head_dim must be 64, 128 or 256, got %lld", fn, (long long)head_dim);
+        return AWQ_ERR_UNSUPPORTED;
+    }
+    const int64_t items = batch * tokens * (num_heads + 2 * num_kv_heads), groups = cdiv(items, 4 * (512 / head_dim));
+    if (groups > 0x7fffffff) return bad(fn, "problem too large");
+    hipStream_t st = (hipStream_t)stream;
+    (void)hipGetLastError();
+#define NQ_GO(TT, HH)                                                                                                     \
+    qkv_norm_rope_kernel<TT, HH><<<dim3((unsigned)groups), dim3(256), 0, st>>>(                                            \
+        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_weight, (const uint16_t*)k_weight,  \
+        cos_sin, positions, per_sequence != 0, (uint16_t*)q_out, (uint16_t*)k_out, (uint16_t*)v_out, items, (int)tokens,   \
+        (int)num_heads, (int)num_kv_heads, max_positions, q_eps, k_eps)
+    if (dtype == AWQ_F16) {
+        if (head_dim == 64) NQ_GO(F16, 64);
+        else if (head_dim == 128) NQ_GO(F16, 128);
+        else NQ_GO(F16, 256);
+    } else {
+        if (head_dim == 64) NQ_GO(BF16, 64);
+        else if (head_dim == 128) NQ_GO(BF16, 128);
+        else NQ_GO(BF16, 256);
+    }
+#undef NQ_GO
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
 }

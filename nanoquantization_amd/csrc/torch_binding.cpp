@@ -7,6 +7,9 @@
 //   torch.ops.nanoquantization_amd.awq_dequantize(qweight, qscales, qzeros) -> Tensor [K, N]
 //   torch.ops.nanoquantization_amd.awq_linear(x, qweight, qscales, qzeros, bias?) -> Tensor [M, N]
 //   torch.ops.nanoquantization_amd.awq_linear_swiglu(x, qweight, qscales, qzeros) -> Tensor [M, N / 2]
+// and the steps between the linears of the Qwen3 modules (nanoquantization/layers/norm.py:18-32, layers/rope.py:24-45,
+// models/qwen3_quantized.py:79-99, 147-152), inference only (none has a derivative):
+//   rms_norm, silu_mul, qkv_norm_rope, causal_attention
 // with Meta kernels (shapes only), so the operators are visible to the dispatcher and to tracing.
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
@@ -18,6 +21,8 @@
 #include <vector>
 
 #include "../../include/awq_hip.h"
+#include "../../include/nq_engine_ops.h"
+#include "../../include/nq_hybrid_ops.h"
 
 namespace {
 
@@ -200,22 +205,146 @@ at::Tensor awq_linear_swiglu_meta(const at::Tensor& x, const at::Tensor& qweight
     return at::empty({x.size(0), qscales.size(1) / 2}, qscales.options());
 }
 
+// ---- the steps between the linears -------------------------------------------------------------------------------------
+int dtype_of(const at::Tensor& t) {
+    TORCH_CHECK(t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16, "float16 or bfloat16 expected, got ",
+                t.scalar_type());
+    return t.scalar_type() == at::kHalf ? AWQ_F16 : AWQ_BF16;
+}
+
+// Dense and 16-byte aligned, as the kernels' accesses want it: a view into the middle of a buffer may be neither.
+at::Tensor dense16(const at::Tensor& t) {
+    const at::Tensor d = t.contiguous();
+    return reinterpret_cast<uintptr_t>(d.data_ptr()) & 15u ? d.clone() : d;
+}
+
+at::Tensor rms_norm_op(const at::Tensor& x, const at::Tensor& weight, double eps) {
+    const int dtype = dtype_of(x);
+    TORCH_CHECK(x.dim() >= 1 && weight.dim() == 1 && x.size(-1) == weight.size(0) && weight.scalar_type() == x.scalar_type(),
+                "weight must be [x.size(-1)] of x's dtype");
+    check_device(x, {&weight});
+    const DeviceGuard guard(x.device());
+    at::Tensor y = at::empty(x.sizes(), x.options());
+    if (x.numel() == 0) return y;
+    const at::Tensor xd = dense16(x), w = dense16(weight);
+    const int64_t hidden = x.size(-1);
+    check_status(nq_add_rmsnorm(xd.data_ptr(), nullptr, w.data_ptr(), y.data_ptr(), x.numel() / hidden, hidden, (float)eps,
+                                dtype, current_stream(x.device().index())),
+                 "nq_add_rmsnorm");
+    return y;
+}
+at::Tensor rms_norm_meta(const at::Tensor& x, const at::Tensor&, double) { return at::empty(x.sizes(), x.options()); }
+
+at::Tensor silu_mul_op(const at::Tensor& gate, const at::Tensor& up) {
+    const int dtype = dtype_of(gate);
+    TORCH_CHECK(gate.dim() >= 1 && gate.sizes() == up.sizes() && gate.scalar_type() == up.scalar_type(),
+                "gate and up must be alike");
+    check_device(gate, {&up});
+    const DeviceGuard guard(gate.device());
+    at::Tensor y = at::empty(gate.sizes(), gate.options());
+    if (gate.numel() == 0) return y;
+    const at::Tensor g = dense16(gate), u = dense16(up);
+    const int64_t inter = gate.size(-1);
+    check_status(nq_silu_mul_pair(g.data_ptr(), u.data_ptr(), y.data_ptr(), gate.numel() / inter, inter, dtype,
+                                  current_stream(gate.device().index())),
+                 "nq_silu_mul_pair");
+    return y;
+}
+at::Tensor silu_mul_meta(const at::Tensor& gate, const at::Tensor&) { return at::empty(gate.sizes(), gate.options()); }
+
+using Three = std::tuple<at::Tensor, at::Tensor, at::Tensor>;
+
+Three qkv_outputs(const at::Tensor& q, int64_t heads, int64_t kv_heads) {
+    const int64_t b = q.size(0), s = q.size(1), hd = q.size(2) / heads;
+    return {at::empty({b, s, heads, hd}, q.options()), at::empty({b, kv_heads, s, hd}, q.options()),
+            at::empty({b, kv_heads, s, hd}, q.options())};
+}
+
+Three qkv_norm_rope_op(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& q_weight,
+                       const at::Tensor& k_weight, const at::Tensor& cos_sin, const at::Tensor& positions, int64_t heads,
+                       int64_t kv_heads, double q_eps, double k_eps) {
+    const int dtype = dtype_of(q);
+    TORCH_CHECK(q.dim() == 3 && k.dim() == 3 && v.dim() == 3 && heads > 0 && kv_heads > 0 && q.size(2) % heads == 0,
+                "q, k and v must be [batch, tokens, heads * head_dim]");
+    const int64_t b = q.size(0), s = q.size(1), hd = q.size(2) / heads;
+    TORCH_CHECK(k.sizes() == v.sizes() && k.size(0) == b && k.size(1) == s && k.size(2) == kv_heads * hd, "k and v do not go with q");
+    TORCH_CHECK(q_weight.dim() == 1 && q_weight.size(0) == hd && k_weight.dim() == 1 && k_weight.size(0) == hd,
+                "norm weights must be [head_dim]");
+    for (const at::Tensor* t : {&k, &v, &q_weight, &k_weight})
+        TORCH_CHECK(t->scalar_type() == q.scalar_type(), "one dtype expected");
+    TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() && cos_sin.numel() > 0 && cos_sin.numel() % hd == 0,
+                "cos_sin must be a dense float32 table of head_dim columns");
+    TORCH_CHECK(positions.scalar_type() == at::kLong && positions.dim() == 2 && positions.size(1) == s &&
+                    (positions.size(0) == 1 || positions.size(0) == b),
+                "positions must be int64 [1 or batch, tokens]");
+    check_device(q, {&k, &v, &q_weight, &k_weight, &cos_sin, &positions});
+    const DeviceGuard guard(q.device());
+    Three out = qkv_outputs(q, heads, kv_heads);
+    if (b * s == 0) return out;
+    const at::Tensor qd = dense16(q), kd = dense16(k), vd = dense16(v), qw = dense16(q_weight), kw = dense16(k_weight),
+                     table = dense16(cos_sin), pos = positions.contiguous();
+    check_status(nq_qkv_norm_rope(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), qw.data_ptr(), kw.data_ptr(),
+                                  table.data_ptr<float>(), pos.data_ptr<int64_t>(), pos.size(0) > 1, std::get<0>(out).data_ptr(),
+                                  std::get<1>(out).data_ptr(), std::get<2>(out).data_ptr(), b, s, heads, kv_heads, hd,
+                                  table.numel() / hd, (float)q_eps, (float)k_eps, dtype, current_stream(q.device().index())),
+                 "nq_qkv_norm_rope");
+    return out;
+}
+Three qkv_norm_rope_meta(const at::Tensor& q, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+                         const at::Tensor&, const at::Tensor&, int64_t heads, int64_t kv_heads, double, double) {
+    return qkv_outputs(q, heads, kv_heads);
+}
+
+at::Tensor causal_attention_op(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, double scale) {
+    TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16 && v.scalar_type() == at::kBFloat16,
+                "bfloat16 expected");
+    TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && k.sizes() == v.sizes() && k.size(0) == q.size(0) && k.size(2) == q.size(1) &&
+                    k.size(3) == q.size(3) && k.size(1) > 0 && q.size(2) % k.size(1) == 0,
+                "q must be [batch, tokens, heads, dim], k and v [batch, kv_heads, tokens, dim]");
+    check_device(q, {&k, &v});
+    const DeviceGuard guard(q.device());
+    at::Tensor out = at::empty({q.size(0), q.size(1), q.size(2) * q.size(3)}, q.options());
+    if (out.numel() == 0) return out;
+    const at::Tensor qd = dense16(q), kd = dense16(k), vd = dense16(v);
+    const int status = nqh_causal_attention(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q.size(0), q.size(1),
+                                            q.size(2), k.size(1), q.size(3), (float)scale, NQH_BF16,
+                                            current_stream(q.device().index()));
+    TORCH_CHECK(status == NQH_OK, "libnq_hybrid: nqh_causal_attention failed (status ", status, "): ", nqh_last_error());
+    return out;
+}
+at::Tensor causal_attention_meta(const at::Tensor& q, const at::Tensor&, const at::Tensor&, double) {
+    return at::empty({q.size(0), q.size(1), q.size(2) * q.size(3)}, q.options());
+}
+
 }  // namespace
 
 TORCH_LIBRARY(nanoquantization_amd, m) {
     m.def("awq_dequantize(Tensor qweight, Tensor qscales, Tensor qzeros) -> Tensor");
     m.def("awq_linear(Tensor x, Tensor qweight, Tensor qscales, Tensor qzeros, Tensor? bias=None) -> Tensor");
     m.def("awq_linear_swiglu(Tensor x, Tensor qweight, Tensor qscales, Tensor qzeros) -> Tensor");
+    m.def("rms_norm(Tensor x, Tensor weight, float eps) -> Tensor");
+    m.def("silu_mul(Tensor gate, Tensor up) -> Tensor");
+    m.def("qkv_norm_rope(Tensor q, Tensor k, Tensor v, Tensor q_weight, Tensor k_weight, Tensor cos_sin, Tensor positions, "
+          "int heads, int kv_heads, float q_eps, float k_eps) -> (Tensor, Tensor, Tensor)");
+    m.def("causal_attention(Tensor q, Tensor k, Tensor v, float scale) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(nanoquantization_amd, CUDA, m) {   // the dispatch key of HIP tensors in PyTorch-ROCm
     m.impl("awq_dequantize", &awq_dequantize_op);
     m.impl("awq_linear", &awq_linear_op);
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_op);
+    m.impl("rms_norm", &rms_norm_op);
+    m.impl("silu_mul", &silu_mul_op);
+    m.impl("qkv_norm_rope", &qkv_norm_rope_op);
+    m.impl("causal_attention", &causal_attention_op);
 }
 
 TORCH_LIBRARY_IMPL(nanoquantization_amd, Meta, m) {
     m.impl("awq_dequantize", &awq_dequantize_meta);
     m.impl("awq_linear", &awq_linear_meta);
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_meta);
+    m.impl("rms_norm", &rms_norm_meta);
+    m.impl("silu_mul", &silu_mul_meta);
+    m.impl("qkv_norm_rope", &qkv_norm_rope_meta);
+    m.impl("causal_attention", &causal_attention_meta);
 }

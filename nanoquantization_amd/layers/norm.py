@@ -1,10 +1,13 @@
 """RMSNorm with the arithmetic of nanoquantization/layers/norm.py:10-35: normalise in fp32, cast back
-to the input dtype, then multiply by the weight in that dtype.  Plain torch ops (adjacent to the AWQ
-path, not a kernel of this library)."""
+to the input dtype, then multiply by the weight in that dtype.  One kernel where no gradient is wanted,
+torch operations otherwise."""
 from __future__ import annotations
 
 import torch
 from torch import nn
+
+from .. import _lib
+from .inference import plain
 
 
 class RMSNorm(nn.Module):
@@ -20,4 +23,8 @@ class RMSNorm(nn.Module):
         return xf.to(x.dtype) * self.weight
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # a workgroup per row: rows of a few hundred elements (the heads') leave most of it idle
+        n = self.weight.numel()
+        if 512 <= n <= 8192 and n % 8 == 0 and x.shape[-1:] == self.weight.shape and plain(x, self.weight):
+            return _lib.torch_ops().rms_norm(x, self.weight, self.eps)
         return self.rms_norm(x)

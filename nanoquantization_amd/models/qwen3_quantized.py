@@ -15,7 +15,9 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import _lib
 from ..layers.gemm import WQLinear_GEMM
+from ..layers.inference import plain, unhooked
 from ..layers.norm import RMSNorm
 from ..layers.rope import RoPE
 
@@ -41,20 +43,43 @@ class Qwen3QuantizedAttention(nn.Module):
 
     def qkv(self, x: torch.Tensor, position_ids: torch.Tensor):
         """Projections, per-head q/k RMSNorm, rotary: [b, s, heads, d], [b, s, kv, d], [b, s, kv, d]."""
-        bs = x.shape[0]
+        return self._norm_rope(self.q_proj(x), self.k_proj(x), self.v_proj(x), position_ids)
+
+    def _norm_rope(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, position_ids: torch.Tensor):
+        bs = q.shape[0]
         if position_ids.dim() == 1:
             position_ids = position_ids.unsqueeze(0)
-        q = self.q_proj(x).view(bs, -1, self.num_heads, self.head_dim)
-        k = self.k_proj(x).view(bs, -1, self.num_kv_heads, self.head_dim)
-        v = self.v_proj(x).view(bs, -1, self.num_kv_heads, self.head_dim)
+        q = q.view(bs, -1, self.num_heads, self.head_dim)
+        k = k.view(bs, -1, self.num_kv_heads, self.head_dim)
+        v = v.view(bs, -1, self.num_kv_heads, self.head_dim)
         q, k = self.rope(self.q_norm(q), self.k_norm(k), position_ids)
         return q, k, v
 
+    def _fused(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: torch.Tensor) -> bool:
+        """Whether norms, rotary and the move of k and v into head order run as one kernel: the head dims it is built for, a
+        position per token, and norms and rotary that are the ones of this package and watched by no hook."""
+        return (q.dim() == 3 and self.head_dim in (64, 128, 256) and type(pos) is torch.Tensor
+                and pos.dtype in (torch.int32, torch.int64) and pos.dim() in (1, 2) and pos.shape[-1] == q.shape[1]
+                and (pos.dim() == 1 or pos.shape[0] in (1, q.shape[0]))
+                and type(self.q_norm) is type(self.k_norm) is RMSNorm and type(self.rope) is RoPE
+                and self.rope.cos_sin_cache.dtype == torch.float32 and pos.device == q.device == self.rope.cos_sin_cache.device
+                and plain(q, k, v, self.q_norm.weight, self.k_norm.weight) and unhooked(self.q_norm, self.k_norm, self.rope))
+
     def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
         bs = x.shape[0]
-        q, k, v = self.qkv(x, position_ids)
-        o = F.scaled_dot_product_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2),
-                                           is_causal=True, enable_gqa=self.num_heads != self.num_kv_heads)
+        q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        if self._fused(q, k, v, position_ids):
+            pos = position_ids if position_ids.dim() == 2 else position_ids.unsqueeze(0)
+            q, k, v = _lib.torch_ops().qkv_norm_rope(q, k, v, self.q_norm.weight, self.k_norm.weight, self.rope.cos_sin_cache,
+                                                     pos.to(torch.int64), self.num_heads, self.num_kv_heads, self.q_norm.eps,
+                                                     self.k_norm.eps)
+            if q.dtype == torch.bfloat16:
+                return self.o_proj(_lib.torch_ops().causal_attention(q, k, v, self.head_dim ** -0.5))
+        else:
+            q, k, v = self._norm_rope(q, k, v, position_ids)
+            k, v = k.transpose(1, 2), v.transpose(1, 2)
+        o = F.scaled_dot_product_attention(q.transpose(1, 2), k, v, is_causal=True,
+                                           enable_gqa=self.num_heads != self.num_kv_heads)
         o = o.transpose(1, 2).reshape(bs, -1, self.num_heads * self.head_dim)
         return self.o_proj(o)
 
@@ -70,7 +95,10 @@ class Qwen3QuantizedMLP(nn.Module):
         self.down_proj = mk(intermediate_size, hidden_size)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+        gate, up = self.gate_proj(x), self.up_proj(x)
+        if gate.shape[-1] % 8 == 0 and plain(gate, up):
+            return self.down_proj(_lib.torch_ops().silu_mul(gate, up))
+        return self.down_proj(F.silu(gate) * up)
 
 
 class Qwen3QuantizedBlock(nn.Module):

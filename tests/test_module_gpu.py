@@ -108,3 +108,104 @@ def test_linear_extreme_widths_default_dispatch(K, N, g):
             err = ((y.float() - ref).abs().max() / ref.abs().max()).item()
             assert y.shape == (M, N) and y.dtype == tdt and err <= tight, (M, err)
         del W
+
+
+def _eager(monkeypatch):
+    """The modules on torch operations only."""
+    from nanoquantization_amd.layers import norm
+    from nanoquantization_amd.models import qwen3_quantized as q3
+    for mod in (norm, q3):
+        monkeypatch.setattr(mod, "plain", lambda *t: False)
+
+
+@pytest.mark.parametrize("tdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hd,heads,kv,b,s,first", [(128, 16, 8, 2, 65, 0), (64, 4, 4, 3, 1, 7), (256, 6, 2, 1, 130, -140), (128, 3, 1, 1, 64, 3)])
+def test_steps_between_the_linears(tdt, hd, heads, kv, b, s, first):
+    """Norms, rotary, SiLU as one kernel each against the torch expressions of the modules: the same two rounding points,
+    each of which may fall one place (ulp, relative) apart where fp32 differs, and rarely does.  Attention against softmax in fp64: weights and output are
+    each rounded once, and 2^-8 relative covers both."""
+    from nanoquantization_amd import _lib
+    from nanoquantization_amd.layers.norm import RMSNorm
+    from nanoquantization_amd.layers.rope import RoPE
+    ops, ulp = _lib.torch_ops(), {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[tdt]
+    print(f"steps between the linears {tdt} hd={hd} heads={heads}/{kv} {b}x{s} from {first}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(hd + s)
+    rnd = lambda *n: torch.randn(*n, device="cuda", generator=gen).to(tdt)
+
+    def same(got, want):
+        assert got.shape == want.shape and got.dtype == want.dtype
+        d, w = (got.float() - want.float()).abs(), want.float().abs()
+        assert (d <= 2 * ulp * w + 1e-6).all() and (d > 0).float().mean() < 0.02
+
+    # a view that starts in the middle of a 16-byte word: the operators have to move it
+    q, k, v = (rnd(b, s, n * hd + 1)[..., 1:] for n in (heads, kv, kv))
+    qn, kn, rope = RMSNorm(hd, 1e-6), RMSNorm(hd, 1e-5), RoPE(hd, 512)
+    qn.weight.data, kn.weight.data = 1 + rnd(hd), 1 + rnd(hd)
+    rope = rope.cuda()
+    pos = torch.arange(first, first + s, device="cuda").repeat(b if first else 1, 1)
+    tq, tk, tv = ops.qkv_norm_rope(q, k, v, qn.weight.detach(), kn.weight.detach(), rope.cos_sin_cache, pos, heads, kv, 1e-6, 1e-5)
+    wq, wk = rope(qn.rms_norm(q.view(b, s, heads, hd)), kn.rms_norm(k.view(b, s, kv, hd)), pos)
+    rot = lambda got, want: ((got.float() - want.float()).abs() <= 2 * ulp * want.float().abs().amax(-1, True)).all()
+    assert rot(tq, wq) and rot(tk, wk.transpose(1, 2))     # x1 cos - x2 sin: a last place of a term, not of the difference
+    assert torch.equal(tv, v.view(b, s, kv, hd).transpose(1, 2))
+    bad = ops.qkv_norm_rope(q, k, v, qn.weight.detach(), kn.weight.detach(), rope.cos_sin_cache, pos * 0 + 512, heads, kv, 1e-6, 1e-5)
+    assert bad[0].isnan().all() and bad[1].isnan().all() and torch.equal(bad[2], tv)
+
+    n = RMSNorm(max(512, heads * hd), 1e-6)
+    x = rnd(b, s, n.norm_size)
+    n.weight.data = 1 + rnd(n.norm_size)
+    with torch.no_grad():
+        same(n(x), n.rms_norm(x))
+        same(n(x.transpose(0, 1)), n.rms_norm(x.transpose(0, 1)))
+    up = rnd(b, s, n.norm_size)
+    same(ops.silu_mul(x * 4, up), torch.nn.functional.silu(x * 4) * up)
+
+    if tdt == torch.bfloat16:
+        o = ops.causal_attention(tq, tk, tv, hd ** -0.5)
+        rep = lambda t: t.double().repeat_interleave(heads // kv, 1)
+        sc = tq.transpose(1, 2).double() @ rep(tk).transpose(-1, -2) * hd ** -0.5
+        w = sc.masked_fill(torch.ones(s, s, dtype=torch.bool, device="cuda").triu(1), float("-inf")).softmax(-1)
+        ref = (w @ rep(tv)).transpose(1, 2).reshape(b, s, heads * hd)
+        scale = (w @ rep(tv).abs()).transpose(1, 2).reshape(b, s, heads * hd)
+        assert ((o.double() - ref).abs() <= 2.0 ** -8 * (scale + ref.abs())).all()
+
+
+def test_when_modules_use_the_operators(monkeypatch):
+    """What the fused steps cannot do runs on torch operations as before: gradients, hooks, transforms, other shapes of
+    positions; and a prompt forward gives the same logits either way."""
+    from nanoquantization_amd.models.qwen3_quantized import Qwen3QuantizedForCausalLM
+    torch.manual_seed(0)
+    m = Qwen3QuantizedForCausalLM(num_hidden_layers=2, vocab_size=128, hidden_size=512, total_num_heads=4, total_num_kv_heads=2,
+                                  max_position_embeddings=64, intermediate_size=256, head_dim=64).to(torch.bfloat16)
+    for mod in m.modules():
+        if isinstance(mod, nq.WQLinear_GEMM):
+            mod.qweight.random_(-2 ** 31, 2 ** 31 - 1)
+            mod.qzeros.random_(-2 ** 31, 2 ** 31 - 1)
+            mod.qscales.uniform_(0.002, 0.006)
+    m = m.cuda()
+    ids, pos = torch.randint(0, 128, (2, 33), device="cuda"), torch.arange(33, device="cuda")
+    attn = m.model.layers[0].self_attn
+    x = torch.randn(2, 33, 512, device="cuda", dtype=torch.bfloat16)
+    seen = []
+    with torch.no_grad():
+        fused, fused_logits = attn(x, pos), m(ids, pos)
+        assert torch.equal(attn(x, pos.int()), fused) and torch.equal(attn(x, pos.expand(2, 33)), fused)
+        handle = attn.q_norm.register_forward_hook(lambda mod, a, out: seen.append(out.shape))
+        hooked = attn(x, pos)
+        handle.remove()
+        assert seen == [(2, 33, 4, 64)]
+        one = attn(x, pos[:1].view(1, 1))                  # one position for all tokens: broadcast by torch
+        mixed = attn(x.half(), pos)                        # float16 into bfloat16 projections
+        assert one.shape == fused.shape and torch.equal(mixed, attn(x.half().bfloat16(), pos))
+    assert not fused.requires_grad
+    norm = next(mod for mod in m.modules() if type(mod).__name__ == "RMSNorm" and mod.norm_size == 512)
+    xg = x.clone().requires_grad_()
+    norm(xg).float().sum().backward()
+    assert xg.grad is not None and norm.weight.grad is not None
+    assert torch.func.vmap(norm.rms_norm)(x).shape == x.shape and torch.equal(torch.func.vmap(norm)(x), norm.rms_norm(x))
+    _eager(monkeypatch)
+    with torch.no_grad():
+        assert torch.equal(attn(x, pos), hooked)
+        for got, want in ((fused, hooked), (fused_logits, m(ids, pos))):
+            # a dozen roundings to 8 bits on the way, of which few fall differently
+            assert (got.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
