@@ -87,7 +87,7 @@ int nqh_attention_prefill(const void* q, const void* k_cache, const void* v_cach
                           int64_t window, float scale, int dtype, void* stream);
 
 /* Causal attention of `batch` sequences of `tokens` tokens over themselves, without a cache: q, out [batch, tokens, heads,
- * dim], k, v [batch, kv_heads, tokens, dim].  bf16; dim 32, 64, 96, 128, 192 or 256. */
+ * dim], k, v [batch, kv_heads, tokens, dim].  bf16; dim 64, 128 or 256. */
 int nqh_causal_attention(const void* q, const void* k, const void* v, void* out, int64_t batch, int64_t tokens, int64_t heads,
                          int64_t kv_heads, int64_t dim, float scale, int dtype, void* stream);
 

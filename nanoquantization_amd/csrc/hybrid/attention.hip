@@ -213,12 +213,12 @@ __device__ __forceinline__ float across_hi(float x) {
 // 128, causal, forms before / now: 32 heads 4 x 2048 tokens 376 / 204 us, 1 x 8192 1218 / 683 (805 TFLOP/s); 16 heads
 // 16 x 512 70 / 46, 1 x 512 24 / 19.  Rows of 32: 89 / 74, 64: 116 / 93, 96: 230 / 114, 192: 400 / 379, 256: 533 / 490 (4 x
 // 2048, 16 heads); expanded latents of 192 / 128: 450 / 298 with tiles of 32 keys, two waves a SIMD (64 keys, one: 424).
-template <int R, int RV, int KT, bool DENSE>
-__global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
+template <int R, int RV, int KT, bool DENSE, bool EVEN>
+__device__ __forceinline__ void attn_tile(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
     const uint16_t* __restrict__ sink, DenseKV dense, uint16_t* __restrict__ out, int heads, int kv_heads, int vdim,
-    int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles, int uniform) {
+    int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles) {
     using L = RowLayout<R>;
     using LV = RowLayout<RV>;
     constexpr int kBytes = KT * R * 2, kLoads = KT * L::kPieces / 256;
@@ -233,18 +233,19 @@ __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
     const int group = heads / kv_heads;
     const int g = id / (q_tiles * group), rest = id - g * q_tiles * group;
     const int qt = rest / group, h = g * group + rest % group;
-    // `uniform`: no lists; sequences of that many tokens from position 0, one cache block each, the tiles with the most keys first
+    // EVEN: no lists; sequences of block_size tokens from position 0, one cache block each, the tiles with the most keys first.
+    // A template argument, since with a branch at run time the paged kernel's look-ups wait for its tile loads.
     int seg, q0, rows, start;
     int64_t first;
-    if (uniform) {
-        const int per = (uniform + kTileRows - 1) / kTileRows, batch = q_tiles / per;
-        seg = qt % batch, q0 = (per - 1 - qt / batch) * kTileRows, rows = uniform, start = 0;
-        first = (int64_t)seg * uniform;
+    if constexpr (EVEN) {
+        const int per = (block_size + kTileRows - 1) / kTileRows, batch = q_tiles / per;
+        seg = qt % batch, q0 = (per - 1 - qt / batch) * kTileRows, rows = block_size, start = 0;
+        first = (int64_t)seg * block_size;
     } else {
         seg = tiles[2 * qt], q0 = tiles[2 * qt + 1], rows = segments[3 * seg + 1], start = segments[3 * seg + 2];
         first = segments[3 * seg];
     }
-    const int32_t* block_table = DENSE || uniform ? nullptr : block_tables + (int64_t)seg * max_blocks;
+    const int32_t* block_table = DENSE || EVEN ? nullptr : block_tables + (int64_t)seg * max_blocks;
     q += first * heads * R;
     out += first * heads * vdim;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
         if constexpr (DENSE) return;
         if (wave != (t & 3)) return;
         const int j = min(k_begin + t * KT + lane % KT, k_end - 1);
-        if (uniform) {
+        if constexpr (EVEN) {
             next_block = seg, next_in_block = j;
             return;
         }
@@ -565,6 +566,27 @@ __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
             }
         }
     }
+}
+
+template <int R, int RV, int KT, bool DENSE>
+__global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
+    const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
+    const uint16_t* __restrict__ sink, DenseKV dense, uint16_t* __restrict__ out, int heads, int kv_heads, int vdim,
+    int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles) {
+    attn_tile<R, RV, KT, DENSE, false>(q, k_cache, v_cache, block_tables, segments, tiles, sink, dense, out, heads, kv_heads, vdim,
+                                       block_size, max_blocks, num_blocks, chunk, window, scale, q_tiles);
+}
+
+// No sink, chunk or window, but given at run time: with them known the compiler holds more across the key loop than the
+// registers take (rows of 128: 435 spilled, 6x the time).
+template <int R, int KT>
+__global__ __launch_bounds__(256, R > 160 ? 1 : 2) void attn_even_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const uint16_t* __restrict__ sink, uint16_t* __restrict__ out, int heads, int kv_heads, int batch, int tokens, int chunk,
+    int window, float scale, int q_tiles) {
+    attn_tile<R, R, KT, false, true>(q, k, v, nullptr, nullptr, nullptr, sink, DenseKV{}, out, heads, kv_heads, R, tokens, 1,
+                                     batch, chunk, window, scale, q_tiles);
 }
 
 // Decode attention.  Workgroup = (sequence, kv head, 16 of its query heads, context split); a wave takes tiles of 32 keys
@@ -1000,7 +1022,7 @@ extern "C" int nqh_attention_prefill(const void* q, const void* k_cache, const v
             attn_tile_kernel<R, R, KT, false><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
                 (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables, segments, tiles,
                 (const uint16_t*)sink, DenseKV{}, (uint16_t*)out, (int)heads, (int)kv_heads, (int)vdim, (int)block_size,
-                (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale, (int)num_tiles, 0);
+                (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale, (int)num_tiles);
         });
         return launched(fn);
     }
@@ -1020,19 +1042,20 @@ extern "C" int nqh_causal_attention(const void* q, const void* k, const void* v,
     if (!q || !k || !v || !out) return fail(NQH_ERR_ARG, fn, "null pointer");
     if (batch <= 0 || tokens <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads != 0 || dim <= 0)
         return fail(NQH_ERR_ARG, fn, "sizes must be positive, heads a multiple of kv_heads");
-    if (!matrix_form(dim, dim, dtype))
-        return fail(NQH_ERR_UNSUPPORTED, fn, "bf16 and head dims of 32, 64, 96, 128, 192 or 256 only");
+    if (dtype != NQH_BF16 || (dim != 64 && dim != 128 && dim != 256))
+        return fail(NQH_ERR_UNSUPPORTED, fn, "bf16 and head dims of 64, 128 or 256 only");
     const int64_t num_tiles = batch * cdiv(tokens, kTileRows), groups = cdiv(num_tiles * heads, 8) * 8;
     if (batch * kv_heads * tokens > kMaxI32 || groups > kMaxI32) return fail(NQH_ERR_ARG, fn, "problem too large");
     if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 8)) return fail(NQH_ERR_ARG, fn, "misaligned pointer");
     (void)hipGetLastError();
-    NQH_WITH_ROW(dim, {
-        constexpr int KT = R >= 192 ? 32 : 64;
-        attn_tile_kernel<R, R, KT, false><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
-            (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, nullptr, nullptr, nullptr, DenseKV{},
-            (uint16_t*)out, (int)heads, (int)kv_heads, (int)dim, (int)tokens, 1, (int)batch, 0, 0, scale, (int)num_tiles,
-            (int)tokens);
-    });
+    const auto go = [&](auto kernel) {
+        kernel<<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
+            (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, (uint16_t*)out, (int)heads, (int)kv_heads, (int)batch,
+            (int)tokens, 0, 0, scale, (int)num_tiles);
+    };
+    if (dim == 64) go(attn_even_kernel<64, 64>);
+    else if (dim == 128) go(attn_even_kernel<128, 64>);
+    else go(attn_even_kernel<256, 32>);
     return launched(fn);
 }
 
@@ -1183,7 +1206,7 @@ extern "C" int nqh_latent_attention_prefill(const void* q, const void* kv, int64
 #define NQH_GO(R, RV, KT)                                                                                                   \
     attn_tile_kernel<R, RV, KT, true><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(                        \
         (const uint16_t*)q, nullptr, nullptr, nullptr, segments, tiles, nullptr, dense, (uint16_t*)out, (int)heads,          \
-        (int)heads, (int)vdim, 1, 0, 0, 0, 0, scale, (int)num_tiles, 0)
+        (int)heads, (int)vdim, 1, 0, 0, 0, 0, scale, (int)num_tiles)
     if (row == 64) NQH_GO(64, 64, 64);
     else if (row == 128 && vdim <= 64) NQH_GO(128, 64, 64);
     else if (row == 128) NQH_GO(128, 128, 64);
