@@ -190,4 +190,15 @@ void take_prefetch_hint(PrefetchRegions* out);
 constexpr int64_t kMaxSplitTiles = 4096;
 constexpr size_t kCounterBytes = (size_t)kMaxSplitTiles * sizeof(int);
 
+// (a & mask) | magic as one v_and_or_b32: gfx950's VOP3 takes no literals and a
+// single scalar operand, so the mask is pinned in an SGPR and the magic in a VGPR.
+struct AndOr {
+    uint32_t mask, magic;
+    __device__ __forceinline__ AndOr(uint32_t m, uint32_t g) : mask(m), magic(g) {
+        asm volatile("" : "+s"(mask));
+        asm volatile("" : "+v"(magic));
+    }
+    __device__ __forceinline__ uint32_t operator()(uint32_t a) const { return (a & mask) | magic; }
+};
+
 }  // namespace awq

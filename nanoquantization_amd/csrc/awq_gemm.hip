@@ -213,9 +213,10 @@ static const GemmVariant kGemmVariants[] = {
     // pipelined kernel under these names too
     {"256x256r", 256, 256, 4},   // every tile cut split_k ways
     {"256x256rt", 256, 256, 4},  // split_k cuts only the tiles beyond the last full round of CUs
+    {"rows128", 128, 128, 4},    // awq_gemm_rows.hip, for a few hundred rows: awq_linear's choice alone (rows_wanted)
 };
 enum { k128x128 = 0, k64x256 = 1, k32x256 = 2 };
-constexpr int kPipeVariant = 3, kPipeTailVariant = 4, kRegbVariant = 5, kRegbTailVariant = 6;
+constexpr int kPipeVariant = 3, kPipeTailVariant = 4, kRegbVariant = 5, kRegbTailVariant = 6, kRowsVariant = 7;
 static bool is_tile256(int v) { return v >= kPipeVariant && v <= kRegbTailVariant; }
 static bool is_tail_variant(int v) { return v == kPipeTailVariant || v == kRegbTailVariant; }
 constexpr int kNumGemmVariants = sizeof(kGemmVariants) / sizeof(kGemmVariants[0]);
@@ -263,6 +264,7 @@ static int gemm_effective_splits(int64_t K, int split_k) {
 
 static size_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int variant, int split_k) {
     if (is_tile256(variant)) return pipe_ws_bytes(make_pipe_plan(M, N, K, split_k, is_tail_variant(variant)));
+    if (variant == kRowsVariant) return rows_ws_bytes(make_rows_plan(M, N, K, 32, split_k), M, N);
     const int splits = gemm_effective_splits(K, split_k);
     if (splits <= 1) return 0;
     return kCounterBytes + (size_t)splits * M * N * sizeof(float);
@@ -377,6 +379,11 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
         set_error("%s: the gated epilogue takes no bias, needs N %% 16 == 0 and runs on the pipelined kernel", fn);
         return AWQ_ERR_UNSUPPORTED;
     }
+    const RowsPlan rows = variant == kRowsVariant ? make_rows_plan(M, N, K, g, split_k) : RowsPlan{};
+    if (variant == kRowsVariant && rows.m_tiles == 0) {
+        set_error("%s: tile rows128 needs a group size that is a multiple of 32 and x below 2 Gi elements", fn);
+        return AWQ_ERR_UNSUPPORTED;
+    }
     const GemmVariant& gv = kGemmVariants[variant];
     if (cdiv(M, gv.BM) > 65535) {
         set_error("%s: M=%lld exceeds the launch grid for tile %s", fn, (long long)M, gv.name);
@@ -403,6 +410,9 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
         AWQ_GEMM_CASE(k128x128, 128, 128, 2, 2)
         AWQ_GEMM_CASE(k64x256, 64, 256, 1, 4)
         AWQ_GEMM_CASE(k32x256, 32, 256, 1, 4)
+        case kRowsVariant:
+            e = launch_rows(rows, dtype, x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K, (int)g, workspace, s);
+            break;
         case kPipeVariant:
         case kPipeTailVariant:
             e = launch_gemm_pipe(dtype, x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K, (int)g,
@@ -492,6 +502,36 @@ extern "C" int awq_gemm(const void* x, const int32_t* qweight, const void* qscal
                               dtype, workspace, workspace_bytes, stream, v, s);
 }
 
+// Microseconds of the fused 256 x 256 kernels: 1.9 a K step and round of 256 workgroups, 10 to fill and store a round's tiles,
+// and 0.05 per K slice of a tile for its fp32 partials and their sum (within 15 % of every size measured between 256 and 8192
+// rows).
+static double fused_linear_us(int64_t M, int64_t N, int64_t K) {
+    int v, split;
+    awq::pick_gemm(M, N, K, &v, &split);
+    const awq::PipePlan p = awq::make_pipe_plan(M, N, K, split, awq::is_tail_variant(v));
+    const double full = (double)awq::cdiv(p.full_tiles, 256), cut = (double)awq::cdiv((int64_t)p.tail_tiles * p.splits, 256);
+    return full * (1.9 * (double)(K / 64) + 10) + cut * (1.9 * p.iters_per_split + 10) + 0.05 * p.tail_tiles * p.splits;
+}
+
+// Short K at up to 2048 rows stays fused: awq_gemm_plan's kernel and K split are what a caller gets there, bit for bit, and
+// the difference is a few microseconds (1024 x 4096 at 1024 rows 31 / 22 us dequantised first).
+static bool always_fused(int64_t M, int64_t K) { return M <= 128 || (M <= 2048 && K < 2048); }
+
+// Whether the tiles of awq_gemm_rows.hip are the fastest way, from the estimates of all three; in one round of the CUs only
+// (5120 x 25600 at 160 rows, 400 tiles: 85 us in fp16 and 101 in bf16 against 85 fused).  Measured, fp16 / bf16 and the faster
+// of the other two: 2816 x 9720 at 333 rows 31 / 34 us against 46, 4096 x 4096 at 200 rows 24 / 25 against 29, at 512 rows
+// 33 / 36 against 41, 12288 x 4096 at 160 rows 35 / 39 against 46, 8192 x 1024 at 1024 rows 36 / 38 against 42, 2048 x 6144 at
+// 640 rows 26 / 27 against 34.
+static bool rows_wanted(int64_t M, int64_t N, int64_t K, int64_t g, awq::RowsPlan* plan) {
+    if (always_fused(M, K)) return false;
+    *plan = awq::make_rows_plan(M, N, K, g);
+    if (plan->m_tiles == 0 || (int64_t)plan->m_tiles * plan->n_tiles * plan->splits > 256 ||
+        plan->us >= 0.95 * fused_linear_us(M, N, K))
+        return false;
+    const double dense = awq::dense_linear_us(M, N, K, g);
+    return dense < 0 || plan->us < 0.95 * dense;
+}
+
 // 65..128 rows go to the GEMV (blocks of 16 rows) on weights up to this size, see kGemvMaxRows in awq_gemv.hip
 static bool gemv_rows_ok(int64_t M, int64_t N, int64_t K) {
     return M <= 64 || (M <= 128 && K * N <= (20ll << 20));
@@ -505,27 +545,23 @@ extern "C" size_t awq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
         const size_t c = awq_gemv_workspace_bytes(16, N, K);
         a = a > c ? a : c;
     }
-    return a > b ? a : b;
+    awq::RowsPlan rows;       // (the largest over the group sizes: they only decide whether it runs)
+    const size_t d = rows_wanted(M, N, K, 32, &rows) ? awq::rows_ws_bytes(rows, M, N) : 0;
+    const size_t most = a > b ? a : b;
+    return most > d ? most : d;
 }
 
-// Whether dequantising the weight first (awq_linear_dense) is the faster way, from estimates of both: the fused 256 x 256
-// kernels take 1.9 us a K step and round of 256 workgroups, 10 us to fill and store a round's tiles, and 0.05 us per K slice
-// of a tile for its fp32 partials and their sum (within 15 % of every size measured between 256 and 8192 rows).  Measured,
-// bf16, fused / dequantised first: 4096 x 12288 at 512 rows 74 / 69 us, 2048 rows 224 / 186, 8192 rows 787 / 575; 12288 x
-// 4096 at 512 rows (32 tiles cut in eight) 71 / 136, 2048 rows 209 / 176, 8192 rows 744 / 568; 1024 x 2048 at 4096 rows
-// 43 / 28; 2560 x 9728 at 333 rows 45 / 44, 8192 rows 441 / 309.
-// Short K at up to 2048 rows stays fused: awq_gemm_plan's kernel and K split are what a caller gets there, bit for bit, and
-// the difference is a few microseconds (1024 x 4096 at 1024 rows 31 / 22 us).
+// Whether dequantising the weight first (awq_linear_dense) is the faster way.  Measured, bf16, fused / dequantised first:
+// 4096 x 12288 at 512 rows 74 / 69 us, 2048 rows 224 / 186, 8192 rows 787 / 575; 12288 x 4096 at 512 rows (32 tiles cut in
+// eight) 71 / 136, 2048 rows 209 / 176, 8192 rows 744 / 568; 1024 x 2048 at 4096 rows 43 / 28; 2560 x 9728 at 333 rows
+// 45 / 44, 8192 rows 441 / 309.
 extern "C" size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size) {
-    if (M <= 128 || (M <= 2048 && K < 2048)) return 0;
+    if (always_fused(M, K)) return 0;
     const double dense = awq::dense_linear_us(M, N, K, group_size);
     if (dense < 0) return 0;
-    int v, split;
-    awq::pick_gemm(M, N, K, &v, &split);
-    const awq::PipePlan p = awq::make_pipe_plan(M, N, K, split, awq::is_tail_variant(v));
-    const double full = (double)awq::cdiv(p.full_tiles, 256), cut = (double)awq::cdiv((int64_t)p.tail_tiles * p.splits, 256);
-    const double fused = full * (1.9 * (double)(K / 64) + 10) + cut * (1.9 * p.iters_per_split + 10) + 0.05 * p.tail_tiles * p.splits;
-    return dense < fused ? awq_linear_dense_scratch_bytes(M, N, K, group_size) : 0;
+    awq::RowsPlan rows;
+    return dense < fused_linear_us(M, N, K) && !rows_wanted(M, N, K, group_size, &rows)
+               ? awq_linear_dense_scratch_bytes(M, N, K, group_size) : 0;
 }
 
 extern "C" size_t awq_linear_swiglu_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -576,6 +612,10 @@ extern "C" int awq_linear(const void* x, const int32_t* qweight, const void* qsc
         }
         return AWQ_OK;
     }
+    awq::RowsPlan rows;
+    if (M > 128 && N >= 8 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, &rows))
+        return awq::gemm_dispatch("awq_linear", x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,
+                                  workspace_bytes, stream, awq::kRowsVariant, rows.splits);
     return awq_gemm(x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,
                     workspace_bytes, stream);
 }

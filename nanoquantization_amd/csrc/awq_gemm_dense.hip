@@ -131,7 +131,9 @@ double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     if (!takes(M, N, K, g)) return -1;
     const int64_t slab = slab_columns(N, K);
     // the dequantise pass moves 2.5 bytes a weight at 6 TB/s (4096 x 12288 20.5 us, 5120 x 25600 62)
-    return 4 + 2.5 * (double)(K * N) / 6.0e6 +
+    // and a slab that the 256 MB cache does not hold is read from memory (5120 x 25600, 262 MB: 640 rows 242 us, 1500 rows 446)
+    const double cold = slab * K * 2 > (192ll << 20) ? 2.0 * (double)(K * N) / 6.0e6 : 0;
+    return 4 + 2.5 * (double)(K * N) / 6.0e6 + cold +
            (double)cdiv(N, slab) * std::min(product_us(M, slab, K, 128), product_us(M, slab, K, 256));
 }
 

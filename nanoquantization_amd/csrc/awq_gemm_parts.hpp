@@ -225,4 +225,18 @@ hipError_t launch_dequant_transpose(int dtype, const int32_t* qweight, const voi
 // awq_gemm_dense.hip: estimated microseconds of awq_linear_dense, -1 where it does not take the sizes.
 double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g);
 
+// awq_gemm_rows.hip: tiles of 80..128 rows by 128 columns for a few hundred rows; `us` an estimate of the time, m_tiles 0 where
+// it does not take the sizes.  split_k 0: the split with the least estimate.
+struct RowsPlan {
+    int m_tiles, n_tiles, mt, splits, steps_per_split;   // mt: 16-row tiles of a workgroup; steps: of 64 rows of K
+    double us;
+};
+RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int split_k = 0);
+inline size_t rows_ws_bytes(const RowsPlan& p, int64_t M, int64_t N) {
+    return p.splits > 1 ? kCounterBytes + (size_t)p.splits * M * N * sizeof(float) : 0;
+}
+hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_t* qweight, const void* qscales,
+                       const int32_t* qzeros, const void* bias, void* y, int M, int N, int K, int g, void* workspace,
+                       hipStream_t st);
+
 }  // namespace awq

@@ -77,17 +77,6 @@ struct Embed<BF16> {
     static constexpr float kMulLo = 1.f, kMulHi = 1.f;
 };
 
-// (a & mask) | magic as one v_and_or_b32: gfx950's VOP3 takes no literals and a
-// single scalar operand, so the mask is pinned in an SGPR and the magic in a VGPR.
-struct AndOr {
-    uint32_t mask, magic;
-    __device__ __forceinline__ AndOr(uint32_t m, uint32_t g) : mask(m), magic(g) {
-        asm volatile("" : "+s"(mask));
-        asm volatile("" : "+v"(magic));
-    }
-    __device__ __forceinline__ uint32_t operator()(uint32_t a) const { return (a & mask) | magic; }
-};
-
 template <int V>
 struct WordVec;
 template <>

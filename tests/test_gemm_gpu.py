@@ -393,3 +393,49 @@ def test_linear_random_shapes_default_dispatch():
         err = ((y.float() - ref).abs().max() / ref.abs().max().clamp_min(1e-6)).item()
         assert err <= (1.5e-3 if tdt == torch.float16 else 6e-3), err
         assert torch.equal(y, gemm_layer._linear("awq_linear", x, qw, qs, qz, bias))
+
+
+# a row, tiles of five to eight 16-row blocks, one row past a tile; less and more stages of K than the ring holds, also cut in
+# three; columns past the last tile; groups of less, as much and more than a stage
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,K,N,g", [(1, 64, 8, 32), (81, 320, 136, 64), (113, 384, 520, 128), (128, 448, 256, 32), (129, 512, 8, 512),
+                                      (270, 192, 264, 192), (333, 1088, 1032, 64)])
+def test_gemm_rows128(dtype, M, K, N, g):
+    print(f"gemm rows128 {dtype} M={M} K={K} N={N} g={g}", flush=True)
+    L = _lib.lib()
+    v = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())].index("rows128")
+    p = random_packed(K, N, g, dtype, seed=M + K)
+    dev = [to_dev(p["qweight"]), to_dev(p["qscales"], dtype), to_dev(p["qzeros"])]
+    xb = make_x(M, K, dtype, seed=M)
+    xd = to_dev(xb, dtype)
+    bias = np.linspace(-2, 2, N).astype(np.float32)
+    bd = to_dev(o.to_bits16(bias, dtype), dtype)
+    for split in (1, 3):
+        y = awq_gemm_variant(xd, *dev, v, split)
+        torch.cuda.synchronize()
+        _check(y, xb, p, dtype)
+        assert torch.equal(y, awq_gemm_variant(xd, *dev, v, split))
+        _check(awq_gemm_variant(xd, *dev, v, split, bias=bd), xb, p, dtype, o.to_dtype_f32(bias, dtype))
+    # the unpacked weight is awq_dequantize's, bit for bit: rows of the identity
+    n = min(M, K)
+    eye = torch.eye(n, K, device="cuda", dtype=xd.dtype)
+    assert torch.equal(awq_gemm_variant(eye, *dev, v, 1), nq.awq_dequantize(*dev)[:n])
+
+
+def test_gemm_rows128_routes():
+    """The default linear takes these tiles for a few hundred rows, with the bits of the forced variant; what they refuse, short
+    K and the plan of awq_gemm stay with the other kernels."""
+    L = _lib.lib()
+    names = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())]
+    v = names.index("rows128")
+    for M, K, N, g, split in ((333, 2816, 1304, 64, 5), (200, 2048, 2048, 128, 4)):
+        p = random_packed(K, N, g, "bf16", seed=9)
+        dev = [to_dev(p["qweight"]), to_dev(p["qscales"], "bf16"), to_dev(p["qzeros"])]
+        x = to_dev(make_x(M, K, "bf16", seed=10), "bf16")
+        y = nq.awq_gemm(x, *dev, 8)
+        assert any(torch.equal(y, awq_gemm_variant(x, *dev, v, s)) for s in range(1, 17)), (M, K, N)
+        assert L.awq_linear_workspace_bytes(M, N, K) >= L.awq_gemm_ex_workspace_bytes(M, N, K, v, split)
+    # groups of 16 rows end inside a wave's 32: an error, before anything is launched
+    args = (x.data_ptr(), dev[0].data_ptr(), dev[1].data_ptr(), dev[2].data_ptr(), None, y.data_ptr())
+    assert L.awq_gemm_ex(*args, M, N, K, 16, _lib.AWQ_BF16, None, 0, None, v, 1) != 0
+    assert b"group size" in L.awq_hip_last_error()
