@@ -85,6 +85,13 @@ size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t gr
 int awq_linear_dense(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
                      const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
                      int gated, void* scratch, size_t scratch_bytes, void* stream);
+/* y [M, N] = dtype(SiLU(x @ gate)) * (x @ up) for two weights [K, N] that lie apart: both are dequantised into `scratch` in one
+ * pass, interleaved, and multiplied as by awq_linear_dense with `gated`.  Scratch (and whether this is the faster way): as for
+ * awq_linear_dense with 2 N columns. */
+int awq_linear_dense_pair(const void* x, const int32_t* gate_qweight, const void* gate_qscales, const int32_t* gate_qzeros,
+                          const int32_t* up_qweight, const void* up_qscales, const int32_t* up_qzeros, void* y, int64_t M,
+                          int64_t N, int64_t K, int64_t group_size, int dtype, void* scratch, size_t scratch_bytes,
+                          void* stream);
 
 /* Bytes of device workspace awq_gemv / awq_gemm / awq_linear need for this
  * problem (0 is possible).  The workspace must be zero-filled ONCE when it is

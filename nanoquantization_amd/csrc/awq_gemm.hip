@@ -446,7 +446,7 @@ extern "C" int awq_dequantize_transposed(const int32_t* qweight, const void* qsc
                        (long long)K, (long long)group_size);
         return AWQ_ERR_UNSUPPORTED;
     }
-    const hipError_t e = awq::launch_dequant_transpose(dtype, qweight, qscales, qzeros, out, (int)N, (int)K,
+    const hipError_t e = awq::launch_dequant_transpose(dtype, {qweight, qscales, qzeros}, nullptr, out, (int)N, (int)K,
                                                        (int)group_size, reinterpret_cast<hipStream_t>(stream), 0, N);
     return e == hipSuccess ? AWQ_OK : awq::hip_fail(fn, e);
 }

@@ -145,6 +145,42 @@ extern "C" size_t awq_linear_dense_scratch_bytes(int64_t M, int64_t N, int64_t K
     return takes(M, N, K, group_size) ? (size_t)(std::min(slab_columns(N, K), N) * K * 2) : 0;
 }
 
+// `second`: the up weight beside `w`, the gate weight, N columns of each.
+static int dense_entry(const char* fn, const void* x, const PackedWeight& w, const PackedWeight* second, const void* bias, void* y,
+                       int64_t M, int64_t N, int64_t K, int64_t g, int dtype, bool gated, void* scratch, size_t scratch_bytes,
+                       void* stream) {
+    const int64_t cols_in_all = second ? 2 * N : N;
+    if (!takes(M, cols_in_all, K, g) || (gated && (bias || cols_in_all % 16 != 0))) {
+        set_error("%s: needs K %% 64 == 0, a group size of 8, 16, 32 or a multiple of 64, and for a gated product N %% 16 == 0 "
+                  "and no bias (M=%lld N=%lld K=%lld g=%lld)", fn, (long long)M, (long long)N, (long long)K, (long long)g);
+        return AWQ_ERR_UNSUPPORTED;
+    }
+    if ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(scratch)) & 15u) {
+        set_error("%s: bias and scratch must be 16-byte aligned", fn);
+        return AWQ_ERR_INVALID_ARG;
+    }
+    const size_t need = awq_linear_dense_scratch_bytes(M, cols_in_all, K, g);
+    if (!scratch || scratch_bytes < need) {
+        set_error("%s: scratch of %zu bytes needed, %zu given", fn, need, scratch ? scratch_bytes : (size_t)0);
+        return AWQ_ERR_WORKSPACE;
+    }
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const int64_t slab = slab_columns(cols_in_all, K);
+    const int xr = product_us(M, slab, K, 128) < product_us(M, slab, K, 256) ? 128 : 256;
+    for (int64_t n = 0; n < cols_in_all; n += slab) {
+        const int64_t cols = std::min(slab, cols_in_all - n), each = second ? 2 : 1;
+        hipError_t e = launch_dequant_transpose(dtype, w, second, scratch, (int)N, (int)K, (int)g, st, n / each, cols / each);
+        const void* b = bias ? static_cast<const uint16_t*>(bias) + n : nullptr;
+        void* out = static_cast<uint16_t*>(y) + (gated ? n / 2 : n);
+        const int ldy = (int)(gated ? cols_in_all / 2 : N);
+        if (e == hipSuccess)
+            e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated, st)
+                                 : launch_dense<BF16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated, st);
+        if (e != hipSuccess) return hip_fail(fn, e);
+    }
+    return AWQ_OK;
+}
+
 extern "C" int awq_linear_dense(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
                                 const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
                                 int gated, void* scratch, size_t scratch_bytes, void* stream) {
@@ -153,34 +189,21 @@ extern "C" int awq_linear_dense(const void* x, const int32_t* qweight, const voi
     take_prefetch_hint(&dropped);
     const int rc = check_linear_args(fn, x, qweight, qscales, qzeros, y, M, N, K, group_size, dtype);
     if (rc != AWQ_OK) return rc;
-    if (!takes(M, N, K, group_size) || (gated && (bias || N % 16 != 0))) {
-        set_error("%s: needs K %% 64 == 0, a group size of 8, 16, 32 or a multiple of 64, and for a gated product N %% 16 == 0 "
-                  "and no bias (M=%lld N=%lld K=%lld g=%lld)", fn, (long long)M, (long long)N, (long long)K,
-                  (long long)group_size);
-        return AWQ_ERR_UNSUPPORTED;
-    }
-    if ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(scratch)) & 15u) {
-        set_error("%s: bias and scratch must be 16-byte aligned", fn);
-        return AWQ_ERR_INVALID_ARG;
-    }
-    if (!scratch || scratch_bytes < awq_linear_dense_scratch_bytes(M, N, K, group_size)) {
-        set_error("%s: scratch of %zu bytes needed, %zu given", fn, awq_linear_dense_scratch_bytes(M, N, K, group_size),
-                  scratch ? scratch_bytes : (size_t)0);
-        return AWQ_ERR_WORKSPACE;
-    }
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const int64_t slab = slab_columns(N, K);
-    const int xr = product_us(M, slab, K, 128) < product_us(M, slab, K, 256) ? 128 : 256;
-    for (int64_t n = 0; n < N; n += slab) {
-        const int64_t cols = std::min(slab, N - n);
-        hipError_t e = launch_dequant_transpose(dtype, qweight, qscales, qzeros, scratch, (int)N, (int)K, (int)group_size, st, n, cols);
-        const void* b = bias ? static_cast<const uint16_t*>(bias) + n : nullptr;
-        void* out = static_cast<uint16_t*>(y) + (gated ? n / 2 : n);
-        const int ldy = (int)(gated ? N / 2 : N);
-        if (e == hipSuccess)
-            e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated != 0, st)
-                                 : launch_dense<BF16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated != 0, st);
-        if (e != hipSuccess) return hip_fail(fn, e);
-    }
-    return AWQ_OK;
+    return dense_entry(fn, x, {qweight, qscales, qzeros}, nullptr, bias, y, M, N, K, group_size, dtype, gated != 0, scratch,
+                       scratch_bytes, stream);
+}
+
+extern "C" int awq_linear_dense_pair(const void* x, const int32_t* gate_qweight, const void* gate_qscales,
+                                     const int32_t* gate_qzeros, const int32_t* up_qweight, const void* up_qscales,
+                                     const int32_t* up_qzeros, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size,
+                                     int dtype, void* scratch, size_t scratch_bytes, void* stream) {
+    const char* fn = "awq_linear_dense_pair";
+    PrefetchRegions dropped;
+    take_prefetch_hint(&dropped);
+    int rc = check_linear_args(fn, x, gate_qweight, gate_qscales, gate_qzeros, y, M, N, K, group_size, dtype);
+    if (rc == AWQ_OK) rc = check_linear_args(fn, x, up_qweight, up_qscales, up_qzeros, y, M, N, K, group_size, dtype);
+    if (rc != AWQ_OK) return rc;
+    const PackedWeight up(up_qweight, up_qscales, up_qzeros);
+    return dense_entry(fn, x, {gate_qweight, gate_qscales, gate_qzeros}, &up, nullptr, y, M, N, K, group_size, dtype, true, scratch,
+                       scratch_bytes, stream);
 }

@@ -218,9 +218,18 @@ hipError_t launch_gemm_regb(int dtype, const void* x, const int32_t* qweight, co
                             void* workspace, int split_k, bool tail_only, hipStream_t stream, int act = 0);
 
 // awq_gemm_pipe.hip: wt [count][K] = columns first .. first + count - 1 of the dequantised weight, transposed (K % 64 == 0,
-// group size a multiple of 64 or a divisor of 64 that is a multiple of 8; first % 8 == 0).
-hipError_t launch_dequant_transpose(int dtype, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
-                                    void* wt, int N, int K, int g, hipStream_t stream, int64_t first, int64_t count);
+// group size a multiple of 64 or a divisor of 64 that is a multiple of 8; first % 8 == 0).  With a second weight of the same
+// sizes wt is [2 count][K], eight columns of the one and eight of the other in turn (count % 8 == 0).
+struct PackedWeight {
+    const uint32_t* qweight;
+    const uint16_t* scales;
+    const uint32_t* qzeros;
+    PackedWeight(const int32_t* w, const void* s, const int32_t* z)
+        : qweight(reinterpret_cast<const uint32_t*>(w)), scales(reinterpret_cast<const uint16_t*>(s)),
+          qzeros(reinterpret_cast<const uint32_t*>(z)) {}
+};
+hipError_t launch_dequant_transpose(int dtype, const PackedWeight& w, const PackedWeight* second, void* wt, int N, int K, int g,
+                                    hipStream_t stream, int64_t first, int64_t count);
 
 // awq_gemm_dense.hip: estimated microseconds of awq_linear_dense, -1 where it does not take the sizes.
 double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g);

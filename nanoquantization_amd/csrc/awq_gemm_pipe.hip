@@ -351,12 +351,15 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_pipe_kernel(
 // a lane owns word column wc for 8 k rows (reads of 128 B per k row), writes its 8 x 8 values as eight 16-byte
 // chunks into an LDS tile [256 n][64 k], and the block leaves as full 128-byte rows.
 // HBM-bound: 0.52 B read + 2 B written per weight.
-template <typename T>
-__global__ __launch_bounds__(256) void dequant_transpose_kernel(const uint32_t* __restrict__ qweight,
-                                                                const uint16_t* __restrict__ scales,
-                                                                const uint32_t* __restrict__ qzeros,
+// PAIR: a second weight of the same sizes in grid z; the rows of the two alternate by eights, the first weight's in front.
+template <typename T, bool PAIR>
+__global__ __launch_bounds__(256) void dequant_transpose_kernel(PackedWeight first_weight, PackedWeight second_weight,
                                                                 uint16_t* __restrict__ wt, int N, int K, int g, int first,
                                                                 int count) {
+    const bool second = PAIR && blockIdx.z;
+    const uint32_t* __restrict__ qweight = second ? second_weight.qweight : first_weight.qweight;
+    const uint16_t* __restrict__ scales = second ? second_weight.scales : first_weight.scales;
+    const uint32_t* __restrict__ qzeros = second ? second_weight.qzeros : first_weight.qzeros;
     __shared__ u32x4 tile[256 * 8];   // [n][8 chunks of 8 k], chunk kc of row n at n*8 + (kc ^ ((n >> 3) & 7))
     const int tid = threadIdx.x, wc = tid & 31, rb = tid >> 5;
     const int words = N >> 3;
@@ -387,8 +390,9 @@ __global__ __launch_bounds__(256) void dequant_transpose_kernel(const uint32_t* 
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int n = j * 32 + (tid >> 3), kc = tid & 7;
+        const int row = PAIR ? (n0 + n) * 2 - (n & 7) + 8 * second : n0 + n;
         if (n0 + n < count)
-            *reinterpret_cast<u32x4*>(wt + (size_t)(n0 + n) * K + k0 + kc * 8) = tile[n * 8 + (kc ^ ((n >> 3) & 7))];
+            *reinterpret_cast<u32x4*>(wt + (size_t)row * K + k0 + kc * 8) = tile[n * 8 + (kc ^ ((n >> 3) & 7))];
     }
 }
 
@@ -497,18 +501,16 @@ hipError_t launch_gemm_pipe(int dtype, const void* x, const int32_t* qweight, co
                                          stream, act);
 }
 
-hipError_t launch_dequant_transpose(int dtype, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
-                                    void* wt, int N, int K, int g, hipStream_t stream, int64_t first, int64_t count) {
+hipError_t launch_dequant_transpose(int dtype, const PackedWeight& w, const PackedWeight* second, void* wt, int N, int K, int g,
+                                    hipStream_t stream, int64_t first, int64_t count) {
     (void)hipGetLastError();
-    const dim3 grid((unsigned)cdiv(count, 256), K / 64), block(256);
-    if (dtype == AWQ_F16)
-        hipLaunchKernelGGL(dequant_transpose_kernel<F16>, grid, block, 0, stream,
-                           reinterpret_cast<const uint32_t*>(qweight), reinterpret_cast<const uint16_t*>(qscales),
-                           reinterpret_cast<const uint32_t*>(qzeros), reinterpret_cast<uint16_t*>(wt), N, K, g, (int)first, (int)count);
-    else
-        hipLaunchKernelGGL(dequant_transpose_kernel<BF16>, grid, block, 0, stream,
-                           reinterpret_cast<const uint32_t*>(qweight), reinterpret_cast<const uint16_t*>(qscales),
-                           reinterpret_cast<const uint32_t*>(qzeros), reinterpret_cast<uint16_t*>(wt), N, K, g, (int)first, (int)count);
+    const dim3 grid((unsigned)cdiv(count, 256), K / 64, second ? 2 : 1), block(256);
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, stream, w, second ? *second : w, reinterpret_cast<uint16_t*>(wt), N, K, g,
+                           (int)first, (int)count);
+    };
+    if (dtype == AWQ_F16) second ? go(dequant_transpose_kernel<F16, true>) : go(dequant_transpose_kernel<F16, false>);
+    else second ? go(dequant_transpose_kernel<BF16, true>) : go(dequant_transpose_kernel<BF16, false>);
     return hipGetLastError();
 }
 

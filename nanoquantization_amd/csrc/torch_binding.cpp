@@ -9,7 +9,7 @@
 //   torch.ops.nanoquantization_amd.awq_linear_swiglu(x, qweight, qscales, qzeros) -> Tensor [M, N / 2]
 // and the steps between the linears of the Qwen3 modules (nanoquantization/layers/norm.py:18-32, layers/rope.py:24-45,
 // models/qwen3_quantized.py:79-99, 147-152), inference only (none has a derivative):
-//   rms_norm, silu_mul, qkv_norm_rope, causal_attention
+//   awq_swiglu_pair, rms_norm, silu_mul, qkv_norm_rope, causal_attention
 // with Meta kernels (shapes only), so the operators are visible to the dispatcher and to tracing.
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
@@ -252,6 +252,39 @@ at::Tensor silu_mul_op(const at::Tensor& gate, const at::Tensor& up) {
 }
 at::Tensor silu_mul_meta(const at::Tensor& gate, const at::Tensor&) { return at::empty(gate.sizes(), gate.options()); }
 
+// gate and up of an MLP that lie apart: one product where the rows are many, else two and the activation.
+at::Tensor awq_swiglu_pair_op(const at::Tensor& x, const at::Tensor& gate_qweight, const at::Tensor& gate_qscales,
+                              const at::Tensor& gate_qzeros, const at::Tensor& up_qweight, const at::Tensor& up_qscales,
+                              const at::Tensor& up_qzeros) {
+    Packed p = check_packed(gate_qweight, gate_qscales, gate_qzeros);
+    const Packed up = check_packed(up_qweight, up_qscales, up_qzeros);
+    TORCH_CHECK(p.K == up.K && p.N == up.N && p.g == up.g && p.dtype == up.dtype, "gate and up must be alike");
+    TORCH_CHECK(x.dim() == 2 && x.size(1) == p.K, "x must be [M, ", p.K, "], got ", x.sizes());
+    check_device(x, {&gate_qweight, &gate_qscales, &gate_qzeros, &up_qweight, &up_qscales, &up_qzeros});
+    const DeviceGuard guard(x.device());
+    const int64_t M = x.size(0);
+    p.N *= 2;
+    const at::Tensor scratch = M > 0 ? dense_scratch(x.device(), M, p) : at::Tensor();
+    if (!scratch.defined())
+        return silu_mul_op(awq_linear_op(x, gate_qweight, gate_qscales, gate_qzeros, c10::nullopt),
+                           awq_linear_op(x, up_qweight, up_qscales, up_qzeros, c10::nullopt));
+    const at::ScalarType dt = gate_qscales.scalar_type();
+    const at::Tensor xc = (x.scalar_type() == dt ? x : x.to(dt)).contiguous();
+    const at::Tensor gw = gate_qweight.contiguous(), gs = gate_qscales.contiguous(), gz = gate_qzeros.contiguous(),
+                     uw = up_qweight.contiguous(), us = up_qscales.contiguous(), uz = up_qzeros.contiguous();
+    at::Tensor out = at::empty({M, up.N}, gs.options());
+    check_status(awq_linear_dense_pair(xc.data_ptr(), gw.data_ptr<int32_t>(), gs.data_ptr(), gz.data_ptr<int32_t>(),
+                                       uw.data_ptr<int32_t>(), us.data_ptr(), uz.data_ptr<int32_t>(), out.data_ptr(), M, up.N, p.K,
+                                       p.g, p.dtype, scratch.data_ptr(), (size_t)scratch.numel(),
+                                       current_stream(x.device().index())),
+                 "awq_linear_dense_pair");
+    return out;
+}
+at::Tensor awq_swiglu_pair_meta(const at::Tensor& x, const at::Tensor&, const at::Tensor& gate_qscales, const at::Tensor&,
+                                const at::Tensor&, const at::Tensor&, const at::Tensor&) {
+    return at::empty({x.size(0), gate_qscales.size(1)}, gate_qscales.options());
+}
+
 using Three = std::tuple<at::Tensor, at::Tensor, at::Tensor>;
 
 Three qkv_outputs(const at::Tensor& q, int64_t heads, int64_t kv_heads) {
@@ -322,6 +355,8 @@ TORCH_LIBRARY(nanoquantization_amd, m) {
     m.def("awq_dequantize(Tensor qweight, Tensor qscales, Tensor qzeros) -> Tensor");
     m.def("awq_linear(Tensor x, Tensor qweight, Tensor qscales, Tensor qzeros, Tensor? bias=None) -> Tensor");
     m.def("awq_linear_swiglu(Tensor x, Tensor qweight, Tensor qscales, Tensor qzeros) -> Tensor");
+    m.def("awq_swiglu_pair(Tensor x, Tensor gate_qweight, Tensor gate_qscales, Tensor gate_qzeros, Tensor up_qweight, "
+          "Tensor up_qscales, Tensor up_qzeros) -> Tensor");
     m.def("rms_norm(Tensor x, Tensor weight, float eps) -> Tensor");
     m.def("silu_mul(Tensor gate, Tensor up) -> Tensor");
     m.def("qkv_norm_rope(Tensor q, Tensor k, Tensor v, Tensor q_weight, Tensor k_weight, Tensor cos_sin, Tensor positions, "
@@ -333,6 +368,7 @@ TORCH_LIBRARY_IMPL(nanoquantization_amd, CUDA, m) {   // the dispatch key of HIP
     m.impl("awq_dequantize", &awq_dequantize_op);
     m.impl("awq_linear", &awq_linear_op);
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_op);
+    m.impl("awq_swiglu_pair", &awq_swiglu_pair_op);
     m.impl("rms_norm", &rms_norm_op);
     m.impl("silu_mul", &silu_mul_op);
     m.impl("qkv_norm_rope", &qkv_norm_rope_op);
@@ -343,6 +379,7 @@ TORCH_LIBRARY_IMPL(nanoquantization_amd, Meta, m) {
     m.impl("awq_dequantize", &awq_dequantize_meta);
     m.impl("awq_linear", &awq_linear_meta);
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_meta);
+    m.impl("awq_swiglu_pair", &awq_swiglu_pair_meta);
     m.impl("rms_norm", &rms_norm_meta);
     m.impl("silu_mul", &silu_mul_meta);
     m.impl("qkv_norm_rope", &qkv_norm_rope_meta);

@@ -95,6 +95,13 @@ class Qwen3QuantizedMLP(nn.Module):
         self.down_proj = mk(intermediate_size, hidden_size)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        g, u = self.gate_proj, self.up_proj
+        if (type(g) is type(u) is WQLinear_GEMM and g.bias is None and u.bias is None and g.qweight.shape == u.qweight.shape
+                and g.qscales.shape == u.qscales.shape and x.shape[-1] == g.qweight.shape[0] and x.dim() > 1
+                and plain(x, g.qscales, u.qscales) and unhooked(g, u)):
+            act = _lib.torch_ops().awq_swiglu_pair(x.reshape(-1, x.shape[-1]), g.qweight, g.qscales, g.qzeros, u.qweight, u.qscales,
+                                                   u.qzeros)
+            return self.down_proj(act.view(*x.shape[:-1], act.shape[-1]))
         gate, up = self.gate_proj(x), self.up_proj(x)
         if gate.shape[-1] % 8 == 0 and plain(gate, up):
             return self.down_proj(_lib.torch_ops().silu_mul(gate, up))

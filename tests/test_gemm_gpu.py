@@ -439,3 +439,30 @@ def test_gemm_rows128_routes():
     args = (x.data_ptr(), dev[0].data_ptr(), dev[1].data_ptr(), dev[2].data_ptr(), None, y.data_ptr())
     assert L.awq_gemm_ex(*args, M, N, K, 16, _lib.AWQ_BF16, None, 0, None, v, 1) != 0
     assert b"group size" in L.awq_hip_last_error()
+
+
+# a row, columns past the last tile, an odd number of words, two slabs (131072 x 1040: 273 MB)
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,K,N,g", [(1, 64, 8, 64), (300, 192, 264, 32), (257, 256, 1024, 128), (30, 131072, 520, 128)])
+def test_linear_dense_pair(dtype, M, K, N, g):
+    """Gate and up that lie apart, in one product: the bits of two products and the activation."""
+    from nanoquantization_amd.engine import ops
+    print(f"linear dense pair {dtype} M={M} K={K} N={N} g={g}", flush=True)
+    tdt, L = torch.float16 if dtype == "f16" else torch.bfloat16, _lib.lib()
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    words = lambda r: torch.randint(-2 ** 31, 2 ** 31 - 1, (r, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    weights = [(words(K), (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 / K ** 0.5 * 8).to(tdt), words(K // g)) for _ in range(2)]
+    x = torch.randn(M, K, device="cuda", generator=gen).to(tdt)
+    scratch = torch.full((L.awq_linear_dense_scratch_bytes(M, 2 * N, K, g),), 0xFF, dtype=torch.uint8, device="cuda")   # NaN
+    tail = (M, N, K, g, _lib.dtype_id(tdt))
+    end = (scratch.data_ptr(), scratch.numel(), _lib.current_stream_ptr(x.device))
+    parts = []
+    for w in weights:
+        parts.append(torch.empty(M, N, dtype=tdt, device="cuda"))
+        _lib.check(L.awq_linear_dense(x.data_ptr(), *(t.data_ptr() for t in w), None, parts[-1].data_ptr(), *tail, 0, *end))
+    y = torch.empty(M, N, dtype=tdt, device="cuda")
+    scratch.fill_(0xFF)
+    _lib.check(L.awq_linear_dense_pair(x.data_ptr(), *(t.data_ptr() for w in weights for t in w), y.data_ptr(), *tail, *end))
+    assert torch.equal(y, _lib.torch_ops().silu_mul(*parts)) and not y.isnan().any()
+    got = _lib.torch_ops().awq_swiglu_pair(x, *weights[0], *weights[1])
+    assert (got.float() - y.float()).norm() <= 2.0 ** -7 * y.float().norm()
