@@ -144,12 +144,14 @@ def run_one(kind, K, N, M, dtype, iters, copies=1, g=G):
 
 
 def gemm_kernel_name(M, N, K, dtype_name, g=G):
-    """The kernel awq_gemm runs for a prefill problem, from the library's own plan."""
+    """The kernel nq.awq_gemm runs for a prefill problem, from the library's own rules."""
     import ctypes
     from nanoquantization_amd import _lib
     L = _lib.lib()
     v, sp = ctypes.c_int(), ctypes.c_int()
     did = _lib.AWQ_F16 if dtype_name == "f16" else _lib.AWQ_BF16
+    if L.awq_linear_dense_wanted_bytes(M, N, K, g):
+        return f"awq::dense_kernel<{'F16' if dtype_name == 'f16' else 'BF16'}> behind awq::dequant_transpose_kernel"
     if L.awq_gemm_plan(M, N, K, g, did, ctypes.byref(v), ctypes.byref(sp)) != 0:
         return "?"
     name = L.awq_gemm_variant_name(v.value).decode()
@@ -449,7 +451,8 @@ def main():
                                  "cases": large}
 
         # ---------------- extra: prefill GEMM, cfg3 -----------------------------------------------------
-        # the fused dequant + MFMA kernel: what awq_linear / WQLinear_GEMM.forward run at these row counts
+        # what WQLinear_GEMM.forward runs at these row counts: the weight dequantised first and a dense product, or the
+        # fused dequant + MFMA kernel
         bdt = torch.bfloat16
         fused = {}
         for (K, N) in ((4096, 12288), (12288, 4096)):
@@ -469,11 +472,9 @@ def main():
             "kernel": fused[best_case]["kernel"] + f" at {best_case} (each case names its own)", "bound": "mfma",
             "achieved": bestf,
             "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": bestf / MFMA_PEAK_TFLOPS,
-            "workload": "cfg3: Qwen3-8B MLP shapes, bf16, M in {512,2048,8192}; the fused dequant + MFMA kernel "
-                        "(default dispatch at every M)",
+            "workload": "cfg3: Qwen3-8B MLP shapes, bf16, M in {512,2048,8192}, default dispatch",
             "cases": fused}
-        # the same shapes in fp16 at the row counts whose work items fill the CUs: the default dispatch runs the
-        # kernel with resident workgroups that builds its B operands in registers there (awq::gemm_regb_kernel)
+        # the same shapes in fp16 at the row counts whose work items fill the CUs
         hdt = torch.float16
         fused16 = {}
         for (K, N) in ((4096, 12288), (12288, 4096)):

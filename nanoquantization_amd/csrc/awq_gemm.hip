@@ -375,8 +375,8 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
         set_error("%s: bad variant %d / split_k %d", fn, variant, split_k);
         return AWQ_ERR_INVALID_ARG;
     }
-    if (act && (bias || N % 16 != 0 || !is_tile256(variant))) {
-        set_error("%s: the gated epilogue takes no bias, needs N %% 16 == 0 and runs on the pipelined kernel", fn);
+    if (act && (bias || N % 16 != 0 || !(is_tile256(variant) || variant == kRowsVariant))) {
+        set_error("%s: the gated epilogue takes no bias, needs N %% 16 == 0 and runs on the 256 x 256 and 128-row tiles", fn);
         return AWQ_ERR_UNSUPPORTED;
     }
     const RowsPlan rows = variant == kRowsVariant ? make_rows_plan(M, N, K, g, split_k) : RowsPlan{};
@@ -411,7 +411,7 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
         AWQ_GEMM_CASE(k64x256, 64, 256, 1, 4)
         AWQ_GEMM_CASE(k32x256, 32, 256, 1, 4)
         case kRowsVariant:
-            e = launch_rows(rows, dtype, x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K, (int)g, workspace, s);
+            e = launch_rows(rows, dtype, x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K, (int)g, workspace, act != 0, s);
             break;
         case kPipeVariant:
         case kPipeTailVariant:
@@ -570,7 +570,9 @@ extern "C" size_t awq_linear_swiglu_workspace_bytes(int64_t M, int64_t N, int64_
     int v, s;
     awq::plan_gemm_tile256(M, N, K, 128, AWQ_F16, &v, &s);   // the workspace is the same for both 256 x 256 kernels
     const size_t b = awq::gemm_ws_bytes(M, N, K, v, s);
-    return a > b ? a : b;
+    awq::RowsPlan rows;
+    const size_t d = rows_wanted(M, N, K, 32, &rows) ? awq::rows_ws_bytes(rows, M, N) : 0, most = a > b ? a : b;
+    return most > d ? most : d;
 }
 
 extern "C" int awq_linear_swiglu(const void* x, const int32_t* qweight, const void* qscales,
@@ -584,6 +586,9 @@ extern "C" int awq_linear_swiglu(const void* x, const int32_t* qweight, const vo
     int v = awq::kPipeVariant, s = 1;
     if (K >= awq::kBK && N >= 16 && M >= 1 && group_size > 0)
         awq::plan_gemm_tile256(M, N, K, group_size, dtype, &v, &s);
+    awq::RowsPlan rows;       // as awq_linear on the same sizes, whose bits the gated product has
+    if (M > 128 && N >= 16 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, &rows))
+        v = awq::kRowsVariant, s = rows.splits;
     return awq::gemm_dispatch("awq_linear_swiglu", x, qweight, qscales, qzeros, nullptr, y, M, N, K, group_size,
                               dtype, workspace, workspace_bytes, stream, v, s, 1);
 }

@@ -86,6 +86,15 @@ __device__ __forceinline__ void swiglu_pair_store(u32x4 mine, u32x4 other, bool 
     *reinterpret_cast<u32x2*>(dst + (odd ? 4 : 0)) = u32x2{o[0], o[1]};
 }
 
+// The same for a lane that holds word `word` of a row of y (gate words even, up words odd, in neighbouring lanes).
+template <typename T>
+__device__ __forceinline__ void swiglu_word_store(u32x4 mine, uint16_t* __restrict__ row, int word) {
+    u32x4 other;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) other[i] = (uint32_t)__shfl_xor((int)mine[i], 1);
+    swiglu_pair_store<T>(mine, other, word & 1, row + (size_t)(word >> 1) * 8);
+}
+
 // acc[a][b][v] of the 32x32x16 MFMA: row (v/4)*8 + (lane/32)*4 + v%4, column lane%32 of tile
 // (a, b) of the wave's sub-tile at (wm0, wn0).
 template <typename T, int BM, int BN, int TM, int TN, int NT>
@@ -121,7 +130,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ partials,
                                                                  const uint16_t* __restrict__ bias,
                                                                  uint16_t* __restrict__ y, int64_t M, int N,
-                                                                 int splits) {
+                                                                 int splits, bool gated) {
     const int64_t vec = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int per_row = N >> 3;
     if (vec >= M * per_row) return;
@@ -156,20 +165,21 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
     u32x4 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[i] = T::pack2(out[2 * i], out[2 * i + 1]);
-    *reinterpret_cast<u32x4*>(y + (size_t)m * N + nn) = o;
+    if (gated) swiglu_word_store<T>(o, y + (size_t)m * (N >> 1), nn >> 3);
+    else *reinterpret_cast<u32x4*>(y + (size_t)m * N + nn) = o;
 }
 
 // Launches the reduction pass on `stream` (after the product kernel that wrote `partials`).
 inline hipError_t launch_splitk_reduce(int dtype, const float* partials, const void* bias, void* y, int64_t M, int N,
-                                       int splits, hipStream_t stream) {
+                                       int splits, hipStream_t stream, bool gated = false) {
     const int64_t vecs = M * (N >> 3);
     const dim3 grid((unsigned)cdiv(vecs, 256)), block(256);
     if (dtype == AWQ_F16)
         gemm_splitk_reduce_kernel<F16><<<grid, block, 0, stream>>>(partials, reinterpret_cast<const uint16_t*>(bias),
-                                                                   reinterpret_cast<uint16_t*>(y), M, N, splits);
+                                                                   reinterpret_cast<uint16_t*>(y), M, N, splits, gated);
     else
         gemm_splitk_reduce_kernel<BF16><<<grid, block, 0, stream>>>(partials, reinterpret_cast<const uint16_t*>(bias),
-                                                                    reinterpret_cast<uint16_t*>(y), M, N, splits);
+                                                                    reinterpret_cast<uint16_t*>(y), M, N, splits, gated);
     return hipGetLastError();
 }
 
@@ -246,6 +256,6 @@ inline size_t rows_ws_bytes(const RowsPlan& p, int64_t M, int64_t N) {
 }
 hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_t* qweight, const void* qscales,
                        const int32_t* qzeros, const void* bias, void* y, int M, int N, int K, int g, void* workspace,
-                       hipStream_t st);
+                       bool gated, hipStream_t st);   // gated: as PipePlan::act
 
 }  // namespace awq

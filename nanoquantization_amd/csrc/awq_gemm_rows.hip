@@ -98,7 +98,7 @@ template <typename T, int MT>
 __device__ __forceinline__ void rows_tile(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales,
     const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-    float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits) {
+    float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
     constexpr int kStage = stage_bytes(MT);
     // runs of consecutive items to each XCD: the row tiles of a column tile read its words through one L2
@@ -336,7 +336,8 @@ __device__ __forceinline__ void rows_tile(
         u32x4 o;
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = T::pack2(v[2 * i], v[2 * i + 1]);
-        *reinterpret_cast<u32x4*>(y + (size_t)m * N + 8 * (size_t)wc) = o;
+        if (gated) swiglu_word_store<T>(o, y + (size_t)m * (N >> 1), wc);
+        else *reinterpret_cast<u32x4*>(y + (size_t)m * N + 8 * (size_t)wc) = o;
     }
 }
 
@@ -344,13 +345,13 @@ template <typename T, int MT>
 __global__ __launch_bounds__(kThreads, 2) void rows_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales,
     const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-    float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits) {
-    rows_tile<T, MT>(x, qweight, scales, qzeros, bias, y, partials, M, N, K, g, m_tiles, items, steps_per_split, splits);
+    float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
+    rows_tile<T, MT>(x, qweight, scales, qzeros, bias, y, partials, M, N, K, g, m_tiles, items, steps_per_split, splits, gated);
 }
 
 template <typename T, int MT>
 hipError_t launch(const RowsPlan& p, const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
-                  const void* bias, void* y, float* partials, int M, int N, int K, int g, hipStream_t st) {
+                  const void* bias, void* y, float* partials, int M, int N, int K, int g, bool gated, hipStream_t st) {
     auto kern = rows_kernel<T, MT>;
     static bool raised = false;      // once per process and instantiation
     if (!raised) {
@@ -363,7 +364,7 @@ hipError_t launch(const RowsPlan& p, const void* x, const int32_t* qweight, cons
     const int items = p.m_tiles * p.n_tiles * p.splits;
     kern<<<dim3((unsigned)(cdiv(items, 8) * 8)), dim3(kThreads), lds_bytes(MT), st>>>(
         (const uint16_t*)x, (const uint32_t*)qweight, (const uint16_t*)qscales, (const uint32_t*)qzeros, (const uint16_t*)bias,
-        (uint16_t*)y, partials, M, N, K, g, p.m_tiles, items, p.steps_per_split, p.splits);
+        (uint16_t*)y, partials, M, N, K, g, p.m_tiles, items, p.steps_per_split, p.splits, gated);
     return hipGetLastError();
 }
 
@@ -396,10 +397,10 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int split_k)
 
 hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_t* qweight, const void* qscales,
                        const int32_t* qzeros, const void* bias, void* y, int M, int N, int K, int g, void* workspace,
-                       hipStream_t st) {
+                       bool gated, hipStream_t st) {
     float* partials = p.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kCounterBytes) : nullptr;
 #define AWQ_ROWS(T, MT) \
-    if (p.mt == MT) e = launch<T, MT>(p, x, qweight, qscales, qzeros, bias, y, partials, M, N, K, g, st);
+    if (p.mt == MT) e = launch<T, MT>(p, x, qweight, qscales, qzeros, bias, y, partials, M, N, K, g, gated, st);
     hipError_t e = hipErrorInvalidValue;
     if (dtype == AWQ_F16) {
         AWQ_ROWS(F16, 5) AWQ_ROWS(F16, 6) AWQ_ROWS(F16, 7) AWQ_ROWS(F16, 8)
@@ -408,7 +409,7 @@ hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_
     }
 #undef AWQ_ROWS
     if (e != hipSuccess || p.splits == 1) return e;
-    return launch_splitk_reduce(dtype, partials, bias, y, M, N, p.splits, st);
+    return launch_splitk_reduce(dtype, partials, bias, y, M, N, p.splits, st, gated);
 }
 
 }  // namespace awq

@@ -25,7 +25,7 @@ import torch
 import torch.nn.functional as F
 
 from ..layers.gemm import _linear, prefetch_hint
-from . import ops
+from . import hybrid_ops, ops
 from .cache import Lease, PagedKVCache
 from .core import EngineCore
 from ..models.qwen3_quantized import Qwen3QuantizedForCausalLM
@@ -78,15 +78,29 @@ class LLMEngine(EngineCore):
             max_batch, o0.out_features, o0.in_features, o0.group_size)
         self.down_add_norm = d0.bias is None and ops.gemv_add_rmsnorm_supported(
             max_batch, d0.out_features, d0.in_features, d0.group_size)
+        # prompts through the cache on the prompt attention kernel, which has matrix forms for these rows
+        self.paged_prefill = self.dtype == torch.bfloat16 and self.hd in (32, 64, 96, 128, 192, 256)
         self.eps = layers[0].input_layernorm.eps
         self.scale = float(self.hd) ** -0.5
 
     # ---- prefill: full causal attention over the prompt itself ------------------------------------
+    def _prompt_layout(self, lens: List[int], leases: List[Lease]) -> Optional[hybrid_ops.PromptPass]:
+        bs = self.block_size
+        return (hybrid_ops.PromptPass([(0, n, l.blocks[:(n + bs - 1) // bs], 0) for n, l in zip(lens, leases)], bs, self.device)
+                if self.paged_prefill else None)
+
+    def _prompt_attention(self, li: int, qkv: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,
+                          layout: hybrid_ops.PromptPass) -> torch.Tensor:
+        attn, k, v = self.model.model.layers[li].self_attn, self.cache.k[li], self.cache.v[li]
+        q = ops.qk_norm_rope_store(qkv, attn.q_norm.weight, attn.k_norm.weight, attn.rope.cos_sin_cache, positions, slots, k, v,
+                                   self.nh, self.nkv, self.hd, attn.q_norm.eps)
+        return hybrid_ops.attention_prefill(q, k, v, layout, self.hd, self.hd, self.scale)
+
     @torch.no_grad()
     def _prefill(self, ids: torch.Tensor, leases: List[Lease]) -> torch.Tensor:
         """ids: [b, s] (equal-length prompts). Returns the next token of every sequence [b].  Same kernels as
         the decode step around the AWQ linears (which take the MFMA GEMM at these row counts); the causal
-        attention over the prompt is torch's scaled_dot_product_attention."""
+        attention over the prompt reads the cache it has just written (torch's scaled_dot_product_attention in float16)."""
         b, s = ids.shape
         m, bs, eps = self.model.model, self.block_size, self.eps
         pos = torch.arange(s, device=self.device).unsqueeze(0).expand(b, s)
@@ -95,20 +109,24 @@ class LLMEngine(EngineCore):
         pos_flat = pos.reshape(-1).contiguous()
         gqa = self.nh != self.nkv
         kvw = self.nkv * self.hd
+        layout = self._prompt_layout([s] * b, leases)
         x = m.embed_tokens(ids).reshape(b * s, -1)                       # residual stream [b*s, hidden]
         delta = None
         for li, layer in enumerate(m.layers):
             attn = layer.self_attn
             h = ops.add_rmsnorm(x, delta, layer.input_layernorm.weight, eps)
             qkv = self.qkv[li](h)
-            q, k = ops.qk_norm_rope_store(qkv, attn.q_norm.weight, attn.k_norm.weight, attn.rope.cos_sin_cache,
-                                          pos_flat, slots, self.cache.k[li], self.cache.v[li], self.nh, self.nkv,
-                                          self.hd, attn.q_norm.eps, dense_k=True)
-            v = qkv[:, -kvw:].view(b, s, self.nkv, self.hd)
-            o = F.scaled_dot_product_attention(q.view(b, s, self.nh, self.hd).transpose(1, 2),
-                                               k.view(b, s, self.nkv, self.hd).transpose(1, 2), v.transpose(1, 2),
-                                               is_causal=True, enable_gqa=gqa)
-            o = o.transpose(1, 2).reshape(b * s, self.nh * self.hd)
+            if layout is not None:
+                o = self._prompt_attention(li, qkv, pos_flat, slots, layout)
+            else:
+                q, k = ops.qk_norm_rope_store(qkv, attn.q_norm.weight, attn.k_norm.weight, attn.rope.cos_sin_cache,
+                                              pos_flat, slots, self.cache.k[li], self.cache.v[li], self.nh, self.nkv,
+                                              self.hd, attn.q_norm.eps, dense_k=True)
+                v = qkv[:, -kvw:].view(b, s, self.nkv, self.hd)
+                o = F.scaled_dot_product_attention(q.view(b, s, self.nh, self.hd).transpose(1, 2),
+                                                   k.view(b, s, self.nkv, self.hd).transpose(1, 2), v.transpose(1, 2),
+                                                   is_causal=True, enable_gqa=gqa)
+                o = o.transpose(1, 2).reshape(b * s, self.nh * self.hd)
             h = ops.add_rmsnorm(x, attn.o_proj(o), layer.post_attention_layernorm.weight, eps)
             act = (ops.awq_linear_swiglu(h, *self.gate_up_il[li]) if self.swiglu_ok
                    else ops.silu_mul(self.gate_up[li](h)))
@@ -140,23 +158,27 @@ class LLMEngine(EngineCore):
         slots = torch.cat(slot_list).contiguous()
         gqa = self.nh != self.nkv
         kvw = self.nkv * self.hd
+        layout = self._prompt_layout(lens, leases)
         x = m.embed_tokens(ids)                                          # residual stream [total, hidden]
         delta = None
         for li, layer in enumerate(m.layers):
             attn = layer.self_attn
             h = ops.add_rmsnorm(x, delta, layer.input_layernorm.weight, eps)
             qkv = self.qkv[li](h)
-            q, k = ops.qk_norm_rope_store(qkv, attn.q_norm.weight, attn.k_norm.weight, attn.rope.cos_sin_cache,
-                                          pos_flat, slots, self.cache.k[li], self.cache.v[li], self.nh, self.nkv,
-                                          self.hd, attn.q_norm.eps, dense_k=True)
-            v = qkv[:, -kvw:].view(total, self.nkv, self.hd)
-            o = torch.empty(total, self.nh * self.hd, dtype=self.dtype, device=dev)
-            for a, n in zip(starts, lens):
-                oi = F.scaled_dot_product_attention(q[a:a + n].transpose(0, 1).unsqueeze(0),
-                                                    k[a:a + n].transpose(0, 1).unsqueeze(0),
-                                                    v[a:a + n].transpose(0, 1).unsqueeze(0),
-                                                    is_causal=True, enable_gqa=gqa)
-                o[a:a + n] = oi[0].transpose(0, 1).reshape(n, self.nh * self.hd)
+            if layout is not None:
+                o = self._prompt_attention(li, qkv, pos_flat, slots, layout)
+            else:
+                q, k = ops.qk_norm_rope_store(qkv, attn.q_norm.weight, attn.k_norm.weight, attn.rope.cos_sin_cache,
+                                              pos_flat, slots, self.cache.k[li], self.cache.v[li], self.nh, self.nkv,
+                                              self.hd, attn.q_norm.eps, dense_k=True)
+                v = qkv[:, -kvw:].view(total, self.nkv, self.hd)
+                o = torch.empty(total, self.nh * self.hd, dtype=self.dtype, device=dev)
+                for a, n in zip(starts, lens):
+                    oi = F.scaled_dot_product_attention(q[a:a + n].transpose(0, 1).unsqueeze(0),
+                                                        k[a:a + n].transpose(0, 1).unsqueeze(0),
+                                                        v[a:a + n].transpose(0, 1).unsqueeze(0),
+                                                        is_causal=True, enable_gqa=gqa)
+                    o[a:a + n] = oi[0].transpose(0, 1).reshape(n, self.nh * self.hd)
             h = ops.add_rmsnorm(x, attn.o_proj(o), layer.post_attention_layernorm.weight, eps)
             act = (ops.awq_linear_swiglu(h, *self.gate_up_il[li]) if self.swiglu_ok
                    else ops.silu_mul(self.gate_up[li](h)))

@@ -25,6 +25,6 @@ class RMSNorm(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # a workgroup per row: rows of a few hundred elements (the heads') leave most of it idle
         n = self.weight.numel()
-        if 512 <= n <= 8192 and n % 8 == 0 and x.shape[-1:] == self.weight.shape and plain(x, self.weight):
+        if type(self) is RMSNorm and 512 <= n <= 8192 and n % 8 == 0 and x.shape[-1:] == self.weight.shape and plain(x, self.weight):
             return _lib.torch_ops().rms_norm(x, self.weight, self.eps)
         return self.rms_norm(x)
