@@ -126,7 +126,7 @@ def torch_binding_compile_cmd(obj: str) -> list[str]:
 def torch_binding_link_cmd(obj: str) -> list[str]:
     _, libdir, _ = _torch_dirs()
     return [CXX, "-shared", "-fPIC", obj, "-o", TORCH_LIB_PATH, f"-L{libdir}", "-ltorch", "-ltorch_cpu", "-lc10",
-            "-lc10_hip", "-ltorch_hip", f"-L{PKG_DIR}", "-lawq_hip", "-lnq_hybrid", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{libdir}"]
+            "-lc10_hip", "-ltorch_hip", f"-L{PKG_DIR}", "-lawq_hip", "-ldl", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{libdir}"]
 
 
 if __name__ == "__main__":
