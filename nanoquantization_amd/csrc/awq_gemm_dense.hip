@@ -24,7 +24,7 @@ __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restric
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
     using P = PingPong<T, XR>;
     int xt, nt;
-    if (!xcd_tile(x_tiles, w_tiles, xt, nt)) return;
+    if (!xcd_tile((int)blockIdx.x, x_tiles, w_tiles, xt, nt)) return;
     P p;
     const int m0 = xt * XR, n0 = nt * (GATED ? 128 : 256), out_cols = GATED ? cols / 2 : cols;
     const uint32_t row_bytes = (uint32_t)K * 2;

@@ -352,7 +352,7 @@ __global__ __launch_bounds__(512, 2) void moe_pingpong_kernel(const uint16_t* __
     using P = awq::PingPong<Bf, XR>;
     constexpr int kCols = GATED ? 128 : 256;
     int tile, group;
-    if (!awq::xcd_tile(tiles[3 * max_tiles], n_groups, tile, group)) return;
+    if (!awq::xcd_tile((int)blockIdx.x, tiles[3 * max_tiles], n_groups, tile, group)) return;
     const int e = tiles[tile], first = tiles[max_tiles + tile], count = tiles[2 * max_tiles + tile];
     const int n0 = group * kCols;
     const uint32_t row_bytes = (uint32_t)n_in * 2, w_bytes = (GATED ? 2 : 1) * (uint32_t)n_out * row_bytes;

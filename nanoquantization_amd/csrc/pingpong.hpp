@@ -215,13 +215,17 @@ struct PingPong {
 };
 
 // Workgroups go round-robin over the 8 XCDs, each with its own L2: every XCD takes a contiguous run of the tiles, in blocks
-// of 8 x tiles with the weight tiles outside, so that both operands are met again in that L2.  Grid: tiles rounded up to a
-// multiple of 8; false for the workgroups beyond the last tile.
-__device__ __forceinline__ bool xcd_tile(int x_tiles, int w_tiles, int& xt, int& wt) {
+// of 8 x tiles with the weight tiles outside, so that both operands are met again in that L2.  Any grid of a multiple of 8
+// that has a workgroup per tile; false for the workgroups that get none.  (`workgroup`: blockIdx.x, an argument so that the
+// host can enumerate the map.)
+__host__ __device__ __forceinline__ bool xcd_tile(int workgroup, int x_tiles, int w_tiles, int& xt, int& wt) {
     const int total = x_tiles * w_tiles, per = (total + 7) >> 3;
-    const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    // past the end of its XCD's run: in a larger grid the sum below would be a tile of the next XCD's
+    if (workgroup >> 3 >= per) return false;
+    const int id = (workgroup & 7) * per + (workgroup >> 3);
     if (id >= total) return false;
-    const int block = id / (8 * w_tiles), in_block = id - block * 8 * w_tiles, rows = min(8, x_tiles - 8 * block);
+    const int block = id / (8 * w_tiles), in_block = id - block * 8 * w_tiles;
+    const int rows = x_tiles - 8 * block < 8 ? x_tiles - 8 * block : 8;
     xt = 8 * block + in_block % rows;
     wt = in_block / rows;
     return true;
