@@ -31,20 +31,23 @@ __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restric
     uint32_t vw[4], vx[P::kXLoads];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int r = p.w_row(q);
+        const int r = P::w_row(q, p.wave, p.lane);
         int col = n0 + r;
         if (GATED) {
             const int c = n0 + r / (2 * P::kHalf) * P::kHalf + r % P::kHalf;
             col = 16 * (c >> 3) + (c & 7) + 8 * (r / P::kHalf & 1);
         }
-        vw[q] = (uint32_t)col * row_bytes + p.piece_bytes(r);
+        vw[q] = P::source(col, cols, row_bytes, r, p.lane);
     }
+    const int rows = min(XR, M - m0);
 #pragma unroll
-    for (int q = 0; q < P::kXLoads; ++q) vx[q] = (uint32_t)p.x_row(q) * row_bytes + p.piece_bytes(p.x_row(q));
-    // rows past the end of either operand read zeros
+    for (int q = 0; q < P::kXLoads; ++q) {
+        const int r = P::x_row(q, p.wave, p.lane);
+        vx[q] = P::source(r, rows, row_bytes, r, p.lane);
+    }
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wt), 0, cols * row_bytes, 0x00020000);
     const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (size_t)m0 * K, 0,
-                                                      min(XR, M - m0) * row_bytes, 0x00020000);
+                                                      rows * row_bytes, 0x00020000);
     p.run(s_mem, rw, vw, rx, vx, K / P::kStage);
     const auto store = [&](int r, int c, u32x4 v) {
         if (m0 + r < M && n0 + c < out_cols) *reinterpret_cast<u32x4*>(y + (size_t)(m0 + r) * ldy + n0 + c) = v;

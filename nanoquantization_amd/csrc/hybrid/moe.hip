@@ -347,7 +347,7 @@ __global__ __launch_bounds__(512, 2) void moe_pingpong_kernel(const uint16_t* __
                                                               const int32_t* __restrict__ order,
                                                               const int32_t* __restrict__ tiles, uint16_t* __restrict__ out,
                                                               int max_tiles, int top, int n_out, int n_in, int n_groups,
-                                                              uint32_t in_bytes) {
+                                                              int in_rows) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_stage[];
     using P = awq::PingPong<Bf, XR>;
     constexpr int kCols = GATED ? 128 : 256;
@@ -360,19 +360,19 @@ __global__ __launch_bounds__(512, 2) void moe_pingpong_kernel(const uint16_t* __
     uint32_t vw[4], vx[P::kXLoads];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int r = p.w_row(q);
-        int row = n0 + r;
+        const int r = P::w_row(q, p.wave, p.lane);
+        int row = min(n0 + r, n_out - 1);
         if (GATED) row = min(n0 + r / (2 * P::kHalf) * P::kHalf + r % P::kHalf, n_out - 1) + (r / P::kHalf & 1) * n_out;
-        vw[q] = (uint32_t)row * row_bytes + p.piece_bytes(r);
+        vw[q] = P::source(row, (GATED ? 2 : 1) * n_out, row_bytes, r, p.lane);
     }
 #pragma unroll
     for (int q = 0; q < P::kXLoads; ++q) {
-        const int r = p.x_row(q), place = first + min(r, count - 1);
-        vx[q] = (uint32_t)(GATED ? order[place] / top : place) * row_bytes + p.piece_bytes(r);
+        const int r = P::x_row(q, p.wave, p.lane), place = first + min(r, count - 1);
+        vx[q] = P::source(GATED ? order[place] / top : place, in_rows, row_bytes, r, p.lane);
     }
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w) + (int64_t)e * (GATED ? 2 : 1) * n_out * n_in, 0,
                                                       w_bytes, 0x00020000);
-    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(in), 0, in_bytes, 0x00020000);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(in), 0, (uint32_t)in_rows * row_bytes, 0x00020000);
     p.run(s_stage, rw, vw, rx, vx, n_in / P::kStage);
     if constexpr (GATED) {
         float score[P::NJ];
@@ -409,7 +409,7 @@ void launch_pingpong(const uint16_t* in, const uint16_t* w, const float* weight,
     }
     const int64_t groups = cdiv(n_out, GATED ? 128 : 256);
     kern<<<dim3((unsigned)(cdiv(max_tiles * groups, 8) * 8)), dim3(P::kThreads), P::kLds, st>>>(
-        in, w, weight, order, tiles, out, max_tiles, top, n_out, n_in, (int)groups, (uint32_t)(in_rows * n_in * 2));
+        in, w, weight, order, tiles, out, max_tiles, top, n_out, n_in, (int)groups, (int)in_rows);
 }
 
 enum class MoeForm { simple, skinny16, skinny32, skinny64, gemm64, gemm128, pingpong128, pingpong256 };

@@ -40,24 +40,30 @@ struct PingPong {
         lo = lane & 15, hi = lane >> 4, wm = wave % kWM, wn = wave / kWM;
     }
 
-    // Rows of the tile that load q of a stage brings for this lane, eight lanes a row, and the 16-byte piece of the stage's
+    // Rows of the tile that load q of a stage brings for a lane, eight lanes a row, and the 16-byte piece of the stage's
     // 128 bytes: pieces are stored at position piece ^ (row / 2 % 8), which spreads the 16 rows of an operand read over all
     // banks; load-to-LDS writes linearly, so the swizzle is in the source addresses.
-    __device__ __forceinline__ int w_row(int q) const { return 64 * q + 8 * wave + (lane >> 3); }     // q < 4
-    __device__ __forceinline__ int x_row(int q) const {                                                // q < kXLoads
+    static __host__ __device__ __forceinline__ int w_row(int q, int wave, int lane) { return 64 * q + 8 * wave + (lane >> 3); }     // q < 4
+    static __host__ __device__ __forceinline__ int x_row(int q, int wave, int lane) {                                                // q < kXLoads
         // XR = 256: loads 0 and 2 bring the first 32 rows of every wave's 64, loads 1 and 3 the others
         if (XR == 256) return 64 * ((q & 2) + (wave >> 2)) + 32 * (q & 1) + 8 * (wave & 3) + (lane >> 3);
         return 64 * q + 8 * wave + (lane >> 3);
     }
-    __device__ __forceinline__ int piece_bytes(int row) const { return ((lane & 7) ^ ((row >> 1) & 7)) * 16; }
+    // Byte offset in an operand of `rows` rows of the piece that comes to `tile_row` from source row `row`: past the end the
+    // last row again, of which nothing is stored.
+    static __host__ __device__ __forceinline__ uint32_t source(int row, int rows, uint32_t row_bytes, int tile_row, int lane) {
+        return (uint32_t)(row < rows ? row : rows - 1) * row_bytes + ((lane & 7) ^ ((tile_row >> 1) & 7)) * 16;
+    }
+    // Byte offset of stage t in a row.  The pipeline asks for two stages past the last one, which nobody reads: the last one
+    // again.  With `source` no request leaves an operand; the count of requests, which the waits rely on, stays.
+    static __host__ __device__ __forceinline__ int stage_bytes(int t, int steps) { return (t < steps ? t : steps - 1) * (kStage * 2); }
 
-    // vw[q], vx[q]: byte offsets of this lane's piece of its rows in the buffers rw and rx (row offset + piece_bytes(row)).
-    // Stages past the last one are asked for as well and never used: what lies behind a row, or the buffers' zeros.
+    // vw[q], vx[q]: `source` of this lane's piece of its rows in the buffers rw and rx.
     __device__ __forceinline__ void run(unsigned char* s_mem, __amdgpu_buffer_rsrc_t rw, const uint32_t (&vw)[4],
                                         __amdgpu_buffer_rsrc_t rx, const uint32_t (&vx)[kXLoads], int steps) {
         const auto load = [&](__amdgpu_buffer_rsrc_t r, uint32_t v, int first_row, int at, int t) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(s_mem + at + first_row * 128),
-                                                     16, v, t * (kStage * 2), 0, 0);
+                                                     16, v, stage_bytes(t, steps), 0, 0);
         };
         const auto load_w = [&](int q, int t, int at) { load(rw, vw[q], 64 * q + 8 * wave, at, t); };
         const auto load_x = [&](int q, int t, int at) {

@@ -38,7 +38,35 @@ static int tiles() {
     return 0;
 }
 
-int main() { return tiles(); }
+// Every request of a tile, those for stages past the last one included, lies inside its operand: `rows` rows of `steps`
+// stages, of which the tile begins at row `first` (the rows behind the last one come from it).
+template <int XR>
+static int requests() {
+    using P = awq::PingPong<awq::BF16, XR>;
+    for (int steps : {1, 2, 3, 5})
+        for (int rows : {1, 2, 8, 31, XR - 1, XR, XR + 1, 3 * XR})
+            for (int first = 0; first < rows; first += XR)
+                for (int wave = 0; wave < 8; ++wave)
+                    for (int lane = 0; lane < 64; ++lane)
+                        for (int t = 0; t < steps + 2; ++t) {
+                            const uint32_t row_bytes = steps * P::kStage * 2, size = rows * row_bytes;
+                            const uint32_t stage = P::stage_bytes(t, steps);
+                            if (t < steps && stage != (uint32_t)t * P::kStage * 2) return fail("wrong stage", t, steps, stage, XR);
+                            for (int q = 0; q < 4; ++q) {
+                                const int r = P::w_row(q, wave, lane);
+                                const uint32_t at = P::source(first + r, rows, row_bytes, r, lane) + stage;
+                                if (r < 0 || r >= P::kWR || at + 16 > size) return fail("weight request", rows, steps, t, at);
+                            }
+                            for (int q = 0; q < P::kXLoads; ++q) {
+                                const int r = P::x_row(q, wave, lane);
+                                const uint32_t at = P::source(first + r, rows, row_bytes, r, lane) + stage;
+                                if (r < 0 || r >= XR || at + 16 > size) return fail("x request", rows, steps, t, at);
+                            }
+                        }
+    return 0;
+}
+
+int main() { return tiles() || requests<128>() || requests<256>(); }
 """
 
 
