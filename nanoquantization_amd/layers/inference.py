@@ -11,17 +11,18 @@ _PLAIN = (torch.Tensor, Parameter)
 
 
 def plain(*tensors: torch.Tensor) -> bool:
-    """Ordinary 16-bit HIP tensors of one type and device, no gradient wanted, no tracing, no transform, no autocast."""
+    """Ordinary 16-bit HIP tensors of one type and device, no gradient wanted, no tracing, no transform, no autocast.  To be
+    asked before any other condition on the tensors."""
+    # types and modes before any property: a tracer's stand-in has no device to compare, and a traced size warns
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or any(type(t) not in _PLAIN for t in tensors):
+        return False
+    if forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active():
+        return False
     first = tensors[0]
-    if torch.compiler.is_compiling() or first.device.type != "cuda" or first.dtype not in (torch.float16, torch.bfloat16):
-        return False
-    if forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active() or torch.jit.is_tracing():
-        return False
-    if torch.is_autocast_enabled("cuda"):
+    if first.device.type != "cuda" or first.dtype not in (torch.float16, torch.bfloat16) or torch.is_autocast_enabled("cuda"):
         return False
     grad = torch.is_grad_enabled()
-    return all(type(t) in _PLAIN and t.dtype == first.dtype and t.device == first.device and not (grad and t.requires_grad)
-               for t in tensors)
+    return all(t.dtype == first.dtype and t.device == first.device and not (grad and t.requires_grad) for t in tensors)
 
 
 def unhooked(*modules: torch.nn.Module) -> bool:

@@ -22,9 +22,13 @@ class RMSNorm(nn.Module):
         xf = xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + self.eps)
         return xf.to(x.dtype) * self.weight
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def _one_kernel(self, x: torch.Tensor) -> bool:
         # a workgroup per row: rows of a few hundred elements (the heads') leave most of it idle
-        n = self.weight.numel()
-        if type(self) is RMSNorm and 512 <= n <= 8192 and n % 8 == 0 and x.shape[-1:] == self.weight.shape and plain(x, self.weight):
-            return _lib.torch_ops().rms_norm(x, self.weight, self.eps)
+        return (type(self) is RMSNorm and plain(x, self.weight) and 512 <= self.weight.numel() <= 8192
+                and self.weight.numel() % 8 == 0 and x.shape[-1:] == self.weight.shape)
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if not torch.jit.is_scripting():
+            if self._one_kernel(x):
+                return _lib.torch_ops().rms_norm(x, self.weight, self.eps)
         return self.rms_norm(x)

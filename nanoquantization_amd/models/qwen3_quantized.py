@@ -58,12 +58,12 @@ class Qwen3QuantizedAttention(nn.Module):
     def _fused(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: torch.Tensor) -> bool:
         """Whether norms, rotary and the move of k and v into head order run as one kernel: the head dims it is built for, a
         position per token, and norms and rotary that are the ones of this package and watched by no hook."""
-        return (q.dim() == 3 and self.head_dim in (64, 128, 256) and type(pos) is torch.Tensor
-                and pos.dtype in (torch.int32, torch.int64) and pos.dim() in (1, 2) and pos.shape[-1] == q.shape[1]
+        return (type(pos) is torch.Tensor and plain(q, k, v, self.q_norm.weight, self.k_norm.weight)
+                and q.dim() == 3 and self.head_dim in (64, 128, 256) and pos.dtype in (torch.int32, torch.int64) and pos.dim() in (1, 2) and pos.shape[-1] == q.shape[1]
                 and (pos.dim() == 1 or pos.shape[0] in (1, q.shape[0]))
                 and type(self.q_norm) is type(self.k_norm) is RMSNorm and type(self.rope) is RoPE
                 and self.rope.cos_sin_cache.dtype == torch.float32 and pos.device == q.device == self.rope.cos_sin_cache.device
-                and plain(q, k, v, self.q_norm.weight, self.k_norm.weight) and unhooked(self.q_norm, self.k_norm, self.rope))
+                and unhooked(self.q_norm, self.k_norm, self.rope))
 
     def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
         bs = x.shape[0]
@@ -96,14 +96,14 @@ class Qwen3QuantizedMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         g, u = self.gate_proj, self.up_proj
-        if (type(g) is type(u) is WQLinear_GEMM and g.bias is None and u.bias is None and g.qweight.shape == u.qweight.shape
-                and g.qscales.shape == u.qscales.shape and x.shape[-1] == g.qweight.shape[0] and x.dim() > 1
-                and plain(x, g.qscales, u.qscales) and unhooked(g, u)):
+        if (type(g) is type(u) is WQLinear_GEMM and plain(x, g.qscales, u.qscales) and g.bias is None and u.bias is None
+                and g.qweight.shape == u.qweight.shape and g.qscales.shape == u.qscales.shape and x.shape[-1] == g.qweight.shape[0]
+                and x.dim() > 1 and unhooked(g, u)):
             act = _lib.torch_ops().awq_swiglu_pair(x.reshape(-1, x.shape[-1]), g.qweight, g.qscales, g.qzeros, u.qweight, u.qscales,
                                                    u.qzeros)
             return self.down_proj(act.view(*x.shape[:-1], act.shape[-1]))
         gate, up = self.gate_proj(x), self.up_proj(x)
-        if gate.shape[-1] % 8 == 0 and plain(gate, up):
+        if plain(gate, up) and gate.shape[-1] % 8 == 0:
             return self.down_proj(_lib.torch_ops().silu_mul(gate, up))
         return self.down_proj(F.silu(gate) * up)
 
