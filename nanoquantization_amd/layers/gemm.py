@@ -16,6 +16,7 @@ import torch
 import torch.nn as nn
 
 from .. import _lib
+from .inference import shipped
 
 AWQ_SUPPORTED_GROUP_SIZES = [-1, 32, 64, 128]
 _PACK_ORDER = (0, 2, 4, 6, 1, 3, 5, 7)
@@ -182,6 +183,7 @@ def pack_awq(intweight: torch.Tensor) -> torch.Tensor:
     return word.to(torch.int32)
 
 
+@shipped("forward")
 class WQLinear_GEMM(nn.Module):
     def __init__(
         self,

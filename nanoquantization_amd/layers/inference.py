@@ -1,6 +1,7 @@
 """When the modules may run on this library's operators between the AWQ linears (norms, rotary, attention, SiLU).  Those compute
 what the torch expressions beside them do, with the same rounding points, but have no derivatives and no rules for torch's
-function transforms: with any of these in play the torch expressions run."""
+function transforms, and they pass over the modules whose work they take: with a gradient, a transform, a hook or a replaced
+method in play the torch expressions run."""
 from __future__ import annotations
 
 import torch
@@ -23,6 +24,22 @@ def plain(*tensors: torch.Tensor) -> bool:
         return False
     grad = torch.is_grad_enabled()
     return all(t.dtype == first.dtype and t.device == first.device and not (grad and t.requires_grad) for t in tensors)
+
+
+_SHIPPED = {}      # (class, method name) -> the method as this package defines it
+
+
+def shipped(*names: str):
+    """Class decorator: remembers these methods, for `keeps`."""
+    def remember(cls):
+        _SHIPPED.update({(cls, n): getattr(cls, n) for n in names})
+        return cls
+    return remember
+
+
+def keeps(module: torch.nn.Module, cls: type, *names: str) -> bool:
+    """These methods of the module are still those of `cls`: replaced neither on the module nor on its class."""
+    return all(n not in module.__dict__ and getattr(type(module), n, None) is _SHIPPED[cls, n] for n in names)
 
 
 def unhooked(*modules: torch.nn.Module) -> bool:

@@ -7,9 +7,10 @@ import torch
 from torch import nn
 
 from .. import _lib
-from .inference import plain
+from .inference import keeps, plain, shipped
 
 
+@shipped("forward", "rms_norm")
 class RMSNorm(nn.Module):
     def __init__(self, norm_size: int, eps: float = 1e-6) -> None:
         super().__init__()
@@ -24,7 +25,7 @@ class RMSNorm(nn.Module):
 
     def _one_kernel(self, x: torch.Tensor) -> bool:
         # a workgroup per row: rows of a few hundred elements (the heads') leave most of it idle
-        return (type(self) is RMSNorm and plain(x, self.weight) and 512 <= self.weight.numel() <= 8192
+        return (type(self) is RMSNorm and keeps(self, RMSNorm, "rms_norm") and plain(x, self.weight) and 512 <= self.weight.numel() <= 8192
                 and self.weight.numel() % 8 == 0 and x.shape[-1:] == self.weight.shape)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

@@ -5,7 +5,10 @@ from __future__ import annotations
 import torch
 from torch import nn
 
+from .inference import shipped
 
+
+@shipped("forward", "apply_rope")
 class RoPE(nn.Module):
     def __init__(self, head_dim: int, max_position_embeddings: int, base: float = 10000):
         super().__init__()

@@ -17,11 +17,12 @@ import torch.nn.functional as F
 
 from .. import _lib
 from ..layers.gemm import WQLinear_GEMM
-from ..layers.inference import plain, unhooked
+from ..layers.inference import keeps, plain, shipped, unhooked
 from ..layers.norm import RMSNorm
 from ..layers.rope import RoPE
 
 
+@shipped("qkv")
 class Qwen3QuantizedAttention(nn.Module):
     def __init__(self, hidden_size: int, total_num_heads: int, total_num_kv_heads: int,
                  max_position_embeddings: int, w_bits: int = 4, group_size: int = 128,
@@ -57,18 +58,21 @@ class Qwen3QuantizedAttention(nn.Module):
 
     def _fused(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, pos: torch.Tensor) -> bool:
         """Whether norms, rotary and the move of k and v into head order run as one kernel: the head dims it is built for, a
-        position per token, and norms and rotary that are the ones of this package and watched by no hook."""
+        position per token, and norms and rotary that are the ones of this package, unchanged and watched by no hook."""
         return (type(pos) is torch.Tensor and plain(q, k, v, self.q_norm.weight, self.k_norm.weight)
                 and q.dim() == 3 and self.head_dim in (64, 128, 256) and pos.dtype in (torch.int32, torch.int64) and pos.dim() in (1, 2) and pos.shape[-1] == q.shape[1]
                 and (pos.dim() == 1 or pos.shape[0] in (1, q.shape[0]))
                 and type(self.q_norm) is type(self.k_norm) is RMSNorm and type(self.rope) is RoPE
+                and keeps(self.q_norm, RMSNorm, "forward", "rms_norm") and keeps(self.k_norm, RMSNorm, "forward", "rms_norm")
+                and keeps(self.rope, RoPE, "forward", "apply_rope")
                 and self.rope.cos_sin_cache.dtype == torch.float32 and pos.device == q.device == self.rope.cos_sin_cache.device
                 and unhooked(self.q_norm, self.k_norm, self.rope))
 
     def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
         bs = x.shape[0]
-        q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
-        if self._fused(q, k, v, position_ids):
+        own = keeps(self, Qwen3QuantizedAttention, "qkv")
+        q, k, v = (self.q_proj(x), self.k_proj(x), self.v_proj(x)) if own else self.qkv(x, position_ids)
+        if own and self._fused(q, k, v, position_ids):
             pos = position_ids if position_ids.dim() == 2 else position_ids.unsqueeze(0)
             q, k, v = _lib.torch_ops().qkv_norm_rope(q, k, v, self.q_norm.weight, self.k_norm.weight, self.rope.cos_sin_cache,
                                                      pos.to(torch.int64), self.num_heads, self.num_kv_heads, self.q_norm.eps,
@@ -76,7 +80,8 @@ class Qwen3QuantizedAttention(nn.Module):
             if q.dtype == torch.bfloat16:
                 return self.o_proj(_lib.torch_ops().causal_attention(q, k, v, self.head_dim ** -0.5))
         else:
-            q, k, v = self._norm_rope(q, k, v, position_ids)
+            if own:
+                q, k, v = self._norm_rope(q, k, v, position_ids)
             k, v = k.transpose(1, 2), v.transpose(1, 2)
         o = F.scaled_dot_product_attention(q.transpose(1, 2), k, v, is_causal=True,
                                            enable_gqa=self.num_heads != self.num_kv_heads)
@@ -98,7 +103,7 @@ class Qwen3QuantizedMLP(nn.Module):
         g, u = self.gate_proj, self.up_proj
         if (type(g) is type(u) is WQLinear_GEMM and plain(x, g.qscales, u.qscales) and g.bias is None and u.bias is None
                 and g.qweight.shape == u.qweight.shape and g.qscales.shape == u.qscales.shape and x.shape[-1] == g.qweight.shape[0]
-                and x.dim() > 1 and unhooked(g, u)):
+                and x.dim() > 1 and keeps(g, WQLinear_GEMM, "forward") and keeps(u, WQLinear_GEMM, "forward") and unhooked(g, u)):
             act = _lib.torch_ops().awq_swiglu_pair(x.reshape(-1, x.shape[-1]), g.qweight, g.qscales, g.qzeros, u.qweight, u.qscales,
                                                    u.qzeros)
             return self.down_proj(act.view(*x.shape[:-1], act.shape[-1]))

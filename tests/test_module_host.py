@@ -1,5 +1,6 @@
 """What the Qwen3 modules accept around their operators (tracing, scripting, replaced parts), without a device: where the
 operators themselves would run, stand-ins do."""
+import types
 import warnings
 
 import pytest
@@ -7,8 +8,12 @@ import torch
 import torch.fx
 
 import nanoquantization_amd as nq
+from nanoquantization_amd import _lib
+from nanoquantization_amd.layers import norm as norm_module
 from nanoquantization_amd.layers.norm import RMSNorm
-from nanoquantization_amd.models.qwen3_quantized import Qwen3QuantizedMLP
+from nanoquantization_amd.layers.rope import RoPE
+from nanoquantization_amd.models import qwen3_quantized as q3
+from nanoquantization_amd.models.qwen3_quantized import Qwen3QuantizedAttention, Qwen3QuantizedMLP
 
 
 @pytest.mark.parametrize("n", [64, 1024])
@@ -33,3 +38,113 @@ def test_mlp_can_be_traced_with_its_linears_as_leaves():
     graph = Tracer().trace(Qwen3QuantizedMLP(64, 128, group_size=64))
     called = [n.target for n in graph.nodes if n.op == "call_module"]
     assert sorted(called) == ["down_proj", "gate_proj", "up_proj"]
+
+
+@pytest.fixture
+def operators(monkeypatch):
+    """The operators' names in the order they were called, where every tensor counts as one they take; the tensors they return
+    have the right shapes."""
+    seen = []
+
+    def qkv_norm_rope(q, k, v, qw, kw, table, pos, heads, kv_heads, *eps):
+        seen.append("qkv_norm_rope")
+        b, s, hd = q.shape[0], q.shape[1], q.shape[2] // heads
+        return q.view(b, s, heads, hd), *(t.reshape(b, s, kv_heads, hd).transpose(1, 2).contiguous() for t in (k, v))
+
+    def pair(x, *weights):
+        seen.append("awq_swiglu_pair")
+        return x.new_zeros(x.shape[0], weights[1].shape[1])
+
+    def rms_norm(x, *rest):
+        seen.append("rms_norm")
+        return torch.zeros_like(x)
+
+    ops = types.SimpleNamespace(qkv_norm_rope=qkv_norm_rope, awq_swiglu_pair=pair, rms_norm=rms_norm,
+                                silu_mul=lambda g, u: g * u, causal_attention=lambda q, k, v, scale: q.flatten(2))
+    monkeypatch.setattr(_lib, "torch_ops", lambda: ops)
+    for mod in (norm_module, q3):
+        monkeypatch.setattr(mod, "plain", lambda *t: True)
+    return seen
+
+
+def _attention():
+    attn = Qwen3QuantizedAttention(64, 4, 2, 32, head_dim=64, group_size=64)
+    gen = torch.Generator().manual_seed(0)
+    for name, heads in (("q_proj", 4), ("k_proj", 2), ("v_proj", 2)):       # the projections run on a device only
+        w = torch.randn(64, heads * 64, generator=gen)
+        getattr(attn, name).forward = lambda x, w=w: x @ w
+    attn.o_proj.forward = lambda x: x
+    return attn, torch.randn(2, 5, 64, generator=gen), torch.arange(5)
+
+
+@pytest.mark.parametrize("where", ["module", "class"])
+@pytest.mark.parametrize("part,cls,method", [("q_norm", RMSNorm, "forward"), ("k_norm", RMSNorm, "rms_norm"), ("rope", RoPE, "forward"),
+                                             ("rope", RoPE, "apply_rope")])
+def test_attention_calls_replaced_parts(operators, monkeypatch, where, part, cls, method):
+    attn, x, pos = _attention()
+    with torch.no_grad():
+        attn(x, pos)
+        assert operators == ["qkv_norm_rope"]
+        called, before = [], getattr(cls, method)
+
+        def replaced(*args):
+            called.append(method)
+            return before(*(args if where == "class" or isinstance(cls.__dict__[method], staticmethod) else (getattr(attn, part), *args)))
+        if where == "class":
+            monkeypatch.setattr(cls, method, staticmethod(replaced) if isinstance(cls.__dict__[method], staticmethod) else replaced)
+        else:
+            setattr(getattr(attn, part), method, replaced)
+        attn(x, pos)
+    assert called and operators == ["qkv_norm_rope"]
+
+
+@pytest.mark.parametrize("where", ["module", "subclass"])
+def test_attention_calls_a_replaced_qkv(operators, where):
+    attn, x, pos = _attention()
+    called, before = [], attn.qkv
+
+    def replaced(x, position_ids):
+        called.append("qkv")
+        return before(x, position_ids)
+    if where == "module":
+        attn.qkv = replaced
+    else:
+        attn.__class__ = type("Sub", (Qwen3QuantizedAttention,), {"qkv": lambda self, x, position_ids: replaced(x, position_ids)})
+    with torch.no_grad():
+        attn(x, pos)
+    assert called == ["qkv"] and operators == []
+
+
+@pytest.mark.parametrize("where", ["gate_proj", "up_proj", "class"])
+def test_mlp_calls_replaced_linears(operators, monkeypatch, where):
+    mlp, x = Qwen3QuantizedMLP(64, 128, group_size=64), torch.randn(2, 3, 64)
+    mlp.down_proj.forward = lambda a: a
+    mlp(x)
+    assert operators == ["awq_swiglu_pair"]
+    called = []
+
+    def replaced(*args):
+        called.append(where)
+        return args[-1].new_ones(*args[-1].shape[:-1], 128)
+    if where == "class":
+        monkeypatch.setattr(nq.WQLinear_GEMM, "forward", replaced)
+        mlp(x)
+        assert called == ["class", "class"]
+    else:
+        setattr(getattr(mlp, where), "forward", replaced)
+        with pytest.raises(_lib.AwqHipError):       # the other projection, which needs a device
+            mlp(x)
+        assert where == "up_proj" or called == ["gate_proj"]
+    assert operators == ["awq_swiglu_pair"]
+
+
+@pytest.mark.parametrize("where", ["module", "class"])
+def test_norm_calls_a_replaced_rms_norm(operators, monkeypatch, where):
+    norm, x = RMSNorm(1024), torch.randn(2, 1024)
+    norm(x)
+    assert operators == ["rms_norm"]
+    if where == "class":
+        monkeypatch.setattr(RMSNorm, "rms_norm", lambda self, x: x + 1)
+    else:
+        norm.rms_norm = lambda x: x + 1
+    assert torch.equal(norm(x), x + 1) and operators == ["rms_norm"]
