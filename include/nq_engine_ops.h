@@ -92,7 +92,7 @@ int nq_silu_mul_pair(const void* gate, const void* up, void* out, int64_t rows, 
 /* q [batch * tokens, num_heads * head_dim], k and v [.., num_kv_heads * head_dim]: outputs of the separate projections.
  * q and k heads are normalised and rotated as by nq_qk_norm_rope_store, at positions[sequence][token] (per_sequence) or
  * positions[token]; a negative position counts from the end of the table,
- * and one outside the table gives NaN.  q_out keeps q's layout, k_out and v_out are
+ * and one outside the table gives NaN (the module refuses such positions before the call).  q_out keeps q's layout, k_out and v_out are
  * [batch, num_kv_heads, tokens, head_dim].  head_dim 64, 128 or 256. */
 int nq_qkv_norm_rope(const void* q, const void* k, const void* v, const void* q_weight, const void* k_weight,
                      const float* cos_sin, const int64_t* positions, int per_sequence, void* q_out, void* k_out,

@@ -35,6 +35,11 @@ class RoPE(nn.Module):
         x1, x2 = torch.chunk(x.float(), 2, dim=-1)
         return torch.cat([x1 * cos - x2 * sin, x1 * sin + x2 * cos], dim=-1).to(x.dtype)
 
+    def refuse_unknown(self, position_ids: torch.Tensor) -> None:
+        """torch's own index error for positions outside the table, as `forward` has it, from one element a position: the
+        operator that takes this module's place reads the table itself and has no way to raise."""
+        self.cos_sin_cache[:, 0, 0][position_ids]
+
     def forward(self, query: torch.Tensor, key: torch.Tensor, position_ids: torch.Tensor):
         """query/key: [batch, seq, heads, head_dim]; position_ids: [batch, seq] (or broadcastable)."""
         cos, sin = torch.chunk(self.cos_sin_cache[position_ids], 2, dim=-1)

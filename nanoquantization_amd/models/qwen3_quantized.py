@@ -73,9 +73,10 @@ class Qwen3QuantizedAttention(nn.Module):
         own = keeps(self, Qwen3QuantizedAttention, "qkv")
         q, k, v = (self.q_proj(x), self.k_proj(x), self.v_proj(x)) if own else self.qkv(x, position_ids)
         if own and self._fused(q, k, v, position_ids):
-            pos = position_ids if position_ids.dim() == 2 else position_ids.unsqueeze(0)
+            pos = (position_ids if position_ids.dim() == 2 else position_ids.unsqueeze(0)).to(torch.int64)
+            self.rope.refuse_unknown(pos)
             q, k, v = _lib.torch_ops().qkv_norm_rope(q, k, v, self.q_norm.weight, self.k_norm.weight, self.rope.cos_sin_cache,
-                                                     pos.to(torch.int64), self.num_heads, self.num_kv_heads, self.q_norm.eps,
+                                                     pos, self.num_heads, self.num_kv_heads, self.q_norm.eps,
                                                      self.k_norm.eps)
             if q.dtype == torch.bfloat16:
                 return self.o_proj(_lib.torch_ops().causal_attention(q, k, v, self.head_dim ** -0.5))

@@ -98,6 +98,22 @@ def test_attention_calls_replaced_parts(operators, monkeypatch, where, part, cls
     assert called and operators == ["qkv_norm_rope"]
 
 
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_attention_refuses_positions_outside_the_table(operators, dtype):
+    attn, x, pos = _attention()                 # a table of 32 positions
+    with torch.no_grad():
+        for first in (0, 27, -32):
+            attn(x, (pos + first).to(dtype))
+            attn(x, (pos + first).expand(2, 5).to(dtype))
+        assert operators == ["qkv_norm_rope"] * 6
+        for first in (28, 1 << 20, -33):
+            with pytest.raises(IndexError):
+                attn(x, (pos + first).to(dtype))
+            with pytest.raises(IndexError):
+                attn(x, (pos + first).expand(2, 5).to(dtype))
+    assert operators == ["qkv_norm_rope"] * 6
+
+
 @pytest.mark.parametrize("where", ["module", "subclass"])
 def test_attention_calls_a_replaced_qkv(operators, where):
     attn, x, pos = _attention()
