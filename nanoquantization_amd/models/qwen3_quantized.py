@@ -65,7 +65,9 @@ class Qwen3QuantizedAttention(nn.Module):
                 and type(self.q_norm) is type(self.k_norm) is RMSNorm and type(self.rope) is RoPE
                 and keeps(self.q_norm, RMSNorm, "forward", "rms_norm") and keeps(self.k_norm, RMSNorm, "forward", "rms_norm")
                 and keeps(self.rope, RoPE, "forward", "apply_rope")
-                and self.rope.cos_sin_cache.dtype == torch.float32 and pos.device == q.device == self.rope.cos_sin_cache.device
+                and self.q_norm.weight.shape == self.k_norm.weight.shape == (self.head_dim,)
+                and self.rope.cos_sin_cache.dtype == torch.float32 and self.rope.cos_sin_cache.shape[1:] == (1, self.head_dim)
+                and self.rope.cos_sin_cache.is_contiguous() and pos.device == q.device == self.rope.cos_sin_cache.device
                 and unhooked(self.q_norm, self.k_norm, self.rope))
 
     def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
@@ -109,7 +111,7 @@ class Qwen3QuantizedMLP(nn.Module):
                                                    u.qzeros)
             return self.down_proj(act.view(*x.shape[:-1], act.shape[-1]))
         gate, up = self.gate_proj(x), self.up_proj(x)
-        if plain(gate, up) and gate.shape[-1] % 8 == 0:
+        if plain(gate, up) and gate.shape == up.shape and gate.shape[-1] % 8 == 0:
             return self.down_proj(_lib.torch_ops().silu_mul(gate, up))
         return self.down_proj(F.silu(gate) * up)
 

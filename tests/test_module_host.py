@@ -114,6 +114,33 @@ def test_attention_refuses_positions_outside_the_table(operators, dtype):
     assert operators == ["qkv_norm_rope"] * 6
 
 
+def test_attention_leaves_other_shapes_to_torch(operators):
+    """Norm weights per head and a table of other strides, which broadcasting and indexing take; a table of another head size,
+    which they refuse."""
+    attn, x, pos = _attention()
+    with torch.no_grad():
+        attn.q_norm.weight = torch.nn.Parameter(torch.rand(4, 64))
+        attn(x, pos)
+        attn, x, pos = _attention()
+        want = attn.qkv(x, pos)
+        attn.rope.cos_sin_cache = attn.rope.cos_sin_cache.transpose(0, 2).contiguous().transpose(0, 2)
+        attn(x, pos)
+        assert all(torch.equal(a, b) for a, b in zip(attn.qkv(x, pos), want))
+        attn.rope = RoPE(32, 64)
+        with pytest.raises(RuntimeError):
+            attn(x, pos)
+    assert operators == []
+
+
+def test_mlp_broadcasts_as_torch_does(operators):
+    mlp, x = Qwen3QuantizedMLP(64, 128, group_size=64), torch.randn(2, 3, 64)
+    mlp.gate_proj, mlp.up_proj, mlp.down_proj = torch.nn.Linear(64, 128), torch.nn.Linear(64, 1), torch.nn.Identity()
+    called = []
+    _lib.torch_ops().silu_mul = lambda g, u: called.append("silu_mul") or g * u
+    want = torch.nn.functional.silu(mlp.gate_proj(x)) * mlp.up_proj(x)
+    assert torch.equal(mlp(x), want) and called == []
+
+
 @pytest.mark.parametrize("where", ["module", "subclass"])
 def test_attention_calls_a_replaced_qkv(operators, where):
     attn, x, pos = _attention()
