@@ -220,22 +220,25 @@ at::Tensor dense16(const at::Tensor& t) {
     return reinterpret_cast<uintptr_t>(d.data_ptr()) & 15u ? d.clone() : d;
 }
 
+// The result has the strides that elementwise operations on x give (x's own, where x is dense in some order of its dimensions).
 at::Tensor rms_norm_op(const at::Tensor& x, const at::Tensor& weight, double eps) {
     const int dtype = dtype_of(x);
     TORCH_CHECK(x.dim() >= 1 && weight.dim() == 1 && x.size(-1) == weight.size(0) && weight.scalar_type() == x.scalar_type(),
                 "weight must be [x.size(-1)] of x's dtype");
     check_device(x, {&weight});
     const DeviceGuard guard(x.device());
-    at::Tensor y = at::empty(x.sizes(), x.options());
+    at::Tensor y = at::empty_like(x);
     if (x.numel() == 0) return y;
+    const at::Tensor out = y.is_contiguous() ? y : at::empty(x.sizes(), x.options());
     const at::Tensor xd = dense16(x), w = dense16(weight);
     const int64_t hidden = x.size(-1);
-    check_status(nq_add_rmsnorm(xd.data_ptr(), nullptr, w.data_ptr(), y.data_ptr(), x.numel() / hidden, hidden, (float)eps,
+    check_status(nq_add_rmsnorm(xd.data_ptr(), nullptr, w.data_ptr(), out.data_ptr(), x.numel() / hidden, hidden, (float)eps,
                                 dtype, current_stream(x.device().index())),
                  "nq_add_rmsnorm");
+    if (!out.is_same(y)) y.copy_(out);
     return y;
 }
-at::Tensor rms_norm_meta(const at::Tensor& x, const at::Tensor&, double) { return at::empty(x.sizes(), x.options()); }
+at::Tensor rms_norm_meta(const at::Tensor& x, const at::Tensor&, double) { return at::empty_like(x); }
 
 at::Tensor silu_mul_op(const at::Tensor& gate, const at::Tensor& up) {
     const int dtype = dtype_of(gate);

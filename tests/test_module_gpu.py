@@ -209,3 +209,14 @@ def test_when_modules_use_the_operators(monkeypatch):
         for got, want in ((fused, hooked), (fused_logits, m(ids, pos))):
             # a dozen roundings to 8 bits on the way, of which few fall differently
             assert (got.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
+@pytest.mark.parametrize("layout", [lambda x: x.transpose(0, 1), lambda x: x[:, -1], lambda x: x.transpose(-1, -2).contiguous().transpose(-1, -2)])
+def test_norm_result_keeps_the_layout(layout):
+    from nanoquantization_amd.layers.norm import RMSNorm
+    norm = RMSNorm(512).to("cuda", torch.bfloat16)
+    x = layout(torch.randn(4, 6, 3, 512, device="cuda", generator=torch.Generator(device="cuda").manual_seed(0)).bfloat16())
+    with torch.no_grad():
+        got, want = norm(x), norm.rms_norm(x)
+    assert got.stride() == want.stride()
+    assert ((got.float() - want.float()).abs() <= 2.0 ** -6 * want.float().abs() + 1e-6).all()      # one place each, as above

@@ -1,5 +1,6 @@
 """What the Qwen3 modules accept around their operators (tracing, scripting, replaced parts), without a device: where the
 operators themselves would run, stand-ins do."""
+import os
 import types
 import warnings
 
@@ -28,6 +29,24 @@ def test_norm_can_be_traced_and_scripted(n):
         warnings.simplefilter("error", torch.jit.TracerWarning)
         traced = torch.jit.trace(norm, (x,))
     assert torch.equal(traced(x[:2]), want[:2])
+
+
+LAYOUTS = [lambda x: x, lambda x: x.transpose(0, 1), lambda x: x.permute(2, 0, 1, 3), lambda x: x[:, -1], lambda x: x[:, ::2],
+           lambda x: x.transpose(-1, -2).contiguous().transpose(-1, -2), lambda x: x[:1].expand(4, -1, -1, -1),
+           lambda x: torch.cat([x, x], -1)[..., :x.shape[-1]].transpose(0, 2)]
+
+
+@pytest.mark.parametrize("layout", range(len(LAYOUTS)))
+def test_norm_result_keeps_the_layout(layout):
+    """The operator's result has the strides of the torch expression's."""
+    if not os.path.exists(_lib.TORCH_LIB_PATH):
+        from nanoquantization_amd.build import build
+        build(verbose=False)
+    norm = RMSNorm(512).to(torch.bfloat16)
+    x = LAYOUTS[layout](torch.randn(4, 6, 3, 512).bfloat16())
+    like = torch.empty_strided(x.shape, x.stride(), dtype=x.dtype, device="meta")
+    got = _lib.torch_ops().rms_norm(like, norm.weight.detach().to("meta"), norm.eps)
+    assert got.shape == x.shape and got.stride() == norm.rms_norm(x).stride()
 
 
 def test_mlp_can_be_traced_with_its_linears_as_leaves():
