@@ -144,20 +144,20 @@ def run_one(kind, K, N, M, dtype, iters, copies=1, g=G):
 
 
 def gemm_kernel_name(M, N, K, dtype_name, g=G):
-    """The kernel nq.awq_gemm runs for a prefill problem, from the library's own rules."""
+    """The kernel nq.awq_gemm runs for a prefill problem, as the library names it."""
     import ctypes
     from nanoquantization_amd import _lib
-    L = _lib.lib()
-    v, sp = ctypes.c_int(), ctypes.c_int()
+    sp = ctypes.c_int()
     did = _lib.AWQ_F16 if dtype_name == "f16" else _lib.AWQ_BF16
-    if L.awq_linear_dense_wanted_bytes(M, N, K, g):
-        return f"awq::dense_kernel<{'F16' if dtype_name == 'f16' else 'BF16'}> behind awq::dequant_transpose_kernel"
-    if L.awq_gemm_plan(M, N, K, g, did, ctypes.byref(v), ctypes.byref(sp)) != 0:
-        return "?"
-    name = L.awq_gemm_variant_name(v.value).decode()
+    name = _lib.lib().awq_linear_route(M, N, K, g, did, 0, ctypes.byref(sp)).decode()
     T = "F16" if dtype_name == "f16" else "BF16"
+    if not name or name.startswith("gemv"):
+        return name or "?"
+    if name == "dense":
+        return f"awq::dense_kernel<{T}> behind awq::dequant_transpose_kernel"
     kern = {"256x256p": f"awq::gemm_pipe_kernel<{T},2,4>", "256x256pt": f"awq::gemm_pipe_kernel<{T},2,4>",
-            "256x256r": f"awq::gemm_regb_kernel<{T}>", "256x256rt": f"awq::gemm_regb_kernel<{T}>"}.get(
+            "256x256r": f"awq::gemm_regb_kernel<{T}>", "256x256rt": f"awq::gemm_regb_kernel<{T}>",
+            "rows128": f"awq::rows_kernel<{T}>"}.get(
                 name, f"awq::gemm_kernel<{T},{name}>")
     return f"{kern} (plan {name}, split {sp.value})"
 

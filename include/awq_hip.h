@@ -93,6 +93,11 @@ int awq_linear_dense_pair(const void* x, const int32_t* gate_qweight, const void
                           int64_t N, int64_t K, int64_t group_size, int dtype, void* scratch, size_t scratch_bytes,
                           void* stream);
 
+/* What a linear of these sizes runs: "gemv", "gemv in blocks of 16 rows", "dense" (awq_linear_dense, where the caller has scratch for
+ * it), or the name of the awq_gemm variant awq_linear (gated: awq_linear_swiglu) takes; *split_k (may be null) its K split.  "" for
+ * sizes that none of them takes.  A static string. */
+const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype, int gated, int* split_k);
+
 /* Bytes of device workspace awq_gemv / awq_gemm / awq_linear need for this
  * problem (0 is possible).  The workspace must be zero-filled ONCE when it is
  * allocated; every call leaves it in that state (its counters are reset by

@@ -36,6 +36,7 @@ SYMBOLS = {
     "awq_quantize_pack_flagged": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "awq_linear_dense_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "awq_linear_dense_wanted_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "awq_linear_route": (ctypes.c_char_p, [_i64] * 4 + [_int, _int, ctypes.POINTER(_int)]),
     "awq_linear_dense": (_int, [_vp] * 6 + [_i64] * 4 + [_int, _int, _vp, _sz, _vp]),
     "awq_linear_dense_pair": (_int, [_vp] * 8 + [_i64] * 4 + [_int, _vp, _sz, _vp]),
     "awq_gemv_workspace_bytes": (_sz, [_i64, _i64, _i64]),

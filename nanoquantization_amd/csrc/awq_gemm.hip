@@ -593,20 +593,47 @@ extern "C" int awq_linear_swiglu(const void* x, const int32_t* qweight, const vo
                               dtype, workspace, workspace_bytes, stream, v, s, 1);
 }
 
+// The regimes of awq_linear as sizes decide them: decode rows on the GEMV (up to 16 on any of its paths, up to 64 on the staged
+// one, 128 on small weights); a K that the MFMA kernels' 64-row steps do not divide (the reference takes any multiple of 32,
+// layers/gemm.py:268) on the GEMV 16 rows at a time -- no real model has such a width, so only the result matters there; tiles.
+enum class Regime { gemv, gemv_blocks, tiles };
+static Regime linear_regime(int64_t M, int64_t N, int64_t K, int64_t g) {
+    const bool staged = N % 128 == 0 && g > 0 && g % 128 == 0;
+    if (M >= 1 && ((M <= 16 && g % 32 == 0) || (gemv_rows_ok(M, N, K) && staged))) return Regime::gemv;
+    if (M > 16 && K % awq::kBK != 0 && K % 32 == 0 && g > 0 && g % 32 == 0 && K % g == 0 && N > 0) return Regime::gemv_blocks;
+    return Regime::tiles;
+}
+
+extern "C" const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype, int gated, int* split_k) {
+    int split = 1;
+    if (!split_k) split_k = &split;
+    *split_k = 1;
+    if (M < 1 || N < (gated ? 16 : 8) || N % (gated ? 16 : 8) != 0 || K < 32 || K % 32 != 0 || group_size < 1 ||
+        K % group_size != 0 || (dtype != AWQ_F16 && dtype != AWQ_BF16))
+        return "";
+    const bool staged = N % 128 == 0 && group_size % 128 == 0;
+    const Regime regime = linear_regime(M, N, K, group_size);
+    if (gated ? M <= 64 && staged : regime == Regime::gemv) return "gemv";
+    if (!gated && regime == Regime::gemv_blocks) return "gemv in blocks of 16 rows";
+    if (K % awq::kBK != 0 || !(group_size % 64 == 0 || (64 % group_size == 0 && group_size % 8 == 0))) return "";
+    if (awq_linear_dense_wanted_bytes(M, N, K, group_size)) return "dense";
+    int variant;
+    awq::RowsPlan rows;
+    if (rows_wanted(M, N, K, group_size, &rows)) variant = awq::kRowsVariant, *split_k = rows.splits;
+    else if (gated) awq::plan_gemm_tile256(M, N, K, group_size, dtype, &variant, split_k);
+    else awq::plan_gemm(M, N, K, group_size, dtype, &variant, split_k);
+    return awq::kGemmVariants[variant].name;
+}
+
 extern "C" int awq_linear(const void* x, const int32_t* qweight, const void* qscales,
                           const int32_t* qzeros, const void* bias, void* y, int64_t M, int64_t N,
                           int64_t K, int64_t group_size, int dtype, void* workspace,
                           size_t workspace_bytes, void* stream) {
-    // decode regime: up to 16 rows on any GEMV path, up to 64 on the staged one (128 on small weights)
-    const bool staged = N % 128 == 0 && group_size > 0 && group_size % 128 == 0;
-    if (M >= 1 && ((M <= 16 && group_size % 32 == 0) || (gemv_rows_ok(M, N, K) && staged)))
+    const Regime regime = linear_regime(M, N, K, group_size);
+    if (regime == Regime::gemv)
         return awq_gemv(x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,
                         workspace_bytes, stream);
-    if (M > 16 && K % awq::kBK != 0 && K % 32 == 0 && group_size > 0 && group_size % 32 == 0 && K % group_size == 0 &&
-        N > 0 && x && y) {
-        // a K the MFMA GEMM's 64-row steps do not divide (the reference takes any multiple of 32,
-        // layers/gemm.py:268): the GEMV, 16 rows at a time -- no real model has such a width, so only
-        // the result matters here
+    if (regime == Regime::gemv_blocks && x && y) {
         const size_t esz = 2;
         for (int64_t m0 = 0; m0 < M; m0 += 16) {
             const int64_t rows = M - m0 < 16 ? M - m0 : 16;

@@ -1,4 +1,6 @@
 """Kernel (c): fused dequant + MFMA GEMM through the C ABI against the fp32-accumulation oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -329,8 +331,16 @@ def test_linear_dense_routes():
     p = random_packed(K, N, 128, "bf16", seed=7)
     dev = [to_dev(p["qweight"]), to_dev(p["qscales"], "bf16"), to_dev(p["qzeros"])]
     assert wanted(M, N, K, 128) > 0
-    x = to_dev(make_x(M, K, "bf16", seed=8), "bf16")
-    want = nq.awq_gemm(x, *dev, 8)
+    xb = make_x(M, K, "bf16", seed=8)
+    x = to_dev(xb, "bf16")
+    want = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    scratch = torch.empty(L.awq_linear_dense_scratch_bytes(M, N, K, 128), dtype=torch.uint8, device="cuda")
+    _lib.check(L.awq_linear_dense(x.data_ptr(), *(t.data_ptr() for t in dev), None, want.data_ptr(), M, N, K, 128, _lib.AWQ_BF16, 0,
+                                  scratch.data_ptr(), scratch.numel(), _lib.current_stream_ptr(want.device)))
+    _check(want, xb, p, "bf16")
+    assert L.awq_linear_route(M, N, K, 128, _lib.AWQ_BF16, 0, None) == b"dense"
+    assert torch.equal(nq.awq_gemm(x, *dev, 8), want)
+    assert torch.equal(_lib.torch_ops().awq_linear(x, *dev, None), want)
     s, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     with torch.cuda.stream(s):
         assert torch.equal(nq.awq_gemm(x, *dev, 8), want)
@@ -433,12 +443,40 @@ def test_gemm_rows128_routes():
         dev = [to_dev(p["qweight"]), to_dev(p["qscales"], "bf16"), to_dev(p["qzeros"])]
         x = to_dev(make_x(M, K, "bf16", seed=10), "bf16")
         y = nq.awq_gemm(x, *dev, 8)
-        assert any(torch.equal(y, awq_gemm_variant(x, *dev, v, s)) for s in range(1, 17)), (M, K, N)
+        chosen = ctypes.c_int()
+        assert L.awq_linear_route(M, N, K, g, _lib.AWQ_BF16, 0, ctypes.byref(chosen)) == b"rows128"
+        assert torch.equal(y, awq_gemm_variant(x, *dev, v, chosen.value)), (M, K, N)
         assert L.awq_linear_workspace_bytes(M, N, K) >= L.awq_gemm_ex_workspace_bytes(M, N, K, v, split)
     # groups of 16 rows end inside a wave's 32: an error, before anything is launched
     args = (x.data_ptr(), dev[0].data_ptr(), dev[1].data_ptr(), dev[2].data_ptr(), None, y.data_ptr())
     assert L.awq_gemm_ex(*args, M, N, K, 16, _lib.AWQ_BF16, None, 0, None, v, 1) != 0
     assert b"group size" in L.awq_hip_last_error()
+
+
+# unsplit and in two to five K splits, rows past the last tile, columns past the last tile (2 x 1032: 16.1 of them)
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,K,inter,g,split", [(200, 2048, 8192, 128, False), (160, 12288, 1024, 128, True), (333, 2816, 1032, 64, True),
+                                               (513, 2048, 1024, 128, True)])
+def test_swiglu_rows128(dtype, M, K, inter, g, split):
+    """The gated epilogue of the 128-row tiles, in the tile and in the sum of the K splits: the bits of the same tiles' product
+    and the separate activation."""
+    from nanoquantization_amd.engine import ops
+    print(f"swiglu rows128 {dtype} M={M} K={K} inter={inter}", flush=True)
+    tdt, L, N = torch.float16 if dtype == "f16" else torch.bfloat16, _lib.lib(), 2 * inter
+    chosen = ctypes.c_int()
+    assert L.awq_linear_route(M, N, K, g, _lib.dtype_id(tdt), 1, ctypes.byref(chosen)) == b"rows128"
+    assert (chosen.value > 1) == split
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    qw = torch.randint(-2 ** 31, 2 ** 31 - 1, (K, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    qz = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // g, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    qs = ((torch.rand(K // g, N, device="cuda", generator=gen) + 0.1) * 0.2 / K ** 0.5).to(tdt)
+    x = torch.randn(M, K, device="cuda", generator=gen).to(tdt)
+    names = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())]
+    plain = awq_gemm_variant(x, qw, qs, qz, names.index("rows128"), chosen.value)
+    assert torch.equal(ops.awq_linear_swiglu(x, qw, qs, qz), ops.silu_mul(plain, interleaved=True))
+    assert torch.equal(_lib.torch_ops().awq_linear_swiglu(x, qw, qs, qz), ops.silu_mul(plain, interleaved=True))
+    ref = x.double() @ nq.awq_dequantize(qw, qs, qz).double()
+    assert (plain.double() - ref).abs().max().item() <= TIGHT[dtype] * ref.abs().max().item()
 
 
 # a row, columns past the last tile, an odd number of words, two slabs (131072 x 1040: 273 MB)
