@@ -79,14 +79,16 @@ int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, void* qscal
  * no bias.  awq_linear_dense_scratch_bytes: at most 256 MiB (a single tile of 256 columns where those are wider); 0 if the
  * sizes are not this path's (K % 64, a group size of 8, 16, 32 or a multiple of 64).  The scratch needs no
  * initialisation and is free again when the call's work on the stream is done.
- * awq_linear_dense_wanted_bytes: the same where this is the faster way (rows in the hundreds and more), else 0. */
+ * awq_linear_scratch_bytes: the same where this is the fastest way for the type (rows in the hundreds and more), else 0.
+ * awq_linear_dense_wanted_bytes: the same for either type. */
 size_t awq_linear_dense_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size);
+size_t awq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype);
 size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size);
 int awq_linear_dense(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
                      const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
                      int gated, void* scratch, size_t scratch_bytes, void* stream);
 /* y [M, N] = dtype(SiLU(x @ gate)) * (x @ up) for two weights [K, N] that lie apart: both are dequantised into `scratch` in one
- * pass, interleaved, and multiplied as by awq_linear_dense with `gated`.  Scratch (and whether this is the faster way): as for
+ * pass, interleaved, and multiplied as by awq_linear_dense with `gated`.  Scratch (and whether this is the fastest way): as for
  * awq_linear_dense with 2 N columns. */
 int awq_linear_dense_pair(const void* x, const int32_t* gate_qweight, const void* gate_qscales, const int32_t* gate_qzeros,
                           const int32_t* up_qweight, const void* up_qscales, const int32_t* up_qzeros, void* y, int64_t M,

@@ -36,6 +36,7 @@ SYMBOLS = {
     "awq_quantize_pack_flagged": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "awq_linear_dense_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "awq_linear_dense_wanted_bytes": (_sz, [_i64, _i64, _i64, _i64]),
+    "awq_linear_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
     "awq_linear_route": (ctypes.c_char_p, [_i64] * 4 + [_int, _int, ctypes.POINTER(_int)]),
     "awq_linear_dense": (_int, [_vp] * 6 + [_i64] * 4 + [_int, _int, _vp, _sz, _vp]),
     "awq_linear_dense_pair": (_int, [_vp] * 8 + [_i64] * 4 + [_int, _vp, _sz, _vp]),
@@ -261,10 +262,10 @@ def workspace_bytes(entry: str, M: int, N: int, K: int, extra: tuple = ()) -> in
     return n
 
 
-def dense_scratch(device: torch.device, M: int, N: int, K: int, group_size: int) -> torch.Tensor | None:
-    """Scratch for awq_linear_dense where that is the faster way, else None.  It comes from torch's caching allocator for this
+def dense_scratch(device: torch.device, M: int, N: int, K: int, group_size: int, dtype: int) -> torch.Tensor | None:
+    """Scratch for awq_linear_dense where that is the fastest way, else None.  It comes from torch's caching allocator for this
     one call (ordered on the current stream like any temporary); without room for it the fused kernels run."""
-    nbytes = lib().awq_linear_dense_wanted_bytes(M, N, K, group_size)
+    nbytes = lib().awq_linear_scratch_bytes(M, N, K, group_size, dtype)
     if not nbytes:
         return None
     try:

@@ -264,7 +264,7 @@ static int gemm_effective_splits(int64_t K, int split_k) {
 
 static size_t gemm_ws_bytes(int64_t M, int64_t N, int64_t K, int variant, int split_k) {
     if (is_tile256(variant)) return pipe_ws_bytes(make_pipe_plan(M, N, K, split_k, is_tail_variant(variant)));
-    if (variant == kRowsVariant) return rows_ws_bytes(make_rows_plan(M, N, K, 32, split_k), M, N);
+    if (variant == kRowsVariant) return rows_ws_bytes(make_rows_plan(M, N, K, 32, AWQ_F16, split_k), M, N);
     const int splits = gemm_effective_splits(K, split_k);
     if (splits <= 1) return 0;
     return kCounterBytes + (size_t)splits * M * N * sizeof(float);
@@ -379,7 +379,7 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
         set_error("%s: the gated epilogue takes no bias, needs N %% 16 == 0 and runs on the 256 x 256 and 128-row tiles", fn);
         return AWQ_ERR_UNSUPPORTED;
     }
-    const RowsPlan rows = variant == kRowsVariant ? make_rows_plan(M, N, K, g, split_k) : RowsPlan{};
+    const RowsPlan rows = variant == kRowsVariant ? make_rows_plan(M, N, K, g, dtype, split_k) : RowsPlan{};
     if (variant == kRowsVariant && rows.m_tiles == 0) {
         set_error("%s: tile rows128 needs a group size that is a multiple of 32 and x below 2 Gi elements", fn);
         return AWQ_ERR_UNSUPPORTED;
@@ -503,14 +503,19 @@ extern "C" int awq_gemm(const void* x, const int32_t* qweight, const void* qscal
 }
 
 // Microseconds of the fused 256 x 256 kernels: 1.9 a K step and round of 256 workgroups, 10 to fill and store a round's tiles,
-// and 0.05 per K slice of a tile for its fp32 partials and their sum (within 15 % of every size measured between 256 and 8192
-// rows).
-static double fused_linear_us(int64_t M, int64_t N, int64_t K) {
+// and 0.05 per K slice of a tile for its fp32 partials and their sum (a fifth less where a launch leaves half of the CUs idle,
+// within 15 % of the other sizes measured between 256 and 8192 rows).  In fp16 the register-operand kernel takes a tenth less
+// than that with whole tiles, or with several items a workgroup (640 x 4096 x 24576 139 us, estimated 170 without, 161
+// dequantised first).
+static double fused_linear_us(int64_t M, int64_t N, int64_t K, int64_t g, int dtype) {
     int v, split;
-    awq::pick_gemm(M, N, K, &v, &split);
+    awq::plan_gemm(M, N, K, g, dtype, &v, &split);
     const awq::PipePlan p = awq::make_pipe_plan(M, N, K, split, awq::is_tail_variant(v));
-    const double full = (double)awq::cdiv(p.full_tiles, 256), cut = (double)awq::cdiv((int64_t)p.tail_tiles * p.splits, 256);
-    return full * (1.9 * (double)(K / 64) + 10) + cut * (1.9 * p.iters_per_split + 10) + 0.05 * p.tail_tiles * p.splits;
+    const int64_t slices = (int64_t)p.tail_tiles * p.splits;
+    const double full = (double)awq::cdiv(p.full_tiles, 256), cut = (double)awq::cdiv(slices, 256);
+    const double us = full * (1.9 * (double)(K / 64) + 10) + cut * (1.9 * p.iters_per_split + 10) + 0.05 * (double)slices;
+    const bool regb = v == awq::kRegbVariant || v == awq::kRegbTailVariant;
+    return regb && dtype == AWQ_F16 && (slices == 0 || p.full_tiles + slices > 256) ? 0.9 * us : us;
 }
 
 // Short K at up to 2048 rows stays fused: awq_gemm_plan's kernel and K split are what a caller gets there, bit for bit, and
@@ -518,18 +523,31 @@ static double fused_linear_us(int64_t M, int64_t N, int64_t K) {
 static bool always_fused(int64_t M, int64_t K) { return M <= 128 || (M <= 2048 && K < 2048); }
 
 // Whether the tiles of awq_gemm_rows.hip are the fastest way, from the estimates of all three; in one round of the CUs only
-// (5120 x 25600 at 160 rows, 400 tiles: 85 us in fp16 and 101 in bf16 against 85 fused).  Measured, fp16 / bf16 and the faster
+// (5120 x 25600 at 160 rows, 400 tiles: 85 us in fp16 and 101 in bf16 against 85 fused).  The estimates know the type: 5120 x
+// 10240 at 129 to 192 rows takes 51-53 us in bf16 here and 46 fused, 41-43 in fp16 against 43-45.  Measured, fp16 / bf16 and the faster
 // of the other two: 2816 x 9720 at 333 rows 31 / 34 us against 46, 4096 x 4096 at 200 rows 24 / 25 against 29, at 512 rows
 // 33 / 36 against 41, 12288 x 4096 at 160 rows 35 / 39 against 46, 8192 x 1024 at 1024 rows 36 / 38 against 42, 2048 x 6144 at
 // 640 rows 26 / 27 against 34.
-static bool rows_wanted(int64_t M, int64_t N, int64_t K, int64_t g, awq::RowsPlan* plan) {
+static bool rows_wanted(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, awq::RowsPlan* plan) {
     if (always_fused(M, K)) return false;
-    *plan = awq::make_rows_plan(M, N, K, g);
+    *plan = awq::make_rows_plan(M, N, K, g, dtype);
     if (plan->m_tiles == 0 || (int64_t)plan->m_tiles * plan->n_tiles * plan->splits > 256 ||
-        plan->us >= 0.95 * fused_linear_us(M, N, K))
+        plan->us >= 0.96 * fused_linear_us(M, N, K, g, dtype))
         return false;
     const double dense = awq::dense_linear_us(M, N, K, g);
     return dense < 0 || plan->us < 0.95 * dense;
+}
+
+// Workspace of those tiles where they are wanted, for either type and any group size: the size decides whether they run and not
+// the split, and they run at a group size of 32 wherever they do at another (fused_linear_us is the largest there).
+static size_t rows_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    size_t most = 0;
+    for (const int dtype : {AWQ_F16, AWQ_BF16}) {
+        awq::RowsPlan rows;
+        const size_t b = rows_wanted(M, N, K, 32, dtype, &rows) ? awq::rows_ws_bytes(rows, M, N) : 0;
+        most = most > b ? most : b;
+    }
+    return most;
 }
 
 // 65..128 rows go to the GEMV (blocks of 16 rows) on weights up to this size, see kGemvMaxRows in awq_gemv.hip
@@ -545,9 +563,7 @@ extern "C" size_t awq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
         const size_t c = awq_gemv_workspace_bytes(16, N, K);
         a = a > c ? a : c;
     }
-    awq::RowsPlan rows;       // (the largest over the group sizes: they only decide whether it runs)
-    const size_t d = rows_wanted(M, N, K, 32, &rows) ? awq::rows_ws_bytes(rows, M, N) : 0;
-    const size_t most = a > b ? a : b;
+    const size_t d = rows_workspace_bytes(M, N, K), most = a > b ? a : b;
     return most > d ? most : d;
 }
 
@@ -555,13 +571,18 @@ extern "C" size_t awq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 // 4096 x 12288 at 512 rows 74 / 69 us, 2048 rows 224 / 186, 8192 rows 787 / 575; 12288 x 4096 at 512 rows (32 tiles cut in
 // eight) 71 / 136, 2048 rows 209 / 176, 8192 rows 744 / 568; 1024 x 2048 at 4096 rows 43 / 28; 2560 x 9728 at 333 rows
 // 45 / 44, 8192 rows 441 / 309.
-extern "C" size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size) {
-    if (always_fused(M, K)) return 0;
+extern "C" size_t awq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype) {
+    if (always_fused(M, K) || (dtype != AWQ_F16 && dtype != AWQ_BF16)) return 0;
     const double dense = awq::dense_linear_us(M, N, K, group_size);
     if (dense < 0) return 0;
     awq::RowsPlan rows;
-    return dense < fused_linear_us(M, N, K) && !rows_wanted(M, N, K, group_size, &rows)
+    return dense < fused_linear_us(M, N, K, group_size, dtype) && !rows_wanted(M, N, K, group_size, dtype, &rows)
                ? awq_linear_dense_scratch_bytes(M, N, K, group_size) : 0;
+}
+
+extern "C" size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size) {
+    const size_t a = awq_linear_scratch_bytes(M, N, K, group_size, AWQ_F16);
+    return a ? a : awq_linear_scratch_bytes(M, N, K, group_size, AWQ_BF16);
 }
 
 extern "C" size_t awq_linear_swiglu_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -570,8 +591,7 @@ extern "C" size_t awq_linear_swiglu_workspace_bytes(int64_t M, int64_t N, int64_
     int v, s;
     awq::plan_gemm_tile256(M, N, K, 128, AWQ_F16, &v, &s);   // the workspace is the same for both 256 x 256 kernels
     const size_t b = awq::gemm_ws_bytes(M, N, K, v, s);
-    awq::RowsPlan rows;
-    const size_t d = rows_wanted(M, N, K, 32, &rows) ? awq::rows_ws_bytes(rows, M, N) : 0, most = a > b ? a : b;
+    const size_t d = rows_workspace_bytes(M, N, K), most = a > b ? a : b;
     return most > d ? most : d;
 }
 
@@ -587,7 +607,7 @@ extern "C" int awq_linear_swiglu(const void* x, const int32_t* qweight, const vo
     if (K >= awq::kBK && N >= 16 && M >= 1 && group_size > 0)
         awq::plan_gemm_tile256(M, N, K, group_size, dtype, &v, &s);
     awq::RowsPlan rows;       // as awq_linear on the same sizes, whose bits the gated product has
-    if (M > 128 && N >= 16 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, &rows))
+    if (M > 128 && N >= 16 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
         v = awq::kRowsVariant, s = rows.splits;
     return awq::gemm_dispatch("awq_linear_swiglu", x, qweight, qscales, qzeros, nullptr, y, M, N, K, group_size,
                               dtype, workspace, workspace_bytes, stream, v, s, 1);
@@ -616,10 +636,10 @@ extern "C" const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t
     if (gated ? M <= 64 && staged : regime == Regime::gemv) return "gemv";
     if (!gated && regime == Regime::gemv_blocks) return "gemv in blocks of 16 rows";
     if (K % awq::kBK != 0 || !(group_size % 64 == 0 || (64 % group_size == 0 && group_size % 8 == 0))) return "";
-    if (awq_linear_dense_wanted_bytes(M, N, K, group_size)) return "dense";
+    if (awq_linear_scratch_bytes(M, N, K, group_size, dtype)) return "dense";
     int variant;
     awq::RowsPlan rows;
-    if (rows_wanted(M, N, K, group_size, &rows)) variant = awq::kRowsVariant, *split_k = rows.splits;
+    if (rows_wanted(M, N, K, group_size, dtype, &rows)) variant = awq::kRowsVariant, *split_k = rows.splits;
     else if (gated) awq::plan_gemm_tile256(M, N, K, group_size, dtype, &variant, split_k);
     else awq::plan_gemm(M, N, K, group_size, dtype, &variant, split_k);
     return awq::kGemmVariants[variant].name;
@@ -645,7 +665,7 @@ extern "C" int awq_linear(const void* x, const int32_t* qweight, const void* qsc
         return AWQ_OK;
     }
     awq::RowsPlan rows;
-    if (M > 128 && N >= 8 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, &rows))
+    if (M > 128 && N >= 8 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
         return awq::gemm_dispatch("awq_linear", x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,
                                   workspace_bytes, stream, awq::kRowsVariant, rows.splits);
     return awq_gemm(x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,

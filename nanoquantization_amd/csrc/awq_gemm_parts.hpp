@@ -245,12 +245,12 @@ hipError_t launch_dequant_transpose(int dtype, const PackedWeight& w, const Pack
 double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g);
 
 // awq_gemm_rows.hip: tiles of 80..128 rows by 128 columns for a few hundred rows; `us` an estimate of the time, m_tiles 0 where
-// it does not take the sizes.  split_k 0: the split with the least estimate.
+// it does not take the sizes.  split_k 0: the split with the least estimate, which depends on the type.
 struct RowsPlan {
     int m_tiles, n_tiles, mt, splits, steps_per_split;   // mt: 16-row tiles of a workgroup; steps: of 64 rows of K
     double us;
 };
-RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int split_k = 0);
+RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, int split_k = 0);
 inline size_t rows_ws_bytes(const RowsPlan& p, int64_t M, int64_t N) {
     return p.splits > 1 ? kCounterBytes + (size_t)p.splits * M * N * sizeof(float) : 0;
 }

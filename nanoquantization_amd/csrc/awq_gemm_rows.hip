@@ -370,7 +370,7 @@ hipError_t launch(const RowsPlan& p, const void* x, const int32_t* qweight, cons
 
 }  // namespace
 
-RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int split_k) {
+RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, int split_k) {
     RowsPlan p{};
     // 32-bit offsets into x, the words and the scales
     if (M < 1 || N < 8 || N % 8 != 0 || K < 64 || K % 64 != 0 || g < 32 || g % 32 != 0 || K % g != 0 ||
@@ -379,10 +379,13 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int split_k)
     const int64_t m_tiles = cdiv(M, 128), n_tiles = cdiv(N, 128), steps = K / 64;
     p.m_tiles = (int)m_tiles, p.n_tiles = (int)n_tiles;
     p.mt = (int)std::max<int64_t>(5, cdiv(cdiv(M, m_tiles), 16));
-    // A round of 256 workgroups: 0.085 us a stage and 16 rows, 5 to fill the ring and store; a K split writes its fp32 sums and
-    // reads them again in a second launch.
+    // A round of 256 workgroups: a stage by type and MT, 6 us to fill the ring and store; a K split writes its fp32 sums and reads
+    // them again in a second launch.  The stages are measured (16 weights of 2048 to 25600 rows, 129 to 640 rows of x, within
+    // 10 % of every time): with few rows the unpacking outlasts the matrix instructions, in bf16 more than in fp16.
+    constexpr double kStage[2][4] = {{0.47, 0.455, 0.53, 0.57}, {0.56, 0.57, 0.62, 0.635}};     // [fp16, bf16][MT - 5]
+    const double stage = kStage[dtype == AWQ_F16 ? 0 : 1][p.mt - 5];
     const auto us = [&](int64_t s) {
-        return (double)cdiv(m_tiles * n_tiles * s, 256) * (0.085 * p.mt * (double)cdiv(steps, s) + 5) +
+        return (double)cdiv(m_tiles * n_tiles * s, 256) * (stage * (double)cdiv(steps, s) + 6) +
                (s > 1 ? 2.5 + (double)s * (double)(M * N) * 8 / 5.0e6 : 0);
     };
     int64_t best = 1;

@@ -98,10 +98,10 @@ at::Tensor workspace(const at::Device& dev, void* stream, size_t nbytes) {
     return ws;
 }
 
-// Scratch for awq_linear_dense where that is the faster way, else undefined.  From the caching allocator for this one call
+// Scratch for awq_linear_dense where that is the fastest way, else undefined.  From the caching allocator for this one call
 // (ordered on the current stream like any temporary); without room for it the fused kernels run.
 at::Tensor dense_scratch(const at::Device& dev, int64_t M, const Packed& p) {
-    const size_t nbytes = M > 128 ? awq_linear_dense_wanted_bytes(M, p.N, p.K, p.g) : 0;
+    const size_t nbytes = M > 128 ? awq_linear_scratch_bytes(M, p.N, p.K, p.g, p.dtype) : 0;
     if (!nbytes) return {};
     try {
         return at::empty({(int64_t)nbytes}, at::TensorOptions().dtype(at::kByte).device(dev));

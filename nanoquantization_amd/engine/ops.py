@@ -342,7 +342,7 @@ def awq_linear_swiglu(x: torch.Tensor, qweight: torch.Tensor, qscales: torch.Ten
     L = _lib.lib()
     with _lib.on_device(dev):
         stream = _stream(dev)
-        scratch = _lib.dense_scratch(dev, M, N, K, g) if M > 128 else None
+        scratch = _lib.dense_scratch(dev, M, N, K, g, _lib.dtype_id(x.dtype)) if M > 128 else None
         if scratch is not None:
             _lib.check(L.awq_linear_dense(x.data_ptr(), qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(), None,
                                           out.data_ptr(), M, N, K, g, _lib.dtype_id(x.dtype), 1, scratch.data_ptr(),

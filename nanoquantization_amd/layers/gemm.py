@@ -98,7 +98,7 @@ def _linear(entry: str, x, qweight, qscales, qzeros, bias, extra=()):
     L = _lib.lib()
     with _lib.on_device(dev):
         stream = _lib.current_stream_ptr(dev)
-        scratch = _lib.dense_scratch(dev, M, N, K, g) if entry == "awq_linear" and M > 128 else None
+        scratch = _lib.dense_scratch(dev, M, N, K, g, _lib.dtype_id(dt)) if entry == "awq_linear" and M > 128 else None
         if scratch is not None:
             _lib.check(L.awq_linear_dense(x.data_ptr(), qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(), _ptr(bias),
                                           out.data_ptr(), M, N, K, g, _lib.dtype_id(dt), 0, scratch.data_ptr(),

@@ -358,3 +358,50 @@ def test_bench_refuses_more_than_one_gpu():
     p = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True,
                        timeout=300)
     assert p.returncode != 0 and "one GPU" in p.stderr and p.stdout.strip() == ""
+
+
+def _route(L, M, K, N, g, dtype, gated=0):
+    s = ctypes.c_int(-1)
+    return L.awq_linear_route(M, N, K, g, dtype, gated, ctypes.byref(s)).decode(), s.value
+
+
+def test_linear_routes():
+    """Host-only: the route of a linear at sizes where the ways were timed against each other (a way that is slower by a tenth is
+    not taken), and over a sweep that the sizes of workspace and scratch go with it."""
+    _ensure_built()
+    L, f16, bf16 = _lib.lib(), _lib.AWQ_F16, _lib.AWQ_BF16
+    for M, K, N, g, dtype, want in (
+            (129, 5120, 10240, 128, bf16, "256x256p"), (192, 5120, 10240, 128, bf16, "256x256p"),      # 46 us; rows128 53, 51
+            (129, 25600, 5120, 128, bf16, "256x256p"),                                                 # 77; 86
+            (600, 4096, 24576, 128, f16, "256x256rt"), (900, 4096, 24576, 128, f16, "256x256rt"),      # 138, 185; dense 160, 214
+            (900, 2048, 16384, 128, f16, "256x256r"), (640, 5120, 34816, 128, f16, "256x256rt"),       # 60, 269; dense 67, 284
+            (333, 2816, 9720, 64, f16, "rows128"), (333, 2816, 9720, 64, bf16, "rows128"),             # 30, 34; fused 46
+            (200, 4096, 4096, 128, bf16, "rows128"), (160, 12288, 4096, 128, bf16, "rows128"),         # 25, 39; fused 29, 46
+            (256, 12288, 4096, 128, f16, "rows128"), (512, 4096, 4096, 128, f16, "rows128"),           # 43, 33; fused 51, 44
+            (8192, 4096, 12288, 128, f16, "dense"), (8192, 4096, 12288, 128, bf16, "dense"),           # 575; fused 730, 787
+            (2048, 12288, 4096, 128, bf16, "dense"), (512, 12288, 4096, 128, bf16, "256x256p"),        # 176, 71; fused 209, dense 136
+            (1024, 1024, 4096, 128, bf16, "256x256p"),                                                 # short K
+            (16, 1024, 3072, 128, f16, "gemv"), (100, 1024, 1024, 128, f16, "gemv"), (100, 5120, 25600, 128, f16, "128x128"),
+            (40, 96, 512, 32, f16, "gemv in blocks of 16 rows"), (300, 192, 520, 24, f16, "")):
+        assert _route(L, M, K, N, g, dtype)[0] == want, (M, K, N, g, dtype, _route(L, M, K, N, g, dtype))
+    names = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())]
+    for K in (64, 1024, 1984, 2048, 4096, 5120, 12288, 25600):
+        for N in (8, 136, 1032, 4096, 12288, 24576, 34816):
+            for M in (1, 17, 128, 129, 160, 200, 257, 333, 512, 640, 1100, 2048, 2049, 8192):
+                both = [L.awq_linear_scratch_bytes(M, N, K, 64, d) for d in (f16, bf16)]
+                assert L.awq_linear_dense_wanted_bytes(M, N, K, 64) == max(both)
+                for g in (8, 32, 64):
+                    for d in (f16, bf16):
+                        for gated in (0, 1):
+                            name, split = _route(L, M, K, N, g, d, gated)
+                            scratch = L.awq_linear_scratch_bytes(M, N, K, g, d)
+                            if gated and N % 16:
+                                assert name == ""
+                                continue
+                            assert (name == "dense") == (scratch > 0), (M, K, N, g, d)
+                            if scratch:
+                                assert scratch == L.awq_linear_dense_scratch_bytes(M, N, K, g)
+                            elif name in names:
+                                need = L.awq_gemm_ex_workspace_bytes(M, N, K, names.index(name), split)
+                                has = (L.awq_linear_swiglu_workspace_bytes if gated else L.awq_linear_workspace_bytes)(M, N, K)
+                                assert need <= has, (M, K, N, g, d, name, split)
