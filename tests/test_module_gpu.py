@@ -220,3 +220,52 @@ def test_norm_result_keeps_the_layout(layout):
         got, want = norm(x), norm.rms_norm(x)
     assert got.stride() == want.stride()
     assert ((got.float() - want.float()).abs() <= 2.0 ** -6 * want.float().abs() + 1e-6).all()      # one place each, as above
+
+
+# one to nine key tiles of 64 (32 at a head dim of 256), one to four query tiles of 128, several sequences of each
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("b,s", [(2, 127), (3, 128), (2, 129), (3, 257), (2, 450), (1, 513)])
+def test_causal_attention_tiles(hd, b, s):
+    """Attention of whole sequences over several tiles against softmax in fp64, the running maximum rising along the keys.  Weights
+    and output are each rounded once, and 2^-8 relative covers both; two runs give the same bits."""
+    from nanoquantization_amd import _lib
+    print(f"causal attention hd={hd} {b}x{s}", flush=True)
+    heads, kv, bf = 6, 2, torch.bfloat16
+    gen = torch.Generator(device="cuda").manual_seed(hd + s)
+    q = torch.randn(b, s, heads, hd, device="cuda", generator=gen).to(bf)
+    k, v = (torch.randn(b, kv, s, hd, device="cuda", generator=gen) for _ in range(2))
+    k, v = (k * (1 + torch.arange(s, device="cuda") / 100).view(-1, 1)).to(bf), v.to(bf)
+    for scale in (hd ** -0.5, -hd ** -0.5):
+        o = _lib.torch_ops().causal_attention(q, k, v, scale)
+        rep = lambda t: t.double().repeat_interleave(heads // kv, 1)
+        sc = q.transpose(1, 2).double() @ rep(k).transpose(-1, -2) * scale
+        w = sc.masked_fill(torch.ones(s, s, dtype=torch.bool, device="cuda").triu(1), float("-inf")).softmax(-1)
+        ref = (w @ rep(v)).transpose(1, 2).reshape(b, s, heads * hd)
+        size = (w @ rep(v).abs()).transpose(1, 2).reshape(b, s, heads * hd)
+        assert ((o.double() - ref).abs() <= 2.0 ** -8 * (size + ref.abs())).all()
+        assert torch.equal(o, _lib.torch_ops().causal_attention(q, k, v, scale))
+
+
+def test_prompt_forward_of_many_tiles(monkeypatch):
+    """Several sequences of several attention tiles, rows enough that gate and up are one product: the same hidden states as on
+    torch operations, to the few roundings that fall differently."""
+    from nanoquantization_amd import _lib
+    from nanoquantization_amd.models.qwen3_quantized import Qwen3QuantizedForCausalLM
+    b, s, hidden, inter = 3, 700, 512, 1024
+    assert _lib.lib().awq_linear_route(b * s, 2 * inter, hidden, 128, _lib.AWQ_BF16, 1, None) == b"dense"
+    m = Qwen3QuantizedForCausalLM(num_hidden_layers=2, vocab_size=128, hidden_size=hidden, total_num_heads=6, total_num_kv_heads=2,
+                                  max_position_embeddings=1024, intermediate_size=inter, head_dim=128).to(torch.bfloat16)
+    torch.manual_seed(0)
+    for mod in m.modules():
+        if isinstance(mod, nq.WQLinear_GEMM):
+            mod.qweight.random_(-2 ** 31, 2 ** 31 - 1)
+            mod.qzeros.random_(-2 ** 31, 2 ** 31 - 1)
+            mod.qscales.uniform_(0.002, 0.006)
+    m = m.cuda()
+    ids, pos = torch.randint(0, 128, (b, s), device="cuda"), torch.arange(s, device="cuda")
+    with torch.no_grad():
+        got = m(ids, pos)
+        assert torch.equal(got, m(ids, pos))
+        _eager(monkeypatch)
+        want = m(ids, pos)
+    assert (got.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
