@@ -532,7 +532,7 @@ static bool rows_wanted(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, a
     if (always_fused(M, K)) return false;
     *plan = awq::make_rows_plan(M, N, K, g, dtype);
     if (plan->m_tiles == 0 || (int64_t)plan->m_tiles * plan->n_tiles * plan->splits > 256 ||
-        plan->us >= 0.96 * fused_linear_us(M, N, K, g, dtype))
+        plan->us >= 0.95 * fused_linear_us(M, N, K, g, dtype))
         return false;
     const double dense = awq::dense_linear_us(M, N, K, g);
     return dense < 0 || plan->us < 0.95 * dense;

@@ -372,7 +372,7 @@ def test_linear_routes():
     L, f16, bf16 = _lib.lib(), _lib.AWQ_F16, _lib.AWQ_BF16
     for M, K, N, g, dtype, want in (
             (129, 5120, 10240, 128, bf16, "256x256p"), (192, 5120, 10240, 128, bf16, "256x256p"),      # 46 us; rows128 53, 51
-            (129, 25600, 5120, 128, bf16, "256x256p"),                                                 # 77; 86
+            (129, 25600, 5120, 128, bf16, "256x256p"), (129, 17408, 5120, 128, bf16, "256x256p"),      # 77, 58; 86, 62
             (600, 4096, 24576, 128, f16, "256x256rt"), (900, 4096, 24576, 128, f16, "256x256rt"),      # 138, 185; dense 160, 214
             (900, 2048, 16384, 128, f16, "256x256r"), (640, 5120, 34816, 128, f16, "256x256rt"),       # 60, 269; dense 67, 284
             (333, 2816, 9720, 64, f16, "rows128"), (333, 2816, 9720, 64, bf16, "rows128"),             # 30, 34; fused 46
