@@ -192,7 +192,7 @@ _torch_ops = None
 
 def torch_ops():
     """torch.ops.nanoquantization_amd: the operators of csrc/torch_binding.cpp (awq_dequantize, awq_linear,
-    awq_linear_swiglu), registered with the dispatcher by loading libawq_torch.so.  Raises if it has not been built."""
+    awq_linear_swiglu; between the linears awq_swiglu_pair, rms_norm, silu_mul, qkv_norm_rope, causal_attention), registered with the dispatcher by loading libawq_torch.so.  Raises if it has not been built."""
     global _torch_ops
     if _torch_ops is None:
         lib()                                           # libawq_hip.so first: the binding links against it

@@ -518,16 +518,16 @@ static double fused_linear_us(int64_t M, int64_t N, int64_t K, int64_t g, int dt
     return regb && dtype == AWQ_F16 && (slices == 0 || p.full_tiles + slices > 256) ? 0.9 * us : us;
 }
 
-// Short K at up to 2048 rows stays fused: awq_gemm_plan's kernel and K split are what a caller gets there, bit for bit, and
-// the difference is a few microseconds (1024 x 4096 at 1024 rows 31 / 22 us dequantised first).
+// Short K at up to 2048 rows stays fused, although dequantising first would often be faster (1024 x 4096 at 1024 rows 31 / 22
+// us): callers get awq_gemm_plan's kernel and K split there, bit for bit.
 static bool always_fused(int64_t M, int64_t K) { return M <= 128 || (M <= 2048 && K < 2048); }
 
 // Whether the tiles of awq_gemm_rows.hip are the fastest way, from the estimates of all three; in one round of the CUs only
 // (5120 x 25600 at 160 rows, 400 tiles: 85 us in fp16 and 101 in bf16 against 85 fused).  The estimates know the type: 5120 x
 // 10240 at 129 to 192 rows takes 51-53 us in bf16 here and 46 fused, 41-43 in fp16 against 43-45.  Measured, fp16 / bf16 and the faster
-// of the other two: 2816 x 9720 at 333 rows 31 / 34 us against 46, 4096 x 4096 at 200 rows 24 / 25 against 29, at 512 rows
-// 33 / 36 against 41, 12288 x 4096 at 160 rows 35 / 39 against 46, 8192 x 1024 at 1024 rows 36 / 38 against 42, 2048 x 6144 at
-// 640 rows 26 / 27 against 34.
+// of the other two: 2816 x 9720 at 300 rows 30 / 34 us against 45, 4096 x 4096 at 192 rows 23 / 25 against 30, at 512 rows
+// 33 / 36 against 41, 12288 x 4096 at 160 rows 35 / 40 against 46, 8192 x 1024 at 1024 rows 36 / 38 against 42, 2048 x 6144 at
+// 640 rows 25 / 28 against 34.
 static bool rows_wanted(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, awq::RowsPlan* plan) {
     if (always_fused(M, K)) return false;
     *plan = awq::make_rows_plan(M, N, K, g, dtype);
@@ -567,10 +567,10 @@ extern "C" size_t awq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     return most > d ? most : d;
 }
 
-// Whether dequantising the weight first (awq_linear_dense) is the faster way.  Measured, bf16, fused / dequantised first:
-// 4096 x 12288 at 512 rows 74 / 69 us, 2048 rows 224 / 186, 8192 rows 787 / 575; 12288 x 4096 at 512 rows (32 tiles cut in
-// eight) 71 / 136, 2048 rows 209 / 176, 8192 rows 744 / 568; 1024 x 2048 at 4096 rows 43 / 28; 2560 x 9728 at 333 rows
-// 45 / 44, 8192 rows 441 / 309.
+// Whether dequantising the weight first (awq_linear_dense) is the faster way.  Measured, bf16 (fp16), fused / dequantised first:
+// 4096 x 12288 at 512 rows 76 / 70 us (72 / 69), 2048 rows 209 / 182 (198 / 191), 8192 rows 732 / 564 (698 / 593); 12288 x
+// 4096 at 512 rows (32 tiles cut in eight) 69 / 136, 2048 rows 202 / 174 (193 / 181), 8192 rows 751 / 556 (709 / 580); 2560 x
+// 9728 at 300 rows 44 / 43, 8192 rows 388 / 292 (370 / 312).
 extern "C" size_t awq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype) {
     if (always_fused(M, K) || (dtype != AWQ_F16 && dtype != AWQ_BF16)) return 0;
     const double dense = awq::dense_linear_us(M, N, K, group_size);

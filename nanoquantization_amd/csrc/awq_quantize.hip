@@ -1,7 +1,8 @@
 // Offline path on the device: per-group asymmetric 4-bit min/max quantisation of an fp32 weight
 // [N, K] fused with the AWQ packing, producing qweight [K, N/8], qzeros [K/g, N/8] and qscales
-// [K/g, N] directly.  The arithmetic is the reference's, operation by operation in fp32 (true
-// divisions, round-half-to-even), so the words equal those of its quantise -> transpose -> pack chain.
+// [K/g, N] directly.  The words equal those of the reference's quantise -> transpose -> pack chain in fp32 (round half
+// to even): step size and zero point by its operations, codes by a product with the reciprocal that is decided by the
+// division wherever the two could round apart (code_of).
 #include <type_traits>
 
 #include "awq_common.hpp"

@@ -1,6 +1,6 @@
 // Mixture of experts: router, grouping of (row, choice) pairs by expert, and the two grouped products.
 //
-// The grouped products exist in three forms, chosen by pairs per expert and operand alignment (moe_form):
+// The grouped products exist in four forms, chosen by pairs per expert and operand alignment (moe_form):
 //   few pairs    tiles of 16, 32 or 64 pairs on the skinny core: the weights stream once, straight into MFMA operands
 //   many pairs   tiles of 64 or 128 pairs x 128 weight rows staged through LDS by load-to-LDS, double-buffered, MFMA 16x16x32
 //   most pairs   tiles of 128 or 256 pairs x 256 weight rows on the product core of pingpong.hpp (rows in whole stages of 64)
@@ -339,8 +339,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const uint16_t* __restric
 // ---- most pairs per expert: XR = 128 or 256 pairs x 256 weight rows per workgroup -------------------------------
 // A gathered row is one 32-bit offset per lane and load, so the gather costs nothing in the loop.  GATED: 128 gate rows and
 // their 128 up rows; a wave's first tiles are gate, the others the up rows of the same columns.  The same sums in the same
-// order as moe_gemm_kernel.  16,384 pairs of 8 experts, 4096 -> 2 x 6144 and back: 2805 us
-// with moe_gemm_kernel, 2007 like this.
+// order as moe_gemm_kernel.  16,384 pairs of 8 experts, 4096 -> 2 x 6144 and back: 2890 us
+// with moe_gemm_kernel, 1950 like this.
 template <bool GATED, int XR>
 __global__ __launch_bounds__(512, 2) void moe_pingpong_kernel(const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
                                                               const float* __restrict__ weight,
@@ -421,9 +421,10 @@ MoeForm moe_form(int64_t pairs, int64_t experts, int64_t width, int64_t ff, int 
     if (pairs <= 40 * experts || pairs <= 64) return MoeForm::skinny64;
     // The ping-pong core wants whole stages and 32-bit offsets into the rows and into an expert's weights, pairs per expert that
     // fill its tiles, and 128 workgroups in the smaller of the two products.  Both products, gemm / 128 / 256 pairs a tile:
-    // 4096 -> 2 x 6144, 8 experts, 192 pairs each 535 / 472 / 501 us, 512 each 898 / 793 / 743, 2048 each 2805 / - / 2007;
-    // 2048 -> 2 x 1024, 64 experts, 144 each 311 / 319 / 385, 192 each 363 / 335 / 416, 384 each 530 / 488 / 447;
-    // 1024 -> 2 x 1536, 8 experts, 256 each 50 / 61 / 65 (80 workgroups), 512 each 72 / 65 / 93, 1024 each 122 / - / 101.
+    // 4096 -> 2 x 6144, 8 experts, 192 pairs each 543 / 358 / 357 us, 512 each 947 / 754 / 673, 2048 each 2890 / 2401 / 1948;
+    // 2048 -> 2 x 1024, 64 experts, 144 each 318 / 277 / 236, 192 each 370 / 274 / 243, 384 each 529 / 422 / 376;
+    // 1024 -> 2 x 1536, 8 experts, 256 each 49 / 45 / 63 (80 workgroups), 512 each 69 / 63 / 69, 1024 each 120 / 122 / 100.
+    // The lines are on the safe side: with many experts the larger tiles are ahead some way below them.
     const bool stages = width % 64 == 0 && ff % 64 == 0 && pairs * std::max(width, ff) * 2 < (1ll << 32) &&
                         width * ff * 4 < (1ll << 32);
     const int64_t groups = std::min(cdiv(width, 256), cdiv(ff, 128));

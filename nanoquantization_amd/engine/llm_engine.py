@@ -139,8 +139,9 @@ class LLMEngine(EngineCore):
     @torch.no_grad()
     def _prefill_ragged(self, prompts: List[List[int]], leases: List[Lease]) -> torch.Tensor:
         """Prompts of any lengths in one pass: every per-token operation (norms, AWQ linears, rotary, cache write)
-        runs once over the concatenated tokens, the causal attention once per prompt over its own slice.  Returns the
-        next token of every prompt [len(prompts)]."""
+        runs once over the concatenated tokens; the causal attention over the cache it has just written in one launch as
+        well (in float16, and at head dims without a matrix form, torch's once per prompt over its own slice).  Returns
+        the next token of every prompt [len(prompts)]."""
         m, bs, eps = self.model.model, self.block_size, self.eps
         dev = self.device
         lens = [len(p) for p in prompts]

@@ -36,9 +36,10 @@ class RoPE(nn.Module):
         return torch.cat([x1 * cos - x2 * sin, x1 * sin + x2 * cos], dim=-1).to(x.dtype)
 
     def refuse_unknown(self, position_ids: torch.Tensor) -> None:
-        """torch's own index error for positions outside the table, as `forward` has it, from one element a position: the
-        operator that takes this module's place reads the table itself and has no way to raise."""
-        self.cos_sin_cache[:, 0, 0][position_ids]
+        """torch's own index error for positions outside the table, as `forward` has it: the operator that takes this module's
+        place reads the table itself and has no way to raise.  It looks up one element a position among as many neighbouring
+        elements as the table has rows (2048 positions 5.7 us; an element of each row, 512 bytes apart, 6.6)."""
+        self.cos_sin_cache.flatten()[:self.cos_sin_cache.shape[0]][position_ids]
 
     def forward(self, query: torch.Tensor, key: torch.Tensor, position_ids: torch.Tensor):
         """query/key: [batch, seq, heads, head_dim]; position_ids: [batch, seq] (or broadcastable)."""
