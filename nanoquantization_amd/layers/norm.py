@@ -25,7 +25,7 @@ class RMSNorm(nn.Module):
 
     def _one_kernel(self, x: torch.Tensor) -> bool:
         # a workgroup per row: rows of a few hundred elements (the heads') leave most of it idle
-        return (type(self) is RMSNorm and keeps(self, RMSNorm, "rms_norm") and plain(x, self.weight) and 512 <= self.weight.numel() <= 8192
+        return (type(self) is RMSNorm and plain(x, self.weight) and keeps(self, RMSNorm, "rms_norm") and 512 <= self.weight.numel() <= 8192
                 and self.weight.numel() % 8 == 0 and x.shape[-1:] == self.weight.shape)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

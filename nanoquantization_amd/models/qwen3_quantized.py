@@ -70,26 +70,31 @@ class Qwen3QuantizedAttention(nn.Module):
                 and self.rope.cos_sin_cache.is_contiguous() and pos.device == q.device == self.rope.cos_sin_cache.device
                 and unhooked(self.q_norm, self.k_norm, self.rope))
 
-    def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
-        bs = x.shape[0]
-        own = keeps(self, Qwen3QuantizedAttention, "qkv")
-        q, k, v = (self.q_proj(x), self.k_proj(x), self.v_proj(x)) if own else self.qkv(x, position_ids)
-        if own and self._fused(q, k, v, position_ids):
-            pos = (position_ids if position_ids.dim() == 2 else position_ids.unsqueeze(0)).to(torch.int64)
-            self.rope.refuse_unknown(pos)
-            q, k, v = _lib.torch_ops().qkv_norm_rope(q, k, v, self.q_norm.weight, self.k_norm.weight, self.rope.cos_sin_cache,
-                                                     pos, self.num_heads, self.num_kv_heads, self.q_norm.eps,
-                                                     self.k_norm.eps)
-            if q.dtype == torch.bfloat16:
-                return self.o_proj(_lib.torch_ops().causal_attention(q, k, v, self.head_dim ** -0.5))
-        else:
-            if own:
-                q, k, v = self._norm_rope(q, k, v, position_ids)
-            k, v = k.transpose(1, 2), v.transpose(1, 2)
-        o = F.scaled_dot_product_attention(q.transpose(1, 2), k, v, is_causal=True,
+    def _attend(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+        """Causal attention and output projection of what `qkv` returns."""
+        o = F.scaled_dot_product_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), is_causal=True,
                                            enable_gqa=self.num_heads != self.num_kv_heads)
-        o = o.transpose(1, 2).reshape(bs, -1, self.num_heads * self.head_dim)
-        return self.o_proj(o)
+        return self.o_proj(o.transpose(1, 2).reshape(q.shape[0], -1, self.num_heads * self.head_dim))
+
+    def _on_operators(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
+        q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        if not self._fused(q, k, v, position_ids):
+            q, k, v = self._norm_rope(q, k, v, position_ids)
+            return self._attend(q, k, v)
+        pos = (position_ids if position_ids.dim() == 2 else position_ids.unsqueeze(0)).to(torch.int64)
+        self.rope.refuse_unknown(pos)
+        q, k, v = _lib.torch_ops().qkv_norm_rope(q, k, v, self.q_norm.weight, self.k_norm.weight, self.rope.cos_sin_cache, pos,
+                                                 self.num_heads, self.num_kv_heads, self.q_norm.eps, self.k_norm.eps)
+        if q.dtype == torch.bfloat16:
+            return self.o_proj(_lib.torch_ops().causal_attention(q, k, v, self.head_dim ** -0.5))
+        return self._attend(q, k.transpose(1, 2), v.transpose(1, 2))
+
+    def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
+        if not torch.jit.is_scripting():        # script sees the torch expressions only
+            if not torch.compiler.is_compiling() and keeps(self, Qwen3QuantizedAttention, "qkv"):
+                return self._on_operators(x, position_ids)
+        q, k, v = self.qkv(x, position_ids)
+        return self._attend(q, k, v)
 
 
 class Qwen3QuantizedMLP(nn.Module):
@@ -102,18 +107,23 @@ class Qwen3QuantizedMLP(nn.Module):
         self.gate_proj = mk(hidden_size, intermediate_size)
         self.down_proj = mk(intermediate_size, hidden_size)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def _activation(self, x: torch.Tensor) -> torch.Tensor:
         g, u = self.gate_proj, self.up_proj
         if (type(g) is type(u) is WQLinear_GEMM and plain(x, g.qscales, u.qscales) and g.bias is None and u.bias is None
                 and g.qweight.shape == u.qweight.shape and g.qscales.shape == u.qscales.shape and x.shape[-1] == g.qweight.shape[0]
                 and x.dim() > 1 and keeps(g, WQLinear_GEMM, "forward") and keeps(u, WQLinear_GEMM, "forward") and unhooked(g, u)):
             act = _lib.torch_ops().awq_swiglu_pair(x.reshape(-1, x.shape[-1]), g.qweight, g.qscales, g.qzeros, u.qweight, u.qscales,
                                                    u.qzeros)
-            return self.down_proj(act.view(*x.shape[:-1], act.shape[-1]))
+            return act.view(*x.shape[:-1], act.shape[-1])
         gate, up = self.gate_proj(x), self.up_proj(x)
         if plain(gate, up) and gate.shape == up.shape and gate.shape[-1] % 8 == 0:
-            return self.down_proj(_lib.torch_ops().silu_mul(gate, up))
-        return self.down_proj(F.silu(gate) * up)
+            return _lib.torch_ops().silu_mul(gate, up)
+        return F.silu(gate) * up
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if not torch.jit.is_scripting():        # script sees the torch expression only
+            return self.down_proj(self._activation(x))
+        return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
 class Qwen3QuantizedBlock(nn.Module):

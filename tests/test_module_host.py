@@ -59,6 +59,29 @@ def test_mlp_can_be_traced_with_its_linears_as_leaves():
     assert sorted(called) == ["down_proj", "gate_proj", "up_proj"]
 
 
+class Product(torch.nn.Module):
+    def __init__(self, n, m):
+        super().__init__()
+        self.w = torch.nn.Parameter(torch.randn(n, m, generator=torch.Generator().manual_seed(n + m)))
+
+    def forward(self, x):
+        return x @ self.w
+
+
+@pytest.mark.parametrize("how", ["script", "trace", "compile"])
+def test_attention_and_mlp_on_other_linears(how):
+    """With linears that can be traced, scripted and compiled the modules can be as well, and give the same result."""
+    mlp, attn = Qwen3QuantizedMLP(64, 128, group_size=64), Qwen3QuantizedAttention(64, 4, 2, 32, head_dim=64, group_size=64)
+    mlp.gate_proj, mlp.up_proj, mlp.down_proj = Product(64, 128), Product(64, 128), Product(128, 64)
+    attn.q_proj, attn.k_proj, attn.v_proj, attn.o_proj = Product(64, 256), Product(64, 128), Product(64, 128), Product(256, 64)
+    x, pos = torch.randn(2, 5, 64, generator=torch.Generator().manual_seed(0)), torch.arange(5)
+    with torch.no_grad():
+        for module, args in ((mlp, (x,)), (attn, (x, pos)), (attn, (x, pos.expand(2, 5)))):
+            made = {"script": torch.jit.script, "trace": lambda m: torch.jit.trace(m, args),
+                    "compile": lambda m: torch.compile(m, backend="eager", fullgraph=True)}[how](module)
+            assert torch.allclose(made(*args), module(*args), rtol=1e-5, atol=1e-5)
+
+
 @pytest.fixture
 def operators(monkeypatch):
     """The operators' names in the order they were called, where every tensor counts as one they take; the tensors they return
