@@ -43,6 +43,7 @@ EXTRA = {
     # longer select as one v_and_or_b32 each
     "awq_gemm_pipe.hip": ["-fno-slp-vectorize"],
     "awq_gemm_regb.hip": ["-fno-slp-vectorize"],
+    "awq_gemm_rows.hip": ["-fno-slp-vectorize"],
 }
 
 

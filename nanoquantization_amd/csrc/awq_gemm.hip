@@ -213,7 +213,7 @@ static const GemmVariant kGemmVariants[] = {
     // pipelined kernel under these names too
     {"256x256r", 256, 256, 4},   // every tile cut split_k ways
     {"256x256rt", 256, 256, 4},  // split_k cuts only the tiles beyond the last full round of CUs
-    {"rows128", 128, 128, 4},    // awq_gemm_rows.hip, for a few hundred rows: awq_linear's choice alone (rows_wanted)
+    {"rows128", 128, 128, 4},    // awq_gemm_rows.hip, for 17 to a few hundred rows: awq_linear's choice alone (rows_wanted)
 };
 enum { k128x128 = 0, k64x256 = 1, k32x256 = 2 };
 constexpr int kPipeVariant = 3, kPipeTailVariant = 4, kRegbVariant = 5, kRegbTailVariant = 6, kRowsVariant = 7;
@@ -411,6 +411,13 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
         AWQ_GEMM_CASE(k64x256, 64, 256, 1, 4)
         AWQ_GEMM_CASE(k32x256, 32, 256, 1, 4)
         case kRowsVariant:
+            if (N < 128) {     // less than a tile's columns: the plain tiles, which take any width
+                e = dtype == AWQ_F16 ? launch_gemm<F16, 128, 128, 2, 2>(x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K,
+                                                                        (int)g, workspace, rows.splits, s)
+                                     : launch_gemm<BF16, 128, 128, 2, 2>(x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K,
+                                                                         (int)g, workspace, rows.splits, s);
+                break;
+            }
             e = launch_rows(rows, dtype, x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K, (int)g, workspace, act != 0, s);
             break;
         case kPipeVariant:
@@ -518,18 +525,23 @@ static double fused_linear_us(int64_t M, int64_t N, int64_t K, int64_t g, int dt
     return regb && dtype == AWQ_F16 && (slices == 0 || p.full_tiles + slices > 256) ? 0.9 * us : us;
 }
 
-// Short K at up to 2048 rows stays fused, although dequantising first would often be faster (1024 x 4096 at 1024 rows 31 / 22
-// us): callers get awq_gemm_plan's kernel and K split there, bit for bit.
-static bool always_fused(int64_t M, int64_t K) { return M <= 128 || (M <= 2048 && K < 2048); }
+// Short K on wide weights at 1024 to 2048 rows stays fused, although dequantising first would often be faster (1024 x 4096 at
+// 1024 rows 31 / 22 us): callers get awq_gemm_plan's kernel and K split there, bit for bit.  Fewer rows and narrower weights go by
+// the estimates (1024 x 1024 at 130 to 1500 rows 20-27 -> 13-17 us, 1024 x 6144 at 512 rows 33 -> 17).
+static bool always_fused(int64_t M, int64_t N, int64_t K) { return M <= 128 || (M >= 1024 && M <= 2048 && K < 2048 && N >= 4096); }
 
-// Whether the tiles of awq_gemm_rows.hip are the fastest way, from the estimates of all three; in one round of the CUs only
-// (5120 x 25600 at 160 rows, 400 tiles: 85 us in fp16 and 101 in bf16 against 85 fused).  The estimates know the type: 5120 x
-// 10240 at 129 to 192 rows takes 51-53 us in bf16 here and 46 fused, 41-43 in fp16 against 43-45.  Measured, fp16 / bf16 and the faster
-// of the other two: 2816 x 9720 at 300 rows 30 / 34 us against 45, 4096 x 4096 at 192 rows 23 / 25 against 30, at 512 rows
-// 33 / 36 against 41, 12288 x 4096 at 160 rows 35 / 40 against 46, 8192 x 1024 at 1024 rows 36 / 38 against 42, 2048 x 6144 at
-// 640 rows 25 / 28 against 34.
+// Whether the tiles of awq_gemm_rows.hip run.  17 to 128 rows: wherever they take the sizes and the GEMV does not (5120 x 25600 in
+// groups of 64 at 64 rows, bf16, 46 -> 41 us against the plain tiles, 5120 x 17408 44 -> 31, at 32 rows 29 -> 26, 15296 x 4680
+// at 18 rows 33 -> 23; 5120 x 25600 at 100 rows 69 -> 47, 25600 x 5120 at 80 rows 61 -> 42, 12288 x 4096 at 128 rows 34 -> 30).
+// From 129 rows where the estimates of all three ways say so, in one round of the CUs only; fp16 / bf16 and the faster of the
+// other two: 2816 x 9720 at 333 rows 30 / 30 us against 46, 4096 x 4096 at 200 rows 25 / 25 against 29, at 512 rows 33 / 35 against
+// 43, 12288 x 4096 at 160 rows 32 / 34 against 45, 2048 x 6144 at 640 rows 25 / 27 against 34.  Up to 192 rows of weights of 50 Mi
+// elements stay on the 256-row tile that holds them all, as callers know it (5120 x 10240 at 192 rows 46 us, here 45; 17408 x
+// 5120 at 129 rows 60 and 52).
 static bool rows_wanted(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, awq::RowsPlan* plan) {
-    if (always_fused(M, K)) return false;
+    if (M <= 16 || N < 128) return false;
+    if (M <= 128) return (*plan = awq::make_rows_plan(M, N, K, g, dtype)).m_tiles != 0;
+    if (always_fused(M, N, K) || (M <= 192 && K * N >= (50ll << 20))) return false;
     *plan = awq::make_rows_plan(M, N, K, g, dtype);
     if (plan->m_tiles == 0 || (int64_t)plan->m_tiles * plan->n_tiles * plan->splits > 256 ||
         plan->us >= 0.95 * fused_linear_us(M, N, K, g, dtype))
@@ -572,7 +584,7 @@ extern "C" size_t awq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 // 4096 at 512 rows (32 tiles cut in eight) 69 / 136, 2048 rows 202 / 174 (193 / 181), 8192 rows 751 / 556 (709 / 580); 2560 x
 // 9728 at 300 rows 44 / 43, 8192 rows 388 / 292 (370 / 312).
 extern "C" size_t awq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype) {
-    if (always_fused(M, K) || (dtype != AWQ_F16 && dtype != AWQ_BF16)) return 0;
+    if (always_fused(M, N, K) || (dtype != AWQ_F16 && dtype != AWQ_BF16)) return 0;
     const double dense = awq::dense_linear_us(M, N, K, group_size);
     if (dense < 0) return 0;
     awq::RowsPlan rows;
@@ -607,7 +619,7 @@ extern "C" int awq_linear_swiglu(const void* x, const int32_t* qweight, const vo
     if (K >= awq::kBK && N >= 16 && M >= 1 && group_size > 0)
         awq::plan_gemm_tile256(M, N, K, group_size, dtype, &v, &s);
     awq::RowsPlan rows;       // as awq_linear on the same sizes, whose bits the gated product has
-    if (M > 128 && N >= 16 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
+    if (M > 16 && N >= 128 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
         v = awq::kRowsVariant, s = rows.splits;
     return awq::gemm_dispatch("awq_linear_swiglu", x, qweight, qscales, qzeros, nullptr, y, M, N, K, group_size,
                               dtype, workspace, workspace_bytes, stream, v, s, 1);
@@ -639,7 +651,9 @@ extern "C" const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t
     if (awq_linear_scratch_bytes(M, N, K, group_size, dtype)) return "dense";
     int variant;
     awq::RowsPlan rows;
-    if (rows_wanted(M, N, K, group_size, dtype, &rows)) variant = awq::kRowsVariant, *split_k = rows.splits;
+    if (rows_wanted(M, N, K, group_size, dtype, &rows))
+        // (up to 128 rows the tile's name is 128x128, whichever kernel awq_gemm runs on it)
+        variant = M > 64 && M <= 128 && !gated ? awq::k128x128 : awq::kRowsVariant, *split_k = rows.splits;
     else if (gated) awq::plan_gemm_tile256(M, N, K, group_size, dtype, &variant, split_k);
     else awq::plan_gemm(M, N, K, group_size, dtype, &variant, split_k);
     return awq::kGemmVariants[variant].name;
@@ -665,7 +679,7 @@ extern "C" int awq_linear(const void* x, const int32_t* qweight, const void* qsc
         return AWQ_OK;
     }
     awq::RowsPlan rows;
-    if (M > 128 && N >= 8 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
+    if (M > 16 && N >= 128 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
         return awq::gemm_dispatch("awq_linear", x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,
                                   workspace_bytes, stream, awq::kRowsVariant, rows.splits);
     return awq_gemm(x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,

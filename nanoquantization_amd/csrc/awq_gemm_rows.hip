@@ -1,57 +1,69 @@
-// y[M, N] = x[M, K] . dequantised W[K, N] (+ bias) for 129 to about 600 rows: too many for the GEMV, too few for 256 x 256 tiles
+// y[M, N] = x[M, K] . dequantised W[K, N] (+ bias) for 17 to about 1000 rows: too many for the GEMV, too few for 256 x 256 tiles
 // to cover the CUs (333 rows by 9720 columns are 76 of them) and for a dequantised weight to pay for its trip through memory.
 //
-// Workgroup: 16 MT rows (MT 5..8) by 128 columns, four waves, one a SIMD.  Wave (bh, kh): the even (bh 0) or odd columns of the
-// tile, the first (kh 0) or second 32 of every 64 rows of K; the two meet in LDS at the end.  That way no word is unpacked
-// twice in a workgroup, and a wave reads 16 MT rows of x from LDS for 64 columns: 64 of the 128 bytes a cycle at the full
-// matrix rate, where four waves side by side would need them all.
-// Stage (64 rows of K): x [16 MT rows][128 B], and per half words [32 rows][16], zero words and scales of the 16 word columns;
-// all load-to-LDS, kDepth stages in a ring, so five are on their way while one is multiplied (a stage is 0.2 us of matrix
-// instructions, a trip to HBM five times that).  The words of the stage after are unpacked to operands beside the matrix
-// instructions of this one: a wave alone on its SIMD has only its own instructions to put there.
+// Workgroup: 16 MT rows (MT 2..8) by 128 columns, eight waves.  Wave (turn, kh, bh): the even (bh 0) or odd columns of the tile,
+// the first (kh 0) or second 32 rows of K of every second stage of 64 (turn); the four parts of K meet in LDS at the end.  That
+// way no word is unpacked twice in a workgroup.  A SIMD has one wave of either turn, half a round apart: while one multiplies,
+// the other reads its next words and rows of x from LDS and unpacks the words to operands, and a barrier hands the roles over;
+// the unpacking (22 vector instructions in bf16, 14 in fp16 for 8 x 1 weights a lane) is as long as the matrix instructions of
+// seven (five) row tiles.  Up to four row tiles leave registers and LDS for two workgroups on a CU, which fill each other's waits.
+// Stage (64 rows of K): x [16 MT rows][128 B], words [2 halves][32 rows][16], scales and zero words of the two halves; all
+// load-to-LDS in pieces of 1 KiB, 16 bytes a lane, in a ring of kDepth stages.
 // Unpacked values are those of awq_dequantize, bit for bit.
-// Measured: 333 x 2816 x 9720 in fp16, groups of 64, 46 -> 30 us (590 TFLOP/s; without the loads from memory 26, so what holds
-// it is the one wave a SIMD, whose matrix instructions come every 19 ns where the CUs do one in 12); 200 x 4096 x 4096 in bf16
-// 29 -> 25, 160 x 12288 x 4096 46 -> 39, 512 x 2048 x 6144 34 -> 27.  Of the ways to get there: 37 us with all of a stage's LDS reads waited
-// for before the first unpacking, 31 with matrix instructions first; rows of x as two halves of 64 bytes a stage the same.
+// What bounds it: the phases, 0.35 us a stage at five rows tiles and 0.45 at eight, of which the matrix instructions take half; no
+// load is waited for (with all of them answered by zeros the time is the same), but asking for them is a fifth of a phase.
+// Measured: 333 x 2816 x 9720 in fp16, groups of 64, 29.8 -> 27.1 us against four waves that each unpack beside their own matrix
+// instructions, in bf16 34.9 -> 30.4; 640 x 2048 x 6144 in bf16 28 -> 26.  5120 x 25600 in groups of 64 at 64 rows, bf16, 46 -> 41 us
+// against the 64 x 256 tiles of awq_gemm.hip, 5120 x 17408 at 57 rows 44 -> 31 and at 32 rows 29 -> 25, 15296 x 4680 at 18 rows
+// 33 -> 23; 5120 x 25600 at 100 rows 69 -> 47 against its 128 x 128 tiles.
 #include "awq_common.hpp"
 #include "awq_gemm_parts.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 #define AWQ_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
+#define AWQ_GPTR(p) ((__attribute__((address_space(1))) const void*)(p))
 
 namespace awq {
 namespace {
 
-constexpr int kDepth = 6, kThreads = 256, kPad = 132;   // kPad: floats a row of the fp32 tile at the end
-constexpr int kHalf = 2048 + 256 + 1024;                 // words, zero words, scales of 32 rows of K
-constexpr int stage_bytes(int MT) { return MT * 2048 + 2 * kHalf; }
-constexpr int lds_bytes(int MT) { return kDepth * stage_bytes(MT); }
-static_assert(lds_bytes(5) >= 80 * kPad * 4 && lds_bytes(8) >= 128 * kPad * 4 && lds_bytes(8) <= 160 * 1024, "LDS");
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t resource(const void* p) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)0xFFFFFFFFu, 0x00020000);
+constexpr int kThreads = 512, kPad = 132;                 // kPad: floats a row of the fp32 tile at the end
+constexpr int stage_bytes(int MT) { return MT * 2048 + 4096 + 1024; }      // x, words, scales and zero words of 64 rows of K
+constexpr int per_cu(int MT) { return MT <= 4 ? 2 : 1; }                      // workgroups that share a CU
+// Four stages on the way while one is read: more take longer to ask for than they save (128 rows of 16384 columns, fp16, K of 128 /
+// 1024 / 4096: 9.5 / 16.8 / 38.8 us with seven to ten, 9.2 / 15.5 / 37.4 with four, 9.1 / 15.5 / 37.2 with three).
+constexpr int kDepth = 5;
+// 16 x 64 tiles that a wave gives away at the end, in the first and in the second exchange
+constexpr int pairs(int MT) { return (MT + 1) / 2; }
+constexpr int fours(int MT) { return (MT + 3) / 4; }
+constexpr int lds_bytes(int MT) {
+    return std::max({kDepth * stage_bytes(MT), 8 * 4096 * pairs(MT), 8 * 4096 * fours(MT) + 16 * MT * kPad * 4});
 }
+static_assert(2 * lds_bytes(2) <= 160 * 1024 && 2 * lds_bytes(3) <= 160 * 1024 && 2 * lds_bytes(4) <= 160 * 1024, "two on a CU");
+static_assert(lds_bytes(5) <= 160 * 1024 && lds_bytes(6) <= 160 * 1024 && lds_bytes(7) <= 160 * 1024 && lds_bytes(8) <= 160 * 1024, "LDS");
 
-// Four columns (2 f + BH) of word pairs.  A nibble is put under the exponent that gives it the weight 1 -- (w & mask) | magic is
-// a float's (half's) 2^e + q -- so unpacking takes one instruction a nibble, and a shift for those that lie too high or low.
-template <typename T, int BH>
+// The even (bh 0) or odd columns 2 f + bh of word pairs.  A nibble is put under the exponent that gives it the weight 1 --
+// (w & mask) | magic is a float's (half's) 2^e + q -- so unpacking takes one instruction a nibble, and a shift for those that
+// lie too high or low.  bh is a register and not a template argument: the four roles of waves share one piece of code.
+template <typename T>
 struct Columns;
 
-template <int BH>
-struct Columns<F16, BH> {
+template <>
+struct Columns<F16> {
     AndOr low, high;     // nibbles 0 and 1 of a 16-bit half: 1024 + q, 64 + q
-    uint32_t zp[4], sc[4];
-    __device__ __forceinline__ Columns() : low(0x000F000Fu, 0x64006400u), high(0x00F000F0u, 0x54005400u) {}
+    uint32_t zp[4], sc[4], pick, pick_scale;
+    __device__ __forceinline__ explicit Columns(int bh)
+        : low(0x000F000Fu, 0x64006400u), high(0x00F000F0u, 0x54005400u), pick(bh ? 0x07060302u : 0x05040100u),
+          pick_scale(bh ? 0x03020302u : 0x01000100u) {}
     __device__ __forceinline__ void embed(uint32_t w1, uint32_t w0, uint32_t (&q)[4]) const {
-        const uint32_t v = __builtin_amdgcn_perm(w1, w0, BH ? 0x07060302u : 0x05040100u), u = v >> 8;
+        const uint32_t v = __builtin_amdgcn_perm(w1, w0, pick), u = v >> 8;
         q[0] = low(v), q[1] = high(v), q[2] = low(u), q[3] = high(u);
     }
     __device__ __forceinline__ void set_group(uint32_t zw, u32x4 sv) {
         embed(zw, zw, zp);
 #pragma unroll
-        for (int f = 0; f < 4; ++f) sc[f] = __builtin_amdgcn_perm(sv[f], sv[f], BH ? 0x03020302u : 0x01000100u);
+        for (int f = 0; f < 4; ++f) sc[f] = __builtin_amdgcn_perm(sv[f], sv[f], pick_scale);
     }
     __device__ __forceinline__ void pair(uint32_t w0, uint32_t w1, uint32_t (&out)[4]) const {
         uint32_t q[4];
@@ -61,36 +73,33 @@ struct Columns<F16, BH> {
     }
 };
 
-template <int BH>
-struct Columns<BF16, BH> {
-    AndOr at8, at12, at16;   // nibble at that bit of a float: 2^15 + q, 2^11 + q, 2^7 + q
-    float sc[4], zp[4];
-    __device__ __forceinline__ Columns()
-        : at8(0xF00u, 0x47000000u), at12(0xF000u, 0x45000000u), at16(0xF0000u, 0x43000000u) {}
-    __device__ __forceinline__ void embed(uint32_t w, float (&q)[4]) const {
-        uint32_t b[4];
-        if constexpr (BH == 0) {
-            const uint32_t u = w << 8;
-            b[0] = at8(u), b[1] = at12(u), b[2] = at8(w), b[3] = at12(w);
-        } else {
-            const uint32_t u = w >> 12;
-            b[0] = at16(w), b[1] = at8(u), b[2] = at12(u), b[3] = at16(u);
-        }
-#pragma unroll
-        for (int f = 0; f < 4; ++f) q[f] = __builtin_bit_cast(float, b[f]);
+template <>
+struct Columns<BF16> {
+    AndOr at8, at12;         // nibble at that bit of a float: 2^15 + q, 2^11 + q
+    float sc[4], nzs[4];     // the scale, and minus scale times what a nibble of the zero point gives
+    int up, down;
+    __device__ __forceinline__ explicit Columns(int bh) : at8(0xF00u, 0x47000000u), at12(0xF000u, 0x45000000u), up(bh ? 0 : 16), down(bh ? 16 : 0) {}
+    __device__ __forceinline__ void embed(uint32_t word, float (&q)[4]) const {
+        const uint32_t w = word >> down, u = w << 8;
+        q[0] = __builtin_bit_cast(float, at8(u)), q[1] = __builtin_bit_cast(float, at12(u));
+        q[2] = __builtin_bit_cast(float, at8(w)), q[3] = __builtin_bit_cast(float, at12(w));
     }
     __device__ __forceinline__ void set_group(uint32_t zw, u32x4 sv) {
-        embed(zw, zp);
+        embed(zw, nzs);
 #pragma unroll
-        for (int f = 0; f < 4; ++f) sc[f] = __builtin_bit_cast(float, BH ? sv[f] & 0xFFFF0000u : sv[f] << 16);
+        for (int f = 0; f < 4; ++f) {
+            sc[f] = __builtin_bit_cast(float, (sv[f] << up) & 0xFFFF0000u);
+            nzs[f] *= -sc[f];
+        }
     }
     __device__ __forceinline__ void pair(uint32_t w0, uint32_t w1, uint32_t (&out)[4]) const {
         float q0[4], q1[4];
         embed(w0, q0);
         embed(w1, q1);
-        // q - z and its product with the scale are exact
+        // 2^15 + z has 16 bits and the scale 8: the product kept in nzs is exact, and so is the sum, (q - z) * s
 #pragma unroll
-        for (int f = 0; f < 4; ++f) out[f] = BF16::pack2((q0[f] - zp[f]) * sc[f], (q1[f] - zp[f]) * sc[f]);
+        for (int f = 0; f < 4; ++f)
+            out[f] = BF16::pack2(__builtin_fmaf(q0[f], sc[f], nzs[f]), __builtin_fmaf(q1[f], sc[f], nzs[f]));
     }
 };
 
@@ -100,18 +109,19 @@ __device__ __forceinline__ void rows_tile(
     const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
     float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
-    constexpr int kStage = stage_bytes(MT);
+    constexpr int kStage = stage_bytes(MT), kWords = MT * 2048, kScales = kWords + 4096;
+    constexpr int kPairs = pairs(MT), kFours = fours(MT), kGiven = 8 * 4096 * kFours;
     // runs of consecutive items to each XCD: the row tiles of a column tile read its words through one L2
     const int per = gridDim.x >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (id >= items) return;
     const int split = id % splits, tile = id / splits;
     const int m0 = tile % m_tiles * (16 * MT), tn = tile / m_tiles;
     const int words = N >> 3;
+    const int word0 = min(16 * tn, words - 16);     // a last tile that is not whole begins earlier (N >= 128) and stores some columns again
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int j = lane & 15, kb = lane >> 4, bh = wave & 1, kh = wave >> 1;
+    const int j = lane & 15, kb = lane >> 4, bh = wave & 1, kh = (wave >> 1) & 1, turn = wave >> 2;
     const int begin = split * steps_per_split, n = min(begin + steps_per_split, K >> 6) - begin;   // 64-row steps
     const int k0 = 64 * begin;
-    const int words_at = MT * 2048 + kh * kHalf, zeros_at = words_at + 2048, scales_at = zeros_at + 256;
 
     f32x4 acc[MT][4];
 #pragma unroll
@@ -119,203 +129,203 @@ __device__ __forceinline__ void rows_tile(
 #pragma unroll
         for (int f = 0; f < 4; ++f) acc[mt][f] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    auto run = [&](auto half) {
-        constexpr int BH = decltype(half)::value;
-        // Pieces of x: eight rows, 128 bytes each; piece i goes to wave i % 4, of an odd MT's the last two to the waves of kh 0.
-        constexpr int XP = MT / 2, kLoads = XP + 4 + 1;     // loads a stage of this wave, but for those two
-        constexpr bool ODD = MT % 2;
-        static_assert((kDepth - 3) * (kLoads + 1) < 64, "the wait counts to 63");
-        uint32_t xsrc[XP + ODD];      // bytes
+    // A stage in pieces of 1024 bytes, piece i to wave i % 8: 2 MT of x (eight rows, 128 bytes each), four of words (16 rows of
+    // 64 bytes), and the scales and zero words of its two groups of 32 rows, which come in one.
+    constexpr int kPieces = 2 * MT + 5, kMost = (kPieces + 7) / 8, kFull = kPieces % 8 ? kPieces % 8 : 8;   // waves below kFull bring kMost
+    constexpr int kGroupPiece = 2 * MT + 4;
+    static_assert((kDepth - 2) * kMost < 64, "the wait counts to 63");
+    uint32_t source[kMost], offset[kMost], step[kMost];      // bytes: of a lane, of the next stage to be asked for, from stage to stage
+    uint64_t operand[kMost];
 #pragma unroll
-        for (int i = 0; i < XP + ODD; ++i) {
+    for (int q = 0; q < kMost; ++q) {
+        const int i = 8 * q + wave;
+        const uint64_t p = reinterpret_cast<uint64_t>(i < 2 * MT ? (const void*)x : (const void*)qweight);
+        // (a descriptor that the compiler does not see to be the same in all lanes costs a loop over the lanes)
+        operand[q] = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
+        if (i < 2 * MT) {
             // 16-byte piece p of a row lies at p ^ row / 2: an operand read meets all banks
-            const int row = 8 * (4 * i + wave) + (lane >> 3);
-            xsrc[i] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 8u) * 2u;
+            const int row = 8 * i + (lane >> 3);
+            source[q] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)K + (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 8u) * 2u;
+            offset[q] = (uint32_t)k0 * 2u, step[q] = 128u;
+        } else {
+            // row 8 a + b of a half's 32 lies at 4 b + a: the lanes of an operand read lie side by side
+            const int at = 16 * ((i - 2 * MT) & 1) + (lane >> 2);
+            source[q] = ((uint32_t)((at & 3) * 8 + (at >> 2)) * (uint32_t)words + (uint32_t)(word0 + 4 * (lane & 3))) * 4u;
+            offset[q] = (uint32_t)(k0 + 32 * ((i - 2 * MT) >> 1)) * (uint32_t)words * 4u, step[q] = 64u * (uint32_t)words * 4u;
         }
-        // columns past the last word read it again; nothing of them is stored
-        const uint32_t word = (uint32_t)min(tn * 16 + j, words - 1);
-        const uint32_t wsrc = ((uint32_t)(8 * kb + 4 * BH) * (uint32_t)words + word) * 4u, zsrc = word * (BH == 0 ? 4u : 16u);
-        // of the next stage to be issued: its rows of x and words in bytes, the group of this half and the rows left of it
-        uint32_t x_off = (uint32_t)k0 * 2u, w_off = (uint32_t)(k0 + 32 * kh) * (uint32_t)words * 4u;
-        int group = __builtin_amdgcn_readfirstlane((k0 + 32 * kh) / g), left = (group + 1) * g - (k0 + 32 * kh);
-        const auto rx = resource(x), rw = resource(qweight), rz = resource(BH == 0 ? (const void*)qzeros : (const void*)scales);
-        auto issue_x = [&](int slot, int i) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, AWQ_LPTR(s_mem + slot * kStage + (4 * i + wave) * 1024), 16, xsrc[i], x_off, 0, 0);
-        };
-        // load `i` of a stage but for the odd piece of x
-        auto issue = [&](int slot, int i) {
-            unsigned char* base = s_mem + slot * kStage;
-            if (i < XP) {
-                issue_x(slot, i);
-            } else if (i < XP + 4) {
-                const int p = i - XP;     // piece 4 BH + p: rows p, 8 + p, 16 + p, 24 + p, so that the lanes of an operand read side by side
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, AWQ_LPTR(base + words_at + (4 * BH + p) * 256), 4, wsrc,
-                                                         w_off + (uint32_t)(p * words) * 4u, 0, 0);
-            } else if (BH == 0) {         // (four times over, which spares a branch)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rz, AWQ_LPTR(base + zeros_at), 4, zsrc, (uint32_t)(group * words) * 4u, 0, 0);
+    }
+    // Scales: lanes 0 .. 15 of the first 32 rows, 16 .. 31 of the second; zero words: lanes 32 .. 35 and 36 .. 39 (and again).
+    const bool second = lane < 32 ? lane & 16 : lane & 4;
+    const unsigned char* group_base = lane < 32 ? reinterpret_cast<const unsigned char*>(scales) + 16 * (size_t)(word0 + j)
+                                                : reinterpret_cast<const unsigned char*>(qzeros) + 4 * (size_t)(word0 + 4 * (lane & 3));
+    const uint32_t group_bytes = (uint32_t)words * (lane < 32 ? 16u : 4u);
+    uint32_t group = (uint32_t)((k0 + (second ? 32 : 0)) / g);              // of this lane, in the next stage to be asked for
+    int left = (int)(group + 1) * g - (k0 + (second ? 32 : 0));             // rows of K until it ends
+    const uint32_t last_group = (uint32_t)(K / g) - 1u;
+
+    // stages asked for, the ring's place (in bytes) of the next one, and the size that the operands' descriptors give: none past the end
+    int asked = 0, ask_at = 0, open = -1;
+    // piece q of the stage `asked`; past the last stage nothing is read (the count of requests, which the waits rely on, stays)
+    auto ask = [&](int q) {
+        const int i = 8 * q + wave;
+        if (q < kMost - 1 || wave < kFull) {
+            if (q == kGroupPiece / 8 && wave == kGroupPiece % 8) {
+                __builtin_amdgcn_global_load_lds(AWQ_GPTR(group_base + (size_t)min(group, last_group) * group_bytes),
+                                                 AWQ_LPTR(s_mem + ask_at + kScales), 16, 0, 0);
+                left -= 64;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {     // twice over at groups of 32
+                    const bool over = left <= 0;
+                    group += over, left += over ? g : 0;
+                }
             } else {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rz, AWQ_LPTR(base + scales_at), 16, zsrc, (uint32_t)(group * words) * 16u, 0, 0);
+                const auto r = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(operand[q]), 0, __builtin_amdgcn_readfirstlane(open), 0x00020000);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, AWQ_LPTR(s_mem + ask_at + i * 1024), 16, source[q], offset[q], 0, 0);
+                offset[q] += step[q];
             }
-        };
-        auto issued = [&] {
-            x_off += 128;
-            w_off += 64u * (uint32_t)words * 4u;
-            left -= 64;
+        }
+    };
+    auto asked_all = [&] {
+        open = __builtin_amdgcn_readfirstlane(++asked < n ? -1 : 0);
+        asm volatile("" : "+s"(open));
+        ask_at = ask_at + kStage == kDepth * kStage ? 0 : ask_at + kStage;
+    };
+    // Where the registers suffice, the words of a wave's next stage come beside its matrix instructions, a phase before its rows.
+    constexpr bool kEarly = MT != 4;
+    constexpr int kOnTheWay = kDepth - (kEarly ? 3 : 2);
+    // This wave's share of all stages but the kOnTheWay last asked for is there; then the barrier that hands the matrix cores
+    // to the other wave of the SIMD.  Nothing is scheduled across.
+    auto hand_over = [&] {
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int most = kOnTheWay * kMost, fewer = kOnTheWay * (kMost - 1);
+        if (wave < kFull) __builtin_amdgcn_s_waitcnt(0x0F70 | (most & 15) | ((most >> 4) << 14));
+        else __builtin_amdgcn_s_waitcnt(0x0F70 | (fewer & 15) | ((fewer >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll 1
+    for (int t = 0; t < kDepth - 1; ++t) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {     // twice over at groups of 32
-                const bool over = left <= 0;
-                group += over, left += over ? g : 0;
+        for (int q = 0; q < kMost; ++q) ask(q);
+        asked_all();
+    }
+    hand_over();
+    if (turn == 1) {       // half a round behind from here on
+#pragma unroll
+        for (int q = 0; q < kMost; ++q) ask(q);
+        asked_all();
+        hand_over();
+    }
+    Columns<T> cols(bh);
+    const int x_at = j * 128 + (((4 * kh + kb) ^ (j >> 1)) & 7) * 16;
+    const int w_at = kWords + kh * 2048 + lane * 4;
+    const int z_at = kScales + 512 + kh * 64 + j * 4, s_at = kScales + kh * 256 + j * 16;
+    int at = turn * kStage;       // of the stage this wave reads next
+    uint32_t w[8], zw;
+    u32x4 sv;
+    auto read_words = [&](int at) {
+        const unsigned char* base = s_mem + at;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) w[r] = *reinterpret_cast<const uint32_t*>(base + w_at + r * 256);
+        zw = *reinterpret_cast<const uint32_t*>(base + z_at);
+        sv = *reinterpret_cast<const u32x4*>(base + s_at);
+    };
+    auto read_rows = [&](int at, u32x4 (&a)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) a[mt] = *reinterpret_cast<const u32x4*>(s_mem + at + x_at + mt * 2048);
+    };
+    if (kEarly) read_words(at);
+    __builtin_amdgcn_s_waitcnt(0xC07F);     // LDS and scalar reads: one still open here would be waited for in every round of the loop
+#pragma unroll 1
+    for (int t = turn; t < n; t += 2) {
+        u32x4 a[MT], b[4];
+        if (!kEarly) read_words(at);
+        read_rows(at, a);
+        cols.set_group(zw, sv);
+#pragma unroll
+        for (int rp = 0; rp < 4; ++rp) {
+            if (rp == 2) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int q = 0; q < kMost; ++q) ask(q);
+                asked_all();
+                __builtin_amdgcn_sched_barrier(0);
             }
-        };
-        struct Operands {
-            u32x4 a[MT], b[4];
-        };
-        Columns<T, BH> cols;
-        uint32_t w[8], zw;
-        u32x4 sv;
-        auto read_words = [&](int slot) {
-            const unsigned char* base = s_mem + slot * kStage;
-#pragma unroll
-            for (int r = 0; r < 8; ++r) w[r] = *reinterpret_cast<const uint32_t*>(base + words_at + r * 256 + lane * 4);
-            zw = *reinterpret_cast<const uint32_t*>(base + zeros_at + j * 4);
-            sv = *reinterpret_cast<const u32x4*>(base + scales_at + j * 16);
-        };
-        auto read_rows = [&](int slot, Operands& o) {
-            const unsigned char* base = s_mem + slot * kStage + j * 128 + (((4 * kh + kb) ^ (j >> 1)) & 7) * 16;
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) o.a[mt] = *reinterpret_cast<const u32x4*>(base + mt * 2048);
-        };
-        auto unpack = [&](int rp, Operands& o) {
             uint32_t v[4];
             cols.pair(w[2 * rp], w[2 * rp + 1], v);
 #pragma unroll
-            for (int f = 0; f < 4; ++f) o.b[f][rp] = v[f];
-        };
-        auto landed = [&](auto newer) {   // all stages but the `newer` last issued
-            constexpr int c = decltype(newer)::value * kLoads, more = decltype(newer)::value * (kLoads + ODD);
-            if (ODD && kh == 0) __builtin_amdgcn_s_waitcnt(0x0F70 | (more & 15) | ((more >> 4) << 14));
-            else __builtin_amdgcn_s_waitcnt(0x0F70 | (c & 15) | ((c >> 4) << 14));
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        };
-        int next = 0;    // ring slot of the next stage to be read
-        // FULL: a stage is issued, into the slot before the one being multiplied, which every wave had read before it came to
-        // this barrier.
-        auto stage = [&](auto full, int t, const Operands& cur, Operands& nxt) {
-            constexpr bool FULL = decltype(full)::value;
-            landed(std::integral_constant<int, FULL ? kDepth - 3 : 0>{});
-            // Seven pieces, each with its share of the matrix instructions and what fills their time: the words and rows of the
-            // next stage from LDS, the loads of a later one, then the words, which are there by now.
-            constexpr int kAll = 4 * MT, kFirst = kAll / 3, kPer = (kAll - kFirst) / 4;
-            auto multiply = [&](int from, int to) {
-#pragma unroll
-                for (int i = 0; i < kAll; ++i)
-                    if (i >= from && i < to) acc[i % MT][i / MT] = T::mfma16(cur.a[i % MT], cur.b[i / MT], acc[i % MT][i / MT]);
-            };
-            const int slot = next >= 2 ? next - 2 : next + kDepth - 2;
-            if (FULL && ODD && kh == 0) issue_x(slot, XP);
-            __builtin_amdgcn_sched_barrier(0);
-            read_words(next);     // past the last stage what an earlier one left there, and nothing uses it
-            multiply(0, 2);
-            __builtin_amdgcn_sched_barrier(0);
-            read_rows(next, nxt);
-            multiply(2, kFirst - 3);
-#pragma unroll
-            for (int i = 2; i < kFirst - 3; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            cols.set_group(zw, sv);
-            multiply(kFirst - 3, kFirst);
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int rp = 0; rp < 4; ++rp) {
-                // a load to every second or third matrix instruction: four waves' loads take the CU that long
-                constexpr int kShare = (kLoads + 3) / 4;
-#pragma unroll
-                for (int i = 0; i < kShare; ++i)
-                    if (FULL && rp * kShare + i < kLoads) issue(slot, rp * kShare + i);
-                unpack(rp, nxt);
-                multiply(kFirst + rp * kPer, rp == 3 ? kAll : kFirst + (rp + 1) * kPer);
-#pragma unroll
-                for (int i = 0; i < kPer; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, T::id == AWQ_F16 ? 3 : 6, 0);
-                    if (FULL && i < kShare) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if constexpr (FULL) issued();
-            // (or the compiler moves the unpacking to its use, in front of the next stage's matrix instructions)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) asm volatile("" : "+v"(nxt.b[f]));
-            next = next + 1 == kDepth ? 0 : next + 1;
-        };
-        Operands even, odd;
-        for (int t = 0; t < kDepth - 1 && t < n; ++t) {
-            if (ODD && kh == 0) issue_x(t, XP);
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i) issue(t, i);
-            issued();
+            for (int f = 0; f < 4; ++f) b[f][rp] = v[f];
         }
-        landed(std::integral_constant<int, 0>{});
-        read_words(0);
-        read_rows(0, even);
-        cols.set_group(zw, sv);
+        // (or the compiler moves the unpacking to its use, behind the barrier)
 #pragma unroll
-        for (int rp = 0; rp < 4; ++rp) unpack(rp, even);
-        __builtin_amdgcn_s_waitcnt(0xC07F);   // the LDS reads: one still open here would be waited for in every round of the loop
-        next = 1;
-        int t = 0;
-        for (; t + kDepth < n; t += 2) {
-            stage(std::true_type{}, t, even, odd);
-            stage(std::true_type{}, t + 1, odd, even);
+        for (int f = 0; f < 4; ++f) asm volatile("" : "+v"(b[f]));
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+v"(a[mt]));
+        at = at + 2 * kStage >= kDepth * kStage ? at + (2 - kDepth) * kStage : at + 2 * kStage;
+        hand_over();
+        if (kEarly) read_words(at);     // past the last stage whatever lies there, and nothing uses it
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < kMost; ++q) {
+#pragma unroll
+            for (int i = 4 * MT * q / kMost; i < 4 * MT * (q + 1) / kMost; ++i) acc[i % MT][i / MT] = T::mfma16(a[i % MT], b[i / MT], acc[i % MT][i / MT]);
+            __builtin_amdgcn_sched_barrier(0);
+            ask(q);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (t + kDepth - 1 < n) {
-            stage(std::true_type{}, t, even, odd);
-            even = odd;
-            ++t;
-        }
-        for (; t < n; t += 2) {
-            stage(std::false_type{}, t, even, odd);
-            if (t + 1 < n) stage(std::false_type{}, t + 1, odd, even);
-        }
-    };
-    if (bh == 0) run(std::integral_constant<int, 0>{});
-    else run(std::integral_constant<int, 1>{});
+        asked_all();
+        hand_over();
+    }
+    if ((n & 1) == turn) __builtin_amdgcn_s_barrier();      // the turn that had one phase fewer
+    __builtin_amdgcn_s_waitcnt(0x0F70);                     // what was asked for past the end has come: the LDS is free
 
-    // The halves of K meet.  fp32 tile [16 MT][column c of word j at 16 c + j], written and read without bank conflicts.
-    float* tile_f = reinterpret_cast<float*>(s_mem);
-    auto at = [&](int mt, int f, int r) { return (16 * mt + 4 * kb + r) * kPad + (2 * f + bh) * 16 + j; };
+    // The four parts of K meet, (0 + 1) + (2 + 3), and every wave ends with a quarter of the row tiles: the two of a turn give each
+    // other every second tile, then the turns every second of those, in the layout of the registers; the sums go to an fp32 tile
+    // [16 MT][column c of word j at 16 c + j], written and read without bank conflicts.  (All through such tiles, of which LDS
+    // holds two, the end took 2.2 us with 128 rows; so 1.7.)
+    float* tile_f = reinterpret_cast<float*>(s_mem + kGiven);
+    const auto meet = [&](auto khc, auto turnc) {
+        constexpr int KH = decltype(khc)::value, TURN = decltype(turnc)::value;
+        f32x4* mine = reinterpret_cast<f32x4*>(s_mem) + wave * (kPairs * 256) + lane;
+        const f32x4* first = reinterpret_cast<const f32x4*>(s_mem) + (wave ^ 2) * (kPairs * 256) + lane;
+        f32x4* mine2 = reinterpret_cast<f32x4*>(s_mem) + wave * (kFours * 256) + lane;
+        const f32x4* other = reinterpret_cast<const f32x4*>(s_mem) + (wave ^ 4) * (kFours * 256) + lane;
+#pragma unroll
+        for (int mt = 1 - KH; mt < MT; mt += 2)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) mine[(mt / 2 * 4 + f) * 64] = acc[mt][f];
+        __syncthreads();
+#pragma unroll
+        for (int mt = KH; mt < MT; mt += 2)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) acc[mt][f] += first[(mt / 2 * 4 + f) * 64];
+        __syncthreads();
+#pragma unroll
+        for (int mt = KH + 2 * (1 - TURN); mt < MT; mt += 4)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) mine2[(mt / 4 * 4 + f) * 64] = acc[mt][f];
+        __syncthreads();
+#pragma unroll
+        for (int mt = KH + 2 * TURN; mt < MT; mt += 4)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                const f32x4 sum = acc[mt][f] + other[(mt / 4 * 4 + f) * 64];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tile_f[(16 * mt + 4 * kb + r) * kPad + (2 * f + bh) * 16 + j] = sum[r];
+            }
+    };
     __syncthreads();
-    if (kh == 1) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int f = 0; f < 4; ++f)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) tile_f[at(mt, f, r)] = acc[mt][f][r];
-    }
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    if (kh == 0 && turn == 0) meet(Zero{}, Zero{});
+    else if (kh == 0) meet(Zero{}, One{});
+    else if (turn == 0) meet(One{}, Zero{});
+    else meet(One{}, One{});
     __syncthreads();
-    if (kh == 0) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int f = 0; f < 4; ++f)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) tile_f[at(mt, f, r)] += acc[mt][f][r];
-    }
-    __syncthreads();
-    const int wc = tn * 16 + j;
-    if (wc >= words) return;
-    for (int p = wave; p < 4 * MT; p += 4) {
+    const int wc = word0 + j;
+    for (int p = wave; p < 4 * MT; p += 8) {
         const int row = 16 * (p >> 2) + 4 * kb + (p & 3), m = m0 + row;
         if (m >= M) continue;
         float v[8];
@@ -342,7 +352,7 @@ __device__ __forceinline__ void rows_tile(
 }
 
 template <typename T, int MT>
-__global__ __launch_bounds__(kThreads, 2) void rows_kernel(
+__global__ __launch_bounds__(kThreads, 2 * per_cu(MT)) void rows_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales,
     const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
     float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
@@ -378,14 +388,18 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, i
         return p;
     const int64_t m_tiles = cdiv(M, 128), n_tiles = cdiv(N, 128), steps = K / 64;
     p.m_tiles = (int)m_tiles, p.n_tiles = (int)n_tiles;
-    p.mt = (int)std::max<int64_t>(5, cdiv(cdiv(M, m_tiles), 16));
-    // A round of 256 workgroups: a stage by type and MT, 6 us to fill the ring and store; a K split writes its fp32 sums and reads
-    // them again in a second launch.  The stages are measured (16 weights of 2048 to 25600 rows, 129 to 640 rows of x, within
-    // 10 % of every time): with few rows the unpacking outlasts the matrix instructions, in bf16 more than in fp16.
-    constexpr double kStage[2][4] = {{0.47, 0.455, 0.53, 0.57}, {0.56, 0.57, 0.62, 0.635}};     // [fp16, bf16][MT - 5]
-    const double stage = kStage[dtype == AWQ_F16 ? 0 : 1][p.mt - 5];
+    p.mt = (int)std::max<int64_t>(2, cdiv(cdiv(M, m_tiles), 16));
+    // Microseconds, by type and MT: of a stage with a CU to itself and with two workgroups on it, and of filling the ring,
+    // the tile's sums and the launch; a K split writes its fp32 sums and reads them again in a second launch.
+    constexpr double kAlone[2][7] = {{0.28, 0.295, 0.38, 0.345, 0.35, 0.37, 0.41}, {0.345, 0.37, 0.445, 0.405, 0.42, 0.45, 0.47}};   // [fp16, bf16][MT - 2]
+    constexpr double kShared[2][3] = {{0.455, 0.45, 0.495}, {0.52, 0.53, 0.575}};
+    const int t = dtype == AWQ_F16 ? 0 : 1;
+    const int64_t slots = 256 * per_cu(p.mt);
     const auto us = [&](int64_t s) {
-        return (double)cdiv(m_tiles * n_tiles * s, 256) * (stage * (double)cdiv(steps, s) + 6) +
+        const int64_t items = m_tiles * n_tiles * s, last = items % slots, n = cdiv(steps, s);
+        const double fixed = 4.6 + 0.95 * p.mt, alone = kAlone[t][p.mt - 2] * (double)n + fixed;
+        const double whole = p.mt <= 4 ? kShared[t][p.mt - 2] * (double)n + fixed : alone;
+        return (double)(items / slots) * whole + (last == 0 ? 0 : last > 256 ? whole : alone) +
                (s > 1 ? 2.5 + (double)s * (double)(M * N) * 8 / 5.0e6 : 0);
     };
     int64_t best = 1;
@@ -406,8 +420,10 @@ hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_
     if (p.mt == MT) e = launch<T, MT>(p, x, qweight, qscales, qzeros, bias, y, partials, M, N, K, g, gated, st);
     hipError_t e = hipErrorInvalidValue;
     if (dtype == AWQ_F16) {
+        AWQ_ROWS(F16, 2) AWQ_ROWS(F16, 3) AWQ_ROWS(F16, 4)
         AWQ_ROWS(F16, 5) AWQ_ROWS(F16, 6) AWQ_ROWS(F16, 7) AWQ_ROWS(F16, 8)
     } else {
+        AWQ_ROWS(BF16, 2) AWQ_ROWS(BF16, 3) AWQ_ROWS(BF16, 4)
         AWQ_ROWS(BF16, 5) AWQ_ROWS(BF16, 6) AWQ_ROWS(BF16, 7) AWQ_ROWS(BF16, 8)
     }
 #undef AWQ_ROWS

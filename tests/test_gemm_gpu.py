@@ -432,6 +432,34 @@ def test_gemm_rows128(dtype, M, K, N, g):
     assert torch.equal(awq_gemm_variant(eye, *dev, v, 1), nq.awq_dequantize(*dev)[:n])
 
 
+# the tiles of which two share a CU, at the first and last row of each; fewer stages than the ring holds, odd and even counts,
+# the last K split one stage long; widths of one tile, a word more, a word less than two, not a multiple of four words
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,K,N,g,split", [(17, 64, 128, 32, 1), (32, 1344, 136, 64, 4), (33, 1088, 248, 32, 3), (48, 576, 1032, 576, 1),
+                                           (49, 640, 264, 128, 5), (64, 2112, 1240, 64, 2), (65, 1152, 520, 1152, 1), (80, 704, 264, 64, 3)])
+def test_gemm_rows128_few_rows(dtype, M, K, N, g, split):
+    print(f"gemm rows128 few rows {dtype} M={M} K={K} N={N} g={g} split={split}", flush=True)
+    L = _lib.lib()
+    v = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())].index("rows128")
+    p = random_packed(K, N, g, dtype, seed=M + K)
+    dev = [to_dev(p["qweight"]), to_dev(p["qscales"], dtype), to_dev(p["qzeros"])]
+    xb = make_x(M, K, dtype, seed=M)
+    xd = to_dev(xb, dtype)
+    bias = np.linspace(-2, 2, N).astype(np.float32)
+    y = awq_gemm_variant(xd, *dev, v, split)
+    _check(y, xb, p, dtype)
+    assert torch.equal(y, awq_gemm_variant(xd, *dev, v, split))
+    _check(awq_gemm_variant(xd, *dev, v, split, bias=to_dev(o.to_bits16(bias, dtype), dtype)), xb, p, dtype, o.to_dtype_f32(bias, dtype))
+    eye = torch.eye(min(M, K), K, device="cuda", dtype=xd.dtype)
+    assert torch.equal(awq_gemm_variant(eye, *dev, v, 1), nq.awq_dequantize(*dev)[:min(M, K)])
+    # the default linear of these rows: the GEMV where it takes the sizes, else these tiles with their own split
+    chosen = ctypes.c_int()
+    name = L.awq_linear_route(M, N, K, g, _lib.dtype_id(xd.dtype), 0, ctypes.byref(chosen))
+    assert name == (b"128x128" if M > 64 else b"rows128") or (name == b"gemv" and g % 128 == 0)
+    if name != b"gemv":
+        assert torch.equal(nq.awq_gemm(xd, *dev, 8), awq_gemm_variant(xd, *dev, v, chosen.value))
+
+
 def test_gemm_rows128_routes():
     """The default linear takes these tiles for a few hundred rows, with the bits of the forced variant; what they refuse, short
     K and the plan of awq_gemm stay with the other kernels."""
