@@ -618,8 +618,10 @@ extern "C" int awq_linear_swiglu(const void* x, const int32_t* qweight, const vo
     int v = awq::kPipeVariant, s = 1;
     if (K >= awq::kBK && N >= 16 && M >= 1 && group_size > 0)
         awq::plan_gemm_tile256(M, N, K, group_size, dtype, &v, &s);
-    awq::RowsPlan rows;       // as awq_linear on the same sizes, whose bits the gated product has
-    if (M > 16 && N >= 128 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
+    // as awq_linear on the same sizes, whose bits the gated product has; 65 to 128 rows of the sizes that the GEMV takes up to 64 rows
+    // keep the 256-row tiles, whose bits callers compare with
+    awq::RowsPlan rows;
+    if (M > (staged ? 128 : 16) && N >= 128 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
         v = awq::kRowsVariant, s = rows.splits;
     return awq::gemm_dispatch("awq_linear_swiglu", x, qweight, qscales, qzeros, nullptr, y, M, N, K, group_size,
                               dtype, workspace, workspace_bytes, stream, v, s, 1);
@@ -651,7 +653,7 @@ extern "C" const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t
     if (awq_linear_scratch_bytes(M, N, K, group_size, dtype)) return "dense";
     int variant;
     awq::RowsPlan rows;
-    if (rows_wanted(M, N, K, group_size, dtype, &rows))
+    if (!(gated && staged && M <= 128) && rows_wanted(M, N, K, group_size, dtype, &rows))
         // (up to 128 rows the tile's name is 128x128, whichever kernel awq_gemm runs on it)
         variant = M > 64 && M <= 128 && !gated ? awq::k128x128 : awq::kRowsVariant, *split_k = rows.splits;
     else if (gated) awq::plan_gemm_tile256(M, N, K, group_size, dtype, &variant, split_k);
