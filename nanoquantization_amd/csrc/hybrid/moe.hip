@@ -418,18 +418,24 @@ MoeForm moe_form(int64_t pairs, int64_t experts, int64_t width, int64_t ff, int 
     // by pairs per expert, so that one tile usually holds all pairs of an expert while there are few
     if (pairs <= 6 * experts || pairs <= 16) return MoeForm::skinny16;
     if (pairs <= 16 * experts || pairs <= 32) return MoeForm::skinny32;
-    if (pairs <= 40 * experts || pairs <= 64) return MoeForm::skinny64;
-    // The ping-pong core wants whole stages and 32-bit offsets into the rows and into an expert's weights, pairs per expert that
-    // fill its tiles, and 128 workgroups in the smaller of the two products.  Both products, gemm / 128 / 256 pairs a tile:
-    // 4096 -> 2 x 6144, 8 experts, 192 pairs each 543 / 358 / 357 us, 512 each 947 / 754 / 673, 2048 each 2890 / 2401 / 1948;
-    // 2048 -> 2 x 1024, 64 experts, 144 each 318 / 277 / 236, 192 each 370 / 274 / 243, 384 each 529 / 422 / 376;
-    // 1024 -> 2 x 1536, 8 experts, 256 each 49 / 45 / 63 (80 workgroups), 512 each 69 / 63 / 69, 1024 each 120 / 122 / 100.
-    // The lines are on the safe side: with many experts the larger tiles are ahead some way below them.
+    // The ping-pong core wants whole stages and 32-bit offsets into the rows and into an expert's weights.  Its tiles stream an
+    // expert's weights once, so they are the fastest from 17 pairs an expert on where every expert's tile of the smaller product
+    // makes 64 workgroups.  Both products, 8 experts, skinny 64 / gemm 64 / pingpong 128 / 256 pairs a tile, us:
+    //   4096 -> 2 x 6144, 20 pairs each 404 / 343 / 269 / 303, 40 each 500 / 346 / 278 / 308, 80 each 803 / 449 / 291 / 317, 115 each
+    //   458 / 330 / 325 with 64 / 128 / 256, 140 each 553 / 342 / 338, 212 each 656 / 362 / 429, 325 each 734 / 547 / 459;
+    //   2048 -> 2 x 3072, 28 each 134 / 110 / 95 / 107, 80 each 144 / 104 / 112 from gemm 64 on, 100 each 138 / 125 / 113, 140 each
+    //   144 / 125 / 124, 250 each 176 / 131 / 169, 425 each 255 / 163 / 175;
+    //   1024 -> 2 x 1536 (32 workgroups), 28 each 40 / 35 / 38 / 55, 115 each 38 / 40 / 57, 173 each 39 / 42 / 60, 212 each 50 / 44 / 61.
+    // 2048 -> 2 x 1024, 64 experts, 144 each 318 / 277 / 236, 384 each 529 / 422 / 376.
     const bool stages = width % 64 == 0 && ff % 64 == 0 && pairs * std::max(width, ff) * 2 < (1ll << 32) &&
                         width * ff * 4 < (1ll << 32);
-    const int64_t groups = std::min(cdiv(width, 256), cdiv(ff, 128));
+    const int64_t groups = std::min(cdiv(width, 256), cdiv(ff, 128)), used = std::min(experts, pairs);
     if (stages && pairs > 320 * experts && pairs * groups >= 128 * 256) return MoeForm::pingpong256;
-    if (stages && pairs > 160 * experts && pairs * groups >= 128 * 128) return MoeForm::pingpong128;
+    if (stages && groups * std::max(used, pairs / 128 + used / 2) >= 64)
+        // pairs vary around their mean: near 128 many an expert has more, which would be a second tile
+        return groups * used >= 64 && pairs > 88 * experts && pairs <= 144 * experts ? MoeForm::pingpong256 : MoeForm::pingpong128;
+    // few experts and short rows: more workgroups, though they read the weights no more than once either
+    if ((pairs <= 40 * experts || pairs <= 64) && used * cdiv(std::min(width, 2 * ff), 128) < 64) return MoeForm::skinny64;
     return pairs <= 256 * experts ? MoeForm::gemm64 : MoeForm::gemm128;
 }
 int moe_form_rows(MoeForm f) {

@@ -418,6 +418,31 @@ def test_experts_with_many_pairs(rows, width, experts, top, ff, tile):
     assert torch.equal(y, ops.moe_experts(h, gu, dn, r))
 
 
+# few pairs on large tiles: just past the skinny tiles, the line to 256 pairs a tile and back; short rows, where the larger tiles come
+# later; few experts, which keep the skinny tiles longer
+@pytest.mark.parametrize("rows,width,experts,top,ff,tile", [(65, 1856, 8, 2, 960, 128), (353, 1856, 8, 2, 960, 256), (600, 1856, 8, 2, 960, 128),
+                                                            (65, 512, 8, 2, 320, 64), (1000, 512, 8, 2, 320, 64), (3000, 1024, 8, 2, 512, 128),
+                                                            (70, 1024, 4, 1, 320, 64), (33, 4096, 1, 1, 4096, 64)])
+def test_experts_with_few_pairs_on_large_tiles(rows, width, experts, top, ff, tile):
+    bf = torch.bfloat16
+    print(f"moe rows={rows} width={width} experts={experts} top={top} ff={ff}", flush=True)
+    h = rand(rows, width, seed=1, dtype=bf).cuda()
+    gu = rand(experts, 2 * ff, width, seed=3, dtype=bf, scale=width ** -0.5).cuda()
+    dn = rand(experts, width, ff, seed=4, dtype=bf, scale=ff ** -0.5).cuda()
+    r = ops.Routing(rows, experts, top, width, ff, 1, h.device)
+    assert r.tile_rows == tile
+    r.expert.copy_(((torch.rand(rows, top, generator=torch.Generator().manual_seed(5)) ** 2) * experts).int())
+    r.weight.copy_(torch.rand(rows, top, generator=torch.Generator().manual_seed(6)))
+    r.order, r.tiles = ops.moe_plan(r.expert, experts, r.tile_rows)
+    u = h.double().unsqueeze(1) * r.weight.double().unsqueeze(-1)
+    want = torch.empty(rows, top, width, dtype=torch.float64, device="cuda")
+    for x in range(experts):
+        at = (r.expert == x).nonzero(as_tuple=True)
+        a, b = u[at] @ gu[x, :ff].double().T, u[at] @ gu[x, ff:].double().T
+        want[at] = (a * torch.sigmoid(a) * b) @ dn[x].double().T
+    close(ops.moe_experts(h, gu, dn, r), want.cpu(), bf, "experts")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,width,experts,top,ff", [(1, 72, 5, 2, 48), (16, 2048, 8, 2, 64), (64, 256, 64, 6, 128),
                                                       (200, 1028, 128, 8, 32), (33, 4096, 3, 3, 24), (300, 64, 8, 2, 32)])
