@@ -95,6 +95,15 @@ int awq_linear_dense_pair(const void* x, const int32_t* gate_qweight, const void
                           int64_t N, int64_t K, int64_t group_size, int dtype, void* scratch, size_t scratch_bytes,
                           void* stream);
 
+/* y[i] [M, N[i]] = x @ weight i for two or three weights of one K, group size and type (the q, k and v projections,
+ * nanoquantization/models/qwen3_quantized.py:79-81) in one launch, without bias.  awq_linear_parts_wanted: 1 where that is the
+ * fastest way, with the bytes of workspace (as for awq_linear: zeroed once, one per stream) and of scratch it takes, else 0. */
+size_t awq_linear_parts_wanted(const int64_t* N, int count, int64_t M, int64_t K, int64_t group_size, int dtype,
+                               size_t* workspace_bytes, size_t* scratch_bytes);
+int awq_linear_parts(const void* x, const int32_t* const* qweight, const void* const* qscales, const int32_t* const* qzeros,
+                     void* const* y, const int64_t* N, int count, int64_t M, int64_t K, int64_t group_size, int dtype,
+                     void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes, void* stream);
+
 /* What a linear of these sizes runs: "gemv", "gemv in blocks of 16 rows", "dense" (awq_linear_dense, where the caller has scratch for
  * it), or the name of the awq_gemm variant awq_linear (gated: awq_linear_swiglu) takes; *split_k (may be null) its K split.  "" for
  * sizes that none of them takes.  A static string. */

@@ -418,7 +418,7 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
                                                                          (int)g, workspace, rows.splits, s);
                 break;
             }
-            e = launch_rows(rows, dtype, x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K, (int)g, workspace, act != 0, s);
+            e = launch_rows(rows, dtype, x, Parts({qweight, qscales, qzeros}, y, N), bias, (int)M, (int)K, (int)g, workspace, act != 0, s);
             break;
         case kPipeVariant:
         case kPipeTailVariant:
@@ -686,4 +686,78 @@ extern "C" int awq_linear(const void* x, const int32_t* qweight, const void* qsc
                                   workspace_bytes, stream, awq::kRowsVariant, rows.splits);
     return awq_gemm(x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,
                     workspace_bytes, stream);
+}
+
+// Estimated microseconds of a linear of more than 128 rows by its fastest way.
+static double linear_us(int64_t M, int64_t N, int64_t K, int64_t g, int dtype) {
+    double us = fused_linear_us(M, N, K, g, dtype);
+    const double dense = awq::dense_linear_us(M, N, K, g);
+    const awq::RowsPlan rows = N >= 128 ? awq::make_rows_plan(M, N, K, g, dtype) : awq::RowsPlan{};
+    if (dense >= 0 && dense < us) us = dense;
+    return rows.m_tiles != 0 && rows.us < us ? rows.us : us;
+}
+
+// Several weights with a common x in one launch, on the tiles of few rows or dequantised first, where the estimate is below the
+// sum of theirs: a weight alone fills the CUs worse, and every launch has its first loads and last stores to itself.  2048, 1024
+// and 1024 columns in bf16, one launch / three: K of 1024, 130 rows 13.6 / 35.8 us, 700 rows 17.2 / 47.6, 8192 rows 66 / 84; K of 2048, 492
+// rows 24.7 / 59.9, 2048 rows 42 / 76.  Up to 128 rows only where the single weights would not run on the GEMV, which does not
+// round its weights.
+extern "C" size_t awq_linear_parts_wanted(const int64_t* N, int count, int64_t M, int64_t K, int64_t group_size, int dtype,
+                                          size_t* workspace_bytes, size_t* scratch_bytes) {
+    size_t none;
+    if (!workspace_bytes) workspace_bytes = &none;
+    if (!scratch_bytes) scratch_bytes = &none;
+    *workspace_bytes = *scratch_bytes = 0;
+    if (!N || count < 2 || count > awq::kMaxParts || M < 17 || K < awq::kBK || K % awq::kBK != 0 || group_size < 1 || K % group_size != 0 ||
+        (dtype != AWQ_F16 && dtype != AWQ_BF16) || (M <= 128 && group_size % 128 == 0))
+        return 0;
+    int64_t total = 0;
+    double separate = 0;
+    for (int i = 0; i < count; ++i) {
+        if (N[i] <= 0 || N[i] % 128 != 0 || N[i] > (1ll << 28)) return 0;
+        total += N[i];
+        if (M > 128) separate += linear_us(M, N[i], K, group_size, dtype);
+    }
+    const awq::RowsPlan rows = awq::make_rows_plan(M, total, K, group_size, dtype);
+    const size_t scratch = M > 128 ? awq::dense_parts_scratch_bytes(N, count, M, K, group_size) : 0;
+    const double dense = scratch ? awq::dense_linear_us(M, total, K, group_size) : -1;
+    if (rows.m_tiles != 0 && (dense < 0 || rows.us <= dense)) {
+        if (M > 128 && rows.us >= separate) return 0;
+        *workspace_bytes = awq::rows_ws_bytes(rows, M, total);
+        return 1;
+    }
+    if (dense < 0 || dense >= separate) return 0;
+    *scratch_bytes = scratch;
+    return 1;
+}
+
+extern "C" int awq_linear_parts(const void* x, const int32_t* const* qweight, const void* const* qscales,
+                                const int32_t* const* qzeros, void* const* y, const int64_t* N, int count, int64_t M, int64_t K,
+                                int64_t group_size, int dtype, void* workspace, size_t workspace_bytes, void* scratch,
+                                size_t scratch_bytes, void* stream) {
+    const char* fn = "awq_linear_parts";
+    awq::PrefetchRegions dropped;            // hints of this thread were meant for this call; the product fills the chip
+    awq::take_prefetch_hint(&dropped);
+    size_t need_workspace, need_scratch;
+    if (!qweight || !qscales || !qzeros || !y ||
+        !awq_linear_parts_wanted(N, count, M, K, group_size, dtype, &need_workspace, &need_scratch)) {
+        awq::set_error("%s: null pointer, or sizes for which awq_linear_parts_wanted says no", fn);
+        return AWQ_ERR_UNSUPPORTED;
+    }
+    awq::Parts parts;
+    parts.count = parts.total = 0;
+    for (int i = 0; i < count; ++i) {
+        const int rc = awq::check_linear_args(fn, x, qweight[i], qscales[i], qzeros[i], y[i], M, N[i], K, group_size, dtype);
+        if (rc != AWQ_OK) return rc;
+        parts.add({qweight[i], qscales[i], qzeros[i]}, y[i], N[i]);
+    }
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (need_scratch) return awq::dense_parts(fn, x, parts, M, K, group_size, dtype, scratch, scratch_bytes, s);
+    if (need_workspace > 0 && (!workspace || workspace_bytes < need_workspace)) {
+        awq::set_error("%s: workspace of %zu bytes needed, %zu given", fn, need_workspace, workspace ? workspace_bytes : (size_t)0);
+        return AWQ_ERR_WORKSPACE;
+    }
+    const awq::RowsPlan rows = awq::make_rows_plan(M, parts.total, K, group_size, dtype);
+    const hipError_t e = awq::launch_rows(rows, dtype, x, parts, nullptr, (int)M, (int)K, (int)group_size, workspace, false, s);
+    return e == hipSuccess ? AWQ_OK : awq::hip_fail(fn, e);
 }

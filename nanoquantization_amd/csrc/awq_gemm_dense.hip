@@ -15,12 +15,24 @@ namespace {
 
 constexpr int64_t kSlabBytes = 256ll << 20;
 
+// Where a slab's columns go: rows of ldy values from column `first` on; a tile lies in one output.
+struct Outputs {
+    uint16_t* y[kMaxParts];
+    int ldy[kMaxParts], first[kMaxParts];
+    Outputs(void* to, int ld) {
+        for (int i = 0; i < kMaxParts; ++i) y[i] = static_cast<uint16_t*>(to), ldy[i] = ld, first[i] = i ? 0x7fffffff : 0;
+    }
+    explicit Outputs(const Parts& p) {
+        for (int i = 0; i < kMaxParts; ++i) y[i] = p.y[i], ldy[i] = p.columns[i], first[i] = p.first[i];
+    }
+};
+
 // GATED: the slab's columns are gate and up words in turn; a tile is 128 gate columns and their up columns, a wave's first
 // tiles gate, the others up.
 template <typename T, int XR, bool GATED>
 __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wt,
-                                                       const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int M,
-                                                       int cols, int K, int ldy, int x_tiles, int w_tiles) {
+                                                       const uint16_t* __restrict__ bias, Outputs out, int M, int cols, int K,
+                                                       int x_tiles, int w_tiles) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
     using P = PingPong<T, XR>;
     int xt, nt;
@@ -49,8 +61,10 @@ __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restric
     const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (size_t)m0 * K, 0,
                                                       rows * row_bytes, 0x00020000);
     p.run(s_mem, rw, vw, rx, vx, K / P::kStage);
+    const int part = (n0 >= out.first[1]) + (n0 >= out.first[2]), ldy = pick_part(out.ldy, part);
+    uint16_t* __restrict__ y = pick_part(out.y, part) + (n0 - pick_part(out.first, part));
     const auto store = [&](int r, int c, u32x4 v) {
-        if (m0 + r < M && n0 + c < out_cols) *reinterpret_cast<u32x4*>(y + (size_t)(m0 + r) * ldy + n0 + c) = v;
+        if (m0 + r < M && n0 + c < out_cols) *reinterpret_cast<u32x4*>(y + (size_t)(m0 + r) * ldy + c) = v;
     };
     if constexpr (GATED) {
         p.template write<128>(s_mem, [&](int i, int j) {
@@ -95,7 +109,7 @@ double product_us(int64_t M, int64_t slab, int64_t K, int xr) {
 }
 
 template <typename T, int XR, bool GATED>
-hipError_t launch(const void* x, const void* wt, const void* bias, void* y, int M, int cols, int K, int ldy, hipStream_t st) {
+hipError_t launch(const void* x, const void* wt, const void* bias, const Outputs& out, int M, int cols, int K, hipStream_t st) {
     using P = PingPong<T, XR>;
     auto kern = dense_kernel<T, XR, GATED>;
     static bool raised = false;      // once per process and instantiation
@@ -108,18 +122,16 @@ hipError_t launch(const void* x, const void* wt, const void* bias, void* y, int 
     const int x_tiles = (int)cdiv(M, XR), w_tiles = (int)cdiv(cols, 256);
     (void)hipGetLastError();
     kern<<<dim3((unsigned)(cdiv((int64_t)x_tiles * w_tiles, 8) * 8)), dim3(P::kThreads), P::kLds, st>>>(
-        (const uint16_t*)x, (const uint16_t*)wt, (const uint16_t*)bias, (uint16_t*)y, M, cols, K, ldy, x_tiles, w_tiles);
+        (const uint16_t*)x, (const uint16_t*)wt, (const uint16_t*)bias, out, M, cols, K, x_tiles, w_tiles);
     return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_dense(const void* x, const void* wt, const void* bias, void* y, int M, int cols, int K, int ldy, int xr,
+hipError_t launch_dense(const void* x, const void* wt, const void* bias, const Outputs& out, int M, int cols, int K, int xr,
                         bool gated, hipStream_t st) {
     if (xr == 256)
-        return gated ? launch<T, 256, true>(x, wt, bias, y, M, cols, K, ldy, st)
-                     : launch<T, 256, false>(x, wt, bias, y, M, cols, K, ldy, st);
-    return gated ? launch<T, 128, true>(x, wt, bias, y, M, cols, K, ldy, st)
-                 : launch<T, 128, false>(x, wt, bias, y, M, cols, K, ldy, st);
+        return gated ? launch<T, 256, true>(x, wt, bias, out, M, cols, K, st) : launch<T, 256, false>(x, wt, bias, out, M, cols, K, st);
+    return gated ? launch<T, 128, true>(x, wt, bias, out, M, cols, K, st) : launch<T, 128, false>(x, wt, bias, out, M, cols, K, st);
 }
 
 // Sizes and group sizes the path takes; 32-bit offsets inside a tile's rows of x and inside a slab.
@@ -138,6 +150,31 @@ double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     const double cold = slab * K * 2 > (192ll << 20) ? 2.0 * (double)(K * N) / 6.0e6 : 0;
     return 4 + 2.5 * (double)(K * N) / 6.0e6 + cold +
            (double)cdiv(N, slab) * std::min(product_us(M, slab, K, 128), product_us(M, slab, K, 256));
+}
+
+size_t dense_parts_scratch_bytes(const int64_t* N, int count, int64_t M, int64_t K, int64_t g) {
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) {
+        if (N[i] <= 0 || N[i] % 256 != 0) return 0;      // a tile lies in one output
+        total += N[i];
+    }
+    return takes(M, total, K, g) && slab_columns(total, K) == total ? (size_t)(total * K * 2) : 0;
+}
+
+int dense_parts(const char* fn, const void* x, const Parts& parts, int64_t M, int64_t K, int64_t g, int dtype, void* scratch,
+                size_t scratch_bytes, hipStream_t st) {
+    const int64_t N[kMaxParts] = {parts.columns[0], parts.columns[1], parts.columns[2]};
+    const size_t need = dense_parts_scratch_bytes(N, parts.count, M, K, g);
+    if (!need || !scratch || scratch_bytes < need || (reinterpret_cast<uintptr_t>(scratch) & 15u)) {
+        set_error("%s: 16-byte aligned scratch of %zu bytes needed, %zu given", fn, need, scratch ? scratch_bytes : (size_t)0);
+        return AWQ_ERR_WORKSPACE;
+    }
+    const int xr = product_us(M, parts.total, K, 128) < product_us(M, parts.total, K, 256) ? 128 : 256;
+    hipError_t e = launch_dequant_transpose_parts(dtype, parts, scratch, (int)K, (int)g, st);
+    if (e == hipSuccess)
+        e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, nullptr, Outputs(parts), (int)M, parts.total, (int)K, xr, false, st)
+                             : launch_dense<BF16>(x, scratch, nullptr, Outputs(parts), (int)M, parts.total, (int)K, xr, false, st);
+    return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
 }
 
 }  // namespace awq
@@ -174,11 +211,10 @@ static int dense_entry(const char* fn, const void* x, const PackedWeight& w, con
         const int64_t cols = std::min(slab, cols_in_all - n), each = second ? 2 : 1;
         hipError_t e = launch_dequant_transpose(dtype, w, second, scratch, (int)N, (int)K, (int)g, st, n / each, cols / each);
         const void* b = bias ? static_cast<const uint16_t*>(bias) + n : nullptr;
-        void* out = static_cast<uint16_t*>(y) + (gated ? n / 2 : n);
-        const int ldy = (int)(gated ? cols_in_all / 2 : N);
+        const Outputs out(static_cast<uint16_t*>(y) + (gated ? n / 2 : n), (int)(gated ? cols_in_all / 2 : N));
         if (e == hipSuccess)
-            e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated, st)
-                                 : launch_dense<BF16>(x, scratch, b, out, (int)M, (int)cols, (int)K, ldy, xr, gated, st);
+            e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, b, out, (int)M, (int)cols, (int)K, xr, gated, st)
+                                 : launch_dense<BF16>(x, scratch, b, out, (int)M, (int)cols, (int)K, xr, gated, st);
         if (e != hipSuccess) return hip_fail(fn, e);
     }
     return AWQ_OK;

@@ -124,22 +124,9 @@ __device__ __forceinline__ void gemm_epilogue(f32x16 (&acc)[TM][TN], const uint1
         }
 }
 
-// Second pass of a split-K product: y = dtype(sum over splits, in split order, of the fp32
-// partials [splits][M][N] (+ bias)).  A thread owns 8 consecutive columns of one row.
-template <typename T>
-__global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ partials,
-                                                                 const uint16_t* __restrict__ bias,
-                                                                 uint16_t* __restrict__ y, int64_t M, int N,
-                                                                 int splits, bool gated) {
-    const int64_t vec = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int per_row = N >> 3;
-    if (vec >= M * per_row) return;
-    const int64_t m = vec / per_row;
-    const int nn = (int)(vec % per_row) * 8;
-    const size_t plane = (size_t)M * N;
-    const float* p = partials + (size_t)m * N + nn;
-    f32x4 lo = f32x4{0.f, 0.f, 0.f, 0.f}, hi = lo;
-    // four splits' loads in flight at a time, added in split order
+// Eight values at p, p + plane, ..: four splits' loads in flight at a time, added in split order.
+__device__ __forceinline__ void add_splits(const float* p, size_t plane, int splits, f32x4& lo, f32x4& hi) {
+    lo = hi = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < splits; s0 += 4) {
         f32x4 a[4], b[4];
 #pragma unroll
@@ -155,6 +142,22 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
                 hi += b[u];
             }
     }
+}
+
+// Second pass of a split-K product: y = dtype(sum over splits, in split order, of the fp32
+// partials [splits][M][N] (+ bias)).  A thread owns 8 consecutive columns of one row.
+template <typename T>
+__global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __restrict__ partials,
+                                                                 const uint16_t* __restrict__ bias,
+                                                                 uint16_t* __restrict__ y, int64_t M, int N,
+                                                                 int splits, bool gated) {
+    const int64_t vec = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int per_row = N >> 3;
+    if (vec >= M * per_row) return;
+    const int64_t m = vec / per_row;
+    const int nn = (int)(vec % per_row) * 8;
+    f32x4 lo, hi;
+    add_splits(partials + (size_t)m * N + nn, (size_t)M * N, splits, lo, hi);
     float out[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     if (bias) {
         const u32x4 bvv = *reinterpret_cast<const u32x4*>(bias + nn);
@@ -241,6 +244,40 @@ struct PackedWeight {
 hipError_t launch_dequant_transpose(int dtype, const PackedWeight& w, const PackedWeight* second, void* wt, int N, int K, int g,
                                     hipStream_t stream, int64_t first, int64_t count);
 
+// Up to three weights of one K and group size whose products with the same x run in one launch, each into its own output
+// [M, columns]; with more than one the columns are whole tiles.  `first`: columns of those before, INT_MAX of those not there.
+constexpr int kMaxParts = 3;
+struct Parts {
+    const uint32_t* qweight[kMaxParts];
+    const uint16_t* scales[kMaxParts];
+    const uint32_t* qzeros[kMaxParts];
+    uint16_t* y[kMaxParts];
+    int columns[kMaxParts], first[kMaxParts];
+    int count, total;        // weights, columns of all
+    Parts() = default;
+    Parts(const PackedWeight& w, void* out, int64_t N) : count(0), total(0) { add(w, out, N); }
+    void add(const PackedWeight& w, void* out, int64_t N) {
+        qweight[count] = w.qweight, scales[count] = w.scales, qzeros[count] = w.qzeros, y[count] = static_cast<uint16_t*>(out);
+        columns[count] = (int)N, first[count] = total;
+        total += (int)N;
+        for (int i = ++count; i < kMaxParts; ++i) {
+            qweight[i] = qweight[0], scales[i] = scales[0], qzeros[i] = qzeros[0], y[i] = y[0];
+            columns[i] = columns[0], first[i] = 0x7fffffff;
+        }
+    }
+    __device__ __forceinline__ int of(int column) const { return (column >= first[1]) + (column >= first[2]); }
+};
+template <typename V>
+__device__ __forceinline__ V pick_part(const V (&a)[kMaxParts], int part) { return part == 0 ? a[0] : (part == 1 ? a[1] : a[2]); }
+
+// awq_gemm_pipe.hip: all of the parts' columns dequantised and transposed, one after the other, in one launch.
+hipError_t launch_dequant_transpose_parts(int dtype, const Parts& parts, void* wt, int K, int g, hipStream_t stream);
+// awq_gemm_dense.hip: the product of many rows over a dequantised slab that holds all parts.
+int dense_parts(const char* fn, const void* x, const Parts& parts, int64_t M, int64_t K, int64_t g, int dtype, void* scratch,
+                size_t scratch_bytes, hipStream_t stream);
+// Bytes of that slab, 0 where the path does not take the sizes.
+size_t dense_parts_scratch_bytes(const int64_t* N, int count, int64_t M, int64_t K, int64_t g);
+
 // awq_gemm_dense.hip: estimated microseconds of awq_linear_dense, -1 where it does not take the sizes.
 double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g);
 
@@ -254,8 +291,7 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, i
 inline size_t rows_ws_bytes(const RowsPlan& p, int64_t M, int64_t N) {
     return p.splits > 1 ? kCounterBytes + (size_t)p.splits * M * N * sizeof(float) : 0;
 }
-hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_t* qweight, const void* qscales,
-                       const int32_t* qzeros, const void* bias, void* y, int M, int N, int K, int g, void* workspace,
-                       bool gated, hipStream_t st);   // gated: as PipePlan::act
+hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const Parts& parts, const void* bias, int M, int K, int g,
+                       void* workspace, bool gated, hipStream_t st);   // the plan of all columns; gated: as PipePlan::act, one part
 
 }  // namespace awq

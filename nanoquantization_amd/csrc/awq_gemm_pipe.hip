@@ -353,17 +353,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_pipe_kernel(
 // HBM-bound: 0.52 B read + 2 B written per weight.
 // PAIR: a second weight of the same sizes in grid z; the rows of the two alternate by eights, the first weight's in front.
 template <typename T, bool PAIR>
-__global__ __launch_bounds__(256) void dequant_transpose_kernel(PackedWeight first_weight, PackedWeight second_weight,
-                                                                uint16_t* __restrict__ wt, int N, int K, int g, int first,
-                                                                int count) {
-    const bool second = PAIR && blockIdx.z;
-    const uint32_t* __restrict__ qweight = second ? second_weight.qweight : first_weight.qweight;
-    const uint16_t* __restrict__ scales = second ? second_weight.scales : first_weight.scales;
-    const uint32_t* __restrict__ qzeros = second ? second_weight.qzeros : first_weight.qzeros;
+__device__ __forceinline__ void dequant_transpose_block(const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales,
+                                                        const uint32_t* __restrict__ qzeros, uint16_t* __restrict__ wt, int N,
+                                                        int K, int g, int first, int count, int n0, bool second) {
     __shared__ u32x4 tile[256 * 8];   // [n][8 chunks of 8 k], chunk kc of row n at n*8 + (kc ^ ((n >> 3) & 7))
     const int tid = threadIdx.x, wc = tid & 31, rb = tid >> 5;
     const int words = N >> 3;
-    const int k0 = blockIdx.y * 64, n0 = blockIdx.x * 256;
+    const int k0 = blockIdx.y * 64;
     const int gwc = min(((first + n0) >> 3) + wc, words - 1);
     const int krow = k0 + rb * 8;
     uint32_t w[8];
@@ -394,6 +390,24 @@ __global__ __launch_bounds__(256) void dequant_transpose_kernel(PackedWeight fir
         if (n0 + n < count)
             *reinterpret_cast<u32x4*>(wt + (size_t)row * K + k0 + kc * 8) = tile[n * 8 + (kc ^ ((n >> 3) & 7))];
     }
+}
+
+template <typename T, bool PAIR>
+__global__ __launch_bounds__(256) void dequant_transpose_kernel(PackedWeight first_weight, PackedWeight second_weight,
+                                                                uint16_t* __restrict__ wt, int N, int K, int g, int first,
+                                                                int count) {
+    const bool second = PAIR && blockIdx.z;
+    const PackedWeight& w = second ? second_weight : first_weight;
+    dequant_transpose_block<T, PAIR>(w.qweight, w.scales, w.qzeros, wt, N, K, g, first, count, blockIdx.x * 256, second);
+}
+
+// The columns of several weights one after the other, each in whole blocks.
+template <typename T>
+__global__ __launch_bounds__(256) void dequant_transpose_parts_kernel(Parts parts, uint16_t* __restrict__ wt, int K, int g) {
+    const int column = blockIdx.x * 256, part = parts.of(column);
+    const int N = pick_part(parts.columns, part), first = pick_part(parts.first, part);
+    dequant_transpose_block<T, false>(pick_part(parts.qweight, part), pick_part(parts.scales, part), pick_part(parts.qzeros, part),
+                                      wt + (size_t)first * K, N, K, g, 0, N, column - first, false);
 }
 
 // Second pass over the tail tiles: y = dtype(sum over K slices, in slice order, of the fp32 partials (+ bias)).
@@ -511,6 +525,14 @@ hipError_t launch_dequant_transpose(int dtype, const PackedWeight& w, const Pack
     };
     if (dtype == AWQ_F16) second ? go(dequant_transpose_kernel<F16, true>) : go(dequant_transpose_kernel<F16, false>);
     else second ? go(dequant_transpose_kernel<BF16, true>) : go(dequant_transpose_kernel<BF16, false>);
+    return hipGetLastError();
+}
+
+hipError_t launch_dequant_transpose_parts(int dtype, const Parts& parts, void* wt, int K, int g, hipStream_t stream) {
+    (void)hipGetLastError();
+    const dim3 grid((unsigned)(parts.total / 256), K / 64), block(256);
+    if (dtype == AWQ_F16) dequant_transpose_parts_kernel<F16><<<grid, block, 0, stream>>>(parts, reinterpret_cast<uint16_t*>(wt), K, g);
+    else dequant_transpose_parts_kernel<BF16><<<grid, block, 0, stream>>>(parts, reinterpret_cast<uint16_t*>(wt), K, g);
     return hipGetLastError();
 }
 

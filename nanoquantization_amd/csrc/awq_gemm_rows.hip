@@ -105,9 +105,8 @@ struct Columns<BF16> {
 
 template <typename T, int MT>
 __device__ __forceinline__ void rows_tile(
-    const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales,
-    const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-    float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
+    const uint16_t* __restrict__ x, const Parts& parts, const uint16_t* __restrict__ bias, float* __restrict__ partials, int M, int K,
+    int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
     constexpr int kStage = stage_bytes(MT), kWords = MT * 2048, kScales = kWords + 4096;
     constexpr int kPairs = pairs(MT), kFours = fours(MT), kGiven = 8 * 4096 * kFours;
@@ -115,7 +114,13 @@ __device__ __forceinline__ void rows_tile(
     const int per = gridDim.x >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (id >= items) return;
     const int split = id % splits, tile = id / splits;
-    const int m0 = tile % m_tiles * (16 * MT), tn = tile / m_tiles;
+    const int m0 = tile % m_tiles * (16 * MT), column = tile / m_tiles * 128, part = parts.of(column);
+    const uint32_t* __restrict__ qweight = pick_part(parts.qweight, part);
+    const uint16_t* __restrict__ scales = pick_part(parts.scales, part);
+    const uint32_t* __restrict__ qzeros = pick_part(parts.qzeros, part);
+    uint16_t* __restrict__ y = pick_part(parts.y, part);
+    const int N = pick_part(parts.columns, part), first = pick_part(parts.first, part), tn = (column - first) >> 7;
+    partials += (size_t)splits * M * first;        // a part's partials [split][M][its columns] behind those of the parts before it
     const int words = N >> 3;
     const int word0 = min(16 * tn, words - 16);     // a last tile that is not whole begins earlier (N >= 128) and stores some columns again
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -139,7 +144,7 @@ __device__ __forceinline__ void rows_tile(
 #pragma unroll
     for (int q = 0; q < kMost; ++q) {
         const int i = 8 * q + wave;
-        const uint64_t p = reinterpret_cast<uint64_t>(i < 2 * MT ? (const void*)x : (const void*)qweight);
+        const uint64_t p = i < 2 * MT ? reinterpret_cast<uint64_t>(x) : reinterpret_cast<uint64_t>(qweight);
         // (a descriptor that the compiler does not see to be the same in all lanes costs a loop over the lanes)
         operand[q] = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
         if (i < 2 * MT) {
@@ -353,15 +358,29 @@ __device__ __forceinline__ void rows_tile(
 
 template <typename T, int MT>
 __global__ __launch_bounds__(kThreads, 2 * per_cu(MT)) void rows_kernel(
-    const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight, const uint16_t* __restrict__ scales,
-    const uint32_t* __restrict__ qzeros, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-    float* __restrict__ partials, int M, int N, int K, int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
-    rows_tile<T, MT>(x, qweight, scales, qzeros, bias, y, partials, M, N, K, g, m_tiles, items, steps_per_split, splits, gated);
+    const uint16_t* __restrict__ x, Parts parts, const uint16_t* __restrict__ bias, float* __restrict__ partials, int M, int K,
+    int g, int m_tiles, int items, int steps_per_split, int splits, bool gated) {
+    rows_tile<T, MT>(x, parts, bias, partials, M, K, g, m_tiles, items, steps_per_split, splits, gated);
+}
+
+// y = dtype(sum over splits, in split order) of every part; a thread owns 8 consecutive columns of one row.
+template <typename T>
+__global__ __launch_bounds__(256) void rows_sum_kernel(const float* __restrict__ partials, Parts parts, int64_t M, int splits) {
+    const int64_t vec = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int per_row = parts.total >> 3;
+    if (vec >= M * per_row) return;
+    const int64_t m = vec / per_row;
+    const int column = (int)(vec % per_row) * 8, part = parts.of(column);
+    const int N = pick_part(parts.columns, part), first = pick_part(parts.first, part);
+    f32x4 lo, hi;
+    add_splits(partials + (size_t)splits * M * first + (size_t)m * N + (column - first), (size_t)M * N, splits, lo, hi);
+    *reinterpret_cast<u32x4*>(pick_part(parts.y, part) + (size_t)m * N + (column - first)) =
+        u32x4{T::pack2(lo[0], lo[1]), T::pack2(lo[2], lo[3]), T::pack2(hi[0], hi[1]), T::pack2(hi[2], hi[3])};
 }
 
 template <typename T, int MT>
-hipError_t launch(const RowsPlan& p, const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
-                  const void* bias, void* y, float* partials, int M, int N, int K, int g, bool gated, hipStream_t st) {
+hipError_t launch(const RowsPlan& p, const void* x, const Parts& parts, const void* bias, float* partials, int M, int K, int g,
+                  bool gated, hipStream_t st) {
     auto kern = rows_kernel<T, MT>;
     static bool raised = false;      // once per process and instantiation
     if (!raised) {
@@ -373,8 +392,7 @@ hipError_t launch(const RowsPlan& p, const void* x, const int32_t* qweight, cons
     (void)hipGetLastError();
     const int items = p.m_tiles * p.n_tiles * p.splits;
     kern<<<dim3((unsigned)(cdiv(items, 8) * 8)), dim3(kThreads), lds_bytes(MT), st>>>(
-        (const uint16_t*)x, (const uint32_t*)qweight, (const uint16_t*)qscales, (const uint32_t*)qzeros, (const uint16_t*)bias,
-        (uint16_t*)y, partials, M, N, K, g, p.m_tiles, items, p.steps_per_split, p.splits, gated);
+        (const uint16_t*)x, parts, (const uint16_t*)bias, partials, M, K, g, p.m_tiles, items, p.steps_per_split, p.splits, gated);
     return hipGetLastError();
 }
 
@@ -412,12 +430,11 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, i
     return p;
 }
 
-hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_t* qweight, const void* qscales,
-                       const int32_t* qzeros, const void* bias, void* y, int M, int N, int K, int g, void* workspace,
-                       bool gated, hipStream_t st) {
+hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const Parts& parts, const void* bias, int M, int K, int g,
+                       void* workspace, bool gated, hipStream_t st) {
     float* partials = p.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kCounterBytes) : nullptr;
 #define AWQ_ROWS(T, MT) \
-    if (p.mt == MT) e = launch<T, MT>(p, x, qweight, qscales, qzeros, bias, y, partials, M, N, K, g, gated, st);
+    if (p.mt == MT) e = launch<T, MT>(p, x, parts, bias, partials, M, K, g, gated, st);
     hipError_t e = hipErrorInvalidValue;
     if (dtype == AWQ_F16) {
         AWQ_ROWS(F16, 2) AWQ_ROWS(F16, 3) AWQ_ROWS(F16, 4)
@@ -428,7 +445,11 @@ hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const int32_
     }
 #undef AWQ_ROWS
     if (e != hipSuccess || p.splits == 1) return e;
-    return launch_splitk_reduce(dtype, partials, bias, y, M, N, p.splits, st, gated);
+    if (parts.count == 1) return launch_splitk_reduce(dtype, partials, bias, parts.y[0], M, parts.total, p.splits, st, gated);
+    const dim3 grid((unsigned)cdiv((int64_t)M * (parts.total >> 3), 256)), block(256);
+    if (dtype == AWQ_F16) rows_sum_kernel<F16><<<grid, block, 0, st>>>(partials, parts, M, p.splits);
+    else rows_sum_kernel<BF16><<<grid, block, 0, st>>>(partials, parts, M, p.splits);
+    return hipGetLastError();
 }
 
 }  // namespace awq

@@ -9,7 +9,7 @@
 //   torch.ops.nanoquantization_amd.awq_linear_swiglu(x, qweight, qscales, qzeros) -> Tensor [M, N / 2]
 // and the steps between the linears of the Qwen3 modules (nanoquantization/layers/norm.py:18-32, layers/rope.py:24-45,
 // models/qwen3_quantized.py:79-99, 147-152), inference only (none has a derivative):
-//   awq_swiglu_pair, rms_norm, silu_mul, qkv_norm_rope, causal_attention
+//   awq_swiglu_pair, awq_linear_three, rms_norm, silu_mul, qkv_norm_rope, causal_attention
 // with Meta kernels (shapes only), so the operators are visible to the dispatcher and to tracing.
 #include <dlfcn.h>
 
@@ -18,6 +18,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/library.h>
 
+#include <array>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -98,16 +99,19 @@ at::Tensor workspace(const at::Device& dev, void* stream, size_t nbytes) {
     return ws;
 }
 
-// Scratch for awq_linear_dense where that is the fastest way, else undefined.  From the caching allocator for this one call
-// (ordered on the current stream like any temporary); without room for it the fused kernels run.
-at::Tensor dense_scratch(const at::Device& dev, int64_t M, const Packed& p) {
-    const size_t nbytes = M > 128 ? awq_linear_scratch_bytes(M, p.N, p.K, p.g, p.dtype) : 0;
-    if (!nbytes) return {};
+// Memory from the caching allocator for one call (ordered on the current stream like any temporary); undefined without room.
+at::Tensor bytes_or_none(const at::Device& dev, size_t nbytes) {
     try {
         return at::empty({(int64_t)nbytes}, at::TensorOptions().dtype(at::kByte).device(dev));
     } catch (const c10::OutOfMemoryError&) {
         return {};
     }
+}
+
+// Scratch for awq_linear_dense where that is the fastest way, else undefined; without room for it the fused kernels run.
+at::Tensor dense_scratch(const at::Device& dev, int64_t M, const Packed& p) {
+    const size_t nbytes = M > 128 ? awq_linear_scratch_bytes(M, p.N, p.K, p.g, p.dtype) : 0;
+    return nbytes ? bytes_or_none(dev, nbytes) : at::Tensor();
 }
 
 at::Tensor awq_dequantize_op(const at::Tensor& qweight, const at::Tensor& qscales, const at::Tensor& qzeros) {
@@ -257,6 +261,54 @@ at::Tensor silu_mul_op(const at::Tensor& gate, const at::Tensor& up) {
 }
 at::Tensor silu_mul_meta(const at::Tensor& gate, const at::Tensor&) { return at::empty(gate.sizes(), gate.options()); }
 
+// Linears without bias of one input, by triples of packed weight, scales and zero points: one launch where that is the fastest
+// way, else one each.
+std::vector<at::Tensor> linear_parts(const at::Tensor& x, const std::vector<std::array<at::Tensor, 3>>& in) {
+    const int count = (int)in.size();
+    Packed p[3];
+    int64_t N[3];
+    TORCH_CHECK(count >= 1 && count <= 3, "one to three weights");
+    for (int i = 0; i < count; ++i) {
+        p[i] = check_packed(in[i][0], in[i][1], in[i][2]);
+        TORCH_CHECK(p[i].K == p[0].K && p[i].g == p[0].g && p[i].dtype == p[0].dtype, "the weights must have one K, group size and type");
+        check_device(x, {&in[i][0], &in[i][1], &in[i][2]});
+        N[i] = p[i].N;
+    }
+    TORCH_CHECK(x.dim() == 2 && x.size(1) == p[0].K, "x must be [M, ", p[0].K, "], got ", x.sizes());
+    const DeviceGuard guard(x.device());
+    const int64_t M = x.size(0);
+    size_t nbytes = 0, scratch_bytes = 0;
+    at::Tensor scratch;
+    std::vector<at::Tensor> out(count);
+    bool one = awq_linear_parts_wanted(N, count, M, p[0].K, p[0].g, p[0].dtype, &nbytes, &scratch_bytes) != 0;
+    if (one && scratch_bytes) one = (scratch = bytes_or_none(x.device(), scratch_bytes)).defined();
+    if (!one) {
+        for (int i = 0; i < count; ++i) out[i] = awq_linear_op(x, in[i][0], in[i][1], in[i][2], c10::nullopt);
+        return out;
+    }
+    const at::ScalarType dt = in[0][1].scalar_type();
+    const at::Tensor xc = (x.scalar_type() == dt ? x : x.to(dt)).contiguous();
+    at::Tensor dense[3][3];
+    const int32_t* words[3];
+    const void* scales[3];
+    const int32_t* zeros[3];
+    void* y[3];
+    for (int i = 0; i < count; ++i) {
+        for (int j = 0; j < 3; ++j) dense[i][j] = in[i][j].contiguous();
+        out[i] = at::empty({M, N[i]}, in[0][1].options());
+        words[i] = dense[i][0].data_ptr<int32_t>(), scales[i] = dense[i][1].data_ptr(), zeros[i] = dense[i][2].data_ptr<int32_t>();
+        y[i] = out[i].data_ptr();
+    }
+    hipStream_t stream = current_stream(x.device().index());
+    at::Tensor ws;
+    if (nbytes) ws = workspace(x.device(), stream, nbytes);
+    check_status(awq_linear_parts(xc.data_ptr(), words, scales, zeros, y, N, count, M, p[0].K, p[0].g, p[0].dtype,
+                                  nbytes ? ws.data_ptr() : nullptr, nbytes ? (size_t)ws.numel() : 0,
+                                  scratch.defined() ? scratch.data_ptr() : nullptr, scratch_bytes, stream),
+                 "awq_linear_parts");
+    return out;
+}
+
 // gate and up of an MLP that lie apart: one product where the rows are many, else two and the activation.
 at::Tensor awq_swiglu_pair_op(const at::Tensor& x, const at::Tensor& gate_qweight, const at::Tensor& gate_qscales,
                               const at::Tensor& gate_qzeros, const at::Tensor& up_qweight, const at::Tensor& up_qscales,
@@ -270,9 +322,10 @@ at::Tensor awq_swiglu_pair_op(const at::Tensor& x, const at::Tensor& gate_qweigh
     const int64_t M = x.size(0);
     p.N *= 2;
     const at::Tensor scratch = M > 0 ? dense_scratch(x.device(), M, p) : at::Tensor();
-    if (!scratch.defined())
-        return silu_mul_op(awq_linear_op(x, gate_qweight, gate_qscales, gate_qzeros, c10::nullopt),
-                           awq_linear_op(x, up_qweight, up_qscales, up_qzeros, c10::nullopt));
+    if (!scratch.defined()) {
+        const std::vector<at::Tensor> y = linear_parts(x, {{gate_qweight, gate_qscales, gate_qzeros}, {up_qweight, up_qscales, up_qzeros}});
+        return silu_mul_op(y[0], y[1]);
+    }
     const at::ScalarType dt = gate_qscales.scalar_type();
     const at::Tensor xc = (x.scalar_type() == dt ? x : x.to(dt)).contiguous();
     const at::Tensor gw = gate_qweight.contiguous(), gs = gate_qscales.contiguous(), gz = gate_qzeros.contiguous(),
@@ -291,6 +344,20 @@ at::Tensor awq_swiglu_pair_meta(const at::Tensor& x, const at::Tensor&, const at
 }
 
 using Three = std::tuple<at::Tensor, at::Tensor, at::Tensor>;
+
+// Three linears without bias of one input.
+Three awq_linear_three_op(const at::Tensor& x, const at::Tensor& qweight0, const at::Tensor& qscales0, const at::Tensor& qzeros0,
+                          const at::Tensor& qweight1, const at::Tensor& qscales1, const at::Tensor& qzeros1,
+                          const at::Tensor& qweight2, const at::Tensor& qscales2, const at::Tensor& qzeros2) {
+    std::vector<at::Tensor> y = linear_parts(x, {{qweight0, qscales0, qzeros0}, {qweight1, qscales1, qzeros1}, {qweight2, qscales2, qzeros2}});
+    return {y[0], y[1], y[2]};
+}
+Three awq_linear_three_meta(const at::Tensor& x, const at::Tensor&, const at::Tensor& qscales0, const at::Tensor&, const at::Tensor&,
+                            const at::Tensor& qscales1, const at::Tensor&, const at::Tensor&, const at::Tensor& qscales2,
+                            const at::Tensor&) {
+    const auto like = [&](const at::Tensor& s) { return at::empty({x.size(0), s.size(1)}, s.options()); };
+    return {like(qscales0), like(qscales1), like(qscales2)};
+}
 
 Three qkv_outputs(const at::Tensor& q, int64_t heads, int64_t kv_heads) {
     const int64_t b = q.size(0), s = q.size(1), hd = q.size(2) / heads;
@@ -377,6 +444,8 @@ TORCH_LIBRARY(nanoquantization_amd, m) {
     m.def("awq_linear_swiglu(Tensor x, Tensor qweight, Tensor qscales, Tensor qzeros) -> Tensor");
     m.def("awq_swiglu_pair(Tensor x, Tensor gate_qweight, Tensor gate_qscales, Tensor gate_qzeros, Tensor up_qweight, "
           "Tensor up_qscales, Tensor up_qzeros) -> Tensor");
+    m.def("awq_linear_three(Tensor x, Tensor qweight0, Tensor qscales0, Tensor qzeros0, Tensor qweight1, Tensor qscales1, Tensor "
+          "qzeros1, Tensor qweight2, Tensor qscales2, Tensor qzeros2) -> (Tensor, Tensor, Tensor)");
     m.def("rms_norm(Tensor x, Tensor weight, float eps) -> Tensor");
     m.def("silu_mul(Tensor gate, Tensor up) -> Tensor");
     m.def("qkv_norm_rope(Tensor q, Tensor k, Tensor v, Tensor q_weight, Tensor k_weight, Tensor cos_sin, Tensor positions, "
@@ -389,6 +458,7 @@ TORCH_LIBRARY_IMPL(nanoquantization_amd, CUDA, m) {   // the dispatch key of HIP
     m.impl("awq_linear", &awq_linear_op);
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_op);
     m.impl("awq_swiglu_pair", &awq_swiglu_pair_op);
+    m.impl("awq_linear_three", &awq_linear_three_op);
     m.impl("rms_norm", &rms_norm_op);
     m.impl("silu_mul", &silu_mul_op);
     m.impl("qkv_norm_rope", &qkv_norm_rope_op);
@@ -400,6 +470,7 @@ TORCH_LIBRARY_IMPL(nanoquantization_amd, Meta, m) {
     m.impl("awq_linear", &awq_linear_meta);
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_meta);
     m.impl("awq_swiglu_pair", &awq_swiglu_pair_meta);
+    m.impl("awq_linear_three", &awq_linear_three_meta);
     m.impl("rms_norm", &rms_norm_meta);
     m.impl("silu_mul", &silu_mul_meta);
     m.impl("qkv_norm_rope", &qkv_norm_rope_meta);

@@ -76,8 +76,19 @@ class Qwen3QuantizedAttention(nn.Module):
                                            enable_gqa=self.num_heads != self.num_kv_heads)
         return self.o_proj(o.transpose(1, 2).reshape(q.shape[0], -1, self.num_heads * self.head_dim))
 
+    def _project(self, x: torch.Tensor):
+        """q, k and v: one call, which may be one launch, where the projections are this package's, unchanged and watched by no hook."""
+        parts = (self.q_proj, self.k_proj, self.v_proj)
+        if (all(type(m) is WQLinear_GEMM and m.bias is None and keeps(m, WQLinear_GEMM, "forward") for m in parts)
+                and plain(x, *(m.qscales for m in parts)) and x.dim() > 1
+                and all(m.qweight.dim() == m.qscales.dim() == m.qzeros.dim() == 2 and m.qweight.shape[0] == x.shape[-1]
+                        and m.qscales.shape[0] == parts[0].qscales.shape[0] for m in parts) and unhooked(*parts)):
+            out = _lib.torch_ops().awq_linear_three(x.reshape(-1, x.shape[-1]), *(t for m in parts for t in (m.qweight, m.qscales, m.qzeros)))
+            return tuple(y.view(*x.shape[:-1], y.shape[-1]) for y in out)
+        return self.q_proj(x), self.k_proj(x), self.v_proj(x)
+
     def _on_operators(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
-        q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        q, k, v = self._project(x)
         if not self._fused(q, k, v, position_ids):
             q, k, v = self._norm_rope(q, k, v, position_ids)
             return self._attend(q, k, v)

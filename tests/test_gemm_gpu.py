@@ -460,6 +460,45 @@ def test_gemm_rows128_few_rows(dtype, M, K, N, g, split):
         assert torch.equal(nq.awq_gemm(xd, *dev, 8), awq_gemm_variant(xd, *dev, v, chosen.value))
 
 
+# tiles of few rows unsplit and in K splits, dequantised first with tiles of 128 and of 256 rows; widths that are no whole tiles, a K
+# and rows that the one launch does not take
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,K,N,g,way", [(129, 1024, (2048, 1024, 1024), 128, "rows"), (200, 4096, (1024, 256, 128), 64, "rows"), (40, 512, (128, 384, 128), 32, "rows"),
+                                         (1700, 2048, (2048, 1024, 1024), 128, "dense"), (4096, 1024, (512, 256, 1280), 64, "dense"),
+                                         (300, 512, (256, 136, 128), 64, ""), (300, 96, (256, 128, 128), 32, ""), (100, 1024, (256, 128, 128), 128, ""), (1, 1024, (256, 128, 128), 64, "")])
+def test_linear_parts(dtype, M, K, N, g, way):
+    """Three weights in one launch: the bits of the same kernel on the weights side by side; else those of three linears."""
+    print(f"linear parts {dtype} M={M} K={K} N={N} g={g} {way}", flush=True)
+    L, tdt = _lib.lib(), torch.float16 if dtype == "f16" else torch.bfloat16
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    words = lambda r, n: torch.randint(-2 ** 31, 2 ** 31 - 1, (r, n // 8), dtype=torch.int32, device="cuda", generator=gen)
+    parts = [(words(K, n), ((torch.rand(K // g, n, device="cuda", generator=gen) + 0.1) * 0.2 / K ** 0.5).to(tdt), words(K // g, n)) for n in N]
+    x = torch.randn(M, K, device="cuda", generator=gen).to(tdt)
+    ws, scratch = ctypes.c_size_t(), ctypes.c_size_t()
+    wanted = L.awq_linear_parts_wanted((ctypes.c_int64 * 3)(*N), 3, M, K, g, _lib.dtype_id(tdt), ctypes.byref(ws), ctypes.byref(scratch))
+    assert bool(wanted) == bool(way) and bool(scratch.value) == (way == "dense")
+    y = _lib.torch_ops().awq_linear_three(x, *(t for p in parts for t in p))
+    assert [tuple(t.shape) for t in y] == [(M, n) for n in N] and all(t.is_contiguous() for t in y)
+    if not way:
+        for t, p in zip(y, parts):
+            assert torch.equal(t, nq.awq_gemm(x, *p, 8))
+        return
+    side = [torch.cat(t, dim=1).contiguous() for t in zip(*parts)]
+    if way == "dense":
+        want, room = torch.empty(M, sum(N), dtype=tdt, device="cuda"), torch.empty(scratch.value, dtype=torch.uint8, device="cuda")
+        _lib.check(L.awq_linear_dense(x.data_ptr(), *(t.data_ptr() for t in side), None, want.data_ptr(), M, sum(N), K, g, _lib.dtype_id(tdt), 0,
+                                      room.data_ptr(), room.numel(), _lib.current_stream_ptr(x.device)))
+    else:
+        v = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())].index("rows128")
+        split = 1
+        while ws.value and L.awq_gemm_ex_workspace_bytes(M, sum(N), K, v, split) != ws.value:
+            split += 1
+        want = awq_gemm_variant(x, *side, v, split)
+    assert torch.equal(torch.cat(y, dim=1), want)
+    ref = x.double() @ nq.awq_dequantize(*side).double()
+    assert (want.double() - ref).abs().max().item() <= TIGHT[dtype] * ref.abs().max().item()
+
+
 def test_gemm_rows128_routes():
     """The default linear takes these tiles for a few hundred rows, with the bits of the forced variant; what they refuse, short
     K and the plan of awq_gemm stay with the other kernels."""
