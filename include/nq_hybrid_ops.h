@@ -239,6 +239,13 @@ int nqh_moe_down(const void* act, const void* down, const int32_t* order, const 
 int nqh_skinny_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
                       int64_t in_features, int out_f32, int act, float param, void* stream);
 
+/* y [rows, out_features] = act(x @ weight^T), bf16, act applied to the product rounded to bf16; for many rows.  in_features a
+ * multiple of 64, out_features one of 8, all pointers 16-byte aligned, rows without padding.  act and param as in nqh_activate.
+ * nqh_dense_activation_wanted: 1 where it takes the sizes and is faster than a library product with nqh_activate behind it. */
+int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_features);
+int nqh_dense_activation(const void* x, const void* weight, void* y, int64_t rows, int64_t out_features, int64_t in_features, int act,
+                         float param, void* stream);
+
 /* Decode-step bookkeeping, as nq_argmax_rows / nq_decode_prepare / nq_decode_advance (nq_engine_ops.h) do it; the
  * logits are fp32. */
 int nqh_argmax_rows(const float* logits, int64_t* out, int64_t rows, int64_t vocab, void* stream);

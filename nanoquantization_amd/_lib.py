@@ -132,6 +132,8 @@ HYBRID_SYMBOLS = {
     "nqh_moe_gate_up": (_int, [_vp] * 6 + [_i64] * 7 + [_int, _vp]),
     "nqh_moe_down": (_int, [_vp] * 5 + [_i64] * 6 + [_int, _vp]),
     "nqh_skinny_linear": (_int, [_vp] * 4 + [_i64] * 3 + [_int, _int, _f32, _vp]),
+    "nqh_dense_activation_wanted": (_int, [_i64] * 3),
+    "nqh_dense_activation": (_int, [_vp] * 3 + [_i64] * 3 + [_int, _f32, _vp]),
     "nqh_argmax_rows": (_int, [_vp, _vp, _i64, _i64, _vp]),
     "nqh_decode_prepare": (_int, [_vp] * 5 + [_i64] * 3 + [_vp]),
     "nqh_decode_advance": (_int, [_vp] * 6 + [_i64] * 2 + [_vp]),

@@ -1,7 +1,11 @@
-// Dense linear for few rows: y = act(x W^T (+ bias)), bf16 operands, fp32 accumulation.
+// Dense linears.  For few rows: y = act(x W^T (+ bias)), bf16 operands, fp32 accumulation.
 //   up to 16 rows    skinny_linear_kernel: both operands straight from memory, the waves split the contraction; also for more
 //                    rows of few features, 16 at a time, where the next would leave most of the chip idle
 //   17 to 64 rows    wide_linear_kernel: the activations, by now as many bytes per workgroup as its weights, go through LDS
+// and y = act(x W^T) for more rows where an activation follows, dense_activation_kernel.
+#include <algorithm>
+
+#include "../pingpong.hpp"
 #include "skinny.hpp"
 
 namespace nqh {
@@ -116,6 +120,82 @@ int launch_wide(const char* fn, const void* x, const void* w, const void* bias, 
     return launched(fn);
 }
 
+// ---- many rows: activation(x @ weight^T) on the tiles of pingpong.hpp -------------------------------------------------
+// The activation of a library product is a pass of its own that reads and writes the result once more.  Here it is applied
+// on the way out of the tile, to the value rounded to bf16 as that pass finds it: the same results but for the order of the sums.
+// Bound by the matrix cores from a few hundred rows on, by the fill and store of its one tile below.
+template <int XR>
+__global__ __launch_bounds__(512, 2) void dense_activation_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                                  uint16_t* __restrict__ y, int rows, int n_out, int n_in, int act,
+                                                                  float param, int x_tiles, int w_tiles) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char s_stage[];
+    using P = awq::PingPong<Bf, XR>;
+    int xt, wt;
+    if (!awq::xcd_tile((int)blockIdx.x, x_tiles, w_tiles, xt, wt)) return;
+    P p;
+    const int m0 = xt * XR, n0 = wt * 256, count = min(XR, rows - m0);
+    const uint32_t row_bytes = (uint32_t)n_in * 2;
+    uint32_t vw[4], vx[P::kXLoads];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int r = P::w_row(q, p.wave, p.lane);
+        vw[q] = P::source(n0 + r, n_out, row_bytes, r, p.lane);
+    }
+#pragma unroll
+    for (int q = 0; q < P::kXLoads; ++q) {
+        const int r = P::x_row(q, p.wave, p.lane);
+        vx[q] = P::source(r, count, row_bytes, r, p.lane);
+    }
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w), 0, (uint32_t)n_out * row_bytes, 0x00020000);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (int64_t)m0 * n_in, 0, (uint32_t)count * row_bytes,
+                                                      0x00020000);
+    p.run(s_stage, rw, vw, rx, vx, n_in / P::kStage);
+    p.template write<256>(s_stage, [&](int i, int j) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = activation_f32(Bf::round(p.acc[i][j][e]), act, param);
+        return u32x2{Bf::pack2(v[0], v[1]), Bf::pack2(v[2], v[3])};
+    }, [&](int r, int c, u32x4 v) {
+        if (r < count && n0 + c < n_out) *reinterpret_cast<u32x4*>(y + (int64_t)(m0 + r) * n_out + n0 + c) = v;
+    });
+}
+
+template <int XR>
+int launch_dense_activation(const char* fn, const void* x, const void* w, void* y, int64_t rows, int64_t n_out, int64_t n_in, int act,
+                            float param, void* stream) {
+    using P = awq::PingPong<Bf, XR>;
+    const auto kernel = dense_activation_kernel<XR>;
+    static bool raised = false;          // once per process and instantiation
+    if (!raised) {
+        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, P::kLds);
+        if (e != hipSuccess) return fail(NQH_ERR_HIP, fn, "%s", hipGetErrorString(e));
+        raised = true;
+    }
+    const int64_t x_tiles = cdiv(rows, XR), w_tiles = cdiv(n_out, 256);
+    kernel<<<dim3((unsigned)(cdiv(x_tiles * w_tiles, 8) * 8)), dim3(P::kThreads), P::kLds, (hipStream_t)stream>>>(
+        (const uint16_t*)x, (const uint16_t*)w, (uint16_t*)y, (int)rows, (int)n_out, (int)n_in, act, param, (int)x_tiles, (int)w_tiles);
+    return launched(fn);
+}
+
+// Whole stages, 16-byte rows of y, 32-bit offsets into the weight and into a tile's rows of x, a launchable grid.
+bool dense_activation_takes(int64_t rows, int64_t n_out, int64_t n_in) {
+    return rows >= 1 && rows <= kMaxI32 - 256 && n_out >= 8 && n_out % 8 == 0 && n_in >= 64 && n_in % 64 == 0 && n_in <= (1 << 20) &&
+           n_out < (1ll << 31) / n_in && cdiv(rows, 128) * cdiv(n_out, 256) <= kMaxI32 / 512;
+}
+
+// Estimated microseconds with tiles of xr rows: rounds of 256 workgroups, a stage of 1.42 and 0.8 us in a full one and less in one
+// that leaves CUs idle (measured with 100 to 256 tiles of 64 stages), filling and storing a tile.
+double dense_activation_us(int64_t rows, int64_t n_out, int64_t n_in, int xr) {
+    const int64_t tiles = cdiv(rows, xr) * cdiv(n_out, 256), full = tiles / 256;
+    const double steps = (double)(n_in / 64), part = (double)(tiles % 256) / 256, ends = xr == 256 ? 5 : 4;
+    const double stage = xr == 256 ? std::max(0.7, 0.45 + 0.97 * part) : 0.6 + 0.2 * part;
+    return full * (steps * (xr == 256 ? 1.42 : 0.8) + ends) + (part > 0 ? steps * stage + ends : 0);
+}
+
+int dense_activation_tile(int64_t rows, int64_t n_out, int64_t n_in) {
+    return dense_activation_us(rows, n_out, n_in, 128) < dense_activation_us(rows, n_out, n_in, 256) ? 128 : 256;
+}
+
 }  // namespace
 }  // namespace nqh
 
@@ -154,4 +234,36 @@ extern "C" int nqh_skinny_linear(const void* x, const void* weight, const void* 
             (const uint16_t*)x, (const uint16_t*)weight, (const uint16_t*)bias, y, (int)rows, (int)out_features, (int)in_features,
             act, param);
     return launched(fn);
+}
+
+// 1 where the tiles are one round of the 256 CUs and estimated to take less time than the library's product and the activation's pass:
+// 1.3 PFLOP/s and 5 TB/s, 28 us at least, which is what two launches take from python.  relu2, this kernel / those two, us: 1024 ->
+// 4608 features at 65 rows 16 / 24, 1500 rows 20 / 26, 3000 rows 31 / 37; 2048 -> 9216 at 128 rows 25 / 25, 700 rows 30 / 35, 1500
+// rows 49 / 57; 4096 -> 18432 at 128 rows 44 / 34 (left to the library), 384 rows 53 / 60, 700 rows 85 / 96.  Roletar prompts through
+// three layers: 0.6B, 400 tokens 754 -> 699, 1000 tokens 805 -> 749, 3000 tokens 884 -> 830; 1.7B, 700 tokens 787 -> 738.  Several rounds
+// stay with the library: in a pass its products lose less to the writes between the rounds (0.6B, 8192 tokens, 576 tiles: 110 here,
+// 83 + 24 there, though 89 / 103 when repeated alone; 1.7B, 4096 tokens, 576 tiles: the pass 1873 -> 1886).
+extern "C" int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_features) {
+    if (!dense_activation_takes(rows, out_features, in_features)) return 0;
+    const int xr = dense_activation_tile(rows, out_features, in_features);
+    if (cdiv(rows, xr) * cdiv(out_features, 256) > 256) return 0;
+    const double work = (double)rows * (double)out_features;
+    return dense_activation_us(rows, out_features, in_features, xr) <
+           std::max(28.0, 2 * work * (double)in_features / 1.3e9 + 4 * work / 5e6 + 5);
+}
+
+extern "C" int nqh_dense_activation(const void* x, const void* weight, void* y, int64_t rows, int64_t out_features, int64_t in_features,
+                                    int act, float param, void* stream) {
+    const char* fn = "nqh_dense_activation";
+    if (!x || !weight || !y || !aligned(x, 16) || !aligned(weight, 16) || !aligned(y, 16))
+        return fail(NQH_ERR_ARG, fn, "null or misaligned pointer");
+    if (!dense_activation_takes(rows, out_features, in_features))
+        return fail(NQH_ERR_UNSUPPORTED, fn, "needs an in_features that is a multiple of 64, an out_features that is one of 8, and a "
+                                             "weight of less than 2^31 elements");
+    if (act < NQH_ACT_NONE || act > NQH_ACT_SOFTCAP || (act == NQH_ACT_SOFTCAP && !(param > 0.f)))
+        return fail(NQH_ERR_ARG, fn, "unknown activation, or a cap that is not positive");
+    (void)hipGetLastError();
+    return dense_activation_tile(rows, out_features, in_features) == 128
+               ? launch_dense_activation<128>(fn, x, weight, y, rows, out_features, in_features, act, param, stream)
+               : launch_dense_activation<256>(fn, x, weight, y, rows, out_features, in_features, act, param, stream);
 }

@@ -163,6 +163,8 @@ class HybridEngine(EngineCore):
                 param: float = 0.0) -> torch.Tensor:
         if ops.skinny_linear_supported(x.shape[0], w):
             return ops.skinny_linear(x, w, b, activation=activation, param=param)
+        if activation is not None and b is None and ops.dense_activation_wanted(x, w):
+            return ops.dense_activation(x, w, activation, param)
         y = F.linear(x, w, b)
         return y if activation is None else ops.activate_(y, activation, param)
 

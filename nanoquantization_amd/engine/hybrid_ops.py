@@ -632,6 +632,24 @@ def skinny_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
     return y
 
 
+def dense_activation_wanted(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether `dense_activation` takes these and is faster than a library product followed by `activate_`."""
+    return (x.dtype == weight.dtype == torch.bfloat16 and x.is_contiguous() and weight.is_contiguous()
+            and (x.data_ptr() | weight.data_ptr()) % 16 == 0
+            and bool(_lib.hybrid_lib().nqh_dense_activation_wanted(x.shape[0], *weight.shape)))
+
+
+def dense_activation(x: torch.Tensor, weight: torch.Tensor, activation: Optional[str], param: float = 0.0) -> torch.Tensor:
+    """activation(x [rows, in] @ weight [out, in]^T), bf16; the product is rounded to bf16 first."""
+    dev = _dev(x, weight)
+    rows, n = x.shape
+    assert weight.shape[1] == n and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+    y = torch.empty(rows, weight.shape[0], dtype=torch.bfloat16, device=dev)
+    _call(dev, "nqh_dense_activation", x.data_ptr(), weight.data_ptr(), y.data_ptr(), rows, weight.shape[0], n, ACTIVATIONS[activation],
+          param)
+    return y
+
+
 def argmax_rows(logits: torch.Tensor) -> torch.Tensor:
     """Greedy sampler: int64 [rows] index of the largest fp32 logit per row (lowest index among equal maxima)."""
     dev = _dev(logits)

@@ -502,6 +502,20 @@ def test_skinny_linear(rows, n_out, n_in):
     close(ops.skinny_linear(x.cuda(), w.cuda(), b.cuda()), want + b.double(), torch.bfloat16)
 
 
+# one row, both tile heights, rows and columns past their tiles (also fewer than a tile), one stage to many; several rounds of tiles
+@pytest.mark.parametrize("rows,n_out,n_in", [(1, 8, 64), (130, 264, 128), (127, 4608, 192), (257, 8, 320), (256, 512, 1024),
+                                             (2049, 4616, 1024), (4000, 1032, 64)])
+def test_dense_activation(rows, n_out, n_in):
+    print(f"dense activation {rows} x {n_in} -> {n_out}", flush=True)
+    x, w = rand(rows, n_in, seed=1, dtype=torch.bfloat16), rand(n_out, n_in, seed=2, dtype=torch.bfloat16, scale=n_in ** -0.5)
+    want = x.double() @ w.double().T
+    got = ops.dense_activation(x.cuda(), w.cuda(), "relu2").cpu()
+    close(got, want.clamp(min=0) ** 2, torch.bfloat16)
+    y = ops.dense_activation(x.cuda(), w.cuda(), None)
+    close(y, want, torch.bfloat16)
+    assert torch.equal(got, ops.activate_(y, "relu2").cpu())      # of the product rounded to bf16
+
+
 def test_argmax_and_bookkeeping():
     for rows, vocab in ((1, 5), (3, 131), (4, 32000), (2, 4098)):
         x = rand(rows, vocab, seed=vocab)
