@@ -828,8 +828,6 @@ struct GemvExtra<kModeResid> { ResidEpilogue re; };
 
 // STREAM: every wave has at most one chunk (decode-size launches) and takes it step by step as it lands; a form of
 // its own because it needs a dozen registers more than the 128 that let four waves of the other form share a SIMD.
-constexpr int kPrefetchRounds = 2;   // round trips of a prefetch thread
-
 template <typename T, int WK, int MODE = 0, bool STREAM = false>
 __global__ __launch_bounds__(64 * WK) void gemv_dma_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
@@ -863,26 +861,20 @@ __global__ __launch_bounds__(64 * WK) void gemv_dma_kernel(
         tile_of_wg = (int)blockIdx.x < groups ? xcd_aware_group(blockIdx.x, groups) : (int)blockIdx.x;
     }
     if (tile_of_wg >= groups) {
+        if (blockIdx.y != 0 || blockIdx.z != 0) return;   // the extra workgroups exist once per split and row block; one set works
         // Prefetch workgroups (launched beside the compute grid on CUs a small GEMV leaves idle): touch one
         // dword of every 128-byte line of the hinted regions -- the packed weights, scales and zeros of the
-        // NEXT launch -- so that it finds them in the Infinity Cache instead of HBM.  They exist once per split and row
-        // block, and all of them work; a thread makes kPrefetchRounds round trips and leaves the rest of a large region to
-        // the launch that reads it.  (One set in as many rounds as it took held a launch for as long as its successor's
-        // weight: 4096 x 2560 at one row in front of 2560 x 19456, 25 MB, took 34 us
-        // instead of 9 where that weight was in the cache already; a Qwen3-4B decode step of four layers 387 -> 288 us, at 16 rows 454
-        // -> 345; Qwen3-0.6B, all 28 layers, 32 rows: 1.59 ms with one set or all, 1.64 without prefetch.)
+        // NEXT launch -- so that it finds them in the Infinity Cache instead of HBM.
         if (pf.count == 0) return;
-        const long long sets = (long long)gridDim.y * gridDim.z, set = blockIdx.y + (long long)gridDim.y * blockIdx.z;
-        const long long nthreads = (long long)(gridDim.x - groups) * blockDim.x * sets;
-        const long long tid = ((long long)(tile_of_wg - groups) * sets + set) * blockDim.x + threadIdx.x;
+        const long long nthreads = (long long)(gridDim.x - groups) * blockDim.x;
+        const long long tid = (long long)(tile_of_wg - groups) * blockDim.x + threadIdx.x;
         uint32_t sink = 0;
-        int rounds = 0;
         for (int r = 0; r < pf.count; ++r) {
             const long long lines = pf.bytes[r] >> 7;
             // four independent loads in flight per thread and round: issued as assembly and waited for once (as
             // volatile accesses the compiler waits after each of them: four memory round trips in a row, which made
             // the prefetch workgroups the last to finish)
-            for (long long l = tid; l < lines && rounds < kPrefetchRounds; l += 4 * nthreads, ++rounds) {
+            for (long long l = tid; l < lines; l += 4 * nthreads) {
                 uint32_t v[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
