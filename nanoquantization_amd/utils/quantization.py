@@ -59,7 +59,8 @@ def quantize_pack(weight: torch.Tensor, group_size: int, output_dtype: torch.dty
     qscales = torch.empty(K // g, N, dtype=output_dtype, device=dev)
     # The kernel looks for NaN on its way: a pass of its own would read the whole weight twice more.  It writes its finding to
     # pinned memory, which needs neither a launch to clear it nor a copy back (4096 x 12288 78 -> 73 us, 1024 x 2048 33 -> 29).
-    nan = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    # (the device is named: a default device of the caller's would put it elsewhere, where nothing can be pinned)
+    nan = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream()
         _lib.check(_lib.lib().awq_quantize_pack_flagged(weight.data_ptr(), qweight.data_ptr(), qscales.data_ptr(),

@@ -84,3 +84,15 @@ def test_quantize_pack_rejects_bad_input():
         nq.quantize_pack(torch.zeros(8, 128), 128)
     with pytest.raises(AssertionError, match="nan"):
         nq.quantize_pack(torch.full((8, 128), float("nan")).cuda(), 128)
+
+
+def test_quantize_pack_under_a_default_device():
+    """The caller's default device is where torch puts what names none: the word for NaN, in pinned host memory, names its own."""
+    import nanoquantization_amd as nq
+    w = torch.randn(16, 256, generator=torch.Generator().manual_seed(3)).cuda()
+    want = nq.quantize_pack(w, 128, torch.bfloat16)
+    with torch.device("cuda"):
+        got = nq.quantize_pack(w, 128, torch.bfloat16)
+        with pytest.raises(AssertionError, match="nan"):
+            nq.quantize_pack(torch.full((8, 128), float("nan"), device="cuda"), 128)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
