@@ -352,6 +352,9 @@ static void plan_gemm_tile256(int64_t M, int64_t N, int64_t K, int64_t g, int dt
     substitute_regb(M, N, K, g, dtype, variant, *split_k);
 }
 
+// Group sizes the tiles take: a 64-row step of K lies in one group, or holds whole groups of at least 8 rows.
+static bool tiles_take_group(int64_t g) { return g > 0 && (g % 64 == 0 || (64 % g == 0 && g % 8 == 0)); }
+
 static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, const void* qscales,
                          const int32_t* qzeros, const void* bias, void* y, int64_t M, int64_t N,
                          int64_t K, int64_t g, int dtype, void* workspace, size_t workspace_bytes,
@@ -362,7 +365,7 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
     take_prefetch_hint(&dropped);
     int rc = check_linear_args(fn, x, qweight, qscales, qzeros, y, M, N, K, g, dtype);
     if (rc != AWQ_OK) return rc;
-    if (K % kBK != 0 || !(g % 64 == 0 || (64 % g == 0 && g % 8 == 0))) {
+    if (K % kBK != 0 || !tiles_take_group(g)) {
         set_error("%s: needs K %% 64 == 0 and a group size of 8, 16, 32 or a multiple of 64 (K=%lld, g=%lld)",
                   fn, (long long)K, (long long)g);
         return AWQ_ERR_UNSUPPORTED;
@@ -447,7 +450,7 @@ extern "C" int awq_dequantize_transposed(const int32_t* qweight, const void* qsc
     const char* fn = "awq_dequantize_transposed";
     int rc = awq::check_linear_args(fn, out, qweight, qscales, qzeros, out, 1, N, K, group_size, dtype);
     if (rc != AWQ_OK) return rc;
-    if (K % awq::kBK != 0 || !(group_size % 64 == 0 || (64 % group_size == 0 && group_size % 8 == 0)) ||
+    if (K % awq::kBK != 0 || !awq::tiles_take_group(group_size) ||
         N > 0x7fffffff || K > 0x7fffffff) {
         awq::set_error("%s: needs K %% 64 == 0 and a group size of 8, 16, 32 or a multiple of 64 (K=%lld, g=%lld)", fn,
                        (long long)K, (long long)group_size);
@@ -649,7 +652,7 @@ extern "C" const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t
     const Regime regime = linear_regime(M, N, K, group_size);
     if (gated ? M <= 64 && staged : regime == Regime::gemv) return "gemv";
     if (!gated && regime == Regime::gemv_blocks) return "gemv in blocks of 16 rows";
-    if (K % awq::kBK != 0 || !(group_size % 64 == 0 || (64 % group_size == 0 && group_size % 8 == 0))) return "";
+    if (K % awq::kBK != 0 || !awq::tiles_take_group(group_size)) return "";
     if (awq_linear_scratch_bytes(M, N, K, group_size, dtype)) return "dense";
     int variant;
     awq::RowsPlan rows;
@@ -708,8 +711,9 @@ extern "C" size_t awq_linear_parts_wanted(const int64_t* N, int count, int64_t M
     if (!workspace_bytes) workspace_bytes = &none;
     if (!scratch_bytes) scratch_bytes = &none;
     *workspace_bytes = *scratch_bytes = 0;
-    if (!N || count < 2 || count > awq::kMaxParts || M < 17 || K < awq::kBK || K % awq::kBK != 0 || group_size < 1 || K % group_size != 0 ||
-        (dtype != AWQ_F16 && dtype != AWQ_BF16) || (M <= 128 && group_size % 128 == 0))
+    if (!N || count < 2 || count > awq::kMaxParts || M < 17 || K < awq::kBK || K % awq::kBK != 0 ||
+        !awq::tiles_take_group(group_size) || K % group_size != 0 || (dtype != AWQ_F16 && dtype != AWQ_BF16) ||
+        (M <= 128 && group_size % 128 == 0))
         return 0;
     int64_t total = 0;
     double separate = 0;

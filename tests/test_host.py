@@ -405,3 +405,20 @@ def test_linear_routes():
                                 need = L.awq_gemm_ex_workspace_bytes(M, N, K, names.index(name), split)
                                 has = (L.awq_linear_swiglu_workspace_bytes if gated else L.awq_linear_workspace_bytes)(M, N, K)
                                 assert need <= has, (M, K, N, g, d, name, split)
+
+
+def test_linear_parts_take_what_a_linear_takes():
+    """Host-only: several weights in one launch only where each alone would run, by type, rows and group size."""
+    _ensure_built()
+    L = _lib.lib()
+    asked = 0
+    for K in (1536, 3072):
+        for g in (8, 16, 24, 32, 48, 64, 96, 128, 192, 384, 768):
+            for M in (17, 100, 128, 129, 300, 1024, 4096):
+                for d in (_lib.AWQ_F16, _lib.AWQ_BF16):
+                    for N in ((1024, 256, 256), (2048, 2048, 2048)):
+                        alone = all(_route(L, M, K, n, g, d)[0] for n in N)
+                        wanted = L.awq_linear_parts_wanted((ctypes.c_int64 * 3)(*N), 3, M, K, g, d, None, None)
+                        assert alone or not wanted, (M, K, N, g, d)
+                        asked += bool(wanted)
+    assert asked
