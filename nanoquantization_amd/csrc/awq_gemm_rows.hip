@@ -9,7 +9,8 @@
 // seven (five) row tiles.  Up to four row tiles leave registers and LDS for two workgroups on a CU, which fill each other's waits.
 // Stage (64 rows of K): x [16 MT rows][128 B], words [2 halves][32 rows][16], scales and zero words of the two halves; all
 // load-to-LDS in pieces of 1 KiB, 16 bytes a lane, in a ring of kDepth stages.
-// Unpacked values are those of awq_dequantize, bit for bit.
+// Unpacked values are those of awq_dequantize, bit for bit; bf16 scales of 2^113 and more, whose quick way to them overflows, in a
+// second pass of the waves that meet one.
 // What bounds it: the phases, 0.35 us a stage at five rows tiles and 0.45 at eight, of which the matrix instructions take half; no
 // load is waited for (with all of them answered by zeros the time is the same), but asking for them is a fifth of a phase.
 // Measured: 333 x 2816 x 9720 in fp16, groups of 64, 29.8 -> 27.1 us against four waves that each unpack beside their own matrix
@@ -96,10 +97,20 @@ struct Columns<BF16> {
         float q0[4], q1[4];
         embed(w0, q0);
         embed(w1, q1);
-        // 2^15 + z has 16 bits and the scale 8: the product kept in nzs is exact, and so is the sum, (q - z) * s
+        // 2^15 + z has 16 bits and the scale 8: the product kept in nzs is exact, and so is the sum, (q - z) * s; unless it leaves the
+        // range of a float, and no weight of the column is a number
 #pragma unroll
         for (int f = 0; f < 4; ++f)
             out[f] = BF16::pack2(__builtin_fmaf(q0[f], sc[f], nzs[f]), __builtin_fmaf(q1[f], sc[f], nzs[f]));
+    }
+    // The same for any scale.
+    __device__ __forceinline__ void pair_exact(uint32_t w0, uint32_t w1, uint32_t zw, uint32_t (&out)[4]) const {
+        float q0[4], q1[4], z[4];
+        embed(w0, q0);
+        embed(w1, q1);
+        embed(zw, z);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) out[f] = BF16::pack2((q0[f] - z[f]) * sc[f], (q1[f] - z[f]) * sc[f]);
     }
 };
 
@@ -248,6 +259,8 @@ __device__ __forceinline__ void rows_tile(
         u32x4 a[MT], b[4];
         if (!kEarly) read_words(at);
         read_rows(at, a);
+        // (without this the compiler mixes the group's constants into the unpacking: 64 rows of 16384 columns, K of 4096, 35 -> 37 us)
+        if (!kEarly && T::id == AWQ_BF16) __builtin_amdgcn_sched_barrier(0);
         cols.set_group(zw, sv);
 #pragma unroll
         for (int rp = 0; rp < 4; ++rp) {
@@ -285,6 +298,45 @@ __device__ __forceinline__ void rows_tile(
     }
     if ((n & 1) == turn) __builtin_amdgcn_s_barrier();      // the turn that had one phase fewer
     __builtin_amdgcn_s_waitcnt(0x0F70);                     // what was asked for past the end has come: the LDS is free
+
+    if constexpr (T::id == AWQ_BF16) {
+        // A weight that was no number has made all rows of its column none, whatever x holds: this wave's part of the tile once more,
+        // straight from memory.  (A branch among the unpacking that looks at the scales costs a third of the whole kernel's time.)
+        bool off = false;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) off |= !(__builtin_fabsf(acc[0][f][0]) <= 3.402823466e38f);
+        if (__builtin_amdgcn_ballot_w64(off)) {
+            int row = j, part_k = 8 * kb;       // (hidden from the compiler, which would keep what the two passes share through the first)
+            asm volatile("" : "+v"(row), "+v"(part_k));
+            const int word = word0 + row;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int f = 0; f < 4; ++f) acc[mt][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int t = turn; t < n; t += 2) {
+                const int k = k0 + 64 * t + 32 * kh;
+                const size_t at_group = (size_t)(k / g) * words + word;
+                const uint32_t zero = qzeros[at_group];
+                cols.set_group(zero, *reinterpret_cast<const u32x4*>(scales + 8 * at_group));
+                u32x4 b[4];
+#pragma unroll
+                for (int rp = 0; rp < 4; ++rp) {
+                    const uint32_t* p = qweight + (size_t)(k + part_k + 2 * rp) * words + word;
+                    uint32_t v[4];
+                    cols.pair_exact(p[0], p[words], zero, v);
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) b[f][rp] = v[f];
+                }
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const u32x4 a = *reinterpret_cast<const u32x4*>(x + (size_t)min(m0 + 16 * mt + row, M - 1) * K + k + part_k);
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) acc[mt][f] = T::mfma16(a, b[f], acc[mt][f]);
+                }
+            }
+        }
+    }
 
     // The four parts of K meet, (0 + 1) + (2 + 3), and every wave ends with a quarter of the row tiles: the two of a turn give each
     // other every second tile, then the turns every second of those, in the layout of the registers; the sums go to an fp32 tile

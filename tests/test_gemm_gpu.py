@@ -460,6 +460,36 @@ def test_gemm_rows128_few_rows(dtype, M, K, N, g, split):
         assert torch.equal(nq.awq_gemm(xd, *dev, 8), awq_gemm_variant(xd, *dev, v, chosen.value))
 
 
+# scales up to the largest for which 15 times one is a number; the quick way to a weight leaves the range of a float from 2^113 on
+@pytest.mark.parametrize("M,K,N,g,split", [(40, 704, 264, 32, 1), (128, 1088, 128, 64, 3), (200, 576, 392, 64, 1)])
+def test_gemm_rows128_large_scales(M, K, N, g, split):
+    print(f"gemm rows128 large scales M={M} K={K} N={N} g={g} split={split}", flush=True)
+    L = _lib.lib()
+    v = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())].index("rows128")
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    words = lambda r: torch.randint(-2 ** 31, 2 ** 31 - 1, (r, N // 8), dtype=torch.int32, device="cuda", generator=gen)
+    qw, qz = words(K), words(K // g)
+    # every 37th column in the middle group alone, at 2^112, 2^113, .. 2^123
+    qs = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 + 0.001).to(torch.bfloat16)
+    for i, c in enumerate(range(3, N, 37)):
+        qs[K // g // 2, c] = 2.0 ** (112 + i % 12) * (1 + i % 2 / 2)
+    w = nq.awq_dequantize(qw, qs, qz)
+    assert w.isfinite().all()
+    eye = torch.eye(min(M, K), K, device="cuda", dtype=torch.bfloat16)
+    eye = torch.roll(eye, K // g // 2 * g, dims=1)           # rows of the group with the large scales
+    assert torch.equal(awq_gemm_variant(eye, qw, qs, qz, v, split), torch.roll(w, -(K // g // 2 * g), dims=0)[:min(M, K)])
+    x = (torch.randn(M, K, device="cuda", generator=gen) * 2.0 ** -20).to(torch.bfloat16)
+    y = awq_gemm_variant(x, qw, qs, qz, v, split)
+    ref = x.double() @ w.double()
+    bound = TIGHT["bf16"] * ref.abs().amax(dim=0)            # a column at a time
+    assert y.isfinite().all() and ((y.double() - ref).abs() <= bound).all()
+    # a scale that is no number concerns its own column
+    qs[0, 1] = float("inf")
+    z = awq_gemm_variant(x, qw, qs, qz, v, split)
+    other = [c for c in range(N) if c != 1]
+    assert not z[:, 1].isfinite().any() and torch.equal(z[:, other], y[:, other])
+
+
 # tiles of few rows unsplit and in K splits, dequantised first with tiles of 128 and of 256 rows; widths that are no whole tiles, a K
 # and rows that the one launch does not take
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
