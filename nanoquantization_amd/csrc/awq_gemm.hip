@@ -414,13 +414,6 @@ static int gemm_dispatch(const char* fn, const void* x, const int32_t* qweight, 
         AWQ_GEMM_CASE(k64x256, 64, 256, 1, 4)
         AWQ_GEMM_CASE(k32x256, 32, 256, 1, 4)
         case kRowsVariant:
-            if (N < 128) {     // less than a tile's columns: the plain tiles, which take any width
-                e = dtype == AWQ_F16 ? launch_gemm<F16, 128, 128, 2, 2>(x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K,
-                                                                        (int)g, workspace, rows.splits, s)
-                                     : launch_gemm<BF16, 128, 128, 2, 2>(x, qweight, qscales, qzeros, bias, y, (int)M, (int)N, (int)K,
-                                                                         (int)g, workspace, rows.splits, s);
-                break;
-            }
             e = launch_rows(rows, dtype, x, Parts({qweight, qscales, qzeros}, y, N), bias, (int)M, (int)K, (int)g, workspace, act != 0, s);
             break;
         case kPipeVariant:

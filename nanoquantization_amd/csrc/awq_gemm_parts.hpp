@@ -281,10 +281,11 @@ size_t dense_parts_scratch_bytes(const int64_t* N, int count, int64_t M, int64_t
 // awq_gemm_dense.hip: estimated microseconds of awq_linear_dense, -1 where it does not take the sizes.
 double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g);
 
-// awq_gemm_rows.hip: tiles of 80..128 rows by 128 columns for a few hundred rows; `us` an estimate of the time, m_tiles 0 where
+// awq_gemm_rows.hip: tiles of 32..128 rows by 128 columns for 17 to about 1000 rows; `us` an estimate of the time, m_tiles 0 where
 // it does not take the sizes.  split_k 0: the split with the least estimate, which depends on the type.
 struct RowsPlan {
     int m_tiles, n_tiles, mt, splits, steps_per_split;   // mt: 16-row tiles of a workgroup; steps: of 64 rows of K
+    bool four;                                            // the four waves of awq_gemm_rows4.hip
     double us;
 };
 RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, int split_k = 0);
@@ -293,5 +294,8 @@ inline size_t rows_ws_bytes(const RowsPlan& p, int64_t M, int64_t N) {
 }
 hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const Parts& parts, const void* bias, int M, int K, int g,
                        void* workspace, bool gated, hipStream_t st);   // the plan of all columns; gated: as PipePlan::act, one part
+// awq_gemm_rows4.hip: the product of launch_rows where the plan says `four`, without the sum of the K splits.
+hipError_t launch_rows4(const RowsPlan& p, int dtype, const void* x, const Parts& parts, const void* bias, float* partials, int M,
+                        int K, int g, bool gated, hipStream_t st);
 
 }  // namespace awq

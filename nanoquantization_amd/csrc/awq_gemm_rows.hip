@@ -458,19 +458,26 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, i
         return p;
     const int64_t m_tiles = cdiv(M, 128), n_tiles = cdiv(N, 128), steps = K / 64;
     p.m_tiles = (int)m_tiles, p.n_tiles = (int)n_tiles;
-    p.mt = (int)std::max<int64_t>(2, cdiv(cdiv(M, m_tiles), 16));
-    // Microseconds, by type and MT: of a stage with a CU to itself and with two workgroups on it, and of filling the ring,
-    // the tile's sums and the launch; a K split writes its fp32 sums and reads them again in a second launch.
-    constexpr double kAlone[2][7] = {{0.28, 0.295, 0.38, 0.345, 0.35, 0.37, 0.41}, {0.345, 0.37, 0.445, 0.405, 0.42, 0.45, 0.47}};   // [fp16, bf16][MT - 2]
+    const bool narrow = N < 128;      // less than a tile's columns: the four waves alone take that
+    p.mt = (int)std::max<int64_t>(narrow ? 5 : 2, cdiv(cdiv(M, m_tiles), 16));
+    // From 65 rows on the four waves are the faster ones up to 18 stages a split in fp16 and 14 in bf16: their end takes 1.2 to 1.5 us
+    // less, a stage 0.1 more.  Against the eight, by stages: fp16 0.83 of the time with 2, 0.91 with 8, 0.97 with 16, 0.99 to 1.02
+    // with 20, 1.02 with 24; bf16 0.87, 0.94, 1.01 with 16, 1.02 with 20.
+    const int few = dtype == AWQ_F16 ? 18 : 14, t = dtype == AWQ_F16 ? 0 : 1;
+    // Microseconds, by type and MT: a stage of the four waves; of the eight with a CU to itself and with two workgroups on it; and of
+    // filling the ring, the tile's sums and the launch.  A K split writes its fp32 sums and reads them again in a second launch.
+    constexpr double kFour[2][4] = {{0.47, 0.435, 0.5, 0.545}, {0.56, 0.55, 0.585, 0.605}};     // [fp16, bf16][MT - 5]
+    constexpr double kAlone[2][7] = {{0.28, 0.295, 0.38, 0.345, 0.35, 0.37, 0.41}, {0.345, 0.37, 0.445, 0.405, 0.42, 0.45, 0.47}};   // [MT - 2]
     constexpr double kShared[2][3] = {{0.455, 0.45, 0.495}, {0.52, 0.53, 0.575}};
-    const int t = dtype == AWQ_F16 ? 0 : 1;
     const int64_t slots = 256 * per_cu(p.mt);
+    const auto four = [&](int64_t s) { return narrow || (p.mt >= 5 && cdiv(steps, s) <= few); };
     const auto us = [&](int64_t s) {
         const int64_t items = m_tiles * n_tiles * s, last = items % slots, n = cdiv(steps, s);
+        const double sums = s > 1 ? 2.5 + (double)s * (double)(M * N) * 8 / 5.0e6 : 0;
+        if (four(s)) return (double)cdiv(items, 256) * (kFour[t][p.mt - 5] * (double)n + 4.7 + 0.2 * p.mt) + sums;
         const double fixed = 4.6 + 0.95 * p.mt, alone = kAlone[t][p.mt - 2] * (double)n + fixed;
         const double whole = p.mt <= 4 ? kShared[t][p.mt - 2] * (double)n + fixed : alone;
-        return (double)(items / slots) * whole + (last == 0 ? 0 : last > 256 ? whole : alone) +
-               (s > 1 ? 2.5 + (double)s * (double)(M * N) * 8 / 5.0e6 : 0);
+        return (double)(items / slots) * whole + (last == 0 ? 0 : last > 256 ? whole : alone) + sums;
     };
     int64_t best = 1;
     for (int64_t s = 2; s <= 16 && s * 4 <= steps; ++s)
@@ -478,6 +485,7 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, i
     if (split_k > 0) best = std::min<int64_t>(split_k, steps);
     p.steps_per_split = (int)cdiv(steps, best);
     p.splits = (int)cdiv(steps, p.steps_per_split);
+    p.four = four(p.splits);
     p.us = us(p.splits);
     return p;
 }
@@ -488,7 +496,9 @@ hipError_t launch_rows(const RowsPlan& p, int dtype, const void* x, const Parts&
 #define AWQ_ROWS(T, MT) \
     if (p.mt == MT) e = launch<T, MT>(p, x, parts, bias, partials, M, K, g, gated, st);
     hipError_t e = hipErrorInvalidValue;
-    if (dtype == AWQ_F16) {
+    if (p.four) {
+        e = launch_rows4(p, dtype, x, parts, bias, partials, M, K, g, gated, st);
+    } else if (dtype == AWQ_F16) {
         AWQ_ROWS(F16, 2) AWQ_ROWS(F16, 3) AWQ_ROWS(F16, 4)
         AWQ_ROWS(F16, 5) AWQ_ROWS(F16, 6) AWQ_ROWS(F16, 7) AWQ_ROWS(F16, 8)
     } else {

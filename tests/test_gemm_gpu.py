@@ -406,10 +406,13 @@ def test_linear_random_shapes_default_dispatch():
 
 
 # a row, tiles of five to eight 16-row blocks, one row past a tile; less and more stages of K than the ring holds, also cut in
-# three; columns past the last tile; groups of less, as much and more than a stage
+# three; columns past the last tile; groups of less, as much and more than a stage; from the third line on both sides of the stages
+# where four waves hand over to eight (14 and 15 in bf16, 18 and 19 in fp16), and more, odd and even
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("M,K,N,g", [(1, 64, 8, 32), (81, 320, 136, 64), (113, 384, 520, 128), (128, 448, 256, 32), (129, 512, 8, 512),
-                                      (270, 192, 264, 192), (333, 1088, 1032, 64)])
+                                      (270, 192, 264, 192), (333, 1088, 1032, 64),
+                                      (1, 1280, 128, 64), (80, 896, 136, 32), (81, 960, 256, 64), (112, 1152, 264, 128), (113, 1216, 392, 64),
+                                      (128, 1344, 256, 32), (257, 3712, 136, 64), (66, 4096, 1032, 128), (96, 4160, 120, 64)])
 def test_gemm_rows128(dtype, M, K, N, g):
     print(f"gemm rows128 {dtype} M={M} K={K} N={N} g={g}", flush=True)
     L = _lib.lib()
