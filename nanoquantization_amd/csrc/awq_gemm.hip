@@ -505,56 +505,59 @@ extern "C" int awq_gemm(const void* x, const int32_t* qweight, const void* qscal
                               dtype, workspace, workspace_bytes, stream, v, s);
 }
 
-// Microseconds of the fused 256 x 256 kernels: 1.9 a K step and round of 256 workgroups, 10 to fill and store a round's tiles,
-// and 0.05 per K slice of a tile for its fp32 partials and their sum: 0.9 to 1.25 times the measured times of 129 to 8192 rows, up
-// to 1.3 where a launch leaves CUs idle (as is the estimate of awq_linear_dense).  In fp16 the register-operand kernel takes a tenth less
-// than that with whole tiles, or with several items a workgroup (640 x 4096 x 24576 139 us, estimated 170 without, 161
-// dequantised first).  What the routes lose to the fastest way over 980 timed calls: 0.3 % on average.
+// Microseconds of the fused 256 x 256 kernels: 1.88 a K step in a full round of 256 workgroups, 1 to 1.82 in one that leaves CUs idle,
+// 9.7 to fill and store a round's tiles; 3 and the time of the fp32 partials at 10.2 TB/s (they stay in the caches) where tiles are cut.
+// The workgroups of the register-operand kernel go through one run of steps each, at 1.82 in fp16 (1.7 with one whole tile each: 900 x
+// 2048 x 16384 60 us) and 1.95 in bf16, and less where a tile's rows are not there.  0.9 to 1.08 times the measured times of 43
+// weights by 130 to 2048 rows, in both types, in 96 of 100; that is what holds the routes: they lose 0.4 % to the fastest way on
+// average, more than 4 % in one of 40.
 static double fused_linear_us(int64_t M, int64_t N, int64_t K, int64_t g, int dtype) {
     int v, split;
     awq::plan_gemm(M, N, K, g, dtype, &v, &split);
     const awq::PipePlan p = awq::make_pipe_plan(M, N, K, split, awq::is_tail_variant(v));
     const int64_t slices = (int64_t)p.tail_tiles * p.splits;
-    const double full = (double)awq::cdiv(p.full_tiles, 256), cut = (double)awq::cdiv(slices, 256);
-    const double us = full * (1.9 * (double)(K / 64) + 10) + cut * (1.9 * p.iters_per_split + 10) + 0.05 * (double)slices;
-    const bool regb = v == awq::kRegbVariant || v == awq::kRegbTailVariant;
-    return regb && dtype == AWQ_F16 && (slices == 0 || p.full_tiles + slices > 256) ? 0.9 * us : us;
+    const double cut = (double)p.tail_tiles / (p.full_tiles + p.tail_tiles);
+    const double sums = slices ? 3 + p.splits * cut * (double)(M * N) * 8 / 10.2e6 : 0;
+    double step = 1.88;
+    if (v == awq::kRegbVariant || v == awq::kRegbTailVariant) {
+        const double there = (double)M / (double)(256 * awq::cdiv(M, 256));
+        step = (dtype == AWQ_BF16 ? 1.95 : (p.full_tiles == 256 && slices == 0 ? 1.7 : 1.82)) * (0.6 + 0.4 * there);
+        if (p.full_tiles + slices > 256)
+            return 14 + step * (double)(p.full_tiles * (K / 64) + slices * p.iters_per_split) / 256 + sums;
+    }
+    const auto rounds = [&](int64_t items, int64_t steps) {
+        const double part = (double)(items % 256) / 256;
+        return (double)(items / 256) * (step * (double)steps + 9.7) + (part > 0 ? (1 + 0.82 * part) * (double)steps + 9.7 : 0);
+    };
+    return rounds(p.full_tiles, K / 64) + rounds(slices, p.iters_per_split) + sums;
 }
 
-// Short K on wide weights at 1024 to 2048 rows stays fused, although dequantising first would often be faster (1024 x 4096 at
-// 1024 rows 31 / 22 us): callers get awq_gemm_plan's kernel and K split there, bit for bit.  Fewer rows and narrower weights go by
-// the estimates (1024 x 1024 at 130 to 1500 rows 20-27 -> 13-17 us, 1024 x 6144 at 512 rows 33 -> 17).
-static bool always_fused(int64_t M, int64_t N, int64_t K) { return M <= 128 || (M >= 1024 && M <= 2048 && K < 2048 && N >= 4096); }
-
-// Whether the tiles of awq_gemm_rows.hip run.  17 to 128 rows: wherever they take the sizes and the GEMV does not (5120 x 25600 in
-// groups of 64 at 64 rows, bf16, 46 -> 41 us against the plain tiles, 5120 x 17408 44 -> 31, at 32 rows 29 -> 26, 15296 x 4680
-// at 18 rows 33 -> 23; 5120 x 25600 at 100 rows 69 -> 47, 25600 x 5120 at 80 rows 61 -> 42, 12288 x 4096 at 128 rows 34 -> 30).
-// From 129 rows where the estimates of all three ways say so, in one round of the CUs only; fp16 / bf16 and the faster of the
-// other two: 2816 x 9720 at 333 rows 30 / 30 us against 46, 4096 x 4096 at 200 rows 25 / 25 against 29, at 512 rows 33 / 35 against
-// 43, 12288 x 4096 at 160 rows 32 / 34 against 45, 2048 x 6144 at 640 rows 25 / 27 against 34.  Up to 192 rows of weights of 50 Mi
-// elements stay on the 256-row tile that holds them all, as callers know it (5120 x 10240 at 192 rows 46 us, here 45; 17408 x
-// 5120 at 129 rows 60 and 52).
+// Whether the tiles of awq_gemm_rows.hip run.  17 to 128 rows: wherever they take the sizes and the GEMV does not, from a whole tile's
+// columns on (5120 x 25600 in groups of 64 at 64 rows, bf16, 46 -> 41 us against the plain tiles, 5120 x 17408 44 -> 31, at 32 rows
+// 29 -> 26, 15296 x 4680 at 18 rows 33 -> 23; 5120 x 25600 at 100 rows 69 -> 47, 25600 x 5120 at 80 rows 61 -> 42; gated, against
+// the 256 x 256 tiles, 65 and 128 rows: 2048 x 12288 32 -> 20 and 24, 5120 x 34816 128 -> 75 and 95, in bf16 125 -> 85 and 101).
+// From 129 rows where the estimates of all three ways say so; fp16 / bf16 and the faster of the other two: 2816 x 9720 at 333 rows
+// 27 / 30 us against 46, 17408 x 5120 at 130 rows 48 / 52 against 63, 4096 x 4096 at 512 rows 33 / 35 against 43, 1024 x 4096 at 1024
+// rows 17 / 18 against 22, 5120 x 17408 at 300 rows (two rounds of the CUs) 81 / 92 against 102, 2048 x 6144 at 640 rows 25 / 27 against 34.
 static bool rows_wanted(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, awq::RowsPlan* plan) {
-    if (M <= 16 || N < 128) return false;
-    if (M <= 128) return (*plan = awq::make_rows_plan(M, N, K, g, dtype)).m_tiles != 0;
-    if (always_fused(M, N, K) || (M <= 192 && K * N >= (50ll << 20))) return false;
+    if (M <= 16 || (M <= 128 && N < 128)) return false;
     *plan = awq::make_rows_plan(M, N, K, g, dtype);
-    if (plan->m_tiles == 0 || (int64_t)plan->m_tiles * plan->n_tiles * plan->splits > 256 ||
-        plan->us >= 0.95 * fused_linear_us(M, N, K, g, dtype))
-        return false;
+    if (plan->m_tiles == 0 || M <= 128) return plan->m_tiles != 0;
+    if (plan->us >= fused_linear_us(M, N, K, g, dtype)) return false;
     const double dense = awq::dense_linear_us(M, N, K, g);
-    return dense < 0 || plan->us < 0.95 * dense;
+    return dense < 0 || plan->us < dense;
 }
 
-// Workspace of those tiles where they are wanted, for either type and any group size: the size decides whether they run and not
-// the split, and they run at a group size of 32 wherever they do at another (fused_linear_us is the largest there).
+// Workspace of those tiles where they are wanted, for either type and any group size: of that the estimates see only whether it is a
+// multiple of 64.
 static size_t rows_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     size_t most = 0;
-    for (const int dtype : {AWQ_F16, AWQ_BF16}) {
-        awq::RowsPlan rows;
-        const size_t b = rows_wanted(M, N, K, 32, dtype, &rows) ? awq::rows_ws_bytes(rows, M, N) : 0;
-        most = most > b ? most : b;
-    }
+    for (const int dtype : {AWQ_F16, AWQ_BF16})
+        for (const int64_t g : {32, 64}) {
+            awq::RowsPlan rows;
+            const size_t b = rows_wanted(M, N, K, g, dtype, &rows) ? awq::rows_ws_bytes(rows, M, N) : 0;
+            most = most > b ? most : b;
+        }
     return most;
 }
 
@@ -580,7 +583,7 @@ extern "C" size_t awq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 // 4096 at 512 rows (32 tiles cut in eight) 69 / 136, 2048 rows 202 / 174 (193 / 181), 8192 rows 751 / 556 (709 / 580); 2560 x
 // 9728 at 300 rows 44 / 43, 8192 rows 388 / 292 (370 / 312).
 extern "C" size_t awq_linear_scratch_bytes(int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype) {
-    if (always_fused(M, N, K) || (dtype != AWQ_F16 && dtype != AWQ_BF16)) return 0;
+    if (M <= 128 || (dtype != AWQ_F16 && dtype != AWQ_BF16)) return 0;
     const double dense = awq::dense_linear_us(M, N, K, group_size);
     if (dense < 0) return 0;
     awq::RowsPlan rows;
@@ -614,10 +617,8 @@ extern "C" int awq_linear_swiglu(const void* x, const int32_t* qweight, const vo
     int v = awq::kPipeVariant, s = 1;
     if (K >= awq::kBK && N >= 16 && M >= 1 && group_size > 0)
         awq::plan_gemm_tile256(M, N, K, group_size, dtype, &v, &s);
-    // as awq_linear on the same sizes, whose bits the gated product has; 65 to 128 rows of the sizes that the GEMV takes up to 64 rows
-    // keep the 256-row tiles, whose bits callers compare with
     awq::RowsPlan rows;
-    if (M > (staged ? 128 : 16) && N >= 128 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
+    if (M > 16 && N >= 16 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
         v = awq::kRowsVariant, s = rows.splits;
     return awq::gemm_dispatch("awq_linear_swiglu", x, qweight, qscales, qzeros, nullptr, y, M, N, K, group_size,
                               dtype, workspace, workspace_bytes, stream, v, s, 1);
@@ -649,7 +650,7 @@ extern "C" const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t
     if (awq_linear_scratch_bytes(M, N, K, group_size, dtype)) return "dense";
     int variant;
     awq::RowsPlan rows;
-    if (!(gated && staged && M <= 128) && rows_wanted(M, N, K, group_size, dtype, &rows))
+    if (rows_wanted(M, N, K, group_size, dtype, &rows))
         // (up to 128 rows the tile's name is 128x128, whichever kernel awq_gemm runs on it)
         variant = M > 64 && M <= 128 && !gated ? awq::k128x128 : awq::kRowsVariant, *split_k = rows.splits;
     else if (gated) awq::plan_gemm_tile256(M, N, K, group_size, dtype, &variant, split_k);
@@ -677,7 +678,7 @@ extern "C" int awq_linear(const void* x, const int32_t* qweight, const void* qsc
         return AWQ_OK;
     }
     awq::RowsPlan rows;
-    if (M > 16 && N >= 128 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
+    if (M > 16 && N >= 8 && K >= awq::kBK && group_size > 0 && rows_wanted(M, N, K, group_size, dtype, &rows))
         return awq::gemm_dispatch("awq_linear", x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,
                                   workspace_bytes, stream, awq::kRowsVariant, rows.splits);
     return awq_gemm(x, qweight, qscales, qzeros, bias, y, M, N, K, group_size, dtype, workspace,

@@ -108,6 +108,18 @@ double product_us(int64_t M, int64_t slab, int64_t K, int xr) {
     return (double)cdiv(cdiv(M, xr) * cdiv(slab, 256), 256) * ((double)(K / 64) * (xr == 256 ? 1.42 : 0.8) + (xr == 256 ? 5 : 4));
 }
 
+int product_tile(int64_t M, int64_t slab, int64_t K) { return product_us(M, slab, K, 128) < product_us(M, slab, K, 256) ? 128 : 256; }
+
+// The same for the comparison with other ways, fitted to the times of 43 weights by 130 to 2048 rows (within 10 % in 94 of 100; the
+// terms have to be taken together): rounds with their ends, the last of which has shorter stages where it leaves CUs idle.
+double rounds_us(int64_t M, int64_t slab, int64_t K) {
+    const int xr = product_tile(M, slab, K);
+    const int64_t tiles = cdiv(M, xr) * cdiv(slab, 256), full = tiles / 256;
+    const double steps = (double)(K / 64), part = (double)(tiles % 256) / 256, ends = xr == 256 ? 0 : 1.6;
+    const double stage = xr == 256 ? 0.62 + 0.6 * part : 0.57 + 0.1 * part;
+    return (double)full * (steps * (xr == 256 ? 1.25 : 0.76) + ends) + (part > 0 ? steps * stage + ends : 0);
+}
+
 template <typename T, int XR, bool GATED>
 hipError_t launch(const void* x, const void* wt, const void* bias, const Outputs& out, int M, int cols, int K, hipStream_t st) {
     using P = PingPong<T, XR>;
@@ -145,11 +157,10 @@ bool takes(int64_t M, int64_t N, int64_t K, int64_t g) {
 double dense_linear_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     if (!takes(M, N, K, g)) return -1;
     const int64_t slab = slab_columns(N, K);
-    // the dequantise pass moves 2.5 bytes a weight at 6 TB/s (4096 x 12288 20.5 us, 5120 x 25600 62)
-    // and a slab that the 256 MB cache does not hold is read from memory (5120 x 25600, 262 MB: 640 rows 242 us, 1500 rows 446)
-    const double cold = slab * K * 2 > (192ll << 20) ? 2.0 * (double)(K * N) / 6.0e6 : 0;
-    return 4 + 2.5 * (double)(K * N) / 6.0e6 + cold +
-           (double)cdiv(N, slab) * std::min(product_us(M, slab, K, 128), product_us(M, slab, K, 256));
+    // the dequantise pass moves 2.5 bytes a weight at 6.4 TB/s (4096 x 12288 20.5 us, 5120 x 25600 62); a slab that the 256 MB cache
+    // does not hold is read from memory (5120 x 25600, 262 MB: 640 rows 242 us, 1500 rows 446); the result is written at 2.7 TB/s
+    const double cold = slab * K * 2 > (192ll << 20) ? 2.3 * (double)(K * N) / 6.0e6 : 0;
+    return 6.9 + 2.5 * (double)(K * N) / 6.4e6 + cold + (double)cdiv(N, slab) * rounds_us(M, slab, K) + (double)(M * N) * 2 / 2.7e6;
 }
 
 size_t dense_parts_scratch_bytes(const int64_t* N, int count, int64_t M, int64_t K, int64_t g) {
@@ -169,7 +180,7 @@ int dense_parts(const char* fn, const void* x, const Parts& parts, int64_t M, in
         set_error("%s: 16-byte aligned scratch of %zu bytes needed, %zu given", fn, need, scratch ? scratch_bytes : (size_t)0);
         return AWQ_ERR_WORKSPACE;
     }
-    const int xr = product_us(M, parts.total, K, 128) < product_us(M, parts.total, K, 256) ? 128 : 256;
+    const int xr = product_tile(M, parts.total, K);
     hipError_t e = launch_dequant_transpose_parts(dtype, parts, scratch, (int)K, (int)g, st);
     if (e == hipSuccess)
         e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, nullptr, Outputs(parts), (int)M, parts.total, (int)K, xr, false, st)
@@ -206,7 +217,7 @@ static int dense_entry(const char* fn, const void* x, const PackedWeight& w, con
     }
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const int64_t slab = slab_columns(cols_in_all, K);
-    const int xr = product_us(M, slab, K, 128) < product_us(M, slab, K, 256) ? 128 : 256;
+    const int xr = product_tile(M, slab, K);
     for (int64_t n = 0; n < cols_in_all; n += slab) {
         const int64_t cols = std::min(slab, cols_in_all - n), each = second ? 2 : 1;
         hipError_t e = launch_dequant_transpose(dtype, w, second, scratch, (int)N, (int)K, (int)g, st, n / each, cols / each);

@@ -466,21 +466,29 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, i
     const int few = dtype == AWQ_F16 ? 18 : 14, t = dtype == AWQ_F16 ? 0 : 1;
     // Microseconds, by type and MT: a stage of the four waves; of the eight with a CU to itself and with two workgroups on it; and of
     // filling the ring, the tile's sums and the launch.  A K split writes its fp32 sums and reads them again in a second launch.
-    constexpr double kFour[2][4] = {{0.47, 0.435, 0.5, 0.545}, {0.56, 0.55, 0.585, 0.605}};     // [fp16, bf16][MT - 5]
-    constexpr double kAlone[2][7] = {{0.28, 0.295, 0.38, 0.345, 0.35, 0.37, 0.41}, {0.345, 0.37, 0.445, 0.405, 0.42, 0.45, 0.47}};   // [MT - 2]
+    // From five row tiles on within 10 % of 96 of 100 measured times (43 weights, 130 to 2048 rows, every split).
+    constexpr double kFour[2][4] = {{0.45, 0.445, 0.485, 0.515}, {0.56, 0.56, 0.595, 0.59}};     // [fp16, bf16][MT - 5]
+    constexpr double kAlone[2][7] = {{0.28, 0.295, 0.38, 0.375, 0.38, 0.405, 0.46}, {0.345, 0.37, 0.445, 0.44, 0.465, 0.485, 0.515}};   // [MT - 2]
     constexpr double kShared[2][3] = {{0.455, 0.45, 0.495}, {0.52, 0.53, 0.575}};
-    const int64_t slots = 256 * per_cu(p.mt);
     const auto four = [&](int64_t s) { return narrow || (p.mt >= 5 && cdiv(steps, s) <= few); };
     const auto us = [&](int64_t s) {
-        const int64_t items = m_tiles * n_tiles * s, last = items % slots, n = cdiv(steps, s);
-        const double sums = s > 1 ? 2.5 + (double)s * (double)(M * N) * 8 / 5.0e6 : 0;
-        if (four(s)) return (double)cdiv(items, 256) * (kFour[t][p.mt - 5] * (double)n + 4.7 + 0.2 * p.mt) + sums;
-        const double fixed = 4.6 + 0.95 * p.mt, alone = kAlone[t][p.mt - 2] * (double)n + fixed;
-        const double whole = p.mt <= 4 ? kShared[t][p.mt - 2] * (double)n + fixed : alone;
-        return (double)(items / slots) * whole + (last == 0 ? 0 : last > 256 ? whole : alone) + sums;
+        const int64_t items = m_tiles * n_tiles * s, n = cdiv(steps, s);
+        const double moved = (double)s * (double)(M * N) * 8;
+        if (p.mt <= 4) {
+            const int64_t last = items % 512;
+            const double fixed = 4.6 + 0.95 * p.mt, alone = kAlone[t][p.mt - 2] * (double)n + fixed;
+            const double whole = kShared[t][p.mt - 2] * (double)n + fixed;
+            return (double)(items / 512) * whole + (last == 0 ? 0 : last > 256 ? whole : alone) + (s > 1 ? 2.5 + moved / 5.0e6 : 0);
+        }
+        const double round = four(s) ? kFour[t][p.mt - 5] * (double)n + 4.1 + 0.31 * p.mt : kAlone[t][p.mt - 2] * (double)n + 5.5 + 0.26 * p.mt;
+        // (full rounds take longer once a launch lasts: 512 x 4096 x 24576, three of them, 128 us in fp16 where this alone says 111)
+        const double rounds = (double)cdiv(items, 256), all = rounds * round, full = (double)items / (256 * rounds);
+        const double held = full > 0.9 ? (t == 0 ? 0.17 : 0.07) * std::max(0.0, all - 24) : 0;
+        return all + held + (s > 1 ? 2 + moved / 3.6e6 : 0);
     };
     int64_t best = 1;
-    for (int64_t s = 2; s <= 16 && s * 4 <= steps; ++s)
+    // (splits of more than a round of the CUs were not timed from five row tiles on)
+    for (int64_t s = 2; s <= 16 && s * 4 <= steps && (p.mt <= 4 || m_tiles * n_tiles * s <= 256); ++s)
         if (us(s) < us(best)) best = s;
     if (split_k > 0) best = std::min<int64_t>(split_k, steps);
     p.steps_per_split = (int)cdiv(steps, best);

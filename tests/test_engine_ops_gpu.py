@@ -317,14 +317,16 @@ def test_gemm_swiglu_equals_unfused(dtype, M, K, inter):
     if M > 128:
         ref_lin = nq.awq_gemm(x, side[0], side[1], side[2], 8)      # same kernel and K split as the fused call
     else:
-        # up to 128 rows the plain dispatch takes a narrower tile; force the pipelined kernel with its split rule
+        # up to 128 rows the plain dispatch takes the GEMV: force what the gated product runs (on the 256 x 256 tiles, which it ran
+        # before, 65 rows of 1024 x 6144 took 23 us, and 13 here)
+        import ctypes
         from nanoquantization_amd import _lib
         from nanoquantization_amd.layers.gemm import awq_gemm_variant
         L = _lib.lib()
         names = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())]
-        tiles = (2 * inter + 255) // 256
-        split = max(1, min(256 // tiles, max(1, K // 64 // 8), 16))
-        ref_lin = awq_gemm_variant(x, side[0], side[1], side[2], names.index("256x256p"), split)
+        split = ctypes.c_int()
+        name = L.awq_linear_route(M, 2 * inter, K, 128, _lib.dtype_id(dtype), 1, ctypes.byref(split)).decode()
+        ref_lin = awq_gemm_variant(x, side[0], side[1], side[2], names.index(name), split.value)
     ref = ops.silu_mul(ref_lin)
     assert fused.shape == (M, inter)
     assert torch.equal(fused, ref)

@@ -371,16 +371,20 @@ def test_linear_routes():
     _ensure_built()
     L, f16, bf16 = _lib.lib(), _lib.AWQ_F16, _lib.AWQ_BF16
     for M, K, N, g, dtype, want in (
-            (129, 5120, 10240, 128, bf16, "256x256p"), (192, 5120, 10240, 128, bf16, "256x256p"),      # 46 us; rows128 53, 51
-            (129, 25600, 5120, 128, bf16, "256x256p"), (129, 17408, 5120, 128, bf16, "256x256p"),      # 77, 58; 86, 62
+            (129, 5120, 10240, 128, bf16, "rows128"), (192, 5120, 10240, 128, bf16, "rows128"),        # 43, 45 us; fused 44, 47
+            (129, 25600, 5120, 128, bf16, "rows128"), (129, 17408, 5120, 128, bf16, "rows128"),        # 75, 54; fused 80, 59
+            (192, 17408, 5120, 128, f16, "rows128"), (300, 5120, 17408, 128, f16, "rows128"),          # 54, 81; fused 62, 125, dense 102
             (600, 4096, 24576, 128, f16, "256x256rt"), (900, 4096, 24576, 128, f16, "256x256rt"),      # 138, 185; dense 160, 214
             (900, 2048, 16384, 128, f16, "256x256r"), (640, 5120, 34816, 128, f16, "256x256rt"),       # 60, 269; dense 67, 284
-            (333, 2816, 9720, 64, f16, "rows128"), (333, 2816, 9720, 64, bf16, "rows128"),             # 30, 34; fused 46
-            (200, 4096, 4096, 128, bf16, "rows128"), (160, 12288, 4096, 128, bf16, "rows128"),         # 25, 39; fused 29, 46
-            (256, 12288, 4096, 128, f16, "rows128"), (512, 4096, 4096, 128, f16, "rows128"),           # 43, 33; fused 51, 44
+            (512, 4096, 24576, 128, f16, "256x256p"), (768, 25600, 5120, 128, bf16, "256x256p"),       # 115, 207; rows128 128, 228
+            (200, 512, 25600, 128, bf16, "256x256p"), (1280, 1024, 4096, 128, bf16, "dense"),          # 20, 24; dense 25, fused 32
+            (333, 2816, 9720, 64, f16, "rows128"), (333, 2816, 9720, 64, bf16, "rows128"),             # 27, 30; fused 46
+            (200, 4096, 4096, 128, bf16, "rows128"), (160, 12288, 4096, 128, bf16, "rows128"),         # 24, 35; fused 29, 46
+            (256, 12288, 4096, 128, f16, "rows128"), (512, 4096, 4096, 128, f16, "rows128"),           # 41, 33; fused 50, 43
+            (512, 4096, 4096, 128, bf16, "rows128"), (1023, 8192, 1024, 128, bf16, "rows128"),         # 35, 36; fused 40, 41
             (8192, 4096, 12288, 128, f16, "dense"), (8192, 4096, 12288, 128, bf16, "dense"),           # 575; fused 730, 787
-            (2048, 12288, 4096, 128, bf16, "dense"), (512, 12288, 4096, 128, bf16, "256x256p"),        # 176, 71; fused 209, dense 136
-            (1024, 1024, 4096, 128, bf16, "256x256p"),                                                 # short K
+            (2048, 12288, 4096, 128, bf16, "dense"), (512, 12288, 4096, 128, bf16, "rows128"),         # 176, 71; fused 209, 70, dense 139
+            (1024, 1024, 4096, 128, bf16, "rows128"), (1023, 1024, 4096, 128, bf16, "rows128"),        # 18; fused 31, dense 23
             (16, 1024, 3072, 128, f16, "gemv"), (100, 1024, 1024, 128, f16, "gemv"), (100, 5120, 25600, 128, f16, "128x128"),
             (40, 96, 512, 32, f16, "gemv in blocks of 16 rows"), (300, 192, 520, 24, f16, "")):
         assert _route(L, M, K, N, g, dtype)[0] == want, (M, K, N, g, dtype, _route(L, M, K, N, g, dtype))
