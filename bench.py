@@ -157,7 +157,7 @@ def gemm_kernel_name(M, N, K, dtype_name, g=G):
         return f"awq::dense_kernel<{T}> behind awq::dequant_transpose_kernel"
     kern = {"256x256p": f"awq::gemm_pipe_kernel<{T},2,4>", "256x256pt": f"awq::gemm_pipe_kernel<{T},2,4>",
             "256x256r": f"awq::gemm_regb_kernel<{T}>", "256x256rt": f"awq::gemm_regb_kernel<{T}>",
-            "rows128": f"awq::rows_kernel<{T}>"}.get(
+            "rows128": f"awq::rows_kernel<{T}> (few stages: rows4_kernel)"}.get(
                 name, f"awq::gemm_kernel<{T},{name}>")
     return f"{kern} (plan {name}, split {sp.value})"
 

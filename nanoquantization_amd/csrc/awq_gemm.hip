@@ -202,7 +202,7 @@ struct GemmVariant {
     int BM, BN, waves;
 };
 static const GemmVariant kGemmVariants[] = {
-    // narrow tiles of gemm_kernel for up to 128 rows (wider and 8-wave forms of it were measured and removed)
+    // narrow tiles of gemm_kernel: awq_gemm's for up to 128 rows, awq_linear's where rows128 does not take the sizes
     {"128x128", 128, 128, 4},
     {"64x256", 64, 256, 4},
     {"32x256", 32, 256, 4},
@@ -213,7 +213,7 @@ static const GemmVariant kGemmVariants[] = {
     // pipelined kernel under these names too
     {"256x256r", 256, 256, 4},   // every tile cut split_k ways
     {"256x256rt", 256, 256, 4},  // split_k cuts only the tiles beyond the last full round of CUs
-    {"rows128", 128, 128, 4},    // awq_gemm_rows.hip, for 17 to a few hundred rows: awq_linear's choice alone (rows_wanted)
+    {"rows128", 128, 128, 4},    // awq_gemm_rows.hip, for 17 to about 1000 rows: awq_linear's choice alone (rows_wanted)
 };
 enum { k128x128 = 0, k64x256 = 1, k32x256 = 2 };
 constexpr int kPipeVariant = 3, kPipeTailVariant = 4, kRegbVariant = 5, kRegbTailVariant = 6, kRowsVariant = 7;
@@ -650,9 +650,7 @@ extern "C" const char* awq_linear_route(int64_t M, int64_t N, int64_t K, int64_t
     if (awq_linear_scratch_bytes(M, N, K, group_size, dtype)) return "dense";
     int variant;
     awq::RowsPlan rows;
-    if (rows_wanted(M, N, K, group_size, dtype, &rows))
-        // (up to 128 rows the tile's name is 128x128, whichever kernel awq_gemm runs on it)
-        variant = M > 64 && M <= 128 && !gated ? awq::k128x128 : awq::kRowsVariant, *split_k = rows.splits;
+    if (rows_wanted(M, N, K, group_size, dtype, &rows)) variant = awq::kRowsVariant, *split_k = rows.splits;
     else if (gated) awq::plan_gemm_tile256(M, N, K, group_size, dtype, &variant, split_k);
     else awq::plan_gemm(M, N, K, group_size, dtype, &variant, split_k);
     return awq::kGemmVariants[variant].name;

@@ -461,7 +461,7 @@ def test_gemm_rows128_few_rows(dtype, M, K, N, g, split):
     # the default linear of these rows: the GEMV where it takes the sizes, else these tiles with their own split
     chosen = ctypes.c_int()
     name = L.awq_linear_route(M, N, K, g, _lib.dtype_id(xd.dtype), 0, ctypes.byref(chosen))
-    assert name == (b"128x128" if M > 64 else b"rows128") or (name == b"gemv" and g % 128 == 0)
+    assert name == b"rows128" or (name == b"gemv" and g % 128 == 0)
     if name != b"gemv":
         assert torch.equal(nq.awq_gemm(xd, *dev, 8), awq_gemm_variant(xd, *dev, v, chosen.value))
 

@@ -385,7 +385,8 @@ def test_linear_routes():
             (8192, 4096, 12288, 128, f16, "dense"), (8192, 4096, 12288, 128, bf16, "dense"),           # 575; fused 730, 787
             (2048, 12288, 4096, 128, bf16, "dense"), (512, 12288, 4096, 128, bf16, "rows128"),         # 176, 71; fused 209, 70, dense 139
             (1024, 1024, 4096, 128, bf16, "rows128"), (1023, 1024, 4096, 128, bf16, "rows128"),        # 18; fused 31, dense 23
-            (16, 1024, 3072, 128, f16, "gemv"), (100, 1024, 1024, 128, f16, "gemv"), (100, 5120, 25600, 128, f16, "128x128"),
+            (16, 1024, 3072, 128, f16, "gemv"), (100, 1024, 1024, 128, f16, "gemv"), (100, 5120, 25600, 128, f16, "rows128"),     # 47; plain tiles 69
+            (100, 5120, 120, 128, f16, "128x128"), (100, 1024, 512, 16, f16, "128x128"),               # what the 128-row tiles do not take
             (40, 96, 512, 32, f16, "gemv in blocks of 16 rows"), (300, 192, 520, 24, f16, "")):
         assert _route(L, M, K, N, g, dtype)[0] == want, (M, K, N, g, dtype, _route(L, M, K, N, g, dtype))
     names = [L.awq_gemm_variant_name(i).decode() for i in range(L.awq_gemm_variant_count())]
