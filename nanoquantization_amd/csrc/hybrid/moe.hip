@@ -6,6 +6,7 @@
 //   most pairs   tiles of 128 or 256 pairs x 256 weight rows on the product core of pingpong.hpp (rows in whole stages of 64)
 //   any sizes    32 x 32 tiles in fp32 on the vector ALU (fp32 operands, rows that are not multiples of 8)
 #include <algorithm>
+#include <cmath>
 
 #include "../pingpong.hpp"
 #include "moe_route.hpp"
@@ -413,30 +414,62 @@ void launch_pingpong(const uint16_t* in, const uint16_t* w, const float* weight,
 }
 
 enum class MoeForm { simple, skinny16, skinny32, skinny64, gemm64, gemm128, pingpong128, pingpong256 };
+// Expected tiles of `rows` pairs: the pairs of an expert vary around their mean, here evenly over 2.2 of its roots to either side
+// (routers are less even than chance), and near whole tiles some of the experts have one more.
+double expected_tiles(int64_t pairs, int64_t experts, int rows) {
+    if (pairs < experts) return (double)pairs;
+    const double mean = (double)pairs / (double)experts, spread = 2.2 * std::sqrt(mean);
+    const double low = std::max(0.0, mean - spread), high = mean + spread;
+    const auto below = [&](double x) {          // the integral of ceil(u / rows) from 0 to x
+        const double k = std::floor(x / rows);
+        return rows * k * (k + 1) / 2 + (k + 1) * (x - k * rows);
+    };
+    return (double)experts * (below(high) - below(low)) / (high - low);
+}
+
+// Microseconds of both products: a stage of 64 of the contraction, in fuller rounds of the CUs a longer one, and the ends of a tile; no
+// less than the weights take from memory.  Fitted to 16 sizes (2 to 128 experts, 512 to 4096 -> 2 x 384 to 2 x 6144) at 20 to 1000 pairs
+// an expert, all forms timed: the least estimate is 0.7 % from the fastest form on average, more than a tenth in one of 30.
+double moe_form_us(MoeForm form, int64_t pairs, int64_t experts, int64_t width, int64_t ff) {
+    const bool gemm = form == MoeForm::gemm64, large = form == MoeForm::pingpong256;
+    const double tiles = expected_tiles(pairs, experts, gemm ? 64 : (large ? 256 : 128)), columns = gemm ? 128 : 256;
+    const auto product = [&](int64_t n_out, int64_t n_in) {
+        const double rounds = tiles * std::ceil((double)n_out / columns) / 256, full = std::floor(rounds), part = rounds - full;
+        const double stages = (double)n_in / 64;
+        if (gemm) return 4.9 + stages * std::max(0.53, 0.23 + 0.436 * rounds);
+        const double alone = large ? 0.744 : 0.53, shared = large ? 0.748 : 0.487;
+        return std::ceil(rounds) * (large ? 10.4 : 6.6) + stages * (full * (alone + shared) + (part > 0 ? alone + shared * part : 0));
+    };
+    const double streamed = (double)(std::min(experts, pairs) * width * ff * 6) / ((gemm ? 3.34 : (large ? 3.6 : 4.23)) * 1e6);
+    return std::max(product(2 * ff, width) + product(width, ff), streamed);
+}
+
 MoeForm moe_form(int64_t pairs, int64_t experts, int64_t width, int64_t ff, int dtype) {
     if (dtype != NQH_BF16 || width % 8 != 0 || ff % 8 != 0) return MoeForm::simple;
     // by pairs per expert, so that one tile usually holds all pairs of an expert while there are few
     if (pairs <= 6 * experts || pairs <= 16) return MoeForm::skinny16;
     if (pairs <= 16 * experts || pairs <= 32) return MoeForm::skinny32;
-    // The ping-pong core wants whole stages and 32-bit offsets into the rows and into an expert's weights.  Its tiles stream an
-    // expert's weights once, so they are the fastest from 17 pairs an expert on where every expert's tile of the smaller product
-    // makes 64 workgroups.  Both products, 8 experts, skinny 64 / gemm 64 / pingpong 128 / 256 pairs a tile, us:
-    //   4096 -> 2 x 6144, 20 pairs each 404 / 343 / 269 / 303, 40 each 500 / 346 / 278 / 308, 80 each 803 / 449 / 291 / 317, 115 each
-    //   458 / 330 / 325 with 64 / 128 / 256, 140 each 553 / 342 / 338, 212 each 656 / 362 / 429, 325 each 734 / 547 / 459;
-    //   2048 -> 2 x 3072, 28 each 134 / 110 / 95 / 107, 80 each 144 / 104 / 112 from gemm 64 on, 100 each 138 / 125 / 113, 140 each
-    //   144 / 125 / 124, 250 each 176 / 131 / 169, 425 each 255 / 163 / 175;
-    //   1024 -> 2 x 1536 (32 workgroups), 28 each 40 / 35 / 38 / 55, 115 each 38 / 40 / 57, 173 each 39 / 42 / 60, 212 each 50 / 44 / 61.
-    // 2048 -> 2 x 1024, 64 experts, 144 each 318 / 277 / 236, 384 each 529 / 422 / 376.
+    // few experts and short rows: more workgroups (2 experts, 1024 -> 2 x 4096, 20 pairs each: 31 us, 50 with 64 x 128 tiles)
+    const int64_t used = std::min(experts, pairs);
+    if ((pairs <= 40 * experts || pairs <= 64) && used * cdiv(std::min(width, 2 * ff), 128) < 64) return MoeForm::skinny64;
+    // The ping-pong core wants whole stages and 32-bit offsets into the rows and into an expert's weights.  Its tiles stream an expert's
+    // weights once and faster; the 64 x 128 tiles have less to fill.  Both products, 64 x 128 / ping-pong 128 / 256 pairs a tile, us:
+    //   8 experts, 4096 -> 2 x 6144, 20 pairs each 291 / 262 / 315, 115 each 430 / 297 / 330, 250 each 682 / 476 / 372;
+    //   8 experts, 2048 -> 2 x 3072, 28 each 98 / 84 / 110, 100 each 130 / 98 / 108, 130 each 133 / 130 / 111;
+    //   8 experts, 1024 -> 2 x 1536, 20 each 33 / 38 / 56, 160 each 39 / 43 / 58, 600 each 87 / 68 / 95;
+    //   64 experts, 1024 -> 2 x 512, 40 each 57 / 43 / 57; 16 experts, 40 each 24 / 28 / 41, 115 each 26 / 30 / 42, 325 each 48 / 35 / 48;
+    //   4 experts, 4096 -> 2 x 1536, 20 each 56 / 64 / 96, 200 each 64 / 70 / 100, 400 each 101 / 80 / 108.
     const bool stages = width % 64 == 0 && ff % 64 == 0 && pairs * std::max(width, ff) * 2 < (1ll << 32) &&
                         width * ff * 4 < (1ll << 32);
-    const int64_t groups = std::min(cdiv(width, 256), cdiv(ff, 128)), used = std::min(experts, pairs);
-    if (stages && pairs > 320 * experts && pairs * groups >= 128 * 256) return MoeForm::pingpong256;
-    if (stages && groups * std::max(used, pairs / 128 + used / 2) >= 64)
-        // pairs vary around their mean: near 128 many an expert has more, which would be a second tile
-        return groups * used >= 64 && pairs > 88 * experts && pairs <= 144 * experts ? MoeForm::pingpong256 : MoeForm::pingpong128;
-    // few experts and short rows: more workgroups, though they read the weights no more than once either
-    if ((pairs <= 40 * experts || pairs <= 64) && used * cdiv(std::min(width, 2 * ff), 128) < 64) return MoeForm::skinny64;
-    return pairs <= 256 * experts ? MoeForm::gemm64 : MoeForm::gemm128;
+    if (!stages) return pairs <= 256 * experts ? MoeForm::gemm64 : MoeForm::gemm128;
+    // (many pairs, a workgroup for half of the CUs in the smaller product: whatever the estimate, which was not fitted to shorter rows)
+    const bool many = pairs > 160 * experts && pairs * std::min(cdiv(width, 256), cdiv(ff, 128)) >= 128 * 128;
+    MoeForm best = MoeForm::pingpong128;
+    for (const MoeForm form : {MoeForm::pingpong256, MoeForm::gemm64})
+        if (!(many && form == MoeForm::gemm64) &&
+            moe_form_us(form, pairs, experts, width, ff) < moe_form_us(best, pairs, experts, width, ff))
+            best = form;
+    return best;
 }
 int moe_form_rows(MoeForm f) {
     switch (f) {

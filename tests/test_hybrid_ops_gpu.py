@@ -418,9 +418,10 @@ def test_experts_with_many_pairs(rows, width, experts, top, ff, tile):
     assert torch.equal(y, ops.moe_experts(h, gu, dn, r))
 
 
-# few pairs on large tiles: just past the skinny tiles, the line to 256 pairs a tile and back; short rows, where the larger tiles come
-# later; few experts, which keep the skinny tiles longer
-@pytest.mark.parametrize("rows,width,experts,top,ff,tile", [(65, 1856, 8, 2, 960, 128), (353, 1856, 8, 2, 960, 256), (600, 1856, 8, 2, 960, 128),
+# few pairs on large tiles: just past the skinny tiles, some 100 pairs an expert, near 128 where 256 pairs a tile are the faster; the same
+# with weights too small for them; short rows, where the larger tiles come later; few experts, which keep the skinny tiles longer
+@pytest.mark.parametrize("rows,width,experts,top,ff,tile", [(70, 1856, 20, 6, 960, 128), (300, 1024, 64, 20, 640, 128), (560, 1024, 40, 10, 640, 256),
+                                                            (65, 1856, 8, 2, 960, 64), (353, 1856, 8, 2, 960, 64), (600, 1856, 8, 2, 960, 64),
                                                             (65, 512, 8, 2, 320, 64), (1000, 512, 8, 2, 320, 64), (3000, 1024, 8, 2, 512, 128),
                                                             (70, 1024, 4, 1, 320, 64), (33, 4096, 1, 1, 4096, 64)])
 def test_experts_with_few_pairs_on_large_tiles(rows, width, experts, top, ff, tile):
