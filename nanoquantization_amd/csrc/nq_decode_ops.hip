@@ -1113,9 +1113,10 @@ extern "C" int nq_add_rmsnorm(void* residual, const void* delta, const void* wei
     }
     hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();
-    // a wave a row from 1024 rows on (256 workgroups); longer rows with a delta are as well or better off with a workgroup each (8192
-    // x 2048 25.7 us there, 29.6 with a wave)
-    if (rows >= 1024 && hidden <= (delta ? 1024 : 4096)) {
+    // a wave a row from 1024 rows on (256 workgroups), longer rows than 2560 from 2048 on (1500 x 4096 8.0 us with a workgroup each, 8.8 with
+    // a wave; 2048 rows 10.2 and 10.1, x 3072 9.1 and 8.5); with a delta those beyond 1024 are as well or better off with a workgroup each (8192 x 2048 25.7 us
+    // there, 29.6 with a wave)
+    if (rows >= (hidden <= 2560 ? 1024 : 2048) && hidden <= (delta ? 1024 : 4096)) {
         const auto go = [&](auto kernel) {
             kernel<<<dim3((unsigned)cdiv(rows, 4)), dim3(256), 0, st>>>((uint16_t*)residual, (const uint16_t*)delta, (const uint16_t*)weight,
                                                                         (uint16_t*)y, rows, (int)hidden, eps);

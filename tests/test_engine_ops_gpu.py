@@ -44,19 +44,21 @@ def test_add_rmsnorm(dtype, rows, hidden):
     _close(y1, _rmsnorm_ref(x + d, w, 1e-6), dtype, what="add + norm")
 
 
-# from 1024 rows a wave takes a row: widths that end inside a 128-column tile, a pass and a wave's last pass; a last workgroup of one row
+# from 1024 rows (2048 of more than 2560 columns) a wave takes a row: widths that end inside a 128-column tile, a pass and a wave's last pass; a last workgroup of one row
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hidden", [8, 136, 512, 520, 1024, 1032, 2048, 2560, 2568, 4096, 4104])
 def test_add_rmsnorm_of_many_rows(dtype, hidden):
     """The bits of the same rows a few at a time, which a workgroup each takes."""
     from nanoquantization_amd.engine import ops
     g = torch.Generator(device="cuda").manual_seed(hidden)
-    x, d = (torch.randn(1025, hidden, generator=g, device="cuda").to(dtype) for _ in range(2))
+    rows, few_rows = (1025, 205) if hidden <= 2560 else (2049, 683)
+    x, d = (torch.randn(rows, hidden, generator=g, device="cuda").to(dtype) for _ in range(2))
     w = (1 + 0.1 * torch.randn(hidden, generator=g, device="cuda")).to(dtype)
     for delta in (None, d):
         many, few = x.clone(), x.clone()
         y = ops.add_rmsnorm(many, delta, w, 1e-6)
-        parts = [ops.add_rmsnorm(few[i:i + 205], None if delta is None else delta[i:i + 205], w, 1e-6) for i in range(0, 1025, 205)]
+        parts = [ops.add_rmsnorm(few[i:i + few_rows], None if delta is None else delta[i:i + few_rows], w, 1e-6)
+                 for i in range(0, rows, few_rows)]
         assert torch.equal(y, torch.cat(parts)) and torch.equal(many, few)
     _close(y, _rmsnorm_ref(x + d, w, 1e-6), dtype, what="add + norm")
 
