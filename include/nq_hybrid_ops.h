@@ -241,7 +241,8 @@ int nqh_skinny_linear(const void* x, const void* weight, const void* bias, void*
 
 /* y [rows, out_features] = act(x @ weight^T), bf16, act applied to the product rounded to bf16; for many rows.  in_features a
  * multiple of 64, out_features one of 8, all pointers 16-byte aligned, rows without padding.  act and param as in nqh_activate.
- * nqh_dense_activation_wanted: 1 where it takes the sizes and is faster than a library product with nqh_activate behind it. */
+ * nqh_dense_activation_wanted: 1 where it takes the sizes and one launch of it is done before a library product with nqh_activate
+ * behind it, both issued one at a time (28 us for the two at least; in a captured graph the library's product may be the faster). */
 int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_features);
 int nqh_dense_activation(const void* x, const void* weight, void* y, int64_t rows, int64_t out_features, int64_t in_features, int act,
                          float param, void* stream);

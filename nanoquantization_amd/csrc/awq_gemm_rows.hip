@@ -11,10 +11,13 @@
 // load-to-LDS in pieces of 1 KiB, 16 bytes a lane, in a ring of kDepth stages.
 // Unpacked values are those of awq_dequantize, bit for bit; bf16 scales of 2^113 and more, whose quick way to them overflows, in a
 // second pass of the waves that meet one.
-// What bounds it: the phases, 0.35 us a stage at five rows tiles and 0.45 at eight, of which the matrix instructions take half; no
-// load is waited for (with all of them answered by zeros the time is the same), but asking for them is a fifth of a phase.
-// Measured: 333 x 2816 x 9720 in fp16, groups of 64, 29.8 -> 27.1 us against four waves that each unpack beside their own matrix
-// instructions, in bf16 34.9 -> 30.4; 640 x 2048 x 6144 in bf16 28 -> 26.  5120 x 25600 in groups of 64 at 64 rows, bf16, 46 -> 41 us
+// What bounds it: the phases, 0.38 us a stage at five row tiles and 0.46 at eight in fp16, 0.44 and 0.51 in bf16.  333 x 2816 x 9720 in
+// fp16, over the time a CU is busy: the matrix cores 34 %, the vector units 39 %, the LDS 20 % without conflicts; of a wave's time a
+// third goes by at hand-overs and for LDS reads, a third for the issue of its next instruction.  (With the loads from memory answered
+// by zeros the time is the same.)  The end, where the four parts of K meet, takes 1.2 us with five row tiles and 1.5 with eight more than
+// without the exchange; few stages are left to awq_gemm_rows4.hip, where two parts meet.
+// Measured: 333 x 2816 x 9720 in fp16, groups of 64, 29.8 -> 26.7 us against those four waves, in bf16 34.9 -> 30.4; 640 x 2048 x 6144
+// in bf16 28 -> 26.  5120 x 25600 in groups of 64 at 64 rows, bf16, 46 -> 41 us
 // against the 64 x 256 tiles of awq_gemm.hip, 5120 x 17408 at 57 rows 44 -> 31 and at 32 rows 29 -> 25, 15296 x 4680 at 18 rows
 // 33 -> 23; 5120 x 25600 at 100 rows 69 -> 47 against its 128 x 128 tiles.
 #include "awq_common.hpp"

@@ -236,11 +236,13 @@ extern "C" int nqh_skinny_linear(const void* x, const void* weight, const void* 
     return launched(fn);
 }
 
-// 1 where the tiles are one round of the 256 CUs and estimated to take less time than the library's product and the activation's pass:
-// 1.3 PFLOP/s and 5 TB/s, 28 us at least, which is what two launches take from python.  relu2, this kernel / those two, us: 1024 ->
-// 4608 features at 65 rows 16 / 24, 1500 rows 20 / 26, 3000 rows 31 / 37; 2048 -> 9216 at 128 rows 25 / 25, 700 rows 30 / 35, 1500
-// rows 49 / 57; 4096 -> 18432 at 128 rows 44 / 34 (left to the library), 384 rows 53 / 60, 700 rows 85 / 96.  Roletar prompts through
-// three layers: 0.6B, 400 tokens 754 -> 699, 1000 tokens 805 -> 749, 3000 tokens 884 -> 830; 1.7B, 700 tokens 787 -> 738.  Several rounds
+// 1 where the tiles are one round of the 256 CUs and estimated to take less time than the library's product and the activation's pass
+// do when a python program issues them: 1.3 PFLOP/s and 5 TB/s, 28 us at least, the two launches.  On the GPU alone, from a graph, the
+// library's smaller tiles are ahead up to some 1000 rows: relu2, this kernel / those two, us, 1024 -> 4608 at 65 rows 16 / 11, 2048 ->
+// 9216 at 100 rows 26 / 17, 2048 -> 1536 at 1000 rows 27 / 18.  What counts is the pass, which the host issues more slowly than the GPU works it
+// off: Roletar prompts through three layers with this kernel / without, wall time and (behind other work, GPU time): 0.6B, 128
+// tokens 666 / 713 (356 / 333), 1000 tokens 696 / 743 (514 / 514); 1.7B, 128 tokens 646 / 751 (495 / 448), 400 tokens 666 / 717 (585 / 590),
+// 1000 tokens 860 / 872; 8B 0 to 2 % less.  Several rounds
 // stay with the library: in a pass its products lose less to the writes between the rounds (0.6B, 8192 tokens, 576 tiles: 110 here,
 // 83 + 24 there, though 89 / 103 when repeated alone; 1.7B, 4096 tokens, 576 tiles: the pass 1873 -> 1886).
 extern "C" int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_features) {

@@ -633,7 +633,7 @@ def skinny_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
 
 
 def dense_activation_wanted(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether `dense_activation` takes these and is faster than a library product followed by `activate_`."""
+    """Whether `dense_activation` takes these and its one launch is done before a library product and `activate_` issued from here."""
     return (x.dtype == weight.dtype == torch.bfloat16 and x.is_contiguous() and weight.is_contiguous()
             and (x.data_ptr() | weight.data_ptr()) % 16 == 0
             and bool(_lib.hybrid_lib().nqh_dense_activation_wanted(x.shape[0], *weight.shape)))
