@@ -508,7 +508,7 @@ extern "C" int awq_gemm(const void* x, const int32_t* qweight, const void* qscal
 // Microseconds of the fused 256 x 256 kernels: 1.88 a K step in a full round of 256 workgroups, 1 to 1.82 in one that leaves CUs idle,
 // 9.7 to fill and store a round's tiles; 3 and the time of the fp32 partials at 10.2 TB/s (they stay in the caches) where tiles are cut.
 // The workgroups of the register-operand kernel go through one run of steps each, at 1.82 in fp16 (1.7 with one whole tile each: 900 x
-// 2048 x 16384 60 us) and 1.95 in bf16, and less where a tile's rows are not there.  0.9 to 1.08 times the measured times of 43
+// 2048 x 16384 60 us) and 1.95 in bf16, and less where a tile's rows are not there.  0.9 to 1.08 times the measured times of 42
 // weights by 130 to 2048 rows, in both types, in 96 of 100; that is what holds the routes: they lose 0.4 % to the fastest way on
 // average, more than 4 % in one of 40.
 static double fused_linear_us(int64_t M, int64_t N, int64_t K, int64_t g, int dtype) {

@@ -110,7 +110,7 @@ double product_us(int64_t M, int64_t slab, int64_t K, int xr) {
 
 int product_tile(int64_t M, int64_t slab, int64_t K) { return product_us(M, slab, K, 128) < product_us(M, slab, K, 256) ? 128 : 256; }
 
-// The same for the comparison with other ways, fitted to the times of 43 weights by 130 to 2048 rows (within 10 % in 94 of 100; the
+// The same for the comparison with other ways, fitted to the times of 42 weights by 130 to 2048 rows (within 10 % in 94 of 100; the
 // terms have to be taken together): rounds with their ends, the last of which has shorter stages where it leaves CUs idle.
 double rounds_us(int64_t M, int64_t slab, int64_t K) {
     const int xr = product_tile(M, slab, K);

@@ -469,7 +469,7 @@ RowsPlan make_rows_plan(int64_t M, int64_t N, int64_t K, int64_t g, int dtype, i
     const int few = dtype == AWQ_F16 ? 18 : 14, t = dtype == AWQ_F16 ? 0 : 1;
     // Microseconds, by type and MT: a stage of the four waves; of the eight with a CU to itself and with two workgroups on it; and of
     // filling the ring, the tile's sums and the launch.  A K split writes its fp32 sums and reads them again in a second launch.
-    // From five row tiles on within 10 % of 96 of 100 measured times (43 weights, 130 to 2048 rows, every split).
+    // From five row tiles on within 10 % of 96 of 100 measured times (42 weights, 130 to 2048 rows, every split).
     constexpr double kFour[2][4] = {{0.45, 0.445, 0.485, 0.515}, {0.56, 0.56, 0.595, 0.59}};     // [fp16, bf16][MT - 5]
     constexpr double kAlone[2][7] = {{0.28, 0.295, 0.38, 0.375, 0.38, 0.405, 0.46}, {0.345, 0.37, 0.445, 0.44, 0.465, 0.485, 0.515}};   // [MT - 2]
     constexpr double kShared[2][3] = {{0.455, 0.45, 0.495}, {0.52, 0.53, 0.575}};
