@@ -305,10 +305,20 @@ __device__ __forceinline__ void rows_tile(
     if constexpr (T::id == AWQ_BF16) {
         // A weight that was no number has made all rows of its column none, whatever x holds: this wave's part of the tile once more,
         // straight from memory.  (A branch among the unpacking that looks at the scales costs a third of the whole kernel's time.)
-        bool off = false;
+        const auto none = [&](int f, int r) { return !(__builtin_fabsf(acc[0][f][r]) <= 3.402823466e38f); };
+        bool some = false;
 #pragma unroll
-        for (int f = 0; f < 4; ++f) off |= !(__builtin_fabsf(acc[0][f][0]) <= 3.402823466e38f);
-        if (__builtin_amdgcn_ballot_w64(off)) {
+        for (int f = 0; f < 4; ++f) some |= none(f, 0);
+        uint64_t off = 0;       // columns that hold none in all of the first 16 rows: a row of x that is none leaves the others
+        if (__builtin_amdgcn_ballot_w64(some)) {
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                uint64_t lanes = __builtin_amdgcn_ballot_w64(none(f, 0) && none(f, 1) && none(f, 2) && none(f, 3));
+                lanes &= lanes >> 32;
+                off |= lanes & (lanes >> 16) & 0xFFFFu;
+            }
+        }
+        if (off != 0) {
             int row = j, part_k = 8 * kb;       // (hidden from the compiler, which would keep what the two passes share through the first)
             asm volatile("" : "+v"(row), "+v"(part_k));
             const int word = word0 + row;

@@ -489,6 +489,11 @@ def test_gemm_rows128_large_scales(M, K, N, g, split):
     ref = x.double() @ w.double()
     bound = TIGHT["bf16"] * ref.abs().amax(dim=0)            # a column at a time
     assert y.isfinite().all() and ((y.double() - ref).abs() <= bound).all()
+    # an element of x that is no number concerns its own row
+    xn = x.clone()
+    xn[0, 5] = float("nan")
+    z = awq_gemm_variant(xn, qw, qs, qz, v, split)
+    assert z[0].isnan().all() and torch.equal(z[1:], y[1:])
     # a scale that is no number concerns its own column
     qs[0, 1] = float("inf")
     z = awq_gemm_variant(x, qw, qs, qz, v, split)
