@@ -19,6 +19,9 @@ extern "C" {
 #endif
 
 enum nqh_dtype { NQH_BF16 = 1, NQH_F32 = 2 };
+/* Added to the dtype of nqh_residual_norm, nqh_residual_norm_route and nqh_hyper_norm_parts: y is fp32 whatever the other types are
+ * (the sums of a product's parts as nqh_skinny_linear_sums leaves them). */
+enum { NQH_Y_F32 = 4 };
 enum nqh_status { NQH_OK = 0, NQH_ERR_ARG = 1, NQH_ERR_UNSUPPORTED = 2, NQH_ERR_WORKSPACE = 3, NQH_ERR_HIP = 4 };
 
 /* What follows a matrix product: nothing, the square of max(v, 0), or param * tanh(v / param). */
@@ -46,6 +49,11 @@ int64_t nqh_hyper_max_streams(void);
 int nqh_hyper_norm(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y, const void* mix,
                    const void* w_out, const void* w_in, const void* norm_weight, void* h, int64_t rows, int64_t streams,
                    int64_t width, float eps, int dtype, void* stream);
+
+/* The same with y [rows, y_parts, width]; the sum of the parts counts. */
+int nqh_hyper_norm_parts(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y, int64_t y_parts,
+                         const void* mix, const void* w_out, const void* w_in, const void* norm_weight, void* h, int64_t rows,
+                         int64_t streams, int64_t width, float eps, int dtype, void* stream);
 
 /* x [count] = activation(x), in place; act is an nqh_activation. */
 int nqh_activate(void* x, int64_t count, int act, float param, int dtype, void* stream);
@@ -238,6 +246,19 @@ int nqh_moe_down(const void* act, const void* down, const int32_t* order, const 
  * act and param as in nqh_activate. */
 int nqh_skinny_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
                       int64_t in_features, int out_f32, int act, float param, void* stream);
+
+/* The same with scratch memory of nqh_skinny_linear_scratch_bytes (16-byte aligned; 0: not wanted): the contraction may be split over
+ * workgroups whose sums a second launch adds.  Without enough of it the call is nqh_skinny_linear.  captured: whether the call goes
+ * into a graph; one that the host issues by itself has to gain the second launch's host time too. */
+size_t nqh_skinny_linear_scratch_bytes(int64_t rows, int64_t out_features, int64_t in_features, int captured);
+int nqh_skinny_linear_ex(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
+                         int64_t in_features, int out_f32, int act, float param, void* scratch, size_t scratch_bytes, void* stream);
+
+/* sums [rows, parts, out_features] fp32, 16-byte aligned: the product x weight^T, its contraction split into
+ * nqh_skinny_linear_parts(rows, out, in) >= 1 parts for a reader that adds them. */
+int64_t nqh_skinny_linear_parts(int64_t rows, int64_t out_features, int64_t in_features);
+int nqh_skinny_linear_sums(const void* x, const void* weight, float* sums, int64_t rows, int64_t out_features, int64_t in_features,
+                           void* stream);
 
 /* y [rows, out_features] = act(x @ weight^T), bf16, act applied to the product rounded to bf16; for many rows.  in_features a
  * multiple of 64, out_features one of 8, all pointers 16-byte aligned, rows without padding.  act and param as in nqh_activate.

@@ -103,6 +103,7 @@ HYBRID_SYMBOLS = {
     "nqh_attention_decode": (_int, [_vp] * 7 + [_i64] * 12 + [_f32, _int, _vp, _sz, _vp]),
     "nqh_hyper_max_streams": (_i64, []),
     "nqh_hyper_norm": (_int, [_vp] * 3 + [_i64] + [_vp] * 6 + [_i64] * 3 + [_f32, _int, _vp]),
+    "nqh_hyper_norm_parts": (_int, [_vp] * 3 + [_i64, _vp, _i64] + [_vp] * 5 + [_i64] * 3 + [_f32, _int, _vp]),
     "nqh_activate": (_int, [_vp, _i64, _int, _f32, _int, _vp]),
     "nqh_latent_store": (_int, [_vp] * 7 + [_i64] * 7 + [_int] + [_i64] * 4 + [_f32, _int, _vp]),
     "nqh_latent_gather": (_int, [_vp] * 5 + [_i64] * 9 + [_vp]),
@@ -132,6 +133,10 @@ HYBRID_SYMBOLS = {
     "nqh_moe_gate_up": (_int, [_vp] * 6 + [_i64] * 7 + [_int, _vp]),
     "nqh_moe_down": (_int, [_vp] * 5 + [_i64] * 6 + [_int, _vp]),
     "nqh_skinny_linear": (_int, [_vp] * 4 + [_i64] * 3 + [_int, _int, _f32, _vp]),
+    "nqh_skinny_linear_scratch_bytes": (_sz, [_i64] * 3 + [_int]),
+    "nqh_skinny_linear_ex": (_int, [_vp] * 4 + [_i64] * 3 + [_int, _int, _f32, _vp, _sz, _vp]),
+    "nqh_skinny_linear_parts": (_i64, [_i64] * 3),
+    "nqh_skinny_linear_sums": (_int, [_vp] * 3 + [_i64] * 3 + [_vp]),
     "nqh_dense_activation_wanted": (_int, [_i64] * 3),
     "nqh_dense_activation": (_int, [_vp] * 3 + [_i64] * 3 + [_int, _f32, _vp]),
     "nqh_argmax_rows": (_int, [_vp, _vp, _i64, _i64, _vp]),

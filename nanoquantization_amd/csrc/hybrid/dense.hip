@@ -1,9 +1,11 @@
 // Dense linears.  For few rows: y = act(x W^T (+ bias)), bf16 operands, fp32 accumulation.
-//   up to 16 rows    skinny_linear_kernel: both operands straight from memory, the waves split the contraction; also for more
-//                    rows of few features, 16 at a time, where the next would leave most of the chip idle
-//   17 to 64 rows    wide_linear_kernel: the activations, by now as many bytes per workgroup as its weights, go through LDS
-// and y = act(x W^T) for more rows where an activation follows, dense_activation_kernel.
+//   skinny_linear_kernel   both operands straight from memory, 16 rows at a time, the waves split the contraction
+//   stream_linear_kernel   up to 64 rows at once: the activations go through LDS; the contraction may be split over workgroups,
+//                          whose sums the reader adds (nqh_skinny_linear_parts) or sum_parts_kernel
+// plan_linear says which.  And y = act(x W^T) for more rows where an activation follows, dense_activation_kernel.
 #include <algorithm>
+#include <atomic>
+#include <cmath>
 
 #include "../pingpong.hpp"
 #include "skinny.hpp"
@@ -33,91 +35,305 @@ __global__ __launch_bounds__(1024) void skinny_linear_kernel(const uint16_t* __r
     }
 }
 
-// 16 MT rows, 16 NT output features per workgroup; its eight waves are NT features tiles x KS parts of every stage of
-// KS * 128 contraction elements.  The stage's activations are brought to LDS once (rows of 128 elements, 16-byte piece p of
-// row r at position (p + r) % 16: the 16 rows of an operand read fall on all banks once), double-buffered; the weights
-// stream into registers, one stage ahead.
-#define NQH_GPTR(p) ((__attribute__((address_space(1))) void*)(p))
+// 16 MT rows, 16 NT output features and a part of the contraction per workgroup; its waves are NT features tiles x KS parts of every
+// stage of KS * 128 contraction elements.  The weights go straight into registers, kAhead stages ahead; the activations, which all
+// waves read, are brought to LDS once, as far ahead (rows of 256 bytes, 16-byte piece p of row r at position (p + r) % 16: the 16
+// rows of an operand read fall on all banks once).  A stage is waited for by the count of the requests behind it, so that the one
+// barrier a stage stops nobody's stream.  Workgroups begin at different stages: in step they would ask the same memory channels,
+// the rows of a weight being a power of two apart as often as not.
+//
+// Bound by the stream of the weights (5 to 5.6 TB/s) and by what a CU takes in, some 45 KB/us of weights and activations alike.  That
+// is why the contraction is split until there is a workgroup for each CU, and why workgroups are wider where there are more rows.
+// Weights from memory, us, before (all of the contraction in one workgroup, one stage ahead, waited for in full) / this with the sums
+// left to the reader: 64 rows 18432 -> 4096 87 / 34, 4096 -> 4096 21 / 10.8, 9216 -> 2048 44 / 12.3; 16 rows 41 / 28, 11.2 / 8.4, 19.6 / 9.4;
+// one row 33.8 / 27.4, 9.4 / 8.3, 14.1 / 9.2.  Unsplit: 64 rows 4096 -> 32768 70 / 53 (63 with all workgroups in step), 4096 ->
+// 12288 37 / 30, 1024 -> 4608 7.8 / 7.5; 32 rows 1024 -> 32768 16.3 / 15.1.  Seven stages ahead are no faster than three.
 #define NQH_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
-__device__ const u32x4 g_zero_piece = {0u, 0u, 0u, 0u};   // what lies past the end of a row
 
-template <int MT, int NT, bool F32OUT>
-__global__ __launch_bounds__(512) void wide_linear_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                          const uint16_t* __restrict__ bias, void* __restrict__ y, int rows,
-                                                          int n_out, int n_in, int act, float param) {
-    constexpr int KS = 8 / NT, kPart = 16 * MT * 256, kBuf = KS * kPart, kLoads = kBuf / 1024 / 8;
-    extern __shared__ __attribute__((aligned(1024))) unsigned char s_x[];   // [buffer][part][row][256 bytes]
+template <int N, typename F>
+__device__ __forceinline__ void each_of(F&& f) {      // f(0) .. f(N - 1), the numbers known to the compiler
+    if constexpr (N > 0) {
+        each_of<N - 1>(f);
+        f(Int<N - 1>());
+    }
+}
+
+// SPLIT: y takes the sums of every part, fp32 [rows, parts, n_out], n_out % 4 == 0; bias and activation are the reader's.
+template <int MT, int NT, int KS, int kAhead, bool F32OUT, bool SPLIT>
+__global__ __launch_bounds__(64 * NT * KS, NT == 8 ? 4 : 2) void stream_linear_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, void* __restrict__ y, int rows,
+    int n_out, int n_in, int act, float param, int pieces_each) {
+    constexpr int NW = NT * KS, kPart = 16 * MT * 256, kBuf = KS * kPart, kLoads = kBuf / 1024 / NW;
+    constexpr int kStageLoads = 4 + kLoads, kStageBufs = kAhead + 1;
+    static_assert(kLoads >= 1 && kLoads * NW * 1024 == kBuf, "every wave brings the same");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char s_x[];   // [buffer][row][256 bytes]
     const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt = wave % NT, part = wave / NT;
-    const int n0 = blockIdx.x * 16 * NT;
-    const uint16_t* w_row = w + (int64_t)min(n0 + 16 * nt + lo, n_out - 1) * n_in;
-    auto stage = [&](int k0, int buf) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nt = wave % NT, part = wave / NT, n0 = (blockIdx.x * NT + nt) * 16, first = blockIdx.y * pieces_each;
+    const int pieces = min(pieces_each, (n_in + kPiece - 1) / kPiece - first), count = (pieces + KS - 1) / KS;
+    // This wave's rows of the weight, past the end the last one.  What lies past the end of a row or behind the last stage is
+    // outside the buffer: zeros without traffic, and the count of requests stays.
+    const int w0 = min(n0, n_out - 1), own = min(n0 + lo, n_out - 1) - w0;
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w) + (int64_t)w0 * n_in, 0,
+                                                      (uint32_t)min(16, n_out - w0) * (uint32_t)n_in * 2, 0x00020000);
+    const uint32_t own_at = (uint32_t)own * (uint32_t)n_in * 2;
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, (uint32_t)rows * (uint32_t)n_in * 2, 0x00020000);
+    constexpr uint32_t kOutside = 0x80000000u;
+    const int turn = (int)(((blockIdx.x * 5) & 31) * (unsigned)count >> 5);      // the stage that comes first here
+    const auto turned = [&](int t) { const int u = t + turn; return t >= count ? t : u >= count ? u - count : u; };
+    const auto load_w = [&](u32x4 (&f)[4], int t0) {
+        const int t = turned(t0);
+        const int k0 = (first + t * KS + part) * kPiece + 8 * hi, end = t * KS + part < pieces ? n_in : 0;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            f[s] = __builtin_amdgcn_raw_buffer_load_b128(rw, k0 + 32 * s < end ? own_at + (uint32_t)(k0 + 32 * s) * 2 : kOutside, 0, 0);
+    };
+    const auto load_x = [&](int t0, int at) {
+        const int t = turned(t0);
+        unsigned char* buf = s_x + at * kBuf;
 #pragma unroll
         for (int i = 0; i < kLoads; ++i) {
-            const int block = i * 8 + wave;                       // 1 KiB: four rows of one part
-            const int p = block / (4 * MT), row = block % (4 * MT) * 4 + (lane >> 4);
-            const int k = k0 + p * kPiece + 8 * (((lane & 15) - row) & 15);
-            const void* src = k < n_in ? (const void*)(x + (int64_t)min(row, rows - 1) * n_in + k) : (const void*)&g_zero_piece;
-            __builtin_amdgcn_global_load_lds(NQH_GPTR(src), NQH_LPTR(s_x + buf * kBuf + block * 1024), 16, 0, 0);
+            const int block = i * NW + wave, p = block / (4 * MT), row = block % (4 * MT) * 4 + (lane >> 4);       // 1 KiB: four rows
+            const int end = t * KS + p < pieces ? n_in : 0;
+            const int k = (first + t * KS + p) * kPiece + 8 * (((lane & 15) - row) & 15);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, NQH_LPTR(buf + block * 1024), 16,
+                                                     k < end ? (uint32_t)(min(row, rows - 1) * n_in + k) * 2 : kOutside, 0, 0, 0);
         }
     };
     f32x4 acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    u32x4 cur[4], nxt[4];
-    stage(0, 0);
-    load_piece_clamped(cur, w_row, part * kPiece, hi, n_in);      // the activations are zero past the end
-    int buf = 0;
-    for (int k0 = 0; k0 < n_in; k0 += KS * kPiece) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's part of the stage and its weights have landed
-        __syncthreads();
-        if (k0 + KS * kPiece < n_in) {
-            load_piece_clamped(nxt, w_row, k0 + (KS + part) * kPiece, hi, n_in);
-            stage(k0 + KS * kPiece, buf ^ 1);
-        }
-        const unsigned char* base = s_x + buf * kBuf + part * kPart;
+    u32x4 f[kStageBufs][4];
+#pragma unroll
+    for (int t = 0; t < kAhead; ++t) {
+        load_x(t, t);
+        load_w(f[t], t);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_wave_barrier();
+    }
+    // stage t lies in buffer and registers `at`; `behind` stages have been asked for since
+    const auto landed = [&](auto behind) {
+        constexpr int c = behind * kStageLoads;
+        static_assert(c < 64, "what the counter holds");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (c & 15) | ((c >> 4) << 14));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const auto multiply = [&](const u32x4 (&cur)[4], int at) {
+        const unsigned char* base = s_x + at * kBuf + part * kPart + lo * 256;
 #pragma unroll
         for (int s = 0; s < 4; ++s)
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                const int row = 16 * m + lo;
-                const u32x4 xf = *reinterpret_cast<const u32x4*>(base + row * 256 + ((4 * s + hi + row) & 15) * 16);
+                const u32x4 xf = *reinterpret_cast<const u32x4*>(base + m * 4096 + ((4 * s + hi + lo) & 15) * 16);
                 acc[m] = Bf::mfma16(cur[s], xf, acc[m]);
             }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) cur[s] = nxt[s];
-        buf ^= 1;
+    };
+    int t = 0;
+#pragma unroll 1
+    for (; t + kStageBufs <= count; t += kStageBufs) {
+        each_of<kStageBufs>([&](auto u) {
+            landed(Int<kAhead - 1>());
+            load_x(t + u + kAhead, (u + kAhead) % kStageBufs);          // where everybody has read the stage before this one
+            load_w(f[(u + kAhead) % kStageBufs], t + u + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(f[u], u);
+        });
     }
-    __syncthreads();                          // the stages are read: their memory takes the parts' sums [part][nt][row][16]
-    float* sums = reinterpret_cast<float*>(s_x);
+    each_of<kAhead>([&](auto u) {
+        if (t + u >= count) return;
+        landed(Int<kAhead - 1 - u>());
+        multiply(f[u], u);
+    });
+    __builtin_amdgcn_s_waitcnt(0x0F70);       // what was asked for past the end has come: the LDS may be given back
+    if constexpr (KS > 1) {
+        __syncthreads();
+        float* sums = reinterpret_cast<float*>(s_x);
+        if (part > 0) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-        *reinterpret_cast<f32x4*>(sums + ((part * NT + nt) * 16 * MT + 16 * m + lo) * 16 + 4 * hi) = acc[m];
-    __syncthreads();
-    for (int i = threadIdx.x; i < NT * MT * 256; i += 512) {
-        const int j = i / (MT * 256), t = i / 16 % (16 * MT), n = n0 + 16 * j + (i & 15);
-        if (t >= rows || n >= n_out) continue;
-        float v = bias ? Bf::to_f32(bias[n]) : 0.f;
+            for (int m = 0; m < MT; ++m) *reinterpret_cast<f32x4*>(sums + (((part - 1) * NT + nt) * MT + m) * 256 + lane * 4) = acc[m];
+        }
+        __syncthreads();
+        if (part > 0) return;
 #pragma unroll
-        for (int p = 0; p < KS; ++p) v += sums[p * NT * MT * 256 + i];
-        v = activation_f32(v, act, param);
-        if constexpr (F32OUT) reinterpret_cast<float*>(y)[(int64_t)t * n_out + n] = v;
-        else reinterpret_cast<uint16_t*>(y)[(int64_t)t * n_out + n] = Bf::from_f32(v);
+        for (int p = 0; p < KS - 1; ++p)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m] += *reinterpret_cast<const f32x4*>(sums + ((p * NT + nt) * MT + m) * 256 + lane * 4);
+    }
+    const int n = n0 + 4 * hi;
+    if (n >= n_out) return;
+    const bool whole = n_out % 4 == 0 && ((uintptr_t)y & 15) == 0;        // a lane's four features: one aligned access
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int row = 16 * m + lo;
+        if (row >= rows) continue;
+        if constexpr (SPLIT) {
+            *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(y) + ((int64_t)row * gridDim.y + blockIdx.y) * n_out + n) = acc[m];
+        } else {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = activation_f32(acc[m][e] + (bias ? Bf::to_f32(bias[min(n + e, n_out - 1)]) : 0.f), act, param);
+            const int64_t at = (int64_t)row * n_out + n;
+            if (whole) {
+                if constexpr (F32OUT) store_vec<Fp, 4>(reinterpret_cast<float*>(y) + at, v);
+                else store_vec<Bf, 4>(reinterpret_cast<uint16_t*>(y) + at, v);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < n_out) {
+                        if constexpr (F32OUT) reinterpret_cast<float*>(y)[at + e] = v[e];
+                        else reinterpret_cast<uint16_t*>(y)[at + e] = Bf::from_f32(v[e]);
+                    }
+            }
+        }
     }
 }
 
-template <int MT, int NT>
-int launch_wide(const char* fn, const void* x, const void* w, const void* bias, void* y, int64_t rows, int64_t n_out,
-                int64_t n_in, int out_f32, int act, float param, void* stream) {
-    constexpr int lds = 2 * (8 / NT) * 16 * MT * 256;
-    const auto kernel = out_f32 ? wide_linear_kernel<MT, NT, true> : wide_linear_kernel<MT, NT, false>;
+// y = act(sum over the parts of the contraction (+ bias)): parts [rows, splits, n_out], four features a thread.
+template <bool F32OUT>
+__global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ parts, const uint16_t* __restrict__ bias,
+                                                        void* __restrict__ y, int n_out, int splits, int act, float param) {
+    const int n = (blockIdx.x * 256 + threadIdx.x) * 4, row = blockIdx.y;
+    if (n >= n_out) return;
+    const float* src = parts + (int64_t)row * splits * n_out + n;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s) {
+        const f32x4 p = *reinterpret_cast<const f32x4*>(src + (int64_t)s * n_out);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += p[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = activation_f32(v[e] + (bias ? Bf::to_f32(bias[n + e]) : 0.f), act, param);
+    const int64_t at = (int64_t)row * n_out + n;
+    if constexpr (F32OUT) store_vec<Fp, 4>(reinterpret_cast<float*>(y) + at, v);
+    else store_vec<Bf, 4>(reinterpret_cast<uint16_t*>(y) + at, v);
+}
+
+template <int MT, int NT, int KS, int kAhead, bool F32OUT, bool SPLIT>
+int launch_stream(const char* fn, const void* x, const void* w, const void* bias, void* y, int64_t rows, int64_t n_out, int64_t n_in,
+                  int act, float param, int64_t splits, hipStream_t stream) {
+    const int64_t each = cdiv(cdiv(n_in, kPiece), splits);
+    constexpr int lds = (kAhead + 1) * KS * 16 * MT * 256;
+    const auto kernel = stream_linear_kernel<MT, NT, KS, kAhead, F32OUT, SPLIT>;
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        static std::atomic<uint64_t> raised{0};          // the devices that this kernel may use so much LDS of
+        int device = 0;
+        hipError_t e = hipGetDevice(&device);
+        if (e == hipSuccess && (device > 63 || !(raised.load(std::memory_order_relaxed) >> device & 1))) {
+            e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (e == hipSuccess && device < 64) raised.fetch_or(1ull << device, std::memory_order_relaxed);
+        }
         if (e != hipSuccess) return fail(NQH_ERR_HIP, fn, "%s", hipGetErrorString(e));
     }
-    kernel<<<dim3((unsigned)cdiv(n_out, 16 * NT)), dim3(512), lds, (hipStream_t)stream>>>(
+    kernel<<<dim3((unsigned)cdiv(n_out, 16 * NT), (unsigned)splits), dim3(64 * NT * KS), lds, stream>>>(
+        (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y, (int)rows, (int)n_out, (int)n_in, act, param, (int)each);
+    return launched(fn);
+}
+
+// What a call runs: skinny_linear_kernel, or stream_linear_kernel with 2 (x 2 parts of a stage), 4 or 8 features tiles to a workgroup
+// and the contraction in `splits` parts.
+enum Form { kSkinny, kTwo, kFour, kEight };
+struct LinearPlan {
+    Form form;
+    int splits;
+};
+// Who may add the parts: nobody, sum_parts_kernel, the same where the host issues call after call, the reader of the result.
+enum class Sums { kNone, kOwnPass, kIssuedPass, kReader };
+
+// The least estimated time.  In us: a launch with its first data; what the fullest CU takes in (KB, at a rate of its own per form) and
+// the weights from memory (MB), the root of the sum of their squares; parts written, and read by a pass of their own or by a reader
+// whose row is one workgroup.  A pass that the host issues takes its 8 us, by which prompts of 40 tokens through small layers were 5 to
+// 12 % longer.  Fitted to 32 weights (544 to 32768 x 1024 to 18432) at 1 to 64 rows, every form and split, from
+// memory: 3.6 % off in the middle, 9.5 % in one of ten; the chosen form takes 0.4 % (nobody adds), 1.6 % (own pass) and 1.1 % (reader)
+// longer than the fastest on average, 16 % at worst.  Long contractions and, the other way, few rows of many features are
+// where skinny_linear_kernel is off the estimate.
+LinearPlan make_linear_plan(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
+    struct Of {
+        double launch, memory, rate, more;       // us, MB/us, KB/us for one tile of rows and so many more for four
+        int tiles, parts;
+    };
+    static constexpr Of kOf[] = {{2.95, 7.95, 30.7, 5.6, 1, 1}, {2.67, 7.05, 48.1, 0, 2, 2}, {2.62, 7.15, 44.0, 3.3, 4, 1}, {3.02, 8.0, 39.8, 2.1, 8, 1}};
+    const auto hypot2 = [](double a, double b) { return std::sqrt(a * a + b * b); };
+    const double mb = 2e-6 * n_out * n_in;
+    const int64_t groups = cdiv(n_out, 16) * cdiv(rows, 16), few = std::min<int64_t>(rows, 16), pieces = cdiv(n_in, kPiece);
+    LinearPlan best{kSkinny, 1};
+    double least = kOf[0].launch + hypot2(cdiv(groups, 256) * n_in * 2e-3 * (16 + few) / (kOf[0].rate + kOf[0].more * few / 16), mb / kOf[0].memory);
+    if (rows <= 4 && n_out >= 16384) least *= 0.93;
+    if (n_in >= 8192) least *= 1.12;
+    if (n_in > (1 << 24)) return best;             // 32-bit offsets into 16 rows of the weight and all of x
+    const int mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+    for (const Form form : {kTwo, kFour, kEight}) {
+        if (form == kEight && mt == 1) continue;
+        const Of& of = kOf[form];
+        const int64_t columns = cdiv(n_out, 16 * of.tiles);
+        const double rate = of.rate + of.more * (mt - 1) / 3;
+        for (int64_t s = 1; s <= 16; ++s) {
+            const int64_t each = cdiv(pieces, s);
+            if (s > 1 && (sums == Sums::kNone || n_out % 4 != 0 || each < 2 || columns * s > 1024)) break;
+            if (cdiv(pieces, each) != s) continue;             // the last part would be empty
+            double us = of.launch + hypot2(cdiv(columns * s, 256) * cdiv(each, of.parts) * of.parts * 4.096 * (of.tiles + mt) / rate, mb / of.memory);
+            if (s > 1) {
+                const double parts = 4e-6 * s * rows * n_out;
+                us += parts / 3.2 + (sums == Sums::kReader ? 0.3 + 4e-3 * s * n_out / 60 : parts / 6 + (sums == Sums::kOwnPass ? 2.65 : 8));
+            }
+            if (us < least) least = us, best = {form, (int)s};
+        }
+    }
+    return best;
+}
+
+// The same, remembered: some 50 estimates take the host 3 us, as long as a launch.
+LinearPlan plan_linear(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
+    struct Entry {
+        int64_t rows, n_out, n_in;
+        Sums sums;
+        LinearPlan plan;
+    };
+    thread_local Entry kept[64] = {};                  // rows 0: empty
+    Entry& e = kept[(uint64_t)(n_out * 31 + n_in * 7 + rows * 3 + (int)sums) * 0x9E3779B97F4A7C15ull >> 58];
+    if (e.rows != rows || e.n_out != n_out || e.n_in != n_in || e.sums != sums)
+        e = {rows, n_out, n_in, sums, make_linear_plan(rows, n_out, n_in, sums)};
+    return e.plan;
+}
+
+size_t parts_bytes(LinearPlan plan, int64_t rows, int64_t n_out) {
+    return plan.splits > 1 ? (size_t)plan.splits * rows * n_out * sizeof(float) : 0;
+}
+
+int run_skinny(const char* fn, const void* x, const void* w, const void* bias, void* y, int64_t rows, int64_t n_out, int64_t n_in,
+               int out_f32, int act, float param, hipStream_t stream) {
+    const int64_t groups = cdiv(n_out, 16);
+    const int waves = skinny_waves(groups * cdiv(rows, 16), n_in);
+    const size_t lds = (size_t)waves * 256 * sizeof(float);
+    const auto kernel = out_f32 ? skinny_linear_kernel<true> : skinny_linear_kernel<false>;
+    kernel<<<dim3((unsigned)groups, (unsigned)cdiv(rows, 16)), dim3((unsigned)waves * 64), lds, stream>>>(
         (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y, (int)rows, (int)n_out, (int)n_in, act, param);
     return launched(fn);
+}
+
+// The product as planned; with parts y takes their sums.
+int run_plan(const char* fn, LinearPlan plan, const void* x, const void* w, const void* bias, void* y, int64_t rows, int64_t n_out,
+             int64_t n_in, int out_f32, int act, float param, hipStream_t stream) {
+    if (plan.form == kSkinny) return run_skinny(fn, x, w, bias, y, rows, n_out, n_in, out_f32, act, param, stream);
+    const auto go = [&](auto mt, auto nt, auto ks, auto ahead) {
+        if (plan.splits > 1)
+            return launch_stream<mt, nt, ks, ahead, true, true>(fn, x, w, bias, y, rows, n_out, n_in, act, param, plan.splits, stream);
+        return out_f32 ? launch_stream<mt, nt, ks, ahead, true, false>(fn, x, w, bias, y, rows, n_out, n_in, act, param, 1, stream)
+                       : launch_stream<mt, nt, ks, ahead, false, false>(fn, x, w, bias, y, rows, n_out, n_in, act, param, 1, stream);
+    };
+    const auto of_rows = [&](auto mt) {
+        if (plan.form == kTwo) return go(mt, Int<2>(), Int<2>(), Int<2>());
+        if constexpr (mt > 1)
+            if (plan.form == kEight) return go(mt, Int<8>(), Int<1>(), Int<3>());
+        return go(mt, Int<4>(), Int<1>(), Int<3>());
+    };
+    return rows <= 16 ? of_rows(Int<1>()) : rows <= 32 ? of_rows(Int<2>()) : of_rows(Int<4>());
+}
+
+bool skinny_takes(int64_t rows, int64_t n_out, int64_t n_in) {
+    return rows > 0 && rows <= 64 && n_out > 0 && n_in > 0 && n_in % 8 == 0 && n_out <= kMaxI32 - 16 && n_in <= (1 << 30);
 }
 
 // ---- many rows: activation(x @ weight^T) on the tiles of pingpong.hpp -------------------------------------------------
@@ -201,39 +417,56 @@ int dense_activation_tile(int64_t rows, int64_t n_out, int64_t n_in) {
 
 using namespace nqh;
 
-extern "C" int nqh_skinny_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows,
-                                 int64_t out_features, int64_t in_features, int out_f32, int act, float param,
-                                 void* stream) {
-    const char* fn = "nqh_skinny_linear";
-    if (!x || !weight || !y || !aligned(x, 16) || !aligned(weight, 16))
+extern "C" int64_t nqh_skinny_linear_parts(int64_t rows, int64_t out_features, int64_t in_features) {
+    return skinny_takes(rows, out_features, in_features) ? plan_linear(rows, out_features, in_features, Sums::kReader).splits : 1;
+}
+
+extern "C" int nqh_skinny_linear_sums(const void* x, const void* weight, float* sums, int64_t rows, int64_t out_features,
+                                      int64_t in_features, void* stream) {
+    const char* fn = "nqh_skinny_linear_sums";
+    if (!x || !weight || !sums || !aligned(x, 16) || !aligned(weight, 16) || !aligned(sums, 16))
         return fail(NQH_ERR_ARG, fn, "null or misaligned pointer");
-    if (rows <= 0 || rows > 64 || out_features <= 0 || in_features <= 0 || in_features % 8 != 0 ||
-        out_features > kMaxI32 - 16 || in_features > (1 << 30))
+    if (!skinny_takes(rows, out_features, in_features))
+        return fail(NQH_ERR_ARG, fn, "1 to 64 rows and an in_features that is a multiple of 8");
+    (void)hipGetLastError();
+    return run_plan(fn, plan_linear(rows, out_features, in_features, Sums::kReader), x, weight, nullptr, sums, rows, out_features,
+                    in_features, 1, NQH_ACT_NONE, 0.f, (hipStream_t)stream);
+}
+
+extern "C" size_t nqh_skinny_linear_scratch_bytes(int64_t rows, int64_t out_features, int64_t in_features, int captured) {
+    if (!skinny_takes(rows, out_features, in_features) ||
+        plan_linear(rows, out_features, in_features, captured ? Sums::kOwnPass : Sums::kIssuedPass).splits == 1)
+        return 0;
+    return parts_bytes(plan_linear(rows, out_features, in_features, Sums::kOwnPass), rows, out_features);
+}
+
+extern "C" int nqh_skinny_linear_ex(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
+                                    int64_t in_features, int out_f32, int act, float param, void* scratch, size_t scratch_bytes,
+                                    void* stream) {
+    const char* fn = "nqh_skinny_linear";
+    if (!x || !weight || !y || !aligned(x, 16) || !aligned(weight, 16) || !aligned(scratch, 16))
+        return fail(NQH_ERR_ARG, fn, "null or misaligned pointer");
+    if (!skinny_takes(rows, out_features, in_features))
         return fail(NQH_ERR_ARG, fn, "1 to 64 rows and an in_features that is a multiple of 8");
     if (act < NQH_ACT_NONE || act > NQH_ACT_SOFTCAP || (act == NQH_ACT_SOFTCAP && !(param > 0.f)))
         return fail(NQH_ERR_ARG, fn, "unknown activation, or a cap that is not positive");
     (void)hipGetLastError();
-    if (rows > 16 && out_features > 1024) {
-        const bool narrow = out_features <= 8192;      // fewer features per workgroup: more workgroups
-        if (rows <= 32)
-            return narrow ? launch_wide<2, 2>(fn, x, weight, bias, y, rows, out_features, in_features, out_f32, act, param, stream)
-                          : launch_wide<2, 4>(fn, x, weight, bias, y, rows, out_features, in_features, out_f32, act, param, stream);
-        return narrow ? launch_wide<4, 2>(fn, x, weight, bias, y, rows, out_features, in_features, out_f32, act, param, stream)
-                      : launch_wide<4, 4>(fn, x, weight, bias, y, rows, out_features, in_features, out_f32, act, param, stream);
-    }
-    const int64_t groups = cdiv(out_features, 16);
-    const int waves = skinny_waves(groups * cdiv(rows, 16), in_features);
-    const size_t lds = (size_t)waves * 256 * sizeof(float);
-    const dim3 grid((unsigned)groups, (unsigned)cdiv(rows, 16)), block((unsigned)waves * 64);
-    if (out_f32)
-        skinny_linear_kernel<true><<<grid, block, lds, (hipStream_t)stream>>>(
-            (const uint16_t*)x, (const uint16_t*)weight, (const uint16_t*)bias, y, (int)rows, (int)out_features, (int)in_features,
-            act, param);
-    else
-        skinny_linear_kernel<false><<<grid, block, lds, (hipStream_t)stream>>>(
-            (const uint16_t*)x, (const uint16_t*)weight, (const uint16_t*)bias, y, (int)rows, (int)out_features, (int)in_features,
-            act, param);
+    const hipStream_t st = (hipStream_t)stream;
+    LinearPlan plan = plan_linear(rows, out_features, in_features, scratch && aligned(y, 16) ? Sums::kOwnPass : Sums::kNone);
+    if (scratch_bytes < parts_bytes(plan, rows, out_features)) plan = plan_linear(rows, out_features, in_features, Sums::kNone);
+    if (plan.splits == 1) return run_plan(fn, plan, x, weight, bias, y, rows, out_features, in_features, out_f32, act, param, st);
+    const int rc = run_plan(fn, plan, x, weight, nullptr, scratch, rows, out_features, in_features, 1, NQH_ACT_NONE, 0.f, st);
+    if (rc != 0) return rc;
+    const auto kernel = out_f32 ? sum_parts_kernel<true> : sum_parts_kernel<false>;
+    kernel<<<dim3((unsigned)cdiv(out_features, 1024), (unsigned)rows), dim3(256), 0, st>>>(
+        (const float*)scratch, (const uint16_t*)bias, y, (int)out_features, plan.splits, act, param);
     return launched(fn);
+}
+
+extern "C" int nqh_skinny_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows,
+                                 int64_t out_features, int64_t in_features, int out_f32, int act, float param,
+                                 void* stream) {
+    return nqh_skinny_linear_ex(x, weight, bias, y, rows, out_features, in_features, out_f32, act, param, nullptr, 0, stream);
 }
 
 // 1 where the tiles are one round of the 256 CUs and estimated to take less time than the library's product and the activation's pass

@@ -1,6 +1,8 @@
 // Shared device/host helpers of the hybrid-decoder kernels (libnq_hybrid.so).
 #pragma once
 
+#include <type_traits>
+
 #include "../awq_common.hpp"
 #include "../../../include/nq_hybrid_ops.h"
 
@@ -86,6 +88,41 @@ __device__ __forceinline__ void store_vec(typename T::elem* p, const float (&f)[
 #pragma unroll
         for (int i = 0; i < V; ++i) T::store(p + i, f[i]);
     }
+}
+
+template <int I>
+using Int = std::integral_constant<int, I>;
+
+// What a sublayer leaves: the sum of `parts` rows `stride` apart, of the call's type or, where it is the sums of a split contraction,
+// fp32.  V consecutive elements from element `at` on; `sum` comes in as zeros.
+struct Parts {
+    const void* y;
+    int parts, f32;
+};
+template <typename T, int V>
+__device__ __forceinline__ void load_parts(const Parts& y, int64_t at, int stride, float (&sum)[V]) {
+    const auto add = [&](auto type) {
+        using E = decltype(type);
+        const typename E::elem* p = reinterpret_cast<const typename E::elem*>(y.y) + at;
+        int j = 0;
+        const auto some = [&](auto n) {              // n of them in flight
+            float t[n][V];
+#pragma unroll
+            for (int u = 0; u < n; ++u) load_vec<E, V>(p + (int64_t)(j + u) * stride, t[u]);
+#pragma unroll
+            for (int u = 0; u < n; ++u)
+#pragma unroll
+                for (int e = 0; e < V; ++e) sum[e] += t[u][e];
+            j += n;
+        };
+#pragma unroll 1
+        while (j + 4 <= y.parts) some(Int<4>());
+        if (j + 2 <= y.parts) some(Int<2>());
+        if (j < y.parts) some(Int<1>());
+    };
+    if (y.parts == 1 && !y.f32) load_vec<T, V>(reinterpret_cast<const typename T::elem*>(y.y) + at, sum);     // straight into place
+    else if (y.f32) add(Fp());
+    else add(T());
 }
 
 // V = 4 consecutive elements as they lie in memory, to be fetched early and unpacked late.

@@ -13,7 +13,7 @@ constexpr int kMaxWidth = 8192;
 template <typename T, int S, int V, int THREADS, int P>
 __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
     float* __restrict__ x, const int64_t* __restrict__ ids, const typename T::elem* __restrict__ table, int64_t table_rows,
-    const typename T::elem* __restrict__ y, const typename T::elem* __restrict__ mix, const typename T::elem* __restrict__ w_out,
+    Parts y, const typename T::elem* __restrict__ mix, const typename T::elem* __restrict__ w_out,
     const typename T::elem* __restrict__ w_in, const typename T::elem* __restrict__ norm_w, typename T::elem* __restrict__ h,
     int streams, int width, float eps) {
     constexpr int WAVES = THREADS / 64;
@@ -43,8 +43,8 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
                 for (int s = 0; s < S; ++s)
                     if (s < streams) load_vec<Fp, V>(xr + (int64_t)s * width + i, v[s][p]);
             }
-            if (y) load_vec<T, V>(y + row * width + i, yv[p]);
             if (h) load_vec<T, V>(norm_w + i, wn[p]);
+            if (y.y) load_parts<T, V>(y, row * y.parts * width + i, width, yv[p]);
         }
     }
     float win[S];
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
 #pragma unroll
                 for (int e = 0; e < V; ++e) v[s][p][e] = v[0][p][e];
     }
-    if (y) {
+    if (y.y) {
         float m[S][S], wo[S];
 #pragma unroll
         for (int t = 0; t < S; ++t) {
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const int i = (p * THREADS + threadIdx.x) * V;
-        if (i < width && (y || ids)) {
+        if (i < width && (y.y || ids)) {
 #pragma unroll
             for (int s = 0; s < S; ++s)
                 if (s < streams) store_vec<Fp, V>(xr + (int64_t)s * width + i, v[s][p]);
@@ -112,13 +112,13 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
 }
 
 template <typename T, int S>
-void launch_hyper(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y, const void* mix,
+void launch_hyper(float* x, const int64_t* ids, const void* table, int64_t table_rows, Parts y, const void* mix,
                   const void* w_out, const void* w_in, const void* norm_w, void* h, int64_t rows, int64_t streams,
                   int64_t width, float eps, bool vec, hipStream_t st) {
     using E = typename T::elem;
 #define NQH_GO(V, THREADS, P)                                                                                              \
     hyper_norm_kernel<T, S, V, THREADS, P><<<dim3((unsigned)rows), dim3(THREADS), 0, st>>>(                                \
-        x, ids, (const E*)table, table_rows, (const E*)y, (const E*)mix, (const E*)w_out, (const E*)w_in, (const E*)norm_w, \
+        x, ids, (const E*)table, table_rows, y, (const E*)mix, (const E*)w_out, (const E*)w_in, (const E*)norm_w, \
         (E*)h, (int)streams, (int)width, eps)
     if (!vec) NQH_GO(1, 1024, 8);
     else if (width <= 1024) NQH_GO(4, 256, 1);
@@ -147,21 +147,23 @@ using namespace nqh;
 
 extern "C" int64_t nqh_hyper_max_streams(void) { return kMaxStreams; }
 
-extern "C" int nqh_hyper_norm(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y,
-                              const void* mix, const void* w_out, const void* w_in, const void* norm_weight, void* h,
-                              int64_t rows, int64_t streams, int64_t width, float eps, int dtype, void* stream) {
+extern "C" int nqh_hyper_norm_parts(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y,
+                                    int64_t y_parts, const void* mix, const void* w_out, const void* w_in, const void* norm_weight,
+                                    void* h, int64_t rows, int64_t streams, int64_t width, float eps, int dtype, void* stream) {
     const char* fn = "nqh_hyper_norm";
+    const int y_f32 = (dtype & NQH_Y_F32) != 0;
+    dtype &= ~NQH_Y_F32;
     if (!x || (ids && (!table || table_rows <= 0)) || (y && (!mix || !w_out)) || (h && !norm_weight))
         return fail(NQH_ERR_ARG, fn, "null pointer");
     if (!dtype_ok(dtype)) return fail(NQH_ERR_ARG, fn, "dtype must be NQH_BF16 or NQH_F32");
-    if (rows <= 0 || rows > kMaxI32 || width <= 0 || streams <= 0) return fail(NQH_ERR_ARG, fn, "sizes must be positive");
+    if (rows <= 0 || rows > kMaxI32 || width <= 0 || streams <= 0 || (y && (y_parts <= 0 || y_parts > kMaxI32))) return fail(NQH_ERR_ARG, fn, "sizes must be positive");
     if (width > kMaxWidth || streams > kMaxStreams)
         return fail(NQH_ERR_UNSUPPORTED, fn, "at most width %d and %d streams", kMaxWidth, kMaxStreams);
     const bool vec = width % 4 == 0 && aligned(x, 16) && aligned(y, 16) && aligned(table, 16) && aligned(norm_weight, 16) &&
                      aligned(h, 16);
     (void)hipGetLastError();
 #define NQH_STREAMS(S) \
-    launch_hyper<T, S>(x, ids, table, table_rows, y, mix, w_out, w_in, norm_weight, h, rows, streams, width, eps, vec, (hipStream_t)stream)
+    launch_hyper<T, S>(x, ids, table, table_rows, Parts{y, (int)y_parts, y_f32}, mix, w_out, w_in, norm_weight, h, rows, streams, width, eps, vec, (hipStream_t)stream)
     NQH_WITH_TYPE(dtype, {
         if (streams == 1) NQH_STREAMS(1);
         else if (streams == 2) NQH_STREAMS(2);
@@ -170,6 +172,13 @@ extern "C" int nqh_hyper_norm(float* x, const int64_t* ids, const void* table, i
     });
 #undef NQH_STREAMS
     return launched(fn);
+}
+
+extern "C" int nqh_hyper_norm(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y,
+                              const void* mix, const void* w_out, const void* w_in, const void* norm_weight, void* h,
+                              int64_t rows, int64_t streams, int64_t width, float eps, int dtype, void* stream) {
+    return nqh_hyper_norm_parts(x, ids, table, table_rows, y, 1, mix, w_out, w_in, norm_weight, h, rows, streams, width, eps, dtype,
+                                stream);
 }
 
 extern "C" int nqh_activate(void* x, int64_t count, int act, float param, int dtype, void* stream) {

@@ -24,8 +24,7 @@ struct RouteArgs {
 
 template <typename T, int V, int THREADS, int P, bool ROUTED>
 __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
-    float* __restrict__ x, int init, const typename T::elem* __restrict__ y, int parts,
-    const typename T::elem* __restrict__ post_w, const int64_t* __restrict__ ids,
+    float* __restrict__ x, int init, Parts y, const typename T::elem* __restrict__ post_w, const int64_t* __restrict__ ids,
     const typename T::elem* __restrict__ table, int64_t table_rows, const typename T::elem* __restrict__ next_w,
     typename T::elem* __restrict__ h, int width, float eps, RouteArgs route) {
     constexpr int WAVES = THREADS / 64;
@@ -58,7 +57,7 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
             if (h) load_vec<T, V>(next_w + i, wn[p]);
         }
     }
-    if (y) {
+    if (y.y) {
         float s[P][V], ss = 0.f;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
@@ -66,13 +65,7 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
 #pragma unroll
             for (int e = 0; e < V; ++e) s[p][e] = 0.f;
             if (i < width) {
-#pragma unroll 2
-                for (int j = 0; j < parts; ++j) {
-                    float t[V];
-                    load_vec<T, V>(y + (row * parts + j) * width + i, t);
-#pragma unroll
-                    for (int e = 0; e < V; ++e) s[p][e] += t[e];
-                }
+                load_parts<T, V>(y, row * y.parts * width + i, width, s[p]);
 #pragma unroll
                 for (int e = 0; e < V; ++e) ss += s[p][e] * s[p][e];
             }
@@ -369,12 +362,14 @@ static bool residual_vec(const void* x, const void* y, const void* post_weight, 
 }
 
 #define NQH_ARGS                                                                                                          \
-    x, init, (const E*)y, (int)y_parts, (const E*)post_weight, ids, (const E*)table, table_rows, (const E*)next_weight,   \
+    x, init, Parts{y, (int)y_parts, y_f32}, (const E*)post_weight, ids, (const E*)table, table_rows, (const E*)next_weight,   \
         (E*)h, (int)width, eps
 extern "C" int nqh_residual_norm(float* x, int init, const void* y, int64_t y_parts, const void* post_weight,
                                  const int64_t* ids, const void* table, int64_t table_rows, const void* next_weight,
                                  void* h, int64_t rows, int64_t width, float eps, int dtype, void* stream) {
     const char* fn = "nqh_residual_norm";
+    const int y_f32 = (dtype & NQH_Y_F32) != 0;
+    dtype &= ~NQH_Y_F32;
     const int rc = check_residual(fn, x, y, y_parts, ids, table, table_rows, next_weight, h, rows, width, dtype);
     if (rc != NQH_OK) return rc;
     const bool vec = residual_vec(x, y, post_weight, table, next_weight, h, width);
@@ -407,6 +402,8 @@ extern "C" int nqh_residual_norm_route(float* x, int init, const void* y, int64_
                                        int64_t top, int64_t tile_rows, int64_t max_tiles, float eps, int dtype,
                                        void* stream) {
     const char* fn = "nqh_residual_norm_route";
+    const int y_f32 = (dtype & NQH_Y_F32) != 0;
+    dtype &= ~NQH_Y_F32;
     const int rc = check_residual(fn, x, y, y_parts, ids, table, table_rows, next_weight, h, rows, width, dtype);
     if (rc != NQH_OK) return rc;
     if (!h || !router || !expert || !weight || !order || !tiles || !counter) return fail(NQH_ERR_ARG, fn, "null pointer");

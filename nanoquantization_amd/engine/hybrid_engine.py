@@ -168,6 +168,10 @@ class HybridEngine(EngineCore):
         y = F.linear(x, w, b)
         return y if activation is None else ops.activate_(y, activation, param)
 
+    def _sublayer_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """The product that ends a sublayer: of few rows as sums of its parts, which the residual's next read adds."""
+        return ops.skinny_linear_sums(x, w) if ops.skinny_linear_supported(x.shape[0], w) else F.linear(x, w)
+
     def _logits(self, h: torch.Tensor) -> torch.Tensor:
         """fp32 logits of normalised rows."""
         w, cap = self.model.head, self.spec.logit_cap
@@ -251,10 +255,10 @@ class HybridEngine(EngineCore):
                 res.add_embedding()
             h = res.read(layer.norm_mixer, layer.mixer_streams)
             o = self._MIXERS[type(ls.mixer)](self, run, ls.mixer, layer.mixer, h, step)
-            res.write(self._linear(o, layer.mixer.out), layer.norm_mixer_out, layer.mixer_streams)
+            res.write(self._sublayer_linear(o, layer.mixer.out), layer.norm_mixer_out, layer.mixer_streams)
             if isinstance(ls.mlp, DenseSpec):
                 h = res.read(layer.norm_mlp, layer.mlp_streams)
-                y = self._linear(self._linear(h, layer.mlp.up, activation=ls.mlp.activation), layer.mlp.down)
+                y = self._sublayer_linear(self._linear(h, layer.mlp.up, activation=ls.mlp.activation), layer.mlp.down)
                 res.write(y, layer.norm_mlp_out, layer.mlp_streams)
             elif ls.mlp is not None:
                 h, routing = res.read_routed(layer.norm_mlp, layer.mlp.router, ls.mlp.top, ls.mlp.ff)

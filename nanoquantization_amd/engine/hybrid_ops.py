@@ -4,6 +4,7 @@ Each function checks shapes on the host, allocates its output with torch (graph-
 and launches on the current stream.  HIP device tensors only; bfloat16 or float32."""
 from __future__ import annotations
 
+import functools
 from typing import Optional, Sequence, Tuple
 
 import numpy as np
@@ -13,6 +14,7 @@ from .. import _lib
 from .cache import upload
 
 _DTYPES = {torch.bfloat16: 1, torch.float32: 2}
+_Y_F32 = 4                          # added to a dtype: the sublayer's output is fp32 sums (skinny_linear_sums)
 SKINNY_ROWS = 64
 ACTIVATIONS = {None: 0, "relu2": 1, "softcap": 2}      # what may follow a product; "softcap" takes the cap as parameter
 
@@ -66,23 +68,30 @@ def _call(dev: torch.device, fn: str, *args) -> None:
         _lib.check_hybrid(getattr(_lib.hybrid_lib(), fn)(*args, _lib.current_stream_ptr(dev)))
 
 
+def _sublayer_output(y, others, rows, width, dtype=None):
+    """(dtype of the call, parts of y): y [rows, width] or [rows, parts, width] is of the other operands' type or, as the sums of a split
+    product, fp32."""
+    dt = others[0].dtype if others else dtype if y is None else y.dtype
+    assert all(t.dtype == dt for t in others)
+    if y is None:
+        return dt, 1
+    assert y.dim() in (2, 3) and y.shape[0] == rows and y.shape[-1] == width
+    assert y.dtype == dt or (y.dtype == torch.float32 and y.dim() == 3)
+    return dt, 1 if y.dim() == 2 else y.shape[1]
+
+
 def _residual_args(x, eps, y, post_weight, ids, table, init, next_weight, dtype):
     dev = _dev(x, y, post_weight, ids, table, next_weight)
     rows, width = x.shape
     assert x.dtype == torch.float32
-    operands = [t for t in (y, post_weight, table, next_weight) if t is not None]
-    dt = operands[0].dtype if operands else dtype
-    assert all(t.dtype == dt for t in operands)
-    parts = 1
-    if y is not None:
-        parts = 1 if y.dim() == 2 else y.shape[1]
-        assert y.shape[0] == rows and y.shape[-1] == width
+    others = [t for t in (post_weight, table, next_weight) if t is not None]
+    dt, parts = _sublayer_output(y, others, rows, width, dtype)
     assert post_weight is None or post_weight.shape == (width,)
     assert next_weight is None or next_weight.shape == (width,)
     if ids is not None:
         assert ids.dtype == torch.int64 and ids.numel() == rows and table.shape[1] == width
     h = torch.empty(rows, width, dtype=dt, device=dev) if next_weight is not None else None
-    return dev, h, dt, (x.data_ptr(), int(init), _ptr(y), parts, _ptr(post_weight), _ptr(ids), _ptr(table),
+    return dev, h, _DTYPES[dt] | (_Y_F32 if y is not None and y.dtype != dt else 0), (x.data_ptr(), int(init), _ptr(y), parts, _ptr(post_weight), _ptr(ids), _ptr(table),
                         0 if table is None else table.shape[0], _ptr(next_weight), _ptr(h))
 
 
@@ -92,7 +101,7 @@ def residual_norm(x: torch.Tensor, eps: float, *, y: Optional[torch.Tensor] = No
     """The fp32 residual stream x [rows, width] IN PLACE: (0 if init) + RMSNorm(sum over parts of y [rows, parts, width]) *
     post_weight + table[ids]; returns RMSNorm(x) * next_weight (None without next_weight)."""
     dev, h, dt, args = _residual_args(x, eps, y, post_weight, ids, table, init, next_weight, dtype)
-    _call(dev, "nqh_residual_norm", *args, *x.shape, eps, _DTYPES[dt])
+    _call(dev, "nqh_residual_norm", *args, *x.shape, eps, dt)
     return h
 
 
@@ -100,21 +109,20 @@ def hyper_norm(x: torch.Tensor, eps: float, *, ids: Optional[torch.Tensor] = Non
                y: Optional[torch.Tensor] = None, mix: Optional[torch.Tensor] = None, write: Optional[torch.Tensor] = None,
                read: Optional[torch.Tensor] = None, next_weight: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """The fp32 residual streams x [rows, streams, width] IN PLACE: all set to table[ids], or mixed anew from the old ones
-    and a sublayer's output y; returns RMSNorm(sum of the streams times read, or of the streams as they are) * next_weight
+    and a sublayer's output y (or the sum over the parts of y [rows, parts, width]); returns RMSNorm(sum of the streams times read, or of the streams as they are) * next_weight
     (None without next_weight)."""
     dev = _dev(x, ids, table, y, mix, write, read, next_weight)
     rows, streams, width = x.shape
     assert x.dtype == torch.float32
-    operands = [t for t in (table, y, mix, write, read, next_weight) if t is not None]
-    dt = operands[0].dtype
-    assert all(t.dtype == dt for t in operands)
+    dt, parts = _sublayer_output(y, [t for t in (table, mix, write, read, next_weight) if t is not None], rows, width)
     assert ids is None or (y is None and ids.dtype == torch.int64 and ids.numel() == rows and table.shape[1] == width)
-    assert y is None or (y.shape == (rows, width) and mix.shape == (streams, streams) and write.shape == (streams,))
+    assert y is None or (mix.shape == (streams, streams) and write.shape == (streams,))
     assert read is None or read.shape == (streams,)
     assert next_weight is None or next_weight.shape == (width,)
     h = torch.empty(rows, width, dtype=dt, device=dev) if next_weight is not None else None
-    _call(dev, "nqh_hyper_norm", x.data_ptr(), _ptr(ids), _ptr(table), 0 if table is None else table.shape[0], _ptr(y),
-          _ptr(mix), _ptr(write), _ptr(read), _ptr(next_weight), _ptr(h), rows, streams, width, eps, _DTYPES[dt])
+    _call(dev, "nqh_hyper_norm_parts", x.data_ptr(), _ptr(ids), _ptr(table), 0 if table is None else table.shape[0], _ptr(y), parts,
+          _ptr(mix), _ptr(write), _ptr(read), _ptr(next_weight), _ptr(h), rows, streams, width, eps,
+          _DTYPES[dt] | (_Y_F32 if y is not None and y.dtype != dt else 0))
     return h
 
 
@@ -152,11 +160,11 @@ def residual_norm_route(x: torch.Tensor, eps: float, router: torch.Tensor, top: 
         return h, route(h, router, top, ff)
     dev, h, dt, args = _residual_args(x, eps, y, post_weight, ids, table, init, next_weight, None)
     _dev(router)
-    r = Routing(rows, experts, top, width, ff, _DTYPES[dt], dev)
+    r = Routing(rows, experts, top, width, ff, dt & ~_Y_F32, dev)
     counter = _lib.workspace(dev, _lib.current_stream_ptr(dev), 4)       # zero between launches; see _lib.workspace
     _call(dev, "nqh_residual_norm_route", *args, router.data_ptr(), r.expert.data_ptr(), r.weight.data_ptr(),
           r.order.data_ptr(), r.tiles.data_ptr(), counter.data_ptr(), rows, width, experts, top, r.tile_rows, r.max_tiles,
-          eps, _DTYPES[dt])
+          eps, dt)
     return h, r
 
 
@@ -615,6 +623,12 @@ def moe_experts(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, r: R
     return y
 
 
+@functools.lru_cache(maxsize=4096)
+def _of_sizes(fn: str, *sizes: int) -> int:
+    """What an entry of the library says of sizes alone, remembered."""
+    return getattr(_lib.hybrid_lib(), fn)(*sizes)
+
+
 def skinny_linear_supported(rows: int, weight: torch.Tensor) -> bool:
     return 1 <= rows <= SKINNY_ROWS and weight.dtype == torch.bfloat16 and weight.shape[1] % 8 == 0
 
@@ -627,9 +641,23 @@ def skinny_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
     assert weight.shape[1] == n and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
     assert bias is None or (bias.shape == (weight.shape[0],) and bias.dtype == torch.bfloat16)
     y = torch.empty(rows, weight.shape[0], dtype=torch.float32 if out_f32 else torch.bfloat16, device=dev)
-    _call(dev, "nqh_skinny_linear", x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), rows, weight.shape[0], n,
-          int(out_f32), ACTIVATIONS[activation], param)
+    nbytes = _of_sizes("nqh_skinny_linear_scratch_bytes", rows, weight.shape[0], n, int(torch.cuda.is_current_stream_capturing()))
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    _call(dev, "nqh_skinny_linear_ex", x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), rows, weight.shape[0], n,
+          int(out_f32), ACTIVATIONS[activation], param, _ptr(scratch), nbytes)
     return y
+
+
+def skinny_linear_sums(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """x [rows <= 64, in] bf16 @ weight [out, in]^T for a reader that adds: fp32 [rows, parts, out], the sums of as many parts of the
+    contraction as keep the GPU busy."""
+    dev = _dev(x, weight)
+    rows, n = x.shape
+    assert weight.shape[1] == n and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+    parts = _of_sizes("nqh_skinny_linear_parts", rows, weight.shape[0], n)
+    sums = torch.empty(rows, parts, weight.shape[0], dtype=torch.float32, device=dev)
+    _call(dev, "nqh_skinny_linear_sums", x.data_ptr(), weight.data_ptr(), sums.data_ptr(), rows, weight.shape[0], n)
+    return sums
 
 
 def dense_activation_wanted(x: torch.Tensor, weight: torch.Tensor) -> bool:

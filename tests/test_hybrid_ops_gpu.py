@@ -503,6 +503,52 @@ def test_skinny_linear(rows, n_out, n_in):
     close(ops.skinny_linear(x.cuda(), w.cuda(), b.cuda()), want + b.double(), torch.bfloat16)
 
 
+# every tile height and workgroup width, whole and split contractions, ends inside a stage, a wave's features, a workgroup; what a
+# former launch left in LDS (NaN here) reaches nothing.  Bounds as for any fp32 sum of these lengths: `close`
+@pytest.mark.parametrize("rows,n_out,n_in", [(1, 64, 8), (5, 132, 1000), (16, 2048, 2048), (16, 544, 4096), (17, 1028, 136), (20, 4608, 1024),
+                                             (32, 2052, 9224), (33, 4096, 4608), (64, 4100, 2056), (64, 12288, 1024), (40, 1030, 520),
+                                             (64, 18432, 2048)])
+def test_skinny_linear_parts(rows, n_out, n_in):
+    print(f"skinny parts {rows} x {n_in} -> {n_out}", flush=True)
+    x, w, b = (rand(*s, seed=i, dtype=torch.bfloat16) for i, s in enumerate([(rows, n_in), (n_out, n_in), (n_out,)]))
+    xd, wd = x.cuda(), w.cuda()
+    want = x.double() @ w.double().T
+    for poison in (False, True):
+        if poison:
+            ops.skinny_linear(torch.full_like(xd, float("nan")), wd)
+        sums = ops.skinny_linear_sums(xd, wd)
+        assert sums.shape[::2] == (rows, n_out)
+        close(sums.double().sum(1), want, torch.float32)
+        close(ops.skinny_linear(xd, wd, b.cuda(), out_f32=True), want + b.double(), torch.float32)
+    close(ops.skinny_linear(xd, wd, b.cuda(), activation="relu2"), (want + b.double()).clamp(min=0) ** 2, torch.bfloat16)
+    # without scratch memory, and where the result does not lie on 16 bytes
+    y = torch.empty(rows * n_out + 1, dtype=torch.bfloat16, device="cuda")[1:].view(rows, n_out)
+    for scratch, nbytes in ((None, 0), (torch.empty(64 << 20, dtype=torch.uint8, device="cuda"), 64 << 20)):
+        ops._call(xd.device, "nqh_skinny_linear_ex", xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), rows, n_out, n_in, 0, 0, 0.0,
+                  ops._ptr(scratch), nbytes)
+        close(y, want, torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows,width,parts", [(1, 64, 1), (3, 1024, 2), (2, 50, 3), (5, 2052, 7), (2, 4096, 16), (300, 72, 5)])
+def test_norms_add_the_parts_of_a_product(rows, width, parts):
+    """The residual's next read with fp32 parts equals the one with their sum."""
+    print(f"parts {rows} x {parts} x {width}", flush=True)
+    y = rand(rows, parts, width, seed=1).cuda()
+    total = y.double().sum(1)
+    x0, wn, wp = rand(rows, width, seed=2), rand(width, seed=3, dtype=torch.bfloat16), rand(width, seed=4, dtype=torch.bfloat16)
+    rms = lambda t, w: t / (t.square().mean(-1, keepdim=True) + 1e-3).sqrt() * w.double()
+    x = x0.cuda()
+    h = ops.residual_norm(x, 1e-3, y=y, post_weight=wp.cuda(), next_weight=wn.cuda())
+    want = x0.double() + rms(total.cpu(), wp)
+    close(x, want, torch.float32)
+    close(h, rms(want, wn), torch.bfloat16)
+    x, mix, write = torch.stack([x0, 2 * x0], 1).cuda(), torch.tensor([[0.5, 0.25], [1.0, 2.0]]), torch.tensor([1.0, 0.5])
+    h = ops.hyper_norm(x, 1e-3, y=y, mix=mix.bfloat16().cuda(), write=write.bfloat16().cuda(), next_weight=wn.cuda())
+    want = torch.einsum("st,rsw->rtw", mix.double(), torch.stack([x0, 2 * x0], 1).double()) + write.double().view(1, 2, 1) * total.cpu().unsqueeze(1)
+    close(x, want, torch.float32)
+    close(h, rms(want.sum(1), wn), torch.bfloat16)
+
+
 # one row, both tile heights, rows and columns past their tiles (also fewer than a tile), one stage to many; several rounds of tiles
 @pytest.mark.parametrize("rows,n_out,n_in", [(1, 8, 64), (130, 264, 128), (127, 4608, 192), (257, 8, 320), (256, 512, 1024),
                                              (2049, 4616, 1024), (4000, 1032, 64)])

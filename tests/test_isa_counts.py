@@ -125,7 +125,7 @@ def test_matrix_core_attention_counts_its_tile_loads(tmp_path):
 def test_hybrid_kernels_wait_for_their_tile_loads(tmp_path):
     """attn_decode_kernel reads its K tile after a counted wait that leaves the V tile's loads outstanding: both tiles are
     R / 16 load-to-LDS instructions, in one run with no other vector-memory instruction between the V loads and the wait.
-    The double-buffered kernels (prompt attention, grouped products, wide linear) must not wait for the loads of the next
+    The double-buffered kernels (prompt attention, grouped products) must not wait for the loads of the next
     stage before they read the current one: no vmcnt(0) between the barrier and the first matrix instruction."""
     def listing(name):
         out = tmp_path / (name + ".s")
@@ -155,11 +155,26 @@ def test_hybrid_kernels_wait_for_their_tile_loads(tmp_path):
         found += 1
     assert found == 6
     found = 0
-    for source, kernel in (("attention", "attn_tile_kernel"), ("attention", "latent_decode_kernel"), ("moe", "moe_gemm_kernel"), ("dense", "wide_linear_kernel")):
+    for source, kernel in (("attention", "attn_tile_kernel"), ("attention", "latent_decode_kernel"), ("moe", "moe_gemm_kernel")):
         for name, ins in bodies(asm if source == "attention" else listing(source), kernel):
             first = next(k for k, l in enumerate(ins) if "v_mfma" in l)
             bar = max(k for k in range(first) if ins[k].startswith("s_barrier"))
             assert any("vmcnt(0)" in l for l in ins[bar - 4:bar]), name          # this stage's loads have landed
             assert not any("vmcnt(0)" in l for l in ins[bar:first]), name
             found += 1
-    assert found == 6 + 7 + 16 + 4 + 8       # attention over cache rows, over expanded latents, over latents; products
+    assert found == 6 + 7 + 16 + 4       # attention over cache rows, over expanded latents, over latents; grouped products
+    # stream_linear_kernel waits by count: in front of every barrier of its loop the requests of all stages but one are open, and
+    # between two of them exactly one stage's are made
+    found = 0
+    for name, ins in bodies(listing("dense"), "stream_linear_kernel"):
+        mt, nt, ks, ahead = (int(v) for v in re.search(r"kernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E", name).groups())
+        stage = 4 + 4 * mt // nt
+        kinds = ["load" if l.startswith("buffer_load_dwordx4") else "barrier" if l.startswith("s_barrier") else "" for l in ins]
+        bars = [k for k, kind in enumerate(kinds) if kind == "barrier"]
+        assert kinds[:bars[0]].count("load") == ahead * stage, name
+        for u in range(ahead + 1):
+            assert any("vmcnt(%d)" % ((ahead - 1) * stage) in l for l in ins[bars[u] - 3:bars[u]]), (name, u)
+            assert kinds[bars[u]:bars[u + 1]].count("load") == stage, (name, u)
+        assert kinds.count("load") == (2 * ahead + 1) * stage, name
+        found += 1
+    assert found == 3 * (2 + 3 + 3)
