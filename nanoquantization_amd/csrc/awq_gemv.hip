@@ -1749,6 +1749,16 @@ static hipError_t launch_gemv_dma(const void* x, const int32_t* qweight, const v
         const long long room = (256 - compute_wgs) / ((long long)splits * row_blocks);   // stay within one wave of workgroups
         pf_wgs = (int)(want < room ? want : room);
         if (pf_wgs < 1) pf_wgs = 1;
+        // Two round trips of the prefetch threads (four lines each) at most, or the launch lasts as long as its successor's weight:
+        // the o_proj launch of a Qwen3-4B step, whose splits leave it 12 workgroups in front of 25 MB, took 34 us instead of 9.  Decode
+        // steps of six such layers 583 -> 416 us at one row, 796 -> 643 at 32 (one trip 631, three 666, four 690); six 1.7B
+        // layers at 32 rows 540 -> 503.  What is left over the launch that reads it fetches itself.  The 0.3 to 1.6 MB regions of Qwen3-0.6B
+        // take one trip: 28 layers 1584 / 1585 (cut to one 1592).
+        long long reach = (long long)pf_wgs * 64 * WK * 4 * 128 * 2;
+        for (int r = 0; r < pf.count; ++r) {
+            pf.bytes[r] = std::min(pf.bytes[r], reach);
+            reach -= pf.bytes[r];
+        }
     } else {
         pf.count = 0;
     }
