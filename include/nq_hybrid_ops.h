@@ -268,6 +268,19 @@ int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_f
 int nqh_dense_activation(const void* x, const void* weight, void* y, int64_t rows, int64_t out_features, int64_t in_features, int act,
                          float param, void* stream);
 
+/* y [rows, out_features] = x @ weight^T (+ bias), bf16, for many rows; sizes and alignment as nqh_dense_activation takes them.  Scratch
+ * memory of nqh_dense_linear_scratch_bytes (16-byte aligned; 0: not wanted) lets it split the contraction; without enough of it it does
+ * not.  nqh_dense_linear_wanted: 1 where it takes the sizes and is estimated to be done before a library product that the host issues
+ * (21 us at least); reader: of the sums, below; busy: other work of the pass keeps the GPU behind the host.
+ * nqh_dense_linear_sums: sums [rows, parts, out_features] fp32 of nqh_dense_linear_parts >= 1 parts, for a reader that adds them. */
+int nqh_dense_linear_wanted(int64_t rows, int64_t out_features, int64_t in_features, int reader, int busy);
+size_t nqh_dense_linear_scratch_bytes(int64_t rows, int64_t out_features, int64_t in_features);
+int nqh_dense_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
+                     int64_t in_features, void* scratch, size_t scratch_bytes, void* stream);
+int64_t nqh_dense_linear_parts(int64_t rows, int64_t out_features, int64_t in_features);
+int nqh_dense_linear_sums(const void* x, const void* weight, float* sums, int64_t rows, int64_t out_features, int64_t in_features,
+                          void* stream);
+
 /* Decode-step bookkeeping, as nq_argmax_rows / nq_decode_prepare / nq_decode_advance (nq_engine_ops.h) do it; the
  * logits are fp32. */
 int nqh_argmax_rows(const float* logits, int64_t* out, int64_t rows, int64_t vocab, void* stream);

@@ -2,7 +2,8 @@
 //   skinny_linear_kernel   both operands straight from memory, 16 rows at a time, the waves split the contraction
 //   stream_linear_kernel   up to 64 rows at once: the activations go through LDS; the contraction may be split over workgroups,
 //                          whose sums the reader adds (nqh_skinny_linear_parts) or sum_parts_kernel
-// plan_linear says which.  And y = act(x W^T) for more rows where an activation follows, dense_activation_kernel.
+// plan_linear says which.  For more rows dense_linear_kernel, an activation or a bias in its epilogue, the contraction split likewise
+// (plan_dense), where it is done before a library product that the host issues.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -194,7 +195,7 @@ __global__ __launch_bounds__(64 * NT * KS, NT == 8 ? 4 : 2) void stream_linear_k
 template <bool F32OUT>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict__ parts, const uint16_t* __restrict__ bias,
                                                         void* __restrict__ y, int n_out, int splits, int act, float param) {
-    const int n = (blockIdx.x * 256 + threadIdx.x) * 4, row = blockIdx.y;
+    const int n = (blockIdx.y * 256 + threadIdx.x) * 4, row = blockIdx.x;
     if (n >= n_out) return;
     const float* src = parts + (int64_t)row * splits * n_out + n;
     float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -211,22 +212,34 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict_
     else store_vec<Bf, 4>(reinterpret_cast<uint16_t*>(y) + at, v);
 }
 
+int launch_sum_parts(const char* fn, const void* parts, const void* bias, void* y, int64_t rows, int64_t n_out, int64_t splits, int out_f32,
+                     int act, float param, hipStream_t stream) {
+    const auto kernel = out_f32 ? sum_parts_kernel<true> : sum_parts_kernel<false>;
+    kernel<<<dim3((unsigned)rows, (unsigned)cdiv(n_out, 1024)), dim3(256), 0, stream>>>((const float*)parts, (const uint16_t*)bias, y, (int)n_out,
+                                                                                  (int)splits, act, param);
+    return launched(fn);
+}
+
+// Lets a kernel use `lds` bytes; `raised`: the devices where that has been done.
+int allow_lds(const char* fn, const void* kernel, int lds, std::atomic<uint64_t>& raised) {
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e == hipSuccess && (device > 63 || !(raised.load(std::memory_order_relaxed) >> device & 1))) {
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e == hipSuccess && device < 64) raised.fetch_or(1ull << device, std::memory_order_relaxed);
+    }
+    return e == hipSuccess ? NQH_OK : fail(NQH_ERR_HIP, fn, "%s", hipGetErrorString(e));
+}
+
 template <int MT, int NT, int KS, int kAhead, bool F32OUT, bool SPLIT>
 int launch_stream(const char* fn, const void* x, const void* w, const void* bias, void* y, int64_t rows, int64_t n_out, int64_t n_in,
                   int act, float param, int64_t splits, hipStream_t stream) {
     const int64_t each = cdiv(cdiv(n_in, kPiece), splits);
     constexpr int lds = (kAhead + 1) * KS * 16 * MT * 256;
     const auto kernel = stream_linear_kernel<MT, NT, KS, kAhead, F32OUT, SPLIT>;
-    if (lds > 65536) {
-        static std::atomic<uint64_t> raised{0};          // the devices that this kernel may use so much LDS of
-        int device = 0;
-        hipError_t e = hipGetDevice(&device);
-        if (e == hipSuccess && (device > 63 || !(raised.load(std::memory_order_relaxed) >> device & 1))) {
-            e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-            if (e == hipSuccess && device < 64) raised.fetch_or(1ull << device, std::memory_order_relaxed);
-        }
-        if (e != hipSuccess) return fail(NQH_ERR_HIP, fn, "%s", hipGetErrorString(e));
-    }
+    static std::atomic<uint64_t> raised{0};
+    const int rc = lds > 65536 ? allow_lds(fn, (const void*)kernel, lds, raised) : NQH_OK;
+    if (rc != NQH_OK) return rc;
     kernel<<<dim3((unsigned)cdiv(n_out, 16 * NT), (unsigned)splits), dim3(64 * NT * KS), lds, stream>>>(
         (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y, (int)rows, (int)n_out, (int)n_in, act, param, (int)each);
     return launched(fn);
@@ -284,18 +297,23 @@ LinearPlan make_linear_plan(int64_t rows, int64_t n_out, int64_t n_in, Sums sums
     return best;
 }
 
-// The same, remembered: some 50 estimates take the host 3 us, as long as a launch.
-LinearPlan plan_linear(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
+// What `make` says, remembered per thread: some 50 estimates take the host 3 us, as long as a launch.
+template <typename Plan, typename F>
+Plan remembered(int64_t rows, int64_t n_out, int64_t n_in, Sums sums, F make) {
     struct Entry {
         int64_t rows, n_out, n_in;
         Sums sums;
-        LinearPlan plan;
+        Plan plan;
     };
     thread_local Entry kept[64] = {};                  // rows 0: empty
     Entry& e = kept[(uint64_t)(n_out * 31 + n_in * 7 + rows * 3 + (int)sums) * 0x9E3779B97F4A7C15ull >> 58];
     if (e.rows != rows || e.n_out != n_out || e.n_in != n_in || e.sums != sums)
-        e = {rows, n_out, n_in, sums, make_linear_plan(rows, n_out, n_in, sums)};
+        e = {rows, n_out, n_in, sums, make(rows, n_out, n_in, sums)};
     return e.plan;
+}
+
+LinearPlan plan_linear(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
+    return remembered<LinearPlan>(rows, n_out, n_in, sums, make_linear_plan);
 }
 
 size_t parts_bytes(LinearPlan plan, int64_t rows, int64_t n_out) {
@@ -336,14 +354,16 @@ bool skinny_takes(int64_t rows, int64_t n_out, int64_t n_in) {
     return rows > 0 && rows <= 64 && n_out > 0 && n_in > 0 && n_in % 8 == 0 && n_out <= kMaxI32 - 16 && n_in <= (1 << 30);
 }
 
-// ---- many rows: activation(x @ weight^T) on the tiles of pingpong.hpp -------------------------------------------------
+// ---- many rows: activation(x @ weight^T (+ bias)) on the tiles of pingpong.hpp -----------------------------------------
 // The activation of a library product is a pass of its own that reads and writes the result once more.  Here it is applied
 // on the way out of the tile, to the value rounded to bf16 as that pass finds it: the same results but for the order of the sums.
-// Bound by the matrix cores from a few hundred rows on, by the fill and store of its one tile below.
-template <int XR>
-__global__ __launch_bounds__(512, 2) void dense_activation_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                                  uint16_t* __restrict__ y, int rows, int n_out, int n_in, int act,
-                                                                  float param, int x_tiles, int w_tiles) {
+// Bound by the matrix cores from a few hundred rows on, by the fill and store of its one tile below.  SPLIT: blockIdx.y is a part of
+// steps_each stages of the contraction, and y takes its sums, fp32 [rows, parts, n_out], n_out % 4 == 0; bias and activation are the
+// reader's.
+template <int XR, bool SPLIT>
+__global__ __launch_bounds__(512, 2) void dense_linear_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+                                                              const uint16_t* __restrict__ bias, void* __restrict__ y, int rows, int n_out,
+                                                              int n_in, int act, float param, int x_tiles, int w_tiles, int steps_each) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_stage[];
     using P = awq::PingPong<Bf, XR>;
     int xt, wt;
@@ -351,45 +371,61 @@ __global__ __launch_bounds__(512, 2) void dense_activation_kernel(const uint16_t
     P p;
     const int m0 = xt * XR, n0 = wt * 256, count = min(XR, rows - m0);
     const uint32_t row_bytes = (uint32_t)n_in * 2;
+    const int first = SPLIT ? (int)blockIdx.y * steps_each : 0, steps = min(steps_each, n_in / P::kStage - first);
     uint32_t vw[4], vx[P::kXLoads];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int r = P::w_row(q, p.wave, p.lane);
-        vw[q] = P::source(n0 + r, n_out, row_bytes, r, p.lane);
+        vw[q] = P::source(n0 + r, n_out, row_bytes, r, p.lane) + first * (P::kStage * 2);
     }
 #pragma unroll
     for (int q = 0; q < P::kXLoads; ++q) {
         const int r = P::x_row(q, p.wave, p.lane);
-        vx[q] = P::source(r, count, row_bytes, r, p.lane);
+        vx[q] = P::source(r, count, row_bytes, r, p.lane) + first * (P::kStage * 2);
     }
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w), 0, (uint32_t)n_out * row_bytes, 0x00020000);
     const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (int64_t)m0 * n_in, 0, (uint32_t)count * row_bytes,
                                                       0x00020000);
-    p.run(s_stage, rw, vw, rx, vx, n_in / P::kStage);
-    p.template write<256>(s_stage, [&](int i, int j) {
-        float v[4];
+    p.run(s_stage, rw, vw, rx, vx, steps);
+    if constexpr (SPLIT) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = activation_f32(Bf::round(p.acc[i][j][e]), act, param);
-        return u32x2{Bf::pack2(v[0], v[1]), Bf::pack2(v[2], v[3])};
-    }, [&](int r, int c, u32x4 v) {
-        if (r < count && n0 + c < n_out) *reinterpret_cast<u32x4*>(y + (int64_t)(m0 + r) * n_out + n0 + c) = v;
-    });
+        for (int j = 0; j < P::NJ; ++j) {
+            const int r = p.wn * (XR / P::kWN) + 16 * j + p.lo;
+            if (r >= count) continue;
+            float* to = reinterpret_cast<float*>(y) + ((int64_t)(m0 + r) * gridDim.y + blockIdx.y) * n_out;
+#pragma unroll
+            for (int i = 0; i < P::MI; ++i) {
+                const int n = n0 + p.wm * (256 / P::kWM) + 16 * i + 4 * p.hi;
+                if (n < n_out) *reinterpret_cast<f32x4*>(to + n) = p.acc[i][j];
+            }
+        }
+    } else {
+        p.template write<256>(s_stage, [&](int i, int j) {
+            const int n = n0 + p.wm * (256 / P::kWM) + 16 * i + 4 * p.hi;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = activation_f32(Bf::round(p.acc[i][j][e] + (bias ? Bf::to_f32(bias[min(n + e, n_out - 1)]) : 0.f)), act, param);
+            return u32x2{Bf::pack2(v[0], v[1]), Bf::pack2(v[2], v[3])};
+        }, [&](int r, int c, u32x4 v) {
+            if (r < count && n0 + c < n_out)
+                *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(y) + (int64_t)(m0 + r) * n_out + n0 + c) = v;
+        });
+    }
 }
 
-template <int XR>
-int launch_dense_activation(const char* fn, const void* x, const void* w, void* y, int64_t rows, int64_t n_out, int64_t n_in, int act,
-                            float param, void* stream) {
+template <int XR, bool SPLIT>
+int launch_dense(const char* fn, const void* x, const void* w, const void* bias, void* y, int64_t rows, int64_t n_out, int64_t n_in,
+                 int act, float param, int64_t splits, void* stream) {
     using P = awq::PingPong<Bf, XR>;
-    const auto kernel = dense_activation_kernel<XR>;
-    static bool raised = false;          // once per process and instantiation
-    if (!raised) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, P::kLds);
-        if (e != hipSuccess) return fail(NQH_ERR_HIP, fn, "%s", hipGetErrorString(e));
-        raised = true;
-    }
+    const auto kernel = dense_linear_kernel<XR, SPLIT>;
+    static std::atomic<uint64_t> raised{0};
+    const int rc = allow_lds(fn, (const void*)kernel, P::kLds, raised);
+    if (rc != NQH_OK) return rc;
     const int64_t x_tiles = cdiv(rows, XR), w_tiles = cdiv(n_out, 256);
-    kernel<<<dim3((unsigned)(cdiv(x_tiles * w_tiles, 8) * 8)), dim3(P::kThreads), P::kLds, (hipStream_t)stream>>>(
-        (const uint16_t*)x, (const uint16_t*)w, (uint16_t*)y, (int)rows, (int)n_out, (int)n_in, act, param, (int)x_tiles, (int)w_tiles);
+    kernel<<<dim3((unsigned)(cdiv(x_tiles * w_tiles, 8) * 8), (unsigned)splits), dim3(P::kThreads), P::kLds, (hipStream_t)stream>>>(
+        (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y, (int)rows, (int)n_out, (int)n_in, act, param, (int)x_tiles,
+        (int)w_tiles, (int)cdiv(n_in / P::kStage, splits));
     return launched(fn);
 }
 
@@ -410,6 +446,48 @@ double dense_activation_us(int64_t rows, int64_t n_out, int64_t n_in, int xr) {
 
 int dense_activation_tile(int64_t rows, int64_t n_out, int64_t n_in) {
     return dense_activation_us(rows, n_out, n_in, 128) < dense_activation_us(rows, n_out, n_in, 256) ? 128 : 256;
+}
+
+// ---- the same without an activation, instead of a library product -----------------------------------------------------------
+struct DensePlan {
+    int xr, splits;
+    double us;
+};
+
+// Estimated microseconds: rounds of 256 workgroups as above, by stages and ends, the weights from memory, parts written and read as in
+// plan_linear (a reader of more rows than CUs: 5.5 TB/s; it reads sums instead of a 16-bit result).  Fitted to 33 weights (96 to 18432 x 1024 to
+// 18432) at 80 to 8192 rows: 5 % off in the middle, 14 % in one of ten; the chosen form 1.2 % from the fastest on average.
+DensePlan make_dense_plan(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
+    const double memory = 3.2 + 2e-6 * n_out * n_in / 3.6;
+    DensePlan best{0, 1, 1e30};
+    for (const int xr : {128, 256}) {
+        const int64_t tiles = cdiv(rows, xr) * cdiv(n_out, 256), steps = n_in / 64;
+        for (int64_t s = 1; s <= 16; ++s) {
+            const int64_t each = cdiv(steps, s), work = tiles * s;
+            const double parts = 4e-6 * s * rows * n_out;
+            if (s > 1 && (sums == Sums::kNone || n_out % 4 != 0 || each < 2 || work > 520 || parts > 268)) break;
+            if (cdiv(steps, each) != s) continue;
+            const double part = (double)(work % 256) / 256, whole = (double)(work / 256);
+            const double stage = xr == 256 ? std::max(0.52, 0.91 + 0.37 * part) : std::max(0.59, 0.6 + 0.32 * part), end = xr == 256 ? 5.4 : 3.3;
+            double us = std::max(memory, 3.2 + whole * (each * (xr == 256 ? 1.36 : 0.85) + end) + (part > 0 ? each * stage + end : 0));
+            if (s > 1) us += parts / 8 + (sums == Sums::kReader ? std::max((parts - 2e-6 * rows * n_out) / 5.5, 4e-3 * s * n_out / 60) : 2.65 + parts / 6);
+            if (us < best.us) best = {xr, (int)s, us};
+        }
+    }
+    return best;
+}
+
+DensePlan plan_dense(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
+    return remembered<DensePlan>(rows, n_out, n_in, sums, make_dense_plan);
+}
+
+// What a library product is worth waiting for: the time that it takes on the GPU, less a margin for being ahead of the estimate in a
+// pass (contractions of 12288 and more it does not split well), or most of the 21 us that it takes the host to issue; busy: of a pass
+// with other work that the GPU takes longer for than the host, which hides a part of that (the figures are beside
+// nqh_dense_linear_wanted).
+double library_us(int64_t rows, int64_t n_out, int64_t n_in, bool busy) {
+    const double size = (double)rows * (double)n_out;
+    return std::max(busy ? 15.0 : 20.0, (n_in >= 12288 ? 0.9 : 0.8) * (6.2 + 2e-9 * size * n_in / (1.4 * size / (size + 1.57e6))));
 }
 
 }  // namespace
@@ -457,10 +535,7 @@ extern "C" int nqh_skinny_linear_ex(const void* x, const void* weight, const voi
     if (plan.splits == 1) return run_plan(fn, plan, x, weight, bias, y, rows, out_features, in_features, out_f32, act, param, st);
     const int rc = run_plan(fn, plan, x, weight, nullptr, scratch, rows, out_features, in_features, 1, NQH_ACT_NONE, 0.f, st);
     if (rc != 0) return rc;
-    const auto kernel = out_f32 ? sum_parts_kernel<true> : sum_parts_kernel<false>;
-    kernel<<<dim3((unsigned)cdiv(out_features, 1024), (unsigned)rows), dim3(256), 0, st>>>(
-        (const float*)scratch, (const uint16_t*)bias, y, (int)out_features, plan.splits, act, param);
-    return launched(fn);
+    return launch_sum_parts(fn, scratch, bias, y, rows, out_features, plan.splits, out_f32, act, param, st);
 }
 
 extern "C" int nqh_skinny_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows,
@@ -476,13 +551,16 @@ extern "C" int nqh_skinny_linear(const void* x, const void* weight, const void* 
 // off: Roletar prompts through three layers with this kernel / without, wall time and (behind other work, GPU time): 0.6B, 128
 // tokens 666 / 713 (356 / 333), 1000 tokens 696 / 743 (514 / 514); 1.7B, 128 tokens 646 / 751 (495 / 448), 400 tokens 666 / 717 (585 / 590),
 // 1000 tokens 860 / 872; 8B 0 to 2 % less.  Several rounds
-// stay with the library: in a pass its products lose less to the writes between the rounds (0.6B, 8192 tokens, 576 tiles: 110 here,
+// of short contractions stay with the library: in a pass its products lose less to the writes between the rounds (0.6B, 8192 tokens, 576 tiles: 110 here,
 // 83 + 24 there, though 89 / 103 when repeated alone; 1.7B, 4096 tokens, 576 tiles: the pass 1873 -> 1886).
+// Of 4096 and more the ends of the tiles weigh less (4000 rows, 4096 -> 18432: 453 here, 365 to 564 + 48 there; the pass 5087 with the product below alone, 4686 with both).
 extern "C" int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_features) {
     if (!dense_activation_takes(rows, out_features, in_features)) return 0;
     const int xr = dense_activation_tile(rows, out_features, in_features);
-    if (cdiv(rows, xr) * cdiv(out_features, 256) > 256) return 0;
     const double work = (double)rows * (double)out_features;
+    if (cdiv(rows, xr) * cdiv(out_features, 256) > 256)
+        return in_features >= 4096 && plan_dense(rows, out_features, in_features, Sums::kNone).us <
+                                          0.92 * (6.2 + 2e-9 * work * (double)in_features / (1.4 * work / (work + 1.57e6)) + 4e-6 * work / 5);
     return dense_activation_us(rows, out_features, in_features, xr) <
            std::max(28.0, 2 * work * (double)in_features / 1.3e9 + 4 * work / 5e6 + 5);
 }
@@ -499,6 +577,64 @@ extern "C" int nqh_dense_activation(const void* x, const void* weight, void* y, 
         return fail(NQH_ERR_ARG, fn, "unknown activation, or a cap that is not positive");
     (void)hipGetLastError();
     return dense_activation_tile(rows, out_features, in_features) == 128
-               ? launch_dense_activation<128>(fn, x, weight, y, rows, out_features, in_features, act, param, stream)
-               : launch_dense_activation<256>(fn, x, weight, y, rows, out_features, in_features, act, param, stream);
+               ? launch_dense<128, false>(fn, x, weight, nullptr, y, rows, out_features, in_features, act, param, 1, stream)
+               : launch_dense<256, false>(fn, x, weight, nullptr, y, rows, out_features, in_features, act, param, 1, stream);
+}
+
+// Products of prompts.  A library product takes the host 21 us to issue, this one 6, and a pass of some hundred rows through small
+// layers is 11 of them; on the GPU the library is ahead by up to a third there.  Where its tiles leave CUs idle over a long
+// contraction it falls far behind (1000 rows of 18432 -> 4096: 217 us, this with the sums left to the reader 114; 900 of 12288 -> 4096 107 /
+// 81; 160 of 8192 -> 4096 48 / 25; 900 of 9728 -> 2560 80 / 51), and with many rows it is ahead by 3 to 10 %.  Prompts through three layers, before / now, us: Roletar 0.6B, 300 tokens
+// 661 / 540, 1000 697 / 638; 1.7B, 500 tokens 728 / 645; 8B, 300 tokens 1066 / 884, 2000 3157 / 2682, 4000 5128 / 4778; Gafulix 0.6B,
+// 100 tokens 556 / 421, 500 661 / 562.  Of Gafulix 1.7B and 8B the experts' weights take the GPU 500 to 900 us, so that the host's
+// time is hidden: a product of 15 to 20 us is the library's there (busy; 1700 rows, 2048 -> 2048: 27 here, 17 there; the passes are
+// within 1 % of what they were).
+extern "C" int nqh_dense_linear_wanted(int64_t rows, int64_t out_features, int64_t in_features, int reader, int busy) {
+    return dense_activation_takes(rows, out_features, in_features) &&
+           plan_dense(rows, out_features, in_features, reader ? Sums::kReader : Sums::kOwnPass).us <
+               library_us(rows, out_features, in_features, busy != 0);
+}
+
+extern "C" size_t nqh_dense_linear_scratch_bytes(int64_t rows, int64_t out_features, int64_t in_features) {
+    if (!dense_activation_takes(rows, out_features, in_features)) return 0;
+    const DensePlan plan = plan_dense(rows, out_features, in_features, Sums::kOwnPass);
+    return plan.splits > 1 ? (size_t)plan.splits * rows * out_features * sizeof(float) : 0;
+}
+
+extern "C" int nqh_dense_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
+                                int64_t in_features, void* scratch, size_t scratch_bytes, void* stream) {
+    const char* fn = "nqh_dense_linear";
+    if (!x || !weight || !y || !aligned(x, 16) || !aligned(weight, 16) || !aligned(y, 16) || !aligned(scratch, 16))
+        return fail(NQH_ERR_ARG, fn, "null or misaligned pointer");
+    if (!dense_activation_takes(rows, out_features, in_features))
+        return fail(NQH_ERR_UNSUPPORTED, fn, "needs an in_features that is a multiple of 64, an out_features that is one of 8, and a "
+                                             "weight of less than 2^31 elements");
+    (void)hipGetLastError();
+    DensePlan plan = plan_dense(rows, out_features, in_features, scratch ? Sums::kOwnPass : Sums::kNone);
+    if (plan.splits > 1 && scratch_bytes < (size_t)plan.splits * rows * out_features * sizeof(float))
+        plan = plan_dense(rows, out_features, in_features, Sums::kNone);
+    if (plan.splits == 1)
+        return plan.xr == 128 ? launch_dense<128, false>(fn, x, weight, bias, y, rows, out_features, in_features, NQH_ACT_NONE, 0.f, 1, stream)
+                              : launch_dense<256, false>(fn, x, weight, bias, y, rows, out_features, in_features, NQH_ACT_NONE, 0.f, 1, stream);
+    const int rc = plan.xr == 128 ? launch_dense<128, true>(fn, x, weight, nullptr, scratch, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream)
+                                  : launch_dense<256, true>(fn, x, weight, nullptr, scratch, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream);
+    return rc != NQH_OK ? rc : launch_sum_parts(fn, scratch, bias, y, rows, out_features, plan.splits, 0, NQH_ACT_NONE, 0.f, (hipStream_t)stream);
+}
+
+extern "C" int64_t nqh_dense_linear_parts(int64_t rows, int64_t out_features, int64_t in_features) {
+    return dense_activation_takes(rows, out_features, in_features) ? plan_dense(rows, out_features, in_features, Sums::kReader).splits : 1;
+}
+
+extern "C" int nqh_dense_linear_sums(const void* x, const void* weight, float* sums, int64_t rows, int64_t out_features,
+                                     int64_t in_features, void* stream) {
+    const char* fn = "nqh_dense_linear_sums";
+    if (!x || !weight || !sums || !aligned(x, 16) || !aligned(weight, 16) || !aligned(sums, 16))
+        return fail(NQH_ERR_ARG, fn, "null or misaligned pointer");
+    if (!dense_activation_takes(rows, out_features, in_features))
+        return fail(NQH_ERR_UNSUPPORTED, fn, "needs an in_features that is a multiple of 64, an out_features that is one of 8, and a "
+                                             "weight of less than 2^31 elements");
+    (void)hipGetLastError();
+    const DensePlan plan = plan_dense(rows, out_features, in_features, Sums::kReader);
+    return plan.xr == 128 ? launch_dense<128, true>(fn, x, weight, nullptr, sums, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream)
+                          : launch_dense<256, true>(fn, x, weight, nullptr, sums, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream);
 }

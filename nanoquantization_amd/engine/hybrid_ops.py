@@ -678,6 +678,49 @@ def dense_activation(x: torch.Tensor, weight: torch.Tensor, activation: Optional
     return y
 
 
+def dense_linear_wanted(x: torch.Tensor, weight: torch.Tensor, reader: bool, busy: bool) -> bool:
+    """Whether `dense_linear` (reader: `dense_linear_sums`) takes these and is done before a library product issued from here.
+    busy: other work of the pass keeps the GPU behind the host."""
+    return (x.dtype == weight.dtype == torch.bfloat16 and x.is_contiguous() and weight.is_contiguous()
+            and (x.data_ptr() | weight.data_ptr()) % 16 == 0
+            and bool(_of_sizes("nqh_dense_linear_wanted", x.shape[0], *weight.shape, int(reader), int(busy))))
+
+
+def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [rows, in] @ weight [out, in]^T (+ bias), bf16."""
+    dev = _dev(x, weight, bias)
+    rows, n = x.shape
+    assert weight.shape[1] == n and x.dtype == weight.dtype == torch.bfloat16
+    assert bias is None or (bias.shape == (weight.shape[0],) and bias.dtype == torch.bfloat16)
+    y = torch.empty(rows, weight.shape[0], dtype=torch.bfloat16, device=dev)
+    scratch = _room(_of_sizes("nqh_dense_linear_scratch_bytes", rows, *weight.shape), dev)
+    _call(dev, "nqh_dense_linear", x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), rows, weight.shape[0], n, _ptr(scratch),
+          0 if scratch is None else scratch.numel())
+    return y
+
+
+def _room(nbytes: int, dev: torch.device) -> Optional[torch.Tensor]:
+    """Memory for one call, None if none is wanted or left."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
+def dense_linear_sums(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """The same as `skinny_linear_sums` gives it: fp32 [rows, parts, out]; None where one part is best or there is no memory for several."""
+    dev = _dev(x, weight)
+    rows, n = x.shape
+    assert weight.shape[1] == n and x.dtype == weight.dtype == torch.bfloat16
+    parts = _of_sizes("nqh_dense_linear_parts", rows, *weight.shape)
+    sums = _room(4 * rows * parts * weight.shape[0], dev) if parts > 1 else None
+    if sums is None:
+        return None
+    sums = sums.view(torch.float32).view(rows, parts, weight.shape[0])
+    _call(dev, "nqh_dense_linear_sums", x.data_ptr(), weight.data_ptr(), sums.data_ptr(), rows, weight.shape[0], n)
+    return sums
+
+
 def argmax_rows(logits: torch.Tensor) -> torch.Tensor:
     """Greedy sampler: int64 [rows] index of the largest fp32 logit per row (lowest index among equal maxima)."""
     dev = _dev(logits)

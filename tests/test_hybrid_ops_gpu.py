@@ -563,6 +563,25 @@ def test_dense_activation(rows, n_out, n_in):
     assert torch.equal(got, ops.activate_(y, "relu2").cpu())      # of the product rounded to bf16
 
 
+# whole and split contractions (the last part shorter), both tile heights, rows and columns past their tiles, fewer than a tile
+@pytest.mark.parametrize("rows,n_out,n_in", [(65, 8, 64), (130, 96, 2048), (127, 4608, 192), (257, 264, 4672), (1000, 1024, 4608),
+                                             (2049, 2056, 1024), (300, 4096, 18432)])
+def test_dense_linear(rows, n_out, n_in):
+    print(f"dense linear {rows} x {n_in} -> {n_out}", flush=True)
+    x, w, b = (rand(*s, seed=i, dtype=torch.bfloat16) for i, s in enumerate([(rows, n_in), (n_out, n_in), (n_out,)]))
+    xd, wd = x.cuda(), w.cuda()
+    want = (xd.double() @ wd.double().T).cpu()
+    close(ops.dense_linear(xd, wd), want, torch.bfloat16)
+    close(ops.dense_linear(xd, wd, b.cuda()), want + b.double(), torch.bfloat16)
+    y = torch.empty(rows, n_out, dtype=torch.bfloat16, device="cuda")           # without scratch memory: one part
+    ops._call(xd.device, "nqh_dense_linear", xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), rows, n_out, n_in, None, 0)
+    close(y, want, torch.bfloat16)
+    sums = ops.dense_linear_sums(xd, wd)
+    assert (sums is None) == (ops._of_sizes("nqh_dense_linear_parts", rows, n_out, n_in) == 1)
+    if sums is not None:
+        close(sums.double().sum(1), want, torch.float32)
+
+
 def test_argmax_and_bookkeeping():
     for rows, vocab in ((1, 5), (3, 131), (4, 32000), (2, 4098)):
         x = rand(rows, vocab, seed=vocab)
