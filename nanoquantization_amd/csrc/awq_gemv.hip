@@ -355,6 +355,12 @@ __device__ __forceinline__ void qkv_rope_store(const float (&out)[8], int m, siz
 }
 
 template <typename T>
+__device__ __forceinline__ float silu_times_up(float gate, float up) {
+    const float g = T::to_f32(T::from_f32(gate));
+    return T::to_f32(T::from_f32(g / (1.f + __expf(-g)))) * T::to_f32(T::from_f32(up));
+}
+
+template <typename T>
 __device__ __forceinline__ void swiglu_store(const float (&out)[8], uint16_t* __restrict__ y, int m, int N,
                                              size_t n0) {
     float other[8];
@@ -366,11 +372,7 @@ __device__ __forceinline__ void swiglu_store(const float (&out)[8], uint16_t* __
         for (int i = 0; i < 4; ++i) {
             float r[2];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const float g = T::to_f32(T::from_f32(out[2 * i + h]));
-                const float u = T::to_f32(T::from_f32(other[2 * i + h]));
-                r[h] = T::to_f32(T::from_f32(g / (1.f + __expf(-g)))) * u;
-            }
+            for (int h = 0; h < 2; ++h) r[h] = silu_times_up<T>(out[2 * i + h], other[2 * i + h]);
             o[i] = T::pack2(r[0], r[1]);
         }
         *reinterpret_cast<u32x4*>(y + (size_t)m * (N >> 1) + (n0 >> 1)) = o;
@@ -1459,53 +1461,54 @@ __global__ __launch_bounds__(128 * WN) void gemv_wide_kernel(
 }
 
 // Second pass of a K-split wide GEMV: y = epilogue(sum over splits, in split order, of partials [splits][M][N]).
-// A thread owns one word (8 columns) of one row; with the gated epilogue neighbouring threads hold a gate word
-// and its up word.
-template <typename T>
-__global__ __launch_bounds__(256) void gemv_wide_reduce_kernel(const float* __restrict__ partials,
-                                                               const uint16_t* __restrict__ bias,
-                                                               uint16_t* __restrict__ y, int M, int N, int splits,
-                                                               int act) {
-    const int words = N >> 3;
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx >= M * words) return;   // words is even: a gate word and its up word leave together
-    const int m = idx / words, wc = idx - m * words;
-    const size_t n0 = (size_t)wc * 8;
-    const size_t plane = (size_t)M * N;
+// A thread owns four columns of one row; with the gated epilogue the neighbour of its neighbour holds the gate columns' up
+// columns.  Latency bounds it (the sums lie in the caches): SS splits' loads are in flight at a time, one round where they
+// are all of them, and a workgroup is one wave so that the sums of few rows are read by all CUs.  With both kernels, against eight
+// columns a thread in workgroups of 256: 4096 x 12288 at 16 / 32 rows 13.4 / 16.2 -> 12.0 / 14.8 us (256 threads on four columns: no
+// gain), 25600 x 5120 at 16 / 64 rows 21.5 / 35.1 -> 20.4 / 34.1, 12288 x 4096 at 32 rows 15.8 -> 14.6; 32 splits in flight: no more.
+template <typename T, int SS>
+__global__ __launch_bounds__(64) void gemv_wide_reduce_kernel(const float* __restrict__ partials,
+                                                              const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
+                                                              int M, int N, int splits, int act) {
+    const int quads = N >> 2;
+    const int idx = blockIdx.x * 64 + threadIdx.x;
+    if (idx >= M * quads) return;   // N is a multiple of 16: gate columns and their up columns leave together
+    const int m = idx / quads, q = idx - m * quads;
+    const size_t n0 = (size_t)q * 4, plane = (size_t)M * N;
     const float* p = partials + (size_t)m * N + n0;
-    f32x4 lo = f32x4{0.f, 0.f, 0.f, 0.f}, hi = lo;
-    // eight splits' loads in flight at a time (a loop of load, add, load, add is one memory round trip per split:
-    // 4.7 us for five splits of 16 rows x 25600 columns), added in split order all the same
-    for (int s0 = 0; s0 < splits; s0 += 8) {
-        f32x4 a[8], b[8];
+    f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < splits; s0 += SS) {
+        f32x4 a[SS];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const size_t off = (size_t)min(s0 + u, splits - 1) * plane;
-            a[u] = *reinterpret_cast<const f32x4*>(p + off);
-            b[u] = *reinterpret_cast<const f32x4*>(p + off + 4);
-        }
+        for (int u = 0; u < SS; ++u) a[u] = *reinterpret_cast<const f32x4*>(p + (size_t)min(s0 + u, splits - 1) * plane);
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (s0 + u < splits) {
-                lo += a[u];
-                hi += b[u];
-            }
+        for (int u = 0; u < SS; ++u)
+            if (s0 + u < splits) sum += a[u];
     }
-    float out[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    float out[4] = {sum[0], sum[1], sum[2], sum[3]};
     if (act) {
-        swiglu_store<T>(out, y, m, N, n0);
+        float up[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) up[c] = __shfl_xor(out[c], 2);
+        if (q & 2) return;
+        uint32_t o[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float r[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) r[h] = silu_times_up<T>(out[2 * i + h], up[2 * i + h]);
+            o[i] = T::pack2(r[0], r[1]);
+        }
+        *reinterpret_cast<u32x2*>(y + (size_t)m * (N >> 1) + (size_t)(q >> 2) * 8 + (q & 1) * 4) = u32x2{o[0], o[1]};
         return;
     }
     if (bias) {
-        const u32x4 bv = *reinterpret_cast<const u32x4*>(bias + n0);
+        const u32x2 bv = *reinterpret_cast<const u32x2*>(bias + n0);
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
+        for (int c = 0; c < 4; ++c)
             out[c] = add_bias<T>(out[c], T::to_f32((uint16_t)((c & 1) ? (bv[c >> 1] >> 16) : (bv[c >> 1] & 0xFFFFu))));
     }
-    u32x4 o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = T::pack2(out[2 * i], out[2 * i + 1]);
-    *reinterpret_cast<u32x4*>(y + (size_t)m * N + n0) = o;
+    *reinterpret_cast<u32x2*>(y + (size_t)m * N + n0) = u32x2{T::pack2(out[0], out[1]), T::pack2(out[2], out[3])};
 }
 
 // The second pass and the residual add + RMSNorm that follows an o_proj or down_proj in one: a workgroup per row
@@ -1851,8 +1854,10 @@ static hipError_t launch_gemv_wide(const void* x, const int32_t* qweight, const 
                            reinterpret_cast<uint16_t*>(y), an->weight, an->normed, M, N, splits, an->eps);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(gemv_wide_reduce_kernel<T>, dim3((unsigned)cdiv((int64_t)M * (N / 8), 256)), dim3(256), 0, stream, partials,
-                       reinterpret_cast<const uint16_t*>(bias), reinterpret_cast<uint16_t*>(y), M, N, splits, act);
+    const dim3 grid((unsigned)cdiv((int64_t)M * (N / 4), 64));
+    const auto add = splits <= 8 ? gemv_wide_reduce_kernel<T, 8> : gemv_wide_reduce_kernel<T, 16>;
+    hipLaunchKernelGGL(add, grid, dim3(64), 0, stream, partials, reinterpret_cast<const uint16_t*>(bias),
+                       reinterpret_cast<uint16_t*>(y), M, N, splits, act);
     return hipGetLastError();
 }
 

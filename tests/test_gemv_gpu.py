@@ -239,6 +239,22 @@ def test_gemv_shared_chunk_four_m_tiles(dtype, M, K, N, plan):
             assert torch.equal(yv, y)
 
 
+@pytest.mark.parametrize("M,split", [(1, 8), (17, 9), (33, 16), (64, 17)])
+def test_gemv_second_pass_rounds(M, split):
+    """The second pass of a K split reads the sums of 8 or 16 splits at a time: whole rounds and one more, with a bias."""
+    K, N = 17 * 128, 512
+    print(f"gemv second pass M={M} split={split}", flush=True)
+    L = _lib.lib()
+    names = [L.awq_gemv_variant_name(i).decode() for i in range(L.awq_gemv_variant_count())]
+    p = random_packed(K, N, 128, "bf16", seed=split)
+    xb = make_x(M, K, "bf16", seed=M)
+    bias = np.linspace(-1, 1, N).astype(np.float32)
+    y = awq_gemv_variant(to_dev(xb, "bf16"), to_dev(p["qweight"]), to_dev(p["qscales"], "bf16"), to_dev(p["qzeros"]),
+                         names.index("wide2d2m1" if M == 1 else "wide2d2m2" if M == 17 else "wide2d2m4"), split,
+                         bias=to_dev(o.to_bits16(bias, "bf16"), "bf16"))
+    _check(y, xb, p, "bf16", o.to_dtype_f32(bias, "bf16"))
+
+
 def test_gemv_reference_test_shape():
     # the reference's own GEMM test: K=1024, N=2048, g=32, 8 tokens, atol=1.0 against x @ w_dq.T
     # (awq/tests/dequantization_kernel.py:108-138)
