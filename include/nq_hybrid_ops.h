@@ -268,7 +268,8 @@ int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_f
 int nqh_dense_activation(const void* x, const void* weight, void* y, int64_t rows, int64_t out_features, int64_t in_features, int act,
                          float param, void* stream);
 
-/* y [rows, out_features] = x @ weight^T (+ bias), bf16, for many rows; sizes and alignment as nqh_dense_activation takes them.  Scratch
+/* y [rows, out_features] = x @ weight^T (+ bias), bf16, for many rows; sizes and alignment as nqh_dense_activation takes them,
+ * rows of x x_stride elements apart (a multiple of 8, at most 2^20).  Scratch
  * memory of nqh_dense_linear_scratch_bytes (16-byte aligned; 0: not wanted) lets it split the contraction; without enough of it it does
  * not.  nqh_dense_linear_wanted: 1 where it takes the sizes and is estimated to be done before a library product that the host issues
  * (21 us at least); reader: of the sums, below; busy: other work of the pass keeps the GPU behind the host.
@@ -276,7 +277,7 @@ int nqh_dense_activation(const void* x, const void* weight, void* y, int64_t row
 int nqh_dense_linear_wanted(int64_t rows, int64_t out_features, int64_t in_features, int reader, int busy);
 size_t nqh_dense_linear_scratch_bytes(int64_t rows, int64_t out_features, int64_t in_features);
 int nqh_dense_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
-                     int64_t in_features, void* scratch, size_t scratch_bytes, void* stream);
+                     int64_t in_features, int64_t x_stride, void* scratch, size_t scratch_bytes, void* stream);
 int64_t nqh_dense_linear_parts(int64_t rows, int64_t out_features, int64_t in_features);
 int nqh_dense_linear_sums(const void* x, const void* weight, float* sums, int64_t rows, int64_t out_features, int64_t in_features,
                           void* stream);

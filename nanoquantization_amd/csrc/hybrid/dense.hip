@@ -363,14 +363,15 @@ bool skinny_takes(int64_t rows, int64_t n_out, int64_t n_in) {
 template <int XR, bool SPLIT>
 __global__ __launch_bounds__(512, 2) void dense_linear_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
                                                               const uint16_t* __restrict__ bias, void* __restrict__ y, int rows, int n_out,
-                                                              int n_in, int act, float param, int x_tiles, int w_tiles, int steps_each) {
+                                                              int n_in, int x_stride, int act, float param, int x_tiles, int w_tiles,
+                                                              int steps_each) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_stage[];
     using P = awq::PingPong<Bf, XR>;
     int xt, wt;
     if (!awq::xcd_tile((int)blockIdx.x, x_tiles, w_tiles, xt, wt)) return;
     P p;
     const int m0 = xt * XR, n0 = wt * 256, count = min(XR, rows - m0);
-    const uint32_t row_bytes = (uint32_t)n_in * 2;
+    const uint32_t row_bytes = (uint32_t)n_in * 2, x_bytes = (uint32_t)x_stride * 2;
     const int first = SPLIT ? (int)blockIdx.y * steps_each : 0, steps = min(steps_each, n_in / P::kStage - first);
     uint32_t vw[4], vx[P::kXLoads];
 #pragma unroll
@@ -381,11 +382,11 @@ __global__ __launch_bounds__(512, 2) void dense_linear_kernel(const uint16_t* __
 #pragma unroll
     for (int q = 0; q < P::kXLoads; ++q) {
         const int r = P::x_row(q, p.wave, p.lane);
-        vx[q] = P::source(r, count, row_bytes, r, p.lane) + first * (P::kStage * 2);
+        vx[q] = P::source(r, count, x_bytes, r, p.lane) + first * (P::kStage * 2);
     }
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w), 0, (uint32_t)n_out * row_bytes, 0x00020000);
-    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (int64_t)m0 * n_in, 0, (uint32_t)count * row_bytes,
-                                                      0x00020000);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (int64_t)m0 * x_stride, 0,
+                                                      (uint32_t)(count - 1) * x_bytes + row_bytes, 0x00020000);
     p.run(s_stage, rw, vw, rx, vx, steps);
     if constexpr (SPLIT) {
 #pragma unroll
@@ -416,7 +417,7 @@ __global__ __launch_bounds__(512, 2) void dense_linear_kernel(const uint16_t* __
 
 template <int XR, bool SPLIT>
 int launch_dense(const char* fn, const void* x, const void* w, const void* bias, void* y, int64_t rows, int64_t n_out, int64_t n_in,
-                 int act, float param, int64_t splits, void* stream) {
+                 int64_t x_stride, int act, float param, int64_t splits, void* stream) {
     using P = awq::PingPong<Bf, XR>;
     const auto kernel = dense_linear_kernel<XR, SPLIT>;
     static std::atomic<uint64_t> raised{0};
@@ -424,7 +425,8 @@ int launch_dense(const char* fn, const void* x, const void* w, const void* bias,
     if (rc != NQH_OK) return rc;
     const int64_t x_tiles = cdiv(rows, XR), w_tiles = cdiv(n_out, 256);
     kernel<<<dim3((unsigned)(cdiv(x_tiles * w_tiles, 8) * 8), (unsigned)splits), dim3(P::kThreads), P::kLds, (hipStream_t)stream>>>(
-        (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y, (int)rows, (int)n_out, (int)n_in, act, param, (int)x_tiles,
+        (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y, (int)rows, (int)n_out, (int)n_in, (int)x_stride, act,
+        param, (int)x_tiles,
         (int)w_tiles, (int)cdiv(n_in / P::kStage, splits));
     return launched(fn);
 }
@@ -483,11 +485,11 @@ DensePlan plan_dense(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
 
 // What a library product is worth waiting for: the time that it takes on the GPU, less a margin for being ahead of the estimate in a
 // pass (contractions of 12288 and more it does not split well), or most of the 21 us that it takes the host to issue; busy: of a pass
-// with other work that the GPU takes longer for than the host, which hides a part of that (the figures are beside
-// nqh_dense_linear_wanted).
+// with other work that the GPU takes longer for than the host, which hides a part of that, as many rows do in any layer (the figures are
+// beside nqh_dense_linear_wanted).
 double library_us(int64_t rows, int64_t n_out, int64_t n_in, bool busy) {
     const double size = (double)rows * (double)n_out;
-    return std::max(busy ? 15.0 : 20.0, (n_in >= 12288 ? 0.9 : 0.8) * (6.2 + 2e-9 * size * n_in / (1.4 * size / (size + 1.57e6))));
+    return std::max(busy || rows > 2400 ? 15.0 : 20.0, (n_in >= 12288 ? 0.9 : 0.8) * (6.2 + 2e-9 * size * n_in / (1.4 * size / (size + 1.57e6))));
 }
 
 }  // namespace
@@ -577,18 +579,19 @@ extern "C" int nqh_dense_activation(const void* x, const void* weight, void* y, 
         return fail(NQH_ERR_ARG, fn, "unknown activation, or a cap that is not positive");
     (void)hipGetLastError();
     return dense_activation_tile(rows, out_features, in_features) == 128
-               ? launch_dense<128, false>(fn, x, weight, nullptr, y, rows, out_features, in_features, act, param, 1, stream)
-               : launch_dense<256, false>(fn, x, weight, nullptr, y, rows, out_features, in_features, act, param, 1, stream);
+               ? launch_dense<128, false>(fn, x, weight, nullptr, y, rows, out_features, in_features, in_features, act, param, 1, stream)
+               : launch_dense<256, false>(fn, x, weight, nullptr, y, rows, out_features, in_features, in_features, act, param, 1, stream);
 }
 
 // Products of prompts.  A library product takes the host 21 us to issue, this one 6, and a pass of some hundred rows through small
 // layers is 11 of them; on the GPU the library is ahead by up to a third there.  Where its tiles leave CUs idle over a long
 // contraction it falls far behind (1000 rows of 18432 -> 4096: 217 us, this with the sums left to the reader 114; 900 of 12288 -> 4096 107 /
 // 81; 160 of 8192 -> 4096 48 / 25; 900 of 9728 -> 2560 80 / 51), and with many rows it is ahead by 3 to 10 %.  Prompts through three layers, before / now, us: Roletar 0.6B, 300 tokens
-// 661 / 540, 1000 697 / 638; 1.7B, 500 tokens 728 / 645; 8B, 300 tokens 1066 / 884, 2000 3157 / 2682, 4000 5128 / 4778; Gafulix 0.6B,
-// 100 tokens 556 / 421, 500 661 / 562.  Of Gafulix 1.7B and 8B the experts' weights take the GPU 500 to 900 us, so that the host's
-// time is hidden: a product of 15 to 20 us is the library's there (busy; 1700 rows, 2048 -> 2048: 27 here, 17 there; the passes are
-// within 1 % of what they were).
+// 692 / 507 (540 while the library took the expansion of the latents, whose rows are columns of a wider tensor), 1000 752 / 620, 2000
+// 777 / 709; 1.7B, 300 tokens 683 / 554; 8B, 300 tokens 1066 / 882, 2000 3157 / 2682, 4000 5128 / 4778; Gafulix 0.6B, 100 tokens 550 /
+// 413, 700 671 / 510.  Of Gafulix 1.7B and 8B the experts' weights take the GPU 200 to 900 us, so that the host's time is hidden: a
+// product of 15 to 20 us is the library's there (busy; 1700 rows, 2048 -> 2048: 27 here, 17 there; the passes are within 1 % of what
+// they were; Gafulix 0.6B, 16 us of weights a layer: 100 tokens 428 busy, 413 not, 500 572 / 500).
 extern "C" int nqh_dense_linear_wanted(int64_t rows, int64_t out_features, int64_t in_features, int reader, int busy) {
     return dense_activation_takes(rows, out_features, in_features) &&
            plan_dense(rows, out_features, in_features, reader ? Sums::kReader : Sums::kOwnPass).us <
@@ -602,22 +605,24 @@ extern "C" size_t nqh_dense_linear_scratch_bytes(int64_t rows, int64_t out_featu
 }
 
 extern "C" int nqh_dense_linear(const void* x, const void* weight, const void* bias, void* y, int64_t rows, int64_t out_features,
-                                int64_t in_features, void* scratch, size_t scratch_bytes, void* stream) {
+                                int64_t in_features, int64_t x_stride, void* scratch, size_t scratch_bytes, void* stream) {
     const char* fn = "nqh_dense_linear";
     if (!x || !weight || !y || !aligned(x, 16) || !aligned(weight, 16) || !aligned(y, 16) || !aligned(scratch, 16))
         return fail(NQH_ERR_ARG, fn, "null or misaligned pointer");
     if (!dense_activation_takes(rows, out_features, in_features))
         return fail(NQH_ERR_UNSUPPORTED, fn, "needs an in_features that is a multiple of 64, an out_features that is one of 8, and a "
                                              "weight of less than 2^31 elements");
+    if (x_stride < in_features || x_stride % 8 != 0 || x_stride > (1 << 20))
+        return fail(NQH_ERR_ARG, fn, "rows of x must be a multiple of 8 elements apart, at least in_features and at most 2^20");
     (void)hipGetLastError();
     DensePlan plan = plan_dense(rows, out_features, in_features, scratch ? Sums::kOwnPass : Sums::kNone);
     if (plan.splits > 1 && scratch_bytes < (size_t)plan.splits * rows * out_features * sizeof(float))
         plan = plan_dense(rows, out_features, in_features, Sums::kNone);
     if (plan.splits == 1)
-        return plan.xr == 128 ? launch_dense<128, false>(fn, x, weight, bias, y, rows, out_features, in_features, NQH_ACT_NONE, 0.f, 1, stream)
-                              : launch_dense<256, false>(fn, x, weight, bias, y, rows, out_features, in_features, NQH_ACT_NONE, 0.f, 1, stream);
-    const int rc = plan.xr == 128 ? launch_dense<128, true>(fn, x, weight, nullptr, scratch, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream)
-                                  : launch_dense<256, true>(fn, x, weight, nullptr, scratch, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream);
+        return plan.xr == 128 ? launch_dense<128, false>(fn, x, weight, bias, y, rows, out_features, in_features, x_stride, NQH_ACT_NONE, 0.f, 1, stream)
+                              : launch_dense<256, false>(fn, x, weight, bias, y, rows, out_features, in_features, x_stride, NQH_ACT_NONE, 0.f, 1, stream);
+    const int rc = plan.xr == 128 ? launch_dense<128, true>(fn, x, weight, nullptr, scratch, rows, out_features, in_features, x_stride, NQH_ACT_NONE, 0.f, plan.splits, stream)
+                                  : launch_dense<256, true>(fn, x, weight, nullptr, scratch, rows, out_features, in_features, x_stride, NQH_ACT_NONE, 0.f, plan.splits, stream);
     return rc != NQH_OK ? rc : launch_sum_parts(fn, scratch, bias, y, rows, out_features, plan.splits, 0, NQH_ACT_NONE, 0.f, (hipStream_t)stream);
 }
 
@@ -635,6 +640,6 @@ extern "C" int nqh_dense_linear_sums(const void* x, const void* weight, float* s
                                              "weight of less than 2^31 elements");
     (void)hipGetLastError();
     const DensePlan plan = plan_dense(rows, out_features, in_features, Sums::kReader);
-    return plan.xr == 128 ? launch_dense<128, true>(fn, x, weight, nullptr, sums, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream)
-                          : launch_dense<256, true>(fn, x, weight, nullptr, sums, rows, out_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream);
+    return plan.xr == 128 ? launch_dense<128, true>(fn, x, weight, nullptr, sums, rows, out_features, in_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream)
+                          : launch_dense<256, true>(fn, x, weight, nullptr, sums, rows, out_features, in_features, in_features, NQH_ACT_NONE, 0.f, plan.splits, stream);
 }

@@ -128,7 +128,9 @@ class HybridEngine(EngineCore):
                          use_graph and all(ops.skinny_linear_supported(max_batch, w) for w in linears))
         self.runs = spec.runs()
         self.prefill_tokens = prefill_tokens
-        self._experts = any(l.mlp is not None and not isinstance(l.mlp, DenseSpec) for l in spec.layers)
+        # experts whose weights take the GPU longer (at 5 TB/s 30 us and more) than the host is ahead by keep it behind the host
+        self._busy = any(l.mlp is not None and not isinstance(s.mlp, DenseSpec)
+                         and l.mlp.gate_up.nbytes + l.mlp.down.nbytes > 150 << 20 for s, l in zip(spec.layers, model.layers))
         mixers = [spec.layers[i].mixer for i, _ in self.runs]
         self.cache = PagedKVCache(len(mixers), self.num_blocks, block_size, dtype=self.dtype, device=self.device,
                                   layer_shapes=[self._cache_shape(m) for m in mixers])
@@ -166,14 +168,14 @@ class HybridEngine(EngineCore):
             return ops.skinny_linear(x, w, b, activation=activation, param=param)
         if activation is not None and b is None and ops.dense_activation_wanted(x, w):
             return ops.dense_activation(x, w, activation, param)
-        y = ops.dense_linear(x, w, b) if ops.dense_linear_wanted(x, w, False, self._experts) else F.linear(x, w, b)
+        y = ops.dense_linear(x, w, b) if ops.dense_linear_wanted(x, w, False, self._busy) else F.linear(x, w, b)
         return y if activation is None else ops.activate_(y, activation, param)
 
     def _sublayer_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """The product that ends a sublayer, as sums of its parts, which the residual's next read adds, where one part leaves CUs idle."""
         if ops.skinny_linear_supported(x.shape[0], w):
             return ops.skinny_linear_sums(x, w)
-        sums = ops.dense_linear_sums(x, w) if ops.dense_linear_wanted(x, w, True, self._experts) else None
+        sums = ops.dense_linear_sums(x, w) if ops.dense_linear_wanted(x, w, True, self._busy) else None
         return self._linear(x, w) if sums is None else sums
 
     def _logits(self, h: torch.Tensor) -> torch.Tensor:

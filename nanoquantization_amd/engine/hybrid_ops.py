@@ -681,21 +681,22 @@ def dense_activation(x: torch.Tensor, weight: torch.Tensor, activation: Optional
 def dense_linear_wanted(x: torch.Tensor, weight: torch.Tensor, reader: bool, busy: bool) -> bool:
     """Whether `dense_linear` (reader: `dense_linear_sums`) takes these and is done before a library product issued from here.
     busy: other work of the pass keeps the GPU behind the host."""
-    return (x.dtype == weight.dtype == torch.bfloat16 and x.is_contiguous() and weight.is_contiguous()
-            and (x.data_ptr() | weight.data_ptr()) % 16 == 0
+    return (x.dtype == weight.dtype == torch.bfloat16 and weight.is_contiguous() and (x.data_ptr() | weight.data_ptr()) % 16 == 0
+            and (x.is_contiguous() or (not reader and x.stride(1) == 1 and x.shape[1] <= x.stride(0) <= 1 << 20 and x.stride(0) % 8 == 0))
             and bool(_of_sizes("nqh_dense_linear_wanted", x.shape[0], *weight.shape, int(reader), int(busy))))
 
 
 def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [rows, in] @ weight [out, in]^T (+ bias), bf16."""
-    dev = _dev(x, weight, bias)
+    """x [rows, in] (a view of columns, maybe) @ weight [out, in]^T (+ bias), bf16."""
+    dev = _dev(weight, bias)
     rows, n = x.shape
-    assert weight.shape[1] == n and x.dtype == weight.dtype == torch.bfloat16
+    _rows_of(x, dev, weight.shape[1])
+    assert x.dtype == weight.dtype == torch.bfloat16
     assert bias is None or (bias.shape == (weight.shape[0],) and bias.dtype == torch.bfloat16)
     y = torch.empty(rows, weight.shape[0], dtype=torch.bfloat16, device=dev)
     scratch = _room(_of_sizes("nqh_dense_linear_scratch_bytes", rows, *weight.shape), dev)
-    _call(dev, "nqh_dense_linear", x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), rows, weight.shape[0], n, _ptr(scratch),
-          0 if scratch is None else scratch.numel())
+    _call(dev, "nqh_dense_linear", x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), rows, weight.shape[0], n, x.stride(0) if rows > 1 else n,
+          _ptr(scratch), 0 if scratch is None else scratch.numel())
     return y
 
 

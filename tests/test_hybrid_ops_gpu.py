@@ -574,8 +574,11 @@ def test_dense_linear(rows, n_out, n_in):
     close(ops.dense_linear(xd, wd), want, torch.bfloat16)
     close(ops.dense_linear(xd, wd, b.cuda()), want + b.double(), torch.bfloat16)
     y = torch.empty(rows, n_out, dtype=torch.bfloat16, device="cuda")           # without scratch memory: one part
-    ops._call(xd.device, "nqh_dense_linear", xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), rows, n_out, n_in, None, 0)
+    ops._call(xd.device, "nqh_dense_linear", xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), rows, n_out, n_in, n_in, None, 0)
     close(y, want, torch.bfloat16)
+    wide = torch.full((rows, n_in + 24), float("nan"), dtype=torch.bfloat16, device="cuda")      # columns of a wider tensor
+    wide[:, 8:8 + n_in] = xd
+    assert torch.equal(ops.dense_linear(wide[:, 8:8 + n_in], wd), ops.dense_linear(xd, wd))
     sums = ops.dense_linear_sums(xd, wd)
     assert (sums is None) == (ops._of_sizes("nqh_dense_linear_parts", rows, n_out, n_in) == 1)
     if sums is not None:
