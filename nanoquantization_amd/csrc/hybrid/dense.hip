@@ -587,7 +587,7 @@ extern "C" int nqh_dense_activation(const void* x, const void* weight, void* y, 
 // layers is 11 of them; on the GPU the library is ahead by up to a third there.  Where its tiles leave CUs idle over a long
 // contraction it falls far behind (1000 rows of 18432 -> 4096: 217 us, this with the sums left to the reader 114; 900 of 12288 -> 4096 107 /
 // 81; 160 of 8192 -> 4096 48 / 25; 900 of 9728 -> 2560 80 / 51), and with many rows it is ahead by 3 to 10 %.  Prompts through three layers, before / now, us: Roletar 0.6B, 300 tokens
-// 692 / 507 (540 while the library took the expansion of the latents, whose rows are columns of a wider tensor), 1000 752 / 620, 2000
+// 699 / 496 (some 510 while the library took the expansion of the latents, whose rows are columns of a wider tensor), 1000 752 / 620, 2000
 // 777 / 709; 1.7B, 300 tokens 683 / 554; 8B, 300 tokens 1066 / 882, 2000 3157 / 2682, 4000 5128 / 4778; Gafulix 0.6B, 100 tokens 550 /
 // 413, 700 671 / 510.  Of Gafulix 1.7B and 8B the experts' weights take the GPU 200 to 900 us, so that the host's time is hidden: a
 // product of 15 to 20 us is the library's there (busy; 1700 rows, 2048 -> 2048: 27 here, 17 there; the passes are within 1 % of what

@@ -168,8 +168,11 @@ class HybridEngine(EngineCore):
             return ops.skinny_linear(x, w, b, activation=activation, param=param)
         if activation is not None and b is None and ops.dense_activation_wanted(x, w):
             return ops.dense_activation(x, w, activation, param)
-        y = ops.dense_linear(x, w, b) if ops.dense_linear_wanted(x, w, False, self._busy) else F.linear(x, w, b)
+        y = self._many_rows(x, w, b)
         return y if activation is None else ops.activate_(y, activation, param)
+
+    def _many_rows(self, x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -> torch.Tensor:
+        return ops.dense_linear(x, w, b) if ops.dense_linear_wanted(x, w, False, self._busy) else F.linear(x, w, b)
 
     def _sublayer_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """The product that ends a sublayer, as sums of its parts, which the residual's next read adds, where one part leaves CUs idle."""
@@ -209,7 +212,7 @@ class HybridEngine(EngineCore):
             q = ops.latent_store(proj, w.latent_norm, cos_sin, step.positions, step.slots, cache, m.heads, m.dim, rot_at, eps,
                                  wide, m.dim, True)
             latents = ops.latent_gather(cache, step.layout, m.rank, rot, rot_at)
-            return ops.latent_attention_prefill(q, F.linear(latents[:, :m.rank], w.expand), latents[:, m.rank:], step.layout,
+            return ops.latent_attention_prefill(q, self._many_rows(latents[:, :m.rank], w.expand), latents[:, m.rank:], step.layout,
                                                 m.dim, m.vdim, m.scale)
         into, out_of = self._per_head[self.runs[run][0]]
         q = ops.latent_store(proj, w.latent_norm, cos_sin, step.positions, step.slots, cache, m.heads, m.dim, rot_at, eps, row,
