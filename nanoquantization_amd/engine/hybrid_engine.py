@@ -28,7 +28,7 @@ import torch.nn.functional as F
 from ..models.hybrid import (AttentionSpec, DenseSpec, GatedLinearSpec, HybridDecoder, LatentAttentionSpec, RotarySpec,
                              SelectiveScanSpec, rotary_table)
 from . import hybrid_ops as ops
-from .cache import Lease, PagedKVCache, RecurrentStateCache, upload
+from .cache import Lease, PagedKVCache, RecurrentStateCache
 from .core import EngineCore
 
 
@@ -132,6 +132,11 @@ class HybridEngine(EngineCore):
         self._busy = any(l.mlp is not None and not isinstance(s.mlp, DenseSpec)
                          and l.mlp.gate_up.nbytes + l.mlp.down.nbytes > 150 << 20 for s, l in zip(spec.layers, model.layers))
         mixers = [spec.layers[i].mixer for i, _ in self.runs]
+        # rows of a piece, by the rows of a pass, for every kind of layer that takes a pass in pieces
+        self._latent = any(isinstance(m, LatentAttentionSpec) for m in mixers)
+        self._piece_sizes = [lambda rows, m=m: ops.scan_piece_rows(rows, m.channels, m.state) if isinstance(m, SelectiveScanSpec) else
+                             ops.gla_piece_rows(rows, m.heads, m.dim, m.vdim)
+                             for m in dict.fromkeys(mixers) if isinstance(m, (SelectiveScanSpec, GatedLinearSpec))]
         self.cache = PagedKVCache(len(mixers), self.num_blocks, block_size, dtype=self.dtype, device=self.device,
                                   layer_shapes=[self._cache_shape(m) for m in mixers])
         state_shapes, tail_shapes = zip(*(self._state_shapes(m) for m in mixers))
@@ -290,7 +295,7 @@ class HybridEngine(EngineCore):
             if n < 1 or p.start < 0 or p.start + n > min(len(p.lease.blocks) * bs, self.max_ctx):
                 raise ValueError(f"{n} tokens from position {p.start} do not fit the sequence's "
                                  f"{len(p.lease.blocks)} blocks of {bs} tokens")
-            plain = isinstance(p.tokens, (range, np.ndarray)) or all(type(t) is int for t in p.tokens)
+            plain = isinstance(p.tokens, (range, np.ndarray)) or set(map(type, p.tokens)) == {int}
             tokens = np.array(p.tokens if plain else [int(t) for t in p.tokens], dtype=np.int64)
             if tokens.min() < 0 or tokens.max() >= self.spec.vocab:
                 raise ValueError("token id outside the vocabulary")
@@ -300,11 +305,11 @@ class HybridEngine(EngineCore):
             slots.append(np.array(p.lease.blocks, dtype=np.int64)[t // bs] * bs + t % bs)
             want += [first + w for w in p.want]
             first += n
-        layout = ops.PromptPass([(p.start, len(p.tokens), p.lease.blocks, p.lease.slot) for p in portions], bs, dev)
-        packed = upload(np.concatenate(ids + pos + slots + [np.array(want, dtype=np.int64)]), dev)
-        ids_d, pos_d, slots_d, rows = packed.split([first, first, first, len(want)])
-
-        step = Step(ids_d, pos_d, slots_d, layout=layout)
+        more = [np.concatenate(x) for x in (ids, pos, slots)] + [np.array(want, dtype=np.int64)]
+        layout = ops.PromptPass([(p.start, len(p.tokens), p.lease.blocks, p.lease.slot) for p in portions], bs, dev,
+                                [size(first) for size in self._piece_sizes], self._latent and first > self.absorb_rows, more)
+        *lists, rows = layout.more
+        step = Step(*lists, layout=layout)
         if not want:        # the pass still fills cache and state
             self._layers(step, trace=trace)
             return torch.empty(0, self.spec.vocab, dtype=torch.float32, device=dev)

@@ -5,7 +5,7 @@ and launches on the current stream.  HIP device tensors only; bfloat16 or float3
 from __future__ import annotations
 
 import functools
-from typing import Optional, Sequence, Tuple
+from typing import List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -206,9 +206,11 @@ def _check_attention(q, k_cache, v_cache, heads):
 class PromptPass:
     """The layout of a pass over portions of several sequences: segment i is `rows` consecutive tokens of one sequence from
     position `start`, with the cache blocks `blocks` and the state slot `slot`; the segments' tokens lie one after the
-    other.  Holds the device-side lists of the prompt kernels."""
+    other.  Holds the device-side lists of the prompt kernels, which come there in one copy (on the host a copy takes some 13 us):
+    those that every pass wants, the pieces of `piece_sizes`, the contexts and the int64 numbers `more`; others when asked for."""
 
-    def __init__(self, segments: Sequence[Tuple[int, int, Sequence[int], int]], block_size: int, device: torch.device):
+    def __init__(self, segments: Sequence[Tuple[int, int, Sequence[int], int]], block_size: int, device: torch.device,
+                 piece_sizes: Sequence[int] = (), contexts: bool = False, more: Sequence[np.ndarray] = ()):
         self.segments = list(segments)                       # (start, rows, blocks, slot)
         self.device = device
         self.rows = sum(s[1] for s in self.segments)
@@ -226,17 +228,33 @@ class PromptPass:
         tiles.sort(reverse=True)                             # the tiles with the most keys first
         flat = [x for _, i, q0 in tiles for x in (i, q0)]
         self.num_tiles, self.max_blocks = len(tiles), width
-        packed = upload(np.concatenate([table.reshape(-1), np.array(seg + flat, dtype=np.int32)]), device)
-        self.tables, self.seg, self.tiles = packed.split([table.size, len(seg), len(flat)])
-        self._pieces, self._contexts, self._row_tables = {}, None, None
+        sizes = list(dict.fromkeys(piece_sizes))
+        lists = [self._piece_list(s) for s in sizes]
+        ahead = self._context_list() if contexts else []
+        parts = [x.view(np.int32) for x in more]             # first: eight bytes each
+        parts += [table.reshape(-1)] + [np.array(x, dtype=np.int32) for x in [seg, flat, ahead] + [l for l, _ in lists]]
+        out = upload(np.concatenate(parts), device).split([len(p) for p in parts])
+        self.more, out = [x.view(torch.int64) for x in out[:len(more)]], out[len(more):]
+        self.tables, self.seg, self.tiles, first_of = out[:4]
+        self._pieces = {s: (x, len(l) // 6, chained) for s, x, (l, chained) in zip(sizes, out[4:], lists)}
+        self._contexts, self._row_tables = self._with_lengths(first_of) if contexts else None, None
 
     def contexts(self) -> Tuple[torch.Tensor, int, int]:
         """The segments' contexts laid out one after the other: (first row of each, int32; rows in all; the longest)."""
         if self._contexts is None:
-            lens = [start + rows for start, rows, _, _ in self.segments]
-            first = [sum(lens[:i]) for i in range(len(lens))]
-            self._contexts = upload(np.array(first, dtype=np.int32), self.device), sum(lens), max(lens)
+            self._contexts = self._with_lengths(upload(np.array(self._context_list(), dtype=np.int32), self.device))
         return self._contexts
+
+    def _context_list(self) -> List[int]:
+        out, at = [], 0
+        for start, rows, _, _ in self.segments:
+            out.append(at)
+            at += start + rows
+        return out
+
+    def _with_lengths(self, first: torch.Tensor) -> Tuple[torch.Tensor, int, int]:
+        lens = [start + rows for start, rows, _, _ in self.segments]
+        return first, sum(lens), max(lens)
 
     def row_tables(self) -> Tuple[torch.Tensor, torch.Tensor]:
         """The pass as a decode step sees it, every token a row of its own: (block tables [rows, max_blocks], tokens in the
@@ -252,15 +270,19 @@ class PromptPass:
         """(list of pieces of at most `size` rows for gla_prefill and scan_prefill, its length, whether a sequence has
         several)."""
         if size not in self._pieces:
-            out, first, chained = [], 0, False
-            for start, rows, _, slot in self.segments:
-                n = (rows + size - 1) // size
-                chained |= n > 1
-                for p in range(n):
-                    out += [first + p * size, min(size, rows - p * size), slot, int(start == 0), p, n]
-                first += rows
+            out, chained = self._piece_list(size)
             self._pieces[size] = upload(np.array(out, dtype=np.int32), self.device), len(out) // 6, chained
         return self._pieces[size]
+
+    def _piece_list(self, size: int) -> Tuple[List[int], bool]:
+        out, first, chained = [], 0, False
+        for start, rows, _, slot in self.segments:
+            n = (rows + size - 1) // size
+            chained |= n > 1
+            for p in range(n):
+                out += [first + p * size, min(size, rows - p * size), slot, int(start == 0), p, n]
+            first += rows
+        return out, chained
 
 
 def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, layout: PromptPass, dim: int, vdim: int,
@@ -520,6 +542,10 @@ def gla_decay(proj: torch.Tensor, up: torch.Tensor, bias: torch.Tensor, heads: i
     return decay
 
 
+def gla_piece_rows(rows: int, heads: int, dim: int, vdim: int) -> int:
+    return _lib.hybrid_lib().nqh_gla_piece_rows(rows, heads, dim, vdim)
+
+
 def gla_prefill(proj: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, layout: PromptPass, heads: int, dim: int,
                 vdim: int, rank: int) -> torch.Tensor:
     """The tokens of the pass through the recurrence: state fp32 [slots, heads, dim, vdim] IN PLACE at the segments' slots
@@ -530,7 +556,7 @@ def gla_prefill(proj: torch.Tensor, decay: torch.Tensor, state: torch.Tensor, la
     assert all(0 <= s[3] < state.shape[0] for s in layout.segments)
     assert decay.shape == (rows, heads * dim) and decay.dtype == torch.float32
     q, k, v, _, _ = _gla_offsets(proj, heads, dim, vdim, rank)
-    pieces, n, chained = layout.pieces(_lib.hybrid_lib().nqh_gla_piece_rows(rows, heads, dim, vdim))
+    pieces, n, chained = layout.pieces(gla_piece_rows(rows, heads, dim, vdim))
     nbytes = _lib.hybrid_lib().nqh_gla_prefill_workspace_bytes(n, heads, dim, vdim) if chained else 0
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
     o = torch.empty(rows, heads * vdim, dtype=torch.float32, device=dev)
