@@ -1143,9 +1143,9 @@ __global__ __launch_bounds__(64 * WK) void gemv_dma_kernel(
 //   buffer = [x: 4 steps x (MT*16 rows x 64 B)] [tile 0..3: 8 KiB weights + 512 B zeros/scales]
 // Waves wn and wn + 4 work on the same column tile and the same rows, one on bytes 0-1 of every word
 // (even output columns), the other on bytes 2-3 (odd columns).  Nothing is unpacked or scaled twice, each
-// wave holds half the accumulators, and every SIMD has two waves.  What bounds this regime is the vector
-// ALU port (one instruction per SIMD every four cycles: about 270 unpack, 140 scale/zero and 2 x 144 MFMA
-// issue slots per 128 x 128 weights at 64 rows), not the memory.
+// wave holds half the accumulators, and every SIMD has two waves.  What bounds this regime is the SIMD's
+// issue port, not the memory: per wave and 128 x 64 weights at 64 rows 80 MFMAs, which take it for 8 of their
+// 16 cycles, and 299 vector instructions at 4.7 (128 of them unpack, 128 apply scale and zero point).
 // At the end the two halves exchange fragments through LDS so that each stores whole words of half the rows.
 // A K split leaves fp32 partials that a second kernel adds in split order -- or, TAIL (one m-tile, a few rows), the
 // last workgroup of the 512 columns to arrive, as in the one-tile kernel.
