@@ -489,6 +489,29 @@ def test_engine_shapes_outside_the_fused_decode_forms(group_size, max_batch):
         assert _teacher_forced_check(model, prompts, got) > 0.5
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 16, 17, 65])
+def test_engine_logits_are_those_of_lm_head(rows):
+    """Up to the rows that its kernel takes and past them, with a bias; and a hook on lm_head sees what passes through it."""
+    from nanoquantization_amd.engine import LLMEngine
+    from nanoquantization_amd.models.random_init import random_awq_qwen3
+    print(f"engine logits of {rows} rows", flush=True)
+    model = random_awq_qwen3(TINY, seed=5, std=0.05)
+    eng = LLMEngine(model, max_batch=4, max_seq_len=64, block_size=16, use_graph=False)
+    head = model.lm_head
+    torch.manual_seed(rows)
+    h = torch.randn(rows, head.in_features, device="cuda").to(head.weight.dtype)
+    want = h.double() @ head.weight.double().T + (0 if head.bias is None else head.bias.double())
+    with torch.no_grad():
+        got = eng._logits(h)
+        assert got.dtype == h.dtype and got.shape == want.shape
+        assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4 * want.abs().max()).all()     # one rounding of fp32 sums
+        seen = []
+        hook = head.register_forward_hook(lambda m, i, o: seen.append(o))
+        assert torch.allclose(eng._logits(h).float(), got.float(), rtol=2.0 ** -7, atol=1e-3) and len(seen) == 1
+        hook.remove()
+
+
 def test_paged_kv_cache_block_bookkeeping():
     """Host logic of the cache: blocks are handed out once, come back on release, exhaustion raises (CPU)."""
     from nanoquantization_amd.engine.llm_engine import PagedKVCache
