@@ -2125,9 +2125,13 @@ static void pick_gemv(int64_t M, int64_t N, int64_t K, int64_t g, int* variant, 
             // streaming-bound, and with 144 workgroups or more any split only adds its tail -- 2560 x 9728 at 64 rows
             // 27.2 us in five splits, 16.8 unsplit (304 workgroups); at 32 rows 16.2 -> 13.1; 2048 x 6144 at 64 rows
             // 12.3 -> 9.7, at 48 rows (144 workgroups) 11.9 -> 10.2; likewise four row blocks of 128 tiles or more:
-            // 2560 x 19456 at 64 rows 33.4 -> 23.4.
+            // 2560 x 19456 at 64 rows 33.4 -> 23.4; and two row blocks of 128 tiles or more up to K of 4096 (where the shared
+            // chunk is not taken, with a norm of its input above all): at 17 / 32 rows 2560 x 19456 18.1 / 21.4 us in five splits,
+            // 15.3 / 16.5 unsplit, 4096 x 24576 28.6 / 31.8 in four, 26.2 / 28.5, 4096 x 16384 20.8 / 23.2 in five, 18.3 / 19.1;
+            // K of 5120 and more is level (5120 x 25600 at 32 rows 34.7 in two, 35.3 unsplit).
             const bool unsplit = row_blocks >= 2 && wgs >= 144 &&
-                                 (K * N < (32ll << 20) || (row_blocks >= 4 && wgs >= 512));
+                                 (K * N < (32ll << 20) || (row_blocks >= 4 && wgs >= 512) ||
+                                  (row_blocks == 2 && wgs >= 256 && chunks <= 32));
             int64_t s0 = wgs < 200 ? cdiv(200, wgs) : 1;
             if (s0 > cap) s0 = cap;
             const int64_t hi = s0 + 5 < cap ? s0 + 5 : cap;
