@@ -22,11 +22,10 @@ from __future__ import annotations
 from typing import List, Optional
 
 import torch
-import torch.nn as nn
 import torch.nn.functional as F
 
 from ..layers.gemm import _linear, prefetch_hint
-from ..layers.inference import plain, unhooked
+from ..layers.inference import is_torch_linear, plain, unhooked
 from . import hybrid_ops, ops
 from .cache import Lease, PagedKVCache
 from .core import EngineCore
@@ -197,7 +196,7 @@ class LLMEngine(EngineCore):
         62.4, of 4096 256 / 203, 253 / 232.  From 17 rows on narrow ones are the library's (1024, 24 / 64 rows 16.5 / 16.9, 17.4 / 19.8), from 49 on
         those below 4096 (2560, 64 rows 39.6 / 41.4)."""
         head = self.model.lm_head
-        if (type(head) is nn.Linear and "forward" not in head.__dict__ and unhooked(head) and plain(h, head.weight)
+        if (is_torch_linear(head) and unhooked(head) and plain(h, head.weight)
                 and hybrid_ops.skinny_linear_supported(h.shape[0], head.weight) and head.weight.is_contiguous()
                 and (head.weight.data_ptr() | h.data_ptr()) % 16 == 0
                 and h.shape[0] <= (16 if head.in_features < 2048 else 48 if head.in_features < 4096 else hybrid_ops.SKINNY_ROWS)

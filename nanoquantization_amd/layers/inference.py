@@ -42,6 +42,12 @@ def keeps(module: torch.nn.Module, cls: type, *names: str) -> bool:
     return all(n not in module.__dict__ and getattr(type(module), n, None) is _SHIPPED[cls, n] for n in names)
 
 
+def is_torch_linear(module: torch.nn.Module) -> bool:
+    """An nn.Linear with the forward that torch gives it, replaced neither on the module nor on the class."""
+    return (type(module) is torch.nn.Linear and "forward" not in module.__dict__
+            and getattr(torch.nn.Linear.forward, "__globals__", None) is vars(torch.nn.modules.linear))
+
+
 def unhooked(*modules: torch.nn.Module) -> bool:
     """No caller wants to see the inputs or outputs of these modules."""
     return not (torch.nn.modules.module._has_any_global_hook() or any(m._forward_hooks or m._forward_pre_hooks for m in modules))

@@ -1,5 +1,6 @@
 """The callers of the hot path: Qwen3 model contract (CPU), checkpoint round trip (CPU), and on the GPU
 the paged-KV engine against the model's own no-cache forward (the reference semantics)."""
+import functools
 import json
 import os
 
@@ -510,6 +511,43 @@ def test_engine_logits_are_those_of_lm_head(rows):
         hook = head.register_forward_hook(lambda m, i, o: seen.append(o))
         assert torch.allclose(eng._logits(h).float(), got.float(), rtol=2.0 ** -7, atol=1e-3) and len(seen) == 1
         hook.remove()
+
+
+@pytest.mark.gpu
+def test_engine_logits_hear_a_replaced_forward(monkeypatch):
+    """lm_head's own kernel stands in for torch's nn.Linear.forward only, not for one that the caller has put there."""
+    from nanoquantization_amd.engine import LLMEngine
+    from nanoquantization_amd.models.random_init import random_awq_qwen3
+    print("engine logits, forward replaced", flush=True)
+    model = random_awq_qwen3(TINY, seed=5, std=0.05)
+    eng = LLMEngine(model, max_batch=4, max_seq_len=64, block_size=16, use_graph=False)
+    h = torch.randn(3, model.lm_head.in_features, device="cuda").to(model.lm_head.weight.dtype)
+    with torch.no_grad():
+        plain = eng._logits(h)
+        shipped = torch.nn.Linear.forward
+        with monkeypatch.context() as m:
+            m.setattr(torch.nn.Linear, "forward", lambda self, x: shipped(self, x) + 1)
+            assert torch.allclose(eng._logits(h).float(), plain.float() + 1, rtol=2.0 ** -7, atol=1e-2)
+        with monkeypatch.context() as m:
+            m.setitem(model.lm_head.__dict__, "forward", lambda x: shipped(model.lm_head, x) + 2)
+            assert torch.allclose(eng._logits(h).float(), plain.float() + 2, rtol=2.0 ** -7, atol=1e-2)
+        assert torch.equal(eng._logits(h), plain)
+
+
+def test_an_nn_linear_is_torchs_own(monkeypatch):
+    """is_torch_linear: no subclass, no forward of the caller's on the module or on the class (CPU)."""
+    from nanoquantization_amd.layers.inference import is_torch_linear
+    head = torch.nn.Linear(4, 4)
+    assert is_torch_linear(head)
+    assert not is_torch_linear(type("Own", (torch.nn.Linear,), {})(4, 4)) and not is_torch_linear(torch.nn.ReLU())
+    with monkeypatch.context() as m:
+        m.setitem(head.__dict__, "forward", lambda x: x)
+        assert not is_torch_linear(head)
+    shipped = torch.nn.Linear.forward
+    with monkeypatch.context() as m:
+        m.setattr(torch.nn.Linear, "forward", functools.wraps(shipped)(lambda self, x: shipped(self, x)))
+        assert not is_torch_linear(head)
+    assert is_torch_linear(head)
 
 
 def test_paged_kv_cache_block_bookkeeping():
