@@ -182,8 +182,9 @@ class HybridEngine(EngineCore):
     def _sublayer_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """The product that ends a sublayer, as sums of its parts, which the residual's next read adds, where one part leaves CUs idle."""
         if ops.skinny_linear_supported(x.shape[0], w):
-            return ops.skinny_linear_sums(x, w)
-        sums = ops.dense_linear_sums(x, w) if ops.dense_linear_wanted(x, w, True, self._busy) else None
+            sums = ops.skinny_linear_sums(x, w)
+        else:
+            sums = ops.dense_linear_sums(x, w) if ops.dense_linear_wanted(x, w, True, self._busy) else None
         return self._linear(x, w) if sums is None else sums
 
     def _logits(self, h: torch.Tensor) -> torch.Tensor:

@@ -668,20 +668,22 @@ def skinny_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
     assert bias is None or (bias.shape == (weight.shape[0],) and bias.dtype == torch.bfloat16)
     y = torch.empty(rows, weight.shape[0], dtype=torch.float32 if out_f32 else torch.bfloat16, device=dev)
     nbytes = _of_sizes("nqh_skinny_linear_scratch_bytes", rows, weight.shape[0], n, int(torch.cuda.is_current_stream_capturing()))
-    scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    scratch = _room(dev, nbytes)
     _call(dev, "nqh_skinny_linear_ex", x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), rows, weight.shape[0], n,
-          int(out_f32), ACTIVATIONS[activation], param, _ptr(scratch), nbytes)
+          int(out_f32), ACTIVATIONS[activation], param, _ptr(scratch), 0 if scratch is None else nbytes)
     return y
 
 
-def skinny_linear_sums(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+def skinny_linear_sums(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
     """x [rows <= 64, in] bf16 @ weight [out, in]^T for a reader that adds: fp32 [rows, parts, out], the sums of as many parts of the
-    contraction as keep the GPU busy."""
+    contraction as keep the GPU busy; None where there is no memory for them."""
     dev = _dev(x, weight)
     rows, n = x.shape
     assert weight.shape[1] == n and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
     parts = _of_sizes("nqh_skinny_linear_parts", rows, weight.shape[0], n)
-    sums = torch.empty(rows, parts, weight.shape[0], dtype=torch.float32, device=dev)
+    sums = _room(dev, rows, parts, weight.shape[0], dtype=torch.float32)
+    if sums is None:
+        return None
     _call(dev, "nqh_skinny_linear_sums", x.data_ptr(), weight.data_ptr(), sums.data_ptr(), rows, weight.shape[0], n)
     return sums
 
@@ -720,16 +722,16 @@ def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
     assert x.dtype == weight.dtype == torch.bfloat16
     assert bias is None or (bias.shape == (weight.shape[0],) and bias.dtype == torch.bfloat16)
     y = torch.empty(rows, weight.shape[0], dtype=torch.bfloat16, device=dev)
-    scratch = _room(_of_sizes("nqh_dense_linear_scratch_bytes", rows, *weight.shape), dev)
+    scratch = _room(dev, _of_sizes("nqh_dense_linear_scratch_bytes", rows, *weight.shape))
     _call(dev, "nqh_dense_linear", x.data_ptr(), weight.data_ptr(), _ptr(bias), y.data_ptr(), rows, weight.shape[0], n, x.stride(0) if rows > 1 else n,
           _ptr(scratch), 0 if scratch is None else scratch.numel())
     return y
 
 
-def _room(nbytes: int, dev: torch.device) -> Optional[torch.Tensor]:
+def _room(dev: torch.device, *sizes: int, dtype: torch.dtype = torch.uint8) -> Optional[torch.Tensor]:
     """Memory for one call, None if none is wanted or left."""
     try:
-        return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+        return torch.empty(sizes, dtype=dtype, device=dev) if all(sizes) else None
     except torch.cuda.OutOfMemoryError:
         return None
 
@@ -740,10 +742,9 @@ def dense_linear_sums(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.T
     rows, n = x.shape
     assert weight.shape[1] == n and x.dtype == weight.dtype == torch.bfloat16
     parts = _of_sizes("nqh_dense_linear_parts", rows, *weight.shape)
-    sums = _room(4 * rows * parts * weight.shape[0], dev) if parts > 1 else None
+    sums = _room(dev, rows, parts, weight.shape[0], dtype=torch.float32) if parts > 1 else None
     if sums is None:
         return None
-    sums = sums.view(torch.float32).view(rows, parts, weight.shape[0])
     _call(dev, "nqh_dense_linear_sums", x.data_ptr(), weight.data_ptr(), sums.data_ptr(), rows, weight.shape[0], n)
     return sums
 

@@ -529,6 +529,34 @@ def test_skinny_linear_parts(rows, n_out, n_in):
         close(y, want, torch.bfloat16)
 
 
+@pytest.mark.parametrize("rows", [16, 65])
+def test_linears_without_memory_for_parts(rows, monkeypatch):
+    """Where no memory is left for the sums of parts, a linear of an engine runs unsplit into its plain result."""
+    from nanoquantization_amd.engine.hybrid_engine import HybridEngine
+    print(f"linear without memory for parts, {rows} rows", flush=True)
+    n_out, n_in = 4096, 18432
+    x, w = (rand(*s, seed=i, dtype=torch.bfloat16) for i, s in enumerate([(rows, n_in), (n_out, n_in)]))
+    xd, wd = x.cuda(), w.cuda()
+    want = (xd.double() @ wd.double().T).cpu()
+    engine = HybridEngine.__new__(HybridEngine)
+    engine._busy = False
+    parts = engine._sublayer_linear(xd, wd)
+    assert parts.dim() == 3 and parts.shape[1] > 1                 # there is something to do without
+    empty = torch.empty
+
+    def little(*size, **kw):
+        t = empty(*size, **kw)
+        if t.numel() * t.element_size() > rows * n_out * 2:
+            raise torch.cuda.OutOfMemoryError("only the result fits")
+        return t
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", little)
+        y, alone = engine._sublayer_linear(xd, wd), engine._linear(xd, wd)
+    assert y.shape == (rows, n_out) and y.dtype == torch.bfloat16
+    close(y, want, torch.bfloat16)
+    close(alone, want, torch.bfloat16)
+
+
 @pytest.mark.parametrize("rows,width,parts", [(1, 64, 1), (3, 1024, 2), (2, 50, 3), (5, 2052, 7), (2, 4096, 16), (300, 72, 5)])
 def test_norms_add_the_parts_of_a_product(rows, width, parts):
     """The residual's next read with fp32 parts equals the one with their sum."""
