@@ -177,6 +177,7 @@ extern "C" int nqh_hyper_norm_parts(float* x, const int64_t* ids, const void* ta
 extern "C" int nqh_hyper_norm(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y,
                               const void* mix, const void* w_out, const void* w_in, const void* norm_weight, void* h,
                               int64_t rows, int64_t streams, int64_t width, float eps, int dtype, void* stream) {
+    if (!dtype_ok(dtype)) return fail(NQH_ERR_ARG, "nqh_hyper_norm", "dtype must be NQH_BF16 or NQH_F32");   // y is of that type here
     return nqh_hyper_norm_parts(x, ids, table, table_rows, y, 1, mix, w_out, w_in, norm_weight, h, rows, streams, width, eps, dtype,
                                 stream);
 }

@@ -5,6 +5,7 @@ import json
 import os
 import re
 
+import numpy as np
 import pytest
 import torch
 
@@ -42,6 +43,15 @@ def test_library_exports_every_declared_symbol():
         for used in range(1, min(pairs, experts) + 1):
             worst = max(worst, (used - 1) + -(-(pairs - used + 1) // rows))
         assert L.nqh_moe_max_tiles(pairs, experts, rows) >= worst
+
+
+def test_hyper_norm_takes_no_fp32_sums():
+    """NQH_Y_F32 belongs to nqh_hyper_norm_parts: nqh_hyper_norm refuses it, before anything is launched."""
+    lib, room = _lib.hybrid_lib(), np.zeros(64, dtype=np.float32)
+    at = room.ctypes.data
+    for dtype in (1 | 4, 2 | 4, 4, 0, 3):
+        assert lib.nqh_hyper_norm(at, None, None, 0, at, at, at, None, at, at, 1, 1, 8, 1e-5, dtype, None) == 1, dtype
+        assert b"dtype" in lib.nqh_last_error()
 
 
 @pytest.mark.parametrize("name", sorted(CONFIGS))
