@@ -177,7 +177,8 @@ class HybridEngine(EngineCore):
         return y if activation is None else ops.activate_(y, activation, param)
 
     def _many_rows(self, x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -> torch.Tensor:
-        return ops.dense_linear(x, w, b) if ops.dense_linear_wanted(x, w, False, self._busy) else F.linear(x, w, b)
+        own = ops.dense_linear_wanted(x, w, False, self._busy) and (b is None or b.is_contiguous())
+        return ops.dense_linear(x, w, b) if own else F.linear(x, w, b)
 
     def _sublayer_linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """The product that ends a sublayer, as sums of its parts, which the residual's next read adds, where one part leaves CUs idle."""

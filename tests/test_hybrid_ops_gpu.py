@@ -529,6 +529,19 @@ def test_skinny_linear_parts(rows, n_out, n_in):
         close(y, want, torch.bfloat16)
 
 
+def test_linear_of_many_rows_with_a_strided_bias():
+    """The library's product takes what dense_linear does not."""
+    from nanoquantization_amd.engine.hybrid_engine import HybridEngine
+    print("linear of 300 rows, strided bias", flush=True)
+    x, w, b = (rand(*s, seed=i, dtype=torch.bfloat16).cuda() for i, s in enumerate([(300, 1024), (2048, 1024), (2048, 2)]))
+    engine = HybridEngine.__new__(HybridEngine)
+    engine._busy = False
+    assert ops.dense_linear_wanted(x, w, False, False)
+    want = (x.double() @ w.double().T + b[:, 1].double()).cpu()
+    close(engine._linear(x, w, b[:, 1]), want, torch.bfloat16)
+    close(engine._linear(x, w, b[:, 1].contiguous()), want, torch.bfloat16)
+
+
 @pytest.mark.parametrize("rows", [16, 65])
 def test_linears_without_memory_for_parts(rows, monkeypatch):
     """Where no memory is left for the sums of parts, a linear of an engine runs unsplit into its plain result."""
