@@ -260,6 +260,12 @@ int64_t nqh_skinny_linear_parts(int64_t rows, int64_t out_features, int64_t in_f
 int nqh_skinny_linear_sums(const void* x, const void* weight, float* sums, int64_t rows, int64_t out_features, int64_t in_features,
                            void* stream);
 
+/* What these run: the tiles of 16 features of a workgroup (1: the waves of one tile split the contraction; 2, 4, 8: a stream of the
+ * weight), *parts (may be null) the parts of the contraction; 0 for sizes that are not taken.  adds: nobody (nqh_skinny_linear), a
+ * pass behind it (nqh_skinny_linear_ex with scratch memory), the reader (nqh_skinny_linear_sums). */
+enum { NQH_ADDS_NOBODY = 0, NQH_ADDS_PASS = 1, NQH_ADDS_READER = 2 };
+int nqh_skinny_linear_form(int64_t rows, int64_t out_features, int64_t in_features, int adds, int64_t* parts);
+
 /* y [rows, out_features] = act(x @ weight^T), bf16, act applied to the product rounded to bf16; for many rows.  in_features a
  * multiple of 64, out_features one of 8, all pointers 16-byte aligned, rows without padding.  act and param as in nqh_activate.
  * nqh_dense_activation_wanted: 1 where it takes the sizes and one launch of it is done before a library product with nqh_activate
@@ -281,6 +287,9 @@ int nqh_dense_linear(const void* x, const void* weight, const void* bias, void* 
 int64_t nqh_dense_linear_parts(int64_t rows, int64_t out_features, int64_t in_features);
 int nqh_dense_linear_sums(const void* x, const void* weight, float* sums, int64_t rows, int64_t out_features, int64_t in_features,
                           void* stream);
+
+/* The rows of the tiles that these run, 128 or 256, and *parts; 0 and adds as for nqh_skinny_linear_form. */
+int nqh_dense_linear_form(int64_t rows, int64_t out_features, int64_t in_features, int adds, int64_t* parts);
 
 /* Decode-step bookkeeping, as nq_argmax_rows / nq_decode_prepare / nq_decode_advance (nq_engine_ops.h) do it; the
  * logits are fp32. */

@@ -136,11 +136,13 @@ HYBRID_SYMBOLS = {
     "nqh_skinny_linear_scratch_bytes": (_sz, [_i64] * 3 + [_int]),
     "nqh_skinny_linear_ex": (_int, [_vp] * 4 + [_i64] * 3 + [_int, _int, _f32, _vp, _sz, _vp]),
     "nqh_skinny_linear_parts": (_i64, [_i64] * 3),
+    "nqh_skinny_linear_form": (_int, [_i64] * 3 + [_int, _vp]),
     "nqh_skinny_linear_sums": (_int, [_vp] * 3 + [_i64] * 3 + [_vp]),
     "nqh_dense_linear_wanted": (_int, [_i64] * 3 + [_int] * 2),
     "nqh_dense_linear_scratch_bytes": (_sz, [_i64] * 3),
     "nqh_dense_linear": (_int, [_vp] * 4 + [_i64] * 4 + [_vp, _sz, _vp]),
     "nqh_dense_linear_parts": (_i64, [_i64] * 3),
+    "nqh_dense_linear_form": (_int, [_i64] * 3 + [_int, _vp]),
     "nqh_dense_linear_sums": (_int, [_vp] * 3 + [_i64] * 3 + [_vp]),
     "nqh_dense_activation_wanted": (_int, [_i64] * 3),
     "nqh_dense_activation": (_int, [_vp] * 3 + [_i64] * 3 + [_int, _f32, _vp]),

@@ -261,7 +261,10 @@ enum class Sums { kNone, kOwnPass, kIssuedPass, kReader };
 // 12 % longer.  Fitted to 32 weights (544 to 32768 x 1024 to 18432) at 1 to 64 rows, every form and split, from
 // memory: 3.6 % off in the middle, 9.5 % in one of ten; the chosen form takes 0.4 % (nobody adds), 1.6 % (own pass) and 1.1 % (reader)
 // longer than the fastest on average, 16 % at worst.  Long contractions and, the other way, few rows of many features are
-// where skinny_linear_kernel is off the estimate.
+// where skinny_linear_kernel is off the estimate; so are few rows where the rows of the weight are a power of two of 8 KB and more
+// apart, which costs the streams a tenth and it nothing (4096 -> 32768 at 4 rows 48.6 us, as streams 51 to 54; 4096 -> 65536 90, 97
+// to 100).  Over 163 weights (96 to 151936 x 512 to 18432) at 1 to 16 rows, nobody adding, the choice is 0.7 % from the fastest on
+// average; with no such factor and 1.12 for long contractions it was 1.2 %, and 16 rows of 12288 -> 1024 took 30.6 us as a stream, 24.9 here.
 LinearPlan make_linear_plan(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) {
     struct Of {
         double launch, memory, rate, more;       // us, MB/us, KB/us for one tile of rows and so many more for four
@@ -273,8 +276,9 @@ LinearPlan make_linear_plan(int64_t rows, int64_t n_out, int64_t n_in, Sums sums
     const int64_t groups = cdiv(n_out, 16) * cdiv(rows, 16), few = std::min<int64_t>(rows, 16), pieces = cdiv(n_in, kPiece);
     LinearPlan best{kSkinny, 1};
     double least = kOf[0].launch + hypot2(cdiv(groups, 256) * n_in * 2e-3 * (16 + few) / (kOf[0].rate + kOf[0].more * few / 16), mb / kOf[0].memory);
-    if (rows <= 4 && n_out >= 16384) least *= 0.93;
-    if (n_in >= 8192) least *= 1.12;
+    if (rows <= 5 && n_out >= 16384) least *= 0.93;
+    if (rows <= 6 && n_out >= 16384 && n_in >= 4096 && (n_in & (n_in - 1)) == 0) least *= 0.9;
+    if (n_in >= 8192) least *= 1.06;
     if (n_in > (1 << 24)) return best;             // 32-bit offsets into 16 rows of the weight and all of x
     const int mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
     for (const Form form : {kTwo, kFour, kEight}) {
@@ -513,6 +517,13 @@ extern "C" int nqh_skinny_linear_sums(const void* x, const void* weight, float* 
                     in_features, 1, NQH_ACT_NONE, 0.f, (hipStream_t)stream);
 }
 
+extern "C" int nqh_skinny_linear_form(int64_t rows, int64_t out_features, int64_t in_features, int adds, int64_t* parts) {
+    if (!skinny_takes(rows, out_features, in_features) || adds < NQH_ADDS_NOBODY || adds > NQH_ADDS_READER) return 0;
+    const LinearPlan plan = plan_linear(rows, out_features, in_features, adds == NQH_ADDS_NOBODY ? Sums::kNone : adds == NQH_ADDS_PASS ? Sums::kOwnPass : Sums::kReader);
+    if (parts) *parts = plan.splits;
+    return 1 << plan.form;
+}
+
 extern "C" size_t nqh_skinny_linear_scratch_bytes(int64_t rows, int64_t out_features, int64_t in_features, int captured) {
     if (!skinny_takes(rows, out_features, in_features) ||
         plan_linear(rows, out_features, in_features, captured ? Sums::kOwnPass : Sums::kIssuedPass).splits == 1)
@@ -596,6 +607,13 @@ extern "C" int nqh_dense_linear_wanted(int64_t rows, int64_t out_features, int64
     return dense_activation_takes(rows, out_features, in_features) &&
            plan_dense(rows, out_features, in_features, reader ? Sums::kReader : Sums::kOwnPass).us <
                library_us(rows, out_features, in_features, busy != 0);
+}
+
+extern "C" int nqh_dense_linear_form(int64_t rows, int64_t out_features, int64_t in_features, int adds, int64_t* parts) {
+    if (!dense_activation_takes(rows, out_features, in_features) || adds < NQH_ADDS_NOBODY || adds > NQH_ADDS_READER) return 0;
+    const DensePlan plan = plan_dense(rows, out_features, in_features, adds == NQH_ADDS_NOBODY ? Sums::kNone : adds == NQH_ADDS_PASS ? Sums::kOwnPass : Sums::kReader);
+    if (parts) *parts = plan.splits;
+    return plan.xr;
 }
 
 extern "C" size_t nqh_dense_linear_scratch_bytes(int64_t rows, int64_t out_features, int64_t in_features) {

@@ -45,6 +45,20 @@ def test_library_exports_every_declared_symbol():
         assert L.nqh_moe_max_tiles(pairs, experts, rows) >= worst
 
 
+@pytest.mark.parametrize("rows,n_out,n_in", [(3, 32768, 4096), (5, 32768, 4096), (4, 65536, 4096), (4, 16384, 8192), (5, 18432, 4096),
+                                             (16, 544, 12288), (16, 1024, 18432), (16, 2048, 9216)])
+def test_linears_that_a_stream_is_slower_for(rows, n_out, n_in):
+    """Measured 5 to 23 % faster with the waves of a workgroup splitting the contraction than as any stream of the weight."""
+    assert _lib.hybrid_lib().nqh_skinny_linear_form(rows, n_out, n_in, 0, None) == 1
+
+
+def test_linears_that_a_stream_is_faster_for():
+    """Likewise 9 to 35 % the other way."""
+    lib = _lib.hybrid_lib()
+    for rows, n_out, n_in in ((16, 32768, 4096), (12, 151936, 2560), (5, 32768, 2560), (6, 12288, 2048), (4, 8192, 2560), (64, 9216, 2560)):
+        assert lib.nqh_skinny_linear_form(rows, n_out, n_in, 0, None) > 1, (rows, n_out, n_in)
+
+
 def test_hyper_norm_takes_no_fp32_sums():
     """NQH_Y_F32 belongs to nqh_hyper_norm_parts: nqh_hyper_norm refuses it, before anything is launched."""
     lib, room = _lib.hybrid_lib(), np.zeros(64, dtype=np.float32)
