@@ -1466,12 +1466,15 @@ __global__ __launch_bounds__(128 * WN) void gemv_wide_kernel(
 // are all of them, and a workgroup is one wave so that the sums of few rows are read by all CUs.  With both kernels, against eight
 // columns a thread in workgroups of 256: 4096 x 12288 at 16 / 32 rows 13.4 / 16.2 -> 12.0 / 14.8 us (256 threads on four columns: no
 // gain), 25600 x 5120 at 16 / 64 rows 21.5 / 35.1 -> 20.4 / 34.1, 12288 x 4096 at 32 rows 15.8 -> 14.6; 32 splits in flight: no more.
+// Where the sums of a split are a multiple of 2 MiB, so that all splits' loads ask the same memory channels, two waves: with one the call lost
+// against the former pass (64 rows 8192 x 8192 25.6 -> 26.2 us, now 25.65; 12288 x 8192 32.1 -> 32.9, now 31.9; elsewhere two waves
+// lose, 4096 x 12288 at 32 rows 16.1 -> 17.6).
 template <typename T, int SS>
-__global__ __launch_bounds__(64) void gemv_wide_reduce_kernel(const float* __restrict__ partials,
+__global__ __launch_bounds__(256) void gemv_wide_reduce_kernel(const float* __restrict__ partials,
                                                               const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
                                                               int M, int N, int splits, int act) {
     const int quads = N >> 2;
-    const int idx = blockIdx.x * 64 + threadIdx.x;
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= M * quads) return;   // N is a multiple of 16: gate columns and their up columns leave together
     const int m = idx / quads, q = idx - m * quads;
     const size_t n0 = (size_t)q * 4, plane = (size_t)M * N;
@@ -1854,9 +1857,9 @@ static hipError_t launch_gemv_wide(const void* x, const int32_t* qweight, const 
                            reinterpret_cast<uint16_t*>(y), an->weight, an->normed, M, N, splits, an->eps);
         return hipGetLastError();
     }
-    const dim3 grid((unsigned)cdiv((int64_t)M * (N / 4), 64));
+    const int threads = M * N % (1 << 19) == 0 ? 128 : 64;
     const auto add = splits <= 8 ? gemv_wide_reduce_kernel<T, 8> : gemv_wide_reduce_kernel<T, 16>;
-    hipLaunchKernelGGL(add, grid, dim3(64), 0, stream, partials, reinterpret_cast<const uint16_t*>(bias),
+    hipLaunchKernelGGL(add, dim3((unsigned)cdiv((int64_t)M * (N / 4), threads)), dim3(threads), 0, stream, partials, reinterpret_cast<const uint16_t*>(bias),
                        reinterpret_cast<uint16_t*>(y), M, N, splits, act);
     return hipGetLastError();
 }

@@ -255,6 +255,21 @@ def test_gemv_second_pass_rounds(M, split):
     _check(y, xb, p, "bf16", o.to_dtype_f32(bias, "bf16"))
 
 
+@pytest.mark.parametrize("M,N,split", [(64, 8192, 3), (32, 16384, 10)])
+def test_gemv_second_pass_of_sums_a_power_of_two_apart(M, N, split):
+    """Sums of a split that are a multiple of 2 MiB go by workgroups of two waves; the whole result against the unsplit kernel's."""
+    K = 10 * 128
+    print(f"gemv second pass M={M} N={N} split={split}", flush=True)
+    L = _lib.lib()
+    names = [L.awq_gemv_variant_name(i).decode() for i in range(L.awq_gemv_variant_count())]
+    p = random_packed(K, N, 128, "bf16", seed=split)
+    args = (to_dev(make_x(M, K, "bf16", seed=M), "bf16"), to_dev(p["qweight"]), to_dev(p["qscales"], "bf16"), to_dev(p["qzeros"]))
+    variant = names.index("wide2d2m4" if M > 32 else "wide2d2m2")
+    got, want = (awq_gemv_variant(*args, variant, s).double() for s in (split, 1))
+    # two orders of the same fp32 sums, each rounded to bf16 once
+    assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-5 * want.abs().max()).all()
+
+
 def test_gemv_reference_test_shape():
     # the reference's own GEMM test: K=1024, N=2048, g=32, 8 tokens, atol=1.0 against x @ w_dq.T
     # (awq/tests/dequantization_kernel.py:108-138)
