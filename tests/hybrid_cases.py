@@ -198,3 +198,11 @@ def logit_error(got, want):
     d = d - d.mean(dim=-1, keepdim=True)
     scale = (want - want.mean(dim=-1, keepdim=True)).pow(2).mean().sqrt()
     return (d.pow(2).mean(dim=-1).sqrt() / scale).max().item()
+
+
+# rows, features, contraction of linears that run every form of stream_linear_kernel (16, 32 and 64 rows x 2, 4 and 8 tiles of features, the
+# contraction whole and in parts, added by a pass and by a reader) and the 256-row tiles of dense_linear_kernel, whole and in parts
+STREAM_SIZES = [(16, 4100, 264), (16, 9220, 1032), (9, 1028, 4104), (16, 4100, 2056), (15, 36, 4104), (31, 4100, 264), (31, 36, 2056),
+                (31, 9220, 1032), (32, 4100, 2056), (31, 2052, 2056), (17, 18436, 1032), (31, 4100, 8200), (32, 8196, 4104), (64, 4100, 520),
+                (33, 36, 2056), (33, 4100, 264), (64, 36, 4104), (33, 18436, 520), (33, 4100, 4104), (64, 8196, 2056)]
+TALL_TILE_SIZES = [(2500, 1032, 4672), (2049, 4104, 192), (1500, 1032, 9280), (3001, 2056, 4672)]

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from hybrid_cases import (ATT, CONFIGS, GLA, LATENT, WIN, config, latent, layer, random_weights, roletar, tensor_shapes, tokens,
+from hybrid_cases import (ATT, CONFIGS, GLA, LATENT, STREAM_SIZES, TALL_TILE_SIZES, WIN, config, latent, layer, random_weights, roletar, tensor_shapes, tokens,
                           write_checkpoint)
 from nanoquantization_amd import _lib
 from nanoquantization_amd.engine.cache import PagedKVCache, RecurrentStateCache
@@ -57,6 +57,23 @@ def test_linears_that_a_stream_is_faster_for():
     lib = _lib.hybrid_lib()
     for rows, n_out, n_in in ((16, 32768, 4096), (12, 151936, 2560), (5, 32768, 2560), (6, 12288, 2048), (4, 8192, 2560), (64, 9216, 2560)):
         assert lib.nqh_skinny_linear_form(rows, n_out, n_in, 0, None) > 1, (rows, n_out, n_in)
+
+
+def test_sizes_of_the_linear_tests_reach_every_form():
+    """What the GPU tests of the linears run (a fit of the estimates may move it: then the sizes have to follow)."""
+    lib, parts = _lib.hybrid_lib(), ctypes.c_int64()
+
+    def form(entry, size, adds):
+        tiles = getattr(lib, entry)(*size, adds, ctypes.byref(parts))
+        return tiles, parts.value > 1
+    for adds in (0, 1, 2):
+        got = {(next(m for m in (16, 32, 64) if s[0] <= m), *form("nqh_skinny_linear_form", s, adds)) for s in STREAM_SIZES}
+        want = {(m, t, p) for m in (16, 32, 64) for t in (2, 4, 8) for p in (False, True) if (m > 16 or t < 8) and (adds or not p)}
+        assert want <= got, (adds, want - got)
+        got = {form("nqh_dense_linear_form", s, adds) for s in TALL_TILE_SIZES}
+        assert got >= ({(256, False), (256, True)} if adds else {(256, False)}), (adds, got)
+    assert lib.nqh_skinny_linear_form(65, 64, 64, 0, None) == 0 and lib.nqh_dense_linear_form(65, 64, 65, 0, None) == 0
+    assert lib.nqh_skinny_linear_form(1, 64, 64, 3, None) == 0 and lib.nqh_dense_linear_form(65, 64, 64, -1, None) == 0
 
 
 def test_hyper_norm_takes_no_fp32_sums():

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from hybrid_cases import STREAM_SIZES, TALL_TILE_SIZES
 from nanoquantization_amd import _lib
 from nanoquantization_amd.engine import hybrid_ops as ops
 from oracle import hybrid_oracle as o
@@ -444,6 +445,21 @@ def test_experts_with_few_pairs_on_large_tiles(rows, width, experts, top, ff, ti
     close(ops.moe_experts(h, gu, dn, r), want.cpu(), bf, "experts")
 
 
+@pytest.mark.parametrize("rows,width,parts", [(1, 72, 1), (16, 2048, 7), (5, 50, 3)])
+def test_residual_norm_route_adds_the_parts_of_a_product(rows, width, parts):
+    """fp32 parts beside bf16 weights, as residual_norm and route take them."""
+    print(f"norm + route of fp32 parts {rows} x {parts} x {width}", flush=True)
+    bf = torch.bfloat16
+    x0, y = rand(rows, width, seed=1).cuda(), rand(rows, parts, width, seed=2).cuda()
+    wb, wn, router = (rand(*s, seed=3 + i, dtype=bf).cuda() for i, s in enumerate([(width,), (width,), (8, width)]))
+    x1, x2 = x0.clone(), x0.clone()
+    h1 = ops.residual_norm(x1, 1e-5, y=y, post_weight=wb, next_weight=wn)
+    h2, r = ops.residual_norm_route(x2, 1e-5, router, 2, 64, wn, y=y, post_weight=wb)
+    assert torch.equal(x1, x2) and torch.equal(h1, h2) and torch.equal(r.expert, ops.route(h1, router, 2, 64).expert)
+    total = y.double().sum(1)
+    close(x1, (x0 + total / (total.square().mean(-1, keepdim=True) + 1e-5).sqrt() * wb).double().cpu(), torch.float32)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,width,experts,top,ff", [(1, 72, 5, 2, 48), (16, 2048, 8, 2, 64), (64, 256, 64, 6, 128),
                                                       (200, 1028, 128, 8, 32), (33, 4096, 3, 3, 24), (300, 64, 8, 2, 32)])
@@ -503,8 +519,8 @@ def test_skinny_linear(rows, n_out, n_in):
     close(ops.skinny_linear(x.cuda(), w.cuda(), b.cuda()), want + b.double(), torch.bfloat16)
 
 
-# every tile height and workgroup width, whole and split contractions, ends inside a stage, a wave's features, a workgroup; what a
-# former launch left in LDS (NaN here) reaches nothing.  Bounds as for any fp32 sum of these lengths: `close`
+# whole and split contractions, ends inside a stage, a wave's features, a workgroup; what a former launch left in LDS (NaN here)
+# reaches nothing.  Bounds as for any fp32 sum of these lengths: `close`.  Every tile height and workgroup width: test_stream_linear_forms
 @pytest.mark.parametrize("rows,n_out,n_in", [(1, 64, 8), (5, 132, 1000), (16, 2048, 2048), (16, 544, 4096), (17, 1028, 136), (20, 4608, 1024),
                                              (32, 2052, 9224), (33, 4096, 4608), (64, 4100, 2056), (64, 12288, 1024), (40, 1030, 520),
                                              (64, 18432, 2048)])
@@ -527,6 +543,24 @@ def test_skinny_linear_parts(rows, n_out, n_in):
         ops._call(xd.device, "nqh_skinny_linear_ex", xd.data_ptr(), wd.data_ptr(), None, y.data_ptr(), rows, n_out, n_in, 0, 0, 0.0,
                   ops._ptr(scratch), nbytes)
         close(y, want, torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows,n_out,n_in", STREAM_SIZES)
+def test_stream_linear_forms(rows, n_out, n_in):
+    """Every form (test_hybrid_host.py checks that the sizes reach them all): into bf16 and fp32, with a bias and an activation, without
+    scratch memory, with it and for a reader.  Bounds as above."""
+    print(f"stream linear {rows} x {n_in} -> {n_out}", flush=True)
+    x, w, b = (rand(*s, seed=i, dtype=torch.bfloat16).cuda() for i, s in enumerate([(rows, n_in), (n_out, n_in), (n_out,)]))
+    want = x.double() @ w.double().T
+    full = ((want + b.double()).clamp(min=0) ** 2).cpu()
+    scratch = torch.full((16 * rows * n_out,), float("nan"), device="cuda")
+    for room in (None, scratch):
+        for f32, dtype in ((0, torch.bfloat16), (1, torch.float32)):
+            y = torch.full((rows, n_out), float("nan"), dtype=dtype, device="cuda")
+            ops._call(x.device, "nqh_skinny_linear_ex", x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), rows, n_out, n_in, f32, 1, 0.0,
+                      ops._ptr(room), 0 if room is None else 4 * room.numel())
+            close(y, full, dtype, (room is None, f32))
+    close(ops.skinny_linear_sums(x, w).double().sum(1), want.cpu(), torch.float32)
 
 
 def test_linear_of_many_rows_with_a_strided_bias():
@@ -604,7 +638,7 @@ def test_dense_activation(rows, n_out, n_in):
     assert torch.equal(got, ops.activate_(y, "relu2").cpu())      # of the product rounded to bf16
 
 
-# whole and split contractions (the last part shorter), both tile heights, rows and columns past their tiles, fewer than a tile
+# whole and split contractions (the last part shorter), rows and columns past their tiles, fewer than a tile, on tiles of 128 rows; of 256: below
 @pytest.mark.parametrize("rows,n_out,n_in", [(65, 8, 64), (130, 96, 2048), (127, 4608, 192), (257, 264, 4672), (1000, 1024, 4608),
                                              (2049, 2056, 1024), (300, 4096, 18432)])
 def test_dense_linear(rows, n_out, n_in):
@@ -624,6 +658,25 @@ def test_dense_linear(rows, n_out, n_in):
     assert (sums is None) == (ops._of_sizes("nqh_dense_linear_parts", rows, n_out, n_in) == 1)
     if sums is not None:
         close(sums.double().sum(1), want, torch.float32)
+
+
+@pytest.mark.parametrize("rows,n_out,n_in", TALL_TILE_SIZES)
+def test_dense_linear_on_tall_tiles(rows, n_out, n_in):
+    """256-row tiles whole and in parts, with rows and columns past the last tile: a bias, a row stride, parts added by a pass and by
+    a reader."""
+    print(f"dense linear on tall tiles {rows} x {n_in} -> {n_out}", flush=True)
+    x, w, b = (rand(*s, seed=i, dtype=torch.bfloat16).cuda() for i, s in enumerate([(rows, n_in), (n_out, n_in), (n_out,)]))
+    want = (x.double() @ w.double().T).cpu()
+    wide = torch.full((rows, n_in + 24), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:, 8:8 + n_in] = x
+    close(ops.dense_linear(x, w, b), want + b.double().cpu(), torch.bfloat16)
+    assert torch.equal(ops.dense_linear(wide[:, 8:8 + n_in], w, b), ops.dense_linear(x, w, b))
+    y = torch.empty(rows, n_out, dtype=torch.bfloat16, device="cuda")           # without scratch memory
+    ops._call(x.device, "nqh_dense_linear", wide[:, 8:].data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), rows, n_out, n_in, n_in + 24, None, 0)
+    close(y, want + b.double().cpu(), torch.bfloat16)
+    sums = torch.full((rows, ops._of_sizes("nqh_dense_linear_parts", rows, n_out, n_in), n_out), float("nan"), device="cuda")
+    ops._call(x.device, "nqh_dense_linear_sums", x.data_ptr(), w.data_ptr(), sums.data_ptr(), rows, n_out, n_in)
+    close(sums.double().sum(1), want, torch.float32)
 
 
 def test_argmax_and_bookkeeping():

@@ -467,6 +467,28 @@ def test_scan_steps_of_a_wide_batch_equal_each_row_alone(dtype):
     assert torch.equal(sa[idle], s0[idle]) and torch.count_nonzero(got[~active]) == 0 and not torch.equal(sa, s0)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N", [16, 32])
+def test_scan_weights_off_a_16_byte_boundary(dtype, N):
+    """a_log and the taps of a convolution that cannot be read as vectors give the same bits: in pieces, in a step, fresh and not."""
+    T, C, rank, taps = 70, 88, 8, 4
+    print(f"scan weights off the boundary N={N} {dtype}", flush=True)
+    xz, sel, conv, bias, up, dt_b, a_log, skip = (t.cuda() for t in scan_case(T, C, N, rank, taps, dtype))
+    off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    dt, start = ops.scan_dt(sel[:, :rank], up, dt_b), torch.tensor([0, 9], device=DEV)
+    layout = ops.PromptPass([(0, 40, range(40), 0), (7, 30, range(37), 1)], 1, torch.device(DEV))
+    slot, active = torch.tensor([1, 0], dtype=torch.int32, device=DEV), torch.ones(2, dtype=torch.bool, device=DEV)
+
+    def go(conv, a_log):
+        state, tail = rand(2, N, C, seed=5).cuda(), rand(2, taps - 1, C, seed=6).cuda()
+        x = ops.conv_silu(xz[:, :C], conv, bias, tail, layout, 32)
+        y = ops.scan_prefill(x, dt, sel[:, rank:], xz[:, C:], a_log, skip, xz[:, :C], state, tail, layout, 32)
+        z = ops.scan_step(x[:2], dt[:2], sel[:2, rank:], xz[:2, C:], a_log, skip, state, slot, start, active)
+        return x, y, z, state, tail
+    assert off(conv).data_ptr() % 16 and off(a_log).data_ptr() % 16 and a_log.data_ptr() % 16 == 0
+    assert all(torch.equal(a, b) for a, b in zip(go(off(conv), off(a_log)), go(conv, a_log)))
+
+
 def test_scan_ragged_pass_equals_each_sequence_alone():
     C, N, rank, taps, dtype = 80, 20, 8, 4, torch.bfloat16
     portions = [(0, 300), (37, 150), (0, 1), (250, 2), (128, 128), (5, 1)]
