@@ -92,6 +92,25 @@ def test_staged_gemv_issues_each_load_once(tmp_path):
         if pending and line.split()[0].startswith(("v_", "ds_", "global_", "buffer_")):
             assert not (vregs(line.split(None, 1)[1] if " " in line else "") & pending), line
     assert fetches >= 500, fetches
+    # and so are the touches of the prefetch workgroups, four of them to a wait
+    pending, touches, issued = set(), 0, False
+    for line in asm.split("\n"):
+        line = line.strip()
+        issued, by_hand = line == ";;#ASMSTART", issued
+        if not line or line[0] in ";." or line.endswith(":"):
+            continue
+        if line.startswith("s_waitcnt") and "vmcnt(0)" in line:
+            pending = set()
+            continue
+        m = re.match(r"global_load_dword (v\d+), (v\[\d+:\d+\]), off$", line)
+        if m and by_hand:
+            assert not (vregs(line) & pending), line
+            pending |= vregs(m.group(1))
+            touches += 1
+        elif pending:
+            assert not line.startswith(("s_cbranch", "s_branch")), line
+            assert not (vregs(line.split(None, 1)[1] if " " in line or "\t" in line else "") & pending), line
+    assert touches >= 4 * 20 and touches % 4 == 0, touches
 
 
 @pytest.mark.skipif(shutil.which(nq_build.HIPCC) is None and not os.path.exists(nq_build.HIPCC), reason="hipcc not found")
@@ -175,6 +194,12 @@ def test_hybrid_kernels_wait_for_their_tile_loads(tmp_path):
         for u in range(ahead + 1):
             assert any("vmcnt(%d)" % ((ahead - 1) * stage) in l for l in ins[bars[u] - 3:bars[u]]), (name, u)
             assert kinds[bars[u]:bars[u + 1]].count("load") == stage, (name, u)
+            # nothing else waits for less to be open there: a wait put in by the compiler (for LDS that a load writes) would drain the ring
+            end = next(k for k in range(bars[u], bars[u + 1] + 1) if ins[k].startswith("s_cbranch") or k == bars[u + 1])
+            assert sum("v_mfma" in l for l in ins[bars[u]:end]) == 4 * mt, (name, u)
+            for l in ins[bars[u]:end]:
+                m = re.search(r"vmcnt\((\d+)\)", l)
+                assert m is None or int(m.group(1)) >= (ahead - 1) * stage, (name, u, l)
         assert kinds.count("load") == (2 * ahead + 1) * stage, name
         found += 1
     assert found == 3 * (2 + 3 + 3)

@@ -501,6 +501,7 @@ def test_engine_logits_are_those_of_lm_head(rows):
     eng = LLMEngine(model, max_batch=4, max_seq_len=64, block_size=16, use_graph=False)
     head = model.lm_head
     torch.manual_seed(rows)
+    head.bias.data.normal_()
     h = torch.randn(rows, head.in_features, device="cuda").to(head.weight.dtype)
     want = h.double() @ head.weight.double().T + (0 if head.bias is None else head.bias.double())
     with torch.no_grad():
@@ -511,6 +512,30 @@ def test_engine_logits_are_those_of_lm_head(rows):
         hook = head.register_forward_hook(lambda m, i, o: seen.append(o))
         assert torch.allclose(eng._logits(h).float(), got.float(), rtol=2.0 ** -7, atol=1e-3) and len(seen) == 1
         hook.remove()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width,rows,own", [(1024, 16, True), (1024, 17, False), (2048, 17, True), (2048, 48, True), (2048, 49, False),
+                                            (4096, 49, True), (4096, 64, True), (4096, 65, False)])
+def test_engine_logits_of_wider_heads(width, rows, own, monkeypatch):
+    """Which rows go to the engine's own kernel, and that both ways give the same logits."""
+    from nanoquantization_amd.engine import LLMEngine, hybrid_ops
+    from nanoquantization_amd.models.random_init import random_awq_qwen3
+    print(f"engine logits of {rows} rows of {width}", flush=True)
+    model = random_awq_qwen3(TINY, seed=5, std=0.05)
+    eng = LLMEngine(model, max_batch=4, max_seq_len=64, block_size=16, use_graph=False)
+    torch.manual_seed(rows)
+    model.lm_head = head = torch.nn.Linear(width, 1000, device="cuda", dtype=torch.bfloat16)
+    head.bias.data.normal_()
+    h = torch.randn(rows, width, device="cuda", dtype=torch.bfloat16)
+    calls, kernel = [], hybrid_ops.skinny_linear
+    monkeypatch.setattr(hybrid_ops, "skinny_linear", lambda *a, **k: calls.append(a[0].shape) or kernel(*a, **k))
+    want = h.double() @ head.weight.double().T + head.bias.double()
+    with torch.no_grad():
+        got = eng._logits(h)
+    assert len(calls) == own
+    # one rounding of fp32 sums; the library rounds the product before the bias is added
+    assert ((got.double() - want).abs() <= 2.0 ** -7 * (want.abs() + head.bias.double().abs()) + 1e-4 * want.abs().max()).all()
 
 
 @pytest.mark.gpu
