@@ -1145,7 +1145,8 @@ __global__ __launch_bounds__(64 * WK) void gemv_dma_kernel(
 // (even output columns), the other on bytes 2-3 (odd columns).  Nothing is unpacked or scaled twice, each
 // wave holds half the accumulators, and every SIMD has two waves.  What bounds this regime is the SIMD's
 // issue port, not the memory: per wave and 128 x 64 weights at 64 rows 80 MFMAs, which take it for 8 of their
-// 16 cycles, and 299 vector instructions at 4.7 (128 of them unpack, 128 apply scale and zero point).
+// 16 cycles, and 299 vector instructions at 4.7 (128 of them unpack, 128 apply scale and zero point); with the rest of the kernel
+// 71 to 80 % of the launch's cycles at 64 x 25600 x 5120, while waves wait for data or the barrier 22 % of their time.
 // At the end the two halves exchange fragments through LDS so that each stores whole words of half the rows.
 // A K split leaves fp32 partials that a second kernel adds in split order -- or, TAIL (one m-tile, a few rows), the
 // last workgroup of the 512 columns to arrive, as in the one-tile kernel.
@@ -1755,9 +1756,10 @@ static hipError_t launch_gemv_dma(const void* x, const int32_t* qweight, const v
         const long long room = (256 - compute_wgs) / ((long long)splits * row_blocks);   // stay within one wave of workgroups
         pf_wgs = (int)(want < room ? want : room);
         if (pf_wgs < 1) pf_wgs = 1;
-        // Two round trips of the prefetch threads (four lines each) at most, or the launch lasts as long as its successor's weight:
-        // the o_proj launch of a Qwen3-4B step, whose splits leave it 12 workgroups in front of 25 MB, took 34 us instead of 9.  Decode
-        // steps of six such layers 583 -> 416 us at one row, 796 -> 643 at 32 (one trip 631, three 666, four 690); six 1.7B
+        // As many lines as two round trips of the prefetch threads bring (four each), and one trip more for every further region that is
+        // left some of them, or the launch lasts as long as its successor's weight: the o_proj launch of a Qwen3-4B step, whose splits
+        // leave it 12 workgroups in front of 25 MB, took 34 us instead of 9.  Decode
+        // steps of six such layers 583 -> 416 us at one row, 796 -> 643 at 32 (lines of one trip 631, three 666, four 690); six 1.7B
         // layers at 32 rows 540 -> 503.  What is left over the launch that reads it fetches itself.  The 0.3 to 1.6 MB regions of Qwen3-0.6B
         // take one trip: 28 layers 1584 / 1585 (cut to one 1592).
         long long reach = (long long)pf_wgs * 64 * WK * 4 * 128 * 2;

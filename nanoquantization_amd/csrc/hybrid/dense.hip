@@ -46,9 +46,8 @@ __global__ __launch_bounds__(1024) void skinny_linear_kernel(const uint16_t* __r
 // Bound by the stream of the weights (5 to 5.6 TB/s) and by what a CU takes in, some 45 KB/us of weights and activations alike.  That
 // is why the contraction is split until there is a workgroup for each CU, and why workgroups are wider where there are more rows.
 // Weights from memory, us, before (all of the contraction in one workgroup, one stage ahead, waited for in full) / this with the sums
-// left to the reader: 64 rows 18432 -> 4096 87 / 34, 4096 -> 4096 21 / 10.8, 9216 -> 2048 44 / 12.3; 16 rows 41 / 28, 11.2 / 8.4, 19.6 / 9.4;
-// one row 33.8 / 27.4, 9.4 / 8.3, 14.1 / 9.2.  Unsplit: 64 rows 4096 -> 32768 70 / 53 (63 with all workgroups in step), 4096 ->
-// 12288 37 / 30, 1024 -> 4608 7.8 / 7.5; 32 rows 1024 -> 32768 16.3 / 15.1.  Seven stages ahead are no faster than three.
+// left to the reader: 18432 -> 4096 at 64, 16 rows and one 87 / 34, 41 / 28, 33.8 / 27.4; unsplit: 64 rows 4096 -> 32768 70 / 53 (63 with
+// all workgroups in step).  Seven stages ahead are no faster than three.
 #define NQH_LPTR(p) ((__attribute__((address_space(3))) void*)(p))
 
 template <int N, typename F>
@@ -254,6 +253,7 @@ struct LinearPlan {
 };
 // Who may add the parts: nobody, sum_parts_kernel, the same where the host issues call after call, the reader of the result.
 enum class Sums { kNone, kOwnPass, kIssuedPass, kReader };
+Sums sums_of(int adds) { return adds == NQH_ADDS_NOBODY ? Sums::kNone : adds == NQH_ADDS_PASS ? Sums::kOwnPass : Sums::kReader; }
 
 // The least estimated time.  In us: a launch with its first data; what the fullest CU takes in (KB, at a rate of its own per form) and
 // the weights from memory (MB), the root of the sum of their squares; parts written, and read by a pass of their own or by a reader
@@ -476,7 +476,8 @@ DensePlan make_dense_plan(int64_t rows, int64_t n_out, int64_t n_in, Sums sums) 
             const double part = (double)(work % 256) / 256, whole = (double)(work / 256);
             const double stage = xr == 256 ? std::max(0.52, 0.91 + 0.37 * part) : std::max(0.59, 0.6 + 0.32 * part), end = xr == 256 ? 5.4 : 3.3;
             double us = std::max(memory, 3.2 + whole * (each * (xr == 256 ? 1.36 : 0.85) + end) + (part > 0 ? each * stage + end : 0));
-            if (s > 1) us += parts / 8 + (sums == Sums::kReader ? std::max((parts - 2e-6 * rows * n_out) / 5.5, 4e-3 * s * n_out / 60) : 2.65 + parts / 6);
+            if (s > 1)
+                us += parts / 8 + (sums == Sums::kReader ? std::max((parts - 2e-6 * rows * n_out) / 5.5, 4e-3 * s * n_out / 60) : 2.65 + parts / 6);
             if (us < best.us) best = {xr, (int)s, us};
         }
     }
@@ -519,7 +520,7 @@ extern "C" int nqh_skinny_linear_sums(const void* x, const void* weight, float* 
 
 extern "C" int nqh_skinny_linear_form(int64_t rows, int64_t out_features, int64_t in_features, int adds, int64_t* parts) {
     if (!skinny_takes(rows, out_features, in_features) || adds < NQH_ADDS_NOBODY || adds > NQH_ADDS_READER) return 0;
-    const LinearPlan plan = plan_linear(rows, out_features, in_features, adds == NQH_ADDS_NOBODY ? Sums::kNone : adds == NQH_ADDS_PASS ? Sums::kOwnPass : Sums::kReader);
+    const LinearPlan plan = plan_linear(rows, out_features, in_features, sums_of(adds));
     if (parts) *parts = plan.splits;
     return 1 << plan.form;
 }
@@ -559,14 +560,12 @@ extern "C" int nqh_skinny_linear(const void* x, const void* weight, const void* 
 
 // 1 where the tiles are one round of the 256 CUs and estimated to take less time than the library's product and the activation's pass
 // do when a python program issues them: 1.3 PFLOP/s and 5 TB/s, 28 us at least, the two launches.  On the GPU alone, from a graph, the
-// library's smaller tiles are ahead up to some 1000 rows: relu2, this kernel / those two, us, 1024 -> 4608 at 65 rows 16 / 11, 2048 ->
-// 9216 at 100 rows 26 / 17, 2048 -> 1536 at 1000 rows 27 / 18.  What counts is the pass, which the host issues more slowly than the GPU works it
-// off: Roletar prompts through three layers with this kernel / without, wall time and (behind other work, GPU time): 0.6B, 128
-// tokens 666 / 713 (356 / 333), 1000 tokens 696 / 743 (514 / 514); 1.7B, 128 tokens 646 / 751 (495 / 448), 400 tokens 666 / 717 (585 / 590),
-// 1000 tokens 860 / 872; 8B 0 to 2 % less.  Several rounds
-// of short contractions stay with the library: in a pass its products lose less to the writes between the rounds (0.6B, 8192 tokens, 576 tiles: 110 here,
-// 83 + 24 there, though 89 / 103 when repeated alone; 1.7B, 4096 tokens, 576 tiles: the pass 1873 -> 1886).
-// Of 4096 and more the ends of the tiles weigh less (4000 rows, 4096 -> 18432: 453 here, 365 to 564 + 48 there; the pass 5087 with the product below alone, 4686 with both).
+// library's smaller tiles are ahead up to some 1000 rows: relu2, this kernel / those two, us, 2048 -> 9216 at 100 rows 26 / 17, 2048 ->
+// 1536 at 1000 rows 27 / 18.  What counts is the pass, which the host issues more slowly than the GPU works it off: Roletar prompts through
+// three layers with this kernel / without, wall time, 1.7B, 128 tokens 646 / 751, 1000 tokens 860 / 872; 8B 0 to 2 % less.
+// Several rounds of short contractions stay with the library: in a pass its products lose less to the writes between the rounds (0.6B,
+// 8192 tokens, 576 tiles: 110 here, 83 + 24 there, though 89 / 103 when repeated alone).  Of 4096 and more the ends of the tiles weigh less
+// (4000 rows, 4096 -> 18432: 453 here, 365 to 564 + 48 there).
 extern "C" int nqh_dense_activation_wanted(int64_t rows, int64_t out_features, int64_t in_features) {
     if (!dense_activation_takes(rows, out_features, in_features)) return 0;
     const int xr = dense_activation_tile(rows, out_features, in_features);
@@ -594,15 +593,13 @@ extern "C" int nqh_dense_activation(const void* x, const void* weight, void* y, 
                : launch_dense<256, false>(fn, x, weight, nullptr, y, rows, out_features, in_features, in_features, act, param, 1, stream);
 }
 
-// Products of prompts.  A library product takes the host 21 us to issue, this one 6, and a pass of some hundred rows through small
-// layers is 11 of them; on the GPU the library is ahead by up to a third there.  Where its tiles leave CUs idle over a long
-// contraction it falls far behind (1000 rows of 18432 -> 4096: 217 us, this with the sums left to the reader 114; 900 of 12288 -> 4096 107 /
-// 81; 160 of 8192 -> 4096 48 / 25; 900 of 9728 -> 2560 80 / 51), and with many rows it is ahead by 3 to 10 %.  Prompts through three layers, before / now, us: Roletar 0.6B, 300 tokens
-// 699 / 496 (some 510 while the library took the expansion of the latents, whose rows are columns of a wider tensor), 1000 752 / 620, 2000
-// 777 / 709; 1.7B, 300 tokens 683 / 554; 8B, 300 tokens 1066 / 882, 2000 3157 / 2682, 4000 5128 / 4778; Gafulix 0.6B, 100 tokens 550 /
-// 413, 700 671 / 510.  Of Gafulix 1.7B and 8B the experts' weights take the GPU 200 to 900 us, so that the host's time is hidden: a
-// product of 15 to 20 us is the library's there (busy; 1700 rows, 2048 -> 2048: 27 here, 17 there; the passes are within 1 % of what
-// they were; Gafulix 0.6B, 16 us of weights a layer: 100 tokens 428 busy, 413 not, 500 572 / 500).
+// Products of prompts.  A library product takes the host 21 us to issue (measured from python on one machine: on a faster one the line lies
+// lower), this one 6, and a pass of some hundred rows through small layers is 11 of them; on the GPU the library is ahead by up to a
+// third there.  Where its tiles leave CUs idle over a long contraction it falls far behind (1000 rows of 18432 -> 4096: 217 us, this with
+// the sums left to the reader 114; 160 of 8192 -> 4096 48 / 25), and with many rows it is ahead by 3 to 10 %.  Prompts through three
+// layers, before / with this kernel, us: Roletar 0.6B, 300 tokens 650 / 434, 8B, 2000 tokens 3157 / 2682; Gafulix 0.6B, 300 tokens 635 / 472.
+// Where experts' weights take the GPU longer than the host is ahead by (Gafulix 1.7B and 8B, 200 to 900 us) a product of 15 to 20 us is
+// the library's (busy; 1700 rows, 2048 -> 2048: 27 here, 17 there); of Gafulix 0.6B, 16 us of weights a layer, it is not (500 tokens 572 busy, 500 not).
 extern "C" int nqh_dense_linear_wanted(int64_t rows, int64_t out_features, int64_t in_features, int reader, int busy) {
     return dense_activation_takes(rows, out_features, in_features) &&
            plan_dense(rows, out_features, in_features, reader ? Sums::kReader : Sums::kOwnPass).us <
@@ -611,7 +608,7 @@ extern "C" int nqh_dense_linear_wanted(int64_t rows, int64_t out_features, int64
 
 extern "C" int nqh_dense_linear_form(int64_t rows, int64_t out_features, int64_t in_features, int adds, int64_t* parts) {
     if (!dense_activation_takes(rows, out_features, in_features) || adds < NQH_ADDS_NOBODY || adds > NQH_ADDS_READER) return 0;
-    const DensePlan plan = plan_dense(rows, out_features, in_features, adds == NQH_ADDS_NOBODY ? Sums::kNone : adds == NQH_ADDS_PASS ? Sums::kOwnPass : Sums::kReader);
+    const DensePlan plan = plan_dense(rows, out_features, in_features, sums_of(adds));
     if (parts) *parts = plan.splits;
     return plan.xr;
 }

@@ -192,9 +192,10 @@ class LLMEngine(EngineCore):
     def _logits(self, h: torch.Tensor) -> torch.Tensor:
         """lm_head of a few rows, a stream of its weight: 4.5 TB/s at best as the library reads it, 5 to 5.6 as the hybrid decoders' kernel
         does.  bf16, 32768 columns, library / own, us: width 1024, 1 / 16 rows 20.0 / 14.0, 18.0 / 15.0; 2048, 1 / 16 / 48 rows 35.8 / 27.9,
-        31.9 / 26.5, 36.2 / 31.4; 4096, 1 / 16 / 64 rows 64.8 / 48.2, 63.0 / 54.4, 62.6 / 55.6; 151936 columns of 1024, 1 / 16 rows 63.4 / 51.6, 63.5 /
-        62.4, of 4096 256 / 203, 253 / 232.  From 17 rows on narrow ones are the library's (1024, 24 / 64 rows 16.5 / 16.9, 17.4 / 19.8), from 49 on
-        those below 4096 (2560, 64 rows 39.6 / 41.4)."""
+        31.9 / 26.5, 36.2 / 31.4; 4096, 1 / 4 / 16 / 64 rows 64.8 / 48.2, 62.4 / 48.6, 63.0 / 54.4, 62.6 / 55.6; 151936 columns of 1024, 1 / 16
+        rows 63.4 / 51.6, 63.5 / 62.4, of 4096 256 / 203, 253 / 232.  From 17 rows on narrow ones are the library's (32768 of 1024, 24 / 64 rows
+        16.5 / 16.9, 17.4 / 19.8; the rule does not ask for the columns, and of 151936 the own kernel is ahead up to 32 rows: 24 / 32 / 48 rows
+        72.0 / 68.8, 73.9 / 71.1, 78.2 / 79.3), from 49 on those below 4096 (2560, 64 rows 39.6 / 41.4)."""
         head = self.model.lm_head
         if (is_torch_linear(head) and unhooked(head) and plain(h, head.weight)
                 and hybrid_ops.skinny_linear_supported(h.shape[0], head.weight) and head.weight.is_contiguous()
