@@ -94,36 +94,40 @@ template <int I>
 using Int = std::integral_constant<int, I>;
 
 // What a sublayer leaves: the sum of `parts` rows `stride` apart, of the call's type or, where it is the sums of a split contraction,
-// fp32.  V consecutive elements from element `at` on; `sum` comes in as zeros.
-struct Parts {
-    const void* y;
-    int parts, f32;
-};
-template <typename T, int V>
-__device__ __forceinline__ void load_parts(const Parts& y, int64_t at, int stride, float (&sum)[V]) {
-    const auto add = [&](auto type) {
-        using E = decltype(type);
-        const typename E::elem* p = reinterpret_cast<const typename E::elem*>(y.y) + at;
-        int j = 0;
-        const auto some = [&](auto n) {              // n of them in flight
-            float t[n][V];
+// fp32 (Y).  V consecutive elements from y on; `sum` comes in as zeros.
+template <typename Y, int V>
+__device__ __forceinline__ void load_parts(const typename Y::elem* __restrict__ y, int parts, int stride, float (&sum)[V]) {
+    if (parts == 1) {
+        load_vec<Y, V>(y, sum);                      // straight into place
+        return;
+    }
+    const auto some = [&](auto n) {                  // n of them in flight
+        float t[n][V];
 #pragma unroll
-            for (int u = 0; u < n; ++u) load_vec<E, V>(p + (int64_t)(j + u) * stride, t[u]);
+        for (int u = 0; u < n; ++u) load_vec<Y, V>(y + (int64_t)u * stride, t[u]);
 #pragma unroll
-            for (int u = 0; u < n; ++u)
+        for (int u = 0; u < n; ++u)
 #pragma unroll
-                for (int e = 0; e < V; ++e) sum[e] += t[u][e];
-            j += n;
-        };
-#pragma unroll 1
-        while (j + 4 <= y.parts) some(Int<4>());
-        if (j + 2 <= y.parts) some(Int<2>());
-        if (j < y.parts) some(Int<1>());
+            for (int e = 0; e < V; ++e) sum[e] += t[u][e];
+        y += (int64_t)n * stride;
+        parts -= n;
     };
-    if (y.parts == 1 && !y.f32) load_vec<T, V>(reinterpret_cast<const typename T::elem*>(y.y) + at, sum);     // straight into place
-    else if (y.f32) add(Fp());
-    else add(T());
+#pragma unroll 1
+    while (parts >= 4) some(Int<4>());
+    if (parts >= 2) some(Int<2>());
+    if (parts > 0) some(Int<1>());
 }
+// The statements with Y, the type of y.
+#define NQH_WITH_Y(y_f32, ...)     \
+    do {                           \
+        if (y_f32) {               \
+            using Y = nqh::Fp;     \
+            __VA_ARGS__;           \
+        } else {                   \
+            using Y = T;           \
+            __VA_ARGS__;           \
+        }                          \
+    } while (0)
 
 // V = 4 consecutive elements as they lie in memory, to be fetched early and unpacked late.
 template <typename T>

@@ -9,11 +9,12 @@ namespace {
 constexpr int kMaxStreams = 8;
 constexpr int kMaxWidth = 8192;
 
-// S: streams held in registers (`streams` of them exist), V elements per thread and step, P steps.
-template <typename T, int S, int V, int THREADS, int P>
+// S: streams held in registers (`streams` of them exist), V elements per thread and step, P steps.  MANY: y has several parts (their loop
+// in the kernel of one costs it 2 to 4 %: 8192 rows of 2 x 1024 35.2 -> 36.4 us).
+template <typename T, typename Y, bool MANY, int S, int V, int THREADS, int P>
 __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
     float* __restrict__ x, const int64_t* __restrict__ ids, const typename T::elem* __restrict__ table, int64_t table_rows,
-    Parts y, const typename T::elem* __restrict__ mix, const typename T::elem* __restrict__ w_out,
+    const typename Y::elem* __restrict__ y, int parts, const typename T::elem* __restrict__ mix, const typename T::elem* __restrict__ w_out,
     const typename T::elem* __restrict__ w_in, const typename T::elem* __restrict__ norm_w, typename T::elem* __restrict__ h,
     int streams, int width, float eps) {
     constexpr int WAVES = THREADS / 64;
@@ -43,8 +44,9 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
                 for (int s = 0; s < S; ++s)
                     if (s < streams) load_vec<Fp, V>(xr + (int64_t)s * width + i, v[s][p]);
             }
+            if (!MANY && y) load_vec<Y, V>(y + row * width + i, yv[p]);
             if (h) load_vec<T, V>(norm_w + i, wn[p]);
-            if (y.y) load_parts<T, V>(y, row * y.parts * width + i, width, yv[p]);
+            if (MANY && y) load_parts<Y, V>(y + row * parts * width + i, parts, width, yv[p]);
         }
     }
     float win[S];
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
 #pragma unroll
                 for (int e = 0; e < V; ++e) v[s][p][e] = v[0][p][e];
     }
-    if (y.y) {
+    if (y) {
         float m[S][S], wo[S];
 #pragma unroll
         for (int t = 0; t < S; ++t) {
@@ -86,7 +88,7 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         const int i = (p * THREADS + threadIdx.x) * V;
-        if (i < width && (y.y || ids)) {
+        if (i < width && (y || ids)) {
 #pragma unroll
             for (int s = 0; s < S; ++s)
                 if (s < streams) store_vec<Fp, V>(xr + (int64_t)s * width + i, v[s][p]);
@@ -111,14 +113,14 @@ __global__ __launch_bounds__(THREADS) void hyper_norm_kernel(
     }
 }
 
-template <typename T, int S>
-void launch_hyper(float* x, const int64_t* ids, const void* table, int64_t table_rows, Parts y, const void* mix,
+template <typename T, typename Y, bool MANY, int S>
+void launch_hyper(float* x, const int64_t* ids, const void* table, int64_t table_rows, const void* y, int64_t parts, const void* mix,
                   const void* w_out, const void* w_in, const void* norm_w, void* h, int64_t rows, int64_t streams,
                   int64_t width, float eps, bool vec, hipStream_t st) {
     using E = typename T::elem;
 #define NQH_GO(V, THREADS, P)                                                                                              \
-    hyper_norm_kernel<T, S, V, THREADS, P><<<dim3((unsigned)rows), dim3(THREADS), 0, st>>>(                                \
-        x, ids, (const E*)table, table_rows, y, (const E*)mix, (const E*)w_out, (const E*)w_in, (const E*)norm_w, \
+    hyper_norm_kernel<T, Y, MANY, S, V, THREADS, P><<<dim3((unsigned)rows), dim3(THREADS), 0, st>>>(                                \
+        x, ids, (const E*)table, table_rows, (const typename Y::elem*)y, (int)parts, (const E*)mix, (const E*)w_out, (const E*)w_in, (const E*)norm_w, \
         (E*)h, (int)streams, (int)width, eps)
     if (!vec) NQH_GO(1, 1024, 8);
     else if (width <= 1024) NQH_GO(4, 256, 1);
@@ -151,7 +153,7 @@ extern "C" int nqh_hyper_norm_parts(float* x, const int64_t* ids, const void* ta
                                     int64_t y_parts, const void* mix, const void* w_out, const void* w_in, const void* norm_weight,
                                     void* h, int64_t rows, int64_t streams, int64_t width, float eps, int dtype, void* stream) {
     const char* fn = "nqh_hyper_norm";
-    const int y_f32 = (dtype & NQH_Y_F32) != 0;
+    const bool y_f32 = (dtype & NQH_Y_F32) != 0;
     dtype &= ~NQH_Y_F32;
     if (!x || (ids && (!table || table_rows <= 0)) || (y && (!mix || !w_out)) || (h && !norm_weight))
         return fail(NQH_ERR_ARG, fn, "null pointer");
@@ -162,14 +164,15 @@ extern "C" int nqh_hyper_norm_parts(float* x, const int64_t* ids, const void* ta
     const bool vec = width % 4 == 0 && aligned(x, 16) && aligned(y, 16) && aligned(table, 16) && aligned(norm_weight, 16) &&
                      aligned(h, 16);
     (void)hipGetLastError();
-#define NQH_STREAMS(S) \
-    launch_hyper<T, S>(x, ids, table, table_rows, Parts{y, (int)y_parts, y_f32}, mix, w_out, w_in, norm_weight, h, rows, streams, width, eps, vec, (hipStream_t)stream)
-    NQH_WITH_TYPE(dtype, {
+#define NQH_STREAMS(S)                                                                                                             \
+    (y && y_parts > 1 ? launch_hyper<T, Y, true, S> : launch_hyper<T, Y, false, S>)(                                               \
+        x, ids, table, table_rows, y, y_parts, mix, w_out, w_in, norm_weight, h, rows, streams, width, eps, vec, (hipStream_t)stream)
+    NQH_WITH_TYPE(dtype, NQH_WITH_Y(y_f32, {
         if (streams == 1) NQH_STREAMS(1);
         else if (streams == 2) NQH_STREAMS(2);
         else if (streams <= 4) NQH_STREAMS(4);
         else NQH_STREAMS(8);
-    });
+    }));
 #undef NQH_STREAMS
     return launched(fn);
 }

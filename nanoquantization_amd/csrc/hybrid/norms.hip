@@ -22,9 +22,9 @@ struct RouteArgs {
     int experts, top, tile_rows, max_tiles;
 };
 
-template <typename T, int V, int THREADS, int P, bool ROUTED>
+template <typename T, typename Y, int V, int THREADS, int P, bool ROUTED>
 __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
-    float* __restrict__ x, int init, Parts y, const typename T::elem* __restrict__ post_w, const int64_t* __restrict__ ids,
+    float* __restrict__ x, int init, const typename Y::elem* __restrict__ y, int parts, const typename T::elem* __restrict__ post_w, const int64_t* __restrict__ ids,
     const typename T::elem* __restrict__ table, int64_t table_rows, const typename T::elem* __restrict__ next_w,
     typename T::elem* __restrict__ h, int width, float eps, RouteArgs route) {
     constexpr int WAVES = THREADS / 64;
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
             if (h) load_vec<T, V>(next_w + i, wn[p]);
         }
     }
-    if (y.y) {
+    if (y) {
         float s[P][V], ss = 0.f;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(THREADS) void residual_norm_kernel(
 #pragma unroll
             for (int e = 0; e < V; ++e) s[p][e] = 0.f;
             if (i < width) {
-                load_parts<T, V>(y, row * y.parts * width + i, width, s[p]);
+                load_parts<Y, V>(y + row * parts * width + i, parts, width, s[p]);
 #pragma unroll
                 for (int e = 0; e < V; ++e) ss += s[p][e] * s[p][e];
             }
@@ -362,13 +362,13 @@ static bool residual_vec(const void* x, const void* y, const void* post_weight, 
 }
 
 #define NQH_ARGS                                                                                                          \
-    x, init, Parts{y, (int)y_parts, y_f32}, (const E*)post_weight, ids, (const E*)table, table_rows, (const E*)next_weight,   \
+    x, init, (const typename Y::elem*)y, (int)y_parts, (const E*)post_weight, ids, (const E*)table, table_rows, (const E*)next_weight,   \
         (E*)h, (int)width, eps
 extern "C" int nqh_residual_norm(float* x, int init, const void* y, int64_t y_parts, const void* post_weight,
                                  const int64_t* ids, const void* table, int64_t table_rows, const void* next_weight,
                                  void* h, int64_t rows, int64_t width, float eps, int dtype, void* stream) {
     const char* fn = "nqh_residual_norm";
-    const int y_f32 = (dtype & NQH_Y_F32) != 0;
+    const bool y_f32 = (dtype & NQH_Y_F32) != 0;
     dtype &= ~NQH_Y_F32;
     const int rc = check_residual(fn, x, y, y_parts, ids, table, table_rows, next_weight, h, rows, width, dtype);
     if (rc != NQH_OK) return rc;
@@ -376,16 +376,18 @@ extern "C" int nqh_residual_norm(float* x, int init, const void* y, int64_t y_pa
     hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();
 #define NQH_GO(V, THREADS, P)                                                                                     \
-    residual_norm_kernel<T, V, THREADS, P, false><<<dim3((unsigned)rows), dim3(THREADS), 0, st>>>(NQH_ARGS, RouteArgs{})
+    residual_norm_kernel<T, Y, V, THREADS, P, false><<<dim3((unsigned)rows), dim3(THREADS), 0, st>>>(NQH_ARGS, RouteArgs{})
     NQH_WITH_TYPE(dtype, {
         using E = typename T::elem;
-        if (!vec) NQH_GO(1, 1024, 8);
-        else if (width <= 1024) NQH_GO(4, 256, 1);
-        else if (rows <= 256 && width <= 4096) NQH_GO(4, 1024, 1);   // few rows: more loads in flight per row
-        else if (rows <= 256) NQH_GO(4, 1024, 2);
-        else if (width <= 2048) NQH_GO(4, 256, 2);
-        else if (width <= 4096) NQH_GO(4, 256, 4);
-        else NQH_GO(4, 256, 8);
+        NQH_WITH_Y(y_f32, {
+            if (!vec) NQH_GO(1, 1024, 8);
+            else if (width <= 1024) NQH_GO(4, 256, 1);
+            else if (rows <= 256 && width <= 4096) NQH_GO(4, 1024, 1);   // few rows: more loads in flight per row
+            else if (rows <= 256) NQH_GO(4, 1024, 2);
+            else if (width <= 2048) NQH_GO(4, 256, 2);
+            else if (width <= 4096) NQH_GO(4, 256, 4);
+            else NQH_GO(4, 256, 8);
+        });
     });
 #undef NQH_GO
     return launched(fn);
@@ -402,7 +404,7 @@ extern "C" int nqh_residual_norm_route(float* x, int init, const void* y, int64_
                                        int64_t top, int64_t tile_rows, int64_t max_tiles, float eps, int dtype,
                                        void* stream) {
     const char* fn = "nqh_residual_norm_route";
-    const int y_f32 = (dtype & NQH_Y_F32) != 0;
+    const bool y_f32 = (dtype & NQH_Y_F32) != 0;
     dtype &= ~NQH_Y_F32;
     const int rc = check_residual(fn, x, y, y_parts, ids, table, table_rows, next_weight, h, rows, width, dtype);
     if (rc != NQH_OK) return rc;
@@ -418,12 +420,14 @@ extern "C" int nqh_residual_norm_route(float* x, int init, const void* y, int64_
     hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();
 #define NQH_GO(V, THREADS, P)                                                                                     \
-    residual_norm_kernel<T, V, THREADS, P, true><<<dim3((unsigned)rows), dim3(THREADS), 0, st>>>(NQH_ARGS, route)
+    residual_norm_kernel<T, Y, V, THREADS, P, true><<<dim3((unsigned)rows), dim3(THREADS), 0, st>>>(NQH_ARGS, route)
     NQH_WITH_TYPE(dtype, {
         using E = typename T::elem;
-        if (width <= 1024) NQH_GO(4, 256, 1);
-        else if (width <= 4096) NQH_GO(4, 1024, 1);
-        else NQH_GO(4, 1024, 2);
+        NQH_WITH_Y(y_f32, {
+            if (width <= 1024) NQH_GO(4, 256, 1);
+            else if (width <= 4096) NQH_GO(4, 1024, 1);
+            else NQH_GO(4, 1024, 2);
+        });
     });
 #undef NQH_GO
     return launched(fn);

@@ -445,6 +445,27 @@ def test_experts_with_few_pairs_on_large_tiles(rows, width, experts, top, ff, ti
     close(ops.moe_experts(h, gu, dn, r), want.cpu(), bf, "experts")
 
 
+@pytest.mark.parametrize("streams,width,parts", [(1, 1024, 1), (2, 1024, 2), (4, 50, 5), (8, 4100, 7)])
+def test_norms_add_parts_of_either_type(streams, width, parts):
+    """Parts of the call's type and the same values as fp32 sums, one part and several: kernels of their own, which may contract their
+    products differently.  At most streams + parts fp32 operations on values of the result's size: 15 x 2^-24, a twentieth of the bound."""
+    print(f"parts of either type {streams} x {width}, {parts}", flush=True)
+    bf, rows = torch.bfloat16, 5
+    y = rand(rows, parts, width, seed=1, dtype=bf).cuda()
+    wn, mix, write = (rand(*s, seed=2 + i, dtype=bf).cuda() for i, s in enumerate([(width,), (streams, streams), (streams,)]))
+    x0 = rand(rows, streams, width, seed=7).cuda()
+    rms = lambda t, w: t / (t.square().mean(-1, keepdim=True) + 1e-3).sqrt() * w.double()
+    total = y.double().sum(1)
+    mixed = torch.einsum("st,rsw->rtw", mix.double(), x0.double()) + write.double().view(1, -1, 1) * total.unsqueeze(1)
+    for v in (y, y.float()):
+        x, r = x0.clone(), x0[:, 0].contiguous()
+        h = ops.hyper_norm(x, 1e-3, y=v, mix=mix, write=write, next_weight=wn)
+        close(x, mixed.cpu(), torch.float32, v.dtype)
+        close(h, rms(mixed.sum(1), wn).cpu(), bf, v.dtype)
+        ops.residual_norm(r, 1e-3, y=v, post_weight=wn, next_weight=wn)
+        close(r, (x0[:, 0].double() + rms(total, wn)).cpu(), torch.float32, v.dtype)
+
+
 @pytest.mark.parametrize("rows,width,parts", [(1, 72, 1), (16, 2048, 7), (5, 50, 3)])
 def test_residual_norm_route_adds_the_parts_of_a_product(rows, width, parts):
     """fp32 parts beside bf16 weights, as residual_norm and route take them."""
