@@ -458,7 +458,7 @@ def test_norms_add_parts_of_either_type(streams, width, parts):
     total = y.double().sum(1)
     mixed = torch.einsum("st,rsw->rtw", mix.double(), x0.double()) + write.double().view(1, -1, 1) * total.unsqueeze(1)
     for v in (y, y.float()):
-        x, r = x0.clone(), x0[:, 0].contiguous()
+        x, r = x0.clone(), x0[:, 0].clone()
         h = ops.hyper_norm(x, 1e-3, y=v, mix=mix, write=write, next_weight=wn)
         close(x, mixed.cpu(), torch.float32, v.dtype)
         close(h, rms(mixed.sum(1), wn).cpu(), bf, v.dtype)
