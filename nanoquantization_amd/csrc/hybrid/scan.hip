@@ -518,8 +518,10 @@ __global__ __launch_bounds__(256) void scan_chain_kernel(const float* __restrict
 }
 
 // ---- one token per sequence ------------------------------------------------------------------------------------------------
-// Workgroup: 64 channels of ROWS rows; its four waves share the states.
-template <typename T, int ROWS>
+// Workgroup: 64 channels of ROWS rows; its four waves share the states: four side by side (WHOLE), so that a_log comes in one load, where
+// that deals them out evenly, every fourth otherwise.  (Side by side for all: 5 states of 1024 channels, one row 3.2 -> 4.0 us, 130 of 512 11.0 ->
+// 14.0, 24 of 2048 4.5 -> 4.8.)
+template <typename T, int ROWS, bool WHOLE>
 __global__ __launch_bounds__(256) void scan_step_kernel(
     const typename T::elem* __restrict__ x, const float* __restrict__ dt, const typename T::elem* __restrict__ bc,
     int64_t bc_stride, const typename T::elem* __restrict__ z, int64_t z_stride, const typename T::elem* __restrict__ a_log,
@@ -544,20 +546,20 @@ __global__ __launch_bounds__(256) void scan_step_kernel(
         dx[r] = d[r] * T::load(x + (int64_t)row * channels + c);
         y[r] = 0.f;
     }
-    const bool side_by_side = states % 4 == 0 && (reinterpret_cast<uintptr_t>(a_log) & 15u) == 0;
-    for (int n0 = 4 * wave; n0 < states; n0 += 16) {          // four of this wave's states of every row in flight
+    constexpr int kApart = WHOLE ? 1 : 4;
+    for (int n0 = WHOLE ? 4 * wave : wave; n0 < states; n0 += 16) {          // four of this wave's states of every row in flight
         float s[ROWS][4], a[4];
-        if (side_by_side) load_vec<T, 4>(a_log + (int64_t)c * states + n0, a);
+        if constexpr (WHOLE) load_vec<T, 4>(a_log + (int64_t)c * states + n0, a);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int n = min(n0 + u, states - 1);
-            if (!side_by_side) a[u] = T::load(a_log + (int64_t)c * states + n);
+            const int n = min(n0 + kApart * u, states - 1);
+            if constexpr (!WHOLE) a[u] = T::load(a_log + (int64_t)c * states + n);
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) s[r][u] = state[slot[r] * size + (int64_t)n * channels + c];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int n = n0 + u;
+            const int n = n0 + kApart * u;
             if (n >= states) break;
             const float A = -expf(a[u]) * kLog2e;
 #pragma unroll
@@ -754,7 +756,9 @@ extern "C" int nqh_scan_step(const void* x, const float* dt, const void* bc, int
     NQH_WITH_TYPE(dtype, {
         using E = typename T::elem;
         const int rows = batch >= 32 ? 4 : 1;                 // several rows share the exponentials of a_log
-        const auto kernel = rows == 4 ? scan_step_kernel<T, 4> : scan_step_kernel<T, 1>;
+        const bool whole = states % 16 == 0 && aligned(a_log, 16);
+        const auto kernel = rows == 4 ? (whole ? scan_step_kernel<T, 4, true> : scan_step_kernel<T, 4, false>)
+                                      : (whole ? scan_step_kernel<T, 1, true> : scan_step_kernel<T, 1, false>);
         kernel<<<dim3((unsigned)cdiv(channels, 64), (unsigned)cdiv(batch, rows)), dim3(256), 0, (hipStream_t)stream>>>(
             (const E*)x, dt, (const E*)bc, bc_stride, (const E*)z, z_stride, (const E*)a_log, (const E*)d_skip, state,
             state_slots, positions, active, (E*)out, (int)batch, (int)num_slots, (int)channels, (int)states);
