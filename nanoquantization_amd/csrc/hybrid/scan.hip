@@ -89,7 +89,8 @@ struct Raw16<Fp> {
     static __device__ __forceinline__ float get(type v, int e) { return v[e]; }
 };
 
-template <typename T, int V>
+// WHOLE: four taps, the weights on 16 bytes.
+template <typename T, int V, bool WHOLE>
 __global__ __launch_bounds__(256) void conv4_silu_kernel(const typename T::elem* __restrict__ x, int64_t x_stride,
                                                          const typename T::elem* __restrict__ w,
                                                          const typename T::elem* __restrict__ bias,
@@ -107,7 +108,7 @@ __global__ __launch_bounds__(256) void conv4_silu_kernel(const typename T::elem*
         v[j] = *reinterpret_cast<const typename Raw::type*>(x + (int64_t)max(pc.first + at, pc.index == 0 ? pc.first : 0) * x_stride + c);
     }
     load_vec<T, V>(bias + c, b);
-    if (taps == 4 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0) {
+    if constexpr (WHOLE) {
         // a lane's weights lie side by side: four loads, where one each is 4 V loads of as many cache lines as there are lanes
         // (8192 rows of 2048 channels: 26.3 -> 20.0 us)
         typename Raw::type wr[4];
@@ -625,16 +626,17 @@ extern "C" int nqh_conv_silu(const void* x, int64_t x_stride, const void* weight
         return fail(NQH_ERR_ARG, fn, "1 to 65535 pieces, and x rows at least as wide as the channels");
     (void)hipGetLastError();
 #define NQH_GO(KERNEL, V, ROWS)                                                                                            \
-    KERNEL<T, V><<<dim3((unsigned)cdiv(channels, 256 * V), (unsigned)num_pieces, (unsigned)cdiv(longest, ROWS)), dim3(256), 0, \
+    KERNEL<<<dim3((unsigned)cdiv(channels, 256 * V), (unsigned)num_pieces, (unsigned)cdiv(longest, ROWS)), dim3(256), 0, \
                    (hipStream_t)stream>>>((const E*)x, x_stride, (const E*)weight, (const E*)bias, tail, pieces, (E*)out,   \
                                           (int)channels, (int)taps)
     NQH_WITH_TYPE(dtype, {
         using E = typename T::elem;
         constexpr int V = 16 / sizeof(E);
         const bool vec = channels % V == 0 && x_stride % V == 0 && aligned(x, 16) && aligned(bias, 16) && aligned(out, 16);
-        if (taps <= 4 && vec) NQH_GO(conv4_silu_kernel, V, kConvRows);
-        else if (vec) NQH_GO(conv_silu_kernel, V, 8);
-        else NQH_GO(conv_silu_kernel, 1, 8);
+        if (taps == 4 && vec && aligned(weight, 16)) NQH_GO((conv4_silu_kernel<T, V, true>), V, kConvRows);
+        else if (taps <= 4 && vec) NQH_GO((conv4_silu_kernel<T, V, false>), V, kConvRows);
+        else if (vec) NQH_GO((conv_silu_kernel<T, V>), V, 8);
+        else NQH_GO((conv_silu_kernel<T, 1>), 1, 8);
     });
 #undef NQH_GO
     return launched(fn);
