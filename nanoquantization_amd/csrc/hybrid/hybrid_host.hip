@@ -10,7 +10,9 @@ namespace {
 thread_local char g_error[512] = "";
 
 // Largest logit per row, the lowest index among equal ones; NaNs are never selected.  As argmax_rows_kernel (nq_decode_ops.hip): a thread
-// keeps the largest of four logits at a time and looks for its place at the end (16 rows of 32768 6.0 -> 4.6 us, of 151936 16.2 -> 8.9).
+// keeps the largest of four logits at a time and looks for its place at the end (16 rows of 32768 6.0 -> 4.6 us, of 151936 16.2 -> 8.9).  Of
+// up to 16384 (FEW: a thread has four vectors) that look costs more than it saves, 2048 3.2 -> 3.35 us, 8200 3.85 -> 4.0.
+template <bool FEW>
 __global__ __launch_bounds__(1024) void argmax_f32_kernel(const float* __restrict__ logits, int64_t* __restrict__ out,
                                                           int vocab) {
     const float* row = logits + (size_t)blockIdx.x * vocab;
@@ -24,16 +26,24 @@ __global__ __launch_bounds__(1024) void argmax_f32_kernel(const float* __restric
     };
     const int nvec = (vocab & 3) == 0 ? vocab >> 2 : 0;   // rows are 16-byte aligned only then
     int bv = -1;                                          // the first of the thread's vectors that holds `best`
-    for (int v0 = threadIdx.x; v0 < nvec; v0 += 8 * 1024) {
-        f32x4 d[8];   // eight loads in flight
+    constexpr int kLoads = FEW ? 4 : 8;                   // in flight
+    for (int v0 = threadIdx.x; v0 < nvec; v0 += kLoads * 1024) {
+        f32x4 d[kLoads];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < kLoads; ++u) {
             const int v = v0 + u * 1024;
             d[u] = *reinterpret_cast<const f32x4*>(row + (size_t)(v < nvec ? v : v0) * 4);
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < kLoads; ++u) {
             const int v = v0 + u * 1024;
+            if constexpr (FEW) {
+                if (v < nvec) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) take(d[u][i], v * 4 + i);
+                }
+                continue;
+            }
             const float m = fmaxf(fmaxf(d[u][0], d[u][1]), fmaxf(d[u][2], d[u][3]));
             if (v < nvec && (m > best || (bv < 0 && m == best))) {
                 best = m;
@@ -92,7 +102,7 @@ extern "C" int nqh_argmax_rows(const float* logits, int64_t* out, int64_t rows, 
     if (rows <= 0 || vocab <= 0 || rows > kMaxI32 || vocab > 0x7ffffff0)
         return fail(NQH_ERR_ARG, fn, "rows and vocab must be positive 31-bit counts");
     (void)hipGetLastError();
-    argmax_f32_kernel<<<dim3((unsigned)rows), dim3(1024), 0, (hipStream_t)stream>>>(logits, out, (int)vocab);
+    (vocab <= 16384 ? argmax_f32_kernel<true> : argmax_f32_kernel<false>)<<<dim3((unsigned)rows), dim3(1024), 0, (hipStream_t)stream>>>(logits, out, (int)vocab);
     return launched(fn);
 }
 
