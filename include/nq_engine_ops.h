@@ -116,6 +116,56 @@ int nq_decode_prepare(const int64_t* positions, const uint8_t* active, const int
 int nq_decode_advance(const int64_t* next_tokens, const uint8_t* active, int64_t* out_log, int64_t* ids,
                       int64_t* positions, int64_t* step, int64_t rows, int64_t out_rows, void* stream);
 
+/* nq_paged_attention_decode with `out` in the input layout of nq_block_step: [ceil(batch / 16) * 16 rows], pieces of 16 rows x 32
+ * columns in the order of the matrix instruction's operand (rows past the batch are not written).  head_dim 128, one or two query
+ * heads per kv head.  Reference code as above. */
+int nq_paged_attention_decode_tiled(const void* q, const void* k_cache, const void* v_cache,
+                                    const int32_t* block_table, const int32_t* context_lens, void* out,
+                                    int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+                                    int64_t head_dim, int64_t block_size, int64_t max_blocks_per_seq,
+                                    int64_t num_blocks, float scale, int dtype, void* workspace,
+                                    size_t workspace_bytes, void* stream);
+
+/* A packed weight (qweight [K, N / 8], qscales [K / group_size, N], qzeros, as in awq_hip.h) laid out for nq_block_step:
+ * per 16 columns and 128 rows one piece of 1 KiB in the order of the matrix instruction's operand, then per column of every
+ * piece its scale and zero point.  N % 16 == 0, K % 128 == 0, group_size % 128 == 0. */
+size_t nq_tiled_weight_bytes(int64_t N, int64_t K);
+int nq_tile_weight(const int32_t* qweight, const void* qscales, const int32_t* qzeros, void* out, int64_t N, int64_t K,
+                   int64_t group_size, int dtype, void* stream);
+
+/* The linears between two attentions of a decode step, in one launch (bf16):
+ *   res_mid = res_in + o_proj(attn);  act = SiLU(gate) * up of RMSNorm(res_mid) * norm_mid;  res_out = res_mid + down_proj(act);
+ *   and, with qkv, the next layer's q|k|v of RMSNorm(res_out) * norm_next with q/k norm, rotary and cache write, as
+ *   awq_gemv_rmsnorm_qkv_rope_store (awq_hip.h) does it.
+ * Without qkv (the last layer) that part is left out; norm_next and what follows it may be NULL then.
+ * The weights are nq_tile_weight's: o [hidden, heads * 128], gate_up [2 * inter, hidden] with gate and up interleaved by words,
+ * down [hidden, inter], qkv [(heads + 2 * kv_heads) * 128, hidden] as [N, K].  res_in, res_out: [rows, hidden]; attn (of heads * 128 columns),
+ * act (inter), tiled_mid and tiled_out (res_mid and res_out, hidden) have nq_paged_attention_decode_tiled's layout; squares_mid and squares_out are
+ * fp32 [ceil(rows / 16) * 16][hidden / 8].  The result's bits are those of the launches one by one with K cut as awq_gemv_add_residual and
+ * awq_gemv_rmsnorm cut it at these sizes (hidden 2048: at up to 16 rows).  Rows past `rows` of attn must be numbers.
+ * `done`: nq_block_step_flag_words() words that are zero when the launch begins, of its own while it runs; `clear`: as many words of another launch
+ * that is over, which this one sets to zero (the launches of a step clear each other's in a ring).  Every buffer is of its own.
+ * The launch's workgroups hand rows to each other and wait for each other; one that has looked `spin` times in vain does what is missing
+ * itself, so that the launch ends whatever part of it runs at a time.  The sums are in a fixed order: results repeat exactly.
+ * rows 1..64, sizes that nq_block_step_supported names.
+ * Qwen3QuantizedBlock.forward, nanoquantization/models/qwen3_quantized.py:194-215 (and :79-93, :147-152), restricted to one token. */
+typedef struct nq_block_step_args {
+    const void *o, *gate_up, *down, *qkv;
+    const void *attn, *res_in, *norm_mid, *norm_next;
+    void *res_out, *tiled_mid, *tiled_out, *act;
+    float *squares_mid, *squares_out;
+    uint32_t *done, *clear;
+    const void *q_weight, *k_weight;
+    const float* cos_sin;
+    const int64_t *positions, *slots;
+    void *q_out, *k_cache, *v_cache;
+    int64_t rows, hidden, inter, heads, kv_heads, max_positions, num_slots, block_size, spin;
+    float eps, head_eps;
+} nq_block_step_args;
+int nq_block_step_supported(int64_t rows, int64_t hidden, int64_t inter, int64_t heads, int64_t kv_heads);
+size_t nq_block_step_flag_words(void);
+int nq_block_step(const nq_block_step_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -85,7 +85,22 @@ SYMBOLS = {
     "nq_argmax_rows": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nq_decode_prepare": (_int, [_vp] * 5 + [_i64] * 3 + [_vp]),
     "nq_decode_advance": (_int, [_vp] * 6 + [_i64] * 2 + [_vp]),
+    "nq_paged_attention_decode_tiled": (_int, [_vp] * 6 + [_i64] * 7 + [ctypes.c_float, _int, _vp, _sz, _vp]),
+    "nq_tiled_weight_bytes": (_sz, [_i64] * 2),
+    "nq_tile_weight": (_int, [_vp] * 4 + [_i64] * 3 + [_int, _vp]),
+    "nq_block_step_supported": (_int, [_i64] * 5),
+    "nq_block_step_flag_words": (_sz, []),
+    "nq_block_step": (_int, [_vp, _vp]),
 }
+
+
+class BlockStepArgs(ctypes.Structure):
+    """nq_block_step_args of include/nq_engine_ops.h"""
+    _fields_ = ([(n, _vp) for n in ("o", "gate_up", "down", "qkv", "attn", "res_in", "norm_mid", "norm_next", "res_out", "tiled_mid",
+                                    "tiled_out", "act", "squares_mid", "squares_out", "done", "clear", "q_weight", "k_weight",
+                                    "cos_sin", "positions", "slots", "q_out", "k_cache", "v_cache")]
+                + [(n, _i64) for n in ("rows", "hidden", "inter", "heads", "kv_heads", "max_positions", "num_slots", "block_size", "spin")]
+                + [("eps", ctypes.c_float), ("head_eps", ctypes.c_float)])
 
 
 # symbol -> (restype, argtypes) of libnq_hybrid.so; every symbol of include/nq_hybrid_ops.h

@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "awq_common.hpp"
+#include "step_epilogues.hpp"
 #include "step_kernels.hpp"
 #include "../../include/nq_engine_ops.h"
 
@@ -411,7 +412,7 @@ template <typename T, int G, int HD, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, uint16_t* __restrict__ out,
-    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, int nsplit, float scale) {
+    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, int nsplit, float scale, int tiled) {
     constexpr int LPT = HD / 8;    // lanes per token
     constexpr int TPW = 64 / LPT;  // tokens per wave step
     constexpr int U = 2;           // token steps in flight
@@ -422,6 +423,15 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int dc = lane % LPT, ts = lane / LPT;
 
+    // the first step's block numbers are asked for beside the context length where they don't hang on it: one trip to memory less before the
+    // first keys
+    const int32_t* table = block_table + (int64_t)b * max_blocks;
+    int blocks[U], blocks0 = 0;
+    if (nsplit == 1) {
+        blocks0 = table[0];
+#pragma unroll
+        for (int u = 0; u < U; ++u) blocks[u] = table[min((wave * TPW + ts + u * WAVES * TPW) / block_size, max_blocks - 1)];
+    }
     int ctx = context_lens[b];
     ctx = ctx < 0 ? 0 : (ctx > max_blocks * block_size ? max_blocks * block_size : ctx);
     const int per = (ctx + nsplit - 1) / nsplit;
@@ -443,7 +453,6 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
         for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
     }
 
-    const int32_t* table = block_table + (int64_t)b * max_blocks;
     for (int t = t0 + wave * TPW + ts; t - ts < t1; t += WAVES * TPW * U) {
         u32x4 kr[U], vr[U];
         bool ok[U];
@@ -452,7 +461,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
             const int tt = t + u * WAVES * TPW;
             ok[u] = tt < t1;
             const int tc = ok[u] ? tt : t0;
-            int blk = table[tc / block_size];
+            int blk = nsplit == 1 && t < WAVES * TPW * U ? (ok[u] ? blocks[u] : blocks0) : table[tc / block_size];
             blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
             const int64_t off = (((int64_t)blk * nkv + kvh) * block_size + tc % block_size) * HD + dc * 8;
             kr[u] = *reinterpret_cast<const u32x4*>(k_cache + off);
@@ -524,7 +533,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
         }
         const int64_t head = (int64_t)b * nh + kvh * G + g;
         if (nsplit == 1) {
-            out[head * HD + d] = T::from_f32(lt > 0.f ? at / lt : 0.f);
+            out[tiled ? tiled_at(b, (kvh * G + g) * HD + d, nh * HD) / 2 : head * HD + d] = T::from_f32(lt > 0.f ? at / lt : 0.f);
         } else {
             float* dst = partial + (head * nsplit + sp) * (HD + 2);
             dst[d] = at;
@@ -913,7 +922,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_tr_kernel(
 // Merge of the context splits: one workgroup of HD threads per (sequence, query head).
 template <typename T, int HD>
 __global__ __launch_bounds__(HD) void paged_attn_merge_kernel(const float* __restrict__ partial,
-                                                              uint16_t* __restrict__ out, int nsplit) {
+                                                              uint16_t* __restrict__ out, int nsplit, int heads) {
     const float* src = partial + (int64_t)blockIdx.x * nsplit * (HD + 2);
     const int d = threadIdx.x;
     float mn = kNegBig;
@@ -924,7 +933,8 @@ __global__ __launch_bounds__(HD) void paged_attn_merge_kernel(const float* __res
         lt += src[s * (HD + 2) + HD + 1] * c;
         at += src[s * (HD + 2) + d] * c;
     }
-    out[(int64_t)blockIdx.x * HD + d] = T::from_f32(lt > 0.f ? at / lt : 0.f);
+    const int64_t at_row = (int64_t)blockIdx.x * HD + d;
+    out[heads ? tiled_at((int)(blockIdx.x / heads), (int)(blockIdx.x % heads) * HD + d, heads * HD) / 2 : at_row] = T::from_f32(lt > 0.f ? at / lt : 0.f);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1043,7 +1053,7 @@ int pick_splits(int64_t batch, int64_t nkv, int64_t max_context, int G, bool tr)
 template <typename T, int G, int HD>
 void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* table, const int32_t* ctx, void* out,
                  float* partial, int64_t batch, int nkv, int bs, int max_blocks, int num_blocks, int nsplit,
-                 float scale, hipStream_t st) {
+                 float scale, int tiled, hipStream_t st) {
     constexpr int WAVES = G <= 2 ? 16 : (G <= 4 ? 8 : 4);
     if constexpr (HD == 128 && G == 8) {
         if (attn_tr(G, HD, bs)) {
@@ -1052,7 +1062,7 @@ void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* t
                 bs, max_blocks, num_blocks, nsplit, scale, G);
             if (nsplit > 1)
                 paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(
-                    partial, (uint16_t*)out, nsplit);
+                    partial, (uint16_t*)out, nsplit, 0);
             return;
         }
     }
@@ -1063,27 +1073,27 @@ void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* t
                 bs, max_blocks, num_blocks, nsplit, scale);
             if (nsplit > 1)
                 paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(
-                    partial, (uint16_t*)out, nsplit);
+                    partial, (uint16_t*)out, nsplit, 0);
             return;
         }
     }
     paged_attn_decode_kernel<T, G, HD, WAVES><<<dim3((unsigned)(batch * nkv * nsplit)), dim3(64 * WAVES), 0, st>>>(
         (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv, bs,
-        max_blocks, num_blocks, nsplit, scale);
+        max_blocks, num_blocks, nsplit, scale, tiled);
     if (nsplit > 1)
         paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(partial, (uint16_t*)out,
-                                                                                               nsplit);
+                                                                                               nsplit, tiled ? nkv * G : 0);
 }
 
 template <typename T, int HD>
 int launch_attn_g(int G, const void* q, const void* kc, const void* vc, const int32_t* table, const int32_t* ctx,
                   void* out, float* partial, int64_t batch, int nkv, int bs, int max_blocks, int num_blocks,
-                  int nsplit, float scale, hipStream_t st) {
+                  int nsplit, float scale, int tiled, hipStream_t st) {
     switch (G) {
 #define NQ_CASE(g)                                                                                              \
     case g:                                                                                                     \
         launch_attn<T, g, HD>(q, kc, vc, table, ctx, out, partial, batch, nkv, bs, max_blocks, num_blocks,      \
-                              nsplit, scale, st);                                                               \
+                              nsplit, scale, tiled, st);                                                        \
         return AWQ_OK;
         NQ_CASE(1) NQ_CASE(2) NQ_CASE(4) NQ_CASE(8)
 #undef NQ_CASE
@@ -1095,7 +1105,7 @@ int launch_attn_g(int G, const void* q, const void* kc, const void* vc, const in
                 bs, max_blocks, num_blocks, nsplit, scale, G);
             if (nsplit > 1)
                 paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(
-                    partial, (uint16_t*)out, nsplit);
+                    partial, (uint16_t*)out, nsplit, 0);
             return AWQ_OK;
         }
     }
@@ -1257,12 +1267,10 @@ extern "C" size_t nq_paged_attention_workspace_bytes(int64_t batch, int64_t num_
     return s > 1 ? (size_t)(batch * num_heads * s * (head_dim + 2)) * sizeof(float) : 0;
 }
 
-extern "C" int nq_paged_attention_decode(const void* q, const void* k_cache, const void* v_cache,
-                                         const int32_t* block_table, const int32_t* context_lens, void* out,
-                                         int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
-                                         int64_t block_size, int64_t max_blocks_per_seq, int64_t num_blocks, float scale,
-                                         int dtype, void* workspace, size_t workspace_bytes, void* stream) {
-    const char* fn = "nq_paged_attention_decode";
+static int paged_attention_decode(const char* fn, const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table,
+                                  const int32_t* context_lens, void* out, int64_t batch, int64_t num_heads, int64_t num_kv_heads,
+                                  int64_t head_dim, int64_t block_size, int64_t max_blocks_per_seq, int64_t num_blocks, float scale, int dtype,
+                                  int tiled, void* workspace, size_t workspace_bytes, void* stream) {
     if (!q || !k_cache || !v_cache || !block_table || !context_lens || !out) return bad(fn, "null pointer argument");
     if (!aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out))
         return bad(fn, "q, caches and out must be 16-byte aligned");
@@ -1292,21 +1300,44 @@ extern "C" int nq_paged_attention_decode(const void* q, const void* k_cache, con
         rc = head_dim == 128
                  ? launch_attn_g<F16, 128>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                            batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                           (int)num_blocks, nsplit, scale, st)
+                                           (int)num_blocks, nsplit, scale, tiled, st)
                  : launch_attn_g<F16, 64>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                           batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                          (int)num_blocks, nsplit, scale, st);
+                                          (int)num_blocks, nsplit, scale, tiled, st);
     else
         rc = head_dim == 128
                  ? launch_attn_g<BF16, 128>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                             batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                            (int)num_blocks, nsplit, scale, st)
+                                            (int)num_blocks, nsplit, scale, tiled, st)
                  : launch_attn_g<BF16, 64>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                            batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                           (int)num_blocks, nsplit, scale, st);
+                                           (int)num_blocks, nsplit, scale, tiled, st);
     if (rc != AWQ_OK) return rc;
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
+}
+
+extern "C" int nq_paged_attention_decode(const void* q, const void* k_cache, const void* v_cache,
+                                         const int32_t* block_table, const int32_t* context_lens, void* out,
+                                         int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                         int64_t block_size, int64_t max_blocks_per_seq, int64_t num_blocks, float scale,
+                                         int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+    return paged_attention_decode("nq_paged_attention_decode", q, k_cache, v_cache, block_table, context_lens, out, batch, num_heads, num_kv_heads,
+                                  head_dim, block_size, max_blocks_per_seq, num_blocks, scale, dtype, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int nq_paged_attention_decode_tiled(const void* q, const void* k_cache, const void* v_cache,
+                                               const int32_t* block_table, const int32_t* context_lens, void* out,
+                                               int64_t batch, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                               int64_t block_size, int64_t max_blocks_per_seq, int64_t num_blocks, float scale,
+                                               int dtype, void* workspace, size_t workspace_bytes, void* stream) {
+    const char* fn = "nq_paged_attention_decode_tiled";
+    if (head_dim != 128 || num_kv_heads <= 0 || (num_heads != num_kv_heads && num_heads != 2 * num_kv_heads)) {
+        set_error("%s: head_dim 128, one or two query heads per kv head", fn);
+        return AWQ_ERR_UNSUPPORTED;
+    }
+    return paged_attention_decode(fn, q, k_cache, v_cache, block_table, context_lens, out, batch, num_heads, num_kv_heads, head_dim, block_size,
+                                  max_blocks_per_seq, num_blocks, scale, dtype, 1, workspace, workspace_bytes, stream);
 }
 
 extern "C" int nq_argmax_rows(const void* logits, int64_t* out, int64_t rows, int64_t vocab, int dtype,

@@ -79,6 +79,15 @@ class LLMEngine(EngineCore):
             max_batch, o0.out_features, o0.in_features, o0.group_size)
         self.down_add_norm = d0.bias is None and ops.gemv_add_rmsnorm_supported(
             max_batch, d0.out_features, d0.in_features, d0.group_size)
+        # the linears between two attentions in one launch, of weights in a layout of their own: two launches per block
+        tiled = lambda m: (m.qweight, m.qscales, m.qzeros)
+        self.block_steps = None
+        if (self.norm_fused_ok and o0.bias is None and d0.bias is None
+                and all(l.self_attn.o_proj.group_size % 128 == 0 and l.mlp.down_proj.group_size % 128 == 0 for l in layers)
+                and ops.BlockSteps.supported(max_batch, hidden, self.inter, self.nh, self.nkv, len(layers), self.dtype)):
+            self.block_steps = ops.BlockSteps([(tiled(self.qkv[i]) if i else None, tiled(l.self_attn.o_proj), self.gate_up_il[i],
+                                                tiled(l.mlp.down_proj)) for i, l in enumerate(layers)],
+                                              max_batch, hidden, self.inter, self.nh, self.nkv, self.device)
         # prompts through the cache on the prompt attention kernel, which has matrix forms for these rows
         self.paged_prefill = self.dtype == torch.bfloat16 and self.hd in (32, 64, 96, 128, 192, 256)
         self.eps = layers[0].input_layernorm.eps
@@ -218,11 +227,24 @@ class LLMEngine(EngineCore):
             x, ssq = ops.embed_row_ssq(self.s_ids, m.embed_tokens.weight)   # residual stream [B, hidden]
             for li, layer in enumerate(m.layers):
                 attn, lin, mlp = layer.self_attn, self.qkv[li], layer.mlp
-                prefetch_hint(attn.o_proj.qweight, attn.o_proj.qscales)
-                q = ops.awq_gemv_rmsnorm_qkv_rope_store(
-                    x, ssq, layer.input_layernorm.weight, eps, lin.qweight, lin.qscales, lin.qzeros,
-                    attn.q_norm.weight, attn.k_norm.weight, attn.rope.cos_sin_cache, pos, slots, self.cache.k[li],
-                    self.cache.v[li], self.nh, self.nkv, attn.q_norm.eps)
+                steps = self.block_steps
+                if steps is None or li == 0:
+                    if steps is None:
+                        prefetch_hint(attn.o_proj.qweight, attn.o_proj.qscales)
+                    q = ops.awq_gemv_rmsnorm_qkv_rope_store(
+                        x, ssq, layer.input_layernorm.weight, eps, lin.qweight, lin.qscales, lin.qzeros,
+                        attn.q_norm.weight, attn.k_norm.weight, attn.rope.cos_sin_cache, pos, slots, self.cache.k[li],
+                        self.cache.v[li], self.nh, self.nkv, attn.q_norm.eps)
+                if steps is not None:
+                    # two launches per block: attention, and all linears up to the next layer's q|k|v
+                    ops.paged_attention_decode(q, self.cache.k[li], self.cache.v[li], self.s_table, ctx, self.scale, steps.attn)
+                    following = None
+                    if li + 1 < nl:
+                        after = m.layers[li + 1].self_attn
+                        following = (m.layers[li + 1].input_layernorm.weight, after.q_norm.weight, after.k_norm.weight,
+                                     after.rope.cos_sin_cache, pos, slots, self.cache.k[li + 1], self.cache.v[li + 1], after.q_norm.eps)
+                    x, q = steps(li, x, layer.post_attention_layernorm.weight, eps, following), steps.q
+                    continue
                 o = ops.paged_attention_decode(q, self.cache.k[li], self.cache.v[li], self.s_table, ctx, self.scale)
                 prefetch_hint(*self.gate_up_il[li][:2])
                 ops.awq_gemv_add_residual(o, attn.o_proj.qweight, attn.o_proj.qscales, attn.o_proj.qzeros, x, ssq)

@@ -4,7 +4,8 @@ Each function checks shapes on the host, allocates its output with torch (graph-
 the caching allocator) and launches on the current stream.  HIP device tensors only."""
 from __future__ import annotations
 
-from typing import Optional
+import ctypes
+from typing import Optional, Sequence
 
 import torch
 
@@ -240,9 +241,10 @@ def awq_gemv_rmsnorm_qkv_rope_store(x: torch.Tensor, ssq: torch.Tensor, norm_wei
 
 
 def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
-                           context_lens: torch.Tensor, scale: float) -> torch.Tensor:
+                           context_lens: torch.Tensor, scale: float, tiled_out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """q [batch, nh, hd]; caches [num_blocks, nkv, block_size, hd]; block_table int32 [batch, max_blocks];
-    context_lens int32 [batch].  Returns [batch, nh * hd]."""
+    context_lens int32 [batch].  Returns [batch, nh * hd], or writes it to `tiled_out` [ceil(batch / 16) * 16, nh * hd] in the
+    layout BlockSteps reads."""
     dev = _dev(q, k_cache, v_cache, block_table, context_lens)
     batch, nh, hd = q.shape
     num_blocks, nkv, block_size, hd2 = k_cache.shape
@@ -250,12 +252,16 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     assert block_table.dtype == torch.int32 and context_lens.dtype == torch.int32
     assert block_table.shape[0] == batch and context_lens.shape == (batch,)
     max_blocks = block_table.shape[1]
-    out = torch.empty(batch, nh * hd, dtype=q.dtype, device=dev)
     L = _lib.lib()
+    if tiled_out is None:
+        out, entry = torch.empty(batch, nh * hd, dtype=q.dtype, device=dev), L.nq_paged_attention_decode
+    else:
+        out, entry = tiled_out, L.nq_paged_attention_decode_tiled
+        assert _dev(out) == dev and out.shape == (-(-batch // 16) * 16, nh * hd) and out.dtype == q.dtype
     with _lib.on_device(dev):
         nbytes = L.nq_paged_attention_workspace_bytes(batch, nh, nkv, hd, block_size * max_blocks)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
-        _lib.check(L.nq_paged_attention_decode(
+        _lib.check(entry(
             q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr(), context_lens.data_ptr(),
             out.data_ptr(), batch, nh, nkv, hd, block_size, max_blocks, num_blocks, scale, _lib.dtype_id(q.dtype),
             None if ws is None else ws.data_ptr(), nbytes, _stream(dev)))
@@ -373,3 +379,77 @@ def awq_gemv_swiglu(x: torch.Tensor, qweight: torch.Tensor, qscales: torch.Tenso
                                      out.data_ptr(), M, N, K, g, _lib.dtype_id(x.dtype),
                                      None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), stream))
     return out
+
+
+def tile_weight(qweight: torch.Tensor, qscales: torch.Tensor, qzeros: torch.Tensor) -> torch.Tensor:
+    """A packed weight in the layout BlockSteps reads (nq_tile_weight)."""
+    dev = _dev(qweight, qscales, qzeros)
+    K, N = qweight.shape[0], qscales.shape[1]
+    g = K // qscales.shape[0]
+    assert qweight.shape == (K, N // 8) and qzeros.shape == (K // g, N // 8)
+    L = _lib.lib()
+    out = torch.empty(L.nq_tiled_weight_bytes(N, K), dtype=torch.uint8, device=dev)
+    with _lib.on_device(dev):
+        _lib.check(L.nq_tile_weight(qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(), out.data_ptr(), N, K, g,
+                                    _lib.dtype_id(qscales.dtype), _stream(dev)))
+    return out
+
+
+class BlockSteps:
+    """The linears between the attentions of a decode step, a launch a layer (nq_block_step): the weights of every layer in its layout and
+    the buffers its launches hand on.  Each layer: (q|k|v, o_proj, interleaved gate|up, down_proj) as (qweight, qscales, qzeros); the
+    first layer's q|k|v is the caller's and None here.  One step at a time (the buffers are the object's)."""
+    SPIN = 1 << 14      # looks, some 0.6 us each: by then a workgroup that is not there yet will not come by itself
+
+    @staticmethod
+    def supported(rows: int, hidden: int, inter: int, heads: int, kv_heads: int, layers: int, dtype: torch.dtype) -> bool:
+        return (dtype == torch.bfloat16 and layers >= 2
+                and bool(_lib.lib().nq_block_step_supported(rows, hidden, inter, heads, kv_heads)))
+
+    def __init__(self, layers: Sequence, rows: int, hidden: int, inter: int, heads: int, kv_heads: int, device: torch.device):
+        self.weights = [[None if w is None else tile_weight(*w) for w in layer] for layer in layers]
+        self.sizes = dict(rows=rows, hidden=hidden, inter=inter, heads=heads, kv_heads=kv_heads)
+        zeros = lambda *shape, dtype=torch.bfloat16: torch.zeros(*shape, dtype=dtype, device=device)
+        padded = -(-rows // 16) * 16
+        self.attn, self.act, self.q = zeros(padded, heads * 128), zeros(padded, inter), zeros(rows, heads, 128)
+        self.residual = [zeros(rows, hidden) for _ in range(2)]
+        self.tiled = [zeros(padded, hidden) for _ in range(2)]
+        self.squares = [zeros(padded, hidden // 8, dtype=torch.float32) for _ in range(2)]
+        # the flags of a launch are cleared by the launch behind it, those of the last layer by the first of the next step; where a step was
+        # not finished, by the host
+        self.done = zeros(len(layers), _lib.lib().nq_block_step_flag_words(), dtype=torch.int32)
+        self.next = 0
+
+    def __call__(self, index: int, residual: torch.Tensor, norm_mid: torch.Tensor, eps: float, following=None, spin: int = SPIN) -> torch.Tensor:
+        """Layer `index` from `self.attn` and its residual [rows, hidden] on; returns the residual behind it.  `following`: (norm weight, q_norm
+        weight, k_norm weight, cos_sin, positions, slots, k_cache, v_cache, q/k norm eps) of the next layer, whose q goes to `self.q`."""
+        w, s = self.weights[index], self.sizes
+        dev = _dev(residual, norm_mid)
+        if index != self.next:
+            self.done.zero_()
+        self.next = -1
+        assert residual.shape == (s["rows"], s["hidden"]) and residual.dtype == torch.bfloat16
+        assert norm_mid.shape == (s["hidden"],) and norm_mid.dtype == torch.bfloat16
+        out = self.residual[index % 2]
+        tensors = dict(o=w[1], gate_up=w[2], down=w[3], attn=self.attn, res_in=residual, res_out=out, act=self.act,
+                       tiled_mid=self.tiled[0], tiled_out=self.tiled[1], squares_mid=self.squares[0], squares_out=self.squares[1],
+                       norm_mid=norm_mid, done=self.done[index], clear=self.done[index - 1])
+        a = _lib.BlockStepArgs(eps=eps, spin=spin, **s)
+        if following is not None:
+            norm, q_norm, k_norm, cos_sin, positions, slots, k_cache, v_cache, head_eps = following
+            assert _dev(norm, q_norm, k_norm, cos_sin, positions, slots, k_cache, v_cache) == dev
+            assert norm.shape == (s["hidden"],) and q_norm.shape == (128,) and k_norm.shape == (128,)
+            assert norm.dtype == q_norm.dtype == k_norm.dtype == k_cache.dtype == v_cache.dtype == torch.bfloat16
+            assert k_cache.dim() == 4 and k_cache.shape == v_cache.shape and k_cache.shape[1] == s["kv_heads"] and k_cache.shape[3] == 128
+            assert cos_sin.dtype == torch.float32 and cos_sin.numel() % 128 == 0
+            assert positions.dtype == slots.dtype == torch.int64 and positions.numel() == slots.numel() == s["rows"]
+            tensors.update(qkv=self.weights[index + 1][0], norm_next=norm, q_weight=q_norm, k_weight=k_norm, cos_sin=cos_sin,
+                           positions=positions, slots=slots, q_out=self.q, k_cache=k_cache, v_cache=v_cache)
+            a.max_positions, a.block_size, a.head_eps = cos_sin.numel() // 128, k_cache.shape[2], head_eps
+            a.num_slots = k_cache.shape[0] * a.block_size
+        for name, t in tensors.items():
+            setattr(a, name, t.data_ptr())
+        with _lib.on_device(dev):
+            _lib.check(_lib.lib().nq_block_step(ctypes.byref(a), _stream(dev)))
+        self.next = (index + 1) % len(self.weights)
+        return out
