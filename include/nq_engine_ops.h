@@ -162,7 +162,7 @@ typedef struct nq_block_step_args {
     int64_t rows, hidden, inter, heads, kv_heads, max_positions, num_slots, block_size, spin;
     float eps, head_eps;
 } nq_block_step_args;
-int nq_block_step_supported(int64_t rows, int64_t hidden, int64_t inter, int64_t heads, int64_t kv_heads);
+size_t nq_block_step_supported(int64_t rows, int64_t hidden, int64_t inter, int64_t heads, int64_t kv_heads);
 size_t nq_block_step_flag_words(void);
 int nq_block_step(const nq_block_step_args* args, void* stream);
 

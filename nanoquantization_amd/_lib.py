@@ -88,7 +88,7 @@ SYMBOLS = {
     "nq_paged_attention_decode_tiled": (_int, [_vp] * 6 + [_i64] * 7 + [ctypes.c_float, _int, _vp, _sz, _vp]),
     "nq_tiled_weight_bytes": (_sz, [_i64] * 2),
     "nq_tile_weight": (_int, [_vp] * 4 + [_i64] * 3 + [_int, _vp]),
-    "nq_block_step_supported": (_int, [_i64] * 5),
+    "nq_block_step_supported": (_sz, [_i64] * 5),
     "nq_block_step_flag_words": (_sz, []),
     "nq_block_step": (_int, [_vp, _vp]),
 }
