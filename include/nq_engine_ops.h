@@ -145,6 +145,7 @@ int nq_tile_weight(const int32_t* qweight, const void* qscales, const int32_t* q
  * awq_gemv_rmsnorm cut it at these sizes (hidden 2048: at up to 16 rows).  Rows past `rows` of attn must be numbers.
  * `done`: nq_block_step_flag_words() words that are zero when the launch begins, of its own while it runs; `clear`: as many words of another launch
  * that is over, which this one sets to zero (the launches of a step clear each other's in a ring).  Every buffer is of its own.
+ * next: up to four regions that the launch after this one reads (NULL: none); workgroups that are idle in the last phase bring them near.
  * The launch's workgroups hand rows to each other and wait for each other; one that has looked `spin` times in vain does what is missing
  * itself, so that the launch ends whatever part of it runs at a time.  The sums are in a fixed order: results repeat exactly.
  * rows 1..64, sizes that nq_block_step_supported names.
@@ -160,6 +161,8 @@ typedef struct nq_block_step_args {
     const int64_t *positions, *slots;
     void *q_out, *k_cache, *v_cache;
     int64_t rows, hidden, inter, heads, kv_heads, max_positions, num_slots, block_size, spin;
+    const void* next[4];
+    size_t next_bytes[4];
     float eps, head_eps;
 } nq_block_step_args;
 size_t nq_block_step_supported(int64_t rows, int64_t hidden, int64_t inter, int64_t heads, int64_t kv_heads);

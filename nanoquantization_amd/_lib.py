@@ -100,7 +100,7 @@ class BlockStepArgs(ctypes.Structure):
                                     "tiled_out", "act", "squares_mid", "squares_out", "done", "clear", "q_weight", "k_weight",
                                     "cos_sin", "positions", "slots", "q_out", "k_cache", "v_cache")]
                 + [(n, _i64) for n in ("rows", "hidden", "inter", "heads", "kv_heads", "max_positions", "num_slots", "block_size", "spin")]
-                + [("eps", ctypes.c_float), ("head_eps", ctypes.c_float)])
+                + [("next", _vp * 4), ("next_bytes", _sz * 4), ("eps", ctypes.c_float), ("head_eps", ctypes.c_float)])
 
 
 # symbol -> (restype, argtypes) of libnq_hybrid.so; every symbol of include/nq_hybrid_ops.h

@@ -59,6 +59,8 @@ struct BlockStep {
     float eps;
     int rows, spin;
     QkvEpilogue qe;
+    const char* next[4];
+    int64_t next_lines[4];
 };
 
 typedef __amdgpu_buffer_rsrc_t Rsrc;
@@ -486,6 +488,17 @@ __global__ __launch_bounds__(kBlockThreads) void block_step_kernel(const BlockSt
     phase(per0, tasks0, shares0, a.done + 2 * kPhaseWords, !a.norm_next, [&](int task) { down_proj(task, false, late); },
           [&](int task) { down_proj(task, true, [] {}); });
     if (!a.norm_next) return;
+    if (own >= 8 * per3) {
+        // Workgroups without a head touch the lines of the weights that the launch behind the next attention reads, which then finds them in the
+        // memory-side cache (28 layers, 32 rows: 1295 -> 1268 us a step).
+        const int64_t threads = (int64_t)(kShares - 8 * per3) * kBlockThreads, at = (int64_t)(own - 8 * per3) * kBlockThreads + threadIdx.x;
+        uint32_t seen = 0;
+        for (int r = 0; r < 4; ++r)
+            for (int64_t line = at; line < a.next_lines[r]; line += threads)
+                seen |= *reinterpret_cast<const volatile uint32_t*>(a.next[r] + line * 128);
+        asm volatile("" ::"v"(seen));
+        return;
+    }
     // q|k|v of the next layer, one head and 16 rows a task
     for (int task = own3; task < end3; task += 32) {
         const int head = over(task, m_tiles), row0 = (task - head * m_tiles) * 16;
@@ -642,6 +655,7 @@ extern "C" int nq_block_step(const nq_block_step_args* p, void* stream) {
     a.qe.q_out = (uint16_t*)q.q_out, a.qe.k_cache = (uint16_t*)q.k_cache, a.qe.v_cache = (uint16_t*)q.v_cache;
     a.qe.nh = (int)q.heads, a.qe.nkv = (int)q.kv_heads, a.qe.max_positions = (int)q.max_positions, a.qe.block_size = (int)q.block_size;
     a.qe.num_slots = q.num_slots, a.qe.eps = q.head_eps;
+    for (int i = 0; i < 4; ++i) a.next[i] = (const char*)q.next[i], a.next_lines[i] = q.next[i] ? (int64_t)(q.next_bytes[i] / 128) : 0;
     const hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();
     const int mt = (int)((q.rows + 15) / 16);

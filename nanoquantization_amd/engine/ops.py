@@ -447,6 +447,8 @@ class BlockSteps:
                            positions=positions, slots=slots, q_out=self.q, k_cache=k_cache, v_cache=v_cache)
             a.max_positions, a.block_size, a.head_eps = cos_sin.numel() // 128, k_cache.shape[2], head_eps
             a.num_slots = k_cache.shape[0] * a.block_size
+            for i, near in enumerate([*self.weights[index + 1][1:], *(w[0] for w in self.weights[index + 2:index + 3])]):
+                a.next[i], a.next_bytes[i] = near.data_ptr(), near.numel()
         for name, t in tensors.items():
             setattr(a, name, t.data_ptr())
         with _lib.on_device(dev):
