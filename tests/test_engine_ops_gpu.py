@@ -216,6 +216,32 @@ def test_paged_attention_decode(dtype, B, nh, nkv, hd, bs, max_blocks):
     assert torch.equal(out, ops.paged_attention_decode(q, kc, vc, table, ctx, scale)), "run-to-run bit-stable"
 
 
+@pytest.mark.parametrize("B,nh,nkv,bs,max_blocks", [
+    (1, 16, 8, 64, 40),           # 16 parts, the most
+    (2, 32, 8, 64, 21),           # 16, four heads per kv head; the second sequence leaves most of them empty
+    (6, 16, 8, 64, 21),           # 5: 240 workgroups
+    (20, 16, 8, 64, 41),          # 3: 480, two a CU
+    (31, 16, 8, 64, 10),          # one below the 256 pairs that are not split
+    (1, 2, 1, 32, 3),             # fewer tokens than two parts' 64
+])
+def test_paged_attention_split_counts(B, nh, nkv, bs, max_blocks):
+    """The number of parts follows from the pairs and the table's length; sequences shorter than that leave parts empty."""
+    from nanoquantization_amd.engine import ops
+    g = torch.Generator().manual_seed(B)
+    nb = B * max_blocks + 1
+    kc = torch.randn(nb, nkv, bs, 128, generator=g).bfloat16().cuda()
+    vc = torch.randn(nb, nkv, bs, 128, generator=g).bfloat16().cuda()
+    q = torch.randn(B, nh, 128, generator=g).bfloat16().cuda()
+    table = torch.randperm(nb, generator=g)[: B * max_blocks].view(B, max_blocks).to(torch.int32).cuda()
+    ctx = torch.randint(1, bs * max_blocks + 1, (B,), generator=g).to(torch.int32)
+    ctx[0], ctx[-1] = bs * max_blocks, bs * max_blocks if B == 1 else 5
+    ctx = ctx.cuda()
+    scale = 128 ** -0.5
+    out = ops.paged_attention_decode(q, kc, vc, table, ctx, scale)
+    _close(out, _attn_ref(q, kc, vc, table, ctx, scale), torch.bfloat16, scale=2.0, what="attention")
+    assert torch.equal(out, ops.paged_attention_decode(q, kc, vc, table, ctx, scale)), "run-to-run bit-stable"
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nh,nkv,bs", [(16, 8, 32), (64, 8, 32), (16, 4, 32), (40, 8, 32), (64, 8, 16), (40, 8, 48)])
 def test_paged_attention_ignores_rows_past_the_context(dtype, nh, nkv, bs):
