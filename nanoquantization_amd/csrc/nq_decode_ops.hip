@@ -546,7 +546,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     }
 }
 
-// The same for 4 or 8 query heads per kv head and 128 head dims, where the kernel above is bound by its
+// The same for 2, 4 or 8 query heads per kv head and 128 head dims, where the kernel above is bound by its
 // vector-ALU dot products (8 FMAs, 4 shuffles and an online-softmax update per token, head and lane).
 // A wave takes tiles of 16 tokens.  Scores: S^T = K q^T on the 16x16x32 MFMA (A = 16 token rows of K, 32 head dims
 // per instruction; B = the G query heads as columns, the rest zero), so a lane ends up with 4 tokens of one head and
@@ -554,13 +554,24 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
 // value phase through a 16 x G array in LDS (private to the wave); there a lane holds 8 head dims of one token's V row
 // as before and adds p * v for the G heads.  Tiles start at multiples of 16 tokens inside a context split and
 // block_size % 16 == 0, so a tile never straddles a cache block.
+// A lane holds the block of one of its wave's next 64 tiles each, so that a tile is one trip to memory and not two.  Rows past the context lie
+// outside the buffer of their load: they are zero and cost no memory access.
+// Bound by memory once 256 workgroups run; then the cache streams past the L2 (`full`: the rounds of workgroups on 256 CUs are three quarters full or
+// more; and the workgroup's context is its share of 16 MB or more).  bf16, 8 kv heads, us, 28 layers' caches in turn; two heads, the vector kernel / this one:
+// 1 x 1300 14.0 / 8.2, 8 x 320 11.2 / 7.8, 12 x 640 21.7 / 13.6, 32 x 640 21.0 / 16.5,
+// 64 x 640 38 / 28.4, 64 x 1000 63.5 / 44.7 = 5.9 TB/s, 1 x 8000 24.9 / 14.7.  Four heads, this one with a tile
+// behind its block number / now: 1 x 1300 13.5 / 8.7, 24 x 640 19.8 / 16.7, 32 x 640 20.2 / 18.2, 64 x 1000 52.4 / 44.9, 1 x 140 5.6 / 5.9.  Through the L2 32 x 640 takes 19.2 and
+// 64 x 1000 50; part rounds and smaller caches are better off there (20 x 640 13.2, past it 14.3; 8 x 140 5.6, 6.2).  Two or more tiles on their way in a
+// wave's registers take longer at every size (32 x 640 19.2 with two, 20.0 with four).
 template <typename T, int G, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, uint16_t* __restrict__ out,
-    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, int nsplit, float scale) {
+    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, int nsplit, float scale, int tiled,
+    int full) {
     constexpr int HD = 128, TT = 16;
-    static_assert(G == 4 || G == 8, "query heads per kv head");
+    static_assert(G == 2 || G == 4, "query heads per kv head");
+    typedef float fG __attribute__((ext_vector_type(G)));
     const int sp = blockIdx.x % nsplit;
     const int kvh = (blockIdx.x / nsplit) % nkv;
     const int b = blockIdx.x / (nsplit * nkv);
@@ -568,15 +579,14 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lo = lane & 15, hi = lane >> 4;   // score phase: head lo, token quad hi; value phase: dims 8*lo.., token hi
 
+    const int32_t* table = block_table + (int64_t)b * max_blocks;
+    // blocks of the wave's tiles first, first + 1, .., one a lane
+    const auto blocks_from = [&](int t0, int first) {
+        const int64_t t = t0 + ((int64_t)(first + lane) * WAVES + wave) * TT, last = (int64_t)max_blocks * block_size - 1;
+        return table[(uint32_t)min(t, last) / (uint32_t)block_size];
+    };
+    int blocks = nsplit == 1 ? blocks_from(0, 0) : 0;     // asked for beside the context length
     int ctx = context_lens[b];
-    ctx = ctx < 0 ? 0 : (ctx > max_blocks * block_size ? max_blocks * block_size : ctx);
-    const int per = ((ctx + nsplit - 1) / nsplit + TT - 1) / TT * TT;
-    const int t0 = sp * per, t1 = min(ctx, t0 + per);
-
-    __shared__ float s_p[WAVES][TT * G + G];   // per wave: p[token][head], then the rescale factor per head
-    __shared__ float s_acc[WAVES][G][HD + 2];
-    float* P = s_p[wave];
-
     u32x4 bq[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -584,6 +594,37 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         if (lo < G)
             bq[i] = *reinterpret_cast<const u32x4*>(q + ((int64_t)b * nh + kvh * G + lo) * HD + 32 * i + 8 * hi);
     }
+    ctx = ctx < 0 ? 0 : (ctx > max_blocks * block_size ? max_blocks * block_size : ctx);
+    const int per = nsplit == 1 ? ctx : ((ctx + nsplit - 1) / nsplit + TT - 1) / TT * TT;
+    const int t0 = sp * per, t1 = min(ctx, t0 + per);
+    const int tiles = t1 - t0 > wave * TT ? (t1 - t0 - wave * TT + WAVES * TT - 1) / (WAVES * TT) : 0;
+    if (nsplit > 1) blocks = blocks_from(t0, 0);
+    int held = 0;
+
+    __shared__ __align__(16) float s_p[WAVES][TT * G + G];   // per wave: p[token][head], then the rescale factor per head
+    __shared__ float s_acc[WAVES][G][HD + 2];
+    float* P = s_p[wave];
+
+    u32x4 ka[4], va[4];
+    const auto load = [&](int tile, auto policy) __attribute__((always_inline)) {
+        constexpr int kPolicy = decltype(policy)::value;
+        if (tile - held >= 64 && tile < tiles) {
+            held = tile;
+            blocks = blocks_from(t0, held);
+        }
+        int blk = __builtin_amdgcn_readlane(blocks, (tile - held) & 63);
+        blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
+        const int tb = t0 + (tile * WAVES + wave) * TT;
+        const uint32_t bytes = tile < tiles ? (uint32_t)min(TT, t1 - tb) * (HD * 2) : 0u;
+        const int64_t base = tile < tiles ? (((int64_t)blk * nkv + kvh) * block_size + tb % block_size) * HD : 0;
+        const __amdgpu_buffer_rsrc_t k = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(k_cache + base), 0, bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t v = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(v_cache + base), 0, bytes, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ka[i] = __builtin_amdgcn_raw_buffer_load_b128(k, lo * 256 + hi * 16 + 64 * i, 0, kPolicy);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) va[u] = __builtin_amdgcn_raw_buffer_load_b128(v, hi * 256 + lo * 16 + 1024 * u, 0, kPolicy);
+    };
+
     const float sc = scale * kLog2e;
     float m = kNegBig, lpart = 0.f;
     float acc[G][8];
@@ -592,28 +633,16 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
 
-    const int32_t* table = block_table + (int64_t)b * max_blocks;
-    for (int tb = t0 + wave * TT; tb < t1; tb += WAVES * TT) {
-        int blk = table[tb / block_size];                         // wave-uniform
-        blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
-        const int64_t base = (((int64_t)blk * nkv + kvh) * block_size + tb % block_size) * HD;
-        u32x4 ka[4], va[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)   // K row of token tb + lo (rows past the context are masked below)
-            ka[i] = *reinterpret_cast<const u32x4*>(k_cache + base + (int64_t)lo * HD + 32 * i + 8 * hi);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {   // V rows: a masked token reads the last valid row (its p is 0, the row is finite)
-            const int tv = min(4 * u + hi, t1 - 1 - tb);
-            va[u] = *reinterpret_cast<const u32x4*>(v_cache + base + (int64_t)tv * HD + 8 * lo);
-        }
+    const auto take = [&](int tile) __attribute__((always_inline)) {
+        const int left = t1 - (t0 + (tile * WAVES + wave) * TT);
         f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) st = T::mfma16(ka[i], bq[i], st);
-        // st[r]: head lo, token tb + 4*hi + r
+        // st[r]: head lo, token 4*hi + r of the tile
         float sv[4], mx = kNegBig;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            sv[r] = (tb + 4 * hi + r < t1) ? st[r] * sc : kNegBig;
+            sv[r] = (4 * hi + r < left) ? st[r] * sc : kNegBig;
             mx = fmaxf(mx, sv[r]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -625,7 +654,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         float pr[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            pr[r] = (tb + 4 * hi + r < t1) ? exp2f(sv[r] - mn) : 0.f;
+            pr[r] = (4 * hi + r < left) ? exp2f(sv[r] - mn) : 0.f;
             ps += pr[r];
         }
         lpart = lpart * c + ps;
@@ -637,25 +666,16 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         asm volatile("" ::: "memory");
         __builtin_amdgcn_wave_barrier();   // LDS operations of a wave execute in order: the reads below see these writes
         asm volatile("" ::: "memory");
-        float cg[G];
-#pragma unroll
-        for (int g = 0; g < G; g += 4) {
-            const f32x4 v4 = *reinterpret_cast<const f32x4*>(P + TT * G + g);
-            cg[g] = v4[0]; cg[g + 1] = v4[1]; cg[g + 2] = v4[2]; cg[g + 3] = v4[3];
-        }
+        const fG cg = *reinterpret_cast<const fG*>(P + TT * G);
 #pragma unroll
         for (int g = 0; g < G; ++g)
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[g][e] *= cg[g];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            float vf[8], pg[G];
+            float vf[8];
             unpack8<T>(va[u], vf);
-#pragma unroll
-            for (int g = 0; g < G; g += 4) {
-                const f32x4 v4 = *reinterpret_cast<const f32x4*>(P + (4 * u + hi) * G + g);
-                pg[g] = v4[0]; pg[g + 1] = v4[1]; pg[g + 2] = v4[2]; pg[g + 3] = v4[3];
-            }
+            const fG pg = *reinterpret_cast<const fG*>(P + (4 * u + hi) * G);
 #pragma unroll
             for (int g = 0; g < G; ++g)
 #pragma unroll
@@ -664,7 +684,16 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         asm volatile("" ::: "memory");
         __builtin_amdgcn_wave_barrier();   // the next tile's writes come after these reads
         asm volatile("" ::: "memory");
-    }
+    };
+    const auto walk = [&](auto policy) {
+        load(0, policy);
+        for (int tile = 0; tile < tiles; ++tile) {
+            take(tile);
+            load(tile + 1, policy);     // (behind a condition the loop takes half as long again, 32 x 640 25.1 us)
+        }
+    };
+    if (full && (int64_t)(t1 - t0) * gridDim.x >= 32768) walk(std::integral_constant<int, 2>{});      // nt
+    else walk(std::integral_constant<int, 0>{});
 
     // the four token groups of the wave share m: their accumulators and partial sums just add
 #pragma unroll
@@ -701,7 +730,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         }
         const int64_t head = (int64_t)b * nh + kvh * G + g;
         if (nsplit == 1) {
-            out[head * HD + d] = T::from_f32(lt > 0.f ? at / lt : 0.f);
+            out[tiled ? tiled_at(b, (kvh * G + g) * HD + d, nh * HD) / 2 : head * HD + d] = T::from_f32(lt > 0.f ? at / lt : 0.f);
         } else {
             float* dst = partial + (head * nsplit + sp) * (HD + 2);
             dst[d] = at;
@@ -1046,12 +1075,9 @@ bool attn_tr(int G, int64_t head_dim, int64_t block_size) {
 }
 int attn_waves(int G, bool tr) { return tr ? 4 : (G <= 2 ? 16 : (G <= 4 ? 8 : 4)); }
 
-// Context splits of a (sequence, kv head) pair. A launch lasts as long as the CU with the most workgroups -- a second one on a CU shares its vector
-// pipes, so 257 to 511 of them take twice what 256 take --, each of its workgroups costs what 250 tokens cost beside the tokens of its split, and the
-// merge what 300 do: the split count with the smallest such sum. Over batches of 1 to 28, contexts of 130 to 8000 tokens and two or four heads per kv
-// head (8 kv heads, bf16) it is within 4.7 % of the best of eleven counts measured, 0.2 % on average. Measured against a count of waves on the chip
-// (and a merge that took 0.6 us a split): two heads, 1 x 1300 tokens 14.9 -> 10.2 us, 6 x 1300 23.6 -> 14.1, 12 x 640 22.2 -> 16.1, 24 x 640 27.8 ->
-// 20.2, 20 x 2600 67 -> 54; four heads, 1 x 2600 17.0 -> 9.4, 10 x 1300 21.1 -> 17.2, 24 x 640 20.2 -> 17.1. 256 pairs or more are not split.
+// Context splits of a (sequence, kv head) pair. A launch lasts as long as the CU with the most workgroups, each of its workgroups costs what 250 tokens
+// cost beside the tokens of its split, and the merge what 400 do: the split count with the smallest such sum. Over batches of 1 to 31, contexts of 140 to
+// 8000 tokens and two or four heads per kv head (8 kv heads, bf16) it is 0.3 % from the best of eight counts on average. 256 pairs or more are not split.
 // Four-wave workgroups (the matrix-core kernel's, and eight heads per kv head without it) run best at about 2048 waves on the chip with 128 tokens or more per split (64 sequences x 8
 // kv heads x 2060 tokens at 8 heads per kv head 124 us in two splits + merge, 105 unsplit).
 int pick_splits(int64_t batch, int64_t nkv, int64_t max_context, int G, bool tr) {
@@ -1065,7 +1091,7 @@ int pick_splits(int64_t batch, int64_t nkv, int64_t max_context, int G, bool tr)
     if (pairs < 256) {
         int64_t least = 250 + max_context;
         for (int s = 2; s <= kMaxSplits && (int64_t)s * 64 <= max_context; ++s) {
-            const int64_t cost = cdiv(pairs * s, 256) * (250 + cdiv(max_context, s)) + 300;
+            const int64_t cost = cdiv(pairs * s, 256) * (250 + cdiv(max_context, s)) + 400;
             if (cost < least) least = cost, best = s;
         }
     }
@@ -1088,14 +1114,23 @@ void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* t
             return;
         }
     }
-    if constexpr (HD == 128 && (G == 4 || G == 8)) {
+    if constexpr (HD == 128 && (G == 2 || G == 4)) {
         if (bs % 16 == 0) {
-            paged_attn_decode_mfma_kernel<T, G, WAVES><<<dim3((unsigned)(batch * nkv * nsplit)), dim3(64 * WAVES), 0, st>>>(
-                (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv,
-                bs, max_blocks, num_blocks, nsplit, scale);
+            // a CU holds one workgroup of eight waves or, where there are more than CUs, several of four, whose last round is shorter (two heads, 40 x
+            // 640 tokens 23.9 us, 26.2 with eight; four heads, 64 x 640 29.5, 32.5; 24 x 640 14.9, 17.1 with four)
+            const int64_t groups = batch * nkv * nsplit;
+            const int full = groups * 4 >= cdiv(groups, 256) * 256 * 3;
+            const auto go = [&](auto waves) {
+                constexpr int W = decltype(waves)::value;
+                paged_attn_decode_mfma_kernel<T, G, W><<<dim3((unsigned)groups), dim3(64 * W), 0, st>>>(
+                    (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv, bs, max_blocks,
+                    num_blocks, nsplit, scale, tiled, full);
+            };
+            if (batch * nkv > 256) go(std::integral_constant<int, 4>{});
+            else go(std::integral_constant<int, 8>{});
             if (nsplit > 1)
                 paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(
-                    partial, (uint16_t*)out, nsplit, 0);
+                    partial, (uint16_t*)out, nsplit, tiled ? nkv * G : 0);
             return;
         }
     }

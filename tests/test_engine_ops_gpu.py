@@ -243,6 +243,42 @@ def test_paged_attention_split_counts(B, nh, nkv, bs, max_blocks):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,nh,nkv,bs,max_blocks", [
+    (33, 16, 8, 16, 9),           # four waves a workgroup, two heads per kv head; the smallest block
+    (33, 32, 8, 64, 3),           # four heads
+    (32, 16, 8, 64, 5),           # the cache past the L2, eight waves
+    (64, 32, 8, 64, 5),           # and four
+    (1, 8, 2, 16, 1100),          # 16 parts
+    (257, 2, 1, 32, 135),         # more than 64 tiles a wave: the block numbers are asked for again
+    (40, 4, 1, 48, 20),           # blocks that tiles of several waves share unevenly
+])
+def test_paged_attention_matrix_forms(dtype, B, nh, nkv, bs, max_blocks):
+    """Two and four heads per kv head: workgroups of four and eight waves, both ways to the cache, contexts from none to the whole table, rows and
+    blocks behind a context never read into a result.  Probabilities and sums are fp32, so what differs from the reference is the rounding of the result."""
+    from nanoquantization_amd.engine import ops
+    g = torch.Generator(device="cuda").manual_seed(B)
+    nb = B * max_blocks
+    kc = torch.randn(nb, nkv, bs, 128, generator=g, device="cuda").to(dtype)
+    vc = torch.randn(nb, nkv, bs, 128, generator=g, device="cuda").to(dtype)
+    q = torch.randn(B, nh, 128, generator=g, device="cuda").to(dtype)
+    table = torch.randperm(nb, generator=g, device="cuda").view(B, max_blocks).to(torch.int32)
+    ctx = torch.randint(1, bs * max_blocks + 1, (B,), generator=g, device="cuda").to(torch.int32)
+    ctx[0] = bs * max_blocks
+    if B > 2:
+        ctx[1], ctx[2] = 0, 17
+    at = torch.arange(max_blocks * bs, device="cuda").view(max_blocks, bs)
+    for b in range(B):
+        behind = (at >= ctx[b]).view(max_blocks, 1, bs, 1)
+        for cache in (kc, vc):
+            cache[table[b].long()] = cache[table[b].long()].masked_fill(behind, float("nan"))
+    out = ops.paged_attention_decode(q, kc, vc, table, ctx, 128 ** -0.5)
+    if B > 2:
+        assert not out[1].any()
+        out, q, table, ctx = (t[torch.arange(B, device="cuda") != 1] for t in (out, q, table, ctx))
+    _close(out, _attn_ref(q, kc, vc, table, ctx, 128 ** -0.5), dtype, scale=2.0, what="attention")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("nh,nkv,bs", [(16, 8, 32), (64, 8, 32), (16, 4, 32), (40, 8, 32), (64, 8, 16), (40, 8, 48)])
 def test_paged_attention_ignores_rows_past_the_context(dtype, nh, nkv, bs):
     """Cache rows past a sequence's context (and unused blocks) hold whatever was there before: NaNs planted there
