@@ -73,6 +73,12 @@ int awq_quantize_pack_flagged(const float* weight, int32_t* qweight, void* qscal
                               int64_t N, int64_t K, int64_t group_size, int dtype, int32_t* nan_flag,
                               void* stream);
 
+/* The same, and waits until it is done: `words` are two int32 in pinned host memory that the caller has zeroed, the first one the flag,
+ * the second set when the results are there. */
+int awq_quantize_pack_checked(const float* weight, int32_t* qweight, void* qscales, int32_t* qzeros,
+                              int64_t N, int64_t K, int64_t group_size, int dtype, int32_t* words,
+                              void* stream);
+
 /* y = x @ dequant(W) (+ bias) for many rows: the weight is dequantised into `scratch`, a slab of columns at a time
  * (the reference's own structure for 256 tokens and more, nanoquantization/layers/gemm.py:558-561), and multiplied by a dense
  * kernel of this library.  gated: W is gate and up interleaved word by word, y [M, N/2] = dtype(SiLU(gate)) * up,

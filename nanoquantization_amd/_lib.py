@@ -33,6 +33,7 @@ SYMBOLS = {
     "awq_dequantize": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "awq_dequantize_transposed": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
     "awq_quantize_pack": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp]),
+    "awq_quantize_pack_checked": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "awq_quantize_pack_flagged": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "awq_linear_dense_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "awq_linear_dense_wanted_bytes": (_sz, [_i64, _i64, _i64, _i64]),

@@ -58,14 +58,13 @@ def quantize_pack(weight: torch.Tensor, group_size: int, output_dtype: torch.dty
     qzeros = torch.empty(K // g, N // 8, dtype=torch.int32, device=dev)
     qscales = torch.empty(K // g, N, dtype=output_dtype, device=dev)
     # The kernel looks for NaN on its way: a pass of its own would read the whole weight twice more.  It writes its finding to
-    # pinned memory, which needs neither a launch to clear it nor a copy back (4096 x 12288 78 -> 73 us, 1024 x 2048 33 -> 29).
+    # pinned memory, which needs neither a launch to clear it nor a copy back (4096 x 12288 78 -> 73 us, 1024 x 2048 33 -> 29), and the call waits
+    # for it on a word of that memory, without torch's objects for device and stream (67 -> 60, 27.5 -> 20).
     # (the device is named: a default device of the caller's would put it elsewhere, where nothing can be pinned)
-    nan = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream()
-        _lib.check(_lib.lib().awq_quantize_pack_flagged(weight.data_ptr(), qweight.data_ptr(), qscales.data_ptr(),
+    words = torch.zeros(2, dtype=torch.int32, device="cpu", pin_memory=True)
+    with _lib.on_device(dev):
+        _lib.check(_lib.lib().awq_quantize_pack_checked(weight.data_ptr(), qweight.data_ptr(), qscales.data_ptr(),
                                                         qzeros.data_ptr(), N, K, g, _lib.dtype_id(output_dtype),
-                                                        nan.data_ptr(), stream.cuda_stream))
-        stream.synchronize()
-    assert not nan.item(), "weight should not contain nan"
+                                                        words.data_ptr(), _lib.current_stream_ptr(dev)))
+    assert not words[0].item(), "weight should not contain nan"
     return qweight, qscales, qzeros

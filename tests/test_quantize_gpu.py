@@ -96,3 +96,29 @@ def test_quantize_pack_under_a_default_device():
         with pytest.raises(AssertionError, match="nan"):
             nq.quantize_pack(torch.full((8, 128), float("nan"), device="cuda"), 128)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("nan", [False, True])
+def test_quantize_behind_queued_work(nan):
+    """Work in front of the kernel that lasts longer than the host looks for its word, on a stream of the caller's: the call then waits for the stream."""
+    import nanoquantization_amd as nq
+    w = torch.randn(256, 512, generator=torch.Generator().manual_seed(5)).cuda()
+    if nan:
+        w[17, 300] = float("nan")
+    torch.cuda.synchronize()
+    big = torch.ones(1 << 28, device="cuda")
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        for _ in range(20):             # 2 GiB each
+            big.mul_(1.0)
+        if nan:
+            with pytest.raises(AssertionError, match="nan"):
+                nq.quantize_pack(w, 128)
+        else:
+            got = nq.quantize_pack(w, 128)
+            assert stream.query(), "the call waits"
+    torch.cuda.synchronize()
+    if not nan:
+        for a, b in zip(got, nq.quantize_pack(w, 128)):
+            assert torch.equal(a, b)
