@@ -1066,9 +1066,17 @@ __global__ __launch_bounds__(64 * WK) void gemv_dma_kernel(
 // issue port, not the memory: per wave and 128 x 64 weights at 64 rows 80 MFMAs, which take it for 8 of their
 // 16 cycles, and 299 vector instructions at 4.7 (128 of them unpack, 128 apply scale and zero point); with the rest of the kernel
 // 71 to 80 % of the launch's cycles at 64 x 25600 x 5120, while waves wait for data or the barrier 22 % of their time.
-// At the end the two halves exchange fragments through LDS so that each stores whole words of half the rows.
+// A K split's sums leave as the fragments they are (sum_at; `fragments`), where the second pass is gemv_wide_add_kernel.  Otherwise the two
+// halves exchange fragments through LDS at the end so that each stores whole words of half the rows: some 700 vector instructions a wave, of 3800
+// with eight chunks, and two barriers (64 x 25600 x 5120 in 25 splits 34.9 us with the
+// exchange and rows, 32.3 with fragments; 12288 x 4096 at 32 / 64 rows 15.7 -> 14.8, 23.5 -> 21.1; from 17 rows on: up to 16 have no room for a whole row tile).
 // A K split leaves fp32 partials that a second kernel adds in split order -- or, TAIL (one m-tile, a few rows), the
 // last workgroup of the 512 columns to arrive, as in the one-tile kernel.
+// Where lane's four sums of fragment f of byte half bh lie: rows 16 * mt + 4 * (lane / 16) + 0..3, column 8 * (lane % 16) + 2 * f + bh of the tile.
+__host__ __device__ __forceinline__ size_t sums_of_split(int M, int N) { return (size_t)((M + 15) / 16 * 16) * N; }
+__device__ __forceinline__ size_t sum_at(int mt, int tile, int bh, int f, int lane, int N) {
+    return ((size_t)(mt * (N >> 7) + tile) * 8 + bh * 4 + f) * 256 + lane * 4;
+}
 __host__ __device__ constexpr int wide_buf_bytes(int MT, int WN = 4) { return 4096 * MT + WN * 8704; }
 
 template <typename T, int DEPTH, int MT, bool TAIL = false, int WN = 4>
@@ -1076,7 +1084,8 @@ __global__ __launch_bounds__(128 * WN) void gemv_wide_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ qweight,
     const uint16_t* __restrict__ scales, const uint32_t* __restrict__ qzeros,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, float* __restrict__ partials,
-    int* __restrict__ counters, int M, int N, int K, int chunks_per_group, int chunks_per_split, int splits, int act) {
+    int* __restrict__ counters, int M, int N, int K, int chunks_per_group, int chunks_per_split, int splits, int act,
+    int fragments) {
     // XP: pieces of x a wave brings per chunk (with one m-tile the four pieces go to waves 0..3, one each);
     // HMT: m-tiles each of the two byte-half waves of a column tile stores at the end
     constexpr int CH = 4, XP = MT >= 2 ? 4 * MT / (2 * WN) : 1, HMT = MT >= 2 ? MT / 2 : 1;
@@ -1347,6 +1356,15 @@ __global__ __launch_bounds__(128 * WN) void gemv_wide_kernel(
             }
             return;
         }
+        if (MT >= 2 && fragments) {
+            float* p = partials + (size_t)split * sums_of_split(M, N);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                if (16 * mt + 4 * kb < M)
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) *reinterpret_cast<f32x4*>(p + sum_at(mt, tile, BH, f, lane, N)) = acc[mt][f];
+            return;
+        }
         // Exchange: this wave stores m-tiles BH*HMT .. and sends its fragments of the other m-tiles to its
         // partner (wave ^ WN).  xch[wave][(ml*4 + f)*4 + r][lane]
         __syncthreads();   // staging is free
@@ -1380,6 +1398,38 @@ __global__ __launch_bounds__(128 * WN) void gemv_wide_kernel(
     else run(std::integral_constant<int, 1>{});
 }
 
+// Columns 4 * q .. 4 * q + 3 of row m to y.  Gated: the lane two further on has the gate columns' up columns; both call it.
+template <typename T>
+__device__ __forceinline__ void store_quad(const f32x4& sum, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int m, int N, int q,
+                                           bool valid, int act) {
+    float out[4] = {sum[0], sum[1], sum[2], sum[3]};
+    if (act) {
+        float up[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) up[c] = __shfl_xor(out[c], 2);
+        if (q & 2 || !valid) return;
+        uint32_t o[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float r[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) r[h] = silu_times_up<T>(out[2 * i + h], up[2 * i + h]);
+            o[i] = T::pack2(r[0], r[1]);
+        }
+        *reinterpret_cast<u32x2*>(y + (size_t)m * (N >> 1) + (size_t)(q >> 2) * 8 + (q & 1) * 4) = u32x2{o[0], o[1]};
+        return;
+    }
+    if (!valid) return;
+    const size_t n0 = (size_t)q * 4;
+    if (bias) {
+        const u32x2 bv = *reinterpret_cast<const u32x2*>(bias + n0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            out[c] = add_bias<T>(out[c], T::to_f32((uint16_t)((c & 1) ? (bv[c >> 1] >> 16) : (bv[c >> 1] & 0xFFFFu))));
+    }
+    *reinterpret_cast<u32x2*>(y + (size_t)m * N + n0) = u32x2{T::pack2(out[0], out[1]), T::pack2(out[2], out[3])};
+}
+
 // Second pass of a K-split wide GEMV: y = epilogue(sum over splits, in split order, of partials [splits][M][N]).
 // A thread owns four columns of one row; with the gated epilogue the neighbour of its neighbour holds the gate columns' up
 // columns.  Latency bounds it (the sums lie in the caches): SS splits' loads are in flight at a time, one round where they
@@ -1397,8 +1447,8 @@ __global__ __launch_bounds__(256) void gemv_wide_reduce_kernel(const float* __re
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= M * quads) return;   // N is a multiple of 16: gate columns and their up columns leave together
     const int m = idx / quads, q = idx - m * quads;
-    const size_t n0 = (size_t)q * 4, plane = (size_t)M * N;
-    const float* p = partials + (size_t)m * N + n0;
+    const size_t plane = (size_t)M * N;
+    const float* p = partials + (size_t)m * N + (size_t)q * 4;
     f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < splits; s0 += SS) {
         f32x4 a[SS];
@@ -1408,30 +1458,34 @@ __global__ __launch_bounds__(256) void gemv_wide_reduce_kernel(const float* __re
         for (int u = 0; u < SS; ++u)
             if (s0 + u < splits) sum += a[u];
     }
-    float out[4] = {sum[0], sum[1], sum[2], sum[3]};
-    if (act) {
-        float up[4];
+    store_quad<T>(sum, bias, y, m, N, q, true, act);
+}
+
+// The same for sums that lie as fragments: a wave adds four rows of eight words, a lane one column of them (16 bytes a split, as above), and takes
+// four columns of a row from there through LDS.
+template <typename T, int SS>
+__global__ __launch_bounds__(64) void gemv_wide_add_kernel(const float* __restrict__ partials, const uint16_t* __restrict__ bias,
+                                                           uint16_t* __restrict__ y, int M, int N, int splits, int act) {
+    constexpr int kPitch = 68;
+    __shared__ __align__(16) float s_sum[4 * kPitch];
+    const int halves = N >> 6, half = blockIdx.x % halves, rows4 = blockIdx.x / halves;
+    const int bh = threadIdx.x >> 5, f = threadIdx.x >> 3 & 3, j = threadIdx.x & 7;
+    const size_t plane = sums_of_split(M, N);
+    const float* p = partials + sum_at(rows4 >> 2, half >> 1, bh, f, (rows4 & 3) * 16 + (half & 1) * 8 + j, N);
+    f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < splits; s0 += SS) {
+        f32x4 a[SS];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) up[c] = __shfl_xor(out[c], 2);
-        if (q & 2) return;
-        uint32_t o[2];
+        for (int u = 0; u < SS; ++u) a[u] = *reinterpret_cast<const f32x4*>(p + (size_t)min(s0 + u, splits - 1) * plane);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            float r[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) r[h] = silu_times_up<T>(out[2 * i + h], up[2 * i + h]);
-            o[i] = T::pack2(r[0], r[1]);
-        }
-        *reinterpret_cast<u32x2*>(y + (size_t)m * (N >> 1) + (size_t)(q >> 2) * 8 + (q & 1) * 4) = u32x2{o[0], o[1]};
-        return;
+        for (int u = 0; u < SS; ++u)
+            if (s0 + u < splits) sum += a[u];
     }
-    if (bias) {
-        const u32x2 bv = *reinterpret_cast<const u32x2*>(bias + n0);
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            out[c] = add_bias<T>(out[c], T::to_f32((uint16_t)((c & 1) ? (bv[c >> 1] >> 16) : (bv[c >> 1] & 0xFFFFu))));
-    }
-    *reinterpret_cast<u32x2*>(y + (size_t)m * N + n0) = u32x2{T::pack2(out[0], out[1]), T::pack2(out[2], out[3])};
+    for (int r = 0; r < 4; ++r) s_sum[r * kPitch + 8 * j + 2 * f + bh] = sum[r];
+    __syncthreads();
+    const int row = threadIdx.x >> 4, q = threadIdx.x & 15, m = rows4 * 4 + row;
+    store_quad<T>(*reinterpret_cast<const f32x4*>(s_sum + row * kPitch + 4 * q), bias, y, m, N, half * 16 + q, m < M, act);
 }
 
 // The second pass and the residual add + RMSNorm that follows an o_proj or down_proj in one: a workgroup per row
@@ -1752,6 +1806,7 @@ static hipError_t launch_gemv_wide(const void* x, const int32_t* qweight, const 
     static_assert(lds <= 160 * 1024 - 1024, "staging buffers exceed the LDS");
     static_assert(!TAIL || lds >= 128 * WN * 128, "the tail stages 128 bytes per thread");
     if ((an || qe) && (splits == 1 || TAIL)) return hipErrorInvalidValue;   // their work is the second pass's
+    const bool fragments = MT >= 2 && M > 16 && splits > 1 && !an && !qe;
     auto kern = gemv_wide_kernel<T, DEPTH, MT, TAIL, WN>;
     static bool raised = false;  // once per process and instantiation
     if (!raised) {
@@ -1765,7 +1820,7 @@ static hipError_t launch_gemv_wide(const void* x, const int32_t* qweight, const 
                        reinterpret_cast<const uint16_t*>(x), reinterpret_cast<const uint32_t*>(qweight),
                        reinterpret_cast<const uint16_t*>(qscales), reinterpret_cast<const uint32_t*>(qzeros),
                        reinterpret_cast<const uint16_t*>(bias), reinterpret_cast<uint16_t*>(y), partials, counters,
-                       M, N, K, g / 128, cps, splits, act);
+                       M, N, K, g / 128, cps, splits, act, (int)fragments);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1 || TAIL) return e;
     if (qe) {
@@ -1776,6 +1831,12 @@ static hipError_t launch_gemv_wide(const void* x, const int32_t* qweight, const 
     if (an) {   // (checked by the caller: splits > 1, no tail, no bias, no gate, N <= 8192)
         hipLaunchKernelGGL(gemv_wide_reduce_add_rmsnorm_kernel<T>, dim3((unsigned)M), dim3(1024), 0, stream, partials,
                            reinterpret_cast<uint16_t*>(y), an->weight, an->normed, M, N, splits, an->eps);
+        return hipGetLastError();
+    }
+    if (fragments) {
+        const auto add = splits <= 8 ? gemv_wide_add_kernel<T, 8> : gemv_wide_add_kernel<T, 16>;
+        hipLaunchKernelGGL(add, dim3((unsigned)(cdiv(M, 4) * (N / 64))), dim3(64), 0, stream, partials, reinterpret_cast<const uint16_t*>(bias),
+                           reinterpret_cast<uint16_t*>(y), M, N, splits, act);
         return hipGetLastError();
     }
     const int threads = M * N % (1 << 19) == 0 ? 128 : 64;

@@ -255,6 +255,34 @@ def test_gemv_second_pass_rounds(M, split):
     _check(y, xb, p, "bf16", o.to_dtype_f32(bias, "bf16"))
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M", [16, 17, 20, 21, 32, 33, 47, 61, 64])
+def test_gemv_second_pass_of_fragments(dtype, M):
+    """From 17 rows on a split's sums lie as fragments of 16 rows: rows that end inside a fragment and inside its four, in every form with more than one
+    row tile, with a bias.  Memory behind the sums and the result stays as it was."""
+    K, N = 8 * 128, 1024
+    L = _lib.lib()
+    names = [L.awq_gemv_variant_name(i).decode() for i in range(L.awq_gemv_variant_count())]
+    p = random_packed(K, N, 128, dtype, seed=M)
+    xb = make_x(M, K, dtype, seed=M)
+    bias = np.linspace(-1, 1, N).astype(np.float32)
+    x, qw, qs, qz = to_dev(xb, dtype), to_dev(p["qweight"]), to_dev(p["qscales"], dtype), to_dev(p["qzeros"])
+    b = to_dev(o.to_bits16(bias, dtype), dtype)
+    forms = [n for n in names if n.startswith("wide") and n.endswith(("m2", "m4")) and M <= 16 * int(n[-1])]
+    assert forms, names
+    for name in forms:
+        for split in (2, 3, 8):
+            size = L.awq_gemv_ex_workspace_bytes(M, N, K, names.index(name), split)
+            ws = torch.zeros(size + 4096, dtype=torch.uint8, device="cuda")
+            ws[size:] = 77
+            y = torch.full((M + 1, N), 3.0, dtype=x.dtype, device="cuda")
+            print(f"gemv fragments {dtype} M={M} {name}/{split}", flush=True)
+            _lib.check(L.awq_gemv_ex(x.data_ptr(), qw.data_ptr(), qs.data_ptr(), qz.data_ptr(), b.data_ptr(), y.data_ptr(), M, N, K, 128,
+                                     _lib.dtype_id(x.dtype), ws.data_ptr(), size, torch.cuda.current_stream().cuda_stream, names.index(name), split))
+            assert (ws[size:] == 77).all() and (y[M] == 3).all()
+            _check(y[:M], xb, p, dtype, o.to_dtype_f32(bias, dtype))
+
+
 @pytest.mark.parametrize("M,N,split", [(64, 8192, 3), (32, 16384, 10)])
 def test_gemv_second_pass_of_sums_a_power_of_two_apart(M, N, split):
     """Sums of a split that are a multiple of 2 MiB go by workgroups of two waves; the whole result against the unsplit kernel's."""
