@@ -281,37 +281,74 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
     }
 }
 
+// The word of lane ^ O.
+template <int O>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t x) {
+    if constexpr (O == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false);        // row_ror:8
+    else if constexpr (O == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false);   // quad_perm:[2,3,0,1]
+    else if constexpr (O == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false);   // quad_perm:[1,0,3,2]
+    else if constexpr (O < 32) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, O << 10 | 0x1F);
+    else return (uint32_t)__shfl_xor((int)x, O);
+}
+template <int O>
+__device__ __forceinline__ float add_lanes(float v) {       // the sum over O + O lanes, xor O first
+    v += __builtin_bit_cast(float, lane_xor<O>(__builtin_bit_cast(uint32_t, v)));
+    if constexpr (O > 1) return add_lanes<O / 2>(v);
+    return v;
+}
+
 // RMSNorm of a head and half-split rotary: HD / 8 neighbouring lanes hold a head, lane dc of them the dims a[0..7] = 8 dc ..;
 // cs: cos | sin of the head's position.  The summation order and rounding points of the q|k|v GEMV's fused epilogue (head_dim
-// 128: tile_ssq), so that all routes give the same bits.
+// 128: tile_ssq), so that all routes give the same bits.  The vector ALU's work bounds the kernels around it, hence two values a word
+// where both are rounded or change lanes, and the sine's sign taken once: both halves are x cos + other sin, a
+// product and a fused multiply-add.
+template <typename T, int HD>
+struct Turn {
+    static constexpr int LPH = HD / 8, HALF = HD / 2;
+    float c[8], s[8];     // cos; -sin in the first half, sin in the second
+    __device__ __forceinline__ Turn(const float* __restrict__ cs, int dc) {
+        const int i0 = (dc % (LPH / 2)) * 8;   // index of this lane's first dim inside its half
+        const bool first = dc < LPH / 2;
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            const f32x4 cv = *reinterpret_cast<const f32x4*>(cs + i0 + e), sv = *reinterpret_cast<const f32x4*>(cs + HALF + i0 + e);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[e + i] = cv[i], s[e + i] = first ? -sv[i] : sv[i];
+        }
+    }
+    __device__ __forceinline__ u32x4 operator()(const float (&a)[8], u32x4 weight, float eps) const {
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(a[e], a[e], ss);
+        const float r = rsqrtf(add_lanes<LPH / 2>(ss) / (float)HD + eps);
+        float w[8], x[8], other[8];
+        unpack8<T>(weight, w);
+        u32x4 xn, turned;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            xn[i] = T::pack2(mul_round<T>(a[2 * i], r) * w[2 * i], mul_round<T>(a[2 * i + 1], r) * w[2 * i + 1]);
+        u32x4 across;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) across[i] = lane_xor<LPH / 2>(xn[i]);
+        unpack8<T>(xn, x);
+        unpack8<T>(across, other);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float y[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int e = 2 * i + h;
+                y[h] = as_f32_result(__builtin_fmaf(x[e], c[e], other[e] * s[e]));
+            }
+            turned[i] = T::pack2(y[0], y[1]);
+        }
+        return turned;
+    }
+};
 template <typename T, int HD>
 __device__ __forceinline__ u32x4 norm_rope(const float (&a)[8], const uint16_t* __restrict__ w, const float* __restrict__ cs,
                                            int dc, float eps) {
-    constexpr int LPH = HD / 8, HALF = HD / 2;
-    float wf[8];
-    unpack8<T>(*reinterpret_cast<const u32x4*>(w + dc * 8), wf);
-    const int i0 = (dc % (LPH / 2)) * 8;   // index of this lane's first dim inside its half
-    const f32x4 c0 = *reinterpret_cast<const f32x4*>(cs + i0), c1 = *reinterpret_cast<const f32x4*>(cs + i0 + 4);
-    const f32x4 s0 = *reinterpret_cast<const f32x4*>(cs + HALF + i0), s1 = *reinterpret_cast<const f32x4*>(cs + HALF + i0 + 4);
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(a[e], a[e], ss);
-#pragma unroll
-    for (int o = LPH / 2; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
-    const float r = rsqrtf(ss / (float)HD + eps);
-    float xn[8], y[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) xn[e] = round_to<T>(mul_round<T>(a[e], r) * wf[e]);
-    const bool first = dc < LPH / 2;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float other = __shfl_xor(xn[e], LPH / 2);
-        const float cc = e < 4 ? c0[e] : c1[e - 4], sn = e < 4 ? s0[e] : s1[e - 4];
-        const float x1 = first ? xn[e] : other, x2 = first ? other : xn[e];
-        y[e] = as_f32_result(first ? __fsub_rn(__fmul_rn(x1, cc), __fmul_rn(x2, sn))
-                                   : __fadd_rn(__fmul_rn(x1, sn), __fmul_rn(x2, cc)));
-    }
-    return pack8<T>(y);
+    return Turn<T, HD>(cs, dc)(a, *reinterpret_cast<const u32x4*>(w + dc * 8), eps);
 }
 
 // The same with 16-byte accesses, for head dims of 64, 128 or 256 and 16-byte aligned tensors (the scalar kernel
@@ -362,39 +399,61 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_vec_kernel(
 
 // The same for the outputs of separate q, k and v projections of `batch` sequences of `tokens` tokens: q stays [token][head],
 // k and v become [sequence][kv head][token], where the attention over the sequences reads a head's tokens in a row.
-// Bound by memory: 8192 tokens of 16 + 8 + 8 heads of 128 (134 MB) 37 us, 3.6 TB/s; as torch
+// A workgroup takes TOKENS tokens and HD / 8 of its lanes a head, two at a time: nothing is divided per lane, and the norm's weights and a token's
+// angles are read once for several heads.  Bound by memory and the vector ALU: 8192 tokens of 16 + 8 + 8
+// heads of 128 (134 MB) 31.5 us, 4.2 TB/s; with a head for every HD / 8 lanes of the launch, whose token and place four 64-bit divisions found, a lane
+// exchange and a rounding for every value and both halves' sums in every lane 43; 512 tokens 5.5 -> 5.2, 8 x 300 tokens of 48 heads 19.9 -> 17.4; as torch
 // operations, which pass over fp32 copies a dozen times, 560.
-template <typename T, int HD>
-__global__ __launch_bounds__(256) void qkv_norm_rope_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+template <typename T, int HD, int TOKENS>
+__global__ __launch_bounds__(512) void qkv_norm_rope_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                             const uint16_t* __restrict__ v, const uint16_t* __restrict__ q_weight,
                                                             const uint16_t* __restrict__ k_weight,
                                                             const float* __restrict__ cos_sin,
                                                             const int64_t* __restrict__ positions, bool per_sequence,
                                                             uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out,
-                                                            uint16_t* __restrict__ v_out, int64_t items, int tokens, int nh,
-                                                            int nkv, int64_t max_positions, float q_eps, float k_eps) {
-    constexpr int LPH = HD / 8, HPW = 64 / LPH;
-    const int heads = nh + 2 * nkv;
-    const int lane = threadIdx.x & 63, dc = lane % LPH;
-    int64_t item = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * HPW + lane / LPH;
-    const bool live = item < items;     // lanes past the end follow the last item (the shuffles need them) and store nothing
-    item = live ? item : items - 1;
-    const int64_t row = item / heads, seq = row / tokens;
-    const int h = (int)(item % heads), t = (int)(row % tokens);
-    const bool is_q = h < nh, is_k = !is_q && h < nh + nkv;
-    const int kv = is_k ? h - nh : h - nh - nkv;
-    const uint16_t* src = is_q ? q + (row * nh + h) * HD : (is_k ? k : v) + (row * nkv + kv) * HD;
-    const u32x4 raw = *reinterpret_cast<const u32x4*>(src + dc * 8);
-    float a[8];
-    unpack8<T>(raw, a);
-    int64_t pos = positions[per_sequence ? row : t];
-    pos += pos < 0 ? max_positions : 0;     // an index from the end, as the table's own indexing takes it
-    const bool known = pos >= 0 && pos < max_positions;     // no angles for any other: not a number, rather than a wrong turn
-    const u32x4 turned = norm_rope<T, HD>(a, is_q ? q_weight : k_weight, cos_sin + (known ? pos : 0) * HD, dc,
-                                          known ? (is_q ? q_eps : k_eps) : __builtin_nanf(""));
-    if (!live) return;
-    uint16_t* dst = is_q ? q_out + (row * nh + h) * HD : (is_k ? k_out : v_out) + ((seq * nkv + kv) * tokens + t) * HD;
-    *reinterpret_cast<u32x4*>(dst + dc * 8) = is_q || is_k ? turned : raw;
+                                                            uint16_t* __restrict__ v_out, int tokens, int nh, int nkv,
+                                                            int64_t max_positions, float q_eps, float k_eps) {
+    constexpr int LPH = HD / 8, U = 2;
+    const int heads = nh + 2 * nkv, groups = blockDim.x / LPH, group = threadIdx.x / LPH, dc = threadIdx.x % LPH;
+    const int64_t seq = blockIdx.y, row0 = seq * tokens;
+    for (int h0 = 0; h0 < heads; h0 += U * groups) {
+        const uint16_t* src[U];     // lanes past the last head follow it (the shuffles need them) and store nothing
+        uint16_t* dst[U];
+        int step[U], out_step[U];
+        u32x4 weight[U];
+        bool plain[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int h = min(h0 + u * groups + group, heads - 1), kv = h < nh + nkv ? h - nh : h - nh - nkv;
+            const bool is_q = h < nh;
+            plain[u] = h >= nh + nkv;
+            step[u] = (is_q ? nh : nkv) * HD;
+            src[u] = (is_q ? q + h * HD : (plain[u] ? v : k) + kv * HD) + row0 * step[u] + dc * 8;
+            out_step[u] = is_q ? nh * HD : HD;
+            dst[u] = (is_q ? q_out + row0 * step[u] + h * HD : (plain[u] ? v_out : k_out) + (seq * nkv + kv) * tokens * HD) + dc * 8;
+            weight[u] = *reinterpret_cast<const u32x4*>((is_q ? q_weight : k_weight) + dc * 8);
+        }
+#pragma unroll
+        for (int i = 0; i < TOKENS; ++i) {
+            const int t = min((int)blockIdx.x * TOKENS + i, tokens - 1);
+            u32x4 raw[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) raw[u] = *reinterpret_cast<const u32x4*>(src[u] + (int64_t)t * step[u]);
+            int64_t pos = positions[per_sequence ? row0 + t : t];
+            pos += pos < 0 ? max_positions : 0;     // an index from the end, as the table's own indexing takes it
+            const bool known = pos >= 0 && pos < max_positions;     // no angles for any other: not a number, rather than a wrong turn
+            const Turn<T, HD> turn(cos_sin + (known ? pos : 0) * HD, dc);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int h = h0 + u * groups + group;
+                float a[8];
+                unpack8<T>(raw[u], a);
+                const u32x4 turned = turn(a, weight[u], known ? (h < nh ? q_eps : k_eps) : __builtin_nanf(""));
+                if (h < heads && (int)blockIdx.x * TOKENS + i < tokens)
+                    *reinterpret_cast<u32x4*>(dst[u] + (int64_t)t * out_step[u]) = plain[u] ? raw[u] : turned;
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1495,25 +1554,34 @@ extern "C" int nq_qkv_norm_rope(const void* q, const void* k, const void* v, con
         set_error("%s: head_dim must be 64, 128 or 256, got %lld", fn, (long long)head_dim);
         return AWQ_ERR_UNSUPPORTED;
     }
-    const int64_t items = batch * tokens * (num_heads + 2 * num_kv_heads), groups = cdiv(items, 4 * (512 / head_dim));
-    if (groups > 0x7fffffff) return bad(fn, "problem too large");
+    const int64_t items = batch * tokens * (num_heads + 2 * num_kv_heads);
+    if (cdiv(items, 4 * (512 / head_dim)) > 0x7fffffff) return bad(fn, "problem too large");
+    // two heads a group of lanes and pass, passes of up to 512 lanes equally full
+    const int64_t each = head_dim / 8, pairs = cdiv(num_heads + 2 * num_kv_heads, 2), passes = cdiv(pairs * each, 512);
+    const int64_t lanes = cdiv(cdiv(pairs, passes) * each, 64) * 64;
     hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();
-#define NQ_GO(TT, HH)                                                                                                     \
-    qkv_norm_rope_kernel<TT, HH><<<dim3((unsigned)groups), dim3(256), 0, st>>>(                                            \
-        (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_weight, (const uint16_t*)k_weight,  \
-        cos_sin, positions, per_sequence != 0, (uint16_t*)q_out, (uint16_t*)k_out, (uint16_t*)v_out, items, (int)tokens,   \
-        (int)num_heads, (int)num_kv_heads, max_positions, q_eps, k_eps)
-    if (dtype == AWQ_F16) {
-        if (head_dim == 64) NQ_GO(F16, 64);
-        else if (head_dim == 128) NQ_GO(F16, 128);
-        else NQ_GO(F16, 256);
-    } else {
-        if (head_dim == 64) NQ_GO(BF16, 64);
-        else if (head_dim == 128) NQ_GO(BF16, 128);
-        else NQ_GO(BF16, 256);
-    }
-#undef NQ_GO
+    const auto go = [&](auto type, auto dim, auto each) {
+        using T = decltype(type);
+        constexpr int HD = decltype(dim)::value, TOKENS = decltype(each)::value;
+        for (int64_t b = 0; b < batch; b += 65535) {     // the grid's second dimension
+            const int64_t some = std::min<int64_t>(batch - b, 65535), r = b * tokens;
+            const auto at = [&](const void* x, int64_t heads) { return (uint16_t*)x + r * heads * HD; };
+            qkv_norm_rope_kernel<T, HD, TOKENS><<<dim3((unsigned)cdiv(tokens, TOKENS), (unsigned)some), dim3((unsigned)lanes), 0, st>>>(
+                at(q, num_heads), at(k, num_kv_heads), at(v, num_kv_heads), (const uint16_t*)q_weight, (const uint16_t*)k_weight, cos_sin,
+                positions + (per_sequence ? r : 0), per_sequence != 0, at(q_out, num_heads), at(k_out, num_kv_heads), at(v_out, num_kv_heads),
+                (int)tokens, (int)num_heads, (int)num_kv_heads, max_positions, q_eps, k_eps);
+        }
+    };
+    const auto of = [&](auto type, auto each) {
+        if (head_dim == 64) go(type, std::integral_constant<int, 64>{}, each);
+        else if (head_dim == 128) go(type, std::integral_constant<int, 128>{}, each);
+        else go(type, std::integral_constant<int, 256>{}, each);
+    };
+    const auto with = [&](auto each) { dtype == AWQ_F16 ? of(F16{}, each) : of(BF16{}, each); };
+    // several tokens a workgroup where the chip has more waves than it holds at a time all the same
+    if (cdiv(batch * tokens, 4) * (lanes / 64) >= 8192) with(std::integral_constant<int, 4>{});
+    else with(std::integral_constant<int, 1>{});
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
 }

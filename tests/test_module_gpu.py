@@ -269,3 +269,36 @@ def test_prompt_forward_of_many_tiles(monkeypatch):
         _eager(monkeypatch)
         want = m(ids, pos)
     assert (got.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("batch,tokens,heads,kv,dim", [
+    (1, 1, 1, 1, 128),            # fewer heads than a wave has lanes for
+    (3, 5, 16, 8, 128),
+    (2, 4099, 24, 8, 128),        # four tokens a workgroup, the last one with three
+    (5, 3301, 5, 1, 64),          # an odd head count
+    (2, 2050, 40, 8, 256),        # several passes over the heads
+])
+def test_qkv_norm_rope_sizes(dtype, batch, tokens, heads, kv, dim):
+    """Head counts and tokens around the kernel's groups, passes and tokens a workgroup, positions per sequence, against the torch expressions in fp32 with
+    the module's roundings: the norm and its product with the weight are rounded to the type, the rotary sums only at the end."""
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    randn = lambda *n: torch.randn(*n, generator=g, device="cuda")
+    q, k, v = (randn(batch, tokens, n * dim).to(dtype) for n in (heads, kv, kv))
+    weights = [(1 + 0.1 * randn(dim)).to(dtype) for _ in range(2)]
+    angles = randn(64, dim // 2)
+    table = torch.cat([angles.cos(), angles.sin()], dim=-1).unsqueeze(1)
+    pos = torch.randint(-64, 64, (batch, tokens), generator=g, device="cuda")
+    got = torch.ops.nanoquantization_amd.qkv_norm_rope(q, k, v, *weights, table, pos, heads, kv, 1e-6, 1e-5)
+    cos, sin = table[pos].chunk(2, dim=-1)
+    for x, w, eps, n, out in ((q, weights[0], 1e-6, heads, got[0]), (k, weights[1], 1e-5, kv, got[1])):
+        x = x.view(batch, tokens, n, dim).float()
+        x = (x * torch.rsqrt(x.square().mean(-1, keepdim=True) + eps)).to(dtype) * w
+        a, b = x.float().chunk(2, dim=-1)
+        want = torch.cat([a * cos - b * sin, a * sin + b * cos], dim=-1)
+        size = torch.cat([(a * cos).abs() + (b * sin).abs(), (a * sin).abs() + (b * cos).abs()], dim=-1)
+        out = out if n == heads and out.shape == want.shape else out.view(batch, n, tokens, dim).transpose(1, 2)
+        # fp32 sums in another order may move x * r over a rounding's edge: one place (eps of its value at most), carried into the product with
+        # the weight, whose own two roundings are half a place away each: 2 eps a term, and half of one for the result's rounding
+        assert ((out.view_as(want).float() - want).abs() <= 2.5 * torch.finfo(dtype).eps * size + 1e-6).all()
+    assert torch.equal(got[2].view(batch, kv, tokens, dim).transpose(1, 2), v.view(batch, tokens, kv, dim))
