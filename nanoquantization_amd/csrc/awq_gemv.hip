@@ -1985,20 +1985,30 @@ static int64_t pick_one_m_tile(int64_t M, int64_t N, int64_t K, int64_t chunks, 
 // 8192 x 5120 at 64 rows 23.5 -> 22.3 us, at 48 rows 19.2 against 21.7), 3584 columns and K = 3584 on (2560 x 19456 at
 // 40 rows 23.4 us against 19.1 in row blocks), any N; plan B with up to 11 chunks a split (with 16, 4096 x 28672
 // runs 38.6 us in 224 workgroups and 36.9 in 448 of 8 chunks; 25600 x 5120 at 40 rows 37.6 us in 12 splits of 17
-// chunks, 33.7 in 25 of 8; 17408 x 5120 at 40 rows 29.8 us in 12 splits of 12, 27.7 in 23 of 6).  Against the
+// chunks, 33.7 in 25 of 8, at 64 rows 40.6 in 12, 38.8 in 20 and 41.0 in 25, from the cache 33.7 in 20 and 33.2 in 25; 17408 x 5120 at
+// 40 rows 29.4 us in 12 splits of 12, 27.8 in 23 of 6).  Against the
 // 512-column form or the one-tile kernel's row blocks at 64 rows: 8192 x 8192 30.4 -> 26.1 us, 5120 x 10240 27.8 ->
 // 23.7, 13824 x 5120 31.4 -> 27.2, 18944 x 3584 31.6 -> 27.7, 8192 x 10240 33.8 -> 29.9, 4096 x 12288 25.9 -> 23.5,
 // 5120 x 17408 34.1 -> 32.5, 4096 x 28672 39.6 -> 36.9, 5120 x 25600 40.8 -> 39.1, 5120 x 51200 70.7 -> 65.6; at 40
 // and 48 rows equal to 10 % faster (12288 x 4096 at 48 rows 25.0 -> 21.5); 4096 x 8192 and 5120 x 8192 keep the row
 // blocks (17.2 and 19.9 against 22.5 and 21.8).
+// 2304 to 3840 columns are too few column tiles for the one-tile kernel: at 17 to 64 rows it splits K five times and more and pays for a tail per row.
+// From 56 chunks on they go with the shared chunk as well, one workgroup per CU as far as splits of four chunks give, above 32 rows where K is 2.4
+// times N, above 32 and up to 48 from 25 M weights on (in fp16, where the one-tile kernel is faster, 9728 x 2560 at 40 rows 15.9 / 16.2; one-tile kernel / shared chunk at 17, 32, 40, 64 rows: 9728 x 2560 14.6, 15.9, 17.3, 21.1 / 12.2, 13.6, 16.7, 18.4; 12288 x 3072 16.5,
+// 17.8, 22.7, 25.0 / 13.6, 14.7, 17.7, 19.0; 16384 x 2304 17.5, 19.4, 23.7, 28.8 / 13.5, 14.1, 17.2, 18.9; 7168 x 3584 12.8, 13.2, 16.1, 16.3 / 11.6, 12.9, 16.2, 18.6).
 static int64_t pick_shared_256(int64_t M, int64_t N, int64_t K, int64_t chunks, int* variant) {
     if (M > 64 || N % 256 != 0 || chunks < 8) return 0;
     const bool four = M > 32;   // m-tiles: four, else two
+    const bool narrow = N >= 2304 && N < 4096 && chunks >= 56 && (!four || (5 * K >= 12 * N && (M > 48 || K * N >= 25000000ll)));
+    auto normalised = [&](int64_t c) { return cdiv(chunks, cdiv(chunks, c)); };
+    const int64_t groups = N / 256;
+    if (narrow) {
+        *variant = four ? kWide2D2M4 : kWide2D2M2;
+        return normalised(std::min(256 / groups, chunks / 4));
+    }
     if (four ? (N < 3584 || chunks < 28 || K * N < (M > 48 ? 40000000ll : 45000000ll))
              : (N < 4096 || N >= 28672 || K * N < 48000000ll))
         return 0;
-    auto normalised = [&](int64_t c) { return cdiv(chunks, cdiv(chunks, c)); };
-    const int64_t groups = N / 256;
     int64_t sb = 256 / groups;
     if (sb > chunks / 4) sb = chunks / 4;
     if (sb >= 2 && normalised(sb) * groups >= (four ? 216 : 218) && (!four || cdiv(chunks, sb) <= 11)) {

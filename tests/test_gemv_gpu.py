@@ -255,6 +255,25 @@ def test_gemv_second_pass_rounds(M, split):
     _check(y, xb, p, "bf16", o.to_dtype_f32(bias, "bf16"))
 
 
+@pytest.mark.parametrize("M,K,N,plan", [(17, 7168, 2304, "wide2d2m2/14"), (32, 16384, 2304, "wide2d2m2/26"), (20, 7168, 3840, "wide2d2m2/14"),
+                                        (64, 9728, 2560, "wide2d2m4/19"), (33, 12288, 3072, "wide2d2m4/20"), (64, 7168, 3584, None),
+                                        (16, 9728, 2560, None), (24, 7040, 2560, None), (24, 9728, 2432, None), (40, 9728, 2560, None)])
+def test_gemv_few_column_tiles(M, K, N, plan):
+    """17 to 64 rows of 2304 to 3840 columns and long K on the shared chunk, and what lies beside that; None: another kernel."""
+    import ctypes
+    L = _lib.lib()
+    names = [L.awq_gemv_variant_name(i).decode() for i in range(L.awq_gemv_variant_count())]
+    v, sp = ctypes.c_int(), ctypes.c_int()
+    assert L.awq_gemv_plan(M, N, K, 128, ctypes.byref(v), ctypes.byref(sp)) == 0
+    assert f"{names[v.value]}/{sp.value}" == plan if plan else not names[v.value].startswith("wide2d2m2") and names[v.value] != "wide2d2m4", names[v.value]
+    if K * N > 40_000_000:
+        return                        # (by its plan alone)
+    p = random_packed(K, N, 128, "bf16", seed=M)
+    xb = make_x(M, K, "bf16", seed=M)
+    y = nq.awq_gemm(to_dev(xb, "bf16"), to_dev(p["qweight"]), to_dev(p["qscales"], "bf16"), to_dev(p["qzeros"]), 8)
+    _check(y, xb, p, "bf16")
+
+
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("M", [16, 17, 20, 21, 32, 33, 47, 61, 64])
 def test_gemv_second_pass_of_fragments(dtype, M):
