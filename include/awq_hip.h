@@ -93,6 +93,12 @@ size_t awq_linear_dense_wanted_bytes(int64_t M, int64_t N, int64_t K, int64_t gr
 int awq_linear_dense(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
                      const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
                      int gated, void* scratch, size_t scratch_bytes, void* stream);
+/* y = residual + x @ dequant(W) with the product rounded to dtype first, as a separate addition would have it; residual [M, N] may be y.  Scratch
+ * as of awq_linear_dense. */
+int awq_linear_dense_add(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
+                         const void* residual, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
+                         void* scratch, size_t scratch_bytes, void* stream);
+
 /* y [M, N] = dtype(SiLU(x @ gate)) * (x @ up) for two weights [K, N] that lie apart: both are dequantised into `scratch` in one
  * pass, interleaved, and multiplied as by awq_linear_dense with `gated`.  Scratch (and whether this is the fastest way): as for
  * awq_linear_dense with 2 N columns. */

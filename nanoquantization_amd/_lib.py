@@ -40,6 +40,7 @@ SYMBOLS = {
     "awq_linear_scratch_bytes": (_sz, [_i64, _i64, _i64, _i64, _int]),
     "awq_linear_route": (ctypes.c_char_p, [_i64] * 4 + [_int, _int, ctypes.POINTER(_int)]),
     "awq_linear_dense": (_int, [_vp] * 6 + [_i64] * 4 + [_int, _int, _vp, _sz, _vp]),
+    "awq_linear_dense_add": (_int, [_vp] * 6 + [_i64] * 4 + [_int, _vp, _sz, _vp]),
     "awq_linear_dense_pair": (_int, [_vp] * 8 + [_i64] * 4 + [_int, _vp, _sz, _vp]),
     "awq_linear_parts_wanted": (_sz, [_vp, _int, _i64, _i64, _i64, _int, _vp, _vp]),
     "awq_linear_parts": (_int, [_vp] * 6 + [_int, _i64, _i64, _i64, _int, _vp, _sz, _vp, _sz, _vp]),

@@ -29,10 +29,13 @@ struct Outputs {
 
 // GATED: the slab's columns are gate and up words in turn; a tile is 128 gate columns and their up columns, a wave's first
 // tiles gate, the others up.
-template <typename T, int XR, bool GATED>
+// ADD: y = residual + dtype(product), rounded once more, as a separate addition leaves it; residual lies as y does.  Its rows are asked for in
+// front of the product (256-row tiles have no registers left for that: behind it), and the addition's own pass over three tensors is gone: 8192 x
+// 1024 of K 2048 / 3072 with a pass of its own 50.6 / 62.1 us, so 43.0 / 56.1; 8192 x 2560 of K 4096 198 and 180.
+template <typename T, int XR, bool GATED, bool ADD>
 __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wt,
-                                                       const uint16_t* __restrict__ bias, Outputs out, int M, int cols, int K,
-                                                       int x_tiles, int w_tiles) {
+                                                       const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual,
+                                                       Outputs out, int M, int cols, int K, int x_tiles, int w_tiles) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
     using P = PingPong<T, XR>;
     int xt, nt;
@@ -60,13 +63,40 @@ __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restric
     const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wt), 0, cols * row_bytes, 0x00020000);
     const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x) + (size_t)m0 * K, 0,
                                                       rows * row_bytes, 0x00020000);
+    u32x4 old[ADD ? P::kStores : 1];
+    const auto ask = [&] {
+        const auto ro = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(residual) + (size_t)m0 * out.ldy[0] + n0, 0,
+                                                          (uint32_t)((rows - 1) * out.ldy[0] + min(256, cols - n0)) * 2, 0x00020000);
+#pragma unroll
+        for (int n = 0; n < P::kStores; ++n)        // past the tile's end: zero, or the next row's
+            old[n] = __builtin_amdgcn_raw_buffer_load_b128(ro, (uint32_t)(P::store_row(n) * out.ldy[0] + P::store_column()) * 2, 0, 0);
+    };
+    if constexpr (ADD && XR == 128) ask();
     p.run(s_mem, rw, vw, rx, vx, K / P::kStage);
+    if constexpr (ADD && XR != 128) ask();
     const int part = (n0 >= out.first[1]) + (n0 >= out.first[2]), ldy = pick_part(out.ldy, part);
     uint16_t* __restrict__ y = pick_part(out.y, part) + (n0 - pick_part(out.first, part));
     const auto store = [&](int r, int c, u32x4 v) {
         if (m0 + r < M && n0 + c < out_cols) *reinterpret_cast<u32x4*>(y + (size_t)(m0 + r) * ldy + c) = v;
     };
-    if constexpr (GATED) {
+    if constexpr (ADD) {
+        p.template to_lds<256>(s_mem, [&](int i, int j) {
+            const f32x4 v = p.acc[i][j];
+            return u32x2{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
+        });
+#pragma unroll
+        for (int n = 0; n < P::kStores; ++n) {
+            const int row = P::store_row(n), c = P::store_column();
+            const u32x4 v = p.template stored<256>(s_mem, row, c);
+            u32x4 sum;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const auto half = [&](uint32_t w, int h) { return T::to_f32((uint16_t)(w >> (16 * h))); };
+                sum[i] = T::pack2(half(old[n][i], 0) + half(v[i], 0), half(old[n][i], 1) + half(v[i], 1));
+            }
+            store(row, c, sum);
+        }
+    } else if constexpr (GATED) {
         p.template write<128>(s_mem, [&](int i, int j) {
             const f32x4 g4 = p.acc[i][j], u4 = p.acc[i + P::MI / 2][j];
             float o[4];
@@ -120,10 +150,10 @@ double rounds_us(int64_t M, int64_t slab, int64_t K) {
     return (double)full * (steps * (xr == 256 ? 1.25 : 0.76) + ends) + (part > 0 ? steps * stage + ends : 0);
 }
 
-template <typename T, int XR, bool GATED>
-hipError_t launch(const void* x, const void* wt, const void* bias, const Outputs& out, int M, int cols, int K, hipStream_t st) {
+template <typename T, int XR, bool GATED, bool ADD = false>
+hipError_t launch(const void* x, const void* wt, const void* bias, const void* residual, const Outputs& out, int M, int cols, int K, hipStream_t st) {
     using P = PingPong<T, XR>;
-    auto kern = dense_kernel<T, XR, GATED>;
+    auto kern = dense_kernel<T, XR, GATED, ADD>;
     static bool raised = false;      // once per process and instantiation
     if (!raised) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -134,16 +164,20 @@ hipError_t launch(const void* x, const void* wt, const void* bias, const Outputs
     const int x_tiles = (int)cdiv(M, XR), w_tiles = (int)cdiv(cols, 256);
     (void)hipGetLastError();
     kern<<<dim3((unsigned)(cdiv((int64_t)x_tiles * w_tiles, 8) * 8)), dim3(P::kThreads), P::kLds, st>>>(
-        (const uint16_t*)x, (const uint16_t*)wt, (const uint16_t*)bias, out, M, cols, K, x_tiles, w_tiles);
+        (const uint16_t*)x, (const uint16_t*)wt, (const uint16_t*)bias, (const uint16_t*)residual, out, M, cols, K, x_tiles, w_tiles);
     return hipGetLastError();
 }
 
 template <typename T>
-hipError_t launch_dense(const void* x, const void* wt, const void* bias, const Outputs& out, int M, int cols, int K, int xr,
-                        bool gated, hipStream_t st) {
-    if (xr == 256)
-        return gated ? launch<T, 256, true>(x, wt, bias, out, M, cols, K, st) : launch<T, 256, false>(x, wt, bias, out, M, cols, K, st);
-    return gated ? launch<T, 128, true>(x, wt, bias, out, M, cols, K, st) : launch<T, 128, false>(x, wt, bias, out, M, cols, K, st);
+hipError_t launch_dense(const void* x, const void* wt, const void* bias, const void* residual, const Outputs& out, int M, int cols, int K,
+                        int xr, bool gated, hipStream_t st) {
+    const auto go = [&](auto rows) {
+        constexpr int XR = decltype(rows)::value;
+        return residual ? launch<T, XR, false, true>(x, wt, nullptr, residual, out, M, cols, K, st)
+               : gated  ? launch<T, XR, true>(x, wt, bias, nullptr, out, M, cols, K, st)
+                        : launch<T, XR, false>(x, wt, bias, nullptr, out, M, cols, K, st);
+    };
+    return xr == 256 ? go(std::integral_constant<int, 256>{}) : go(std::integral_constant<int, 128>{});
 }
 
 // Sizes and group sizes the path takes; 32-bit offsets inside a tile's rows of x and inside a slab.
@@ -183,8 +217,8 @@ int dense_parts(const char* fn, const void* x, const Parts& parts, int64_t M, in
     const int xr = product_tile(M, parts.total, K);
     hipError_t e = launch_dequant_transpose_parts(dtype, parts, scratch, (int)K, (int)g, st);
     if (e == hipSuccess)
-        e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, nullptr, Outputs(parts), (int)M, parts.total, (int)K, xr, false, st)
-                             : launch_dense<BF16>(x, scratch, nullptr, Outputs(parts), (int)M, parts.total, (int)K, xr, false, st);
+        e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, nullptr, nullptr, Outputs(parts), (int)M, parts.total, (int)K, xr, false, st)
+                             : launch_dense<BF16>(x, scratch, nullptr, nullptr, Outputs(parts), (int)M, parts.total, (int)K, xr, false, st);
     return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
 }
 
@@ -197,8 +231,8 @@ extern "C" size_t awq_linear_dense_scratch_bytes(int64_t M, int64_t N, int64_t K
 }
 
 // `second`: the up weight beside `w`, the gate weight, N columns of each.
-static int dense_entry(const char* fn, const void* x, const PackedWeight& w, const PackedWeight* second, const void* bias, void* y,
-                       int64_t M, int64_t N, int64_t K, int64_t g, int dtype, bool gated, void* scratch, size_t scratch_bytes,
+static int dense_entry(const char* fn, const void* x, const PackedWeight& w, const PackedWeight* second, const void* bias, const void* residual,
+                       void* y, int64_t M, int64_t N, int64_t K, int64_t g, int dtype, bool gated, void* scratch, size_t scratch_bytes,
                        void* stream) {
     const int64_t cols_in_all = second ? 2 * N : N;
     if (!takes(M, cols_in_all, K, g) || (gated && (bias || cols_in_all % 16 != 0))) {
@@ -206,8 +240,8 @@ static int dense_entry(const char* fn, const void* x, const PackedWeight& w, con
                   "and no bias (M=%lld N=%lld K=%lld g=%lld)", fn, (long long)M, (long long)N, (long long)K, (long long)g);
         return AWQ_ERR_UNSUPPORTED;
     }
-    if ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(scratch)) & 15u) {
-        set_error("%s: bias and scratch must be 16-byte aligned", fn);
+    if ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(scratch) | reinterpret_cast<uintptr_t>(residual)) & 15u) {
+        set_error("%s: bias, residual and scratch must be 16-byte aligned", fn);
         return AWQ_ERR_INVALID_ARG;
     }
     const size_t need = awq_linear_dense_scratch_bytes(M, cols_in_all, K, g);
@@ -222,10 +256,11 @@ static int dense_entry(const char* fn, const void* x, const PackedWeight& w, con
         const int64_t cols = std::min(slab, cols_in_all - n), each = second ? 2 : 1;
         hipError_t e = launch_dequant_transpose(dtype, w, second, scratch, (int)N, (int)K, (int)g, st, n / each, cols / each);
         const void* b = bias ? static_cast<const uint16_t*>(bias) + n : nullptr;
+        const void* res = residual ? static_cast<const uint16_t*>(residual) + n : nullptr;
         const Outputs out(static_cast<uint16_t*>(y) + (gated ? n / 2 : n), (int)(gated ? cols_in_all / 2 : N));
         if (e == hipSuccess)
-            e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, b, out, (int)M, (int)cols, (int)K, xr, gated, st)
-                                 : launch_dense<BF16>(x, scratch, b, out, (int)M, (int)cols, (int)K, xr, gated, st);
+            e = dtype == AWQ_F16 ? launch_dense<F16>(x, scratch, b, res, out, (int)M, (int)cols, (int)K, xr, gated, st)
+                                 : launch_dense<BF16>(x, scratch, b, res, out, (int)M, (int)cols, (int)K, xr, gated, st);
         if (e != hipSuccess) return hip_fail(fn, e);
     }
     return AWQ_OK;
@@ -239,7 +274,27 @@ extern "C" int awq_linear_dense(const void* x, const int32_t* qweight, const voi
     take_prefetch_hint(&dropped);
     const int rc = check_linear_args(fn, x, qweight, qscales, qzeros, y, M, N, K, group_size, dtype);
     if (rc != AWQ_OK) return rc;
-    return dense_entry(fn, x, {qweight, qscales, qzeros}, nullptr, bias, y, M, N, K, group_size, dtype, gated != 0, scratch,
+    return dense_entry(fn, x, {qweight, qscales, qzeros}, nullptr, bias, nullptr, y, M, N, K, group_size, dtype, gated != 0, scratch,
+                       scratch_bytes, stream);
+}
+
+extern "C" int awq_linear_dense_add(const void* x, const int32_t* qweight, const void* qscales, const int32_t* qzeros,
+                                    const void* residual, void* y, int64_t M, int64_t N, int64_t K, int64_t group_size, int dtype,
+                                    void* scratch, size_t scratch_bytes, void* stream) {
+    const char* fn = "awq_linear_dense_add";
+    PrefetchRegions dropped;
+    take_prefetch_hint(&dropped);
+    const int rc = check_linear_args(fn, x, qweight, qscales, qzeros, y, M, N, K, group_size, dtype);
+    if (rc != AWQ_OK) return rc;
+    if (!residual) {
+        set_error("%s: null pointer argument", fn);
+        return AWQ_ERR_INVALID_ARG;
+    }
+    if (N > (1 << 22)) {        // a tile's rows of the residual lie within 32-bit offsets
+        set_error("%s: too many columns", fn);
+        return AWQ_ERR_UNSUPPORTED;
+    }
+    return dense_entry(fn, x, {qweight, qscales, qzeros}, nullptr, nullptr, residual, y, M, N, K, group_size, dtype, false, scratch,
                        scratch_bytes, stream);
 }
 
@@ -254,6 +309,6 @@ extern "C" int awq_linear_dense_pair(const void* x, const int32_t* gate_qweight,
     if (rc == AWQ_OK) rc = check_linear_args(fn, x, up_qweight, up_qscales, up_qzeros, y, M, N, K, group_size, dtype);
     if (rc != AWQ_OK) return rc;
     const PackedWeight up(up_qweight, up_qscales, up_qzeros);
-    return dense_entry(fn, x, {gate_qweight, gate_qscales, gate_qzeros}, &up, nullptr, y, M, N, K, group_size, dtype, true, scratch,
+    return dense_entry(fn, x, {gate_qweight, gate_qscales, gate_qzeros}, &up, nullptr, nullptr, y, M, N, K, group_size, dtype, true, scratch,
                        scratch_bytes, stream);
 }

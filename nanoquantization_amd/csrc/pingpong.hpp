@@ -203,6 +203,15 @@ struct PingPong {
     // columns (two words) of tile pair (i, j), i < COLS / 16 / kWM; store(row, column, eight values) writes 16 bytes of a row.
     template <int COLS, typename V, typename S>
     __device__ __forceinline__ void write(unsigned char* s_mem, V&& value, S&& store) {
+        to_lds<COLS>(s_mem, value);
+#pragma unroll 4
+        for (int q = threadIdx.x; q < XR * COLS / 8; q += kThreads) {
+            const int r = q / (COLS / 8), c = q % (COLS / 8) * 8;
+            store(r, c, stored<COLS>(s_mem, r, c));
+        }
+    }
+    template <int COLS, typename V>
+    __device__ __forceinline__ void to_lds(unsigned char* s_mem, V&& value) {
         constexpr int kTiles = COLS / 16 / kWM, kBytes = COLS * 2;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
@@ -212,12 +221,16 @@ struct PingPong {
                 *reinterpret_cast<u32x2*>(s_mem + r * kBytes + ((c * 2) ^ ((r & 15) << 4))) = value(i, j);
             }
         __syncthreads();
-#pragma unroll 4
-        for (int q = threadIdx.x; q < XR * COLS / 8; q += kThreads) {
-            const int r = q / (COLS / 8), c = q % (COLS / 8) * 8;
-            store(r, c, *reinterpret_cast<const u32x4*>(s_mem + r * kBytes + ((c * 2) ^ ((r & 15) << 4))));
-        }
     }
+    template <int COLS>
+    static __device__ __forceinline__ u32x4 stored(const unsigned char* s_mem, int r, int c) {
+        return *reinterpret_cast<const u32x4*>(s_mem + r * COLS * 2 + ((c * 2) ^ ((r & 15) << 4)));
+    }
+
+    // Eight values a thread and store of `write<256>`: how many, and which store n of this thread is.
+    static constexpr int kStores = XR * 32 / kThreads;
+    static __device__ __forceinline__ int store_row(int n) { return (threadIdx.x + n * kThreads) >> 5; }
+    static __device__ __forceinline__ int store_column() { return (threadIdx.x & 31) * 8; }
 };
 
 // Workgroups go round-robin over the 8 XCDs, each with its own L2: every XCD takes a contiguous run of the tiles, in blocks

@@ -9,7 +9,7 @@
 //   torch.ops.nanoquantization_amd.awq_linear_swiglu(x, qweight, qscales, qzeros) -> Tensor [M, N / 2]
 // and the steps between the linears of the Qwen3 modules (nanoquantization/layers/norm.py:18-32, layers/rope.py:24-45,
 // models/qwen3_quantized.py:79-99, 147-152), inference only (none has a derivative):
-//   awq_swiglu_pair, awq_linear_three, rms_norm, silu_mul, qkv_norm_rope, causal_attention
+//   awq_swiglu_pair, awq_linear_three, awq_linear_add, rms_norm, silu_mul, qkv_norm_rope, causal_attention
 // with Meta kernels (shapes only), so the operators are visible to the dispatcher and to tracing.
 #include <dlfcn.h>
 
@@ -168,6 +168,34 @@ at::Tensor awq_linear_op(const at::Tensor& x, const at::Tensor& qweight, const a
                             nbytes ? ws.data_ptr() : nullptr, nbytes ? (size_t)ws.numel() : 0, stream),
                  "awq_linear");
     return out;
+}
+
+// residual + awq_linear(x): in the product's last step where the weight is dequantised first, else an addition of its own.
+at::Tensor awq_linear_add_op(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& qscales, const at::Tensor& qzeros,
+                             const at::Tensor& residual) {
+    const Packed p = check_packed(qweight, qscales, qzeros);
+    TORCH_CHECK(x.dim() == 2 && x.size(1) == p.K, "x must be [M, ", p.K, "], got ", x.sizes());
+    const int64_t M = x.size(0);
+    TORCH_CHECK(residual.dim() == 2 && residual.size(0) == M && residual.size(1) == p.N && residual.scalar_type() == qscales.scalar_type(),
+                "residual must be [", M, ", ", p.N, "] of the scales' type, got ", residual.sizes());
+    check_device(x, {&qweight, &qscales, &qzeros, &residual});
+    const DeviceGuard guard(x.device());
+    const bool dense = residual.is_contiguous() && !(reinterpret_cast<uintptr_t>(residual.data_ptr()) & 15u) && p.N <= (1 << 22);
+    if (const at::Tensor scratch = dense ? dense_scratch(x.device(), M, p) : at::Tensor(); scratch.defined()) {
+        const at::ScalarType dt = qscales.scalar_type();
+        const at::Tensor xc = (x.scalar_type() == dt ? x : x.to(dt)).contiguous();
+        const at::Tensor qw = qweight.contiguous(), qs = qscales.contiguous(), qz = qzeros.contiguous();
+        at::Tensor out = at::empty({M, p.N}, qs.options());
+        check_status(awq_linear_dense_add(xc.data_ptr(), qw.data_ptr<int32_t>(), qs.data_ptr(), qz.data_ptr<int32_t>(), residual.data_ptr(),
+                                          out.data_ptr(), M, p.N, p.K, p.g, p.dtype, scratch.data_ptr(), (size_t)scratch.numel(),
+                                          current_stream(x.device().index())),
+                     "awq_linear_dense_add");
+        return out;
+    }
+    return at::add(residual, awq_linear_op(x, qweight, qscales, qzeros, c10::nullopt));
+}
+at::Tensor awq_linear_add_meta(const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor& residual) {
+    return at::empty(residual.sizes(), residual.options());
 }
 
 at::Tensor awq_linear_meta(const at::Tensor& x, const at::Tensor& qweight, const at::Tensor& qscales,
@@ -444,6 +472,7 @@ TORCH_LIBRARY(nanoquantization_amd, m) {
     m.def("awq_linear_swiglu(Tensor x, Tensor qweight, Tensor qscales, Tensor qzeros) -> Tensor");
     m.def("awq_swiglu_pair(Tensor x, Tensor gate_qweight, Tensor gate_qscales, Tensor gate_qzeros, Tensor up_qweight, "
           "Tensor up_qscales, Tensor up_qzeros) -> Tensor");
+    m.def("awq_linear_add(Tensor x, Tensor qweight, Tensor qscales, Tensor qzeros, Tensor residual) -> Tensor");
     m.def("awq_linear_three(Tensor x, Tensor qweight0, Tensor qscales0, Tensor qzeros0, Tensor qweight1, Tensor qscales1, Tensor "
           "qzeros1, Tensor qweight2, Tensor qscales2, Tensor qzeros2) -> (Tensor, Tensor, Tensor)");
     m.def("rms_norm(Tensor x, Tensor weight, float eps) -> Tensor");
@@ -459,6 +488,7 @@ TORCH_LIBRARY_IMPL(nanoquantization_amd, CUDA, m) {   // the dispatch key of HIP
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_op);
     m.impl("awq_swiglu_pair", &awq_swiglu_pair_op);
     m.impl("awq_linear_three", &awq_linear_three_op);
+    m.impl("awq_linear_add", &awq_linear_add_op);
     m.impl("rms_norm", &rms_norm_op);
     m.impl("silu_mul", &silu_mul_op);
     m.impl("qkv_norm_rope", &qkv_norm_rope_op);
@@ -471,6 +501,7 @@ TORCH_LIBRARY_IMPL(nanoquantization_amd, Meta, m) {
     m.impl("awq_linear_swiglu", &awq_linear_swiglu_meta);
     m.impl("awq_swiglu_pair", &awq_swiglu_pair_meta);
     m.impl("awq_linear_three", &awq_linear_three_meta);
+    m.impl("awq_linear_add", &awq_linear_add_meta);
     m.impl("rms_norm", &rms_norm_meta);
     m.impl("silu_mul", &silu_mul_meta);
     m.impl("qkv_norm_rope", &qkv_norm_rope_meta);

@@ -22,7 +22,21 @@ from ..layers.norm import RMSNorm
 from ..layers.rope import RoPE
 
 
-@shipped("qkv")
+_ADD_FROM = 1 << 20      # elements from which an addition is worth more than the questions whether it can be left to the product before it
+
+
+def _add_linear(residual: torch.Tensor, linear: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """residual + linear(x): one operator where the linear is this package's, unchanged and watched by no hook."""
+    if (type(linear) is WQLinear_GEMM and linear.bias is None and keeps(linear, WQLinear_GEMM, "forward") and plain(x, linear.qscales, residual)
+            and linear.qscales.dim() == 2 and residual.is_contiguous() and x.shape[:-1] == residual.shape[:-1]
+            and residual.shape[-1] == linear.qscales.shape[-1] and unhooked(linear)):
+        y = _lib.torch_ops().awq_linear_add(x.reshape(-1, x.shape[-1]), linear.qweight, linear.qscales, linear.qzeros,
+                                            residual.view(-1, residual.shape[-1]))
+        return y.view(residual.shape)
+    return residual + linear(x)
+
+
+@shipped("qkv", "forward")
 class Qwen3QuantizedAttention(nn.Module):
     def __init__(self, hidden_size: int, total_num_heads: int, total_num_kv_heads: int,
                  max_position_embeddings: int, w_bits: int = 4, group_size: int = 128,
@@ -87,18 +101,21 @@ class Qwen3QuantizedAttention(nn.Module):
             return tuple(y.view(*x.shape[:-1], y.shape[-1]) for y in out)
         return self.q_proj(x), self.k_proj(x), self.v_proj(x)
 
-    def _on_operators(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
+    def _on_operators(self, x: torch.Tensor, position_ids: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """With a residual: the sum of it and what the module returns."""
+        added = (lambda y: y) if residual is None else lambda y: residual + y
         q, k, v = self._project(x)
         if not self._fused(q, k, v, position_ids):
             q, k, v = self._norm_rope(q, k, v, position_ids)
-            return self._attend(q, k, v)
+            return added(self._attend(q, k, v))
         pos = (position_ids if position_ids.dim() == 2 else position_ids.unsqueeze(0)).to(torch.int64)
         self.rope.refuse_unknown(pos)
         q, k, v = _lib.torch_ops().qkv_norm_rope(q, k, v, self.q_norm.weight, self.k_norm.weight, self.rope.cos_sin_cache, pos,
                                                  self.num_heads, self.num_kv_heads, self.q_norm.eps, self.k_norm.eps)
         if q.dtype == torch.bfloat16:
-            return self.o_proj(_lib.torch_ops().causal_attention(q, k, v, self.head_dim ** -0.5))
-        return self._attend(q, k.transpose(1, 2), v.transpose(1, 2))
+            o = _lib.torch_ops().causal_attention(q, k, v, self.head_dim ** -0.5)
+            return self.o_proj(o) if residual is None else _add_linear(residual, self.o_proj, o)
+        return added(self._attend(q, k.transpose(1, 2), v.transpose(1, 2)))
 
     def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
         if not torch.jit.is_scripting():        # script sees the torch expressions only
@@ -108,6 +125,7 @@ class Qwen3QuantizedAttention(nn.Module):
         return self._attend(q, k, v)
 
 
+@shipped("forward")
 class Qwen3QuantizedMLP(nn.Module):
     def __init__(self, hidden_size: int, intermediate_size: int, w_bits: int = 4, group_size: int = 128):
         super().__init__()
@@ -151,7 +169,19 @@ class Qwen3QuantizedBlock(nn.Module):
         self.input_layernorm = RMSNorm(hidden_size, rms_norm_eps)
         self.post_attention_layernorm = RMSNorm(hidden_size, rms_norm_eps)
 
+    def _adds_in_products(self, x: torch.Tensor) -> bool:
+        """Whether the residual additions may go with the products before them: enough rows, and an attention and an MLP that are the ones of
+        this package, unchanged and watched by no hook."""
+        attn, mlp = self.self_attn, self.mlp
+        return (x.numel() >= _ADD_FROM and plain(x) and x.is_contiguous() and type(attn) is Qwen3QuantizedAttention
+                and type(mlp) is Qwen3QuantizedMLP and keeps(attn, Qwen3QuantizedAttention, "qkv", "forward")
+                and keeps(mlp, Qwen3QuantizedMLP, "forward") and unhooked(attn, mlp))
+
     def forward(self, x: torch.Tensor, position_ids: torch.Tensor) -> torch.Tensor:
+        if not torch.jit.is_scripting():        # script sees the torch expressions only
+            if not torch.compiler.is_compiling() and not torch.jit.is_tracing() and self._adds_in_products(x):
+                x = self.self_attn._on_operators(self.input_layernorm(x), position_ids, x)
+                return _add_linear(x, self.mlp.down_proj, self.mlp._activation(self.post_attention_layernorm(x)))
         x = x + self.self_attn(self.input_layernorm(x), position_ids)
         return x + self.mlp(self.post_attention_layernorm(x))
 

@@ -302,3 +302,55 @@ def test_qkv_norm_rope_sizes(dtype, batch, tokens, heads, kv, dim):
         # the weight, whose own two roundings are half a place away each: 2 eps a term, and half of one for the result's rounding
         assert ((out.view_as(want).float() - want).abs() <= 2.5 * torch.finfo(dtype).eps * size + 1e-6).all()
     assert torch.equal(got[2].view(batch, kv, tokens, dim).transpose(1, 2), v.view(batch, tokens, kv, dim))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K,N", [(2048, 512, 1024), (300, 1024, 264), (4097, 256, 1032), (1, 256, 256), (129, 1024, 2560), (2048, 128, 8200)])
+def test_linear_with_a_residual(dtype, M, K, N):
+    """residual + linear(x) in the product's last step or behind it, whole and part tiles of both sizes: the bits of the two operations."""
+    ops = _lib_ops()
+    g = torch.Generator(device="cuda").manual_seed(M)
+    words = lambda *n: torch.randint(-2 ** 31, 2 ** 31 - 1, n, generator=g, device="cuda", dtype=torch.int64).int()
+    w = (words(K, N // 8), (torch.rand(K // 128, N, generator=g, device="cuda") * 0.01 + 0.01).to(dtype), words(K // 128, N // 8))
+    x, r = (torch.randn(M, n, generator=g, device="cuda").to(dtype) for n in (K, N))
+    want = r + ops.awq_linear(x, *w, None)
+    assert torch.equal(ops.awq_linear_add(x, *w, r), want)
+    odd = torch.empty(M, N + 1, dtype=dtype, device="cuda")[:, 1:].copy_(r)      # rows that are neither dense nor aligned
+    assert torch.equal(ops.awq_linear_add(x, *w, odd), want)
+    with pytest.raises(RuntimeError, match="residual must be"):
+        ops.awq_linear_add(x, *w, r[:, 8:])
+
+
+def _lib_ops():
+    from nanoquantization_amd import _lib
+    return _lib.torch_ops()
+
+
+def test_block_leaves_its_additions_to_the_products(monkeypatch):
+    """The forward of a model with the residual additions in the products before them, and without: the same bits; whoever watches or replaces a part
+    of a block hears of every call."""
+    import nanoquantization_amd.models.qwen3_quantized as q3
+    from nanoquantization_amd.models.random_init import QWEN3_0P6B, random_awq_qwen3
+    model = random_awq_qwen3(dict(QWEN3_0P6B, num_hidden_layers=2, vocab_size=512, max_position_embeddings=512), seed=3, std=0.02)
+    ids = torch.randint(0, 512, (2, 300), generator=torch.Generator().manual_seed(1)).cuda()
+    pos = torch.arange(300, device="cuda").unsqueeze(0)
+    calls = []
+    with torch.no_grad():
+        monkeypatch.setattr(q3, "_ADD_FROM", 1 << 62)
+        want = model(ids, pos)
+        monkeypatch.setattr(q3, "_ADD_FROM", 0)
+        add = q3._add_linear
+        monkeypatch.setattr(q3, "_add_linear", lambda *a: (calls.append(a[1]), add(*a))[1])
+        assert torch.equal(model(ids, pos), want) and len(calls) == 4
+        block = model.model.layers[0]
+        for part, expected in ((block.self_attn, 2), (block.mlp, 2), (block.self_attn.o_proj, 4), (block.mlp.down_proj, 4), (block.input_layernorm, 4)):
+            heard = []
+            hook = part.register_forward_hook(lambda *a: heard.append(1))
+            calls.clear()
+            assert torch.equal(model(ids, pos), want) and heard == [1] and len(calls) == expected
+            hook.remove()
+        for part in (block.self_attn, block.mlp, block.self_attn.o_proj, block.mlp.down_proj):
+            heard, forward = [], part.forward
+            part.forward = lambda *a: (heard.append(1), forward(*a))[1]
+            assert torch.equal(model(ids, pos), want) and heard == [1]
+            del part.forward
