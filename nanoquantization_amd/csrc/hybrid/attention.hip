@@ -590,7 +590,9 @@ __global__ __launch_bounds__(256, R > 160 ? 1 : 2) void attn_even_kernel(
 }
 
 // Decode attention.  Workgroup = (sequence, kv head, 16 of its query heads, context split); a wave takes tiles of 32 keys
-// through its own part of LDS, no barriers until the merge.
+// through its own part of LDS, no barriers until the merge.  Bound by memory; the block numbers are asked for a tile ahead, and large launches stream
+// past the L2 (us, 8 kv heads of 128, two query heads each, caches from HBM, before both / now: 1 x 8000 tokens 17.9 / 16.8, 16 x 640 16.9 / 15.3, 16 x
+// 2048 30.2 / 28.2, 32 x 640 20.6 / 18.4, 64 x 1000 52.6 / 47.8; heads of 256 64 x 500 53.8 / 46.6; past the L2 in 640 workgroups 40 x 1000 37.8, through it 37.0).
 template <int R, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
@@ -632,68 +634,76 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(
 #pragma unroll
     for (int w = 0; w < R / 16; ++w) acc[w] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int32_t* table = block_table + (int64_t)b * max_blocks;
-    for (int tb = t0 + wave * TT; tb < t1; tb += WAVES * TT) {
-        // the cache row of key tb + lane % 32 (past the split's end the last key stands in)
-        const int j = min(tb + (lane & 31), t1 - 1);
-        int blk = table[j / block_size];
-        blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
-        const int my_row = (blk * kv_heads + g) * block_size + j % block_size;
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int n = i * 64 + lane, row = n / L::kPieces;
-            const int64_t base = (int64_t)__shfl(my_row, row) * R;
-            __builtin_amdgcn_global_load_lds(NQH_GPTR(k_cache + base + L::k_source(row, n % L::kPieces)),
-                                             NQH_LPTR(kt + i * 1024), 16, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int n = i * 64 + lane, row = n / L::kPieces;
-            const int64_t base = (int64_t)__shfl(my_row, row) * R;
-            __builtin_amdgcn_global_load_lds(NQH_GPTR(v_cache + base + L::v_source(row, n % L::kPieces)),
-                                             NQH_LPTR(vt + i * 1024), 16, 0, 0);
-        }
-        // a wave's loads return in order: with at most the V tile's outstanding, the K tile has landed
-        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads) : "memory");
-        f32x4 st[2];
-        st[0] = st[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int s = 0; s < R / 32; ++s)
-                st[a] = Bf::mfma16(*reinterpret_cast<const u32x4*>(kt + L::k_at(16 * a + lo, 4 * s + hi)), bq[s], st[a]);
-        float mx = kNegBig;
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                st[a][r] = tb + 16 * a + 4 * hi + r < t1 ? st[a][r] * sc : -__builtin_inff();
-                mx = fmaxf(mx, st[a][r]);
+    const auto walk = [&](auto policy) __attribute__((always_inline)) {
+        constexpr int kPolicy = decltype(policy)::value;
+        // the key tb + lane % 32 (past the split's end the last one stands in) of the tile and its block, asked for a tile ahead
+        int key = min(t0 + wave * TT + (lane & 31), t1 - 1), block = t0 + wave * TT < t1 ? table[key / block_size] : 0;
+        for (int tb = t0 + wave * TT; tb < t1; tb += WAVES * TT) {
+            const int blk = block < 0 ? 0 : (block >= num_blocks ? num_blocks - 1 : block);
+            const int my_row = (blk * kv_heads + g) * block_size + key % block_size;
+            key = min(tb + WAVES * TT + (lane & 31), t1 - 1);
+            block = table[key / block_size];
+    #pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                const int n = i * 64 + lane, row = n / L::kPieces;
+                const int64_t base = (int64_t)__shfl(my_row, row) * R;
+                __builtin_amdgcn_global_load_lds(NQH_GPTR(k_cache + base + L::k_source(row, n % L::kPieces)),
+                                                 NQH_LPTR(kt + i * 1024), 16, 0, kPolicy);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(m, mx);
-        const float f = exp2_raw(m - mn);
-        m = mn;
-        float p[2][4], ps = 0.f;
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                p[a][r] = exp2_raw(st[a][r] - mn);
-                ps += p[a][r];
+    #pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                const int n = i * 64 + lane, row = n / L::kPieces;
+                const int64_t base = (int64_t)__shfl(my_row, row) * R;
+                __builtin_amdgcn_global_load_lds(NQH_GPTR(v_cache + base + L::v_source(row, n % L::kPieces)),
+                                                 NQH_LPTR(vt + i * 1024), 16, 0, kPolicy);
             }
-        l = l * f + ps;
-        const u32x4 pb = u32x4{Bf::pack2(p[0][0], p[0][1]), Bf::pack2(p[0][2], p[0][3]), Bf::pack2(p[1][0], p[1][1]),
-                               Bf::pack2(p[1][2], p[1][3])};
-#pragma unroll
-        for (int w = 0; w < R / 16; ++w)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[w][r] *= f;
-        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-#pragma unroll
-        for (int w = 0; w < R / 16; ++w) acc[w] = Bf::mfma16(value_operand<R>(vt, 0, w, lane), pb, acc[w]);
-        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");   // the tile is free for the next loads
-    }
+            // a wave's loads return in order: with at most the V tile's outstanding, the K tile has landed
+            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads) : "memory");
+            f32x4 st[2];
+            st[0] = st[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    #pragma unroll
+            for (int a = 0; a < 2; ++a)
+    #pragma unroll
+                for (int s = 0; s < R / 32; ++s)
+                    st[a] = Bf::mfma16(*reinterpret_cast<const u32x4*>(kt + L::k_at(16 * a + lo, 4 * s + hi)), bq[s], st[a]);
+            float mx = kNegBig;
+    #pragma unroll
+            for (int a = 0; a < 2; ++a)
+    #pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    st[a][r] = tb + 16 * a + 4 * hi + r < t1 ? st[a][r] * sc : -__builtin_inff();
+                    mx = fmaxf(mx, st[a][r]);
+                }
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float mn = fmaxf(m, mx);
+            const float f = exp2_raw(m - mn);
+            m = mn;
+            float p[2][4], ps = 0.f;
+    #pragma unroll
+            for (int a = 0; a < 2; ++a)
+    #pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    p[a][r] = exp2_raw(st[a][r] - mn);
+                    ps += p[a][r];
+                }
+            l = l * f + ps;
+            const u32x4 pb = u32x4{Bf::pack2(p[0][0], p[0][1]), Bf::pack2(p[0][2], p[0][3]), Bf::pack2(p[1][0], p[1][1]),
+                                   Bf::pack2(p[1][2], p[1][3])};
+    #pragma unroll
+            for (int w = 0; w < R / 16; ++w)
+    #pragma unroll
+                for (int r = 0; r < 4; ++r) acc[w][r] *= f;
+            asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    #pragma unroll
+            for (int w = 0; w < R / 16; ++w) acc[w] = Bf::mfma16(value_operand<R>(vt, 0, w, lane), pb, acc[w]);
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");   // the tile is free for the next loads
+        }
+    };
+    // past the L2 where the launch fills the CUs, two workgroups each, in whole rounds but for a quarter, and this split is its share of 16 MB or more
+    const unsigned last = gridDim.x % 512;
+    if ((gridDim.x <= 512 ? gridDim.x >= 192 : last == 0 || last >= 384) && (int64_t)(t1 - t0) * gridDim.x * R >= (4 << 20)) walk(std::integral_constant<int, 2>{});      // nt
+    else walk(std::integral_constant<int, 0>{});
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     // per-wave results [head][RS] over the wave's own tiles, then merged over the waves
