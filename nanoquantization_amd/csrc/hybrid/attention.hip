@@ -592,9 +592,10 @@ __global__ __launch_bounds__(256, R > 160 ? 1 : 2) void attn_even_kernel(
 // Decode attention.  Workgroup = (sequence, kv head, 16 of its query heads, context split); a wave takes tiles of 32 keys
 // through its own part of LDS, no barriers until the merge.  Bound by memory; the block numbers are asked for a tile ahead, and large launches stream
 // past the L2 (us, 8 kv heads of 128, two query heads each, caches from HBM, before both / now: 1 x 8000 tokens 17.9 / 16.8, 16 x 640 16.9 / 15.3, 16 x
-// 2048 30.2 / 28.2, 32 x 640 20.6 / 18.4, 64 x 1000 52.6 / 47.8; heads of 256 64 x 500 53.8 / 46.6; past the L2 in 640 workgroups 40 x 1000 37.8, through it 37.0).
-template <int R, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(
+// 2048 30.2 / 28.2, 32 x 640 20.6 / 18.4, 64 x 1000 52.6 / 47.8; heads of 256 64 x 500 53.8 / 46.6; past the L2 in 640 workgroups 40 x 1000 37.8, through it
+// 35.0).  attn_decode_past_l2_kernel is the same by another name: a kernel that holds both has its tiles in two loops.
+template <int R, int WAVES, int kPolicy>
+__device__ __forceinline__ void attn_decode(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, const uint16_t* __restrict__ sink,
     uint16_t* __restrict__ out, float* __restrict__ partial, int heads, int kv_heads, int vdim, int block_size, int max_blocks,
@@ -634,76 +635,69 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(
 #pragma unroll
     for (int w = 0; w < R / 16; ++w) acc[w] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int32_t* table = block_table + (int64_t)b * max_blocks;
-    const auto walk = [&](auto policy) __attribute__((always_inline)) {
-        constexpr int kPolicy = decltype(policy)::value;
-        // the key tb + lane % 32 (past the split's end the last one stands in) of the tile and its block, asked for a tile ahead
-        int key = min(t0 + wave * TT + (lane & 31), t1 - 1), block = t0 + wave * TT < t1 ? table[key / block_size] : 0;
-        for (int tb = t0 + wave * TT; tb < t1; tb += WAVES * TT) {
-            const int blk = block < 0 ? 0 : (block >= num_blocks ? num_blocks - 1 : block);
-            const int my_row = (blk * kv_heads + g) * block_size + key % block_size;
-            key = min(tb + WAVES * TT + (lane & 31), t1 - 1);
-            block = table[key / block_size];
-    #pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int n = i * 64 + lane, row = n / L::kPieces;
-                const int64_t base = (int64_t)__shfl(my_row, row) * R;
-                __builtin_amdgcn_global_load_lds(NQH_GPTR(k_cache + base + L::k_source(row, n % L::kPieces)),
-                                                 NQH_LPTR(kt + i * 1024), 16, 0, kPolicy);
-            }
-    #pragma unroll
-            for (int i = 0; i < kLoads; ++i) {
-                const int n = i * 64 + lane, row = n / L::kPieces;
-                const int64_t base = (int64_t)__shfl(my_row, row) * R;
-                __builtin_amdgcn_global_load_lds(NQH_GPTR(v_cache + base + L::v_source(row, n % L::kPieces)),
-                                                 NQH_LPTR(vt + i * 1024), 16, 0, kPolicy);
-            }
-            // a wave's loads return in order: with at most the V tile's outstanding, the K tile has landed
-            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads) : "memory");
-            f32x4 st[2];
-            st[0] = st[1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    #pragma unroll
-            for (int a = 0; a < 2; ++a)
-    #pragma unroll
-                for (int s = 0; s < R / 32; ++s)
-                    st[a] = Bf::mfma16(*reinterpret_cast<const u32x4*>(kt + L::k_at(16 * a + lo, 4 * s + hi)), bq[s], st[a]);
-            float mx = kNegBig;
-    #pragma unroll
-            for (int a = 0; a < 2; ++a)
-    #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    st[a][r] = tb + 16 * a + 4 * hi + r < t1 ? st[a][r] * sc : -__builtin_inff();
-                    mx = fmaxf(mx, st[a][r]);
-                }
-            mx = fmaxf(mx, __shfl_xor(mx, 16));
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
-            const float mn = fmaxf(m, mx);
-            const float f = exp2_raw(m - mn);
-            m = mn;
-            float p[2][4], ps = 0.f;
-    #pragma unroll
-            for (int a = 0; a < 2; ++a)
-    #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    p[a][r] = exp2_raw(st[a][r] - mn);
-                    ps += p[a][r];
-                }
-            l = l * f + ps;
-            const u32x4 pb = u32x4{Bf::pack2(p[0][0], p[0][1]), Bf::pack2(p[0][2], p[0][3]), Bf::pack2(p[1][0], p[1][1]),
-                                   Bf::pack2(p[1][2], p[1][3])};
-    #pragma unroll
-            for (int w = 0; w < R / 16; ++w)
-    #pragma unroll
-                for (int r = 0; r < 4; ++r) acc[w][r] *= f;
-            asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-    #pragma unroll
-            for (int w = 0; w < R / 16; ++w) acc[w] = Bf::mfma16(value_operand<R>(vt, 0, w, lane), pb, acc[w]);
-            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");   // the tile is free for the next loads
+    // the key tb + lane % 32 (past the split's end the last one stands in) of the tile and its block, asked for a tile ahead
+    int key = min(t0 + wave * TT + (lane & 31), t1 - 1), block = t0 + wave * TT < t1 ? table[key / block_size] : 0;
+    for (int tb = t0 + wave * TT; tb < t1; tb += WAVES * TT) {
+        const int blk = block < 0 ? 0 : (block >= num_blocks ? num_blocks - 1 : block);
+        const int my_row = (blk * kv_heads + g) * block_size + key % block_size;
+        key = min(tb + WAVES * TT + (lane & 31), t1 - 1);
+        block = table[key / block_size];
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int n = i * 64 + lane, row = n / L::kPieces;
+            const int64_t base = (int64_t)__shfl(my_row, row) * R;
+            __builtin_amdgcn_global_load_lds(NQH_GPTR(k_cache + base + L::k_source(row, n % L::kPieces)),
+                                             NQH_LPTR(kt + i * 1024), 16, 0, kPolicy);
         }
-    };
-    // past the L2 where the launch fills the CUs, two workgroups each, in whole rounds but for a quarter, and this split is its share of 16 MB or more
-    const unsigned last = gridDim.x % 512;
-    if ((gridDim.x <= 512 ? gridDim.x >= 192 : last == 0 || last >= 384) && (int64_t)(t1 - t0) * gridDim.x * R >= (4 << 20)) walk(std::integral_constant<int, 2>{});      // nt
-    else walk(std::integral_constant<int, 0>{});
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const int n = i * 64 + lane, row = n / L::kPieces;
+            const int64_t base = (int64_t)__shfl(my_row, row) * R;
+            __builtin_amdgcn_global_load_lds(NQH_GPTR(v_cache + base + L::v_source(row, n % L::kPieces)),
+                                             NQH_LPTR(vt + i * 1024), 16, 0, kPolicy);
+        }
+        // a wave's loads return in order: with at most the V tile's outstanding, the K tile has landed
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads) : "memory");
+        f32x4 st[2];
+        st[0] = st[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int s = 0; s < R / 32; ++s)
+                st[a] = Bf::mfma16(*reinterpret_cast<const u32x4*>(kt + L::k_at(16 * a + lo, 4 * s + hi)), bq[s], st[a]);
+        float mx = kNegBig;
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                st[a][r] = tb + 16 * a + 4 * hi + r < t1 ? st[a][r] * sc : -__builtin_inff();
+                mx = fmaxf(mx, st[a][r]);
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float mn = fmaxf(m, mx);
+        const float f = exp2_raw(m - mn);
+        m = mn;
+        float p[2][4], ps = 0.f;
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                p[a][r] = exp2_raw(st[a][r] - mn);
+                ps += p[a][r];
+            }
+        l = l * f + ps;
+        const u32x4 pb = u32x4{Bf::pack2(p[0][0], p[0][1]), Bf::pack2(p[0][2], p[0][3]), Bf::pack2(p[1][0], p[1][1]),
+                               Bf::pack2(p[1][2], p[1][3])};
+#pragma unroll
+        for (int w = 0; w < R / 16; ++w)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[w][r] *= f;
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+#pragma unroll
+        for (int w = 0; w < R / 16; ++w) acc[w] = Bf::mfma16(value_operand<R>(vt, 0, w, lane), pb, acc[w]);
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");   // the tile is free for the next loads
+    }
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
     // per-wave results [head][RS] over the wave's own tiles, then merged over the waves
@@ -774,6 +768,23 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(
             }
         }
     }
+}
+
+template <int R, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
+    const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, const uint16_t* __restrict__ sink,
+    uint16_t* __restrict__ out, float* __restrict__ partial, int heads, int kv_heads, int vdim, int block_size, int max_blocks,
+    int num_blocks, int chunk, int window, float scale, int splits, int head_tiles) {
+    attn_decode<R, WAVES, 0>(q, k_cache, v_cache, block_table, context_lens, sink, out, partial, heads, kv_heads, vdim, block_size, max_blocks, num_blocks, chunk, window, scale, splits, head_tiles);
+}
+template <int R, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attn_decode_past_l2_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
+    const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, const uint16_t* __restrict__ sink,
+    uint16_t* __restrict__ out, float* __restrict__ partial, int heads, int kv_heads, int vdim, int block_size, int max_blocks,
+    int num_blocks, int chunk, int window, float scale, int splits, int head_tiles) {
+    attn_decode<R, WAVES, 2>(q, k_cache, v_cache, block_table, context_lens, sink, out, partial, heads, kv_heads, vdim, block_size, max_blocks, num_blocks, chunk, window, scale, splits, head_tiles);      // nt
 }
 
 // Decode attention over latent rows of R elements, the first RL of which are the value.  Workgroup = (sequence, 16 HT heads,
@@ -1099,7 +1110,10 @@ extern "C" int nqh_attention_decode(const void* q, const void* k_cache, const vo
         if (groups > kMaxI32 || batch * heads > kMaxI32) return fail(NQH_ERR_ARG, fn, "problem too large");
         NQH_WITH_ROW(k_row, {
             constexpr int WAVES = decode_waves(R);
-            attn_decode_kernel<R, WAVES><<<dim3((unsigned)groups), dim3(64 * WAVES), 0, (hipStream_t)stream>>>(
+            // the cache goes past the L2 where the launch fills the CUs, two workgroups each, in whole rounds but for a quarter, with 16 MB or more
+            const int64_t last = groups % 512, keys = most_keys(max_context, chunk, window);
+            const bool past = (groups <= 512 ? groups >= 192 : last == 0 || last >= 384) && batch * kv_heads * keys * R >= (4 << 20);
+            (past ? attn_decode_past_l2_kernel<R, WAVES> : attn_decode_kernel<R, WAVES>)<<<dim3((unsigned)groups), dim3(64 * WAVES), 0, (hipStream_t)stream>>>(
                 (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_table, context_lens,
                 (const uint16_t*)sink, (uint16_t*)out, (float*)workspace, (int)heads, (int)kv_heads, (int)vdim, (int)block_size,
                 (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale, splits, (int)head_tiles);
