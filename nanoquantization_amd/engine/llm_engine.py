@@ -15,7 +15,8 @@ decoding over the block table), o_proj GEMV, add+RMSNorm, fused gate|up GEMV, Si
 (include/nq_engine_ops.h + include/awq_hip.h).  Where the shapes allow (head_dim 128, hidden a multiple of 128, gate|up
 interleaved) the two add+RMSNorm kernels disappear as well: the o_proj and down_proj GEMVs add into the residual
 stream and leave its RMSNorm statistics, the q|k|v and gate|up GEMVs normalise their input on the way in -- five
-launches per block, same bits.  The decode graph and the schedulers are those of EngineCore.
+launches per block, same bits; and for the sizes of ops.BlockSteps all of them are one launch, of weights in a layout of its own, two per block with
+the attention.  The decode graph and the schedulers are those of EngineCore.
 """
 from __future__ import annotations
 
