@@ -206,6 +206,10 @@ __device__ __forceinline__ float across_hi(float x) {
 // only across the two waves of a SIMD.  Keys are therefore staged a tile ahead of the values.  (Leaving the running maximum
 // alone until a score exceeds it by 2^8 saves 4 % of the time, but then the largest probability is no longer 1, which 16 bits
 // hold exactly: the error against 64 bits grows by up to a fifth where few keys dominate.)
+// From the first product of a tile to its last a wave goes before the other workgroup's wave on its SIMD, so that the two fall into different parts
+// of their tiles: 16 heads 4 x 2048 tokens 106 -> 97 us, 1 x 8192 320 -> 285 (0.97 PFLOP/s), 32 heads 1 x 4096 171 -> 160.  With the settling of the
+// maxima too 100, 292, 159; around the value product alone no gain.  Workgroups of up to 1024 keys are level or lose by it (8 x 512 22.9 -> 23.6,
+// 16 x 300 26.2 -> 28.0).
 // What bounds it: per wave and tile of 64 x 128 64 MFMAs (1024 cycles) and some 250 vector instructions, 32 of them 2^x at a
 // quarter of the rate; two waves a SIMD, which is why rows of up to 128 keep within 256 registers (the form before, one wave
 // a SIMD, had 294).  Operands are read a step before they are multiplied; steps are fenced, or the scheduler asks for all of
@@ -479,6 +483,7 @@ __device__ __forceinline__ void attn_tile(
                 Probs pb;
                 load_keys(buf ^ 1, 0, ka[0]);
                 settle(t, st);
+                if (n_tiles * KT > 1024) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int a = 0; a < KT / 16; ++a) {
                     if (a + 1 < KT / 16) load_keys(buf ^ 1, a + 1, ka[(a + 1) & 1]);
@@ -493,6 +498,7 @@ __device__ __forceinline__ void attn_tile(
                     gather(i, va[i & 1], pb);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                __builtin_amdgcn_s_setprio(0);
             } else if (then) {
 #pragma unroll
                 for (int a = 0; a < KT / 16; ++a) {
