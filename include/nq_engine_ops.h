@@ -148,7 +148,7 @@ int nq_tile_weight(const int32_t* qweight, const void* qscales, const int32_t* q
  * next: up to four regions that the launch after this one reads (NULL: none); workgroups that are idle in the last phase bring them near.
  * The launch's workgroups hand rows to each other and wait for each other; one that has looked `spin` times in vain does what is missing
  * itself, so that the launch ends whatever part of it runs at a time.  The sums are in a fixed order: results repeat exactly.
- * rows 1..64, sizes that nq_block_step_supported names.
+ * rows 1..64, sizes that nq_block_step_supported names (with the head ratios of nq_paged_attention_decode_tiled, which writes attn).
  * Qwen3QuantizedBlock.forward, nanoquantization/models/qwen3_quantized.py:194-215 (and :79-93, :147-152), restricted to one token. */
 typedef struct nq_block_step_args {
     const void *o, *gate_up, *down, *qkv;

@@ -608,7 +608,8 @@ hipError_t launch_block_step(const BlockStep& a, hipStream_t st) {
 
 extern "C" size_t nq_block_step_supported(int64_t rows, int64_t hidden, int64_t inter, int64_t heads, int64_t kv_heads) {
     // (more rows of the second size have no registers left for their sums: six layers at 40 / 64 rows 560 / 610 us in launches one by one, 584 / 623)
-    return rows >= 1 && heads == 16 && kv_heads > 0 && kv_heads <= 16 &&
+    // head ratios: those whose attention leaves its result in the layout that o_proj reads (nq_paged_attention_decode_tiled)
+    return rows >= 1 && heads == 16 && (kv_heads == heads || 2 * kv_heads == heads) &&
            ((hidden == 1024 && inter == 3072 && rows <= 64) || (hidden == 2048 && inter == 6144 && rows <= 32));
 }
 

@@ -172,8 +172,9 @@ def test_block_step(size, rows):
 def test_sizes_without_a_form_are_refused():
     from nanoquantization_amd import _lib
     from nanoquantization_amd.engine import ops
-    ok = lambda rows, hidden, inter, heads=16, layers=2, dtype=torch.bfloat16: ops.BlockSteps.supported(rows, hidden, inter, heads, 8, layers, dtype)
-    assert ok(64, 1024, 3072) and ok(32, 2048, 6144)
+    ok = lambda rows, hidden, inter, heads=16, layers=2, dtype=torch.bfloat16, kv=8: ops.BlockSteps.supported(rows, hidden, inter, heads, kv, layers, dtype)
+    assert ok(64, 1024, 3072) and ok(32, 2048, 6144) and ok(64, 1024, 3072, kv=16)
+    assert not any(ok(8, 1024, 3072, kv=kv) or ok(8, 2048, 6144, kv=kv) for kv in (1, 2, 4, 5, 32))
     assert not any((ok(65, 1024, 3072), ok(33, 2048, 6144), ok(0, 1024, 3072), ok(8, 2560, 9728, 32), ok(8, 1024, 3072, 32), ok(8, 1024, 3072, layers=1),
                     ok(8, 1024, 3072, dtype=torch.float16)))
     c = _Case("0.6b", 2, seed=1)
@@ -229,3 +230,25 @@ def test_engine_decodes_alike_with_and_without_block_steps(batch, monkeypatch):
         for _ in range(2):
             logits.append(eng.decode([(l, 89, int(t)) for l, t in zip(leases, tokens[:, -1])]).clone())
     assert all(torch.equal(l, logits[0]) for l in logits)
+
+
+@pytest.mark.parametrize("kv", [1, 2, 4, 16])
+def test_engine_decodes_with_other_numbers_of_kv_heads(kv, monkeypatch):
+    """16 query heads over 1, 2 and 4 kv heads have no block step and decode one launch for each linear; over 16 they have one, and both ways
+    the logits are the same."""
+    from nanoquantization_amd.engine import LLMEngine, ops
+    from nanoquantization_amd.models.random_init import QWEN3_0P6B, random_awq_qwen3
+    cfg = dict(QWEN3_0P6B, num_hidden_layers=2, vocab_size=2048, max_position_embeddings=256, total_num_kv_heads=kv)
+    model = random_awq_qwen3(cfg, seed=kv, std=0.02)
+    torch.manual_seed(7)
+    tokens = torch.randint(0, 2048, (3, 40))
+    logits = []
+    for on in (True, False):
+        if not on:
+            monkeypatch.setattr(ops.BlockSteps, "supported", staticmethod(lambda *a: False))
+        eng = LLMEngine(model, max_batch=3, max_seq_len=64, block_size=32)
+        assert (eng.block_steps is not None) == (on and kv == 16)
+        leases = [eng.acquire(2) for _ in range(3)]
+        eng._prefill(tokens[:, :-1].cuda(), leases)
+        logits.append(eng.decode([(l, 39, int(t)) for l, t in zip(leases, tokens[:, -1])]).clone())
+    assert logits[0].isfinite().all() and torch.equal(*logits)

@@ -45,6 +45,21 @@ def test_library_exports_every_declared_symbol():
     assert L.awq_gemv_ex_workspace_bytes(4, 1024, 1024, 0, 4) == 4096 * 4 + 4 * 4 * 1024 * 4
 
 
+def test_block_steps_only_behind_an_attention_of_their_layout():
+    """Sizes of which a block step exists are sizes whose attention writes what it reads: that one goes on to look at its pointers."""
+    _ensure_built()
+    L = _lib.lib()
+    taken = set()
+    for kv in range(0, 18):
+        for hidden, inter in ((1024, 3072), (2048, 6144)):
+            if not L.nq_block_step_supported(8, hidden, inter, 16, kv):
+                continue
+            taken.add((hidden, kv))
+            rc = L.nq_paged_attention_decode_tiled(*[None] * 6, 8, 16, kv, 128, 64, 4, 32, 0.1, 1, None, 0, None)
+            assert rc == 1 and b"null pointer" in L.awq_hip_last_error(), (kv, rc, L.awq_hip_last_error())
+    assert taken == {(h, kv) for h in (1024, 2048) for kv in (8, 16)}
+
+
 def test_pseudo_quantize_matches_oracle_bitwise():
     torch.manual_seed(0)
     w = torch.randn(96, 512) * 0.02
