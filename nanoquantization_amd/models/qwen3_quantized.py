@@ -173,7 +173,7 @@ class Qwen3QuantizedBlock(nn.Module):
         """Whether the residual additions may go with the products before them: enough rows, and an attention and an MLP that are the ones of
         this package, unchanged and watched by no hook."""
         attn, mlp = self.self_attn, self.mlp
-        return (x.numel() >= _ADD_FROM and plain(x) and x.is_contiguous() and type(attn) is Qwen3QuantizedAttention
+        return (plain(x) and x.numel() >= _ADD_FROM and x.is_contiguous() and type(attn) is Qwen3QuantizedAttention
                 and type(mlp) is Qwen3QuantizedMLP and keeps(attn, Qwen3QuantizedAttention, "qkv", "forward")
                 and keeps(mlp, Qwen3QuantizedMLP, "forward") and unhooked(attn, mlp))
 

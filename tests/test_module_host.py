@@ -59,6 +59,24 @@ def test_mlp_can_be_traced_with_its_linears_as_leaves():
     assert sorted(called) == ["down_proj", "gate_proj", "up_proj"]
 
 
+@pytest.mark.parametrize("what", ["block", "model"])
+def test_block_can_be_traced_with_its_parts_as_leaves(what):
+    leaves = (Qwen3QuantizedAttention, Qwen3QuantizedMLP, RMSNorm, torch.nn.Embedding)
+
+    class Tracer(torch.fx.Tracer):
+        def is_leaf_module(self, m, name):
+            return isinstance(m, leaves) or super().is_leaf_module(m, name)
+
+    sizes = dict(group_size=64, hidden_size=64, total_num_heads=4, total_num_kv_heads=2, max_position_embeddings=32, intermediate_size=128, head_dim=64)
+    parts = ["input_layernorm", "self_attn", "post_attention_layernorm", "mlp"]
+    if what == "block":
+        graph = Tracer().trace(q3.Qwen3QuantizedBlock(**sizes))
+    else:
+        graph = Tracer().trace(q3.Qwen3QuantizedModel(num_hidden_layers=2, vocab_size=96, **sizes))
+        parts = ["embed_tokens", *(f"layers.{i}.{p}" for i in range(2) for p in parts), "norm"]
+    assert [n.target for n in graph.nodes if n.op == "call_module"] == parts
+
+
 class Product(torch.nn.Module):
     def __init__(self, n, m):
         super().__init__()
