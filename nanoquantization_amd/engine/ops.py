@@ -399,7 +399,11 @@ class BlockSteps:
     """The linears between the attentions of a decode step, a launch a layer (nq_block_step): the weights of every layer in its layout and
     the buffers its launches hand on.  Each layer: (q|k|v, o_proj, interleaved gate|up, down_proj) as (qweight, qscales, qzeros); the
     first layer's q|k|v is the caller's and None here.  One step at a time (the buffers are the object's)."""
-    SPIN = 1 << 14      # looks, some 0.6 us each: by then a workgroup that is not there yet will not come by itself
+    # Looks of some 0.6 us.  A launch that has the GPU to itself waits for 15 us at most (0.6B, 12 layers, 32 rows, 64 looks or 16384: 508 and 512 us a
+    # step, 32 510, 16 723; 1.7B, 24 rows, from 16 looks on 346).  Two launches that each hold a part of the CUs wait for workgroups that have no room: then
+    # the count is what either loses before it does the missing shares itself, 77 us a phase with this one.  Two such engines on two streams: 760 us for a
+    # step of both, as with any count from 64 on for 0.6B, 588 for 1.7B (32 looks 696).
+    SPIN = 128
 
     @staticmethod
     def supported(rows: int, hidden: int, inter: int, heads: int, kv_heads: int, layers: int, dtype: torch.dtype) -> bool:

@@ -252,3 +252,37 @@ def test_engine_decodes_with_other_numbers_of_kv_heads(kv, monkeypatch):
         eng._prefill(tokens[:, :-1].cuda(), leases)
         logits.append(eng.decode([(l, 39, int(t)) for l, t in zip(leases, tokens[:, -1])]).clone())
     assert logits[0].isfinite().all() and torch.equal(*logits)
+
+
+@pytest.mark.parametrize("size,layers,batch", [("0.6b", 6, 32), ("1.7b", 3, 24)])
+def test_two_engines_decode_at_once(size, layers, batch):
+    """Two engines on two streams, whose block steps each may hold a part of the GPU: the logits of one after the other, and no wait for
+    workgroups without room that is longer than a quarter of a millisecond in a launch (three phases)."""
+    from nanoquantization_amd.engine import LLMEngine, ops
+    from nanoquantization_amd.models.random_init import QWEN3_0P6B, random_awq_qwen3
+    assert 3 * ops.BlockSteps.SPIN * 0.6e-6 <= 0.25e-3
+    cfg = dict(QWEN3_0P6B, num_hidden_layers=layers, vocab_size=2048, max_position_embeddings=512, hidden_size=SIZES[size][0],
+               intermediate_size=SIZES[size][1])
+    model = random_awq_qwen3(cfg, seed=5, std=0.02)
+    streams, engines, rows, want = [torch.cuda.Stream() for _ in range(2)], [], [], []
+    for seed in range(2):
+        eng = LLMEngine(model, max_batch=batch, max_seq_len=384, block_size=64)
+        assert eng.block_steps is not None
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        for t in (*eng.cache.k, *eng.cache.v):
+            t.copy_(torch.randn(t.shape, generator=gen, device="cuda"))
+        rows.append([(eng.acquire(6), 320, 7 + i + seed) for i in range(batch)])
+        engines.append(eng)
+        for _ in range(2):
+            logits = eng.decode(rows[seed])
+        want.append(logits.clone())
+    torch.cuda.synchronize()
+    for _ in range(4):
+        got = []
+        for _ in range(5):
+            for i in range(2):
+                with torch.cuda.stream(streams[i]):
+                    logits = engines[i].decode(rows[i])
+                    got = got[-1:] + [logits]
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
