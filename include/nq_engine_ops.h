@@ -144,7 +144,8 @@ int nq_tile_weight(const int32_t* qweight, const void* qscales, const int32_t* q
  * fp32 [ceil(rows / 16) * 16][hidden / 8].  The result's bits are those of the launches one by one with K cut as awq_gemv_add_residual and
  * awq_gemv_rmsnorm cut it at these sizes (hidden 2048: at up to 16 rows).  Rows past `rows` of attn must be numbers.
  * `done`: nq_block_step_flag_words() words that are zero when the launch begins, of its own while it runs; `clear`: as many words of another launch
- * that is over, which this one sets to zero (the launches of a step clear each other's in a ring).  Every buffer is of its own.
+ * that is over, which this one sets to zero (the launches of a step clear each other's in a ring).  Every buffer is of its own,
+ * 16-byte aligned, and attn, res_out, act, q_out, the tiled residuals, the squares, done and clear begin on a line of 128 bytes.
  * next: up to four regions that the launch after this one reads (NULL: none); workgroups that are idle in the last phase bring them near.
  * The launch's workgroups hand rows to each other and wait for each other; one that has looked `spin` times in vain does what is missing
  * itself, so that the launch ends whatever part of it runs at a time.  The sums are in a fixed order: results repeat exactly.

@@ -21,8 +21,8 @@
 // result is written from one XCD.  A share that is done sets its bit in the word of its XCD, the last of a word its bit in the root, the last
 // of all rings 32 bells, each looked at by eight workgroups.  (All workgroups looking at the eight words delays the bits by up to 1.5 us, a
 // word whose bits come from several XCDs by 3, and so do loads in flight in the wave that looks, whose answers come in order: hence the weights
-// are asked for at the beginning.)  What crosses workgroups is stored past the L2 (sc1) and was read by nobody earlier in the launch, so that
-// ordinary loads, which the XCD's L2 shares, find no older line.  A workgroup never relies on another one to start: after `spin` looks it
+// are asked for at the beginning.)  What crosses workgroups is stored past the L2 (sc1) and its lines, which hold nothing else, were read by nobody earlier in
+// the launch, so that ordinary loads, which the XCD's L2 shares, find no older one.  A workgroup never relies on another one to start: after `spin` looks it
 // takes the first share that is missing itself; shares read only what earlier phases have written and write the same values whoever runs them.
 #include <type_traits>
 
@@ -629,6 +629,11 @@ extern "C" int nq_block_step(const nq_block_step_args* p, void* stream) {
                            (uintptr_t)q.norm_mid | (uintptr_t)q.norm_next | (uintptr_t)q.done | (uintptr_t)q.clear | (uintptr_t)q.q_weight |
                            (uintptr_t)q.k_weight | (uintptr_t)q.cos_sin | (uintptr_t)q.q_out | (uintptr_t)q.k_cache | (uintptr_t)q.v_cache;
     if (bits & 15u) return bad(fn, "every tensor must be 16-byte aligned");
+    // What one phase writes and a later one reads through the L2 has lines of its own (their sizes are whole lines at any number of rows): nobody
+    // brings one in by reading its neighbour before it is written.  The flags of another launch are cleared beside this one's.
+    const uintptr_t lines = (uintptr_t)q.act | (uintptr_t)q.tiled_mid | (uintptr_t)q.tiled_out | (uintptr_t)q.squares_mid | (uintptr_t)q.squares_out |
+                            (uintptr_t)q.done | (uintptr_t)q.clear | (uintptr_t)q.attn | (uintptr_t)q.res_out | (uintptr_t)q.q_out;
+    if (lines & 127u) return bad(fn, "attn, res_out, act, q_out, the tiled residuals, the squares and the flags must be 128-byte aligned");
     if (!nq_block_step_supported(q.rows, q.hidden, q.inter, q.heads, q.kv_heads)) {
         set_error("%s: no form for these sizes", fn);
         return AWQ_ERR_UNSUPPORTED;

@@ -60,6 +60,28 @@ def test_block_steps_only_behind_an_attention_of_their_layout():
     assert taken == {(h, kv) for h in (1024, 2048) for kv in (8, 16)}
 
 
+def test_block_step_wants_lines_of_its_own():
+    """What one phase writes and another reads begins on a line: no neighbour's read brings it into a cache before it is written.  (The addresses are made
+    up; a negative count of looks refuses the call behind the question of alignment.)"""
+    _ensure_built()
+    L = _lib.lib()
+
+    def refusal(**moved):
+        a = _lib.BlockStepArgs(rows=8, hidden=1024, inter=3072, heads=16, kv_heads=8, max_positions=64, num_slots=64, block_size=16, spin=-1)
+        pointers = [n for n, t in _lib.BlockStepArgs._fields_ if t is ctypes.c_void_p]
+        for i, name in enumerate(pointers):
+            setattr(a, name, (i + 1 << 24) + moved.get(name, 0))
+        assert L.nq_block_step(ctypes.byref(a), None) == 1
+        return L.awq_hip_last_error()
+
+    assert b"spin" in refusal()
+    for name in ("attn", "res_out", "act", "q_out", "tiled_mid", "tiled_out", "squares_mid", "squares_out", "done", "clear"):
+        assert b"128-byte aligned" in refusal(**{name: 64}) and b"128-byte aligned" in refusal(**{name: 16}), name
+        assert b"spin" in refusal(**{name: 128})
+    for name in ("o", "res_in", "norm_mid", "k_cache", "cos_sin"):
+        assert b"spin" in refusal(**{name: 16}) and b"16-byte aligned" in refusal(**{name: 8}), name
+
+
 def test_pseudo_quantize_matches_oracle_bitwise():
     torch.manual_seed(0)
     w = torch.randn(96, 512) * 0.02
