@@ -193,6 +193,12 @@ __device__ __forceinline__ f32x4 add_sums(const char* arena, int tile, int lane)
     return out;
 }
 
+// Where the sum of a row's squares of columns n .. n + 7 lies, in bytes: the 16 of 128 columns are half a line, and the line is of two rows of the same
+// columns, which one XCD writes.
+__device__ __forceinline__ uint32_t square_at(int row, int n, int width) {
+    return (uint32_t)((((row >> 4) * (width >> 7) + (n >> 7)) * 16 + (row & 15)) * 64 + (n >> 3 & 15) * 4);
+}
+
 // RMSNorm of what this wave has of 16 MT rows, x = T(T(x * r) * weight).  `squares` holds the sums of the rows' squares eight columns at a time: a wave
 // adds those of a tile of 128 (in the order of tile_ssq, awq_common.hpp), the tiles meet in LDS and are added in their order.
 template <typename T, int MT, int C>
@@ -207,7 +213,7 @@ __device__ __forceinline__ void normalise(u32x4 (&v)[C][MT][4], const Rsrc& squa
 #pragma unroll
         for (int m = 0; m < MT; ++m)
             part[d][m] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                       squares, (uint32_t)((row0 + 16 * m + (lane & 15)) * (kTiles * 16) + tile * 16 + (lane >> 4) * 4) * 4, 0,
+                                                       squares, square_at(row0 + 16 * m + (lane & 15), tile * 128, kTiles * 128) + (lane >> 4) * 16, 0,
                                                        kShared));
 #pragma unroll
         for (int s = 0; s < 4; ++s) w[d][s] = *reinterpret_cast<const u32x4*>(weight + tile * 128 + 32 * s + 8 * (lane >> 4));
@@ -385,7 +391,7 @@ __global__ __launch_bounds__(kBlockThreads) void block_step_kernel(const BlockSt
         if (r.to_rows) __builtin_amdgcn_raw_buffer_store_b128(out, r.rows, (uint32_t)(row * width + n) * 2, 0, kAgent);
         if (r.to_tiled) {
             __builtin_amdgcn_raw_buffer_store_b128(out, r.tiled, tiled_at(row, n, width), 0, kAgent);
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ss), r.squares, (uint32_t)(row * (width / 8) + (n >> 3)) * 4, 0, kAgent);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, ss), r.squares, square_at(row, n, width), 0, kAgent);
         }
     };
     const auto o_proj = [&](int task, bool reload, auto hook) {

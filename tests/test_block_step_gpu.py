@@ -164,6 +164,10 @@ def test_block_step(size, rows):
         assert rel(cache[block, :, at], want[live]) <= 6e-3, (name, rel(cache[block, :, at], want[live]))
         cache[block, :, at] = 0
         assert not cache.any(), name
+    # the sums of squares of the residual between o_proj and gate|up, whole lines of 128 columns a group of workgroups
+    mid = c.steps.tiled[0].view(-1, c.hidden // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(-1, c.hidden).double()
+    squares = c.steps.squares[0].view(-1, c.hidden // 128, 16, 16).transpose(1, 2).reshape(-1, c.hidden // 8)
+    assert torch.allclose(squares[:rows].double(), mid.square().view(-1, c.hidden // 8, 8).sum(-1)[:rows], rtol=8 * 2.0 ** -24, atol=0)
     # whoever does the work: nobody waits, every workgroup does what it finds missing
     for a, b in zip((x1, q, x2), (lambda t: (t[0], t[1], t[4]))(c.run(spin=0))):
         assert torch.equal(a, b)
