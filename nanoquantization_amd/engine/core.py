@@ -76,6 +76,9 @@ class EngineCore:
     def _decode_step(self) -> None:
         raise NotImplementedError
 
+    def _follow_weights(self) -> None:
+        """Before a call's first step: weights that the engine keeps in a layout of its own for its steps alone, as the modules hold them now."""
+
     # ---- leases ----------------------------------------------------------------------------------
     def acquire(self, num_blocks: int) -> Lease:
         lease = Lease(self.cache.allocate(num_blocks))
@@ -125,6 +128,7 @@ class EngineCore:
             state["s_table"][i, :len(lease.blocks)] = lease.blocks
         state["s_active"][:n] = True
         upload(state.reshape(1).view(np.uint8), self.device, out=self._decode_state)
+        self._follow_weights()      # (beside the copy)
         self._run_decode()
         return self.s_logits[:n]
 
@@ -176,6 +180,7 @@ class EngineCore:
             raise ValueError("this engine batches prompts of equal length only")
         if plen + max_new_tokens > self.max_ctx:
             raise ValueError("prompt + max_new_tokens exceeds max_seq_len")
+        self._follow_weights()
         leases: List[Lease] = []
         try:
             for _ in range(n):
@@ -231,6 +236,7 @@ class EngineCore:
                 raise ValueError("every request needs a non-empty prompt and max_new_tokens >= 1")
             if len(prompt) + max_new > self.max_ctx:
                 raise ValueError("prompt + max_new_tokens exceeds max_seq_len")
+        self._follow_weights()
         out: List[List[int]] = [[] for _ in requests]
         waiting = deque(range(len(requests)))
         free_rows = list(range(self.max_batch - 1, -1, -1))

@@ -20,6 +20,7 @@ the attention.  The decode graph and the schedulers are those of EngineCore.
 """
 from __future__ import annotations
 
+import operator
 from typing import List, Optional
 
 import torch
@@ -33,6 +34,9 @@ from .core import EngineCore
 from ..models.qwen3_quantized import Qwen3QuantizedForCausalLM
 
 
+_VERSION = operator.attrgetter("_version")
+
+
 class _FusedLinear:
     """Packed buffers of several WQLinear_GEMM with a common input, concatenated along N."""
 
@@ -44,6 +48,13 @@ class _FusedLinear:
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         return _linear("awq_linear", x, self.qweight, self.qscales, self.qzeros, None)
+
+
+def _times_written(tensors: List[torch.Tensor]) -> List[int]:
+    try:
+        return list(map(_VERSION, tensors))
+    except RuntimeError:        # an inference tensor does not count
+        return [0 if t.is_inference() else t._version for t in tensors]
 
 
 class LLMEngine(EngineCore):
@@ -89,10 +100,31 @@ class LLMEngine(EngineCore):
             self.block_steps = ops.BlockSteps([(tiled(self.qkv[i]) if i else None, tiled(l.self_attn.o_proj), self.gate_up_il[i],
                                                 tiled(l.mlp.down_proj)) for i, l in enumerate(layers)],
                                               max_batch, hidden, self.inter, self.nh, self.nkv, self.device)
+            self._weights = self._weights_now()
+            self._written = _times_written(self._weights)
         # prompts through the cache on the prompt attention kernel, which has matrix forms for these rows
         self.paged_prefill = self.dtype == torch.bfloat16 and self.hd in (32, 64, 96, 128, 192, 256)
         self.eps = layers[0].input_layernorm.eps
         self.scale = float(self.hd) ** -0.5
+
+    def _weights_now(self) -> List[torch.Tensor]:
+        return [t for l in self.model.model.layers for m in (l.self_attn.o_proj, l.mlp.down_proj) for t in (m.qweight, m.qscales, m.qzeros)]
+
+    def _follow_weights(self) -> None:
+        """The launches one by one read o_proj and down_proj where the modules have them (q|k|v and gate|up are copies made with the
+        engine): the block steps' copies of these follow what is written there in place and, without a graph, the tensors that take their
+        place.  Writes that torch does not count (through .data or a raw pointer, to inference tensors) are not seen.  Without a change 28 layers
+        take 8 us of the host."""
+        if self.block_steps is None:
+            return
+        weights = self._weights if self.use_graph else self._weights_now()
+        written = _times_written(weights)
+        if written == self._written and (self.use_graph or all(map(operator.is_, weights, self._weights))):
+            return
+        for i in range(0, len(weights), 3):
+            if written[i:i + 3] != self._written[i:i + 3] or any(map(operator.is_not, weights[i:i + 3], self._weights[i:i + 3])):
+                self.block_steps.replace(i // 6, ("o_proj", "down_proj")[i // 3 % 2], weights[i:i + 3])
+        self._weights, self._written = weights, written
 
     # ---- prefill: full causal attention over the prompt itself ------------------------------------
     def _prompt_layout(self, lens: List[int], leases: List[Lease]) -> Optional[hybrid_ops.PromptPass]:

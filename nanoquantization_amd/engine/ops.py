@@ -381,14 +381,17 @@ def awq_gemv_swiglu(x: torch.Tensor, qweight: torch.Tensor, qscales: torch.Tenso
     return out
 
 
-def tile_weight(qweight: torch.Tensor, qscales: torch.Tensor, qzeros: torch.Tensor) -> torch.Tensor:
-    """A packed weight in the layout BlockSteps reads (nq_tile_weight)."""
+def tile_weight(qweight: torch.Tensor, qscales: torch.Tensor, qzeros: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """A packed weight in the layout BlockSteps reads (nq_tile_weight), in `out` if given."""
     dev = _dev(qweight, qscales, qzeros)
     K, N = qweight.shape[0], qscales.shape[1]
     g = K // qscales.shape[0]
     assert qweight.shape == (K, N // 8) and qzeros.shape == (K // g, N // 8)
     L = _lib.lib()
-    out = torch.empty(L.nq_tiled_weight_bytes(N, K), dtype=torch.uint8, device=dev)
+    nbytes = L.nq_tiled_weight_bytes(N, K)
+    if out is None:
+        out = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    assert _dev(out) == dev and out.shape == (nbytes,) and out.dtype == torch.uint8
     with _lib.on_device(dev):
         _lib.check(L.nq_tile_weight(qweight.data_ptr(), qscales.data_ptr(), qzeros.data_ptr(), out.data_ptr(), N, K, g,
                                     _lib.dtype_id(qscales.dtype), _stream(dev)))
@@ -397,7 +400,7 @@ def tile_weight(qweight: torch.Tensor, qscales: torch.Tensor, qzeros: torch.Tens
 
 class BlockSteps:
     """The linears between the attentions of a decode step, a launch a layer (nq_block_step): the weights of every layer in its layout and
-    the buffers its launches hand on.  Each layer: (q|k|v, o_proj, interleaved gate|up, down_proj) as (qweight, qscales, qzeros); the
+    the buffers its launches hand on.  Each layer: (q|k|v, o_proj, interleaved gate|up, down_proj) as (qweight, qscales, qzeros), copied; the
     first layer's q|k|v is the caller's and None here.  One step at a time (the buffers are the object's)."""
     # Looks of some 0.6 us.  A launch that has the GPU to itself waits for 15 us at most (0.6B, 12 layers, 32 rows, 64 looks or 16384: 508 and 512 us a
     # step, 32 510, 16 723; 1.7B, 24 rows, from 16 looks on 346).  Two launches that each hold a part of the CUs wait for workgroups that have no room: then
@@ -423,6 +426,10 @@ class BlockSteps:
         # not finished, by the host
         self.done = zeros(len(layers), _lib.lib().nq_block_step_flag_words(), dtype=torch.int32)
         self.next = 0
+
+    def replace(self, index: int, linear: str, weight: Sequence[torch.Tensor]) -> None:
+        """Another o_proj or down_proj for a layer, (qweight, qscales, qzeros) of the same sizes."""
+        tile_weight(*weight, out=self.weights[index][{"o_proj": 1, "down_proj": 3}[linear]])
 
     def __call__(self, index: int, residual: torch.Tensor, norm_mid: torch.Tensor, eps: float, following=None, spin: int = SPIN) -> torch.Tensor:
         """Layer `index` from `self.attn` and its residual [rows, hidden] on; returns the residual behind it.  `following`: (norm weight, q_norm

@@ -290,3 +290,36 @@ def test_two_engines_decode_at_once(size, layers, batch):
                     got = got[-1:] + [logits]
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_decode_follows_weights_written_behind_the_engine(use_graph):
+    """o_proj and down_proj are the module's own: what is written there in place (without a graph also another tensor in its place) is what the next
+    decode step multiplies by."""
+    from nanoquantization_amd.engine import LLMEngine
+    from nanoquantization_amd.models.random_init import QWEN3_0P6B, random_awq_qwen3
+    cfg = dict(QWEN3_0P6B, num_hidden_layers=3, vocab_size=2048, max_position_embeddings=256)
+    model = random_awq_qwen3(cfg, seed=9, std=0.02)
+    tokens = torch.randint(0, 2048, (4, 40), generator=torch.Generator().manual_seed(1))
+
+    def engine():
+        eng = LLMEngine(model, max_batch=4, max_seq_len=64, block_size=32, use_graph=use_graph)
+        assert eng.block_steps is not None
+        return eng, [eng.acquire(2) for _ in range(4)]
+
+    def logits(eng, leases):
+        eng._prefill(tokens[:, :-1].cuda(), leases)
+        return eng.decode([(l, 39, int(t)) for l, t in zip(leases, tokens[:, -1])]).clone()
+
+    kept = engine()
+    before = logits(*kept)
+    layers = model.model.layers
+    other = random_awq_qwen3(cfg, seed=10, std=0.02).model.layers
+    with torch.no_grad():
+        layers[0].mlp.down_proj.qscales.mul_(2)
+        layers[1].self_attn.o_proj.load_state_dict(other[1].self_attn.o_proj.state_dict())
+        if not use_graph:
+            layers[2].self_attn.o_proj.qzeros = other[2].self_attn.o_proj.qzeros
+    after = logits(*kept)
+    assert not torch.equal(before, after) and torch.equal(after, logits(*engine()))
+    assert torch.equal(after, logits(*kept))
