@@ -399,59 +399,52 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_vec_kernel(
 
 // The same for the outputs of separate q, k and v projections of `batch` sequences of `tokens` tokens: q stays [token][head],
 // k and v become [sequence][kv head][token], where the attention over the sequences reads a head's tokens in a row.
-// A workgroup takes TOKENS tokens and HD / 8 of its lanes a head, two at a time: nothing is divided per lane, and the norm's weights and a token's
+// A workgroup takes a token and HD / 8 of its lanes a head, U heads at a time: nothing is divided per lane, and the norm's weights and the token's
 // angles are read once for several heads.  Bound by memory and the vector ALU: 8192 tokens of 16 + 8 + 8
-// heads of 128 (134 MB) 31.5 us, 4.2 TB/s; with a head for every HD / 8 lanes of the launch, whose token and place four 64-bit divisions found, a lane
-// exchange and a rounding for every value and both halves' sums in every lane 43; 512 tokens 5.5 -> 5.2, 8 x 300 tokens of 48 heads 19.9 -> 17.4; as torch
-// operations, which pass over fp32 copies a dozen times, 560.
-template <typename T, int HD, int TOKENS>
+// heads of 128 (134 MB) 29.5 us, 4.5 TB/s; with a head for every HD / 8 lanes of the launch, whose token and place four 64-bit divisions found, a lane
+// exchange and a rounding for every value and both halves' sums in every lane 40; 512 tokens 5.5 -> 5.1, 8192 sequences of one token 40 -> 29 (66 with
+// four tokens of a sequence a workgroup, which gain nothing at any length); as torch operations, which pass over fp32 copies a dozen times, 560.
+template <typename T, int HD, int U>
 __global__ __launch_bounds__(512) void qkv_norm_rope_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                             const uint16_t* __restrict__ v, const uint16_t* __restrict__ q_weight,
                                                             const uint16_t* __restrict__ k_weight,
                                                             const float* __restrict__ cos_sin,
                                                             const int64_t* __restrict__ positions, bool per_sequence,
                                                             uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out,
-                                                            uint16_t* __restrict__ v_out, int tokens, int nh, int nkv,
+                                                            uint16_t* __restrict__ v_out, int sequences, int tokens, int nh, int nkv, bool beside_tokens,
                                                             int64_t max_positions, float q_eps, float k_eps) {
-    constexpr int LPH = HD / 8, U = 2;
+    constexpr int LPH = HD / 8;
     const int heads = nh + 2 * nkv, groups = blockDim.x / LPH, group = threadIdx.x / LPH, dc = threadIdx.x % LPH;
-    const int64_t seq = blockIdx.y, row0 = seq * tokens;
-    for (int h0 = 0; h0 < heads; h0 += U * groups) {
-        const uint16_t* src[U];     // lanes past the last head follow it (the shuffles need them) and store nothing
+    // U == 1: blockDim.y tokens or sequences a workgroup.  Lanes past the last one or the last head follow it (the shuffles need them) and store nothing.
+    const int tokens_here = U == 1 && beside_tokens ? blockDim.y : 1, sequences_here = U == 1 && !beside_tokens ? blockDim.y : 1;
+    const int own_t = blockIdx.x * tokens_here + (tokens_here > 1 ? threadIdx.y : 0), own_seq = blockIdx.y * sequences_here + (sequences_here > 1 ? threadIdx.y : 0);
+    const int t = min(own_t, tokens - 1), seq = min(own_seq, sequences - 1);
+    const int64_t row = (int64_t)seq * tokens + t;
+    int64_t pos = positions[per_sequence ? row : t];
+    pos += pos < 0 ? max_positions : 0;     // an index from the end, as the table's own indexing takes it
+    const bool known = pos >= 0 && pos < max_positions;     // no angles for any other: not a number, rather than a wrong turn
+    const float* angles = cos_sin + (known ? pos : 0) * HD;
+    for (int h0 = blockIdx.z * U * groups; h0 < heads; h0 += gridDim.z * U * groups) {
+        u32x4 raw[U], weight[U];
         uint16_t* dst[U];
-        int step[U], out_step[U];
-        u32x4 weight[U];
         bool plain[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int h = min(h0 + u * groups + group, heads - 1), kv = h < nh + nkv ? h - nh : h - nh - nkv;
             const bool is_q = h < nh;
             plain[u] = h >= nh + nkv;
-            step[u] = (is_q ? nh : nkv) * HD;
-            src[u] = (is_q ? q + h * HD : (plain[u] ? v : k) + kv * HD) + row0 * step[u] + dc * 8;
-            out_step[u] = is_q ? nh * HD : HD;
-            dst[u] = (is_q ? q_out + row0 * step[u] + h * HD : (plain[u] ? v_out : k_out) + (seq * nkv + kv) * tokens * HD) + dc * 8;
+            raw[u] = *reinterpret_cast<const u32x4*>((is_q ? q + (row * nh + h) * HD : (plain[u] ? v : k) + (row * nkv + kv) * HD) + dc * 8);
+            dst[u] = (is_q ? q_out + (row * nh + h) * HD : (plain[u] ? v_out : k_out) + (((int64_t)seq * nkv + kv) * tokens + t) * HD) + dc * 8;
             weight[u] = *reinterpret_cast<const u32x4*>((is_q ? q_weight : k_weight) + dc * 8);
         }
+        const Turn<T, HD> turn(angles, dc);
 #pragma unroll
-        for (int i = 0; i < TOKENS; ++i) {
-            const int t = min((int)blockIdx.x * TOKENS + i, tokens - 1);
-            u32x4 raw[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) raw[u] = *reinterpret_cast<const u32x4*>(src[u] + (int64_t)t * step[u]);
-            int64_t pos = positions[per_sequence ? row0 + t : t];
-            pos += pos < 0 ? max_positions : 0;     // an index from the end, as the table's own indexing takes it
-            const bool known = pos >= 0 && pos < max_positions;     // no angles for any other: not a number, rather than a wrong turn
-            const Turn<T, HD> turn(cos_sin + (known ? pos : 0) * HD, dc);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int h = h0 + u * groups + group;
-                float a[8];
-                unpack8<T>(raw[u], a);
-                const u32x4 turned = turn(a, weight[u], known ? (h < nh ? q_eps : k_eps) : __builtin_nanf(""));
-                if (h < heads && (int)blockIdx.x * TOKENS + i < tokens)
-                    *reinterpret_cast<u32x4*>(dst[u] + (int64_t)t * out_step[u]) = plain[u] ? raw[u] : turned;
-            }
+        for (int u = 0; u < U; ++u) {
+            const int h = h0 + u * groups + group;
+            float a[8];
+            unpack8<T>(raw[u], a);
+            const u32x4 turned = turn(a, weight[u], known ? (h < nh ? q_eps : k_eps) : __builtin_nanf(""));
+            if (h < heads && own_t < tokens && own_seq < sequences) *reinterpret_cast<u32x4*>(dst[u]) = plain[u] ? raw[u] : turned;
         }
     }
 }
@@ -1556,32 +1549,40 @@ extern "C" int nq_qkv_norm_rope(const void* q, const void* k, const void* v, con
     }
     const int64_t items = batch * tokens * (num_heads + 2 * num_kv_heads);
     if (cdiv(items, 4 * (512 / head_dim)) > 0x7fffffff) return bad(fn, "problem too large");
-    // two heads a group of lanes and pass, passes of up to 512 lanes equally full
-    const int64_t each = head_dim / 8, pairs = cdiv(num_heads + 2 * num_kv_heads, 2), passes = cdiv(pairs * each, 512);
-    const int64_t lanes = cdiv(cdiv(pairs, passes) * each, 64) * 64;
+    // Two heads a group of lanes and pass, passes of up to 512 lanes equally full.  One head, and not two behind one another, where a wave has lanes for all
+    // of them (then with several tokens or sequences a workgroup: 8192 x 1 token of 4 + 1 + 1 heads of 64 6.6 us, 8.6 with two heads in a
+    // wave of its own) and where the launch has fewer waves than the chip holds at a time (then over several workgroups of 128 lanes: 64 tokens of
+    // 16 + 8 + 8 heads of 128 3.6 us, of 64 + 8 + 8 3.9; 4.1 and 5.3).
+    const int64_t heads = num_heads + 2 * num_kv_heads, each = head_dim / 8;
+    const bool few = heads * each <= 64, small = !few && batch * tokens * heads * each <= 2048 * 64;
+    const int64_t parts = cdiv(heads, 2), passes = cdiv(parts * each, 512);
+    const int64_t lanes = few ? heads * each : small ? 128 : cdiv(cdiv(parts, passes) * each, 64) * 64, shares = small ? cdiv(heads * each, lanes) : 1;
+    const bool beside_tokens = few && tokens >= 256 / lanes;
+    const int64_t tokens_beside = beside_tokens ? 256 / lanes : 1, sequences_beside = few && !beside_tokens ? std::min<int64_t>(batch, 256 / lanes) : 1;
     hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();
-    const auto go = [&](auto type, auto dim, auto each) {
+    const auto go = [&](auto type, auto dim, auto wide) {
         using T = decltype(type);
-        constexpr int HD = decltype(dim)::value, TOKENS = decltype(each)::value;
-        for (int64_t b = 0; b < batch; b += 65535) {     // the grid's second dimension
-            const int64_t some = std::min<int64_t>(batch - b, 65535), r = b * tokens;
+        constexpr int HD = decltype(dim)::value, U = decltype(wide)::value;
+        const int64_t most = 65535 * sequences_beside;
+        for (int64_t b = 0; b < batch; b += most) {     // the grid's second dimension
+            const int64_t some = std::min<int64_t>(batch - b, most), r = b * tokens;
             const auto at = [&](const void* x, int64_t heads) { return (uint16_t*)x + r * heads * HD; };
-            qkv_norm_rope_kernel<T, HD, TOKENS><<<dim3((unsigned)cdiv(tokens, TOKENS), (unsigned)some), dim3((unsigned)lanes), 0, st>>>(
+            qkv_norm_rope_kernel<T, HD, U><<<dim3((unsigned)cdiv(tokens, tokens_beside), (unsigned)cdiv(some, sequences_beside), (unsigned)shares),
+                                             dim3((unsigned)lanes, (unsigned)(tokens_beside * sequences_beside)), 0, st>>>(
                 at(q, num_heads), at(k, num_kv_heads), at(v, num_kv_heads), (const uint16_t*)q_weight, (const uint16_t*)k_weight, cos_sin,
                 positions + (per_sequence ? r : 0), per_sequence != 0, at(q_out, num_heads), at(k_out, num_kv_heads), at(v_out, num_kv_heads),
-                (int)tokens, (int)num_heads, (int)num_kv_heads, max_positions, q_eps, k_eps);
+                (int)some, (int)tokens, (int)num_heads, (int)num_kv_heads, beside_tokens, max_positions, q_eps, k_eps);
         }
     };
-    const auto of = [&](auto type, auto each) {
-        if (head_dim == 64) go(type, std::integral_constant<int, 64>{}, each);
-        else if (head_dim == 128) go(type, std::integral_constant<int, 128>{}, each);
-        else go(type, std::integral_constant<int, 256>{}, each);
+    const auto of = [&](auto type, auto wide) {
+        if (head_dim == 64) go(type, std::integral_constant<int, 64>{}, wide);
+        else if (head_dim == 128) go(type, std::integral_constant<int, 128>{}, wide);
+        else go(type, std::integral_constant<int, 256>{}, wide);
     };
-    const auto with = [&](auto each) { dtype == AWQ_F16 ? of(F16{}, each) : of(BF16{}, each); };
-    // several tokens a workgroup where the chip has more waves than it holds at a time all the same
-    if (cdiv(batch * tokens, 4) * (lanes / 64) >= 8192) with(std::integral_constant<int, 4>{});
-    else with(std::integral_constant<int, 1>{});
+    const auto with = [&](auto wide) { dtype == AWQ_F16 ? of(F16{}, wide) : of(BF16{}, wide); };
+    if (few || small) with(std::integral_constant<int, 1>{});
+    else with(std::integral_constant<int, 2>{});
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);
 }

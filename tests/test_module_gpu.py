@@ -278,6 +278,10 @@ def test_prompt_forward_of_many_tiles(monkeypatch):
     (2, 4099, 24, 8, 128),        # four tokens a workgroup, the last one with three
     (5, 3301, 5, 1, 64),          # an odd head count
     (2, 2050, 40, 8, 256),        # several passes over the heads
+    (1, 67, 37, 5, 128),          # fewer waves than the chip holds: heads over workgroups, the last one part full
+    (1, 3, 4, 1, 64), (2, 4097, 4, 1, 64), (1, 2, 1, 1, 256),      # a wave has lanes for all heads: five tokens a workgroup, or the sequences there are
+    (4098, 1, 4, 1, 64), (513, 3, 1, 1, 128),      # sequences beside one another
+    (65537, 1, 5, 1, 128),        # more sequences than the grid's second dimension holds
 ])
 def test_qkv_norm_rope_sizes(dtype, batch, tokens, heads, kv, dim):
     """Head counts and tokens around the kernel's groups, passes and tokens a workgroup, positions per sequence, against the torch expressions in fp32 with
