@@ -469,6 +469,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     constexpr int LPT = HD / 8;    // lanes per token
     constexpr int TPW = 64 / LPT;  // tokens per wave step
     constexpr int U = 2;           // token steps in flight
+    constexpr bool kEarly = G == 4;   // block numbers of the first step beside the context length
     const int sp = blockIdx.x % nsplit;
     const int kvh = (blockIdx.x / nsplit) % nkv;
     const int b = blockIdx.x / (nsplit * nkv);
@@ -476,11 +477,13 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int dc = lane % LPT, ts = lane / LPT;
 
-    // the first step's block numbers are asked for beside the context length where they don't hang on it: one trip to memory less before the
-    // first keys
+    // With four heads the first step's block numbers are asked for beside the context length where they don't hang on it: one trip to memory less before
+    // the first keys, and registers that the compiler lays out better (us, blocks of 24 tokens, asked for step by step / so: 16 x 300 tokens of heads of
+    // 128 21.1 / 18.3, 64 x 1300 119 / 88; heads of 64 24 x 4000 88 / 65).  Eight heads lose a fifth by it (heads of 64 31 x 4000 130 / 163, heads of 128 1 x
+    // 140 17.6 / 22.4), one and two a twentieth up to 140 tokens (4.8 / 5.0, 7.2 / 7.6).
     const int32_t* table = block_table + (int64_t)b * max_blocks;
     int blocks[U], blocks0 = 0;
-    if (nsplit == 1) {
+    if (kEarly && nsplit == 1) {
         blocks0 = table[0];
 #pragma unroll
         for (int u = 0; u < U; ++u) blocks[u] = table[min((wave * TPW + ts + u * WAVES * TPW) / block_size, max_blocks - 1)];
@@ -514,7 +517,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
             const int tt = t + u * WAVES * TPW;
             ok[u] = tt < t1;
             const int tc = ok[u] ? tt : t0;
-            int blk = nsplit == 1 && t < WAVES * TPW * U ? (ok[u] ? blocks[u] : blocks0) : table[tc / block_size];
+            int blk = kEarly && nsplit == 1 && t < WAVES * TPW * U ? (ok[u] ? blocks[u] : blocks0) : table[tc / block_size];
             blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
             const int64_t off = (((int64_t)blk * nkv + kvh) * block_size + tc % block_size) * HD + dc * 8;
             kr[u] = *reinterpret_cast<const u32x4*>(k_cache + off);
@@ -1002,24 +1005,25 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_tr_kernel(
 }
 
 // Merge of the context splits: one workgroup of HD threads per (sequence, query head).
-template <typename T, int HD>
+// MOST: at least their number (31 sequences x 64 heads of two parts: the whole call 29.3 us with four parts' values in registers, 30.5 with 16).
+template <typename T, int HD, int MOST>
 __global__ __launch_bounds__(HD) void paged_attn_merge_kernel(const float* __restrict__ partial,
                                                               uint16_t* __restrict__ out, int nsplit, int heads) {
     const float* src = partial + (int64_t)blockIdx.x * nsplit * (HD + 2);
     const int d = threadIdx.x;
     // every part's values are asked for before the first is used: one trip to memory whatever their number
-    float m[kMaxSplits], l[kMaxSplits], v[kMaxSplits];
+    float m[MOST], l[MOST], v[MOST];
 #pragma unroll
-    for (int s = 0; s < kMaxSplits; ++s) {
+    for (int s = 0; s < MOST; ++s) {
         const float* p = src + (s < nsplit ? s : 0) * (HD + 2);
         m[s] = p[HD], l[s] = p[HD + 1], v[s] = p[d];
     }
     float mn = kNegBig;
 #pragma unroll
-    for (int s = 0; s < kMaxSplits; ++s) mn = s < nsplit ? fmaxf(mn, m[s]) : mn;
+    for (int s = 0; s < MOST; ++s) mn = s < nsplit ? fmaxf(mn, m[s]) : mn;
     float lt = 0.f, at = 0.f;
 #pragma unroll
-    for (int s = 0; s < kMaxSplits; ++s) {
+    for (int s = 0; s < MOST; ++s) {
         const float c = exp2f(m[s] - mn);
         lt = s < nsplit ? lt + l[s] * c : lt;
         at = s < nsplit ? at + v[s] * c : at;
@@ -1150,6 +1154,12 @@ int pick_splits(int64_t batch, int64_t nkv, int64_t max_context, int G, bool tr)
     return best;
 }
 
+template <typename T, int HD>
+void launch_merge(const float* partial, void* out, int nsplit, int64_t rows, int heads, hipStream_t st) {
+    const auto kernel = nsplit <= 4 ? paged_attn_merge_kernel<T, HD, 4> : paged_attn_merge_kernel<T, HD, kMaxSplits>;
+    kernel<<<dim3((unsigned)rows), dim3(HD), 0, st>>>(partial, (uint16_t*)out, nsplit, heads);
+}
+
 template <typename T, int G, int HD>
 void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* table, const int32_t* ctx, void* out,
                  float* partial, int64_t batch, int nkv, int bs, int max_blocks, int num_blocks, int nsplit,
@@ -1161,8 +1171,7 @@ void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* t
                 (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv,
                 bs, max_blocks, num_blocks, nsplit, scale, G);
             if (nsplit > 1)
-                paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(
-                    partial, (uint16_t*)out, nsplit, 0);
+                launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, 0, st);
             return;
         }
     }
@@ -1181,8 +1190,7 @@ void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* t
             if (batch * nkv > 256) go(std::integral_constant<int, 4>{});
             else go(std::integral_constant<int, 8>{});
             if (nsplit > 1)
-                paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(
-                    partial, (uint16_t*)out, nsplit, tiled ? nkv * G : 0);
+                launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, tiled ? nkv * G : 0, st);
             return;
         }
     }
@@ -1190,8 +1198,7 @@ void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* t
         (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv, bs,
         max_blocks, num_blocks, nsplit, scale, tiled);
     if (nsplit > 1)
-        paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(partial, (uint16_t*)out,
-                                                                                               nsplit, tiled ? nkv * G : 0);
+        launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, tiled ? nkv * G : 0, st);
 }
 
 template <typename T, int HD>
@@ -1213,8 +1220,7 @@ int launch_attn_g(int G, const void* q, const void* kc, const void* vc, const in
                 (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv,
                 bs, max_blocks, num_blocks, nsplit, scale, G);
             if (nsplit > 1)
-                paged_attn_merge_kernel<T, HD><<<dim3((unsigned)(batch * nkv * G)), dim3(HD), 0, st>>>(
-                    partial, (uint16_t*)out, nsplit, 0);
+                launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, 0, st);
             return AWQ_OK;
         }
     }
