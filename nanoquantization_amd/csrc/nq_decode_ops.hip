@@ -601,7 +601,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     }
 }
 
-// The same for 2, 4 or 8 query heads per kv head and 128 head dims, where the kernel above is bound by its
+// The same for 2 or 4 query heads per kv head and 128 head dims, where the kernel above is bound by its
 // vector-ALU dot products (8 FMAs, 4 shuffles and an online-softmax update per token, head and lane).
 // A wave takes tiles of 16 tokens.  Scores: S^T = K q^T on the 16x16x32 MFMA (A = 16 token rows of K, 32 head dims
 // per instruction; B = the G query heads as columns, the rest zero), so a lane ends up with 4 tokens of one head and
@@ -615,9 +615,10 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
 // more; and the workgroup's context is its share of 16 MB or more).  bf16, 8 kv heads, us, 28 layers' caches in turn; two heads, the vector kernel / this one:
 // 1 x 1300 14.0 / 8.2, 8 x 320 11.2 / 7.8, 12 x 640 21.7 / 13.6, 32 x 640 21.0 / 16.5,
 // 64 x 640 38 / 28.4, 64 x 1000 63.5 / 44.7 = 5.9 TB/s, 1 x 8000 24.9 / 14.7.  Four heads, this one with a tile
-// behind its block number / now: 1 x 1300 13.5 / 8.7, 24 x 640 19.8 / 16.7, 32 x 640 20.2 / 18.2, 64 x 1000 52.4 / 44.9, 1 x 140 5.6 / 5.9.  Through the L2 32 x 640 takes 19.2 and
+// behind its block number / now: 1 x 1300 13.5 / 8.7, 24 x 640 19.8 / 16.7, 32 x 640 20.2 / 18.2, 64 x 1000 52.4 / 44.9, 1 x 140 5.75 / 5.9.  Through the L2 32 x 640 takes 19.2 and
 // 64 x 1000 50; part rounds and smaller caches are better off there (20 x 640 13.2, past it 14.3; 8 x 140 5.6, 6.2).  Two or more tiles on their way in a
-// wave's registers take longer at every size (32 x 640 19.2 with two, 20.0 with four).
+// wave's registers take longer at every size (32 x 640 19.2 with two, 20.0 with four).  The last tile stands behind the loop, which asks for no tile that
+// is not there: a workgroup waits for such loads before it adds its waves' sums (four heads, 32 x 64 6.1 -> 5.8 us, 24 x 300 10.8 -> 10.1, 64 x 140 11.8 -> 11.3).
 template <typename T, int G, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
@@ -637,8 +638,9 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
     const int32_t* table = block_table + (int64_t)b * max_blocks;
     // blocks of the wave's tiles first, first + 1, .., one a lane
     const auto blocks_from = [&](int t0, int first) {
-        const int64_t t = t0 + ((int64_t)(first + lane) * WAVES + wave) * TT, last = (int64_t)max_blocks * block_size - 1;
-        return table[(uint32_t)min(t, last) / (uint32_t)block_size];
+        // (a context is below 2^31, and the last of 64 tiles lies less than 2^14 behind its end)
+        const uint32_t t = (uint32_t)t0 + ((uint32_t)(first + lane) * WAVES + wave) * TT, last = (uint32_t)max_blocks * block_size - 1;
+        return table[min(t, last) / (uint32_t)block_size];
     };
     int blocks = nsplit == 1 ? blocks_from(0, 0) : 0;     // asked for beside the context length
     int ctx = context_lens[b];
@@ -663,15 +665,15 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
     u32x4 ka[4], va[4];
     const auto load = [&](int tile, auto policy) __attribute__((always_inline)) {
         constexpr int kPolicy = decltype(policy)::value;
-        if (tile - held >= 64 && tile < tiles) {
+        if (tile - held >= 64) {
             held = tile;
             blocks = blocks_from(t0, held);
         }
         int blk = __builtin_amdgcn_readlane(blocks, (tile - held) & 63);
         blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
         const int tb = t0 + (tile * WAVES + wave) * TT;
-        const uint32_t bytes = tile < tiles ? (uint32_t)min(TT, t1 - tb) * (HD * 2) : 0u;
-        const int64_t base = tile < tiles ? (((int64_t)blk * nkv + kvh) * block_size + tb % block_size) * HD : 0;
+        const uint32_t bytes = (uint32_t)min(TT, t1 - tb) * (HD * 2);
+        const int64_t base = (((int64_t)blk * nkv + kvh) * block_size + (uint32_t)tb % (uint32_t)block_size) * HD;
         const __amdgpu_buffer_rsrc_t k = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(k_cache + base), 0, bytes, 0x00020000);
         const __amdgpu_buffer_rsrc_t v = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(v_cache + base), 0, bytes, 0x00020000);
 #pragma unroll
@@ -741,14 +743,17 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         asm volatile("" ::: "memory");
     };
     const auto walk = [&](auto policy) {
-        load(0, policy);
-        for (int tile = 0; tile < tiles; ++tile) {
+        for (int tile = 0; tile + 1 < tiles; ++tile) {
             take(tile);
             load(tile + 1, policy);     // (behind a condition the loop takes half as long again, 32 x 640 25.1 us)
         }
     };
-    if (full && (int64_t)(t1 - t0) * gridDim.x >= 32768) walk(std::integral_constant<int, 2>{});      // nt
-    else walk(std::integral_constant<int, 0>{});
+    if (tiles) {
+        load(0, std::integral_constant<int, 0>{});
+        if (full && (int64_t)(t1 - t0) * gridDim.x >= 32768) walk(std::integral_constant<int, 2>{});      // nt
+        else walk(std::integral_constant<int, 0>{});
+        take(tiles - 1);
+    }
 
     // the four token groups of the wave share m: their accumulators and partial sums just add
 #pragma unroll
