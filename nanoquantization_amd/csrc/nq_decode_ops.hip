@@ -451,7 +451,7 @@ __global__ __launch_bounds__(512) void qkv_norm_rope_kernel(const uint16_t* __re
 
 // ---------------------------------------------------------------------------------------------
 // Attention of one new token per sequence over its paged KV cache (flash-decoding).
-// Workgroup = (sequence, kv head, context split), WAVES waves (16 for up to 2 query heads per kv head, 8 for
+// Workgroup = (sequence, kv head, context split), WAVES waves (here 16 for up to 2 query heads per kv head, 8 for
 // 4, 4 for 8: the wave merge buffer grows with G); with enough waves per workgroup a batch of sequences
 // needs no context split and no second kernel.  A wave covers TPW = 64 / (HD/8) tokens
 // per step: a lane holds 8 head dims of one token's K and V rows (one 16-byte load each), the G
@@ -460,19 +460,24 @@ __global__ __launch_bounds__(512) void qkv_norm_rope_kernel(const uint16_t* __re
 // groups, then waves (LDS), then splits (fp32 partials + a second kernel).
 constexpr float kNegBig = -3.0e38f;
 constexpr int kMaxSplits = 16;
+// Context splits of a (sequence, kv head) pair: workgroups are launched for `most`, split by split; a sequence of fewer than `from` tokens lies in the
+// first `few`, and the workgroups of the others are done at once.
+struct Splits {
+    int pairs, most, few, from;
+    __device__ __forceinline__ int of(int context) const { return context >= from ? most : few; }
+};
 
 template <typename T, int G, int HD, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, uint16_t* __restrict__ out,
-    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, int nsplit, float scale, int tiled) {
+    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, Splits splits, float scale, int tiled) {
     constexpr int LPT = HD / 8;    // lanes per token
     constexpr int TPW = 64 / LPT;  // tokens per wave step
     constexpr int U = 2;           // token steps in flight
     constexpr bool kEarly = G == 4;   // block numbers of the first step beside the context length
-    const int sp = blockIdx.x % nsplit;
-    const int kvh = (blockIdx.x / nsplit) % nkv;
-    const int b = blockIdx.x / (nsplit * nkv);
+    const int sp = blockIdx.x / (uint32_t)splits.pairs, pair = blockIdx.x % (uint32_t)splits.pairs;
+    const int kvh = pair % (uint32_t)nkv, b = pair / (uint32_t)nkv;
     const int nh = nkv * G;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int dc = lane % LPT, ts = lane / LPT;
@@ -483,13 +488,15 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
     // 140 17.6 / 22.4), one and two a twentieth up to 140 tokens (4.8 / 5.0, 7.2 / 7.6).
     const int32_t* table = block_table + (int64_t)b * max_blocks;
     int blocks[U], blocks0 = 0;
-    if (kEarly && nsplit == 1) {
+    if (kEarly && splits.most == 1) {
         blocks0 = table[0];
 #pragma unroll
         for (int u = 0; u < U; ++u) blocks[u] = table[min((wave * TPW + ts + u * WAVES * TPW) / block_size, max_blocks - 1)];
     }
     int ctx = context_lens[b];
     ctx = ctx < 0 ? 0 : (ctx > max_blocks * block_size ? max_blocks * block_size : ctx);
+    const int nsplit = splits.of(ctx);
+    if (sp >= nsplit) return;
     const int per = (ctx + nsplit - 1) / nsplit;
     const int t0 = sp * per, t1 = min(ctx, t0 + per);
 
@@ -517,7 +524,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
             const int tt = t + u * WAVES * TPW;
             ok[u] = tt < t1;
             const int tc = ok[u] ? tt : t0;
-            int blk = kEarly && nsplit == 1 && t < WAVES * TPW * U ? (ok[u] ? blocks[u] : blocks0) : table[tc / block_size];
+            int blk = kEarly && splits.most == 1 && t < WAVES * TPW * U ? (ok[u] ? blocks[u] : blocks0) : table[tc / block_size];
             blk = blk < 0 ? 0 : (blk >= num_blocks ? num_blocks - 1 : blk);
             const int64_t off = (((int64_t)blk * nkv + kvh) * block_size + tc % block_size) * HD + dc * 8;
             kr[u] = *reinterpret_cast<const u32x4*>(k_cache + off);
@@ -591,7 +598,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_kernel(
         if (nsplit == 1) {
             out[tiled ? tiled_at(b, (kvh * G + g) * HD + d, nh * HD) / 2 : head * HD + d] = T::from_f32(lt > 0.f ? at / lt : 0.f);
         } else {
-            float* dst = partial + (head * nsplit + sp) * (HD + 2);
+            float* dst = partial + (head * splits.most + sp) * (HD + 2);
             dst[d] = at;
             if (d == 0) {
                 dst[HD] = mn;
@@ -623,14 +630,13 @@ template <typename T, int G, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, const int32_t* __restrict__ context_lens, uint16_t* __restrict__ out,
-    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, int nsplit, float scale, int tiled,
+    float* __restrict__ partial, int nkv, int block_size, int max_blocks, int num_blocks, Splits splits, float scale, int tiled,
     int full) {
     constexpr int HD = 128, TT = 16;
     static_assert(G == 2 || G == 4, "query heads per kv head");
     typedef float fG __attribute__((ext_vector_type(G)));
-    const int sp = blockIdx.x % nsplit;
-    const int kvh = (blockIdx.x / nsplit) % nkv;
-    const int b = blockIdx.x / (nsplit * nkv);
+    const int sp = blockIdx.x / (uint32_t)splits.pairs, pair = blockIdx.x % (uint32_t)splits.pairs;
+    const int kvh = pair % (uint32_t)nkv, b = pair / (uint32_t)nkv;
     const int nh = nkv * G;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lo = lane & 15, hi = lane >> 4;   // score phase: head lo, token quad hi; value phase: dims 8*lo.., token hi
@@ -642,7 +648,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         const uint32_t t = (uint32_t)t0 + ((uint32_t)(first + lane) * WAVES + wave) * TT, last = (uint32_t)max_blocks * block_size - 1;
         return table[min(t, last) / (uint32_t)block_size];
     };
-    int blocks = nsplit == 1 ? blocks_from(0, 0) : 0;     // asked for beside the context length
+    int blocks = splits.most == 1 ? blocks_from(0, 0) : 0;     // asked for beside the context length
     int ctx = context_lens[b];
     u32x4 bq[4];
 #pragma unroll
@@ -652,10 +658,12 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
             bq[i] = *reinterpret_cast<const u32x4*>(q + ((int64_t)b * nh + kvh * G + lo) * HD + 32 * i + 8 * hi);
     }
     ctx = ctx < 0 ? 0 : (ctx > max_blocks * block_size ? max_blocks * block_size : ctx);
+    const int nsplit = splits.of(ctx);
+    if (sp >= nsplit) return;
     const int per = nsplit == 1 ? ctx : ((ctx + nsplit - 1) / nsplit + TT - 1) / TT * TT;
     const int t0 = sp * per, t1 = min(ctx, t0 + per);
     const int tiles = t1 - t0 > wave * TT ? (t1 - t0 - wave * TT + WAVES * TT - 1) / (WAVES * TT) : 0;
-    if (nsplit > 1) blocks = blocks_from(t0, 0);
+    if (splits.most > 1) blocks = blocks_from(t0, 0);
     int held = 0;
 
     __shared__ __align__(16) float s_p[WAVES][TT * G + G];   // per wave: p[token][head], then the rescale factor per head
@@ -750,7 +758,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
     };
     if (tiles) {
         load(0, std::integral_constant<int, 0>{});
-        if (full && (int64_t)(t1 - t0) * gridDim.x >= 32768) walk(std::integral_constant<int, 2>{});      // nt
+        if ((full >> (nsplit < splits.most) & 1) && (int64_t)(t1 - t0) * splits.pairs * nsplit >= 32768) walk(std::integral_constant<int, 2>{});      // nt
         else walk(std::integral_constant<int, 0>{});
         take(tiles - 1);
     }
@@ -792,7 +800,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_mfma_kernel(
         if (nsplit == 1) {
             out[tiled ? tiled_at(b, (kvh * G + g) * HD + d, nh * HD) / 2 : head * HD + d] = T::from_f32(lt > 0.f ? at / lt : 0.f);
         } else {
-            float* dst = partial + (head * nsplit + sp) * (HD + 2);
+            float* dst = partial + (head * splits.most + sp) * (HD + 2);
             dst[d] = at;
             if (d == 0) {
                 dst[HD] = mn;
@@ -1013,16 +1021,18 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attn_decode_tr_kernel(
 // MOST: at least their number (31 sequences x 64 heads of two parts: the whole call 29.3 us with four parts' values in registers, 30.5 with 16).
 template <typename T, int HD, int MOST>
 __global__ __launch_bounds__(HD) void paged_attn_merge_kernel(const float* __restrict__ partial,
-                                                              uint16_t* __restrict__ out, int nsplit, int heads) {
-    const float* src = partial + (int64_t)blockIdx.x * nsplit * (HD + 2);
-    const int d = threadIdx.x;
+                                                              const int32_t* __restrict__ context_lens, uint16_t* __restrict__ out,
+                                                              Splits splits, int heads, int tiled) {
+    const int b = blockIdx.x / heads, d = threadIdx.x, nsplit = splits.of(context_lens[b]);
+    const float* src = partial + (int64_t)blockIdx.x * splits.most * (HD + 2);
     // every part's values are asked for before the first is used: one trip to memory whatever their number
     float m[MOST], l[MOST], v[MOST];
 #pragma unroll
     for (int s = 0; s < MOST; ++s) {
-        const float* p = src + (s < nsplit ? s : 0) * (HD + 2);
+        const float* p = src + (s < splits.most ? s : 0) * (HD + 2);
         m[s] = p[HD], l[s] = p[HD + 1], v[s] = p[d];
     }
+    if (nsplit == 1) return;        // that workgroup has written the result
     float mn = kNegBig;
 #pragma unroll
     for (int s = 0; s < MOST; ++s) mn = s < nsplit ? fmaxf(mn, m[s]) : mn;
@@ -1034,7 +1044,7 @@ __global__ __launch_bounds__(HD) void paged_attn_merge_kernel(const float* __res
         at = s < nsplit ? at + v[s] * c : at;
     }
     const int64_t at_row = (int64_t)blockIdx.x * HD + d;
-    out[heads ? tiled_at((int)(blockIdx.x / heads), (int)(blockIdx.x % heads) * HD + d, heads * HD) / 2 : at_row] = T::from_f32(lt > 0.f ? at / lt : 0.f);
+    out[tiled ? tiled_at(b, (int)(blockIdx.x % heads) * HD + d, heads * HD) / 2 : at_row] = T::from_f32(lt > 0.f ? at / lt : 0.f);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1134,19 +1144,24 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 bool attn_tr(int G, int64_t head_dim, int64_t block_size) {
     return (G == 8 || (G != 1 && G != 2 && G != 4 && G >= 1 && G <= 16)) && head_dim == 128 && block_size % 16 == 0;
 }
+// the vector kernel's waves, and those of the kernel with both products on the matrix cores (two and four heads on the matrix cores: launch_attn)
 int attn_waves(int G, bool tr) { return tr ? 4 : (G <= 2 ? 16 : (G <= 4 ? 8 : 4)); }
 
 // Context splits of a (sequence, kv head) pair. A launch lasts as long as the CU with the most workgroups, each of its workgroups costs what 250 tokens
 // cost beside the tokens of its split, and the merge what 400 do: the split count with the smallest such sum. Over batches of 1 to 31, contexts of 140 to
 // 8000 tokens and two or four heads per kv head (8 kv heads, bf16) it is 0.3 % from the best of eight counts on average. 256 pairs or more are not split.
-// Four-wave workgroups (the matrix-core kernel's, and eight heads per kv head without it) run best at about 2048 waves on the chip with 128 tokens or more per split (64 sequences x 8
-// kv heads x 2060 tokens at 8 heads per kv head 124 us in two splits + merge, 105 unsplit).
-int pick_splits(int64_t batch, int64_t nkv, int64_t max_context, int G, bool tr) {
+// The host knows the table's length and not the contexts.  Several rounds of workgroups pay near that length alone, so that sequences shorter
+// than where the sums meet keep to one round (four heads, 24 sequences with a table of 4096 tokens, at 64 / 300 / 900 / 4000 tokens: four splits, three
+// rounds, 15.5, 20.2, 29.9, 76 us; two, as a rule of waves on the chip has it, 10.0, 14.4, 26.3, 87; now 8.2, 11.4, 22.7, 75).
+// Four-wave workgroups (eight heads per kv head, with or without the matrix cores) run best at about 2048 waves on the chip with 128 tokens or more per
+// split (64 sequences x 8 kv heads x 2060 tokens at 8 heads per kv head 124 us in two splits + merge, 105 unsplit).
+Splits pick_splits(int64_t batch, int64_t nkv, int64_t max_context, int G, bool tr) {
     const int64_t pairs = batch * nkv, waves = attn_waves(G, tr);
     if (waves == 4) {
         const int64_t s = cdiv(2048, pairs * waves), cap = max_context / 128 > 1 ? max_context / 128 : 1;
         const int64_t m = s < cap ? s : cap;
-        return (int)(m > kMaxSplits ? kMaxSplits : (m < 1 ? 1 : m));
+        const int n = (int)(m > kMaxSplits ? kMaxSplits : (m < 1 ? 1 : m));
+        return Splits{(int)pairs, n, n, 0};
     }
     int best = 1;
     if (pairs < 256) {
@@ -1156,27 +1171,31 @@ int pick_splits(int64_t batch, int64_t nkv, int64_t max_context, int G, bool tr)
             if (cost < least) least = cost, best = s;
         }
     }
-    return best;
+    const int one = (int)std::max<int64_t>(1, std::min<int64_t>(best, 256 / pairs));
+    if (one == best) return Splits{(int)pairs, best, best, 0};
+    const double rounds = (double)cdiv(pairs * best, 256), gain = 1.0 / one - rounds / best;     // a token
+    const double from = gain > 0 ? ((rounds - 1) * 250 + (one == 1 ? 400 : 0)) / gain : (double)max_context;
+    return Splits{(int)pairs, best, one, (int)std::min(from + 1, (double)max_context)};
 }
 
 template <typename T, int HD>
-void launch_merge(const float* partial, void* out, int nsplit, int64_t rows, int heads, hipStream_t st) {
-    const auto kernel = nsplit <= 4 ? paged_attn_merge_kernel<T, HD, 4> : paged_attn_merge_kernel<T, HD, kMaxSplits>;
-    kernel<<<dim3((unsigned)rows), dim3(HD), 0, st>>>(partial, (uint16_t*)out, nsplit, heads);
+void launch_merge(const float* partial, const int32_t* ctx, void* out, Splits splits, int64_t batch, int heads, int tiled, hipStream_t st) {
+    if (splits.most == 1) return;
+    const auto kernel = splits.most <= 4 ? paged_attn_merge_kernel<T, HD, 4> : paged_attn_merge_kernel<T, HD, kMaxSplits>;
+    kernel<<<dim3((unsigned)(batch * heads)), dim3(HD), 0, st>>>(partial, ctx, (uint16_t*)out, splits, heads, tiled);
 }
 
 template <typename T, int G, int HD>
 void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* table, const int32_t* ctx, void* out,
-                 float* partial, int64_t batch, int nkv, int bs, int max_blocks, int num_blocks, int nsplit,
+                 float* partial, int64_t batch, int nkv, int bs, int max_blocks, int num_blocks, Splits splits,
                  float scale, int tiled, hipStream_t st) {
     constexpr int WAVES = G <= 2 ? 16 : (G <= 4 ? 8 : 4);
     if constexpr (HD == 128 && G == 8) {
         if (attn_tr(G, HD, bs)) {
-            paged_attn_decode_tr_kernel<T, G, 4><<<dim3((unsigned)(batch * nkv * nsplit)), dim3(256), 0, st>>>(
+            paged_attn_decode_tr_kernel<T, G, 4><<<dim3((unsigned)(batch * nkv * splits.most)), dim3(256), 0, st>>>(
                 (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv,
-                bs, max_blocks, num_blocks, nsplit, scale, G);
-            if (nsplit > 1)
-                launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, 0, st);
+                bs, max_blocks, num_blocks, splits.most, scale, G);
+            launch_merge<T, HD>(partial, ctx, out, splits, batch, nkv * G, 0, st);
             return;
         }
     }
@@ -1184,48 +1203,46 @@ void launch_attn(const void* q, const void* kc, const void* vc, const int32_t* t
         if (bs % 16 == 0) {
             // a CU holds one workgroup of eight waves or, where there are more than CUs, several of four, whose last round is shorter (two heads, 40 x
             // 640 tokens 23.9 us, 26.2 with eight; four heads, 64 x 640 29.5, 32.5; 24 x 640 14.9, 17.1 with four)
-            const int64_t groups = batch * nkv * nsplit;
-            const int full = groups * 4 >= cdiv(groups, 256) * 256 * 3;
+            const int64_t groups = batch * nkv * splits.most;
+            const auto fills = [](int64_t n) { return n * 4 >= cdiv(n, 256) * 256 * 3; };
+            const int full = fills(groups) | fills(batch * nkv * splits.few) << 1;
             const auto go = [&](auto waves) {
                 constexpr int W = decltype(waves)::value;
                 paged_attn_decode_mfma_kernel<T, G, W><<<dim3((unsigned)groups), dim3(64 * W), 0, st>>>(
                     (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv, bs, max_blocks,
-                    num_blocks, nsplit, scale, tiled, full);
+                    num_blocks, splits, scale, tiled, full);
             };
             if (batch * nkv > 256) go(std::integral_constant<int, 4>{});
             else go(std::integral_constant<int, 8>{});
-            if (nsplit > 1)
-                launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, tiled ? nkv * G : 0, st);
+            launch_merge<T, HD>(partial, ctx, out, splits, batch, nkv * G, tiled, st);
             return;
         }
     }
-    paged_attn_decode_kernel<T, G, HD, WAVES><<<dim3((unsigned)(batch * nkv * nsplit)), dim3(64 * WAVES), 0, st>>>(
+    paged_attn_decode_kernel<T, G, HD, WAVES><<<dim3((unsigned)(batch * nkv * splits.most)), dim3(64 * WAVES), 0, st>>>(
         (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv, bs,
-        max_blocks, num_blocks, nsplit, scale, tiled);
-    if (nsplit > 1)
-        launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, tiled ? nkv * G : 0, st);
+        max_blocks, num_blocks, splits, scale, tiled);
+    launch_merge<T, HD>(partial, ctx, out, splits, batch, nkv * G, tiled, st);
 }
 
 template <typename T, int HD>
 int launch_attn_g(int G, const void* q, const void* kc, const void* vc, const int32_t* table, const int32_t* ctx,
                   void* out, float* partial, int64_t batch, int nkv, int bs, int max_blocks, int num_blocks,
-                  int nsplit, float scale, int tiled, hipStream_t st) {
+                  Splits splits, float scale, int tiled, hipStream_t st) {
     switch (G) {
 #define NQ_CASE(g)                                                                                              \
     case g:                                                                                                     \
         launch_attn<T, g, HD>(q, kc, vc, table, ctx, out, partial, batch, nkv, bs, max_blocks, num_blocks,      \
-                              nsplit, scale, tiled, st);                                                        \
+                              splits, scale, tiled, st);                                                        \
         return AWQ_OK;
         NQ_CASE(1) NQ_CASE(2) NQ_CASE(4) NQ_CASE(8)
 #undef NQ_CASE
     }
     if constexpr (HD == 128) {
         if (attn_tr(G, HD, bs)) {   // any other ratio up to 16: the matrix-core kernel with the count at run time
-            paged_attn_decode_tr_kernel<T, 0, 4><<<dim3((unsigned)(batch * nkv * nsplit)), dim3(256), 0, st>>>(
+            paged_attn_decode_tr_kernel<T, 0, 4><<<dim3((unsigned)(batch * nkv * splits.most)), dim3(256), 0, st>>>(
                 (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, table, ctx, (uint16_t*)out, partial, nkv,
-                bs, max_blocks, num_blocks, nsplit, scale, G);
-            if (nsplit > 1)
-                launch_merge<T, HD>(partial, out, nsplit, batch * nkv * G, 0, st);
+                bs, max_blocks, num_blocks, splits.most, scale, G);
+            launch_merge<T, HD>(partial, ctx, out, splits, batch, nkv * G, 0, st);
             return AWQ_OK;
         }
     }
@@ -1382,8 +1399,8 @@ extern "C" size_t nq_paged_attention_workspace_bytes(int64_t batch, int64_t num_
     if (batch <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || max_context <= 0) return 0;
     // the block size decides the kernel and with it the split count: room for either
     const int G = (int)(num_heads / num_kv_heads);
-    int s = pick_splits(batch, num_kv_heads, max_context, G, false);
-    if (attn_tr(G, head_dim, 32)) s = std::max(s, pick_splits(batch, num_kv_heads, max_context, G, true));
+    int s = pick_splits(batch, num_kv_heads, max_context, G, false).most;
+    if (attn_tr(G, head_dim, 32)) s = std::max(s, pick_splits(batch, num_kv_heads, max_context, G, true).most);
     return s > 1 ? (size_t)(batch * num_heads * s * (head_dim + 2)) * sizeof(float) : 0;
 }
 
@@ -1405,9 +1422,9 @@ static int paged_attention_decode(const char* fn, const void* q, const void* k_c
     const int64_t max_context = block_size * max_blocks_per_seq;
     if (max_context > 0x7fffffff || num_blocks * block_size > 0x7fffffff || batch * num_kv_heads * 16 > 0x7fffffff)
         return bad(fn, "problem too large");
-    const int nsplit = pick_splits(batch, num_kv_heads, max_context, (int)(num_heads / num_kv_heads),
+    const Splits splits = pick_splits(batch, num_kv_heads, max_context, (int)(num_heads / num_kv_heads),
                                    attn_tr((int)(num_heads / num_kv_heads), head_dim, block_size));
-    const size_t need = nsplit > 1 ? (size_t)(batch * num_heads * nsplit * (head_dim + 2)) * sizeof(float) : 0;
+    const size_t need = splits.most > 1 ? (size_t)(batch * num_heads * splits.most * (head_dim + 2)) * sizeof(float) : 0;
     if (need && (!workspace || workspace_bytes < need || !aligned16(workspace))) {
         set_error("%s: workspace of %zu bytes needed, %zu given", fn, need, workspace ? workspace_bytes : (size_t)0);
         return AWQ_ERR_WORKSPACE;
@@ -1420,18 +1437,18 @@ static int paged_attention_decode(const char* fn, const void* q, const void* k_c
         rc = head_dim == 128
                  ? launch_attn_g<F16, 128>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                            batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                           (int)num_blocks, nsplit, scale, tiled, st)
+                                           (int)num_blocks, splits, scale, tiled, st)
                  : launch_attn_g<F16, 64>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                           batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                          (int)num_blocks, nsplit, scale, tiled, st);
+                                          (int)num_blocks, splits, scale, tiled, st);
     else
         rc = head_dim == 128
                  ? launch_attn_g<BF16, 128>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                             batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                            (int)num_blocks, nsplit, scale, tiled, st)
+                                            (int)num_blocks, splits, scale, tiled, st)
                  : launch_attn_g<BF16, 64>(G, q, k_cache, v_cache, block_table, context_lens, out, (float*)workspace,
                                            batch, (int)num_kv_heads, (int)block_size, (int)max_blocks_per_seq,
-                                           (int)num_blocks, nsplit, scale, tiled, st);
+                                           (int)num_blocks, splits, scale, tiled, st);
     if (rc != AWQ_OK) return rc;
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? AWQ_OK : hip_fail(fn, e);

@@ -242,6 +242,44 @@ def test_paged_attention_split_counts(B, nh, nkv, bs, max_blocks):
     assert torch.equal(out, ops.paged_attention_decode(q, kc, vc, table, ctx, scale)), "run-to-run bit-stable"
 
 
+@pytest.mark.parametrize("B,nh,nkv,hd,bs,max_blocks,edge", [
+    (24, 32, 8, 128, 64, 64, 3601),      # four parts from the edge on, one below it
+    (12, 16, 8, 128, 64, 256, 4001),     # eight and two; two heads per kv head
+    (24, 8, 8, 128, 24, 170, 3601),      # the vector kernel, one head
+    (12, 32, 8, 64, 32, 125, 2501),      # and four, heads of 64; five and two
+    (20, 16, 8, 64, 64, 41, 1950),       # three and one
+])
+def test_paged_attention_parts_follow_the_context(B, nh, nkv, hd, bs, max_blocks, edge):
+    """A table for several rounds of workgroups and sequences on both sides of the context from which they pay, beside one another: the parts that
+    a short sequence leaves out are neither written nor read."""
+    from nanoquantization_amd import _lib
+    from nanoquantization_amd.engine import ops
+    g = torch.Generator(device="cuda").manual_seed(B)
+    nb, most = 300, bs * max_blocks
+    kc, vc = (torch.randn(nb, nkv, bs, hd, generator=g, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(B, nh, hd, generator=g, device="cuda").bfloat16()
+    table = torch.randint(0, nb, (B, max_blocks), generator=g, device="cuda").int()
+    ctx = torch.randint(1, most + 1, (B,), generator=g, device="cuda").int()
+    ctx[:8] = torch.tensor([most, edge, edge - 1, edge + 1, 1, 20, 300, edge // 2])
+    want = _attn_ref(q, kc, vc, table, ctx, hd ** -0.5)
+    out = ops.paged_attention_decode(q, kc, vc, table, ctx, hd ** -0.5)
+    _close(out, want, torch.bfloat16, scale=2.0, what="attention")
+    ctx[9] = 0
+    L, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    size = L.nq_paged_attention_workspace_bytes(B, nh, nkv, hd, most)
+    ws = torch.full((size + 4096,), 0xFF, dtype=torch.uint8, device="cuda")        # NaN in every part that nobody writes
+    again = torch.full_like(out, float("nan"))
+    _lib.check(L.nq_paged_attention_decode(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), table.data_ptr(), ctx.data_ptr(), again.data_ptr(), B, nh, nkv, hd,
+                                           bs, max_blocks, nb, hd ** -0.5, _lib.dtype_id(q.dtype), ws.data_ptr(), size, stream))
+    rows = torch.arange(B, device="cuda") != 9
+    assert torch.equal(again[rows], out[rows]) and not again[9].any() and (ws[size:] == 0xFF).all()
+    part = ws[:size].view(torch.float32).view(B, nh, -1, hd + 2)
+    written = (~part.isnan()).any(-1)[:, 0].sum(-1)
+    assert written[0] == written[1] == written[3] == part.shape[2]
+    few = written[2].item()                     # one part writes no sums but the result
+    assert few < part.shape[2] and all(written[i] == few for i in (4, 5, 6, 7))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,nh,nkv,bs,max_blocks", [
     (33, 16, 8, 16, 9),           # four waves a workgroup, two heads per kv head; the smallest block
