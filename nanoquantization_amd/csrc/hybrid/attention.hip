@@ -207,9 +207,11 @@ __device__ __forceinline__ float across_hi(float x) {
 // alone until a score exceeds it by 2^8 saves 4 % of the time, but then the largest probability is no longer 1, which 16 bits
 // hold exactly: the error against 64 bits grows by up to a fifth where few keys dominate.)
 // From the first product of a tile to its last a wave goes before the other workgroup's wave on its SIMD, so that the two fall into different parts
-// of their tiles: 16 heads 4 x 2048 tokens 106 -> 97 us, 1 x 8192 320 -> 285 (0.97 PFLOP/s), 32 heads 1 x 4096 171 -> 160.  With the settling of the
-// maxima too 100, 292, 159; around the value product alone no gain.  Workgroups of up to 1024 keys are level or lose by it (8 x 512 22.9 -> 23.6,
-// 16 x 300 26.2 -> 28.0).
+// of their tiles: 16 heads 4 x 2048 tokens 103 -> 98 us, 8 x 1000 60 -> 56, 1 x 8192 328 -> 304 (0.9 PFLOP/s), 32 heads 1 x 4096 185 -> 164.  With the
+// settling of the maxima too 100, 292, 159 where the products alone had 97, 285, 160; around the value product alone no gain.  Where all workgroups
+// start at once, two a CU, there is nothing to gain, and the one that goes before leaves the other to run alone at the end: up to 640 of them are 1
+// to 7 % slower with it (16 heads 1 x 4096 112 -> 116, heads of 64 76 -> 80), 704 and more up to 14 % faster, on both sides of the line at 1000 to 8192 keys, 8 to
+// 64 heads.  Sequences of up to 512 keys are level or lose up to 7 % (16 x 300 26.2 -> 28.0), from 800 on they gain.
 // What bounds it: per wave and tile of 64 x 128 64 MFMAs (1024 cycles) and some 250 vector instructions, 32 of them 2^x at a
 // quarter of the rate; two waves a SIMD, which is why rows of up to 128 keep within 256 registers (the form before, one wave
 // a SIMD, had 294).  Operands are read a step before they are multiplied; steps are fenced, or the scheduler asks for all of
@@ -217,7 +219,7 @@ __device__ __forceinline__ float across_hi(float x) {
 // 128, causal, forms before / now: 32 heads 4 x 2048 tokens 376 / 204 us, 1 x 8192 1218 / 683 (805 TFLOP/s); 16 heads
 // 16 x 512 70 / 46, 1 x 512 24 / 19.  Rows of 32: 89 / 74, 64: 116 / 93, 96: 230 / 114, 192: 400 / 379, 256: 533 / 490 (4 x
 // 2048, 16 heads); expanded latents of 192 / 128: 450 / 298 with tiles of 32 keys, two waves a SIMD (64 keys, one: 424).
-template <int R, int RV, int KT, bool DENSE, bool EVEN>
+template <int R, int RV, int KT, bool DENSE, bool EVEN, bool FIRST>
 __device__ __forceinline__ void attn_tile(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
@@ -483,7 +485,8 @@ __device__ __forceinline__ void attn_tile(
                 Probs pb;
                 load_keys(buf ^ 1, 0, ka[0]);
                 settle(t, st);
-                if (n_tiles * KT > 1024) __builtin_amdgcn_s_setprio(1);
+                if constexpr (FIRST)        // (dense keys: the host does not know how many)
+                    if (!DENSE || n_tiles * KT > 1024) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int a = 0; a < KT / 16; ++a) {
                     if (a + 1 < KT / 16) load_keys(buf ^ 1, a + 1, ka[(a + 1) & 1]);
@@ -498,7 +501,7 @@ __device__ __forceinline__ void attn_tile(
                     gather(i, va[i & 1], pb);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                __builtin_amdgcn_s_setprio(0);
+                if constexpr (FIRST) __builtin_amdgcn_s_setprio(0);
             } else if (then) {
 #pragma unroll
                 for (int a = 0; a < KT / 16; ++a) {
@@ -574,24 +577,24 @@ __device__ __forceinline__ void attn_tile(
     }
 }
 
-template <int R, int RV, int KT, bool DENSE>
+template <int R, int RV, int KT, bool DENSE, bool FIRST>
 __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
     const uint16_t* __restrict__ sink, DenseKV dense, uint16_t* __restrict__ out, int heads, int kv_heads, int vdim,
     int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles) {
-    attn_tile<R, RV, KT, DENSE, false>(q, k_cache, v_cache, block_tables, segments, tiles, sink, dense, out, heads, kv_heads, vdim,
+    attn_tile<R, RV, KT, DENSE, false, FIRST>(q, k_cache, v_cache, block_tables, segments, tiles, sink, dense, out, heads, kv_heads, vdim,
                                        block_size, max_blocks, num_blocks, chunk, window, scale, q_tiles);
 }
 
 // No sink, chunk or window, but given at run time: with them known the compiler holds more across the key loop than the
 // registers take (rows of 128: 435 spilled, 6x the time).
-template <int R, int KT>
+template <int R, int KT, bool FIRST>
 __global__ __launch_bounds__(256, R > 160 ? 1 : 2) void attn_even_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ sink, uint16_t* __restrict__ out, int heads, int kv_heads, int batch, int tokens, int chunk,
     int window, float scale, int q_tiles) {
-    attn_tile<R, R, KT, false, true>(q, k, v, nullptr, nullptr, nullptr, sink, DenseKV{}, out, heads, kv_heads, R, tokens, 1,
+    attn_tile<R, R, KT, false, true, FIRST>(q, k, v, nullptr, nullptr, nullptr, sink, DenseKV{}, out, heads, kv_heads, R, tokens, 1,
                                      batch, chunk, window, scale, q_tiles);
 }
 
@@ -1019,6 +1022,9 @@ int check_attention(const char* fn, const void* q, const void* k, const void* v,
     return NQH_OK;
 }
 
+// Whether waves may go before one another (attn_tile): more workgroups than start at once, and keys enough.
+bool go_first(int64_t groups, int64_t keys) { return groups > 640 && keys >= 768; }
+
 }  // namespace
 }  // namespace nqh
 
@@ -1046,7 +1052,9 @@ extern "C" int nqh_attention_prefill(const void* q, const void* k_cache, const v
             return fail(NQH_ERR_ARG, fn, "misaligned pointer");
         NQH_WITH_ROW(k_row, {
             constexpr int KT = R >= 192 ? 32 : 64;
-            attn_tile_kernel<R, R, KT, false><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
+            // (the table's length stands in for that of the longest sequence, which is on the device)
+            const bool first = go_first(groups, most_keys(block_size * max_blocks, chunk, window));
+            (first ? attn_tile_kernel<R, R, KT, false, true> : attn_tile_kernel<R, R, KT, false, false>)<<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
                 (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables, segments, tiles,
                 (const uint16_t*)sink, DenseKV{}, (uint16_t*)out, (int)heads, (int)kv_heads, (int)vdim, (int)block_size,
                 (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale, (int)num_tiles);
@@ -1080,9 +1088,10 @@ extern "C" int nqh_causal_attention(const void* q, const void* k, const void* v,
             (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, (uint16_t*)out, (int)heads, (int)kv_heads, (int)batch,
             (int)tokens, 0, 0, scale, (int)num_tiles);
     };
-    if (dim == 64) go(attn_even_kernel<64, 64>);
-    else if (dim == 128) go(attn_even_kernel<128, 64>);
-    else go(attn_even_kernel<256, 32>);
+    const bool first = go_first(groups, tokens);
+    if (dim == 64) go(first ? attn_even_kernel<64, 64, true> : attn_even_kernel<64, 64, false>);
+    else if (dim == 128) go(first ? attn_even_kernel<128, 64, true> : attn_even_kernel<128, 64, false>);
+    else go(attn_even_kernel<256, 32, false>);
     return launched(fn);
 }
 
@@ -1234,7 +1243,8 @@ extern "C" int nqh_latent_attention_prefill(const void* q, const void* kv, int64
     const DenseKV dense{(const uint16_t*)kv, (const uint16_t*)rot, first, kv_stride, rot_stride, heads * dim, (int)dim, (int)rot_dim};
     (void)hipGetLastError();
 #define NQH_GO(R, RV, KT)                                                                                                   \
-    attn_tile_kernel<R, RV, KT, true><<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(                        \
+    (go_first(groups, kMaxI32) ? attn_tile_kernel<R, RV, KT, true, true> : attn_tile_kernel<R, RV, KT, true, false>)<<<    \
+        dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(                                                       \
         (const uint16_t*)q, nullptr, nullptr, nullptr, segments, tiles, nullptr, dense, (uint16_t*)out, (int)heads,          \
         (int)heads, (int)vdim, 1, 0, 0, 0, 0, scale, (int)num_tiles)
     if (row == 64) NQH_GO(64, 64, 64);

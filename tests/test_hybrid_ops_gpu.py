@@ -359,6 +359,42 @@ def test_attention_prefill_tile_edges(dim, block):
             at += n
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("heads", [10, 16])      # 640 workgroups, which all start at once, and more, whose waves go before one another
+def test_prompt_attention_of_many_workgroups(dim, heads):
+    """Dense, paged and latent prompts of many workgroups give the bits of each sequence alone, whichever wave goes first."""
+    gen, bf, dev = torch.Generator(device="cuda").manual_seed(heads), torch.bfloat16, torch.device("cuda")
+    randn = lambda *n: torch.randn(*n, generator=gen, device="cuda").to(bf)
+    G, bs, scale = 2, 64, dim ** -0.5
+    causal = _lib.torch_ops().causal_attention
+    q, k, v = randn(8, 1000, heads, dim), randn(8, G, 1000, dim), randn(8, G, 1000, dim)
+    print(f"many workgroups dim={dim} heads={heads}", flush=True)
+    got = causal(q, k, v, scale)
+    for b in range(8):
+        assert torch.equal(got[b:b + 1], causal(q[b:b + 1], k[b:b + 1], v[b:b + 1], scale)), b
+    # 65 tiles of queries, sequences on both sides of where the host's line for keys and the kernel's for dense keys lie
+    lens = [1500, 1100, 1000, 900, 770, 640, 300, 129, 128, 1200]
+    nb = [-(-n // bs) for n in lens]
+    first = [sum(nb[:i]) for i in range(len(nb))]
+    segs = [(0, n, list(range(f, f + m)), 0) for n, f, m in zip(lens, first, nb)]
+    kc, vc, q = randn(sum(nb), G, bs, dim), randn(sum(nb), G, bs, dim), randn(sum(lens), heads, dim)
+    kv, rot = randn(sum(lens), heads * (dim + 64)), randn(sum(lens), 32)
+    width = _lib.hybrid_lib().nqh_latent_attention_prefill_query_row(dim, 32, 64, 1)
+    ql = torch.zeros(sum(lens), heads, width, dtype=bf, device="cuda")
+    ql[..., :dim + 32] = randn(sum(lens), heads, dim + 32)
+    lay = ops.PromptPass(segs, bs, dev)
+    paged = ops.attention_prefill(q, kc, vc, lay, dim, dim, scale)
+    windowed = ops.attention_prefill(q, kc, vc, lay, dim, dim, scale, window=500)
+    latent = ops.latent_attention_prefill(ql, kv, rot, lay, dim, 64, scale)
+    at = 0
+    for seg in segs:
+        one, part = ops.PromptPass([seg], bs, dev), slice(at, at + seg[1])
+        assert torch.equal(paged[part], ops.attention_prefill(q[part], kc, vc, one, dim, dim, scale)), seg[1]
+        assert torch.equal(windowed[part], ops.attention_prefill(q[part], kc, vc, one, dim, dim, scale, window=500)), seg[1]
+        assert torch.equal(latent[part], ops.latent_attention_prefill(ql[part], kv[part], rot[part], one, dim, 64, scale)), seg[1]
+        at += seg[1]
+
+
 # ---- mixture of experts --------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,width,experts,top,ff", [(1, 72, 5, 2, 48), (37, 64, 9, 1, 40), (20, 128, 7, 7, 64),
