@@ -34,7 +34,7 @@ struct Outputs {
 // 1024 of K 2048 / 3072 with a pass of its own 50.6 / 62.1 us, so 43.0 / 56.1; 8192 x 2560 of K 4096 198 and 180.
 template <typename T, int XR, bool GATED, bool ADD>
 __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ wt,
-                                                       const uint16_t* __restrict__ bias, const uint16_t* __restrict__ residual,
+                                                       const uint16_t* __restrict__ bias, const uint16_t* residual,
                                                        Outputs out, int M, int cols, int K, int x_tiles, int w_tiles) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mem[];
     using P = PingPong<T, XR>;
@@ -75,7 +75,8 @@ __global__ __launch_bounds__(512, 2) void dense_kernel(const uint16_t* __restric
     p.run(s_mem, rw, vw, rx, vx, K / P::kStage);
     if constexpr (ADD && XR != 128) ask();
     const int part = (n0 >= out.first[1]) + (n0 >= out.first[2]), ldy = pick_part(out.ldy, part);
-    uint16_t* __restrict__ y = pick_part(out.y, part) + (n0 - pick_part(out.first, part));
+    using Result = std::conditional_t<ADD, uint16_t*, uint16_t* __restrict__>;       // the residual may be the result
+    const Result y = pick_part(out.y, part) + (n0 - pick_part(out.first, part));
     const auto store = [&](int r, int c, u32x4 v) {
         if (m0 + r < M && n0 + c < out_cols) *reinterpret_cast<u32x4*>(y + (size_t)(m0 + r) * ldy + c) = v;
     };

@@ -285,7 +285,7 @@ def test_gemm_largest_shapes_properties(M, K, N):
 # buffers in flight at the start), every group size form, a weight of two slabs (131072 x 1032: 270 MB)
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 @pytest.mark.parametrize("M,K,N,g", [(1, 64, 8, 64), (129, 128, 264, 32), (300, 192, 520, 64), (256, 256, 256, 128),
-                                      (4352, 320, 4104, 64), (700, 1024, 1032, 1024), (40, 131072, 1032, 128)])
+                                      (4352, 320, 4104, 64), (8200, 320, 4104, 64), (700, 1024, 1032, 1024), (40, 131072, 1032, 128)])
 def test_linear_dense(dtype, M, K, N, g):
     """The weight dequantised first, with bias and with the gated epilogue, against the fp64 product of the dequantised
     weight and against the separate activation kernel; rows of zeros stay zero, two runs give the same bits."""
@@ -318,6 +318,13 @@ def test_linear_dense(dtype, M, K, N, g):
     assert M == 1 or torch.count_nonzero(y[M // 2]) == 0
     if N % 16 == 0:
         assert torch.equal(dense(None, True), ops.silu_mul(y, interleaved=True))
+    # with a residual, in a tensor of its own and in place: the bits of an addition behind the product, and nothing behind the rows
+    r = torch.randn(M + 1, N, device="cuda", generator=gen).to(tdt)
+    for out in (torch.full_like(r, 3.0), r.clone()):
+        last, res = out[M].clone(), out if torch.equal(out, r) else r
+        _lib.check(L.awq_linear_dense_add(x.data_ptr(), qw.data_ptr(), qs.data_ptr(), qz.data_ptr(), res.data_ptr(), out.data_ptr(), M, N, K, g,
+                                          _lib.dtype_id(tdt), scratch.data_ptr(), scratch.numel(), _lib.current_stream_ptr(y.device)))
+        assert torch.equal(out[:M], r[:M] + y) and torch.equal(out[M], last)
 
 
 def test_linear_dense_routes():
