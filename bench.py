@@ -176,8 +176,9 @@ def gemv_kernel_name(M, N, K, dtype_name, g=G):
     if wide:
         wn = 2 if wide.group(1) else 4
         kern = f"awq::gemv_wide_kernel<{T},{wide.group(2)},{wide.group(3)},{'true' if wide.group(4) else 'false'},{wn}>"
-        if not wide.group(4):   # the K splits are added by a second kernel
-            kern += f" + awq::gemv_wide_reduce_kernel<{T}>"
+        if not wide.group(4) and sp.value > 1:   # the K splits are added by a second kernel: fragments above 16 rows, rows up to there
+            second = "add" if M > 16 and int(wide.group(3)) >= 2 else "reduce"
+            kern += f" + awq::gemv_wide_{second}_kernel<{T},{8 if sp.value <= 8 else 16}>"
     elif name.startswith("dma"):
         kern = f"awq::gemv_dma_kernel<{T},{name[5]},plain>"
     else:
@@ -436,7 +437,7 @@ def main():
             del copies
             torch.cuda.empty_cache()
         out["batched_decode_gemv"] = {
-            "kernel": "awq::gemv_wide_kernel + awq::gemv_wide_reduce_kernel (each case names its own form)",
+            "kernel": "awq::gemv_wide_kernel + awq::gemv_wide_add_kernel (each case names its own form)",
             "unit": "GB/s of packed weights",
             "note": "17..64 rows (cfg5 decodes at 64): bound by the SIMDs' issue ports (MFMA + unpack + fold + load-to-LDS "
                     "instructions; at 33..64 rows the 244 registers a wave holds leave two waves per SIMD) plus the K "
@@ -610,7 +611,7 @@ def main():
                 "decode_ms_per_step": round(ms_step, 2),
                 "roofline": step_roofline(decode_step_bytes(model, B * (P + 8)), ms_step,
                                           "decode step: awq::gemv_wide_kernel / gemv_dma_kernel forms + "
-                                          "awq::paged_attn_decode_mfma_kernel"),
+                                          "awq::paged_attn_decode_tr_kernel"),
             }
             del eng, model
             torch.cuda.empty_cache()
