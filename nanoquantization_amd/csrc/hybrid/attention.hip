@@ -577,14 +577,24 @@ __device__ __forceinline__ void attn_tile(
     }
 }
 
-template <int R, int RV, int KT, bool DENSE, bool FIRST>
+template <int R, int RV, int KT, bool DENSE>
 __global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
     const uint16_t* __restrict__ sink, DenseKV dense, uint16_t* __restrict__ out, int heads, int kv_heads, int vdim,
     int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles) {
-    attn_tile<R, RV, KT, DENSE, false, FIRST>(q, k_cache, v_cache, block_tables, segments, tiles, sink, dense, out, heads, kv_heads, vdim,
-                                       block_size, max_blocks, num_blocks, chunk, window, scale, q_tiles);
+    attn_tile<R, RV, KT, DENSE, false, false>(q, k_cache, v_cache, block_tables, segments, tiles, sink, dense, out, heads, kv_heads, vdim,
+                                              block_size, max_blocks, num_blocks, chunk, window, scale, q_tiles);
+}
+// the same with waves that go before one another
+template <int R, int RV, int KT, bool DENSE>
+__global__ __launch_bounds__(256, R + RV > 320 ? 1 : 2) void attn_tile_first_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
+    const int32_t* __restrict__ block_tables, const int32_t* __restrict__ segments, const int32_t* __restrict__ tiles,
+    const uint16_t* __restrict__ sink, DenseKV dense, uint16_t* __restrict__ out, int heads, int kv_heads, int vdim,
+    int block_size, int max_blocks, int num_blocks, int chunk, int window, float scale, int q_tiles) {
+    attn_tile<R, RV, KT, DENSE, false, true>(q, k_cache, v_cache, block_tables, segments, tiles, sink, dense, out, heads, kv_heads, vdim,
+                                             block_size, max_blocks, num_blocks, chunk, window, scale, q_tiles);
 }
 
 // No sink, chunk or window, but given at run time: with them known the compiler holds more across the key loop than the
@@ -595,7 +605,7 @@ __global__ __launch_bounds__(256, R > 160 ? 1 : 2) void attn_even_kernel(
     const uint16_t* __restrict__ sink, uint16_t* __restrict__ out, int heads, int kv_heads, int batch, int tokens, int chunk,
     int window, float scale, int q_tiles) {
     attn_tile<R, R, KT, false, true, FIRST>(q, k, v, nullptr, nullptr, nullptr, sink, DenseKV{}, out, heads, kv_heads, R, tokens, 1,
-                                     batch, chunk, window, scale, q_tiles);
+                                            batch, chunk, window, scale, q_tiles);
 }
 
 // Decode attention.  Workgroup = (sequence, kv head, 16 of its query heads, context split); a wave takes tiles of 32 keys
@@ -1054,7 +1064,7 @@ extern "C" int nqh_attention_prefill(const void* q, const void* k_cache, const v
             constexpr int KT = R >= 192 ? 32 : 64;
             // (the table's length stands in for that of the longest sequence, which is on the device)
             const bool first = go_first(groups, most_keys(block_size * max_blocks, chunk, window));
-            (first ? attn_tile_kernel<R, R, KT, false, true> : attn_tile_kernel<R, R, KT, false, false>)<<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
+            (first ? attn_tile_first_kernel<R, R, KT, false> : attn_tile_kernel<R, R, KT, false>)<<<dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(
                 (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables, segments, tiles,
                 (const uint16_t*)sink, DenseKV{}, (uint16_t*)out, (int)heads, (int)kv_heads, (int)vdim, (int)block_size,
                 (int)max_blocks, (int)num_blocks, (int)chunk, (int)window, scale, (int)num_tiles);
@@ -1243,7 +1253,7 @@ extern "C" int nqh_latent_attention_prefill(const void* q, const void* kv, int64
     const DenseKV dense{(const uint16_t*)kv, (const uint16_t*)rot, first, kv_stride, rot_stride, heads * dim, (int)dim, (int)rot_dim};
     (void)hipGetLastError();
 #define NQH_GO(R, RV, KT)                                                                                                   \
-    (go_first(groups, kMaxI32) ? attn_tile_kernel<R, RV, KT, true, true> : attn_tile_kernel<R, RV, KT, true, false>)<<<    \
+    (go_first(groups, kMaxI32) ? attn_tile_first_kernel<R, RV, KT, true> : attn_tile_kernel<R, RV, KT, true>)<<<            \
         dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream>>>(                                                       \
         (const uint16_t*)q, nullptr, nullptr, nullptr, segments, tiles, nullptr, dense, (uint16_t*)out, (int)heads,          \
         (int)heads, (int)vdim, 1, 0, 0, 0, 0, scale, (int)num_tiles)

@@ -203,3 +203,37 @@ def test_hybrid_kernels_wait_for_their_tile_loads(tmp_path):
         assert kinds.count("load") == (2 * ahead + 1) * stage, name
         found += 1
     assert found == 3 * (2 + 3 + 3)
+
+
+@pytest.mark.skipif(shutil.which(nq_build.HIPCC) is None and not os.path.exists(nq_build.HIPCC), reason="hipcc not found")
+def test_hybrid_attention_by_its_other_names(tmp_path):
+    """The decode kernel past the L2, the prompt kernels whose waves go before one another and those of dense keys wait for their tile loads as
+    their namesakes do: a count that leaves the V tile's open, and none for the next stage in front of the first matrix instruction."""
+    out = tmp_path / "attention.s"
+    flags = [f for f in nq_build.FLAGS if f not in ("-shared", "-fPIC")]
+    cmd = [nq_build.HIPCC, *flags, "--cuda-device-only", "-S", os.path.join(nq_build.HYBRID_CSRC, "attention.hip"), "-o", str(out)]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert proc.returncode == 0, proc.stdout[-2000:]
+    asm, found = out.read_text(), {}
+    for kernel in ("attn_decode_past_l2_kernel", "attn_tile_first_kernel", "attn_even_kernel"):
+        for name in re.findall(r"^(_ZN3nqh\S*\d%s[^:\s]*):" % kernel, asm, re.M):
+            begin = asm.index("\n" + name + ":")
+            ins = [l.strip() for l in asm[begin:asm.index(".Lfunc_end", begin)].split("\n")]
+            ins = [l for l in ins if l and l[0] not in ";." and not l.endswith(":")]
+            found[kernel] = found.get(kernel, 0) + 1
+            if "decode" in kernel:
+                loads = int(re.search(r"kernelILi(\d+)E", name).group(1)) // 16
+                dma = [k for k, l in enumerate(ins) if "global_load_lds_dwordx4" in l]
+                assert len(dma) == 2 * loads and all(ins[k].endswith(" nt") for k in dma), (name, len(dma))
+                wait = next(k for k in range(dma[-1] + 1, len(ins)) if ins[k].startswith("s_waitcnt") and "vmcnt" in ins[k])
+                assert "vmcnt(%d)" % loads in ins[wait], (name, ins[wait])
+                assert not any(l.startswith(("global_", "buffer_", "flat_", "ds_read")) for l in ins[dma[-1] + 1:wait]), name
+                continue
+            first = next(k for k, l in enumerate(ins) if "v_mfma" in l)
+            bar = max(k for k in range(first) if ins[k].startswith("s_barrier"))
+            assert any("vmcnt(0)" in l for l in ins[bar - 4:bar]) and not any("vmcnt(0)" in l for l in ins[bar:first]), name
+            raised, settled = (sum(l == "s_setprio %d" % p for l in ins) for p in (1, 0))
+            rows = sum(int(v) for v in re.search(r"kernelILi(\d+)ELi(\d+)E", name).groups()) if "first" in kernel else 0
+            goes_first = 0 < rows < 512 or "even" in kernel and "ELb1EEE" in name       # (rows of 256 keys and values have a loop of their own)
+            assert raised == settled and (raised > 0) == goes_first, (name, raised, settled)
+    assert found == {"attn_decode_past_l2_kernel": 6, "attn_tile_first_kernel": 13, "attn_even_kernel": 5}
