@@ -76,8 +76,9 @@ class EngineCore:
     def _decode_step(self) -> None:
         raise NotImplementedError
 
-    def _follow_weights(self) -> None:
-        """Before a call's first step: weights that the engine keeps in a layout of its own for its steps alone, as the modules hold them now."""
+    def _follow_weights(self) -> bool:
+        """Weights that the engine keeps in a layout of its own for its steps alone, as the modules hold them now: whether any had changed."""
+        return False
 
     # ---- leases ----------------------------------------------------------------------------------
     def acquire(self, num_blocks: int) -> Lease:
@@ -127,9 +128,13 @@ class EngineCore:
             state["s_ids"][i], state["s_pos"][i], state["s_slot"][i] = int(token), int(pos), lease.slot
             state["s_table"][i, :len(lease.blocks)] = lease.blocks
         state["s_active"][:n] = True
-        upload(state.reshape(1).view(np.uint8), self.device, out=self._decode_state)
-        self._follow_weights()      # (beside the copy)
-        self._run_decode()
+        def step():
+            upload(state.reshape(1).view(np.uint8), self.device, out=self._decode_state)
+            self._run_decode()
+        step()
+        # looked at while the step runs; where something had changed the step is taken again, from the same state to the same cache slots
+        if self._follow_weights():
+            step()
         return self.s_logits[:n]
 
     def _finish_step(self, logits: torch.Tensor) -> None:

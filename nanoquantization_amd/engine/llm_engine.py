@@ -110,21 +110,22 @@ class LLMEngine(EngineCore):
     def _weights_now(self) -> List[torch.Tensor]:
         return [t for l in self.model.model.layers for m in (l.self_attn.o_proj, l.mlp.down_proj) for t in (m.qweight, m.qscales, m.qzeros)]
 
-    def _follow_weights(self) -> None:
+    def _follow_weights(self) -> bool:
         """The launches one by one read o_proj and down_proj where the modules have them (q|k|v and gate|up are copies made with the
         engine): the block steps' copies of these follow what is written there in place and, without a graph, the tensors that take their
         place.  Writes that torch does not count (through .data or a raw pointer, to inference tensors) are not seen.  Without a change 28 layers
         take 8 us of the host."""
         if self.block_steps is None:
-            return
+            return False
         weights = self._weights if self.use_graph else self._weights_now()
         written = _times_written(weights)
         if written == self._written and (self.use_graph or all(map(operator.is_, weights, self._weights))):
-            return
+            return False
         for i in range(0, len(weights), 3):
             if written[i:i + 3] != self._written[i:i + 3] or any(map(operator.is_not, weights[i:i + 3], self._weights[i:i + 3])):
                 self.block_steps.replace(i // 6, ("o_proj", "down_proj")[i // 3 % 2], weights[i:i + 3])
         self._weights, self._written = weights, written
+        return True
 
     # ---- prefill: full causal attention over the prompt itself ------------------------------------
     def _prompt_layout(self, lens: List[int], leases: List[Lease]) -> Optional[hybrid_ops.PromptPass]:
