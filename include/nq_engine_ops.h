@@ -142,7 +142,7 @@ int nq_tile_weight(const int32_t* qweight, const void* qscales, const int32_t* q
  * down [hidden, inter], qkv [(heads + 2 * kv_heads) * 128, hidden] as [N, K].  res_in, res_out: [rows, hidden]; attn (of heads * 128 columns),
  * act (inter), tiled_mid and tiled_out (res_mid and res_out, hidden) have nq_paged_attention_decode_tiled's layout; squares_mid and squares_out are
  * fp32 [ceil(rows / 16)][hidden / 128][16 rows][16 sums of eight columns' squares].  The result's bits are those of the launches one by one with K cut as awq_gemv_add_residual and
- * awq_gemv_rmsnorm cut it at these sizes (hidden 2048: at up to 16 rows).  Rows past `rows` of attn must be numbers.
+ * awq_gemv_rmsnorm cut it at these sizes (hidden 2048: at 5 to 16 rows).  Rows past `rows` of attn must be numbers.
  * `done`: nq_block_step_flag_words() words that are zero when the launch begins, of its own while it runs; `clear`: as many words of another launch
  * that is over, which this one sets to zero (the launches of a step clear each other's in a ring).  Every buffer is of its own,
  * 16-byte aligned, and attn, res_out, act, q_out, the tiled residuals, the squares, done and clear begin on a line of 128 bytes.

@@ -6,14 +6,14 @@
 // a phase is: the phase before is known to be over, x arrives, some matrix instructions, the sums of the chunks of K, the result leaves.  Times
 // inside a launch, Qwen3-0.6B, 32 rows, us: o_proj 6.9 (its weights and x come from memory), the others 4.2 to 5; of a phase 1.3 go by until the phase
 // before is known to be over, 1.2 for x, 0.6 for the norm, 0.5 for the product, 0.9 for the sums and the epilogue, 0.4 until the results are out.
-// Whole decode steps before (five launches a layer) / now, us: Qwen3-0.6B, 28 layers, 32 sequences of 640 tokens 1576 / 1287; six layers, 1 / 16 / 64
+// Whole decode steps, the attention beside it unchanged, before (five launches a layer) / now, us: Qwen3-0.6B, 28 layers, 32 sequences of 640 tokens 1576 / 1287; six layers, 1 / 16 / 64
 // rows 283 / 244, 333 / 277, 479 / 423; six layers of Qwen3-1.7B, 1 / 16 / 32 rows 346 / 333, 402 / 353, 451 / 406.
 //
 // Weights lie in pieces of 128 rows x 16 columns in operand order (nq_tile_weight): a load is 1 KiB without gaps, where the packed
 // layout gives a CU 64 bytes of a row at a time, and eight codes of a lane unpack with seven instructions.  A task is a row tile of 16 (or two) by one
 // column tile (three of gate|up, the eight of a head of q|k|v); the eight waves of a workgroup share its K.  Narrow tiles because 1024
 // columns have to keep as many CUs busy as there are.  Between phases x lies in operand order too: rows as they are cost 2.7 us instead of 1.3.
-// The sums are added in the GEMVs' order and the norm rounds where theirs does, so that a model of 28 layers gives the same logits (with the norm
+// The sums are added in the GEMVs' order (hidden 2048: as they have it at 5 to 16 rows) and the norm rounds where theirs does, so that a model of 28 layers gives the same logits (with the norm
 // round the sums, 1 / rms behind the product, a step takes 30 us less and its logits are 4.6 % of their norm away, as far as both are from
 // 64 bits).
 //
@@ -159,8 +159,8 @@ __device__ __forceinline__ void multiply(const u32x4 (&v)[C][MT][4], f32x4 (&y)[
 }
 
 // The sums of the wave's chunks to its part of LDS; then, behind a barrier, lane (column, 4 rows) of tile t = (c, m) adds those of all chunks: up to
-// eight one after the other, more in fours whose sums are added one after the other (the order of the GEMVs' waves and K splits at up to 16 rows
-// and, of the first size, at all).
+// eight one after the other, more in fours whose sums are added one after the other (the order of the GEMVs' waves and K splits, of the
+// second size at 5 to 16 rows).
 template <int CT, int MT, int C>
 __device__ __forceinline__ void sums_to_lds(const f32x4 (&y)[C][CT][MT], char* mine, int lane) {
 #pragma unroll
